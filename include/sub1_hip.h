@@ -270,8 +270,8 @@ int sub1_moe_prepare_codes(const sub1_moe_stack *stack, const sub1_moe_prepared 
  * and 4-byte aligned).  Nothing is stacked first: a layer is loaded into its
  * Sub1Linear buffers as the reference does (sub1.py:284-292) and prepared from
  * there, and the only memory a launch needs afterwards is the prepared pair.
- * Both calls copy the six tables to the host to look at them (they synchronise
- * the stream).  Same results as preparing the stacked copy of these buffers.
+ * Both calls look the six tables over on the GPU first (they synchronise the
+ * stream).  Same results as preparing the stacked copy of these buffers.
  */
 typedef struct sub1_moe_layers {
   const int32_t *dec;

@@ -86,7 +86,7 @@ struct MetaLayout {
   int kinds;
   int64_t counts;       // i32 [all slices + 1] chunk counts, scanned in place
   int64_t status;       // i32 [4]: [0] rows whose codes do not cover the width, [1], [2]
-                        // longest slice of kind 0 / 1 in chunks
+                        // longest slice of kind 0 / 1 in chunks, [3] what check_on_device found
   int64_t bytes;
 };
 
@@ -268,58 +268,157 @@ __global__ __launch_bounds__(256) void count_entries_kernel(
   row_len[g] = static_cast<uint16_t>(min(entries, kMaxRowEntries));
 }
 
-// One workgroup per matrix: order the rows by entry count, longest first, and
-// describe the 64-row slices.  The order is a counting sort carried out by one
-// thread, so it is the same on every run.  Dynamic LDS: the histogram
-// (kMaxRowEntries + 2 counters), then the entry count of the first row of up to
-// 1024 slices.
-constexpr size_t kOrderRowsLds = (kMaxRowEntries + 2 + 1024) * sizeof(int);
-__global__ __launch_bounds__(256) void order_rows_kernel(
+// One workgroup per matrix: order the rows by entry count, longest first, rows
+// of equal count by row number, and describe the 64-row slices.  A counting sort,
+// the same order on every run: a histogram over the counts between the smallest
+// and the largest, its prefix sums, then the rows 64 at a time, each after the
+// places that the ones before it have taken.  That last part is a chain, so only
+// what has to be is in it: a row's rank among the equal counts of its 64 is found
+// beforehand by all wavefronts (a ballot per bit of the count), one wavefront then
+// needs two LDS accesses per 64 rows.  128 base experts: 24 us
+// for wi (3072 rows), 10 for wo, where one thread that walked the histogram and took
+// the rows one by one needed 750 and 325.
+// Dynamic LDS: the bins, the entry count of the first row of up to 1024 slices
+// (65534 rows), a few words per wavefront, and a byte per row.
+constexpr int kOrderThreads = 1024;
+constexpr int kOrderWaves = kOrderThreads / 64;
+constexpr int kOrderBins = kMaxRowEntries + 1;
+constexpr int kOrderAhead = 8;   // runs of 64 rows whose counts are asked for together
+size_t order_rows_lds(int height) {
+  return (kOrderBins + 1024 + 2 * kOrderWaves) * sizeof(int) + static_cast<size_t>(height + 63) / 64 * 64;
+}
+__global__ __launch_bounds__(kOrderThreads) void order_rows_kernel(
     const uint16_t *__restrict__ row_len_all, KindSource ks,
     uint16_t *__restrict__ row_idx, uint32_t *__restrict__ minmax_sorted,
     uint16_t *__restrict__ slice_len, int32_t *__restrict__ counts,
     int32_t *__restrict__ status, int height, int slices, int kind) {
   extern __shared__ int order_lds[];
-  int *hist = order_lds;
-  int *first_len = order_lds + kMaxRowEntries + 2;
-  const int e = blockIdx.x;
+  int *bins = order_lds;
+  int *first_len = bins + kOrderBins;
+  int *wave_a = first_len + 1024, *wave_b = wave_a + kOrderWaves;
+  uint8_t *rank = reinterpret_cast<uint8_t *>(wave_b + kOrderWaves);
+  const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint16_t *rl = row_len_all + static_cast<int64_t>(e) * height;
   const uint32_t *mm = ks.minmax_of ? ks.minmax_of[e] : ks.minmax + static_cast<int64_t>(e) * height;
   const int64_t lane0 = static_cast<int64_t>(e) * slices * 64;
-  for (int i = threadIdx.x; i < kMaxRowEntries + 2; i += blockDim.x) hist[i] = 0;
-  __syncthreads();
-  for (int r = threadIdx.x; r < height; r += blockDim.x)
-    atomicAdd(&hist[min(static_cast<int>(rl[r]), kMaxRowEntries)], 1);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int run = 0;  // rows with a larger count come first
-    for (int len = kMaxRowEntries; len >= 0; len--) {
-      int n = hist[len];
-      hist[len] = run;
-      run += n;
-    }
-    for (int r = 0; r < height; r++) {
-      const int len = min(static_cast<int>(rl[r]), kMaxRowEntries);
-      int p = hist[len]++;
-      row_idx[lane0 + p] = static_cast<uint16_t>(r);
-      minmax_sorted[lane0 + p] = mm[r];
-      if ((p & 63) == 0 && (p >> 6) < 1024) first_len[p >> 6] = len;
-    }
+
+  int low = kMaxRowEntries, high = 0;
+  for (int r = tid; r < height; r += kOrderThreads) {
+    low = min(low, static_cast<int>(rl[r]));
+    high = max(high, static_cast<int>(rl[r]));
   }
-  for (int p = height + threadIdx.x; p < slices * 64; p += blockDim.x) {
-    row_idx[lane0 + p] = 0xffffu;
-    minmax_sorted[lane0 + p] = 0u;
+  for (int m = 1; m < 64; m <<= 1) {
+    low = min(low, __shfl_xor(low, m, 64));
+    high = max(high, __shfl_xor(high, m, 64));
+  }
+  if (lane == 0) {
+    wave_a[wave] = low;
+    wave_b[wave] = high;
   }
   __syncthreads();
-  for (int s = threadIdx.x; s < slices; s += blockDim.x) {
-    // a slice is as long as its first row, and at least one entry
-    int len = s < 1024 ? first_len[s] : static_cast<int>(rl[row_idx[lane0 + 64 * s]]);
-    len = max(len, 1);
-    int64_t g = static_cast<int64_t>(e) * slices + s;
+  for (int w = 0; w < kOrderWaves; w++) {
+    low = min(low, wave_a[w]);
+    high = max(high, wave_b[w]);
+  }
+  const int range = high - low + 1;   // bin b: the rows of high - b entries
+  for (int i = tid; i < range; i += kOrderThreads) bins[i] = 0;
+  __syncthreads();
+  for (int r0 = wave * 64; r0 < height; r0 += kOrderThreads) {
+    const int r = r0 + lane;
+    const int bin = r < height ? high - rl[r] : 0;
+    unsigned long long same = __ballot(r < height);
+    for (int bit = 1; bit < range; bit <<= 1) {
+      const unsigned long long with = __ballot((bin & bit) != 0);
+      same &= (bin & bit) ? with : ~with;
+    }
+    if (r < height) {
+      const int before = __popcll(same & ((1ull << lane) - 1));
+      const bool last = lane == 63 - __clzll(same);
+      rank[r] = static_cast<uint8_t>(before | (last ? 64 : 0));
+      if (last) atomicAdd(&bins[bin], before + 1);
+    }
+  }
+  __syncthreads();
+  int carry = 0;
+  for (int b0 = 0; b0 < range; b0 += kOrderThreads) {   // every bin's first place
+    const int n = b0 + tid < range ? bins[b0 + tid] : 0;
+    int upto = n;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(upto, d, 64);
+      if (lane >= d) upto += v;
+    }
+    if (lane == 63) wave_a[wave] = upto;
+    __syncthreads();
+    int before = carry;
+    for (int w = 0; w < kOrderWaves; w++) {
+      if (w < wave) before += wave_a[w];
+      carry += wave_a[w];
+    }
+    if (b0 + tid < range) bins[b0 + tid] = before + upto - n;
+    __syncthreads();
+  }
+  if (wave == 0) {
+    volatile int *place = bins;   // read and written by this wavefront alone, in program order
+    for (int r0 = 0; r0 < height; r0 += 64 * kOrderAhead) {
+      int len[kOrderAhead];
+#pragma unroll
+      for (int u = 0; u < kOrderAhead; u++) {
+        const int r = r0 + 64 * u + lane;
+        len[u] = r < height ? rl[r] : 0;
+      }
+#pragma unroll
+      for (int u = 0; u < kOrderAhead; u++) {
+        const int r = r0 + 64 * u + lane;
+        if (r < height) {
+          const int mine = rank[r];
+          const int p = place[high - len[u]] + (mine & 63);
+          if (mine & 64) place[high - len[u]] = p + 1;
+          row_idx[lane0 + p] = static_cast<uint16_t>(r);
+          if ((p & 63) == 0) first_len[p >> 6] = len[u];
+        }
+      }
+    }
+  } else {
+    for (int p = height + tid - 64; p < slices * 64; p += kOrderThreads - 64) {
+      row_idx[lane0 + p] = 0xffffu;
+      minmax_sorted[lane0 + p] = 0u;
+    }
+  }
+  __syncthreads();   // covers row_idx too: one workgroup, one L1
+  for (int p = tid; p < height; p += kOrderThreads) minmax_sorted[lane0 + p] = mm[row_idx[lane0 + p]];
+  for (int s = tid; s < slices; s += kOrderThreads) {
+    const int len = max(first_len[s], 1);   // a slice is as long as its first row, and at least one entry
+    const int64_t g = static_cast<int64_t>(e) * slices + s;
     slice_len[g] = static_cast<uint16_t>(len);
     counts[g + 1] = chunks_of(len);
     atomicMax(&status[1 + kind], chunks_of(len));
   }
+}
+
+// What the prepare passes take on trust is looked at on the GPU first: whether
+// dec is the fixed dictionary's table, and the tables of device pointers entry by
+// entry.  A workgroup of 256 compares 4 KB of dec; the workgroups then share the
+// pointers.  *found: bit 0 = dec differs, bit 1 = a pointer is NULL or misaligned.
+struct PointerTables {
+  const void *const *table[6];
+  uint32_t align[6];
+  int n, count;
+};
+constexpr int kCheckBlocks = SUB1_DEC_WORDS / 4 / 256;
+__global__ __launch_bounds__(256) void check_source_kernel(const int32_t *__restrict__ dec,
+                                                           const int32_t *__restrict__ fixed,
+                                                           PointerTables pt, int32_t *found) {
+  const int at = blockIdx.x * 256 + threadIdx.x;
+  int32_t a[4], b[4];
+  __builtin_memcpy(a, dec + 4 * at, 16);
+  __builtin_memcpy(b, fixed + 4 * at, 16);
+  int bad = ((a[0] ^ b[0]) | (a[1] ^ b[1]) | (a[2] ^ b[2]) | (a[3] ^ b[3])) ? 1 : 0;
+  for (int t = 0; t < pt.n; t++)
+    for (int i = at; i < pt.count; i += kCheckBlocks * 256) {
+      const uintptr_t v = reinterpret_cast<uintptr_t>(pt.table[t][i]);
+      if (v == 0 || (v & (pt.align[t] - 1)) != 0) bad |= 2;
+    }
+  if (bad) atomicOr(found, bad);
 }
 
 // In-place inclusive prefix sum over v[1..n], v[0] = 0; one workgroup.
@@ -2133,18 +2232,29 @@ __global__ __launch_bounds__(kMaxThreads) void matvec_group_kernel(PreparedArgs 
 // ------------------------------------------------------------ host side --
 
 // The prepare kernels read dec as the fixed dictionary's table (symbols 0..2,
-// unused digits zero): refuse any other.  Compared in full on every call (a
-// 512 KB copy and a synchronisation; preparing is a load-time step).
-int check_dec(const int32_t *dec, hipStream_t stream) {
-  std::vector<int32_t> want(SUB1_DEC_WORDS), got(SUB1_DEC_WORDS);
-  int rc = sub1_build_tables(want.data(), nullptr);
-  if (rc) return fail(rc, "sub1_build_tables failed");
-  HIP_TRY(hipMemcpyAsync(got.data(), dec, got.size() * sizeof(int32_t), hipMemcpyDeviceToHost,
-                         stream));
-  HIP_TRY(hipStreamSynchronize(stream));
-  if (std::memcmp(want.data(), got.data(), want.size() * sizeof(int32_t)) != 0)
-    return fail(SUB1_ERR_SHAPE,
-                "sub1_moe_prepare: dec is not the fixed dictionary; use sub1_moe_grouped");
+// unused digits zero) and refuse any other; dec is compared in full on every
+// call, with this copy of the table (512 KB a GPU, filled on its first prepare
+// and held until the process ends).  Building the table on the host and fetching
+// dec to compare it there, as it was done first, took 9 ms a call, two calls to
+// a layer; the kernel and reading its answer back take about 20 us.
+static __device__ __align__(16) int32_t fixed_dec[SUB1_DEC_WORDS];
+std::mutex g_fixed_mutex;
+std::vector<int> g_fixed_devices;   // where fixed_dec is filled
+
+int fixed_dec_of_current_device(const int32_t **out) {
+  int device = 0;
+  void *address = nullptr;
+  HIP_TRY(hipGetDevice(&device));
+  HIP_TRY(hipGetSymbolAddress(&address, HIP_SYMBOL(fixed_dec)));
+  std::lock_guard<std::mutex> lock(g_fixed_mutex);
+  if (std::find(g_fixed_devices.begin(), g_fixed_devices.end(), device) == g_fixed_devices.end()) {
+    std::vector<int32_t> table(SUB1_DEC_WORDS);
+    const int rc = sub1_build_tables(table.data(), nullptr);
+    if (rc) return fail(rc, "sub1_build_tables failed");
+    HIP_TRY(hipMemcpy(address, table.data(), table.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    g_fixed_devices.push_back(device);
+  }
+  *out = static_cast<const int32_t *>(address);
   return SUB1_OK;
 }
 
@@ -2156,11 +2266,10 @@ struct Source {
   int height[2], width[2];
 };
 
-// Pointer tables are copied to the host once and looked at entry by entry.
-int check_pointer_table(const void *const *table, int count, size_t align, const char *what,
-                        const char *who, hipStream_t s) {
-  if (!table) return fail(SUB1_ERR_NULL, "%s: NULL table of %s pointers", who, what);
-  if (misaligned(table, 8)) return fail(SUB1_ERR_ALIGN, "%s: misaligned table of %s pointers", who, what);
+// Names the first NULL or misaligned entry of a pointer table (its contents are
+// fetched for that: check_source_kernel has found that there is one).
+int name_bad_pointer(const void *const *table, int count, size_t align, const char *what,
+                     const char *who, hipStream_t s) {
   std::vector<const void *> host(count);
   HIP_TRY(hipMemcpyAsync(host.data(), table, sizeof(void *) * count, hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
@@ -2172,7 +2281,44 @@ int check_pointer_table(const void *const *table, int count, size_t align, const
   return SUB1_OK;
 }
 
-int check_source(const Source &src, const char *who, hipStream_t s = nullptr) {
+// dec and the pointer tables, looked at on the GPU; `word` is a device word to
+// leave the answer in.  Synchronises the stream.
+int check_on_device(const Source &src, int32_t *word, hipStream_t s, const char *who) {
+  const int32_t *fixed = nullptr;
+  int rc = fixed_dec_of_current_device(&fixed);
+  if (rc) return rc;
+  const char *const names[3] = {"w_comp", "row_off", "ter_minmax"};
+  PointerTables pt{};
+  pt.count = src.count;
+  for (int i = 0; i < src.kinds; i++) {
+    const KindSource &k = src.k[i];
+    if (!k.w_comp_of) continue;
+    const void *const *of[3] = {reinterpret_cast<const void *const *>(k.w_comp_of),
+                                reinterpret_cast<const void *const *>(k.row_off_of),
+                                reinterpret_cast<const void *const *>(k.minmax_of)};
+    for (int j = 0; j < 3; j++) {
+      pt.table[pt.n] = of[j];
+      pt.align[pt.n++] = j == 0 ? 2 : 4;
+    }
+  }
+  zero_words_kernel<<<1, 64, 0, s>>>(word, 1);
+  check_source_kernel<<<kCheckBlocks, 256, 0, s>>>(src.dec, fixed, pt, word);
+  HIP_TRY(hipGetLastError());
+  int32_t found = 0;
+  HIP_TRY(hipMemcpyAsync(&found, word, sizeof found, hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipStreamSynchronize(s));
+  if (found & 2)
+    for (int t = 0; t < pt.n; t++) {
+      rc = name_bad_pointer(pt.table[t], pt.count, pt.align[t], names[t % 3], who, s);
+      if (rc) return rc;
+    }
+  if (found & 1)
+    return fail(SUB1_ERR_SHAPE,
+                "sub1_moe_prepare: dec is not the fixed dictionary; use sub1_moe_grouped");
+  return SUB1_OK;
+}
+
+int check_source(const Source &src, const char *who) {
   if (!src.dec) return fail(SUB1_ERR_NULL, "%s: NULL pointer", who);
   if (src.count < 1) return fail(SUB1_ERR_SHAPE, "%s: %d matrices", who, src.count);
   int64_t slices = 0;
@@ -2183,15 +2329,14 @@ int check_source(const Source &src, const char *who, hipStream_t s = nullptr) {
       return fail(SUB1_ERR_SHAPE, "%s: matrix %d x %d (height 1..65534, width 1..%d)", who,
                   src.height[i], src.width[i], SUB1_PREPARED_MAX_WIDTH);
     if (k.w_comp_of || k.row_off_of || k.minmax_of) {
-      int rc = check_pointer_table(reinterpret_cast<const void *const *>(k.w_comp_of), src.count, 2,
-                                   "w_comp", who, s);
-      if (!rc)
-        rc = check_pointer_table(reinterpret_cast<const void *const *>(k.row_off_of), src.count, 4,
-                                 "row_off", who, s);
-      if (!rc)
-        rc = check_pointer_table(reinterpret_cast<const void *const *>(k.minmax_of), src.count, 4,
-                                 "ter_minmax", who, s);
-      if (rc) return rc;
+      const void *const tables[3] = {k.w_comp_of, k.row_off_of, k.minmax_of};
+      const char *const names[3] = {"w_comp", "row_off", "ter_minmax"};
+      for (int j = 0; j < 3; j++) {
+        if (!tables[j])
+          return fail(SUB1_ERR_NULL, "%s: NULL table of %s pointers", who, names[j]);
+        if (misaligned(tables[j], 8))
+          return fail(SUB1_ERR_ALIGN, "%s: misaligned table of %s pointers", who, names[j]);
+      }
     } else {
       if (!k.w_comp || !k.row_off || !k.minmax || (src.count > 1 && !k.code_base))
         return fail(SUB1_ERR_NULL, "%s: NULL pointer", who);
@@ -2284,15 +2429,15 @@ int prepare_layout(const Source &src, void *meta, int64_t meta_bytes, LayoutResu
   const MetaLayout m = meta_layout(src.count, src.kinds, src.height, src.width);
   if (meta_bytes < m.bytes)
     return fail(SUB1_ERR_SHAPE, "%s: meta needs %lld bytes", who, static_cast<long long>(m.bytes));
-  int rc = check_dec(src.dec, s);
-  if (rc) return rc;
   char *base = static_cast<char *>(meta);
   int32_t *status = reinterpret_cast<int32_t *>(base + m.status);
+  int rc = check_on_device(src, status + 3, s, who);
+  if (rc) return rc;
   int32_t *counts = reinterpret_cast<int32_t *>(base + m.counts);
-  zero_words_kernel<<<1, 64, 0, s>>>(status, 4);
+  zero_words_kernel<<<1, 64, 0, s>>>(status, 3);
   HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(order_rows_kernel),
                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                              static_cast<int>(kOrderRowsLds)));
+                              static_cast<int>(order_rows_lds(65534))));
   int64_t slice0 = 0;
   for (int i = 0; i < src.kinds; i++) {
     const KindMeta &k = m.k[i];
@@ -2300,7 +2445,7 @@ int prepare_layout(const Source &src, void *meta, int64_t meta_bytes, LayoutResu
     const int64_t rows = static_cast<int64_t>(src.count) * k.height;
     count_entries_kernel<<<static_cast<unsigned>((rows + 255) / 256), 256, 0, s>>>(
         src.k[i], src.dec, row_len, status, k.height, k.width, rows);
-    order_rows_kernel<<<src.count, 256, kOrderRowsLds, s>>>(
+    order_rows_kernel<<<src.count, kOrderThreads, order_rows_lds(k.height), s>>>(
         row_len, src.k[i], reinterpret_cast<uint16_t *>(base + k.row_idx),
         reinterpret_cast<uint32_t *>(base + k.minmax),
         reinterpret_cast<uint16_t *>(base + k.slice_len), counts + slice0, status, k.height,
@@ -2309,7 +2454,7 @@ int prepare_layout(const Source &src, void *meta, int64_t meta_bytes, LayoutResu
   }
   scan_counts_kernel<<<1, 1024, 0, s>>>(counts, static_cast<int>(slice0));
   HIP_TRY(hipGetLastError());
-  int32_t host[4] = {0, 0, 0, 0};
+  int32_t host[3] = {0, 0, 0};
   int32_t total = 0;
   HIP_TRY(hipMemcpyAsync(host, status, sizeof host, hipMemcpyDeviceToHost, s));
   HIP_TRY(hipMemcpyAsync(&total, counts + slice0, 4, hipMemcpyDeviceToHost, s));
@@ -2331,15 +2476,15 @@ int prepare_codes(const Source &src, const Prepared &p, hipStream_t s, const cha
   if (!p.meta || !p.codes) return fail(SUB1_ERR_NULL, "%s: NULL argument", who);
   if (misaligned(p.meta, 256) || misaligned(p.codes, 256))
     return fail(SUB1_ERR_ALIGN, "%s: buffers must be 256-byte aligned", who);
-  int rc = check_dec(src.dec, s);
-  if (rc) return rc;
   const MetaLayout m = meta_layout(src.count, src.kinds, src.height, src.width);
-  const char *base = static_cast<const char *>(p.meta);
+  char *base = static_cast<char *>(const_cast<void *>(p.meta));
   int64_t nslices = 0;
   for (int i = 0; i < src.kinds; i++) nslices += static_cast<int64_t>(src.count) * m.k[i].slices;
   if (p.total_chunks < 0 || p.meta_bytes < m.bytes ||
       p.code_bytes < p.total_chunks * 512 + (p.total_chunks / kGroupChunks + nslices + 1) * 128)
     return fail(SUB1_ERR_SHAPE, "%s: buffers smaller than the layout needs", who);
+  const int rc = check_on_device(src, reinterpret_cast<int32_t *>(base + m.status) + 3, s, who);
+  if (rc) return rc;
   uint2 *stream = static_cast<uint2 *>(const_cast<void *>(p.codes));
   uint16_t *ckpt = reinterpret_cast<uint16_t *>(stream + p.total_chunks * 64);
   int64_t first_slice = 0;
@@ -2927,12 +3072,12 @@ int check_moe_stack(const sub1_moe_stack *st, const char *who) {
   return check_source(moe_source(st), who);
 }
 
-int check_moe_layers(const sub1_moe_layers *l, const char *who, hipStream_t s) {
+int check_moe_layers(const sub1_moe_layers *l, const char *who) {
   if (!l) return fail(SUB1_ERR_NULL, "%s: NULL layers", who);
   if (l->experts < 1 || l->d_model < 1 || l->d_ff < 1)
     return fail(SUB1_ERR_SHAPE, "%s: experts %d d_model %d d_ff %d", who, l->experts, l->d_model,
                 l->d_ff);
-  return check_source(layers_source(l), who, s);
+  return check_source(layers_source(l), who);
 }
 
 void fill_moe_prepared(sub1_moe_prepared *out, void *meta, const LayoutResult &r, int experts,
@@ -2982,7 +3127,7 @@ extern "C" int sub1_moe_prepare_layout_from_layers(const sub1_moe_layers *layers
                                                    void *stream) {
   const char *who = "sub1_moe_prepare_layout_from_layers";
   hipStream_t s = static_cast<hipStream_t>(stream);
-  int rc = check_moe_layers(layers, who, s);
+  int rc = check_moe_layers(layers, who);
   if (rc) return rc;
   if (!out) return fail(SUB1_ERR_NULL, "%s: NULL argument", who);
   LayoutResult r;
@@ -3161,7 +3306,7 @@ extern "C" int sub1_moe_prepare_codes_from_layers(const sub1_moe_layers *layers,
                                                   const sub1_moe_prepared *p, void *stream) {
   const char *who = "sub1_moe_prepare_codes_from_layers";
   hipStream_t s = static_cast<hipStream_t>(stream);
-  int rc = check_moe_layers(layers, who, s);
+  int rc = check_moe_layers(layers, who);
   if (rc) return rc;
   if (!p) return fail(SUB1_ERR_NULL, "%s: NULL argument", who);
   if (p->experts != layers->experts || p->d_model != layers->d_model || p->d_ff != layers->d_ff)
