@@ -106,6 +106,21 @@ int sub1_pack_emit(const int32_t *w_tern, const int32_t *row_off, int16_t *w_com
                    int height, int width, void *stream);
 
 /*
+ * The encoder straight from dense weights (reference sub1.py:145-166, where
+ * torch finds the rows' extremes and marks the symbols in an int32 matrix
+ * first): w bf16 [H, W], a weight equal to its row's smallest is symbol 1, to its
+ * largest symbol 2 (which wins where both are equal), any other 0; fixed
+ * dictionary.  The first call writes (min, max) of every row to ter_minmax bf16
+ * [2H], the rows' codes to `codes` uint16 [H, (W + 1) / 2] and the cumulative
+ * counts to row_off [H+1]; the caller reads row_off[H] to size w_comp, which the
+ * second call fills.  w is only read.
+ */
+int sub1_pack_weights_count(const void *w, uint16_t *codes, void *ter_minmax, int32_t *row_off,
+                            int height, int width, void *stream);
+int sub1_pack_weights_emit(const uint16_t *codes, const int32_t *row_off, int16_t *w_comp,
+                           int height, int width, void *stream);
+
+/*
  * Decoder without the product, for checking: out_tern (uint8 [H, W], symbols)
  * and/or out_w (bf16 [H, W], dequantised weights) may each be NULL.  What the
  * Python `decompress` of reference test.py:103-115 computes.

@@ -167,6 +167,52 @@ __device__ __forceinline__ void leave_launch(int32_t *ctrl, int workgroups) {
   }
 }
 
+// In-place inclusive prefix sum over v[1..n], v[0] = 0, by one workgroup of
+// kScanThreads: 4096 values a turn, the next turn's loads in flight behind it
+// (a thread with a run of its own, as it was first, reads every line 64 times).
+constexpr int kScanThreads = 1024;
+__device__ __forceinline__ void scan_in_place(int32_t *v, int n) {
+  __shared__ int32_t wave_sum[2][kScanThreads / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  auto load = [&](int first, int32_t (&w)[4]) {
+    const int i = first + 4 * tid;
+    if (i + 4 <= n + 1) {
+      __builtin_memcpy(w, v + i, 16);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++) w[j] = i + j <= n ? v[i + j] : 0;
+    }
+  };
+  int32_t next[4], carry = 0;
+  load(1, next);
+  if (tid == 0) v[0] = 0;
+  int side = 0;
+  for (int first = 1; first <= n; first += 4 * kScanThreads, side ^= 1) {
+    int32_t w[4] = {next[0], next[1], next[2], next[3]};
+    if (first + 4 * kScanThreads <= n) load(first + 4 * kScanThreads, next);
+    w[1] += w[0];
+    w[2] += w[1];
+    w[3] += w[2];
+    int32_t upto = w[3];
+    for (int d = 1; d < 64; d <<= 1) {
+      const int32_t u = __shfl_up(upto, d, 64);
+      if (lane >= d) upto += u;
+    }
+    if (lane == 63) wave_sum[side][wave] = upto;
+    __syncthreads();   // the other side's readers are past it by the next turn's barrier
+    int32_t before = carry + upto - w[3];
+    for (int k = 0; k < kScanThreads / 64; k++) {
+      const int32_t u = wave_sum[side][k];
+      if (k < wave) before += u;
+      carry += u;
+    }
+    const int i = first + 4 * tid;
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (i + j <= n) v[i + j] = before + w[j];
+  }
+}
+
 }  // namespace sub1
 
 #define HIP_TRY(expr)                                                               \

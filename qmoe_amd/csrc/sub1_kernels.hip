@@ -1,6 +1,6 @@
 // gfx950 kernels and C ABI of libsub1_hip on the reference's packed layout:
 // the decode-fused matrix-vector product over dictionary-coded ternary
-// weights, the encoder, a plain decoder and the grouped expert-FFN launch that
+// weights, a plain decoder and the grouped expert-FFN launch that
 // needs no preparation.  Written for 64-wide wavefronts.  The single product
 // (matvec_wave_kernel) gives a wavefront to a row: lane j takes codeword j of
 // each run of 64, a prefix sum across the lanes places it, a butterfly adds the
@@ -11,8 +11,6 @@
 //
 // Reference behaviour being reproduced (not its implementation):
 //   sub1_cuda_kernel.cu:129-202  Sub1MatVec       -> matvec_wave_kernel / moe_kernel
-//   sub1_cuda_kernel.cu:211-239  Sub1PreparePack  -> pack_count_kernel
-//   sub1_cuda_kernel.cu:241-250  Sub1Pack         -> pack_emit_kernel
 //   test.py:103-115              decompress       -> decode_kernel
 //   sub1.py:306-321              expert loop      -> moe_kernel
 #include <hip/hip_runtime.h>
@@ -434,79 +432,6 @@ __global__ void decode_kernel(const int32_t *__restrict__ dec,
   if (idx != ((width + 1) & ~1) && bad_rows) atomicAdd(bad_rows, 1);
 }
 
-// --------------------------------------------------------------- pack ------
-
-constexpr int kTrieRoot = SUB1_DICT_ENTRIES;
-
-__global__ void pack_count_kernel(const int32_t *__restrict__ trie,
-                                  int32_t *__restrict__ w_tern,
-                                  int32_t *__restrict__ row_cnt, int height,
-                                  int width) {
-  int row = blockIdx.x * blockDim.x + threadIdx.x;
-  if (row >= height) return;
-  int32_t *w = w_tern + static_cast<int64_t>(row) * width;
-  int node = kTrieRoot;
-  int n = 0;
-  for (int i = 0; i < width; i += 2) {
-    int lo = w[i];
-    int hi = i + 1 < width ? w[i + 1] : 0;
-    int sym = 3 * hi + lo;
-    int child = trie[9 * node + sym];
-    if (child < 0) {
-      // n <= i/2 < i: the slot written was already consumed
-      w[n++] = node;
-      child = trie[9 * kTrieRoot + sym];
-    }
-    node = child;
-  }
-  w[n++] = node;
-  row_cnt[row + 1] = n;
-}
-
-// Inclusive prefix sum over cnt[1..height] in place, cnt[0] = 0.  One
-// workgroup; each thread owns a contiguous segment.
-constexpr int kScanThreads = 1024;
-
-__global__ __launch_bounds__(kScanThreads) void row_offset_scan_kernel(
-    int32_t *__restrict__ cnt, int height) {
-  __shared__ int32_t part[kScanThreads];
-  const int tid = threadIdx.x;
-  const int seg = (height + kScanThreads - 1) / kScanThreads;
-  const int lo = 1 + tid * seg;
-  const int hi = min(height + 1, lo + seg);
-  int32_t s = 0;
-  for (int i = lo; i < hi; i++) s += cnt[i];
-  part[tid] = s;
-  __syncthreads();
-  for (int d = 1; d < kScanThreads; d *= 2) {
-    int32_t v = tid >= d ? part[tid - d] : 0;
-    __syncthreads();
-    part[tid] += v;
-    __syncthreads();
-  }
-  int32_t run = tid ? part[tid - 1] : 0;
-  if (tid == 0) cnt[0] = 0;
-  for (int i = lo; i < hi; i++) {
-    run += cnt[i];
-    cnt[i] = run;
-  }
-}
-
-__global__ void pack_emit_kernel(const int32_t *__restrict__ w_codes,
-                                 const int32_t *__restrict__ row_off,
-                                 uint16_t *__restrict__ w_comp, int height,
-                                 int width) {
-  // one wavefront per row, lanes stride over the row's codes
-  int row = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
-  if (row >= height) return;
-  int lane = threadIdx.x % 64;
-  int off = row_off[row];
-  int n = row_off[row + 1] - off;
-  const int32_t *src = w_codes + static_cast<int64_t>(row) * width;
-  for (int i = lane; i < n; i += 64)
-    w_comp[off + i] = static_cast<uint16_t>(src[i]);
-}
-
 // ------------------------------------------------------ grouped experts ----
 //
 // Persistent grid.  Work is cut into tiles (token, projection, block of
@@ -773,37 +698,6 @@ extern "C" int sub1_matvec(const int32_t *dec, const int16_t *w_comp,
                            void *stream) {
   return sub1_matvec_tokens(dec, w_comp, row_off, ter_minmax, x, y, height, width, 1,
                             width, height, stream);
-}
-
-extern "C" int sub1_pack_count(const int32_t *trie, int32_t *w_tern, int32_t *row_off,
-                               int height, int width, void *stream) {
-  if (!trie || !w_tern || !row_off) return fail(SUB1_ERR_NULL, "sub1_pack_count: NULL argument");
-  if (height < 1 || width < 1)
-    return fail(SUB1_ERR_SHAPE, "sub1_pack_count: height %d width %d", height, width);
-  if (misaligned(trie, 4) || misaligned(w_tern, 4) || misaligned(row_off, 4))
-    return fail(SUB1_ERR_ALIGN, "sub1_pack_count: misaligned pointer");
-  // the cumulative count is kept in int32 like the reference's row_off
-  if (static_cast<int64_t>(height) * ((width + 1) / 2) > INT32_MAX)
-    return fail(SUB1_ERR_SHAPE, "sub1_pack_count: more than 2^31 pairs in one call");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  pack_count_kernel<<<(height + 63) / 64, 64, 0, s>>>(trie, w_tern, row_off, height, width);
-  row_offset_scan_kernel<<<1, kScanThreads, 0, s>>>(row_off, height);
-  HIP_TRY(hipGetLastError());
-  return SUB1_OK;
-}
-
-extern "C" int sub1_pack_emit(const int32_t *w_tern, const int32_t *row_off,
-                              int16_t *w_comp, int height, int width, void *stream) {
-  if (!w_tern || !row_off || !w_comp) return fail(SUB1_ERR_NULL, "sub1_pack_emit: NULL argument");
-  if (height < 1 || width < 1)
-    return fail(SUB1_ERR_SHAPE, "sub1_pack_emit: height %d width %d", height, width);
-  if (misaligned(w_tern, 4) || misaligned(row_off, 4) || misaligned(w_comp, 2))
-    return fail(SUB1_ERR_ALIGN, "sub1_pack_emit: misaligned pointer");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  pack_emit_kernel<<<(height + 3) / 4, 256, 0, s>>>(
-      w_tern, row_off, reinterpret_cast<uint16_t *>(w_comp), height, width);
-  HIP_TRY(hipGetLastError());
-  return SUB1_OK;
 }
 
 extern "C" int sub1_decode(const int32_t *dec, const int16_t *w_comp,

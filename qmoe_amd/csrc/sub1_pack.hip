@@ -1,0 +1,587 @@
+// The encoder: rows of ternary weights to dictionary codes, the longest entry at
+// every place (reference sub1_cuda_kernel.cu:90-126, 211-250 and sub1.py:145-166).
+//
+// The reference walks the trie pair by pair, one row a thread.  The walk is a
+// chain of dependent reads of a 2.4 MB table, 1040 of them for a row of 2080
+// weights, and it cannot be cut: a parse that starts elsewhere in the row hardly
+// ever falls in step with the true one.  For the fixed dictionary the walk is not
+// needed.  Its entries are all strings of pairs with
+//   * at most two non-zero symbols, up to 14 pairs,
+//   * three, up to 12 pairs, and some of 13 pairs,
+// so that the longest entry at a place follows from where the third and the
+// fourth non-zero symbol after it stand, for all places of the row at once, and
+// the entry's number from one look into a table by string.  Both tables are
+// derived from the dictionary on the host, which refuses a dictionary that is not
+// of this form.
+//
+// pack_rows_kernel (a wavefront per row) does this; pack_count_kernel walks a
+// caller's trie where that is not the fixed one.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <mutex>
+#include <type_traits>
+#include <vector>
+
+#include "sub1_common.h"
+
+namespace {
+
+using sub1::fail;
+using sub1::misaligned;
+
+// ------------------------------------------------ the dictionary by string --
+
+constexpr int kMaxPairs = 14;                     // pairs of an entry
+constexpr int kFreeNonzeros = 2;                  // up to so many non-zeros, every string is an entry
+constexpr int kBorderPairs = 13;                  // with one more: every string shorter than this,
+constexpr int kBorderStrings = 2600 * 8;          // and some of this length, C(26, 3) places x 2^3 symbols
+
+// A string of `pairs` pairs: bit d of nz set where symbol d is not zero, of mx
+// where it is 2.  Strings with k non-zeros, shorter ones first, by the places of
+// the non-zeros (colexicographic), then by their symbols.
+__host__ __device__ inline int combinations2(int n) { return n * (n - 1) / 2; }
+__host__ __device__ inline int combinations3(int n) { return n * (n - 1) * (n - 2) / 6; }
+
+__host__ __device__ inline int string_places(uint32_t nz, uint32_t mx, int k) {
+  int places = 0, symbols = 0;
+  for (int j = 1; j <= k; j++) {
+    const int d = __builtin_ctz(nz);
+    nz &= nz - 1;
+    places += j == 1 ? d : j == 2 ? combinations2(d) : combinations3(d);
+    symbols |= static_cast<int>((mx >> d) & 1u) << (j - 1);
+  }
+  return (places << k) + symbols;
+}
+
+constexpr int kFirst1 = kMaxPairs;                               // one string of zeros per length
+constexpr int kFirst2 = kFirst1 + 2 * kMaxPairs * (kMaxPairs + 1);
+constexpr int kFirst3 = kFirst2 + 4 * (kMaxPairs * (kMaxPairs + 1) * (4 * kMaxPairs - 1) / 6);
+constexpr int kStrings = kFirst3 + 8 * (kBorderPairs * kBorderPairs * (kBorderPairs * kBorderPairs - 1) / 3);
+__host__ __device__ inline int string_index(uint32_t nz, uint32_t mx, int pairs) {
+  const int k = __builtin_popcount(nz), m = pairs - 1;
+  if (k == 0) return m;
+  // strings of fewer pairs: sums over l of 2 C(2l, 1), 4 C(2l, 2), 8 C(2l, 3)
+  const int first = k == 1   ? kFirst1 + 2 * m * (m + 1)
+                    : k == 2 ? kFirst2 + 4 * (m * (m + 1) * (4 * m - 1) / 6)
+                             : kFirst3 + 8 * (m * m * (m * m - 1) / 3);
+  return first + string_places(nz, mx, k);
+}
+
+static __device__ uint16_t string_code[kStrings];
+static __device__ uint32_t border_entry[kBorderStrings / 32];    // which 13-pair strings are entries
+static __device__ int32_t fixed_trie[SUB1_TRIE_WORDS];
+
+struct PackTables {
+  const uint16_t *code;
+  const uint32_t *border;
+  const int32_t *trie;
+};
+
+std::mutex g_tables_mutex;
+std::vector<int> g_tables_devices;   // where the three arrays are filled
+
+int fill_tables(const PackTables &t) {
+  std::vector<int32_t> dec(SUB1_DEC_WORDS), trie(SUB1_TRIE_WORDS);
+  int rc = sub1_build_tables(dec.data(), trie.data());
+  if (rc) return fail(rc, "sub1_build_tables failed");
+  std::vector<uint16_t> code(kStrings, 0);
+  std::vector<uint32_t> border(kBorderStrings / 32, 0);
+  int64_t short_strings = 0;   // entries below the border
+  for (int e = 0; e < SUB1_DICT_ENTRIES; e++) {
+    const uint32_t w[2] = {static_cast<uint32_t>(dec[2 * e]), static_cast<uint32_t>(dec[2 * e + 1])};
+    const int pairs = static_cast<int>(w[0] & 15u);
+    uint32_t nz = 0, mx = 0;
+    for (int d = 0; d < 2 * kMaxPairs; d++) {
+      const uint32_t sym = (w[d / 14] >> (4 + 2 * (d % 14))) & 3u;
+      if (sym) nz |= 1u << d;
+      if (sym == 2) mx |= 1u << d;
+    }
+    const int k = __builtin_popcount(nz);
+    const bool at_border = k == kFreeNonzeros + 1 && pairs == kBorderPairs;
+    if (k > kFreeNonzeros + 1 || pairs < 1 || pairs > kMaxPairs ||
+        (k == kFreeNonzeros + 1 && pairs > kBorderPairs) || (nz >> 1) >> (2 * pairs - 1))
+      return fail(SUB1_ERR_INTERNAL, "dictionary entry %d is outside the form of the encoder", e);
+    if (at_border) {
+      const int i = string_places(nz, mx, k);
+      border[i / 32] |= 1u << (i % 32);
+    } else {
+      short_strings++;
+    }
+    code[string_index(nz, mx, pairs)] = static_cast<uint16_t>(e);
+  }
+  // every string below the border has to be an entry (they are distinct)
+  if (short_strings != kStrings - kBorderStrings)
+    return fail(SUB1_ERR_INTERNAL, "the dictionary lacks strings below the border");
+  HIP_TRY(hipMemcpy(const_cast<uint16_t *>(t.code), code.data(), code.size() * 2, hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(const_cast<uint32_t *>(t.border), border.data(), border.size() * 4, hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(const_cast<int32_t *>(t.trie), trie.data(), trie.size() * 4, hipMemcpyHostToDevice));
+  return SUB1_OK;
+}
+
+// The three arrays on the current device (2.7 MB a GPU, filled on the first call
+// there and held until the process ends).
+int tables_of_current_device(PackTables *t) {
+  int device = 0;
+  void *code = nullptr, *border = nullptr, *trie = nullptr;
+  HIP_TRY(hipGetDevice(&device));
+  HIP_TRY(hipGetSymbolAddress(&code, HIP_SYMBOL(string_code)));
+  HIP_TRY(hipGetSymbolAddress(&border, HIP_SYMBOL(border_entry)));
+  HIP_TRY(hipGetSymbolAddress(&trie, HIP_SYMBOL(fixed_trie)));
+  *t = {static_cast<const uint16_t *>(code), static_cast<const uint32_t *>(border),
+        static_cast<const int32_t *>(trie)};
+  std::lock_guard<std::mutex> lock(g_tables_mutex);
+  if (std::find(g_tables_devices.begin(), g_tables_devices.end(), device) == g_tables_devices.end()) {
+    const int rc = fill_tables(*t);
+    if (rc) return rc;
+    g_tables_devices.push_back(device);
+  }
+  return SUB1_OK;
+}
+
+// --------------------------------------------------- rows by wavefront ------
+
+struct PackArgs {
+  int32_t *symbols;          // int32 [height, width], overwritten with the rows' codes; or
+  const uint16_t *weights;   // bf16 [height, width] and
+  uint16_t *codes;           // u16 [height, (width + 1) / 2], where the rows' codes go
+  uint32_t *minmax;          // with weights: (min, max) of every row, as two bf16
+  int32_t *row_cnt;          // [height + 1]: entry row + 1 receives the row's number of codes
+  const int32_t *foreign;    // a word that is not zero where the caller's trie is not the fixed one (NULL: it is)
+  PackTables tables;
+  int height, width;
+  int window;                // pairs of a row taken at a time
+};
+
+constexpr int kPackWaves = 4;           // rows per workgroup
+constexpr int kPackWindow = 4096;       // pairs of a row in LDS at most
+constexpr int kBorderLdsWords = (kBorderStrings / 32 + 3) / 4 * 4;
+constexpr int kAhead = 4;               // loads of a lane that are asked for together
+constexpr int kLookahead = 2 * kMaxPairs;   // symbols past a place that decide its entry
+
+// LDS of a wavefront: two bit planes over the window's symbols (which are not
+// zero, which are 2), and the pairs at which the parse has an entry.
+__host__ __device__ constexpr int plane_words(int window) { return (2 * window + kLookahead + 31) / 32 + 1; }
+__host__ __device__ constexpr size_t pack_lds_per_wave(int window) {
+  return static_cast<size_t>(2 * plane_words(window)) * 4 + (static_cast<size_t>(window) * 2 + 15) / 16 * 16;
+}
+
+__device__ __forceinline__ void wave_lds_fence() {
+  // LDS accesses of a wavefront take place in program order; this keeps the
+  // compiler to it across lanes
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ uint32_t plane_bits(const uint32_t *plane, int at) {
+  const uint32_t lo = plane[at >> 5], hi = plane[(at >> 5) + 1];
+  return __builtin_amdgcn_alignbit(hi, lo, at & 31) & ((1u << kLookahead) - 1);
+}
+
+// Eight values of a row from `at` on, as they lie in memory.  Where that would go
+// past the row's end the last eight of it are read instead, so that a lane's
+// loads take no branch; what was asked for is then `at - from_of(at)` places
+// further up.  (Rows of fewer than eight values: those, the last one repeated.)
+__device__ __forceinline__ int from_of(int at, int width) { return max(min(at, width - 8), 0); }
+struct EightWeights {
+  uint32_t v[4];
+  __device__ __forceinline__ EightWeights(const uint16_t *row, int at, int width) {
+    if (width >= 8) {
+      __builtin_memcpy(v, row + from_of(at, width), sizeof v);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        v[j] = row[min(2 * j, width - 1)] | static_cast<uint32_t>(row[min(2 * j + 1, width - 1)]) << 16;
+    }
+  }
+};
+struct EightSymbols {
+  uint32_t v[8];
+  __device__ __forceinline__ EightSymbols(const int32_t *row, int at, int width) {
+    if (width >= 8) {
+      __builtin_memcpy(v, row + from_of(at, width), sizeof v);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; j++) v[j] = static_cast<uint32_t>(row[min(j, width - 1)]);
+    }
+  }
+};
+// Bits of the eight values asked for at `at`, zero past the row's end.
+__device__ __forceinline__ uint32_t eight_bits(uint32_t bits, int at, int width) {
+  return at < width ? (bits >> (at - from_of(at, width))) & ((1u << min(width - at, 8)) - 1) : 0u;
+}
+
+// bf16 pairs as pairs of int16 in the order of their values (-0 below 0, NaNs
+// outside the infinities); its own inverse.
+typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ i16x2 ordered(i16x2 v) { return v ^ ((v >> 15) & static_cast<int16_t>(0x7fff)); }
+__device__ __forceinline__ int16_t ordered_one(int16_t v) { return v ^ ((v >> 15) & 0x7fff); }
+
+// 1 in either half whose value is not the one sought (`mask` leaves the sign out
+// where that is a zero).
+__device__ __forceinline__ uint32_t not_equal(uint32_t pair, uint32_t mask, uint32_t sought) {
+  const u16x2 d = __builtin_bit_cast(u16x2, (pair & mask) ^ sought);
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(d, u16x2{1, 1}));
+}
+// Four pairs of bits 0 and 16 to eight bits.
+__device__ __forceinline__ uint32_t gather_bits(const uint32_t (&pair)[4]) {
+  const uint32_t x = pair[0] | pair[1] << 2 | pair[2] << 4 | pair[3] << 6;
+  return (x | x >> 15) & 0xffu;
+}
+// The even bits of the low half.
+__device__ __forceinline__ uint32_t even_bits(uint32_t x) {
+  x &= 0x5555u;
+  x = (x | x >> 1) & 0x3333u;
+  x = (x | x >> 2) & 0x0f0fu;
+  return (x | x >> 4) & 0xffu;
+}
+
+template <bool kWeights>
+__device__ __forceinline__ auto row_source(const uint16_t *w, const int32_t *t) {
+  if constexpr (kWeights) return w; else return t;
+}
+
+// What bounds it: instructions.  A 6144 x 2080 matrix takes 33 us, of which 7.5
+// find the rows' extremes (25 MB read, 5 us at the copy rate), 5.5 the planes, 10 the
+// lengths (75 vector instructions for 64 places, 7.5 million over the chip), 6 the
+// way from entry to entry (a scalar read of a lane each, hidden behind the other
+// five rows of a SIMD), 2.5 the codes; 2080 x 6144: 45, with two rows a SIMD its
+// latencies show.  The walk of the trie took 472 us after 60 for the symbols and 33
+// for the extremes in torch.  Looking border strings up only where the parse comes
+// by them (in scalar code) measured 41, the lengths in LDS instead of registers 37.
+template <bool kWeights>
+__global__ __launch_bounds__(64 * kPackWaves) void pack_rows_kernel(PackArgs a) {
+  extern __shared__ uint32_t pack_lds[];
+  if (a.foreign && *a.foreign) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row = blockIdx.x * kPackWaves + wave;
+  uint32_t *border = pack_lds;
+  for (int i = threadIdx.x; i < kBorderStrings / 32; i += 64 * kPackWaves) border[i] = a.tables.border[i];
+  __syncthreads();
+  if (row >= a.height) return;
+  const int words = plane_words(a.window);
+  uint32_t *nz_plane = pack_lds + kBorderLdsWords + wave * (pack_lds_per_wave(a.window) / 4);
+  uint32_t *mx_plane = nz_plane + words;
+  uint16_t *entry_at = reinterpret_cast<uint16_t *>(mx_plane + words);
+  const int64_t row_first = static_cast<int64_t>(row) * a.width;
+  const uint16_t *w = kWeights ? a.weights + row_first : nullptr;
+  int32_t *t = kWeights ? nullptr : a.symbols + row_first;
+
+  // the row's smallest and largest weight, and what finds them: bits sought, under a mask
+  uint32_t low = 0, high = 0, low_mask = 0, high_mask = 0;
+  if (kWeights) {
+    i16x2 least = {0x7fff, 0x7fff}, most = {-0x8000, -0x8000};
+    for (int c0 = 8 * lane; c0 - 8 * lane < a.width; c0 += 512 * kAhead) {
+      EightWeights v[kAhead] = {{w, c0, a.width}, {w, c0 + 512, a.width}, {w, c0 + 1024, a.width},
+                                {w, c0 + 1536, a.width}};
+#pragma unroll
+      for (int u = 0; u < kAhead; u++) {
+        if (c0 - 8 * lane + 512 * u >= a.width) break;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const i16x2 o = ordered(__builtin_bit_cast(i16x2, v[u].v[j]));
+          least = __builtin_elementwise_min(least, o);
+          most = __builtin_elementwise_max(most, o);
+        }
+      }
+    }
+    int l = min(least.x, least.y), h = max(most.x, most.y);
+    for (int m = 1; m < 64; m <<= 1) {
+      l = min(l, __shfl_xor(l, m, 64));
+      h = max(h, __shfl_xor(h, m, 64));
+    }
+    low = static_cast<uint16_t>(ordered_one(static_cast<int16_t>(l)));
+    high = static_cast<uint16_t>(ordered_one(static_cast<int16_t>(h)));
+    const bool nan = h > 0x7f80 || l < ordered_one(static_cast<int16_t>(0xff80));
+    if (nan) low = high = 0x7fc0;   // a NaN makes both NaN, and nothing equals one
+    if (lane == 0) a.minmax[row] = low | high << 16;
+    low_mask = low & 0x7fffu ? 0xffffffffu : 0x7fff7fffu;
+    high_mask = high & 0x7fffu ? 0xffffffffu : 0x7fff7fffu;
+    if (nan) low_mask = high_mask = 0;   // (x & 0) ^ 0x7fc0 is never zero
+    low = (low | low << 16) & (nan ? ~0u : low_mask);
+    high = (high | high << 16) & (nan ? ~0u : high_mask);
+  }
+
+  const int pairs = (a.width + 1) / 2;
+  int first = 0, out = 0;   // the window's first pair, the row's codes so far
+  while (first < pairs) {
+    const int here = min(pairs - first, a.window);   // pairs that may start an entry
+    const int col0 = 2 * first;
+    // eight symbols a lane to a byte of either plane, zeros past the row's end
+    const int bytes = min(4 * words, (a.width - col0 + 7) / 8 + 8);   // with zeros to look ahead into
+    for (int b0 = lane; b0 - lane < bytes; b0 += 64 * kAhead) {
+      using Loaded = std::conditional_t<kWeights, EightWeights, EightSymbols>;
+      const auto *src = row_source<kWeights>(w, t);
+      const int c0 = col0 + 8 * b0;
+      Loaded v[kAhead] = {{src, c0, a.width}, {src, c0 + 512, a.width}, {src, c0 + 1024, a.width},
+                          {src, c0 + 1536, a.width}};
+#pragma unroll
+      for (int u = 0; u < kAhead; u++) {
+        if (b0 - lane + 64 * u >= bytes) break;
+        uint32_t nz, mx;
+        if constexpr (kWeights) {
+          uint32_t not_mx[4], neither[4];
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            not_mx[j] = not_equal(v[u].v[j], high_mask, high);   // a row of one value: all 2
+            neither[j] = not_mx[j] & not_equal(v[u].v[j], low_mask, low);
+          }
+          nz = gather_bits(neither) ^ 0xffu;
+          mx = gather_bits(not_mx) ^ 0xffu;
+        } else {
+          uint32_t both = 0;
+#pragma unroll
+          for (int j = 0; j < 8; j++) both |= v[u].v[j] << (2 * j);
+          nz = even_bits(both | both >> 1);
+          mx = even_bits(both >> 1);
+        }
+        const int b = b0 + 64 * u;
+        if (b < bytes) {
+          const int at = col0 + 8 * b;
+          reinterpret_cast<uint8_t *>(nz_plane)[b] = static_cast<uint8_t>(eight_bits(nz, at, a.width));
+          reinterpret_cast<uint8_t *>(mx_plane)[b] = static_cast<uint8_t>(eight_bits(mx, at, a.width));
+        }
+      }
+    }
+    wave_lds_fence();
+    // The longest entry at every pair, a lane each, two runs of 64 at a time: up to
+    // the pair of the third non-zero, or up to that of the fourth as far as entries
+    // with three reach.  Then from entry to entry by scalar reads of the lengths.
+    int n = 0, at = 0;   // entries found, the pair after the last of them
+    for (int p0 = 0; p0 < here; p0 += 128) {
+      int len[2];
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const int p = min(p0 + 64 * u + lane, here - 1);
+        const uint32_t nz = plane_bits(nz_plane, 2 * p);
+        uint32_t rest = nz & (nz - 1);
+        rest &= rest - 1;                                                        // from the third non-zero on
+        const uint32_t end = 1u << kLookahead;
+        const int upto2 = __builtin_ctz(rest | end) >> 1;
+        const uint32_t rest3 = rest & (rest - 1);
+        const int upto3 = min(__builtin_ctz(rest3 | end) >> 1, kBorderPairs);
+        const int longest = min(max(upto2, upto3), pairs - first - p);
+        // for every lane, so that the two runs' LDS reads are in flight together: a
+        // string of other than three non-zeros looks up something within the table
+        const uint32_t three = (nz & ((1u << (2 * kBorderPairs)) - 1)) | 7u << (2 * kBorderPairs);
+        const int i = min(string_places(three, plane_bits(mx_plane, 2 * p), kFreeNonzeros + 1), kBorderStrings - 1);
+        const int entry = (border[i >> 5] >> (i & 31)) & 1u;
+        const bool at_border = upto3 == kBorderPairs && upto2 < kBorderPairs && longest == kBorderPairs;
+        len[u] = at_border ? kBorderPairs - 1 + entry : longest;
+      }
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const int limit = min(here - p0 - 64 * u, 64);
+        unsigned long long starts = 0;
+        int q = at - p0 - 64 * u;
+        while (q < limit) {
+          starts |= 1ull << q;
+          q += __builtin_amdgcn_readlane(len[u], q);
+        }
+        at = p0 + 64 * u + q;
+        if ((starts >> lane) & 1)
+          entry_at[n + __popcll(starts & ((1ull << lane) - 1))] = static_cast<uint16_t>(p0 + 64 * u + lane);
+        n += __popcll(starts);
+      }
+    }
+    wave_lds_fence();
+    for (int i0 = 0; i0 < n; i0 += 64 * kAhead) {
+      uint16_t code[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; u++) {
+        const int i = i0 + 64 * u + lane;
+        if (i < n) {
+          const int from = entry_at[i];
+          const int len = (i + 1 < n ? entry_at[i + 1] : at) - from;
+          const uint32_t mask = (1u << (2 * len)) - 1;
+          const uint32_t nz = plane_bits(nz_plane, 2 * from) & mask;
+          code[u] = a.tables.code[string_index(nz, plane_bits(mx_plane, 2 * from), len)];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; u++) {
+        const int i = i0 + 64 * u + lane;
+        if (i < n) {
+          if (kWeights)
+            a.codes[static_cast<int64_t>(row) * pairs + out + i] = code[u];
+          else
+            t[out + i] = code[u];   // at most as many as pairs taken: never ahead of what is still to be read
+        }
+      }
+    }
+    out += n;
+    first += at;
+    wave_lds_fence();
+  }
+  if (lane == 0) a.row_cnt[row + 1] = out;
+}
+
+// ---------------------------------------------------- a caller's own trie ---
+
+// *foreign, zero before, is set where trie is not the fixed dictionary's.
+__global__ __launch_bounds__(256) void compare_trie_kernel(const int32_t *__restrict__ trie,
+                                                           const int32_t *__restrict__ fixed,
+                                                           int32_t *foreign) {
+  const int i = 4 * (blockIdx.x * 256 + threadIdx.x);
+  int32_t v[4] = {0, 0, 0, 0}, f[4] = {0, 0, 0, 0};
+  if (i + 4 <= SUB1_TRIE_WORDS) {
+    __builtin_memcpy(v, trie + i, 16);
+    __builtin_memcpy(f, fixed + i, 16);
+  } else {
+    for (int j = 0; i + j < SUB1_TRIE_WORDS; j++) {
+      v[j] = trie[i + j];
+      f[j] = fixed[i + j];
+    }
+  }
+  if ((v[0] ^ f[0]) | (v[1] ^ f[1]) | (v[2] ^ f[2]) | (v[3] ^ f[3])) *foreign = 1;
+}
+
+constexpr int kTrieRoot = SUB1_DICT_ENTRIES;
+
+// A thread per row walks the trie, for a trie that is not the fixed one.
+__global__ void pack_count_kernel(const int32_t *__restrict__ trie, int32_t *__restrict__ w_tern,
+                                  int32_t *__restrict__ row_cnt, int height, int width) {
+  if (!row_cnt[0]) return;   // the fixed trie: pack_rows_kernel has packed the rows
+  int row = blockIdx.x * blockDim.x + threadIdx.x;
+  if (row >= height) return;
+  int32_t *w = w_tern + static_cast<int64_t>(row) * width;
+  int node = kTrieRoot;
+  int n = 0;
+  for (int i = 0; i < width; i += 2) {
+    int lo = w[i];
+    int hi = i + 1 < width ? w[i + 1] : 0;
+    int sym = 3 * hi + lo;
+    int child = trie[9 * node + sym];
+    if (child < 0) {
+      // n <= i/2 < i: the slot written was already consumed
+      w[n++] = node;
+      child = trie[9 * kTrieRoot + sym];
+    }
+    node = child;
+  }
+  w[n++] = node;
+  row_cnt[row + 1] = n;
+}
+
+__global__ void zero_word_kernel(int32_t *p) { *p = 0; }
+
+// ------------------------------------------------ offsets and compaction ----
+
+__global__ __launch_bounds__(sub1::kScanThreads) void row_offset_scan_kernel(int32_t *cnt, int height) {
+  sub1::scan_in_place(cnt, height);
+}
+
+// A wavefront per row, lanes stride over the row's codes.
+template <typename Code>
+__global__ __launch_bounds__(256) void pack_emit_kernel(const Code *__restrict__ codes,
+                                                        const int32_t *__restrict__ row_off,
+                                                        uint16_t *__restrict__ w_comp, int height,
+                                                        int stride) {
+  int row = blockIdx.x * 4 + threadIdx.x / 64;
+  if (row >= height) return;
+  int lane = threadIdx.x % 64;
+  int off = row_off[row];
+  int n = row_off[row + 1] - off;
+  const Code *src = codes + static_cast<int64_t>(row) * stride;
+  for (int i = lane; i < n; i += 64) w_comp[off + i] = static_cast<uint16_t>(src[i]);
+}
+
+int check_pack_shape(const char *who, int height, int width) {
+  if (height < 1 || width < 1) return fail(SUB1_ERR_SHAPE, "%s: height %d width %d", who, height, width);
+  // the cumulative count is kept in int32 like the reference's row_off
+  if (static_cast<int64_t>(height) * ((width + 1) / 2) > INT32_MAX)
+    return fail(SUB1_ERR_SHAPE, "%s: more than 2^31 pairs in one call", who);
+  return SUB1_OK;
+}
+
+template <bool kWeights>
+int launch_pack_rows(PackArgs &a, hipStream_t s) {
+  a.window = std::min((a.width + 1) / 2, kPackWindow);
+  pack_rows_kernel<kWeights><<<(a.height + kPackWaves - 1) / kPackWaves, 64 * kPackWaves,
+                               kBorderLdsWords * 4 + kPackWaves * pack_lds_per_wave(a.window), s>>>(a);
+  HIP_TRY(hipGetLastError());
+  return SUB1_OK;
+}
+
+}  // namespace
+
+extern "C" int sub1_pack_count(const int32_t *trie, int32_t *w_tern, int32_t *row_off,
+                               int height, int width, void *stream) {
+  if (!trie || !w_tern || !row_off) return fail(SUB1_ERR_NULL, "sub1_pack_count: NULL argument");
+  int rc = check_pack_shape("sub1_pack_count", height, width);
+  if (rc) return rc;
+  if (misaligned(trie, 4) || misaligned(w_tern, 4) || misaligned(row_off, 4))
+    return fail(SUB1_ERR_ALIGN, "sub1_pack_count: misaligned pointer");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  PackArgs a{};
+  rc = tables_of_current_device(&a.tables);
+  if (rc) return rc;
+  // row_off[0] is zero in the end; until then it says whose trie this is
+  zero_word_kernel<<<1, 1, 0, s>>>(row_off);
+  compare_trie_kernel<<<(SUB1_TRIE_WORDS / 4 + 256) / 256, 256, 0, s>>>(trie, a.tables.trie, row_off);
+  a.symbols = w_tern;
+  a.row_cnt = row_off;
+  a.foreign = row_off;
+  a.height = height;
+  a.width = width;
+  rc = launch_pack_rows<false>(a, s);
+  if (rc) return rc;
+  pack_count_kernel<<<(height + 63) / 64, 64, 0, s>>>(trie, w_tern, row_off, height, width);
+  row_offset_scan_kernel<<<1, sub1::kScanThreads, 0, s>>>(row_off, height);
+  HIP_TRY(hipGetLastError());
+  return SUB1_OK;
+}
+
+extern "C" int sub1_pack_emit(const int32_t *w_tern, const int32_t *row_off,
+                              int16_t *w_comp, int height, int width, void *stream) {
+  if (!w_tern || !row_off || !w_comp) return fail(SUB1_ERR_NULL, "sub1_pack_emit: NULL argument");
+  if (height < 1 || width < 1)
+    return fail(SUB1_ERR_SHAPE, "sub1_pack_emit: height %d width %d", height, width);
+  if (misaligned(w_tern, 4) || misaligned(row_off, 4) || misaligned(w_comp, 2))
+    return fail(SUB1_ERR_ALIGN, "sub1_pack_emit: misaligned pointer");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  pack_emit_kernel<<<(height + 3) / 4, 256, 0, s>>>(
+      w_tern, row_off, reinterpret_cast<uint16_t *>(w_comp), height, width);
+  HIP_TRY(hipGetLastError());
+  return SUB1_OK;
+}
+
+extern "C" int sub1_pack_weights_count(const void *w, uint16_t *codes, void *ter_minmax,
+                                       int32_t *row_off, int height, int width, void *stream) {
+  const char *who = "sub1_pack_weights_count";
+  if (!w || !codes || !ter_minmax || !row_off) return fail(SUB1_ERR_NULL, "%s: NULL argument", who);
+  int rc = check_pack_shape(who, height, width);
+  if (rc) return rc;
+  if (misaligned(w, 2) || misaligned(codes, 2) || misaligned(ter_minmax, 4) || misaligned(row_off, 4))
+    return fail(SUB1_ERR_ALIGN, "%s: misaligned pointer", who);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  PackArgs a{};
+  rc = tables_of_current_device(&a.tables);
+  if (rc) return rc;
+  a.weights = static_cast<const uint16_t *>(w);
+  a.codes = codes;
+  a.minmax = static_cast<uint32_t *>(ter_minmax);
+  a.row_cnt = row_off;
+  a.height = height;
+  a.width = width;
+  rc = launch_pack_rows<true>(a, s);
+  if (rc) return rc;
+  row_offset_scan_kernel<<<1, sub1::kScanThreads, 0, s>>>(row_off, height);
+  HIP_TRY(hipGetLastError());
+  return SUB1_OK;
+}
+
+extern "C" int sub1_pack_weights_emit(const uint16_t *codes, const int32_t *row_off, int16_t *w_comp,
+                                      int height, int width, void *stream) {
+  const char *who = "sub1_pack_weights_emit";
+  if (!codes || !row_off || !w_comp) return fail(SUB1_ERR_NULL, "%s: NULL argument", who);
+  if (height < 1 || width < 1) return fail(SUB1_ERR_SHAPE, "%s: height %d width %d", who, height, width);
+  if (misaligned(codes, 2) || misaligned(row_off, 4) || misaligned(w_comp, 2))
+    return fail(SUB1_ERR_ALIGN, "%s: misaligned pointer", who);
+  pack_emit_kernel<<<(height + 3) / 4, 256, 0, static_cast<hipStream_t>(stream)>>>(
+      codes, row_off, reinterpret_cast<uint16_t *>(w_comp), height, (width + 1) / 2);
+  HIP_TRY(hipGetLastError());
+  return SUB1_OK;
+}

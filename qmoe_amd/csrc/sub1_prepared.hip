@@ -421,29 +421,8 @@ __global__ __launch_bounds__(256) void check_source_kernel(const int32_t *__rest
   if (bad) atomicOr(found, bad);
 }
 
-// In-place inclusive prefix sum over v[1..n], v[0] = 0; one workgroup.
-__global__ __launch_bounds__(1024) void scan_counts_kernel(int32_t *__restrict__ v, int n) {
-  __shared__ int32_t part[1024];
-  const int tid = threadIdx.x;
-  const int seg = (n + 1023) / 1024;
-  const int lo = 1 + tid * seg;
-  const int hi = min(n + 1, lo + seg);
-  int32_t s = 0;
-  for (int i = lo; i < hi; i++) s += v[i];
-  part[tid] = s;
-  __syncthreads();
-  for (int d = 1; d < 1024; d *= 2) {
-    int32_t t = tid >= d ? part[tid - d] : 0;
-    __syncthreads();
-    part[tid] += t;
-    __syncthreads();
-  }
-  int32_t run = tid ? part[tid - 1] : 0;
-  if (tid == 0) v[0] = 0;
-  for (int i = lo; i < hi; i++) {
-    run += v[i];
-    v[i] = run;
-  }
+__global__ __launch_bounds__(sub1::kScanThreads) void scan_counts_kernel(int32_t *v, int n) {
+  sub1::scan_in_place(v, n);
 }
 
 // Position checkpoints.  For every slice and every group of kGroupChunks chunks,
@@ -2452,7 +2431,7 @@ int prepare_layout(const Source &src, void *meta, int64_t meta_bytes, LayoutResu
         k.slices, i);
     slice0 += static_cast<int64_t>(src.count) * k.slices;
   }
-  scan_counts_kernel<<<1, 1024, 0, s>>>(counts, static_cast<int>(slice0));
+  scan_counts_kernel<<<1, sub1::kScanThreads, 0, s>>>(counts, static_cast<int>(slice0));
   HIP_TRY(hipGetLastError());
   int32_t host[3] = {0, 0, 0};
   int32_t total = 0;

@@ -116,19 +116,11 @@ class Sub1Linear(nn.Module):
     def make(w):
         """Ternarise and pack a dense matrix whose rows take the values
         {row min, 0, row max} (reference sub1.py:145-166; ties go to max)."""
-        w = w.bfloat16()
-        ter_minmax = torch.column_stack((w.min(1)[0], w.max(1)[0])).flatten()
-        row_off = torch.zeros(w.shape[0] + 1, dtype=torch.int32, device=w.device)
-        w_tern = torch.zeros(w.shape, dtype=torch.int32, device=w.device)
-        w_tern[w == ter_minmax[0::2].reshape((-1, 1))] = 1
-        w_tern[w == ter_minmax[1::2].reshape((-1, 1))] = 2
-        _, table = device_tables(w.device)
-        w_comp = sub1_hip.sub1pack(table, w_tern, row_off)
-
-        linear = Sub1Linear(w.shape[0], w_comp.shape[0])
-        linear.w_comp.data = w_comp
-        linear.row_off.data = row_off
-        linear.ter_minmax = ter_minmax
+        if w.device.type != 'cuda' or not GPUS:
+            raise RuntimeError('the compressed-expert kernels need a GPU; got %s' % w.device)
+        linear = Sub1Linear(0, 0)
+        linear.w_comp, linear.row_off, linear.ter_minmax = sub1_hip.sub1pack_weights(
+            w.bfloat16().contiguous())
         return linear
 
 

@@ -161,6 +161,28 @@ def sub1pack(trie, w_tern, row_off):
     return w_comp
 
 
+def sub1pack_weights(w):
+    """(w_comp int16 [C], row_off int32 [H+1], ter_minmax bf16 [2H]) of dense
+    bf16 weights [H, W] whose rows take the values {row min, 0, row max}, by the
+    fixed dictionary: what sub1pack gives for their symbols (reference
+    sub1.py:145-159)."""
+    p_w = _need(w, torch.bfloat16, 'w', dim=2)
+    height, width = w.shape
+    dev = w.device
+    lib = _lib.load()
+    row_off = torch.empty(height + 1, dtype=torch.int32, device=dev)
+    minmax = torch.empty(2 * height, dtype=torch.bfloat16, device=dev)
+    codes = torch.empty((height, (width + 1) // 2), dtype=torch.int16, device=dev)
+    with _on_device(dev):
+        _lib.check(lib.sub1_pack_weights_count(p_w, codes.data_ptr(), minmax.data_ptr(),
+                                               row_off.data_ptr(), height, width, _stream()))
+        total = int(row_off[height].item())      # the one host sync, as in the reference
+        w_comp = torch.empty(total, dtype=torch.int16, device=dev)
+        _lib.check(lib.sub1_pack_weights_emit(codes.data_ptr(), row_off.data_ptr(), w_comp.data_ptr(),
+                                              height, width, _stream()))
+    return w_comp, row_off, minmax
+
+
 def sub1decode(dec, w_comp, row_off, ter_minmax, width, want_tern=True, want_w=True):
     """Decode without multiplying: (symbols uint8 [H, W] or None, weights bf16
     [H, W] or None, number of rows whose codes do not cover the width)."""

@@ -1,4 +1,4 @@
-"""Preparing, packing and expanding at the sizes where their kernels change
+"""Preparing and packing at the sizes where their kernels change
 hands: a row more or less than a wavefront, than a workgroup's turn, row
 lengths that are all alike or that fill more bins than a workgroup has threads.
 The symbols a form was made from are the reference: they come back whole."""
@@ -83,3 +83,69 @@ def test_preparing_names_a_bad_pointer(gpu):
         assert lib.sub1_moe_prepare_layout_from_layers(ctypes.byref(layers), meta.data_ptr(), meta.numel(),
                                                        ctypes.byref(out), stream) == status
         assert words in lib.sub1_last_error().decode()
+
+
+def symbols_by_torch(w):
+    """The rule of reference sub1.py:146-155 in torch: (symbols, ter_minmax)."""
+    minmax = torch.column_stack((w.min(1)[0], w.max(1)[0])).flatten()
+    symbols = torch.zeros(w.shape, dtype=torch.uint8, device=w.device)
+    symbols[w == minmax[0::2].reshape(-1, 1)] = 1
+    symbols[w == minmax[1::2].reshape(-1, 1)] = 2
+    return symbols, minmax
+
+
+@pytest.mark.parametrize('height,width,share', [
+    (5, 1, 0.5), (3, 2, 1.0), (9, 27, 0.1), (9, 29, 0.1),          # shorter than an entry, one symbol more
+    (70, 127, 0.15), (66, 513, 0.02), (64, 1040, 0.35),            # bytes of a plane, a lane's turn
+    (6, 8191, 0.1), (6, 8194, 0.1), (3, 16400, 0.12)])             # one window of a row, two, three
+def test_weights_pack_like_their_symbols(gpu, oracle, height, width, share):
+    sub1, op = gpu
+    symbols = symbols_of(height, width, [share, share / 3, 0.0, 0.7], seed=height * width)
+    scale = torch.rand(height, 1, generator=torch.Generator().manual_seed(2)).cuda() + 0.5
+    w = (torch.tensor([0.0, -1.0, 1.0], device='cuda')[symbols.long()] * scale).bfloat16()
+    if height > 8:   # rows of one value, of zeros of both signs, with an infinity, with a NaN
+        w[0], w[1], w[2, 0], w[3, -1] = 0.25, -0.0, float('inf'), float('nan')
+        w[4], w[4, ::2] = 0.0, 3.0
+    want, minmax = symbols_by_torch(w)
+    before = w.clone()
+    w_comp, row_off, got_minmax = op.sub1pack_weights(w)
+    assert torch.equal(w.view(torch.int16), before.view(torch.int16))
+    assert torch.equal(torch.nan_to_num(got_minmax.float()), torch.nan_to_num(minmax.float()))
+    codes, offsets = oracle.encode(want.cpu().numpy())
+    assert (row_off.cpu().numpy() == offsets).all()
+    assert (w_comp.cpu().numpy().view('uint16') == codes).all()
+    # and from the symbols themselves
+    p_comp, p_off = packed(gpu, want)
+    assert torch.equal(p_comp, w_comp) and torch.equal(p_off, row_off)
+
+
+def test_packing_with_a_trie_of_ones_own(gpu):
+    """A trie that is not the fixed dictionary's (here: cut off below three
+    pairs, and with the symbols' order of a few entries changed) is walked as it
+    is."""
+    sub1, op = gpu
+    trie = sub1.trie.clone()
+    depth3 = set()
+    level = [int(c) for c in trie[65536]]
+    for _ in range(2):
+        level = [int(c) for n in level for c in trie[n] if c >= 0]
+    depth3.update(level)
+    trie[sorted(depth3)] = -1
+    trie[65536, 1], trie[65536, 2] = trie[65536, 2].clone(), trie[65536, 1].clone()
+    symbols = symbols_of(70, 201, [0.1, 0.5, 0.0], seed=11)
+    row_off = torch.zeros(71, dtype=torch.int32, device='cuda')
+    w_comp = op.sub1pack(trie.cuda(), symbols.to(torch.int32), row_off)
+    want, offsets = [], [0]
+    for row in symbols.cpu().tolist():
+        row.append(0)
+        node = 65536
+        for i in range(0, 201, 2):
+            child = int(trie[node, row[i] + 3 * row[i + 1]])
+            if child < 0:
+                want.append(node)
+                child = int(trie[65536, row[i] + 3 * row[i + 1]])
+            node = child
+        want.append(node)
+        offsets.append(len(want))
+    assert row_off.tolist() == offsets
+    assert w_comp.cpu().numpy().view('uint16').tolist() == want
