@@ -15,6 +15,7 @@
 //   sub1.py:306-321              expert loop      -> moe_kernel
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdarg>
 #include <cstdio>
@@ -105,12 +106,10 @@ using sub1::row_result;
 // of which at most three are non-zero.  The kernels use a derived one-word
 // form that lists the non-zeros:
 //   bits 0-3          pair count L (the entry spans 2L weights)
-//   bits 4+7j..10+7j  slot j = 3*pos + sym  (pos 0..27, sym 1 = row min,
-//                     2 = row max), 0 = no further non-zero
-// 3*pos+sym is directly an offset into the tripled activation array below.
+//   bits 4+7j..8+7j   slot j: the non-zero's place in the entry (0..27)
+//   bit 9+7j, 10+7j   set where it is the row min, the row max (neither: no slot j)
 constexpr int kSlots = 3;
 constexpr int kSlotBits = 7;
-constexpr uint32_t kSlotMask = (1u << kSlotBits) - 1;
 
 __global__ void derive_slot_table_kernel(const int32_t *__restrict__ dec,
                                          uint32_t *__restrict__ tab,
@@ -130,7 +129,7 @@ __global__ void derive_slot_table_kernel(const int32_t *__restrict__ dec,
       bad = true;
       break;
     }
-    out |= static_cast<uint32_t>(3 * d + t) << (4 + kSlotBits * n);
+    out |= static_cast<uint32_t>(d | (t << 5)) << (4 + kSlotBits * n);
     n++;
   }
   tab[e] = out;
@@ -160,115 +159,42 @@ __device__ __forceinline__ void compare_print(const int32_t *__restrict__ dec,
 
 // ----------------------------------------------- activations in LDS --------
 //
-// x is kept in LDS as fp32, tripled:  M[3k] = 0, M[3k+1] = x[k], M[3k+2] = 0.
-// Reading the pair (M[i], M[i-1]) at i = 3k+sym gives (x,0) for sym 1, (0,x)
-// for sym 2 and (0,0) for an empty slot (i = 3k), so a slot costs two adds and
-// no select; the pair is one ds_read2_b32.  One spare dword in front makes
-// M[-1] readable, and 28 zero columns behind the row cover the digits of a
-// last codeword that hang over the row end (the reference pads the same way,
-// sub1_cuda_kernel.cu:147-151).
-__host__ __device__ constexpr int lds_dwords_for_width(int width) {
-  return 1 + 3 * (width + 28) + 3;
-}
+// x is kept in LDS as fp32, with zeros behind the row for the digits of a last
+// codeword that hang over its end (the reference pads the same way,
+// sub1_cuda_kernel.cu:147-151) and for lanes that have no codeword left.
+__host__ __device__ constexpr int lds_dwords_for_width(int width) { return (width + 32 + 3) / 4 * 4; }
 
 template <int kThreads>
-__device__ __forceinline__ void stage_activations(float *lds, const uint16_t *x,
-                                                  int width) {
-  const int n = width + 29;
-  if (threadIdx.x == 0) lds[0] = 0.f;
-  for (int k = threadIdx.x; k < n; k += kThreads) {
-    float v = k < width ? bf16_to_f32(x[k]) : 0.f;
-    float *m = lds + 1 + 3 * k;
-    m[0] = 0.f;
-    m[1] = v;
-    m[2] = 0.f;
+__device__ __forceinline__ void stage_activations(float *lds, const uint16_t *x, int width) {
+  const int n = lds_dwords_for_width(width);
+  for (int k = 4 * threadIdx.x; k < n; k += 4 * kThreads) {
+    uint16_t v[4] = {0, 0, 0, 0};
+    if (k + 4 <= width) {
+      __builtin_memcpy(v, x + k, 8);
+    } else {
+      for (int j = 0; j < 4 && k + j < width; j++) v[j] = x[k + j];
+    }
+    *reinterpret_cast<float4 *>(lds + k) =
+        make_float4(bf16_to_f32(v[0]), bf16_to_f32(v[1]), bf16_to_f32(v[2]), bf16_to_f32(v[3]));
   }
 }
 
-// One codeword: three slots, then advance the column (in dwords of M).
-__device__ __forceinline__ void add_codeword(uint32_t e, const float *M, int &colw,
-                                             float &s1, float &s2) {
-#pragma unroll
-  for (int j = 0; j < kSlots; j++) {
-    int idx = colw + static_cast<int>((e >> (4 + kSlotBits * j)) & kSlotMask);
-    s1 += M[idx];
-    s2 += M[idx - 1];
-  }
-  colw += static_cast<int>(e & 0xfu) * 6;
-}
-
-__device__ __forceinline__ void load_codes8(const uint16_t *p, uint32_t (&w)[4]) {
-  // the stream is only 2-byte aligned; gfx950 global loads take any alignment
-  __builtin_memcpy(w, p, 16);
-}
-
-// Sum of activations under the symbol-1 and symbol-2 weights of one row, in
-// fp32, in the library's canonical order: the row's codes in groups of 32, a
-// partial sum per group taken left to right from zero, the partial sums added
-// first group first.  (The grouping lets the prepared kernels split a row
-// between wavefronts without changing a bit of the result.)
 // The table word of a code: from the copy of the table's first `held` words in
 // LDS where the code lies in it, from the table in global memory otherwise.  A
 // gather from the 256 KB table costs a compute unit about 54 ns per wavefront
 // instruction (every lane fetches a cache line of its own through the L1), one
 // from LDS 3 ns, and the low codes are the frequent ones: the first 21 500
-// entries take 64% of the codes of weights with 90% zeros.
-struct TableView {
-  const uint32_t *tab;
-  const uint32_t *held_words;
-  uint32_t held;
-  __device__ __forceinline__ uint32_t operator[](uint32_t code) const {
-    return code < held ? held_words[code] : tab[code];
-  }
-};
-
-__device__ __forceinline__ void row_sums(const TableView tab,
-                                         const uint16_t *__restrict__ codes, int len,
-                                         const float *M, float &s1, float &s2) {
-  s1 = 0.f;
-  s2 = 0.f;
-  float p1 = 0.f, p2 = 0.f;
-  int colw = 0;
-  int i = 0;
-  uint32_t w[4];
-  if (len >= 8) load_codes8(codes, w);
-  for (; i + 8 <= len; i += 8) {
-    uint32_t cur[4] = {w[0], w[1], w[2], w[3]};
-    if (i + 16 <= len) load_codes8(codes + i + 8, w);
-    uint32_t e[8];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      e[2 * j] = tab[cur[j] & 0xffffu];
-      e[2 * j + 1] = tab[cur[j] >> 16];
-    }
-#pragma unroll
-    for (int j = 0; j < 8; j++) add_codeword(e[j], M, colw, p1, p2);
-    if (((i + 8) & 31) == 0) {   // a group of 32 codes is complete
-      s1 += p1;
-      s2 += p2;
-      p1 = 0.f;
-      p2 = 0.f;
-    }
-  }
-  int rem = len - i;
-  if (rem > 0) {
-    if (len >= 8) {
-      // the row's last eight codes; the first 8-rem of them are already done
-      load_codes8(codes + len - 8, w);
-      int skip = 8 - rem;
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        uint32_t code = (j & 1) ? (w[j / 2] >> 16) : (w[j / 2] & 0xffffu);
-        uint32_t e = tab[code];
-        if (j < skip) e = 0u;  // entry 0 of the slot form: nothing, no advance
-        add_codeword(e, M, colw, p1, p2);
-      }
-    } else {
-      for (int j = 0; j < rem; j++) add_codeword(tab[codes[j]], M, colw, p1, p2);
-    }
-  }
-  s1 += p1;   // the last, possibly partial, group (adds +0 if it was just folded)
-  s2 += p2;
+// entries take 64% of the codes of weights with 90% zeros.  Lanes whose code is
+// held all read the table's first word, one line, so that the two reads need no
+// branch and every lane's are in flight together.
+template <bool kHeld>
+__device__ __forceinline__ uint32_t table_word(const uint32_t *__restrict__ tab,
+                                               const uint32_t *held_words, uint32_t held,
+                                               uint32_t code) {
+  if (!kHeld) return tab[code];
+  const uint32_t far = tab[code < held ? 0u : code];
+  const uint32_t near = held_words[min(code, held - 1)];
+  return code < held ? near : far;
 }
 
 // ------------------------------------------------------------- matvec ------
@@ -434,12 +360,29 @@ __global__ void decode_kernel(const int32_t *__restrict__ dec,
 
 // ------------------------------------------------------ grouped experts ----
 //
-// Persistent grid.  Work is cut into tiles (token, projection, block of
-// kThreads rows), numbered with all wi tiles before all wo tiles, and handed
-// out by an atomic ticket.  A wo tile of token t needs all of h[t], so it
-// waits until the wi tiles of t have signalled; those have smaller tickets,
-// were therefore taken by workgroups that are already running, and never wait
-// themselves, so the wait always ends.
+// Persistent grid.  Work is cut into tiles (token, projection, part of its rows),
+// numbered with all wi tiles before all wo tiles, and handed out by an atomic
+// ticket.  A wo tile of token t needs all of h[t], so it waits until the wi tiles
+// of t have signalled; those have smaller tickets, were therefore taken by
+// workgroups that are already running, and never wait themselves, so the wait
+// always ends.
+//
+// Within a tile the wavefronts take runs of rows from a counter in LDS and give a
+// LANE to a GROUP of 32 codes, not to a row: a row's sum is the sum of its groups'
+// sums in order (the library's canonical order on this layout), so groups are
+// what can be worked on side by side.  Rows differ in length by a factor of 20 where
+// their shares of zeros differ, and a wavefront of rows takes as long as the
+// longest of them; a wavefront of groups takes 32 codes.  A lane reads its codes in
+// four 16-byte loads, next to its neighbours', fetches all their table words at
+// once, and from the words' lengths a prefix sum over the lanes gives the column at
+// which each group starts.
+//
+// What bounds it: LDS gathers of activations (three a codeword, 8 ns a wavefront and
+// compute unit), the words outside the held head of the table (54 ns times the share
+// of lanes that miss), 27 vector instructions a codeword (11 ns).  A wavefront's 64
+// codewords take 16-20 ns.  Switch shapes with shares of zeros between 75 and 98 %,
+// 64 tokens, us: base 381 -> 74, large 526 -> 105, c-2048 956 -> 230, where the lane per
+// row waited for the longest of 64; with 90 % everywhere 99 -> 51, 109 -> 61, 255 -> 133.
 struct MoeArgs {
   const uint32_t *tab;
   const uint16_t *w_comp;
@@ -456,7 +399,6 @@ struct MoeArgs {
   int32_t *ctrl;  // the control words (sub1_common.h): ticket, fault counts, a word per token
   int tokens, d_model, d_ff, experts;
   int wi_tiles, wo_tiles;  // per token
-  int tile_rows;           // rows of a tile: the workgroup's threads (a row each) or more (rows in turn)
   int act_dwords;          // LDS dwords of the activations; the table's first words follow
   int held;                // words of the table kept in LDS (0: none)
   int wi_expect;           // wi tiles a wo tile waits for (wi_tiles outside tests)
@@ -468,17 +410,186 @@ struct MoeArgs {
 
 using sub1::kCtrlHeader;
 
+constexpr int kGroupCodes = 32;   // codes per partial sum: part of the results' definition
+constexpr int kGroupStep = 30;    // what a turn of 64 groups takes, in steps of a lane with a row of its own
+
+// Table words of a lane's group: `count` codes from `codes` on, of a row that
+// ends at codes + count at the earliest eight codes after it began (`whole`), or of
+// a shorter row; zero words (nothing, no advance) make up the rest.
+template <bool kHeld>
+__device__ __forceinline__ void group_words(const uint32_t *__restrict__ tab, const uint32_t *held_words,
+                                            uint32_t held, const uint16_t *codes, int count, bool whole,
+                                            uint32_t (&e)[kGroupCodes]) {
+  uint32_t w[kGroupCodes / 8][4];
+  int skip[kGroupCodes / 8];   // codes of an eight that are not the group's: the first ones
+#pragma unroll
+  for (int k = 0; k < kGroupCodes / 8; k++) {
+    // a partial eight, and one behind the group's end, is read from eight codes
+    // before that end (lanes without a group: from where they stand)
+    const int left = min(max(count - 8 * k, 0), 8);
+    skip[k] = whole ? 8 - left : 8;
+    const uint16_t *from = codes + (left > 0 ? 8 * k - (8 - left) : count > 0 ? count - 8 : 0);
+    if (whole) {
+      __builtin_memcpy(w[k], from, 16);   // any alignment
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++) w[k][j] = 0;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kGroupCodes; i++) {
+    const uint32_t code = (i & 1) ? w[i / 8][(i & 7) / 2] >> 16 : w[i / 8][(i & 7) / 2] & 0xffffu;
+    const uint32_t word = table_word<kHeld>(tab, held_words, held, code);
+    e[i] = (i & 7) < skip[i / 8] ? 0u : word;
+  }
+  if (!whole)   // rows of up to seven codes
+#pragma unroll
+    for (int i = 0; i < 7; i++)
+      if (i < count) e[i] = table_word<kHeld>(tab, held_words, held, codes[i]);
+}
+
+// The activations under a codeword's weights onto the sums of either symbol, left
+// to right; `at`, the column at which it starts, moves on.
+__device__ __forceinline__ void add_codeword(uint32_t e, const float *X, int &at, float &p1, float &p2) {
+#pragma unroll
+  for (int j = 0; j < kSlots; j++) {
+    const uint32_t slot = e >> (4 + kSlotBits * j);
+    const uint32_t xv = __float_as_uint(X[at + static_cast<int>(slot & 31u)]);
+    const uint32_t is1 = static_cast<uint32_t>(static_cast<int32_t>(slot << 26) >> 31);
+    const uint32_t is2 = static_cast<uint32_t>(static_cast<int32_t>(slot << 25) >> 31);
+    p1 += __uint_as_float(xv & is1);
+    p2 += __uint_as_float(xv & is2);
+  }
+  at += 2 * static_cast<int>(e & 15u);
+}
+
+// A lane's row from its first code to its last: the sums of its groups, first
+// group first.
+template <bool kHeld>
+__device__ __forceinline__ void row_by_lane(const uint32_t *__restrict__ tab, const uint32_t *held_words,
+                                            uint32_t held, const uint16_t *codes, int len,
+                                            const float *X, float &s1, float &s2) {
+  s1 = s2 = 0.f;
+  float p1 = 0.f, p2 = 0.f;
+  int at = 0;
+  uint32_t next[4];
+  if (len >= 8) __builtin_memcpy(next, codes, 16);
+  for (int i = 0; i < len; i += 8) {
+    const uint32_t w[4] = {next[0], next[1], next[2], next[3]};
+    // the row's last, partial eight is read from eight codes before its end
+    const int ahead = min(i + 8, max(len - 8, 0));
+    if (i + 8 < len) __builtin_memcpy(next, codes + ahead, 16);
+    const int skip = len >= 8 ? max(i + 8 - len, 0) : 8;
+    uint32_t e[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const uint32_t code = (j & 1) ? w[j / 2] >> 16 : w[j / 2] & 0xffffu;
+      e[j] = table_word<kHeld>(tab, held_words, held, code);
+      if (j < skip) e[j] = 0u;
+    }
+    if (len < 8)   // a row of up to seven codes
+      for (int j = 0; j < len; j++) add_codeword(table_word<kHeld>(tab, held_words, held, codes[j]), X, at, p1, p2);
+#pragma unroll
+    for (int j = 0; j < 8; j++) add_codeword(e[j], X, at, p1, p2);
+    if (((i + 8) & (kGroupCodes - 1)) == 0) {   // a group is complete
+      s1 += p1;
+      s2 += p2;
+      p1 = p2 = 0.f;
+    }
+  }
+  s1 += p1;   // the last, possibly partial, group (adds +0 if it was just folded)
+  s2 += p2;
+}
+
+// Rows row0 .. row0 + rows - 1 of one matrix (rows <= 64, a wavefront): lane r
+// receives the sums of row row0 + r.  `partial` is the wavefront's own LDS, 64 pairs.
+template <bool kHeld>
+__device__ __forceinline__ void rows_by_groups(const uint32_t *__restrict__ tab, const uint32_t *held_words,
+                                               uint32_t held, const uint16_t *__restrict__ codes,
+                                               const int32_t *__restrict__ row_off, int row0, int rows,
+                                               const float *X, float2 *partial, float &s1, float &s2) {
+  const int lane = threadIdx.x & 63;
+  const bool mine = lane < rows;
+  const int off = mine ? row_off[row0 + lane] : 0;
+  const int len = mine ? row_off[row0 + lane + 1] - off : 0;
+  const int groups = (max(len, 0) + kGroupCodes - 1) / kGroupCodes;
+  const int last = wave_prefix_sum(groups), first = last - groups;   // the row's groups, among the run's
+  const int total = __builtin_amdgcn_readlane(last, 63);
+  // A lane to a row instead where the rows are alike and there are enough of them: it
+  // then takes as many steps as the longest has codes, and no prefix sums.  (256
+  // tokens, us: groups always 125 base, 163 large, 428 c-2048; rows always 103, 163,
+  // 483, and 685, 960, 2176 where the shares of zeros differ from row to row; by this
+  // rule 98, 149, 416, and 165, 263, 651.)
+  int longest = len;
+  for (int m = 1; m < 64; m <<= 1) longest = max(longest, __shfl_xor(longest, m, 64));
+  if ((longest + 7) / 8 * 8 <= (total + 63) / 64 * kGroupStep) {
+    row_by_lane<kHeld>(tab, held_words, held, codes + off, len, X, s1, s2);
+    return;
+  }
+  s1 = 0.f;
+  s2 = 0.f;
+  int carry = 0;   // the column reached in a row that goes on from the turn before
+  for (int turn = 0; turn < total; turn += 64) {
+    // the row of this lane's group: the first whose groups end behind it
+    const int g = min(turn + lane, total - 1);
+    int r = 0;
+#pragma unroll
+    for (int step = 32; step >= 1; step >>= 1)
+      if (__shfl(last, r + step - 1, 64) <= g) r += step;
+    const int r_first = __shfl(first, r, 64);
+    const int r_off = __shfl(off, r, 64), r_len = __shfl(len, r, 64);
+    const bool active = turn + lane < total;
+    const int in_row = active ? kGroupCodes * (g - r_first) : 0;
+    const int count = active ? min(r_len - in_row, kGroupCodes) : 0;
+    uint32_t e[kGroupCodes];
+    group_words<kHeld>(tab, held_words, held, codes + r_off + in_row, count, r_len >= 8, e);
+    int span = 0;
+#pragma unroll
+    for (int i = 0; i < kGroupCodes; i++) span += static_cast<int>(e[i] & 15u);
+    span *= 2;
+    const int before = wave_prefix_sum(span) - span;
+    const int row_before = __shfl(before, max(r_first - turn, 0), 64);
+    const int at = before - row_before + (r_first < turn ? carry : 0);
+    carry = __builtin_amdgcn_readlane(at + span, 63);
+    float2 p = {0.f, 0.f};
+    int col = at;
+#pragma unroll
+    for (int i = 0; i < kGroupCodes; i++) add_codeword(e[i], X, col, p.x, p.y);
+    partial[lane] = p;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (int i = max(first - turn, 0); i < min(last - turn, 64); i++) {
+      const float2 q = partial[i];
+      s1 += q.x;
+      s2 += q.y;
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// Rows that a wavefront takes at a time: a lane each where a tile has that many
+// for all its wavefronts, but at least about 64 groups of them (a row of W weights
+// with 90% zeros has W / 23 codes).
+__device__ __forceinline__ int rows_at_a_time(int rows, int width, int waves) {
+  return min(max(max(rows / waves, 64 * 640 / (width + 640)), 1), 64);
+}
+
 template <int kThreads>
-__global__ __launch_bounds__(kThreads) void moe_kernel(MoeArgs a) {
-  extern __shared__ float lds[];
-  __shared__ int s_ticket;
+__global__ __launch_bounds__(kThreads, 4) void moe_kernel(MoeArgs a) {
+  constexpr bool kHeld = kThreads == 1024;   // the form with the table's head in LDS
+  extern __shared__ __align__(16) float lds[];
+  __shared__ int s_ticket, s_row;
+  __shared__ float2 s_partial[kThreads];
   const int n_wi = a.tokens * a.wi_tiles;
   const int n_all = n_wi + a.tokens * a.wo_tiles;
   if (blockIdx.x == 0) compare_print(a.dec, a.print, a.sticky);
   // the table's first words into LDS, once per workgroup (a persistent grid)
   uint32_t *held_words = reinterpret_cast<uint32_t *>(lds + a.act_dwords);
-  for (int i = threadIdx.x; i < a.held; i += kThreads) held_words[i] = a.tab[i];
-  const TableView table{a.tab, held_words, static_cast<uint32_t>(a.held)};
+  if (kHeld)
+    for (int i = 4 * threadIdx.x; i < a.held; i += 4 * kThreads)
+      *reinterpret_cast<uint4 *>(held_words + i) = *reinterpret_cast<const uint4 *>(a.tab + i);
+  float2 *partial = s_partial + (threadIdx.x & ~63u);
   for (;;) {
     __syncthreads();  // previous tile's readers of lds and s_ticket are done
     if (threadIdx.x == 0)
@@ -488,77 +599,75 @@ __global__ __launch_bounds__(kThreads) void moe_kernel(MoeArgs a) {
     const int ticket = s_ticket;
     if (ticket >= n_all) break;
 
-    if (ticket < n_wi) {
-      const int t = ticket / a.wi_tiles;
-      const int blk = ticket - t * a.wi_tiles;
-      int e = a.token_expert[t];
-      if (e >= a.experts) e = -1;
-      if (e >= 0) {
-        stage_activations<kThreads>(lds, a.x + static_cast<int64_t>(t) * a.d_model,
-                                    a.d_model);
-        __syncthreads();
-        const int row_end = min(a.d_ff, (blk + 1) * a.tile_rows);
-        for (int row = blk * a.tile_rows + threadIdx.x; row < row_end; row += kThreads) {
-          const int32_t *ro = a.wi_row_off + static_cast<int64_t>(e) * (a.d_ff + 1);
-          const int off = ro[row];
-          const int len = ro[row + 1] - off;
-          float s1, s2;
-          row_sums(table, a.w_comp + a.wi_code_base[e] + off, len, lds + 1, s1, s2);
-          float res = row_result(
-              a.wi_minmax[static_cast<int64_t>(e) * a.d_ff + row], s1, s2);
-          uint16_t hb = f32_to_bf16(res);
-          if (hb & 0x8000u) hb = 0;  // relu
+    const bool is_wi = ticket < n_wi;
+    const int j = is_wi ? ticket : ticket - n_wi;
+    const int tiles = is_wi ? a.wi_tiles : a.wo_tiles;
+    const int t = j / tiles, part = j - t * tiles;
+    const int height = is_wi ? a.d_ff : a.d_model, width = is_wi ? a.d_model : a.d_ff;
+    const int row_begin = static_cast<int>(static_cast<int64_t>(height) * part / tiles);
+    const int row_end = static_cast<int>(static_cast<int64_t>(height) * (part + 1) / tiles);
+    int e = a.token_expert[t];
+    if (e >= a.experts) {
+      if (!is_wi && part == 0 && threadIdx.x == 0)
+        __hip_atomic_fetch_add(&a.ctrl[sub1::kCtrlBadIds], 1, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+      e = -1;
+    }
+    if (e < 0) {
+      if (!is_wi)
+        for (int row = row_begin + threadIdx.x; row < row_end; row += kThreads) {
+          const int64_t i = static_cast<int64_t>(t) * a.d_model + row;
+          a.y[i] = a.x[i];
+        }
+      continue;   // a dropped token's word stays untouched
+    }
+    if (threadIdx.x == 0) {
+      s_row = row_begin;
+      if (!is_wi)
+        sub1::bounded_wait(&a.ctrl[sub1::token_word(t)], a.wi_expect, a.wait_ticks, a.sticky,
+                           &a.ctrl[sub1::kCtrlGaveUp]);
+    }
+    __syncthreads();  // thread 0's acquire covers the whole workgroup
+    stage_activations<kThreads>(lds, (is_wi ? a.x : a.h) + static_cast<int64_t>(t) * width, width);
+    __syncthreads();
+    const int32_t *row_off = (is_wi ? a.wi_row_off : a.wo_row_off) + static_cast<int64_t>(e) * (height + 1);
+    const uint16_t *codes = a.w_comp + (is_wi ? a.wi_code_base : a.wo_code_base)[e];
+    const uint32_t *minmax = (is_wi ? a.wi_minmax : a.wo_minmax) + static_cast<int64_t>(e) * height;
+    const int at_a_time = rows_at_a_time(row_end - row_begin, width, kThreads / 64);
+    for (;;) {
+      int row0 = 0;
+      if ((threadIdx.x & 63) == 0) row0 = atomicAdd(&s_row, at_a_time);
+      row0 = __builtin_amdgcn_readfirstlane(row0);
+      if (row0 >= row_end) break;
+      const int rows = min(at_a_time, row_end - row0);
+      const int row = row0 + (threadIdx.x & 63);
+      float s1, s2;
+      rows_by_groups<kHeld>(a.tab, held_words, a.held, codes, row_off, row0, rows, lds, partial, s1, s2);
+      if ((threadIdx.x & 63) < rows) {
+        uint16_t b = f32_to_bf16(row_result(minmax[row], s1, s2));
+        if (is_wi) {
+          if (b & 0x8000u) b = 0;  // relu
           // stored at agent scope: written through this die's L2, where the
           // workgroups on other dies will read it
-          __hip_atomic_store(&a.h[static_cast<int64_t>(t) * a.d_ff + row], hb, __ATOMIC_RELAXED,
+          __hip_atomic_store(&a.h[static_cast<int64_t>(t) * a.d_ff + row], b, __ATOMIC_RELAXED,
                              __HIP_MEMORY_SCOPE_AGENT);
+        } else {
+          a.y[static_cast<int64_t>(t) * a.d_model + row] = b;
         }
       }
+    }
+    if (is_wi) {
       // every wavefront waits for its h stores to be acknowledged, then the
       // barrier, then thread 0 counts the tile (a release fence here would write
       // back the whole L2)
       sub1::drain_stores();
       __syncthreads();
-      if (threadIdx.x == 0 && e >= 0)   // a dropped token's word stays untouched
+      if (threadIdx.x == 0)
         __hip_atomic_fetch_add(&a.ctrl[sub1::token_word(t)], 1, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
-    } else {
-      const int j = ticket - n_wi;
-      const int t = j / a.wo_tiles;
-      const int blk = j - t * a.wo_tiles;
-      int e = a.token_expert[t];
-      if (e >= a.experts) {
-        if (blk == 0 && threadIdx.x == 0)
-          __hip_atomic_fetch_add(&a.ctrl[sub1::kCtrlBadIds], 1, __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT);
-        e = -1;
-      }
-      const int row_end = min(a.d_model, (blk + 1) * a.tile_rows);
-      if (e < 0) {
-        for (int row = blk * a.tile_rows + threadIdx.x; row < row_end; row += kThreads) {
-          int64_t i = static_cast<int64_t>(t) * a.d_model + row;
-          a.y[i] = a.x[i];
-        }
-        continue;
-      }
-      if (threadIdx.x == 0)
-        sub1::bounded_wait(&a.ctrl[sub1::token_word(t)], a.wi_expect, a.wait_ticks, a.sticky,
-                           &a.ctrl[sub1::kCtrlGaveUp]);
-      __syncthreads();  // thread 0's acquire now covers the whole workgroup
-      stage_activations<kThreads>(lds, a.h + static_cast<int64_t>(t) * a.d_ff, a.d_ff);
-      __syncthreads();
-      for (int row = blk * a.tile_rows + threadIdx.x; row < row_end; row += kThreads) {
-        const int32_t *ro = a.wo_row_off + static_cast<int64_t>(e) * (a.d_model + 1);
-        const int off = ro[row];
-        const int len = ro[row + 1] - off;
-        float s1, s2;
-        row_sums(table, a.w_comp + a.wo_code_base[e] + off, len, lds + 1, s1, s2);
-        float res = row_result(
-            a.wo_minmax[static_cast<int64_t>(e) * a.d_model + row], s1, s2);
-        a.y[static_cast<int64_t>(t) * a.d_model + row] = f32_to_bf16(res);
-      }
+    } else if (threadIdx.x == 0) {
       // said once the tile's work is done: it takes a round trip to memory
-      if (threadIdx.x == 0) sub1::waited_on(&a.ctrl[sub1::token_word(t)], a.wo_tiles);
+      sub1::waited_on(&a.ctrl[sub1::token_word(t)], a.wo_tiles);
     }
   }
   if (threadIdx.x == 0) sub1::leave_launch(a.ctrl, gridDim.x);
@@ -638,7 +747,6 @@ int slot_table_for(const int32_t *dec, hipStream_t stream, TableSlot *out, int32
   return SUB1_OK;
 }
 
-constexpr int kMatvecThreads = 256;
 constexpr int kMoeThreads = 256;
 constexpr int kMoeSweepThreads = 1024;   // one workgroup per compute unit, the table's head in its LDS
 
@@ -784,28 +892,24 @@ extern "C" int sub1_moe_grouped(const sub1_moe_stack *st, const int32_t *token_e
   HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
   const int wmax = st->d_model > st->d_ff ? st->d_model : st->d_ff;
   a.act_dwords = lds_dwords_for_width(wmax);
-  // With at least a token per compute unit the launch is a sweep, and what
-  // bounds it is the table: one workgroup of 16 wavefronts per compute unit,
-  // whole projections as tiles (a thread takes rows in turn), and all the LDS
-  // that the activations leave for the table's first words.  Fewer tokens: tiles
-  // of 256 rows, several workgroups per compute unit, the table from memory
-  // (staging it would cost every workgroup more than it saves on one tile).
-  const size_t lds_limit = 160 * 1024 - 64;
-  const bool sweep = tokens >= cus &&
+  // One workgroup of 16 wavefronts per compute unit with all the LDS that the
+  // activations leave for the table's first words, or workgroups of 4 wavefronts,
+  // several to a compute unit, and the table from memory.  Staging the table takes
+  // a workgroup about 10 us, which it has back once it has a few microseconds' worth of
+  // codes: 12 tokens through the base, large and c-2048 shapes 44, 45 and 63 us
+  // against 50, 61 and 107; 8 tokens 43, 45 and 62 against 39, 48 and 89; one token
+  // 42, 42 and 56 against 30, 31 and 45.
+  const size_t lds_limit = 160 * 1024 - 64 - kMoeSweepThreads * sizeof(float2);
+  const bool worth_it = tokens >= cus || (tokens >= 10 && static_cast<int64_t>(tokens) * st->d_model *
+                                                              st->d_ff >= (1 << 24));
+  const bool sweep = worth_it &&
                      a.act_dwords * sizeof(float) + 16384 * sizeof(uint32_t) <= lds_limit;
   const int threads = sweep ? kMoeSweepThreads : kMoeThreads;
-  a.tile_rows = sweep ? wmax : kMoeThreads;
   a.held = 0;
   if (sweep) {
-    const size_t room = (lds_limit - a.act_dwords * sizeof(float)) / sizeof(uint32_t);
+    const size_t room = (lds_limit - a.act_dwords * sizeof(float)) / sizeof(uint32_t) / 4 * 4;
     a.held = static_cast<int>(room < SUB1_DICT_ENTRIES ? room : SUB1_DICT_ENTRIES);
   }
-  a.wi_tiles = (st->d_ff + a.tile_rows - 1) / a.tile_rows;
-  a.wo_tiles = (st->d_model + a.tile_rows - 1) / a.tile_rows;
-  a.wi_expect = a.wi_tiles + sub1::expect_extra();
-  int64_t tiles = static_cast<int64_t>(tokens) * (a.wi_tiles + a.wo_tiles);
-  if (tiles > INT32_MAX - (1 << 20))
-    return fail(SUB1_ERR_SHAPE, "sub1_moe_grouped: too many tiles");
   const size_t lds = (static_cast<size_t>(a.act_dwords) + a.held) * sizeof(float);
   if (sweep) {
     rc = allow_lds(moe_kernel<kMoeSweepThreads>, lds);
@@ -819,6 +923,31 @@ extern "C" int sub1_moe_grouped(const sub1_moe_stack *st, const int32_t *token_e
   if (rc) return rc;
   if (per_cu < 1) return fail(SUB1_ERR_INTERNAL, "sub1_moe_grouped: kernel does not fit a CU");
   int64_t grid = static_cast<int64_t>(cus) * per_cu;
+  // Parts of a projection: the number with which its tiles take the least time in
+  // rounds of the grid.  A tile costs about 8 us (ticket, activations, the wait, the
+  // wavefronts that finish early) besides its share of the projection, of which a
+  // compute unit takes some 80 000 weights a microsecond.
+  const double tile_share = 8.0 * 80000.0 / (static_cast<double>(st->d_model) * st->d_ff);
+  const int threads_rows = threads / 4;   // at least so many rows to a tile
+  auto parts_of = [&](int height) {
+    int best = 1;
+    double best_cost = 1e30;
+    for (int parts = 1; parts <= std::max(1, height / threads_rows); parts++) {
+      const int64_t rounds = (static_cast<int64_t>(tokens) * parts + grid - 1) / grid;
+      const double cost = rounds * (1.0 / parts + tile_share);
+      if (cost < best_cost - 1e-9) {
+        best_cost = cost;
+        best = parts;
+      }
+    }
+    return best;
+  };
+  a.wi_tiles = parts_of(st->d_ff);
+  a.wo_tiles = parts_of(st->d_model);
+  a.wi_expect = a.wi_tiles + sub1::expect_extra();
+  const int64_t tiles = static_cast<int64_t>(tokens) * (a.wi_tiles + a.wo_tiles);
+  if (tiles > INT32_MAX - (1 << 20))
+    return fail(SUB1_ERR_SHAPE, "sub1_moe_grouped: too many tiles");
   if (grid > tiles) grid = tiles;
 
   if (sweep) {
