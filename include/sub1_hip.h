@@ -125,7 +125,7 @@ int sub1_pack_weights_emit(const uint16_t *codes, const int32_t *row_off, int16_
  * and/or out_w (bf16 [H, W], dequantised weights) may each be NULL.  What the
  * Python `decompress` of reference test.py:103-115 computes.
  * bad_rows (int32 [1], device, may be NULL) is incremented for every row whose
- * codes do not cover exactly the row width.
+ * codes do not cover exactly the row width; columns they do not reach become zero.
  */
 int sub1_decode(const int32_t *dec, const int16_t *w_comp, const int32_t *row_off,
                 const void *ter_minmax, uint8_t *out_tern, void *out_w,

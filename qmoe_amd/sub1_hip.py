@@ -193,8 +193,8 @@ def sub1decode(dec, w_comp, row_off, ter_minmax, width, want_tern=True, want_w=T
     p_ro = _need(row_off, torch.int32, 'row_off', dev)
     p_mm = _need(ter_minmax, torch.bfloat16, 'ter_minmax', dev, numel=2 * height) \
         if ter_minmax is not None else None
-    tern = torch.zeros((height, width), dtype=torch.uint8, device=dev) if want_tern else None
-    w = torch.zeros((height, width), dtype=torch.bfloat16, device=dev) if want_w else None
+    tern = torch.empty((height, width), dtype=torch.uint8, device=dev) if want_tern else None
+    w = torch.empty((height, width), dtype=torch.bfloat16, device=dev) if want_w else None
     bad = torch.zeros(1, dtype=torch.int32, device=dev)
     with _on_device(dev):
         _lib.check(_lib.load().sub1_decode(

@@ -149,3 +149,48 @@ def test_packing_with_a_trie_of_ones_own(gpu):
         offsets.append(len(want))
     assert row_off.tolist() == offsets
     assert w_comp.cpu().numpy().view('uint16').tolist() == want
+
+
+@pytest.mark.parametrize('height,width,shares', [
+    (1, 1, [1.0]), (7, 3, [0.5]), (66, 31, [0.2]), (5, 1023, [0.1, 0.0]),      # rows that begin at any byte of a word
+    (4, 1024, [0.1]), (3, 9001, [0.0, 0.05, 0.99])])                          # runs of 64 codes, and many of them
+def test_expanding_gives_the_symbols_and_their_weights(gpu, height, width, shares):
+    sub1, op = gpu
+    symbols = symbols_of(height, width, shares, seed=width)
+    w_comp, row_off = packed(gpu, symbols)
+    minmax = torch.randn(2 * height, generator=torch.Generator().manual_seed(4)).bfloat16().cuda()
+    values = torch.cat((torch.zeros((height, 1), dtype=torch.bfloat16, device='cuda'), minmax.view(-1, 2)), 1)
+    want = values.gather(1, symbols.long())
+    tern, w, bad = op.sub1decode(sub1.DEC[0], w_comp, row_off, minmax, width)
+    assert bad == 0 and torch.equal(tern, symbols) and torch.equal(w, want)
+    # either alone, and both into buffers that begin within a word, with what lies around them
+    import ctypes
+    lib, stream = op._lib.load(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    n = height * width
+    for at_t, at_w in ((0, None), (None, 0), (1, 1), (3, 2), (2, 0)):
+        t_buf = torch.full((n + 8,), 77, dtype=torch.uint8, device='cuda')
+        w_buf = torch.full((n + 8,), 77.0, dtype=torch.bfloat16, device='cuda')
+        assert lib.sub1_decode(sub1.DEC[0].data_ptr(), w_comp.data_ptr(), row_off.data_ptr(), minmax.data_ptr(),
+                               None if at_t is None else t_buf[at_t:].data_ptr(),
+                               None if at_w is None else w_buf[at_w:].data_ptr(), None, height, width, stream) == 0
+        for buf, at, ref in ((t_buf, at_t, symbols), (w_buf, at_w, want)):
+            if at is not None:
+                assert torch.equal(buf[at:at + n].view(height, width), ref)
+                assert bool((buf[:at] == 77).all()) and bool((buf[at + n:] == 77).all())
+
+
+def test_expanding_codes_that_do_not_fit_the_width(gpu):
+    """Rows whose codes end before the row does are filled with zeros and counted,
+    rows with codes to spare are cut off and counted."""
+    sub1, op = gpu
+    symbols = symbols_of(3, 4000, [0.3], seed=9)
+    w_comp, row_off = packed(gpu, symbols)
+    minmax = torch.ones(6, dtype=torch.bfloat16, device='cuda')
+    moved = row_off.clone()
+    moved[1] -= 200
+    tern, _, bad = op.sub1decode(sub1.DEC[0], w_comp, moved, minmax, 4000)
+    assert bad == 2
+    whole, _, _ = op.sub1decode(sub1.DEC[0], w_comp, row_off, minmax, 4000)
+    assert torch.equal(tern[2], whole[2])
+    kept = int((tern[0] != whole[0]).nonzero()[0])           # the first symbol lost
+    assert 0 < kept < 4000 and torch.equal(tern[0, :kept], whole[0, :kept]) and not tern[0, kept:].any()
