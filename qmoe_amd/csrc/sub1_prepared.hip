@@ -86,7 +86,8 @@ struct MetaLayout {
   int kinds;
   int64_t counts;       // i32 [all slices + 1] chunk counts, scanned in place
   int64_t status;       // i32 [4]: [0] rows whose codes do not cover the width, [1], [2]
-                        // longest slice of kind 0 / 1 in chunks, [3] what check_on_device found
+                        // longest slice of kind 0 / 1 in chunks, [3] what check_on_device
+                        // found, then all slices' chunks
   int64_t bytes;
 };
 
@@ -137,41 +138,6 @@ MetaLayout matrix_layout(int count, int height, int width) {
 
 // ---------------------------------------------------------- prepare kernels --
 
-// Calls nz(column, symbol) for every non-zero weight of a row, in column order,
-// and returns the columns the row's codes cover.  Digit d of dictionary entry e
-// is (dec[2e + d/14] >> (4 + 2 (d % 14))) & 3, the low nibble of dec[2e] the
-// entry's pair count (reference sub1.py:60-72, sub1_cuda_kernel.cu:186-192).
-template <class F>
-__device__ __forceinline__ int for_each_nonzero(const uint16_t *codes, int n,
-                                                const int32_t *__restrict__ dec, int width,
-                                                F &&nz) {
-  int col = 0;
-  // the code after next and the next code's entry are asked for before this
-  // code's digits are walked: a row is a chain of dependent loads otherwise
-  int e_next = n > 1 ? codes[1] : 0;
-  const int e_first = n > 0 ? codes[0] : 0;
-  int32_t next0 = dec[2 * e_first], next1 = dec[2 * e_first + 1];
-  for (int i = 0; i < n; i++) {
-    const uint32_t w0 = static_cast<uint32_t>(next0);
-    const uint32_t w1 = static_cast<uint32_t>(next1);
-    if (i + 1 < n) {
-      next0 = dec[2 * e_next];
-      next1 = dec[2 * e_next + 1];
-    }
-    if (i + 2 < n) e_next = codes[i + 2];
-    unsigned long long digits = static_cast<unsigned long long>(w0 >> 4) |
-                                (static_cast<unsigned long long>(w1 >> 4) << 28);
-    while (digits) {
-      const int d = (__ffsll(digits) - 1) >> 1;
-      const int sym = static_cast<int>(digits >> (2 * d)) & 3;
-      digits &= ~(3ull << (2 * d));
-      if (col + d < width) nz(col + d, sym);   // digits past the width are dropped
-    }
-    col += 2 * static_cast<int>(w0 & 15u);
-  }
-  return col;
-}
-
 // A slice is as long as its longest row, counted in ENTRIES; its chunks, and how
 // many entries of the last one are walked (1..9; the rest of that chunk is
 // padding nobody reads).
@@ -194,32 +160,6 @@ __host__ __device__ constexpr int position_of(int c, int sym) {
 __host__ __device__ constexpr int physical_columns(int width) {
   return (physical_column(width - 1) / kZeroPeriod + 1) * kZeroPeriod + 1;
 }
-
-// Non-zeros to entries.  An entry is the step from the row's position (0 at
-// the start) to the next, 0..127.  A longer gap goes over zero columns, as far
-// as each step reaches; after the last non-zero the row parks on the next zero
-// column, where steps of 0 pad it to the length of its slice.
-struct EntryWriter {
-  int j = 0;
-  template <class E>
-  __device__ __forceinline__ void nonzero(int col, int sym, E &&emit) {
-    const int target = position_of(col, sym);
-    while (target - j > kMaxStep) {
-      const int z = (j + kMaxStep) / (2 * kZeroPeriod) * (2 * kZeroPeriod);
-      emit(z - j, j);
-      j = z;
-    }
-    emit(target - j, j);
-    j = target;
-  }
-  template <class E>
-  __device__ __forceinline__ void park(E &&emit) {
-    if ((j >> 1) % kZeroPeriod == 0) return;
-    const int z = (j + 2 * kZeroPeriod - 1) / (2 * kZeroPeriod) * (2 * kZeroPeriod);
-    emit(z - j, j);
-    j = z;
-  }
-};
 
 // Where the matrices of one kind come from: one buffer of codes with a base
 // offset per matrix and [count, height + 1] / [count, height] arrays of row
@@ -247,25 +187,214 @@ __device__ __forceinline__ const uint16_t *row_codes(const KindSource &ks, int e
   return codes + ro[r];
 }
 
-// One thread per row: how many entries its non-zeros take (the step onto a zero
-// column that a padded row makes after them is not counted: it fits the padding).
-__global__ __launch_bounds__(256) void count_entries_kernel(
-    KindSource ks, const int32_t *__restrict__ dec, uint16_t *__restrict__ row_len,
-    int32_t *__restrict__ status, int height, int width, int64_t rows_total) {
-  const int64_t g = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (g >= rows_total) return;
-  const int e = static_cast<int>(g / height);
-  const int r = static_cast<int>(g % height);
-  int n;
-  const uint16_t *codes = row_codes(ks, e, r, height, width, n);
-  int entries = 0;
-  auto emit = [&](int, int) { entries++; };
-  EntryWriter wr;
-  const int covered =
-      for_each_nonzero(codes, n, dec, width, [&](int col, int sym) { wr.nonzero(col, sym, emit); });
+// Both prepare passes walk all rows' codes, a lane to a row, through the fixed
+// dictionary in a form of one word per entry: the pair count in bits 0-3, then up
+// to three non-zeros of seven bits each, the place (0..27) below two bits that are 0
+// for none, 1 for a row min, 2 for a row max.  What bounds them is fetching that
+// word: a wavefront's gather from the 256 KB table costs a compute unit 54 ns, one
+// from LDS 3 ns.  So a compute unit takes one workgroup, persistent, that keeps the
+// table's first 40 000 words in LDS (the low codes are the frequent ones: three
+// quarters of the codes of weights with 90% zeros and more), and a lane asks for
+// eight codes and their eight words at once.
+constexpr int kWalkThreads = 1024;
+constexpr int kHeldWords = 40000;
+constexpr size_t kWalkLds = kHeldWords * sizeof(uint32_t);
+
+struct HeldTable {
+  const uint32_t *all;    // global memory
+  const uint32_t *head;   // LDS
+  __device__ __forceinline__ uint32_t operator[](uint32_t code) const {
+    // lanes whose code is held read the table's first word, one line for all of them
+    const uint32_t far = all[code < kHeldWords ? 0u : code];
+    const uint32_t near = head[min(code, kHeldWords - 1u)];
+    return code < kHeldWords ? near : far;
+  }
+};
+
+__device__ __forceinline__ HeldTable hold_table(const uint32_t *table, uint32_t *lds) {
+  for (int i = 4 * threadIdx.x; i < kHeldWords; i += 4 * kWalkThreads)
+    *reinterpret_cast<uint4 *>(lds + i) = *reinterpret_cast<const uint4 *>(table + i);
+  __syncthreads();
+  return HeldTable{table, lds};
+}
+
+// The rows' codes are followed through pointers read from memory; as a global
+// address, a load of them need not wait for the LDS too.
+typedef const __attribute__((address_space(1))) uint16_t global_u16;
+typedef uint32_t unaligned_u32x4 __attribute__((ext_vector_type(4), aligned(2)));   // eight codes
+__device__ __forceinline__ unaligned_u32x4 eight_codes(global_u16 *codes) {
+  return *(const __attribute__((address_space(1))) unaligned_u32x4 *)codes;
+}
+
+// A row's non-zeros as entries.  An entry is the step from the row's position (0 at
+// the start) to the next, 0..127; a longer gap goes over zero columns, as far as each
+// step reaches.  Calls emit(step, position after it) and returns the columns that
+// the codes cover; `at` is the position reached.
+template <class E>
+__device__ __forceinline__ int walk_row(const HeldTable &table, const uint16_t *row, int n, int width,
+                                        int &at, E &&emit) {
+  global_u16 *codes = (global_u16 *)row;
+  int col = 0;
+  at = 0;
+  auto word = [&](uint32_t w) {
+#pragma unroll
+    for (int s = 0; s < 3; s++) {
+      const uint32_t slot = w >> (4 + 7 * s);
+      const int c = col + static_cast<int>(slot & 31u);
+      if ((slot & 0x60u) && c < width) {   // digits past the width are dropped
+        const int target = position_of(c, 1) + static_cast<int>((slot >> 6) & 1u);
+        // two non-zeros of one entry are 27 columns apart at most: within a step
+        if (s == 0)
+#pragma unroll 1
+          while (target - at > kMaxStep) {
+            const int zero = (at + kMaxStep) / (2 * kZeroPeriod) * (2 * kZeroPeriod);
+            const int step = zero - at;
+            at = zero;
+            emit(step, at);
+          }
+        const int step = target - at;
+        at = target;
+        emit(step, at);
+      }
+    }
+    col += 2 * static_cast<int>(w & 15u);
+  };
+  if (n < 8) {
+#pragma unroll 1
+    for (int i = 0; i < n; i++) word(table[codes[i]]);
+    return col;
+  }
+  unaligned_u32x4 next = eight_codes(codes);
+#pragma unroll 1
+  for (int i = 0; i < n; i += 8) {
+    const unaligned_u32x4 four = next;
+    // the row's last, partial eight is read from eight codes before its end
+    if (i + 8 < n) next = eight_codes(codes + min(i + 8, n - 8));
+    const int skip = max(i + 8 - n, 0);
+    uint32_t w[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      w[j] = table[(j & 1) ? four[j / 2] >> 16 : four[j / 2] & 0xffffu];
+      if (j < skip) w[j] = 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++) word(w[j]);
+  }
+  return col;
+}
+
+// A prepare pass over all rows of one kind of matrices, 64 at a time; kinds with
+// longer rows first, so that the launch does not end on them.
+struct WalkKind {
+  KindSource source;
+  int height, width, slices;
+  int64_t tasks;                // of 64 rows (counting: in the matrices' own order; emitting: slices)
+  int64_t first_slice;          // emitting: among all kinds' slices
+  uint16_t *row_len;            // counting
+  const uint32_t *slice_base;   // emitting
+  const uint16_t *slice_len, *row_idx;
+};
+struct WalkArgs {
+  WalkKind k[2];
+  int kinds, count;
+  const uint32_t *table;
+  int32_t *status;
+  uint2 *stream;
+  uint16_t *ckpt;
+};
+
+// How many entries the non-zeros of every row take (the step onto a zero column
+// that a padded row makes after them is not counted: it fits the padding).
+__device__ __forceinline__ void count_rows(const HeldTable &table, const WalkKind &k, int count,
+                                           int64_t task, int32_t *status) {
+  // rows of a task: from row `first` of a matrix on, and of the next ones
+  const int64_t g = task * 64 + (threadIdx.x & 63);
+  if (g >= static_cast<int64_t>(count) * k.height) return;
+  const int first_e = static_cast<int>(task * 64 / k.height);
+  const uint32_t past = static_cast<uint32_t>(g - static_cast<int64_t>(first_e) * k.height);
+  const int e = first_e + static_cast<int>(past / static_cast<uint32_t>(k.height));
+  const int r = static_cast<int>(past % static_cast<uint32_t>(k.height));
+  int n, at, entries = 0;
+  const uint16_t *codes = row_codes(k.source, e, r, k.height, k.width, n);
+  const int covered = walk_row(table, codes, n, k.width, at, [&](int, int) { entries++; });
   // a row's codes cover its width rounded up to a whole pair, exactly
-  if (covered != ((width + 1) & ~1)) atomicAdd(&status[0], 1);
-  row_len[g] = static_cast<uint16_t>(min(entries, kMaxRowEntries));
+  if (covered != ((k.width + 1) & ~1)) atomicAdd(&status[0], 1);
+  k.row_len[g] = static_cast<uint16_t>(min(entries, kMaxRowEntries));
+}
+
+// Position checkpoints.  For every slice and every group of kGroupChunks chunks,
+// the position at which each lane's row stands when the group begins: 64 x u16
+// per group, groups of slice g stored from entry slice_base[g]/kGroupChunks + g
+// on.  With them a wavefront can start in the middle of a slice, which is how a
+// small batch is spread over the GPU.
+__device__ __forceinline__ int64_t checkpoint_entry(uint32_t slice_base, int64_t slice) {
+  return static_cast<int64_t>(slice_base / kGroupChunks) + slice;
+}
+
+// A slice's rows, a lane each, into the interleaved stream, nine entries to a chunk;
+// a row shorter than its slice then steps onto the next zero column and stays there
+// (steps of 0) to the end of the slice's last chunk; and the row's position at the
+// start of every group of chunks into the checkpoints.
+__device__ __forceinline__ void emit_rows(const HeldTable &table, const WalkKind &k, int64_t slice,
+                                          uint2 *__restrict__ stream, uint16_t *__restrict__ ckpt) {
+  const int lane = threadIdx.x & 63;
+  const int e = static_cast<int>(slice / k.slices);
+  const int ridx = k.row_idx[slice * 64 + lane];
+  const uint32_t base = k.slice_base[slice];
+  const int len = k.slice_len[slice];
+  const int nch = chunks_of(len);
+  uint2 *d = stream + static_cast<int64_t>(base) * 64 + lane;
+  uint16_t *ck = ckpt + checkpoint_entry(base, k.first_slice + slice) * 64 + lane;
+  int c = 0, q = 0;
+  uint32_t lo = 0, hi = 0;   // the chunk so far, its newest entry in bits 56..62
+  ck[0] = 0;
+  auto emit = [&](int step, int after) {
+    lo = __builtin_amdgcn_alignbit(hi, lo, kFieldBits);
+    hi = (hi >> kFieldBits) | static_cast<uint32_t>(step) << 24;
+    if (++q == kFields) {
+      q = 0;
+      if (c < nch) d[c * 64] = make_uint2(lo, hi);   // the slice is as long as its longest row
+      c++;
+      if (c % kGroupChunks == 0 && c < nch) ck[(c / kGroupChunks) * 64] = static_cast<uint16_t>(after);
+    }
+  };
+  int at = 0;
+  if (ridx != 0xffff) {
+    int n;
+    const uint16_t *codes = row_codes(k.source, e, ridx, k.height, k.width, n);
+    walk_row(table, codes, n, k.width, at, emit);
+    if (c * kFields + q < len && (at >> 1) % kZeroPeriod != 0) {   // padding follows: it must read zeros
+      const int zero = (at + 2 * kZeroPeriod - 1) / (2 * kZeroPeriod) * (2 * kZeroPeriod);
+      const int step = zero - at;
+      at = zero;
+      emit(step, at);
+    }
+  }
+#pragma unroll 1
+  while (c < nch) emit(0, at);
+}
+
+// Task t goes to workgroup t mod grid first: a matrix of a few slices is spread over
+// as many compute units.  128 base experts (26 million codes): counting takes 59 us
+// (194 with the two-word table in global memory and a code at a time), emitting 132
+// (313); both are bound by their instructions, about 60 and 110 a code, emitting also by the
+// stores of lanes that fill their chunks at different times.  One code a turn
+// instead of eight (a tenth of the code) measured 93 and 169.
+template <bool kEmit>
+__global__ __launch_bounds__(kWalkThreads) void walk_rows_kernel(WalkArgs a) {
+  extern __shared__ __align__(16) uint32_t held[];
+  const HeldTable table = hold_table(a.table, held);
+  const int64_t step = static_cast<int64_t>(gridDim.x) * (kWalkThreads / 64);
+  int64_t task = blockIdx.x + static_cast<int64_t>(gridDim.x) * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int i = 0; i < a.kinds; i++) {
+    for (; task < a.k[i].tasks; task += step) {
+      if (kEmit)
+        emit_rows(table, a.k[i], task, a.stream, a.ckpt);
+      else
+        count_rows(table, a.k[i], a.count, task, a.status);
+    }
+    task -= a.k[i].tasks;
+  }
 }
 
 // One workgroup per matrix: order the rows by entry count, longest first, rows
@@ -421,61 +550,11 @@ __global__ __launch_bounds__(256) void check_source_kernel(const int32_t *__rest
   if (bad) atomicOr(found, bad);
 }
 
-__global__ __launch_bounds__(sub1::kScanThreads) void scan_counts_kernel(int32_t *v, int n) {
+// ... and the total once more beside the status words, where one copy fetches all.
+__global__ __launch_bounds__(sub1::kScanThreads) void scan_counts_kernel(int32_t *v, int n, int32_t *total) {
   sub1::scan_in_place(v, n);
-}
-
-// Position checkpoints.  For every slice and every group of kGroupChunks chunks,
-// the position at which each lane's row stands when the group begins: 64 x u16
-// per group, groups of slice g stored from entry slice_base[g]/kGroupChunks + g
-// on.  With them a wavefront can start in the middle of a slice, which is how a
-// small batch is spread over the GPU.
-__device__ __forceinline__ int64_t checkpoint_entry(uint32_t slice_base, int64_t slice) {
-  return static_cast<int64_t>(slice_base / kGroupChunks) + slice;
-}
-
-// One thread per lane of every slice: the row's entries into the interleaved
-// stream, nine to a chunk; a row shorter than its slice then steps onto the
-// next zero column and stays there (steps of 0) to the end of the slice's last
-// chunk; and the row's position at the start of every group of chunks into the
-// checkpoints.
-__global__ __launch_bounds__(256) void emit_entries_kernel(
-    KindSource ks, const int32_t *__restrict__ dec,
-    const uint32_t *__restrict__ slice_base, const uint16_t *__restrict__ slice_len,
-    const uint16_t *__restrict__ row_idx, uint2 *__restrict__ dst, uint16_t *__restrict__ ckpt,
-    int height, int width, int slices, int64_t first_slice, int64_t lanes_total) {
-  const int64_t gl = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (gl >= lanes_total) return;
-  const int64_t slice = gl >> 6;
-  const int ln = static_cast<int>(gl & 63);
-  const int e = static_cast<int>(slice / slices);
-  const int ridx = row_idx[gl];
-  const uint32_t base = slice_base[slice];
-  const int len = slice_len[slice];
-  const int nch = chunks_of(len);
-  uint2 *d = dst + static_cast<int64_t>(base) * 64 + ln;
-  uint16_t *ck = ckpt + checkpoint_entry(base, first_slice + slice) * 64 + ln;
-  int c = 0, q = 0;
-  unsigned long long w = 0;
-  auto emit = [&](int step, int from) {
-    if (c >= nch) return;   // the slice is as long as its longest row: not reached
-    if (q == 0 && c % kGroupChunks == 0) ck[(c / kGroupChunks) * 64] = static_cast<uint16_t>(from);
-    w |= static_cast<unsigned long long>(step) << (kFieldBits * q);
-    if (++q == kFields) {
-      d[c * 64] = make_uint2(static_cast<uint32_t>(w), static_cast<uint32_t>(w >> 32));
-      c++;
-      q = 0;
-      w = 0;
-    }
-  };
-  EntryWriter wr;
-  if (ridx != 0xffff) {
-    int n;
-    const uint16_t *codes = row_codes(ks, e, ridx, height, width, n);
-    for_each_nonzero(codes, n, dec, width, [&](int col, int sym) { wr.nonzero(col, sym, emit); });
-    if (c * kFields + q < len) wr.park(emit);   // padding follows: it must read zeros
-  }
-  while (c < nch) emit(0, wr.j);
+  __syncthreads();
+  if (threadIdx.x == 0) *total = v[n];
 }
 
 // The symbols of one prepared matrix back out of the stream: out[row, column]
@@ -2217,23 +2296,42 @@ __global__ __launch_bounds__(kMaxThreads) void matvec_group_kernel(PreparedArgs 
 // dec to compare it there, as it was done first, took 9 ms a call, two calls to
 // a layer; the kernel and reading its answer back take about 20 us.
 static __device__ __align__(16) int32_t fixed_dec[SUB1_DEC_WORDS];
+static __device__ __align__(16) uint32_t fixed_slots[SUB1_DICT_ENTRIES];   // the walks' one-word form
 std::mutex g_fixed_mutex;
 std::vector<int> g_fixed_devices;   // where fixed_dec is filled
 
-int fixed_dec_of_current_device(const int32_t **out) {
+int fixed_tables_of_current_device(const int32_t **dec, const uint32_t **slots) {
   int device = 0;
-  void *address = nullptr;
+  void *at_dec = nullptr, *at_slots = nullptr;
   HIP_TRY(hipGetDevice(&device));
-  HIP_TRY(hipGetSymbolAddress(&address, HIP_SYMBOL(fixed_dec)));
+  HIP_TRY(hipGetSymbolAddress(&at_dec, HIP_SYMBOL(fixed_dec)));
+  HIP_TRY(hipGetSymbolAddress(&at_slots, HIP_SYMBOL(fixed_slots)));
   std::lock_guard<std::mutex> lock(g_fixed_mutex);
   if (std::find(g_fixed_devices.begin(), g_fixed_devices.end(), device) == g_fixed_devices.end()) {
     std::vector<int32_t> table(SUB1_DEC_WORDS);
     const int rc = sub1_build_tables(table.data(), nullptr);
     if (rc) return fail(rc, "sub1_build_tables failed");
-    HIP_TRY(hipMemcpy(address, table.data(), table.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    std::vector<uint32_t> words(SUB1_DICT_ENTRIES);
+    for (int e = 0; e < SUB1_DICT_ENTRIES; e++) {
+      // digit d of entry e is (dec[2e + d/14] >> (4 + 2 (d % 14))) & 3, the low nibble of
+      // dec[2e] its pair count (reference sub1.py:60-72, sub1_cuda_kernel.cu:186-192)
+      uint32_t w = static_cast<uint32_t>(table[2 * e]) & 15u;
+      int n = 0;
+      for (int d = 0; d < 28; d++) {
+        const uint32_t t = (static_cast<uint32_t>(table[2 * e + d / 14]) >> (4 + 2 * (d % 14))) & 3u;
+        if (t == 0) continue;
+        if (t == 3 || n == 3)
+          return fail(SUB1_ERR_INTERNAL, "dictionary entry %d is outside the form of the walks", e);
+        w |= (static_cast<uint32_t>(d) | t << 5) << (4 + 7 * n++);
+      }
+      words[e] = w;
+    }
+    HIP_TRY(hipMemcpy(at_dec, table.data(), table.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(at_slots, words.data(), words.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
     g_fixed_devices.push_back(device);
   }
-  *out = static_cast<const int32_t *>(address);
+  *dec = static_cast<const int32_t *>(at_dec);
+  *slots = static_cast<const uint32_t *>(at_slots);
   return SUB1_OK;
 }
 
@@ -2261,10 +2359,12 @@ int name_bad_pointer(const void *const *table, int count, size_t align, const ch
 }
 
 // dec and the pointer tables, looked at on the GPU; `word` is a device word to
-// leave the answer in.  Synchronises the stream.
-int check_on_device(const Source &src, int32_t *word, hipStream_t s, const char *who) {
+// leave the answer in, *slots receives the dictionary as the walks read it.
+// Synchronises the stream.
+int check_on_device(const Source &src, int32_t *word, const uint32_t **slots, hipStream_t s,
+                    const char *who) {
   const int32_t *fixed = nullptr;
-  int rc = fixed_dec_of_current_device(&fixed);
+  int rc = fixed_tables_of_current_device(&fixed, slots);
   if (rc) return rc;
   const char *const names[3] = {"w_comp", "row_off", "ter_minmax"};
   PointerTables pt{};
@@ -2401,6 +2501,34 @@ struct LayoutResult {
   int max_chunks[2];
 };
 
+// Where kind i stands in a walk's order: longer rows first.
+int walk_place(const Source &src, int i) {
+  return src.kinds == 2 && src.width[1] > src.width[0] ? 1 - i : i;
+}
+
+template <bool kEmit>
+int launch_walk(const Source &src, const MetaLayout &m, WalkArgs &w, hipStream_t s) {
+  w.kinds = src.kinds;
+  w.count = src.count;
+  int64_t tasks = 0;
+  for (int i = 0; i < src.kinds; i++) {
+    WalkKind &k = w.k[walk_place(src, i)];
+    k.source = src.k[i];
+    k.height = m.k[i].height;
+    k.width = m.k[i].width;
+    k.slices = m.k[i].slices;
+    tasks += k.tasks;
+  }
+  int device = 0, cus = 0;
+  HIP_TRY(hipGetDevice(&device));
+  HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+  HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(walk_rows_kernel<kEmit>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kWalkLds)));
+  walk_rows_kernel<kEmit><<<static_cast<unsigned>(std::min<int64_t>(tasks, cus)), kWalkThreads, kWalkLds, s>>>(w);
+  HIP_TRY(hipGetLastError());
+  return SUB1_OK;
+}
+
 int prepare_layout(const Source &src, void *meta, int64_t meta_bytes, LayoutResult *out,
                    hipStream_t s, const char *who) {
   if (!meta || !out) return fail(SUB1_ERR_NULL, "%s: NULL argument", who);
@@ -2410,34 +2538,40 @@ int prepare_layout(const Source &src, void *meta, int64_t meta_bytes, LayoutResu
     return fail(SUB1_ERR_SHAPE, "%s: meta needs %lld bytes", who, static_cast<long long>(m.bytes));
   char *base = static_cast<char *>(meta);
   int32_t *status = reinterpret_cast<int32_t *>(base + m.status);
-  int rc = check_on_device(src, status + 3, s, who);
+  WalkArgs w{};
+  int rc = check_on_device(src, status + 3, &w.table, s, who);
   if (rc) return rc;
   int32_t *counts = reinterpret_cast<int32_t *>(base + m.counts);
   zero_words_kernel<<<1, 64, 0, s>>>(status, 3);
+  w.status = status;
+  for (int i = 0; i < src.kinds; i++) {
+    const KindMeta &k = m.k[i];
+    WalkKind &wk = w.k[walk_place(src, i)];
+    wk.row_len = reinterpret_cast<uint16_t *>(base + k.row_len);
+    wk.tasks = (static_cast<int64_t>(src.count) * k.height + 63) / 64;
+  }
+  rc = launch_walk<false>(src, m, w, s);
+  if (rc) return rc;
   HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(order_rows_kernel),
                               hipFuncAttributeMaxDynamicSharedMemorySize,
                               static_cast<int>(order_rows_lds(65534))));
   int64_t slice0 = 0;
   for (int i = 0; i < src.kinds; i++) {
     const KindMeta &k = m.k[i];
-    uint16_t *row_len = reinterpret_cast<uint16_t *>(base + k.row_len);
-    const int64_t rows = static_cast<int64_t>(src.count) * k.height;
-    count_entries_kernel<<<static_cast<unsigned>((rows + 255) / 256), 256, 0, s>>>(
-        src.k[i], src.dec, row_len, status, k.height, k.width, rows);
     order_rows_kernel<<<src.count, kOrderThreads, order_rows_lds(k.height), s>>>(
-        row_len, src.k[i], reinterpret_cast<uint16_t *>(base + k.row_idx),
+        reinterpret_cast<const uint16_t *>(base + k.row_len), src.k[i],
+        reinterpret_cast<uint16_t *>(base + k.row_idx),
         reinterpret_cast<uint32_t *>(base + k.minmax),
         reinterpret_cast<uint16_t *>(base + k.slice_len), counts + slice0, status, k.height,
         k.slices, i);
     slice0 += static_cast<int64_t>(src.count) * k.slices;
   }
-  scan_counts_kernel<<<1, sub1::kScanThreads, 0, s>>>(counts, static_cast<int>(slice0));
+  scan_counts_kernel<<<1, sub1::kScanThreads, 0, s>>>(counts, static_cast<int>(slice0), status + 3);
   HIP_TRY(hipGetLastError());
-  int32_t host[3] = {0, 0, 0};
-  int32_t total = 0;
+  int32_t host[4] = {0, 0, 0, 0};
   HIP_TRY(hipMemcpyAsync(host, status, sizeof host, hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipMemcpyAsync(&total, counts + slice0, 4, hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
+  const int32_t total = host[3];
   if (host[0])
     return fail(SUB1_ERR_SHAPE, "%s: the codes of %d rows do not cover the width", who, host[0]);
   if (total < 0) return fail(SUB1_ERR_SHAPE, "%s: stream too large", who);
@@ -2462,24 +2596,25 @@ int prepare_codes(const Source &src, const Prepared &p, hipStream_t s, const cha
   if (p.total_chunks < 0 || p.meta_bytes < m.bytes ||
       p.code_bytes < p.total_chunks * 512 + (p.total_chunks / kGroupChunks + nslices + 1) * 128)
     return fail(SUB1_ERR_SHAPE, "%s: buffers smaller than the layout needs", who);
-  const int rc = check_on_device(src, reinterpret_cast<int32_t *>(base + m.status) + 3, s, who);
+  WalkArgs w{};
+  const int rc = check_on_device(src, reinterpret_cast<int32_t *>(base + m.status) + 3, &w.table, s, who);
   if (rc) return rc;
   uint2 *stream = static_cast<uint2 *>(const_cast<void *>(p.codes));
   uint16_t *ckpt = reinterpret_cast<uint16_t *>(stream + p.total_chunks * 64);
+  w.stream = stream;
+  w.ckpt = ckpt;
   int64_t first_slice = 0;
   for (int i = 0; i < src.kinds; i++) {
     const KindMeta &k = m.k[i];
-    const int64_t kslices = static_cast<int64_t>(src.count) * k.slices;
-    const int64_t lanes = kslices * 64;
-    emit_entries_kernel<<<static_cast<unsigned>((lanes + 255) / 256), 256, 0, s>>>(
-        src.k[i], src.dec, reinterpret_cast<const uint32_t *>(base + k.slice_base),
-        reinterpret_cast<const uint16_t *>(base + k.slice_len),
-        reinterpret_cast<const uint16_t *>(base + k.row_idx), stream, ckpt, k.height, k.width,
-        k.slices, first_slice, lanes);
-    first_slice += kslices;
+    WalkKind &wk = w.k[walk_place(src, i)];
+    wk.slice_base = reinterpret_cast<const uint32_t *>(base + k.slice_base);
+    wk.slice_len = reinterpret_cast<const uint16_t *>(base + k.slice_len);
+    wk.row_idx = reinterpret_cast<const uint16_t *>(base + k.row_idx);
+    wk.first_slice = first_slice;
+    wk.tasks = static_cast<int64_t>(src.count) * k.slices;
+    first_slice += wk.tasks;
   }
-  HIP_TRY(hipGetLastError());
-  return SUB1_OK;
+  return launch_walk<true>(src, m, w, s);
 }
 
 // Cut of the matrices for a batch that cannot occupy the GPU with a wavefront

@@ -124,6 +124,16 @@ class Sub1Linear(nn.Module):
         return linear
 
 
+def _buffers_of(layer):
+    """(w_comp, row_off, ter_minmax) of a Sub1Linear or what stands in for one;
+    straight from the module's buffers where they are, which a layer of hundreds
+    of experts notices."""
+    held = getattr(layer, '_buffers', None)
+    if held and 'w_comp' in held and 'row_off' in held and 'ter_minmax' in held:
+        return held['w_comp'], held['row_off'], held['ter_minmax']
+    return layer.w_comp, layer.row_off, layer.ter_minmax
+
+
 class Sub1Experts(nn.Module):
     """All experts of one MoE layer behind one launch.
 
@@ -137,8 +147,8 @@ class Sub1Experts(nn.Module):
         dev = wi_layers[0].w_comp.device
         self._dec = DEC[dev.index]
         # the layers' own tensors: read when a launcher is made, never copied whole
-        self._wi = [(l.w_comp, l.row_off, l.ter_minmax) for l in wi_layers]
-        self._wo = [(l.w_comp, l.row_off, l.ter_minmax) for l in wo_layers]
+        self._wi = [_buffers_of(l) for l in wi_layers]
+        self._wo = [_buffers_of(l) for l in wo_layers]
         self._d_ff = self._wi[0][1].numel() - 1
         self._d_model = self._wo[0][1].numel() - 1
         self._prepared = None
