@@ -406,6 +406,13 @@ int sub1_matvec_prepared(const sub1_matrix_prepared *prepared, const int32_t *to
                          const void *x, int64_t ldx, void *y, int64_t ldy, int tokens,
                          void *stream);
 
+/*
+ * One matrix (the first), into a y that holds nothing yet: y[t, :] = W x[t, :], the
+ * bits that sub1_matvec_prepared gives on a y of zeros, without filling or reading it.
+ */
+int sub1_product_prepared(const sub1_matrix_prepared *prepared, const void *x, int64_t ldx, void *y,
+                          int64_t ldy, int tokens, void *stream);
+
 int sub1_matrix_prepared_decode(const sub1_matrix_prepared *prepared, int matrix,
                                 void *tern_out, void *stream);
 
@@ -469,6 +476,13 @@ int sub1_tiles_entries(const sub1_matrix_set *set, const sub1_tiles *tiles, void
 
 int sub1_matvec_tiles(const sub1_tiles *tiles, int matrix, const void *x, int64_t ldx, void *y,
                       int64_t ldy, int tokens, void *stream);
+
+/*
+ * The same into a y that holds nothing yet: y[t, :] = W_m x[t, :], the bits that
+ * sub1_matvec_tiles gives on a y of zeros, without filling or reading it.
+ */
+int sub1_product_tiles(const sub1_tiles *tiles, int matrix, const void *x, int64_t ldx, void *y,
+                       int64_t ldy, int tokens, void *stream);
 
 /*
  * For tests (no counterpart in the reference): later sub1_matvec_tiles launches

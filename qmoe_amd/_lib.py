@@ -102,11 +102,13 @@ PROTOTYPES = {
                                          ctypes.POINTER(MatrixPrepared), _vp]),
     'sub1_matvec_prepared': (_int, [ctypes.POINTER(MatrixPrepared), _vp, _vp, _i64, _vp, _i64,
                                     _int, _vp]),
+    'sub1_product_prepared': (_int, [ctypes.POINTER(MatrixPrepared), _vp, _i64, _vp, _i64, _int, _vp]),
     'sub1_matrix_prepared_decode': (_int, [ctypes.POINTER(MatrixPrepared), _int, _vp, _vp]),
     'sub1_tiles_meta_bytes': (_i64, [_int, _int, _int]),
     'sub1_tiles_layout': (_int, [ctypes.POINTER(MatrixSet), _vp, _i64, ctypes.POINTER(Tiles), _vp]),
     'sub1_tiles_entries': (_int, [ctypes.POINTER(MatrixSet), ctypes.POINTER(Tiles), _vp]),
     'sub1_matvec_tiles': (_int, [ctypes.POINTER(Tiles), _int, _vp, _i64, _vp, _i64, _int, _vp]),
+    'sub1_product_tiles': (_int, [ctypes.POINTER(Tiles), _int, _vp, _i64, _vp, _i64, _int, _vp]),
     'sub1_tiles_decode': (_int, [ctypes.POINTER(Tiles), _int, _vp, _vp]),
     'sub1_route_from_mask': (_int, [_vp, _int, _int, _int, _vp, _vp, _vp]),
     'sub1_timing_begin': (_int, [_vp]),

@@ -622,6 +622,7 @@ struct PreparedArgs {
   int32_t *ctrl;                 // NULL: no dependencies between tiles, static tile order
   int64_t ldx, ldy;              // element strides between tokens of x and y
   int kinds;                     // 2: y = wo(relu(wi x));  1: y += W x
+  int fresh;                     // kinds == 1: y counts as zeros and is not read
   int tokens, experts;
   int xdwords;                   // LDS dwords reserved for the activations
   int hdwords;                   // fused kernel: LDS dwords of h (wo's activations)
@@ -990,7 +991,8 @@ __device__ __forceinline__ int slice_of_pass(int pass, int wave, int waves, int 
 }
 
 // How a row's result leaves the kernel.
-enum OutMode { kStoreRelu = 0, kStore = 1, kAccumulate = 2 };
+// kFresh: kAccumulate onto a y that counts as zeros and is not read.
+enum OutMode { kStoreRelu = 0, kStore = 1, kAccumulate = 2, kFresh = 3 };
 
 __device__ __forceinline__ void write_row(uint16_t *dst, int ridx, float res, int mode) {
   if (ridx == 0xffff) return;   // padding lane
@@ -1004,6 +1006,8 @@ __device__ __forceinline__ void write_row(uint16_t *dst, int ridx, float res, in
   } else if (mode == kAccumulate) {
     // reference sub1_cuda_kernel.cu:200: y[row] += bf16(res), the sum in bf16
     out = f32_to_bf16(bf16_to_f32(dst[ridx]) + bf16_to_f32(out));
+  } else if (mode == kFresh) {
+    out = f32_to_bf16(0.f + bf16_to_f32(out));   // (0 + -0 is 0)
   }
   dst[ridx] = out;
 }
@@ -1327,7 +1331,7 @@ __device__ __forceinline__ uint16_t *tile_output(const PreparedArgs &a, const Ki
     mode = kStoreRelu;
     return a.h + static_cast<int64_t>(t) * k.height;
   }
-  mode = a.kinds == 2 ? kStore : kAccumulate;
+  mode = a.kinds == 2 ? kStore : a.fresh ? kFresh : kAccumulate;
   return a.y + static_cast<int64_t>(t) * a.ldy;
 }
 
@@ -2280,7 +2284,8 @@ __global__ __launch_bounds__(kMaxThreads) void matvec_group_kernel(PreparedArgs 
 #pragma unroll
       for (int t = 0; t < kGroupTokens; t++)
         if (t < left)
-          write_row(a.y + static_cast<int64_t>(t0 + t) * a.ldy, cur.ridx, res.v[t], kAccumulate);
+          write_row(a.y + static_cast<int64_t>(t0 + t) * a.ldy, cur.ridx, res.v[t],
+                    a.fresh ? kFresh : kAccumulate);
       if (s_next < count) cur = nxt;
       s = s_next;
     }
@@ -2730,7 +2735,7 @@ double part_passes(int slices, int waves, int groups_max) {
 // split in two (a piece is not split again).
 int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *x, int64_t ldx,
                     void *y, int64_t ldy, int tokens, void *workspace, int64_t workspace_bytes,
-                    hipStream_t s, const char *who, int piece = 0, bool may_allocate = true) {
+                    hipStream_t s, const char *who, int piece = 0, bool may_allocate = true, bool fresh = false) {
   if (!p.meta || !p.codes || !x || !y) return fail(SUB1_ERR_NULL, "%s: NULL argument", who);
   if (p.kinds == 2 && !token_matrix) return fail(SUB1_ERR_NULL, "%s: NULL token_expert", who);
   if (tokens < 0 || tokens > (1 << 20))
@@ -2753,6 +2758,7 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
 
   PreparedArgs a;
   a.by_ticket = 0;
+  a.fresh = fresh;
   a.tagged = nullptr;
   a.lane_parts = 1;
   a.stream = static_cast<const uint2 *>(p.codes);
@@ -3499,6 +3505,17 @@ extern "C" int sub1_matvec_prepared(const sub1_matrix_prepared *p, const int32_t
                 p->height, p->width);
   return launch_prepared(from_matrix(p), token_matrix, x, ldx, y, ldy, tokens, nullptr, 0,
                          static_cast<hipStream_t>(stream), "sub1_matvec_prepared");
+}
+
+extern "C" int sub1_product_prepared(const sub1_matrix_prepared *p, const void *x, int64_t ldx,
+                                     void *y, int64_t ldy, int tokens, void *stream) {
+  if (!p) return fail(SUB1_ERR_NULL, "sub1_product_prepared: NULL argument");
+  if (tokens == 0) return SUB1_OK;
+  if (bad_dims(p->count, p->height, p->width))
+    return fail(SUB1_ERR_SHAPE, "sub1_product_prepared: %d matrices of %d x %d", p->count,
+                p->height, p->width);
+  return launch_prepared(from_matrix(p), nullptr, x, ldx, y, ldy, tokens, nullptr, 0,
+                         static_cast<hipStream_t>(stream), "sub1_product_prepared", 0, true, true);
 }
 
 extern "C" int sub1_matrix_prepared_decode(const sub1_matrix_prepared *p, int matrix,

@@ -12,16 +12,21 @@
 // holds the weights of row 32 u + r that it feeds the matrix core as its share
 // of the B operand: in step s (0..7) of the window the eight columns
 // 128 w + 16 s + 8 h + q.  Word s / 2 of its 16 bytes holds steps s and s + 1;
-// the weight of step s = 2 m + e and q = 2 k + o sits in bits
-// 16 o + 8 e + 2 k (+1) of word m, as 0 (the row's min), 1 (its max) or 2
+// the weight of step s = 2 m + e and q = 4 f + b sits in bits
+// 8 b + 4 e + 2 f (+1) of word m, as 0 (the row's min), 1 (its max) or 2
 // (zero).  A wavefront fetches a unit with one coalesced 16-byte load per
 // lane.  Rows are padded to a multiple of 64 and columns to a multiple of 128
 // with zeros; (min, max) per row are copied.
 //
-// From the codes to bf16 pairs without a table: (word >> 2 k) & 0x00030003
-// times 0x0202 plus 0x01000100 is a byte selector that picks, out of the row's
-// (min, max) word and a zero word, the two weights of pair k (v_perm_b32):
-// four plain instructions per pair of weights.
+// From the codes to bf16 pairs without a table in memory: (word >> (4 e + 2 f))
+// & 0x03030303 is the codes of four weights a byte each, which is a byte
+// selector (v_perm_b32) into (min, max, 0, 0) of the row's upper and of its
+// lower bytes; two more permutes put the four upper and lower bytes together as
+// two pairs.  Twelve plain instructions for the eight weights of an operand.
+// (With a pair's codes 16 bits apart, widened to a selector into the row's
+// (min, max) word by a multiply-add, it is sixteen: behind an operand that
+// serves 64 tokens that is eight instructions per MFMA instead of six, and six
+// are what an MFMA hides.)
 //
 // Kernel: a workgroup owns 64 rows x 64 tokens; its wavefronts split the
 // windows of 128 columns among themselves (wavefront v takes v, v + n, ...).  Per
@@ -161,7 +166,7 @@ __device__ __forceinline__ void code_place(int c, int &half, int &word, int &shi
   const int step = c >> 4, q = c & 7;
   half = (c >> 3) & 1;
   word = step >> 1;
-  shift = 16 * (q & 1) + 8 * (step & 1) + 2 * (q >> 1);
+  shift = 8 * (q & 3) + 4 * (step & 1) + 2 * (q >> 2);
 }
 
 // One thread per row of every matrix: its codes into the units (all zero
@@ -256,6 +261,7 @@ struct TileArgs {
   int64_t ldx, ldy;
   int height, width, tokens;
   int units_down, windows, matrix;
+  int fresh;   // y holds nothing yet: it counts as zeros and is not read
 };
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -268,12 +274,55 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_over(const void *base, 
 }
 constexpr uint32_t kOutside = 0x80000000u;   // an offset past every buffer here
 
-// The bf16 pair of weights of pair k (0..7) of a word of codes: `min_max` is
-// the row's (min, max) word.
-__device__ __forceinline__ uint32_t weight_pair(uint32_t codes, int k, uint32_t min_max) {
-  const uint32_t two = (codes >> (2 * k)) & 0x00030003u;
-  const uint32_t pick = two * 0x0202u + 0x01000100u;
-  return __builtin_amdgcn_perm(0u, min_max, pick);
+// (min, max, 0, 0) of a row's lower bytes and of its upper ones, from its
+// (min, max) word: what the codes select from.
+struct RowTables {
+  uint32_t lo[2], hi[2];   // of a lane's two rows
+};
+__device__ __forceinline__ void set_tables(RowTables &t, int j, uint32_t min_max) {
+  t.lo[j] = __builtin_amdgcn_perm(0u, min_max, 0x0c0c0200u);
+  t.hi[j] = __builtin_amdgcn_perm(0u, min_max, 0x0c0c0301u);
+}
+
+// The B operands of a step in the making: the weights of a lane's two rows from
+// half kE of a word of codes each, as 24 instructions of which none needs the
+// one just before it.  They are issued in equal shares behind the MFMAs of the
+// step before.
+struct WeightsInTheMaking {
+  uint32_t at[4], lo[4], hi[4];   // [2 row + f]: codes, lower and upper bytes of four weights
+};
+constexpr int kDecodeOps = 24;
+template <int kOp, int kE>
+__device__ __forceinline__ void decode_op(WeightsInTheMaking &m, uint32_t word0, uint32_t word1,
+                                          const RowTables &rows, u32x4 (&wv)[2]) {
+  // (each is pinned to its place: the scheduler would gather them elsewhere)
+  if constexpr (kOp < 4) {
+    constexpr int shift = 4 * kE + 2 * (kOp & 1);
+    m.at[kOp] = (kOp >> 1 ? word1 : word0) >> shift;
+    if (shift) asm volatile("" : "+v"(m.at[kOp]));
+  } else if constexpr (kOp < 8) {
+    m.at[kOp - 4] &= 0x03030303u;
+    asm volatile("" : "+v"(m.at[kOp - 4]));
+  } else if constexpr (kOp < 16) {
+    constexpr int i = (kOp - 8) >> 1;
+    uint32_t &out = kOp & 1 ? m.hi[i] : m.lo[i];
+    out = __builtin_amdgcn_perm(0u, kOp & 1 ? rows.hi[i >> 1] : rows.lo[i >> 1], m.at[i]);
+    asm volatile("" : "+v"(out));
+  } else {
+    constexpr int i = (kOp - 16) >> 1;
+    uint32_t pair = __builtin_amdgcn_perm(m.hi[i], m.lo[i], kOp & 1 ? 0x07030602u : 0x05010400u);
+    asm volatile("" : "+v"(pair));
+    wv[i >> 1][2 * (i & 1) + (kOp & 1)] = pair;
+  }
+}
+// Share kSlot of kSlots of them.
+template <int kSlot, int kSlots, int kE, int kAt = kSlot * kDecodeOps / kSlots>
+__device__ __forceinline__ void decode_share(WeightsInTheMaking &m, uint32_t word0, uint32_t word1,
+                                             const RowTables &rows, u32x4 (&wv)[2]) {
+  if constexpr (kAt < (kSlot + 1) * kDecodeOps / kSlots) {
+    decode_op<kAt, kE>(m, word0, word1, rows, wv);
+    decode_share<kSlot, kSlots, kE, kAt + 1>(m, word0, word1, rows, wv);
+  }
 }
 
 // What the kernels share.  A workgroup owns rows 64 block .. +64 and tokens
@@ -283,7 +332,7 @@ __device__ __forceinline__ uint32_t weight_pair(uint32_t codes, int k, uint32_t 
 // 256 t + 16 (p ^ (t % 16)) of the wavefront's 16 KB.
 struct TileLane {
   int lane, half, block, t0, rows_here;
-  uint32_t min_max[2];
+  RowTables rows;
   uint32_t unit_at[2];   // byte offset of the lane's codes in window 0, per unit
   uint32_t get_at;       // of its A operand of step 0 in the wavefront's tile
 };
@@ -298,7 +347,8 @@ __device__ __forceinline__ TileLane tile_lane(const TileArgs &a) {
 #pragma unroll
   for (int j = 0; j < 2; j++) {
     const int row = l.block * kRows + j * kUnitRows + (l.lane & 31);
-    l.min_max[j] = row < a.height ? a.minmax[static_cast<int64_t>(a.matrix) * a.height + row] : 0u;
+    set_tables(l.rows, j,
+               row < a.height ? a.minmax[static_cast<int64_t>(a.matrix) * a.height + row] : 0u);
     l.unit_at[j] = static_cast<uint32_t>(j * a.windows * 1024 + l.lane * 16);
   }
   l.get_at = static_cast<uint32_t>((l.lane & 31) * 256 + ((l.half ^ (l.lane & 15)) << 4));
@@ -335,16 +385,15 @@ __device__ __forceinline__ void window_steps(const unsigned char *tile, const Ti
   u32x4 wv[2];
 #pragma unroll
   for (int i = 0; i < 2; i++) xa[i] = *reinterpret_cast<const bf16x8 *>(get + i * (32 * 256));
-#pragma unroll
-  for (int j = 0; j < 2; j++)
-#pragma unroll
-    for (int k = 0; k < 4; k++) wv[j][k] = weight_pair(codes[j][0], k, l.min_max[j]);
+  WeightsInTheMaking m;
+  decode_share<0, 1, 0>(m, codes[0][0], codes[1][0], l.rows, wv);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int s = 0; s < kSteps; s++) {
     bf16x8 xa_next[2];
     u32x4 wv_next[2];
     const int sn = s + 1 < kSteps ? s + 1 : s;   // after the last step nothing new
+    const uint32_t word0 = codes[0][sn >> 1], word1 = codes[1][sn >> 1];
     if (s + 1 < kSteps) {
 #pragma unroll
       for (int i = 0; i < 2; i++)
@@ -352,18 +401,22 @@ __device__ __forceinline__ void window_steps(const unsigned char *tile, const Ti
             tile + (l.get_at ^ static_cast<uint32_t>(32 * sn)) + i * (32 * 256));
     }
     const bf16x8 wb0 = __builtin_bit_cast(bf16x8, wv[0]), wb1 = __builtin_bit_cast(bf16x8, wv[1]);
-#pragma unroll
-    for (int quarter = 0; quarter < 4; quarter++) {
-      const int i = quarter >> 1, j = quarter & 1;
-      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[i], j ? wb1 : wb0, acc[i][j], 0, 0, 0);
+    auto next_weights = [&](auto slot) {
+      constexpr int kSlot = decltype(slot)::value;
       if (s + 1 < kSteps) {
-        const int jn = quarter >> 1, k0 = 2 * (quarter & 1);
-#pragma unroll
-        for (int k = k0; k < k0 + 2; k++)
-          wv_next[jn][k] = weight_pair(codes[jn][sn >> 1], 4 * (sn & 1) + k, l.min_max[jn]);
+        if (sn & 1) decode_share<kSlot, 4, 1>(m, word0, word1, l.rows, wv_next);
+        else decode_share<kSlot, 4, 0>(m, word0, word1, l.rows, wv_next);
       }
       __builtin_amdgcn_sched_barrier(0);
-    }
+    };
+    acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[0], wb0, acc[0][0], 0, 0, 0);
+    next_weights(std::integral_constant<int, 0>{});
+    acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[0], wb1, acc[0][1], 0, 0, 0);
+    next_weights(std::integral_constant<int, 1>{});
+    acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[1], wb0, acc[1][0], 0, 0, 0);
+    next_weights(std::integral_constant<int, 2>{});
+    acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[1], wb1, acc[1][1], 0, 0, 0);
+    next_weights(std::integral_constant<int, 3>{});
     if (s + 1 < kSteps) {
       xa[0] = xa_next[0];
       xa[1] = xa_next[1];
@@ -377,22 +430,24 @@ __device__ __forceinline__ void window_steps(const unsigned char *tile, const Ti
 // rounded to bf16 and added onto y in bf16 (reference sub1_cuda_kernel.cu:199-
 // 200).  The wavefronts share the tokens, a lane has row `lane` of the block;
 // the y of a lane's tokens are all requested before anything else (tokens past
-// the last: loads that return zero, stores that are dropped).  `partial` is
+// the last: loads that return zero, stores that are dropped; a fresh y: an empty
+// buffer, and the sum is added onto zero as it would be after a fill).  `partial` is
 // LDS that no wavefront reads any more.  kPer = 64 / waves.
 template <int kPer>
 __device__ __forceinline__ void finish_tile(const TileArgs &a, const TileLane &l, int wave,
                                             int waves, float *partial, const f32x16 (&acc)[2][2]) {
   const int row = l.block * kRows + l.lane;
-  const __amdgpu_buffer_rsrc_t yb = buffer_over(
-      a.y + static_cast<int64_t>(l.t0) * a.ldy,
-      static_cast<uint32_t>((static_cast<int64_t>(l.rows_here - 1) * a.ldy + a.height) * 2));
+  const uint32_t y_bytes =
+      static_cast<uint32_t>((static_cast<int64_t>(l.rows_here - 1) * a.ldy + a.height) * 2);
+  uint16_t *y = a.y + static_cast<int64_t>(l.t0) * a.ldy;
+  const __amdgpu_buffer_rsrc_t yb = buffer_over(y, y_bytes), was = buffer_over(y, a.fresh ? 0u : y_bytes);
   // rows past the height: outside the buffer
   const uint32_t y_at = row < a.height ? static_cast<uint32_t>(row * 2) : kOutside;
   const uint32_t y_step = static_cast<uint32_t>(a.ldy * 2);
   uint16_t before[kPer];
 #pragma unroll
   for (int k = 0; k < kPer; k++)
-    before[k] = __builtin_amdgcn_raw_buffer_load_b16(yb, y_at + (wave + k * waves) * y_step, 0, 0);
+    before[k] = __builtin_amdgcn_raw_buffer_load_b16(was, y_at + (wave + k * waves) * y_step, 0, 0);
   // Element (token i, row j) of an accumulator block sits in lane
   // j + 32 * ((i / 4) % 2), register 4 * (i / 8) + i % 4.
   float *mine = partial + wave * (kTokens * kRows);
@@ -516,30 +571,33 @@ __device__ __forceinline__ void window_steps_counted(uint32_t tile, uint32_t blo
   lds_request<32 * 256>(get, xa[0], xa[1]);
   lds_arrived(codes[0], codes[1]);
   lds_arrived(xa[0], xa[1]);
-#pragma unroll
-  for (int j = 0; j < 2; j++)
-#pragma unroll
-    for (int k = 0; k < 4; k++) wv[j][k] = weight_pair(codes[j][0], k, l.min_max[j]);
+  WeightsInTheMaking m;
+  decode_share<0, 1, 0>(m, codes[0][0], codes[1][0], l.rows, wv);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int s = 0; s < kSteps; s++) {
     u32x4 xa_next[2], wv_next[2];
     const int sn = s + 1 < kSteps ? s + 1 : s;   // after the last step nothing new
+    const uint32_t word0 = codes[0][sn >> 1], word1 = codes[1][sn >> 1];
     if (s + 1 < kSteps) lds_request<32 * 256>(get ^ static_cast<uint32_t>(32 * sn), xa_next[0], xa_next[1]);
     const bf16x8 wb0 = __builtin_bit_cast(bf16x8, wv[0]), wb1 = __builtin_bit_cast(bf16x8, wv[1]);
     const bf16x8 xa0 = __builtin_bit_cast(bf16x8, xa[0]), xa1 = __builtin_bit_cast(bf16x8, xa[1]);
-#pragma unroll
-    for (int quarter = 0; quarter < 4; quarter++) {
-      const int i = quarter >> 1, j = quarter & 1;
-      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(i ? xa1 : xa0, j ? wb1 : wb0, acc[i][j], 0, 0, 0);
+    auto next_weights = [&](auto slot) {
+      constexpr int kSlot = decltype(slot)::value;
       if (s + 1 < kSteps) {
-        const int jn = quarter >> 1, k0 = 2 * (quarter & 1);
-#pragma unroll
-        for (int k = k0; k < k0 + 2; k++)
-          wv_next[jn][k] = weight_pair(codes[jn][sn >> 1], 4 * (sn & 1) + k, l.min_max[jn]);
+        if (sn & 1) decode_share<kSlot, 4, 1>(m, word0, word1, l.rows, wv_next);
+        else decode_share<kSlot, 4, 0>(m, word0, word1, l.rows, wv_next);
       }
       __builtin_amdgcn_sched_barrier(0);
-    }
+    };
+    acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa0, wb0, acc[0][0], 0, 0, 0);
+    next_weights(std::integral_constant<int, 0>{});
+    acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa0, wb1, acc[0][1], 0, 0, 0);
+    next_weights(std::integral_constant<int, 1>{});
+    acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa1, wb0, acc[1][0], 0, 0, 0);
+    next_weights(std::integral_constant<int, 2>{});
+    acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa1, wb1, acc[1][1], 0, 0, 0);
+    next_weights(std::integral_constant<int, 3>{});
     if (s + 1 < kSteps) {
       lds_arrived(xa_next[0], xa_next[1]);
       xa[0] = xa_next[0];
@@ -559,7 +617,7 @@ void matvec_tiles_kernel(TileArgs a) {
   const TileLane l = tile_lane(a);
   const Fetch f = fetch_of(a, l.lane);
   // (the rows' min and max are waited for here, while nothing else is on its way)
-  asm volatile("" ::"v"(l.min_max[0]), "v"(l.min_max[1]));
+  asm volatile("" ::"v"(l.rows.lo[0]), "v"(l.rows.lo[1]));
   const lds_bytes my_tiles = (lds_bytes)tiles + wave * kTileBytes;
   const lds_bytes my_blocks = (lds_bytes)blocks + wave * kBlockBytes;
   const int last = a.windows - 1;
@@ -669,31 +727,6 @@ struct StepOperands {
   u32x4 wv[2];
 };
 
-// The B operands of a step in the making: the eight pairs of weights of a
-// wavefront's two units go through four stages (shift, mask, selector, pick),
-// and each stage of a group of pairs is issued together, so that no
-// instruction has to wait for the one just before it.
-struct PairsInTheMaking {
-  uint32_t v[8];
-};
-template <int kStage, int kE>
-__device__ __forceinline__ void pair_stage(PairsInTheMaking &t, int p, uint32_t word0, uint32_t word1,
-                                           const uint32_t (&min_max)[2], u32x4 (&wv)[2]) {
-  const int q = 4 * kE + (p & 3);   // the pair's place in its word
-  if (kStage == 0) t.v[p] = (p >> 2 ? word1 : word0) >> (2 * q);
-  if (kStage == 1) t.v[p] &= 0x00030003u;
-  if (kStage == 2) t.v[p] = __umul24(t.v[p], 0x0202u) + 0x01000100u;
-  if (kStage == 3) wv[p >> 2][p & 3] = __builtin_amdgcn_perm(0u, min_max[p >> 2], t.v[p]);
-}
-// (keeps a stage where it was written: what it produced is not known before)
-__device__ __forceinline__ void settle(PairsInTheMaking &t, int from, int count) {
-  if (count == 8)
-    asm volatile("" : "+v"(t.v[0]), "+v"(t.v[1]), "+v"(t.v[2]), "+v"(t.v[3]), "+v"(t.v[4]), "+v"(t.v[5]),
-                 "+v"(t.v[6]), "+v"(t.v[7]));
-  else
-    asm volatile("" : "+v"(t.v[from]), "+v"(t.v[from + 1]), "+v"(t.v[from + 2]), "+v"(t.v[from + 3]));
-}
-
 // One step: 2 kLive MFMAs on `now`.  Each MFMA is followed by an equal share
 // of the work for the step after it, which the matrix core's time covers: the
 // B operands from half kE of `word0` and `word1` (the codes of the two units),
@@ -702,64 +735,34 @@ __device__ __forceinline__ void settle(PairsInTheMaking &t, int from, int count)
 // fences keep every MFMA ahead of the work that hides behind it.
 template <int kLive, int kNB, int kE, int kStride = 8192, class Extra>
 __device__ __forceinline__ void tile_step(StepOperands<kLive> &now, uint32_t next_get,
-                                          uint32_t word0, uint32_t word1,
-                                          const uint32_t (&min_max)[2], f32x16 (&acc)[kNB][2],
-                                          Extra &&extra) {
+                                          uint32_t word0, uint32_t word1, const RowTables &rows,
+                                          f32x16 (&acc)[kNB][2], Extra &&extra) {
   StepOperands<kLive> next;
-  PairsInTheMaking t;
+  WeightsInTheMaking making;
   // (nothing that derives from the words is to be computed before this step)
   asm volatile("" : "+v"(word0), "+v"(word1));
   lds_request_blocks<kLive, kStride>(next_get, next.xa);
   const bf16x8 wb0 = __builtin_bit_cast(bf16x8, now.wv[0]), wb1 = __builtin_bit_cast(bf16x8, now.wv[1]);
   __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int m = 0; m < 2 * kLive; m++) {
-    const int i = m >> 1, j = m & 1;
-    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, now.xa[i]),
-                                                         j ? wb1 : wb0, acc[i][j], 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (kLive == 4) {
-      // eight MFMAs: stage m % 4 of the pairs of unit m / 4
-      const int from = 4 * (m >> 2);
-#pragma unroll
-      for (int p = from; p < from + 4; p++) {
-        if ((m & 3) == 0) pair_stage<0, kE>(t, p, word0, word1, min_max, next.wv);
-        if ((m & 3) == 1) pair_stage<1, kE>(t, p, word0, word1, min_max, next.wv);
-        if ((m & 3) == 2) pair_stage<2, kE>(t, p, word0, word1, min_max, next.wv);
-        if ((m & 3) == 3) pair_stage<3, kE>(t, p, word0, word1, min_max, next.wv);
-      }
-      if ((m & 3) != 3) settle(t, from, 4);
-      else asm volatile("" : "+v"(next.wv[m >> 2]));
-    } else if constexpr (kLive == 2) {
-      // four MFMAs: stage m of all eight pairs
-#pragma unroll
-      for (int p = 0; p < 8; p++) {
-        if (m == 0) pair_stage<0, kE>(t, p, word0, word1, min_max, next.wv);
-        if (m == 1) pair_stage<1, kE>(t, p, word0, word1, min_max, next.wv);
-        if (m == 2) pair_stage<2, kE>(t, p, word0, word1, min_max, next.wv);
-        if (m == 3) pair_stage<3, kE>(t, p, word0, word1, min_max, next.wv);
-      }
-      if (m != 3) settle(t, 0, 8);
-      else asm volatile("" : "+v"(next.wv[0]), "+v"(next.wv[1]));
-    } else {
-      // two MFMAs: two stages of all eight pairs behind each
-#pragma unroll
-      for (int p = 0; p < 8; p++) {
-        if (m == 0) pair_stage<0, kE>(t, p, word0, word1, min_max, next.wv);
-        else pair_stage<2, kE>(t, p, word0, word1, min_max, next.wv);
-      }
-      settle(t, 0, 8);
-#pragma unroll
-      for (int p = 0; p < 8; p++) {
-        if (m == 0) pair_stage<1, kE>(t, p, word0, word1, min_max, next.wv);
-        else pair_stage<3, kE>(t, p, word0, word1, min_max, next.wv);
-      }
-      if (m == 0) settle(t, 0, 8);
-      else asm volatile("" : "+v"(next.wv[0]), "+v"(next.wv[1]));
+  auto slot = [&](auto m_c) {
+    constexpr int m = decltype(m_c)::value;
+    if constexpr (m < 2 * kLive) {
+      acc[m >> 1][m & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          __builtin_bit_cast(bf16x8, now.xa[m >> 1]), m & 1 ? wb1 : wb0, acc[m >> 1][m & 1], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      decode_share<m, 2 * kLive, kE>(making, word0, word1, rows, next.wv);
+      extra(m);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    extra(m);
-    __builtin_amdgcn_sched_barrier(0);
-  }
+  };
+  slot(std::integral_constant<int, 0>{});
+  slot(std::integral_constant<int, 1>{});
+  slot(std::integral_constant<int, 2>{});
+  slot(std::integral_constant<int, 3>{});
+  slot(std::integral_constant<int, 4>{});
+  slot(std::integral_constant<int, 5>{});
+  slot(std::integral_constant<int, 6>{});
+  slot(std::integral_constant<int, 7>{});
   lds_arrived_blocks<kLive>(next.xa);
   now = next;
 }
@@ -786,7 +789,8 @@ void matvec_tiles_shared_kernel(TileArgs a) {
 #pragma unroll
   for (int j = 0; j < 2; j++) {
     const int row = l.block * kRows + j * kUnitRows + (l.lane & 31);
-    l.min_max[j] = row < a.height ? a.minmax[static_cast<int64_t>(a.matrix) * a.height + row] : 0u;
+    set_tables(l.rows, j,
+               row < a.height ? a.minmax[static_cast<int64_t>(a.matrix) * a.height + row] : 0u);
     l.unit_at[j] = static_cast<uint32_t>(j * a.windows * 1024 + l.lane * 16);
   }
   l.get_at = static_cast<uint32_t>((l.lane & 31) * 256 + ((l.half ^ (l.lane & 15)) << 4));
@@ -859,10 +863,8 @@ void matvec_tiles_shared_kernel(TileArgs a) {
     constexpr int kPerSlot = (kLoads + kSlots - 1) / kSlots;   // loads issued behind each
     StepOperands<kLive> now;
     lds_request_blocks<kLive>(tile_at[0], now.xa);
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int q = 0; q < 4; q++) now.wv[j][q] = weight_pair(codes_a[j][0], q, l.min_max[j]);
+    WeightsInTheMaking first;
+    decode_share<0, 1, 0>(first, codes_a[0][0], codes_a[1][0], l.rows, now.wv);
     lds_arrived_blocks<kLive>(now.xa);
     auto nothing = [](int) {};
     // one window: the tile and codes `cur`, then on to `nxt`
@@ -872,19 +874,19 @@ void matvec_tiles_shared_kernel(TileArgs a) {
       const __amdgpu_buffer_rsrc_t x2 = tokens_of(a, l, w2 < a.windows);
       if (has_rows && w < a.windows) {
         const uint32_t get = tile_at[cur];
-        tile_step<kLive, kNB, 1>(now, get ^ 32u, codes_cur[0][0], codes_cur[1][0], l.min_max, acc, nothing);
-        tile_step<kLive, kNB, 0>(now, get ^ 64u, codes_cur[0][1], codes_cur[1][1], l.min_max, acc, nothing);
-        tile_step<kLive, kNB, 1>(now, get ^ 96u, codes_cur[0][1], codes_cur[1][1], l.min_max, acc, nothing);
-        tile_step<kLive, kNB, 0>(now, get ^ 128u, codes_cur[0][2], codes_cur[1][2], l.min_max, acc, nothing);
-        tile_step<kLive, kNB, 1>(now, get ^ 160u, codes_cur[0][2], codes_cur[1][2], l.min_max, acc, nothing);
-        tile_step<kLive, kNB, 0>(now, get ^ 192u, codes_cur[0][3], codes_cur[1][3], l.min_max, acc, nothing);
-        tile_step<kLive, kNB, 1>(now, get ^ 224u, codes_cur[0][3], codes_cur[1][3], l.min_max, acc, nothing);
+        tile_step<kLive, kNB, 1>(now, get ^ 32u, codes_cur[0][0], codes_cur[1][0], l.rows, acc, nothing);
+        tile_step<kLive, kNB, 0>(now, get ^ 64u, codes_cur[0][1], codes_cur[1][1], l.rows, acc, nothing);
+        tile_step<kLive, kNB, 1>(now, get ^ 96u, codes_cur[0][1], codes_cur[1][1], l.rows, acc, nothing);
+        tile_step<kLive, kNB, 0>(now, get ^ 128u, codes_cur[0][2], codes_cur[1][2], l.rows, acc, nothing);
+        tile_step<kLive, kNB, 1>(now, get ^ 160u, codes_cur[0][2], codes_cur[1][2], l.rows, acc, nothing);
+        tile_step<kLive, kNB, 0>(now, get ^ 192u, codes_cur[0][3], codes_cur[1][3], l.rows, acc, nothing);
+        tile_step<kLive, kNB, 1>(now, get ^ 224u, codes_cur[0][3], codes_cur[1][3], l.rows, acc, nothing);
         // the next window is there (this wavefront's share of it, and after
         // the barrier everyone's), and everyone has read the last of this one
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         const uint32_t word0 = codes_nxt[0][0], word1 = codes_nxt[1][0];
-        tile_step<kLive, kNB, 0>(now, tile_at[cur ^ 1], word0, word1, l.min_max, acc, [&](int m) {
+        tile_step<kLive, kNB, 0>(now, tile_at[cur ^ 1], word0, word1, l.rows, acc, [&](int m) {
 #pragma unroll
           for (int u = m * kPerSlot; u < (m + 1) * kPerSlot && u < kLoads; u++) issue_x(x2, w2, cur, u);
           if (m == kSlots - 1) issue_codes(w2, codes_cur);
@@ -913,9 +915,10 @@ void matvec_tiles_shared_kernel(TileArgs a) {
   float *sums = reinterpret_cast<float *>(shared_tiles);   // [wavefront][32 tokens][64 rows]
   const int pair = l.lane & 31;                            // rows 2 pair, 2 pair + 1 of the group
   const int row = l.block * kRows + 2 * pair;
-  const __amdgpu_buffer_rsrc_t yb = buffer_over(
-      a.y + static_cast<int64_t>(l.t0) * a.ldy,
-      static_cast<uint32_t>((static_cast<int64_t>(l.rows_here - 1) * a.ldy + a.height) * 2));
+  const uint32_t y_bytes =
+      static_cast<uint32_t>((static_cast<int64_t>(l.rows_here - 1) * a.ldy + a.height) * 2);
+  uint16_t *y = a.y + static_cast<int64_t>(l.t0) * a.ldy;
+  const __amdgpu_buffer_rsrc_t yb = buffer_over(y, y_bytes), was = buffer_over(y, a.fresh ? 0u : y_bytes);
   const uint32_t y_at = has_rows && row < a.height ? static_cast<uint32_t>(row * 2) : kOutside;
   const uint32_t y_step = static_cast<uint32_t>(a.ldy * 2);
   constexpr int kMine = 16 / kKP;   // pairs of tokens of a block that this wavefront finishes
@@ -926,7 +929,7 @@ void matvec_tiles_shared_kernel(TileArgs a) {
 #pragma unroll
     for (int n = 0; n < kMine; n++)
       before[n] = __builtin_amdgcn_raw_buffer_load_b32(
-          yb, y_at + (32 * i + k * (32 / kKP) + 2 * n + l.half) * y_step, 0, 0);
+          was, y_at + (32 * i + k * (32 / kKP) + 2 * n + l.half) * y_step, 0, 0);
     // Element (token t, row r) of an accumulator block sits in lane
     // r + 32 * ((t / 4) % 2), register 4 * (t / 8) + t % 4.
     float *mine = sums + wave * (32 * kRows);
@@ -946,11 +949,10 @@ void matvec_tiles_shared_kernel(TileArgs a) {
         lo += at[part * kRG * (32 * kRows)];
         hi += at[part * kRG * (32 * kRows) + 1];
       }
-      const uint32_t was = before[n];
       const uint32_t now =
-          static_cast<uint32_t>(f32_to_bf16(bf16_to_f32(static_cast<uint16_t>(was & 0xffffu)) +
+          static_cast<uint32_t>(f32_to_bf16(bf16_to_f32(static_cast<uint16_t>(before[n] & 0xffffu)) +
                                             bf16_to_f32(f32_to_bf16(lo)))) |
-          static_cast<uint32_t>(f32_to_bf16(bf16_to_f32(static_cast<uint16_t>(was >> 16)) +
+          static_cast<uint32_t>(f32_to_bf16(bf16_to_f32(static_cast<uint16_t>(before[n] >> 16)) +
                                             bf16_to_f32(f32_to_bf16(hi)))) << 16;
       __builtin_amdgcn_raw_buffer_store_b32(now, yb, y_at + (32 * i + t) * y_step, 0, 0);
     }
@@ -1186,9 +1188,10 @@ extern "C" int sub1_tiles_entries(const sub1_matrix_set *ms, const sub1_tiles *t
   return SUB1_OK;
 }
 
-extern "C" int sub1_matvec_tiles(const sub1_tiles *t, int matrix, const void *x, int64_t ldx,
-                                 void *y, int64_t ldy, int tokens, void *stream) {
-  const char *who = "sub1_matvec_tiles";
+namespace {
+
+int launch_product(const sub1_tiles *t, int matrix, const void *x, int64_t ldx, void *y, int64_t ldy,
+                   int tokens, bool fresh, void *stream, const char *who) {
   if (tokens == 0) return SUB1_OK;
   int rc = check_tiles(t, who);
   if (rc) return rc;
@@ -1214,6 +1217,7 @@ extern "C" int sub1_matvec_tiles(const sub1_tiles *t, int matrix, const void *x,
   a.units_down = l.units_down;
   a.windows = l.windows;
   a.matrix = matrix;
+  a.fresh = fresh;
   const bool wide = !misaligned(x, 16) && ldx % 8 == 0 && t->width % 8 == 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (ldx >= (1 << 24) || ldy >= (1 << 24))
@@ -1245,6 +1249,18 @@ extern "C" int sub1_matvec_tiles(const sub1_tiles *t, int matrix, const void *x,
   else launch_tiles<4>(a, wide, grid, s);
   HIP_TRY(hipGetLastError());
   return SUB1_OK;
+}
+
+}  // namespace
+
+extern "C" int sub1_matvec_tiles(const sub1_tiles *t, int matrix, const void *x, int64_t ldx,
+                                 void *y, int64_t ldy, int tokens, void *stream) {
+  return launch_product(t, matrix, x, ldx, y, ldy, tokens, false, stream, "sub1_matvec_tiles");
+}
+
+extern "C" int sub1_product_tiles(const sub1_tiles *t, int matrix, const void *x, int64_t ldx,
+                                  void *y, int64_t ldy, int tokens, void *stream) {
+  return launch_product(t, matrix, x, ldx, y, ldy, tokens, true, stream, "sub1_product_tiles");
 }
 
 extern "C" int sub1_test_tiles_kernel(int which) {

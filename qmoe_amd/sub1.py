@@ -97,19 +97,18 @@ class Sub1Linear(nn.Module):
 
     def forward(self, x):
         """x bf16 [T, width] -> bf16 [T, height] (reference sub1.py:132-143)."""
+        tokens = x.shape[0]
+        if self.fast and tokens:
+            if self.tile_tokens is not None and tokens >= self.tile_tokens:
+                return self._copy('tiles', x.shape[1]).product_tokens(x.contiguous())
+            if tokens > self.packed_tokens and x.shape[1] <= sub1_hip.PREPARED_MAX_WIDTH:
+                return self._prepared(x.shape[1]).product_tokens(x.contiguous())
         height = self.row_off.shape[0] - 1
-        y = torch.zeros((x.shape[0], height), dtype=torch.bfloat16, device=x.device)
-        if x.shape[0] == 0:
-            return y
-        x = x.contiguous()
-        if self.fast and self.tile_tokens is not None and x.shape[0] >= self.tile_tokens:
-            self._copy('tiles', x.shape[1]).matvec_tokens(x, y)
-        elif (self.fast and x.shape[0] > self.packed_tokens
-              and x.shape[1] <= sub1_hip.PREPARED_MAX_WIDTH):
-            self._prepared(x.shape[1]).matvec_tokens(x, y)
-        else:
+        y = torch.zeros((tokens, height), dtype=torch.bfloat16, device=x.device)
+        if tokens:
             table = DEC[self.w_comp.device.index]
-            sub1_hip.sub1matvec_tokens(table, self.w_comp, self.row_off, self.ter_minmax, x, y)
+            sub1_hip.sub1matvec_tokens(table, self.w_comp, self.row_off, self.ter_minmax,
+                                       x.contiguous(), y)
         return y
 
     @staticmethod

@@ -523,6 +523,23 @@ class PreparedMatrix:
             _lib.check(_lib.load().sub1_matvec_prepared(
                 ctypes.byref(self._c), p_tm, p_x, self.width, p_y, self.height, tokens, _stream()))
 
+    def product_tokens(self, x):
+        """W x[t] for all tokens of x [T, width] into a new tensor: what
+        matvec_tokens adds onto zeros, without the fill.  One matrix."""
+        p_x = _need(x, torch.bfloat16, 'x', self.device, dim=2)
+        tokens = x.shape[0]
+        if x.shape[1] != self.width:
+            raise ValueError('x must be [T, %d]' % self.width)
+        if self.count > 1:
+            raise ValueError('token_matrix is required with %d matrices' % self.count)
+        y = torch.empty((tokens, self.height), dtype=torch.bfloat16, device=self.device)
+        if tokens:
+            with _on_device(self.device):
+                _lib.check(_lib.load().sub1_product_prepared(
+                    ctypes.byref(self._c), p_x, self.width, y.data_ptr(), self.height, tokens,
+                    _stream()))
+        return y
+
     def decode(self, matrix=0):
         """uint8 [height, width]: the symbols of one matrix read back from the
         prepared stream."""
@@ -584,6 +601,21 @@ class TiledMatrix:
         with _on_device(dev):
             _lib.check(_lib.load().sub1_matvec_tiles(
                 ctypes.byref(self._c), matrix, p_x, self.width, p_y, self.height, tokens, _stream()))
+
+    def product_tokens(self, x, matrix=0):
+        """W x[t] for all tokens of x [T, width] into a new tensor: what
+        matvec_tokens adds onto zeros, without the fill."""
+        p_x = _need(x, torch.bfloat16, 'x', self.device, dim=2)
+        tokens = x.shape[0]
+        if x.shape[1] != self.width:
+            raise ValueError('x must be [T, %d]' % self.width)
+        y = torch.empty((tokens, self.height), dtype=torch.bfloat16, device=self.device)
+        if tokens:
+            with _on_device(self.device):
+                _lib.check(_lib.load().sub1_product_tiles(
+                    ctypes.byref(self._c), matrix, p_x, self.width, y.data_ptr(), self.height, tokens,
+                    _stream()))
+        return y
 
     def decode(self, matrix=0):
         """uint8 [height, width]: the symbols of one matrix read back from the

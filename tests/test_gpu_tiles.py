@@ -305,3 +305,31 @@ def test_tiles_multiply_zero_weights_like_the_reference(gpu, oracle):
     assert torch.equal(w_inf[3][no_weight], w_clean[3][no_weight])
     assert not torch.isfinite(w_inf[3][~no_weight].float()).any()
     assert torch.equal(w_inf[others], w_clean[others])
+
+
+@pytest.mark.parametrize('height,width,tokens', [(256, 520, 1), (256, 520, 129), (4096, 1024, 1200),
+                                                 (77, 333, 100), (131, 264, 67)])
+def test_a_product_into_a_new_tensor_is_the_sum_onto_zeros(gpu, oracle, height, width, tokens):
+    """product_tokens neither fills nor reads what it writes: the bits of
+    matvec_tokens on zeros, also where a result is a negative zero (0 + -0 is 0)
+    and where the memory held NaN, for every kernel of both forms."""
+    sub1, op = gpu
+    from qmoe_amd import _lib
+    c = dev_case(oracle, height, width, 0.9, seed=height + tokens)
+    rng = np.random.default_rng(tokens)
+    xs = rng.standard_normal((tokens, width)).astype(np.float32)
+    xs[tokens // 2] *= 1e-40                          # results round to zeros of either sign
+    x = bf16_dev(so.f32_to_bf16_bits(xs))
+    for make in (op.TiledMatrix, op.PreparedMatrix):
+        m = make(sub1.DEC[0], c['w_comp'], c['row_off_d'], c['mm_d'], width)
+        for which in (0, 1, 2, 3) if make is op.TiledMatrix else (0,):
+            _lib.check(_lib.load().sub1_test_tiles_kernel(which))
+            try:
+                want = torch.zeros((tokens, height), dtype=torch.bfloat16, device='cuda')
+                m.matvec_tokens(x, want)
+                held = torch.full((tokens, height), float('nan'), dtype=torch.bfloat16, device='cuda')
+                del held                              # what torch hands out next
+                got = m.product_tokens(x)
+            finally:
+                _lib.check(_lib.load().sub1_test_tiles_kernel(0))
+            assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (make.__name__, which)
