@@ -321,6 +321,35 @@ int sub1_moe_grouped_prepared(const sub1_moe_prepared *prepared, const int32_t *
                               const void *x, void *y, int tokens, void *workspace,
                               int64_t workspace_bytes, void *stream);
 
+/*
+ * sub1_moe_grouped_prepared for batches with many tokens per expert, on the matrix
+ * cores: tokens are grouped by expert on the GPU, a slice of 64 rows is expanded from
+ * the prepared stream into LDS once for up to 64 of them, and multiplied there.  The
+ * reference calls one product per token (sub1.py:139-142, 312-317).  Same semantics and
+ * same workspace (control words); a row's result is the same fp32 sum of products
+ * that are exact, taken in the matrix cores' order, so it agrees with
+ * sub1_moe_grouped_prepared to rounding, not to the bit; it does not depend on the
+ * other tokens.  Tokens whose x or h hold an infinity or NaN go through the walking
+ * kernel, with its results.  y may be x.
+ *
+ * scratch: sub1_moe_batch_scratch_bytes(p, tokens) bytes of device memory, 256-byte
+ * aligned, contents arbitrary before and after (0: no such form for these shapes - a
+ * row's codes must fit LDS - and the call is refused).  It stops growing at 8192
+ * tokens: larger batches run in equal pieces.
+ *
+ * sub1_moe_batch_pays: 1 where this is estimated to be faster than
+ * sub1_moe_grouped_prepared for `tokens` tokens spread over the experts (from about 16
+ * tokens an expert on, never below 8), 0 otherwise.
+ */
+int64_t sub1_moe_batch_scratch_bytes(const sub1_moe_prepared *prepared, int tokens);
+
+int sub1_moe_batch_pays(const sub1_moe_prepared *prepared, int tokens);
+
+int sub1_moe_batch_prepared(const sub1_moe_prepared *prepared, const int32_t *token_expert,
+                            const void *x, void *y, int tokens, void *workspace,
+                            int64_t workspace_bytes, void *scratch, int64_t scratch_bytes,
+                            void *stream);
+
 int sub1_moe_prepared_decode(const sub1_moe_prepared *prepared, int expert, int projection,
                              void *tern_out, void *stream);
 

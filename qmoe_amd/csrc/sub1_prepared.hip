@@ -2292,6 +2292,8 @@ __global__ __launch_bounds__(kMaxThreads) void matvec_group_kernel(PreparedArgs 
   }
 }
 
+#include "sub1_batch.h"
+
 // ------------------------------------------------------------ host side --
 
 // The prepare kernels read dec as the fixed dictionary's table (symbols 0..2,
@@ -3160,6 +3162,194 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
   return SUB1_OK;
 }
 
+// ---- batches on the matrix cores (sub1_batch.h) ----
+
+// The scratch memory of a piece, arrays back to back, 256-byte aligned.
+struct BatchLayout {
+  int64_t totals, slots, spoiled, block_expert, chunks, tiles;
+  int64_t x, h_rows, h;   // y's rows take x's place, which is done with by then
+  int64_t bytes;
+  int max_blocks, max_chunks;
+};
+
+BatchLayout batch_layout(const Prepared &p, int tokens) {
+  BatchLayout b;
+  const int64_t hit = std::min(tokens, p.count);
+  // every bucket's tokens (the experts hit, and one of tokens without an expert) fill
+  // all of their blocks but the last
+  b.max_blocks = static_cast<int>((tokens + (kBlockTokens - 1) * (hit + 1)) / kBlockTokens);
+  b.max_chunks = static_cast<int>((b.max_blocks + (kChunkBlocks - 1) * hit) / kChunkBlocks);
+  int64_t off = 0;
+  auto take = [&](int64_t bytes) {
+    const int64_t o = off;
+    off += align256(bytes);
+    return o;
+  };
+  const int64_t blocks = b.max_blocks, slots = blocks * kBlockTokens;
+  b.totals = take(kTotalWords * 4);
+  b.slots = take(slots * 4);
+  b.spoiled = take(slots * 4);
+  b.block_expert = take(blocks * 4);
+  b.chunks = take((static_cast<int64_t>(b.max_chunks) + 7) / 8 * 8 * 16);
+  b.tiles = take(slots * 8);
+  b.x = take(blocks * std::max(steps_of(p.width[0]) * 1024, p.height[1] * kBlockTokens * 2));
+  b.h_rows = take(blocks * p.height[0] * kBlockTokens * 2);
+  b.h = take(blocks * steps_of(p.width[1]) * 1024);
+  b.bytes = off;
+  return b;
+}
+
+int batch_piece(int tokens) {
+  const int pieces = (tokens + kBatchPiece - 1) / kBatchPiece;
+  return (tokens + pieces - 1) / pieces;
+}
+
+// How a product's slices are given to workgroups.
+struct BatchPlan {
+  int per_group, parts;
+  size_t lds;
+};
+
+// LDS holds the codes of `fit` slices: with room for three and more, workgroups of four
+// wavefronts, one to a SIMD; for two, of eight; for one, of twelve.  (128 base experts on 4096
+// tokens: 131 us; with wi's workgroups of 8 wavefronts 134, with wo's of 6, 8 and 12
+// 142, 132 and 153.  40 c-2048 experts on 700 tokens, wo, whose codes take 98 KB, with
+// 4, 8, 12 and 16 wavefronts: 205, 166, 162 and 165.)  Wavefronts share a slice as long as
+// each gets a group of chunks, the least that one can expand, and take slices of their
+// own beyond that (c-2048 wi by 1, 2 and 4 to a slice: 208, 181, 166 us; base wi, of
+// hardly two groups, 134, 131, 144).
+bool plan_batch(const Prepared &p, int kind, size_t lds_limit, BatchPlan *out) {
+  const int slices[2] = {(p.height[0] + 63) / 64, (p.height[1] + 63) / 64};
+  const double weight = static_cast<double>(slices[0]) * p.width[0] + static_cast<double>(slices[1]) * p.width[1];
+  const double chunks = static_cast<double>(p.total_chunks) / p.count * p.width[kind] / weight;
+  const size_t code_bytes = slice_code_bytes(p.width[kind]);
+  const int fit = static_cast<int>(lds_limit / code_bytes);
+  const int waves = fit >= 3 ? 4 : fit == 2 ? 8 : 12;
+  int parts = 1;
+  while (parts < waves && parts * kGroupChunks < 0.75 * chunks) parts *= 2;
+  parts = std::min(parts, waves);
+  int per_group = std::min(waves / parts, slices[kind]);
+  for (;; per_group--) {
+    if (per_group == 0) return false;
+    const size_t sums = parts > 1 ? static_cast<size_t>(2 * per_group * parts) * 4096 : 0;
+    out->lds = std::max(per_group * code_bytes, sums);
+    if (out->lds <= lds_limit) break;
+  }
+  out->per_group = per_group;
+  out->parts = parts;
+  return true;
+}
+
+constexpr size_t kBatchLds = 160 * 1024 - 64;
+
+bool batch_takes(const Prepared &p) {
+  BatchPlan plan;
+  const size_t lds_fused = (static_cast<size_t>(activation_dwords(p.width[0])) + activation_dwords(p.width[1])) * 4;
+  return p.count <= kBatchMaxExperts && lds_fused <= kBatchLds && plan_batch(p, 0, kBatchLds, &plan) &&
+         plan_batch(p, 1, kBatchLds, &plan);
+}
+
+// Whether the matrix cores are the faster way for `tokens` tokens, by estimates fitted to
+// both at 1 to 64 tokens an expert through 8 to 128 experts of the three Switch shapes and of
+// two odd ones (80 and 95 % zeros), in microseconds.  Here: 36 and, per million weights of the experts hit, 0.03 for every
+// 64 of an expert's tokens and 0.09 for every 32 (base 128: 103 measured at 16 tokens an expert
+// and 132 at 32, 105 and 133 estimated; c-2048 40: 167 at 16, 159).  Walking: as launch_prepared has
+// it, a token on a compute unit 8 + entries / 23400, less where four tokens walk together
+// (base 128: 108, 177 and 270 at 8, 16 and 32).  The estimates are some 10 % off either way,
+// so the matrix cores must promise that much: below 8 tokens an expert they never do.
+bool batch_pays(const Prepared &p, int tokens, int cus) {
+  if (tokens < 8 * static_cast<int64_t>(p.count) || !batch_takes(p)) return false;
+  const double each = static_cast<double>(tokens) / p.count;
+  const double blocks = each / kBlockTokens + 0.5, chunks = blocks / kChunkBlocks;
+  const double weights = 2e-6 * p.count * p.height[0] * p.width[0];
+  const double batch_us = 36.0 + weights * (0.03 * std::max(1.0, chunks) + 0.09 * std::max(1.0, blocks));
+  const double token_us = 8.0 + static_cast<double>(p.total_chunks) * (64.0 * kFields) / p.count / 23400.0;
+  const bool together = tokens >= 4 * cus;
+  const double gain = together ? std::min(1.7, std::max(1.0, 0.85 + 0.027 * each)) : 1.0;
+  return 1.1 * batch_us < tokens * token_us / cus / gain;
+}
+
+int launch_batch(const Prepared &p, const int32_t *token_expert, const uint16_t *x, uint16_t *y, int tokens,
+                 int32_t *ctrl, char *scratch, hipStream_t s, const char *who) {
+  const BatchLayout b = batch_layout(p, tokens);
+  const MetaLayout m = meta_layout(p.count, p.kinds, p.height, p.width);
+  const char *meta = static_cast<const char *>(p.meta);
+  int32_t *totals = reinterpret_cast<int32_t *>(scratch + b.totals);
+  int32_t *slots = reinterpret_cast<int32_t *>(scratch + b.slots);
+  int32_t *spoiled = reinterpret_cast<int32_t *>(scratch + b.spoiled);
+  int32_t *block_expert = reinterpret_cast<int32_t *>(scratch + b.block_expert);
+  int4 *chunks = reinterpret_cast<int4 *>(scratch + b.chunks);
+  int2 *tiles = reinterpret_cast<int2 *>(scratch + b.tiles);
+  u32x4 *xs = reinterpret_cast<u32x4 *>(scratch + b.x), *hs = reinterpret_cast<u32x4 *>(scratch + b.h);
+  uint16_t *h_rows = reinterpret_cast<uint16_t *>(scratch + b.h_rows);
+  uint16_t *y_rows = reinterpret_cast<uint16_t *>(scratch + b.x);
+  const int d_model = p.width[0], d_ff = p.height[0];
+  const bool aligned = d_model % 8 == 0 && !misaligned(x, 16) && !misaligned(y, 16);
+
+  group_blocks_kernel<<<1, 1024, static_cast<size_t>(p.count + 1) * 8, s>>>(
+      token_expert, tokens, p.count, slots, spoiled, block_expert, chunks, totals, ctrl);
+  const auto shares = [](int work, int per) { return static_cast<unsigned>(std::max(1, std::min(16, (work + per - 1) / per))); };
+  pack_tokens_kernel<<<dim3(b.max_blocks, shares(steps_of(d_model), 16)), 256, 0, s>>>(
+      x, y, d_model, d_model, d_model, aligned, slots, spoiled, totals, xs);
+  const void *fn = reinterpret_cast<const void *>(batch_product_kernel);
+  PreparedArgs a = {};
+  a.stream = static_cast<const uint2 *>(p.codes);
+  a.ckpt = reinterpret_cast<const uint16_t *>(a.stream + p.total_chunks * 64);
+  int64_t first_slice = 0;
+  for (int i = 0; i < 2; i++) {
+    BatchPlan plan;
+    if (!plan_batch(p, i, kBatchLds, &plan)) return fail(SUB1_ERR_SHAPE, "%s: widths too large", who);
+    const KindMeta &k = m.k[i];
+    KindArgs &ka = a.k[i];
+    ka.slice_base = reinterpret_cast<const uint32_t *>(meta + k.slice_base);
+    ka.slice_len = reinterpret_cast<const uint16_t *>(meta + k.slice_len);
+    ka.row_idx = reinterpret_cast<const uint16_t *>(meta + k.row_idx);
+    ka.minmax = reinterpret_cast<const uint32_t *>(meta + k.minmax);
+    ka.slices = k.slices;
+    ka.height = k.height;
+    ka.width = k.width;
+    ka.first_slice = first_slice;
+    first_slice += static_cast<int64_t>(p.count) * k.slices;
+    BatchArgs b_args;
+    b_args.stream = a.stream;
+    b_args.ckpt = a.ckpt;
+    b_args.k = ka;
+    b_args.in = i ? hs : xs;
+    b_args.out = i ? y_rows : h_rows;
+    b_args.chunks = chunks;
+    b_args.totals = totals;
+    b_args.steps = steps_of(k.width);
+    b_args.parts = plan.parts;
+    b_args.per_group = plan.per_group;
+    b_args.slice_groups = (k.slices + plan.per_group - 1) / plan.per_group;
+    b_args.relu = i == 0;
+    HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(plan.lds)));
+    batch_product_kernel<<<static_cast<unsigned>((b.max_chunks + 7) / 8 * 8 * b_args.slice_groups),
+                           64 * plan.per_group * plan.parts, plan.lds, s>>>(b_args);
+    if (i == 0)
+      pack_hidden_kernel<<<dim3(b.max_blocks, shares(steps_of(d_ff), 32)), 256, 0, s>>>(h_rows, d_ff, spoiled,
+                                                                                       totals, hs);
+  }
+  unpack_tokens_kernel<<<dim3(b.max_blocks, shares(d_model, 128)), 256, 0, s>>>(
+      y_rows, y, d_model, d_model, aligned, slots, spoiled, block_expert, totals, tiles, ctrl);
+  // what the tokens listed there need of the walking kernels
+  a.order = slots;
+  a.groups = tiles;
+  a.x = x;
+  a.y = y;
+  a.ldx = a.ldy = d_model;
+  a.ctrl = ctrl;
+  a.xdwords = activation_dwords(d_model);
+  a.hdwords = activation_dwords(d_ff);
+  const size_t lds = static_cast<size_t>(a.xdwords + a.hdwords) * 4;
+  HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(walk_listed_kernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+  walk_listed_kernel<<<std::min(tokens, 256), kMaxThreads, lds, s>>>(a);
+  HIP_TRY(hipGetLastError());
+  sub1::note_kernel("batch_product_kernel");
+  return SUB1_OK;
+}
+
 // The symbols of matrix `index` of kind `kind`, read back from the stream.
 int decode_prepared(const Prepared &p, int kind, int index, void *tern_out, hipStream_t s,
                     const char *who) {
@@ -3445,6 +3635,54 @@ extern "C" int sub1_moe_grouped_prepared(const sub1_moe_prepared *p, const int32
   return launch_prepared(from_moe(p), token_expert, x, p->d_model, y, p->d_model, tokens,
                          workspace, workspace_bytes, static_cast<hipStream_t>(stream),
                          "sub1_moe_grouped_prepared");
+}
+
+extern "C" int64_t sub1_moe_batch_scratch_bytes(const sub1_moe_prepared *p, int tokens) {
+  if (!p || tokens < 1 || tokens > (1 << 20) || bad_dims(p->experts, p->d_ff, p->d_model) ||
+      bad_dims(p->experts, p->d_model, p->d_ff))
+    return 0;
+  const Prepared q = from_moe(p);
+  return batch_takes(q) ? batch_layout(q, batch_piece(tokens)).bytes : 0;
+}
+
+extern "C" int sub1_moe_batch_pays(const sub1_moe_prepared *p, int tokens) {
+  if (sub1_moe_batch_scratch_bytes(p, tokens) <= 0) return 0;
+  int device = 0, cus = 0;
+  if (hipGetDevice(&device) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1)
+    return 0;
+  return batch_pays(from_moe(p), tokens, cus);
+}
+
+extern "C" int sub1_moe_batch_prepared(const sub1_moe_prepared *p, const int32_t *token_expert, const void *x,
+                                       void *y, int tokens, void *workspace, int64_t workspace_bytes,
+                                       void *scratch, int64_t scratch_bytes, void *stream) {
+  const char *who = "sub1_moe_batch_prepared";
+  if (!p) return fail(SUB1_ERR_NULL, "%s: NULL argument", who);
+  if (tokens == 0) return SUB1_OK;
+  if (bad_dims(p->experts, p->d_ff, p->d_model) || bad_dims(p->experts, p->d_model, p->d_ff))
+    return fail(SUB1_ERR_SHAPE, "%s: experts %d d_model %d d_ff %d", who, p->experts, p->d_model, p->d_ff);
+  if (!p->meta || !p->codes || !token_expert || !x || !y || !workspace || !scratch)
+    return fail(SUB1_ERR_NULL, "%s: NULL argument", who);
+  if (tokens < 0 || tokens > (1 << 20)) return fail(SUB1_ERR_SHAPE, "%s: tokens %d outside 0..2^20", who, tokens);
+  const Prepared q = from_moe(p);
+  if (!batch_takes(q)) return fail(SUB1_ERR_SHAPE, "%s: shapes that have no such form", who);
+  const int piece = batch_piece(tokens);
+  if (scratch_bytes < batch_layout(q, piece).bytes || workspace_bytes < sub1_moe_workspace_bytes(piece, p->d_ff))
+    return fail(SUB1_ERR_SHAPE, "%s: scratch or workspace too small", who);
+  if (p->meta_bytes < moe_layout(p->experts, p->d_model, p->d_ff).bytes)
+    return fail(SUB1_ERR_SHAPE, "%s: meta smaller than its layout", who);
+  if (misaligned(p->meta, 256) || misaligned(p->codes, 256) || misaligned(token_expert, 4) || misaligned(x, 2) ||
+      misaligned(y, 2) || misaligned(workspace, 256) || misaligned(scratch, 256))
+    return fail(SUB1_ERR_ALIGN, "%s: misaligned pointer", who);
+  for (int first = 0; first < tokens; first += piece) {
+    const int64_t at = static_cast<int64_t>(first) * p->d_model;
+    const int rc = launch_batch(q, token_expert + first, static_cast<const uint16_t *>(x) + at,
+                                static_cast<uint16_t *>(y) + at, std::min(piece, tokens - first),
+                                static_cast<int32_t *>(workspace), static_cast<char *>(scratch), static_cast<hipStream_t>(stream), who);
+    if (rc) return rc;
+  }
+  return SUB1_OK;
 }
 
 extern "C" int sub1_moe_prepared_decode(const sub1_moe_prepared *p, int expert, int projection,

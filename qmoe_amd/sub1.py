@@ -201,9 +201,20 @@ class Sub1Experts(nn.Module):
             self._prepared = sub1_hip.PreparedStack.from_layers(self._dec, self._wi, self._wo)
         return self._prepared
 
+    # Batches with many tokens per expert (from about 16 on, where it is estimated to be
+    # faster) go through the matrix cores: results equal to rounding, not to the bit, to
+    # those of smaller batches.  False gives a token the same bits in every batch.
+    matrix_cores = True
+
     def forward(self, x, expert_index):
-        return self._launcher().forward(x.contiguous(),
-                                        expert_index.to(torch.int32).contiguous())
+        return _run_experts(self._launcher(), x.contiguous(),
+                            expert_index.to(torch.int32).contiguous(), self.matrix_cores)
+
+
+def _run_experts(launcher, x, route, matrix_cores):
+    if matrix_cores and isinstance(launcher, sub1_hip.PreparedStack) and launcher.batch_pays(x.shape[0]):
+        return launcher.forward_batch(x, route)
+    return launcher.forward(x, route)
 
 
 def _router_outputs(outputs, experts):
@@ -280,6 +291,8 @@ class FasterMLP(nn.Module):
             if act is not None and not isinstance(act, nn.ReLU):
                 raise ValueError('FasterMLP runs ReLU experts; this one has %r' % (act,))
 
+    matrix_cores = True     # as Sub1Experts.matrix_cores
+
     def _sentinels(self):
         # a few of the experts' tensors stand for all of them in the per-call
         # check (looking at every tensor of 2048 experts costs milliseconds)
@@ -348,7 +361,7 @@ class FasterMLP(nn.Module):
         # has an all-zero mask row: expert -1 for the launch
         route, expert_index = sub1_hip.route_from_mask(router_mask)
         x = hidden_states.reshape(-1, hidden_states.shape[-1]).to(torch.bfloat16).contiguous()
-        next_states = self._launcher().forward(x, route)
+        next_states = _run_experts(self._launcher(), x, route, self.matrix_cores)
         hidden_states = router_probs * next_states.view(hidden_states.shape).to(hidden_states.dtype)
         if self.router_outputs:
             return hidden_states, (router_logits, expert_index)

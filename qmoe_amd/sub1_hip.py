@@ -447,6 +447,44 @@ class PreparedStack:
                 _stream()))
         return y
 
+    def batch_pays(self, tokens):
+        """Whether forward_batch is estimated to be the faster one (it never is
+        below 8 tokens an expert)."""
+        if tokens < 128 or tokens < 8 * self.experts:
+            return False
+        with _on_device(self.device):
+            return bool(_lib.load().sub1_moe_batch_pays(ctypes.byref(self._c), tokens))
+
+    def forward_batch(self, x, token_expert, y=None):
+        """forward() on the matrix cores, for many tokens per expert: results
+        agree with it to rounding, not to the bit, and a token's do not depend
+        on the other tokens.  Scratch memory (about 5 d_ff + 2 d_model bytes a
+        token, up to 8192 tokens' worth) comes from torch's allocator for the
+        call."""
+        dev = self.device
+        _lib.check_faults()       # what earlier launches reported (host memory, no sync)
+        lib = _lib.load()
+        p_x = _need(x, torch.bfloat16, 'x', dev, dim=2)
+        tokens = x.shape[0]
+        if x.shape[1] != self.d_model:
+            raise ValueError('x must be [T, %d]' % self.d_model)
+        p_te = _need(token_expert, torch.int32, 'token_expert', dev, numel=tokens)
+        if y is None:
+            y = torch.empty_like(x)
+        if tokens == 0:
+            return y
+        p_y = _need(y, torch.bfloat16, 'y', dev, numel=x.numel())
+        ws = self.workspace(tokens)
+        need = lib.sub1_moe_batch_scratch_bytes(ctypes.byref(self._c), tokens)
+        if need <= 0:
+            raise ValueError('shapes that forward_batch does not take')
+        with _on_device(dev):
+            scratch = torch.empty(need, dtype=torch.uint8, device=dev)
+            _lib.check(lib.sub1_moe_batch_prepared(
+                ctypes.byref(self._c), p_te, p_x, p_y, tokens, ws.data_ptr(), ws.numel(),
+                scratch.data_ptr(), need, _stream()))
+        return y
+
     def launch_faults(self, tokens):
         """As ExpertStack.launch_faults."""
         return _fault_delta(self, tokens)

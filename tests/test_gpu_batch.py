@@ -1,0 +1,185 @@
+"""The expert layer on the matrix cores (forward_batch).
+
+The first test's numbers are small integers times powers of two, with few enough
+terms that every fp32 sum of them is exact whatever its order: the results must be
+the oracle's to the bit.  |x| <= 2 and |weights| <= 2 give |h| <= 4 width and, h
+rounded to bf16, sums of multiples of 1/4 below 8 d_model d_ff < 2^22 (at these shapes):
+24 bits hold them.  The others compare with the walking kernels; where sums are
+not exact, the two orders differ by bf16 roundings here and there: 2e-4 of the norm
+(4.5e-5 at most between any two of this library's orders)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import sub1_oracle as so
+from test_gpu_parity import bf16_dev, bits_host
+
+
+def layers(oracle, height, width, p0, seed):
+    rng = np.random.default_rng(seed)
+    share = 1 - p0 if np.isscalar(p0) else 1 - np.asarray(p0)[np.arange(height) % len(p0)][:, None]
+    t = ((rng.random((height, width)) < share) * rng.integers(1, 3, (height, width))).astype(np.int32)
+    minmax = rng.choice([0.5, 1.0, 2.0], (height, 2)) * (-1.0, 1.0)
+    return oracle.encode(t) + (so.f32_to_bf16_bits(minmax.ravel().astype(np.float32)),)
+
+
+def prepared(wi, wo):
+    from qmoe_amd import sub1, sub1_hip
+
+    def dev(layer):
+        codes, row_off, minmax = layer
+        return torch.from_numpy(codes.view(np.int16)).cuda(), torch.from_numpy(row_off).cuda(), bf16_dev(minmax)
+
+    return sub1_hip.PreparedStack.from_layers(sub1.DEC[0], [dev(l) for l in wi], [dev(l) for l in wo])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('d_model,d_ff,p0,counts', [
+    (1, 1, 0.0, [1, 0, 33]),                              # one step, a row alone in its slice
+    (15, 65, 0.5, [31, 32, 33, 64]), (16, 64, 0.5, [65, 1, 96]), (17, 63, 0.5, [2, 129, 0]),
+    (33, 130, [0.0, 1.0, 0.5], [40, 40]),                 # whole rows and empty ones
+    (768, 400, 0.9, [33, 5]), (400, 768, 0.9, [5, 64]),
+    (1100, 470, [0.9] * 63 + [0.02], [70, 3]),            # a row of many groups in every slice
+    (130, 3500, 0.98, [34]),                              # eight wavefronts to a slice
+    (66, 6200, 0.985, [65])])                             # twelve, and codes that fill LDS
+def test_exact_sums_equal_the_oracle(oracle, d_model, d_ff, p0, counts):
+    experts = len(counts)
+    wi = [layers(oracle, d_ff, d_model, p0, 10 + e) for e in range(experts)]
+    wo = [layers(oracle, d_model, d_ff, p0, 20 + e) for e in range(experts)]
+    prep = prepared(wi, wo)
+    rng = np.random.default_rng(1)
+    route = np.concatenate([np.full(n, e) for e, n in enumerate(counts)] + [[-1, experts, -7]]).astype(np.int32)
+    rng.shuffle(route)
+    xs = so.f32_to_bf16_bits(rng.integers(-2, 3, (route.size, d_model)).astype(np.float32))
+    x, te = bf16_dev(xs), torch.from_numpy(route).cuda()
+    y = prep.forward_batch(x, te)
+    assert prep.launch_faults(route.size) == (0, 1)
+    got = bits_host(y)
+    for i in range(route.size):
+        e = route[i]
+        if e < 0 or e >= experts:
+            assert np.array_equal(got[i], xs[i])
+        elif i % 7 == 0 or route.size < 50:
+            assert np.array_equal(got[i], oracle.expert_ffn(wi[e], wo[e], xs[i], order=2)[0]), (i, e)
+    # every token, and into its own input
+    assert torch.equal(prep.forward(x, te), y)
+    own = x.clone()
+    assert prep.forward_batch(own, te, y=own) is own and torch.equal(own, y)
+
+
+@pytest.mark.gpu
+def test_a_token_without_finite_activations_spoils_no_other(oracle):
+    """x with an infinity or a NaN, and x whose h overflows: what the walking kernel
+    gives for the token alone; the tokens of its block are as without it."""
+    wi = [layers(oracle, 200, 96, 0.9, 1)]
+    wo = [layers(oracle, 96, 200, 0.9, 2)]
+    prep = prepared(wi, wo)
+    x = torch.randn((70, 96), generator=torch.Generator().manual_seed(3)).bfloat16().cuda()
+    te = torch.zeros(70, dtype=torch.int32, device='cuda')
+    plain = prep.forward_batch(x, te)
+    x[3, 5] = float('inf')
+    x[40, 95] = float('nan')
+    x[41] = -float('inf')
+    x[69] = 3e38
+    y = prep.forward_batch(x, te)
+    spoiled = [3, 40, 41, 69]
+    for t in spoiled:
+        alone = prep.forward(x[t:t + 1].contiguous(), te[:1])
+        assert torch.equal(y[t].view(torch.int16), alone[0].view(torch.int16)), t
+    others = [t for t in range(70) if t not in spoiled]
+    assert torch.equal(y[others], plain[others])
+    assert torch.isfinite(y[others].float()).all()
+
+
+@pytest.mark.gpu
+def test_large_batches_through_the_layer():
+    """What Sub1Experts sends where: equal to rounding either way, a token's bits the
+    same in any batch that goes through the matrix cores, batches of several pieces,
+    views that are not aligned."""
+    from qmoe_amd import sub1, sub1_hip, synthetic
+    experts, d_model, d_ff = 12, 512, 1030
+    stack = synthetic.build_stack(experts, d_model, d_ff, 0.9, seed=4)
+    pairs = [synthetic.expert_layers(stack, e) for e in range(experts)]
+
+    def linear(buffers):
+        layer = sub1.Sub1Linear(buffers[1].numel() - 1, buffers[0].numel())
+        layer.w_comp, layer.row_off, layer.ter_minmax = buffers
+        return layer
+
+    layer = sub1.Sub1Experts([linear(p[0]) for p in pairs], [linear(p[1]) for p in pairs])
+    prep = layer._launcher()
+    last = lambda: sub1_hip._lib.load().sub1_last_kernel().decode()
+    tokens = 20000
+    x = synthetic.activations(tokens, d_model, seed=5)
+    route = synthetic.softmax_router(tokens, experts, seed=6)
+    y = layer(x, route)
+    assert last() == 'batch_product_kernel'
+    layer.matrix_cores = False
+    walked = layer(x, route)
+    assert last() != 'batch_product_kernel'
+    assert (y.float() - walked.float()).norm() <= 2e-4 * walked.float().norm()
+    assert torch.equal(prep.forward_batch(x[700:1500], route[700:1500]), y[700:1500])
+    shifted = torch.empty(1000 * d_model + 1, dtype=torch.bfloat16, device='cuda')[1:].view(1000, d_model)
+    shifted.copy_(x[:1000])
+    assert torch.equal(prep.forward_batch(shifted, route[:1000]), y[:1000])
+    one = torch.full((300,), 7, dtype=torch.int32, device='cuda')       # all to one expert
+    assert torch.equal(prep.forward_batch(x[:300], one)[route[:300] == 7], y[:300][route[:300] == 7])
+    layer.matrix_cores = True
+    layer(x[:64], route[:64])
+    assert last() != 'batch_product_kernel'
+
+
+@pytest.mark.gpu
+def test_replays_from_a_graph():
+    from qmoe_amd import synthetic
+    stack = synthetic.build_stack(4, 200, 300, 0.9, seed=7)
+    prep = stack.prepare()
+    x = synthetic.activations(150, 200, seed=8)
+    route = synthetic.softmax_router(150, 4, seed=9)
+    y = torch.empty_like(x)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        prep.forward_batch(x, route, y=y)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        prep.forward_batch(x, route, y=y)
+    for rep in range(3):
+        x.copy_(synthetic.activations(150, 200, seed=20 + rep))
+        route.copy_(synthetic.softmax_router(150, 4, seed=30 + rep))
+        want = prep.forward_batch(x, route)
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want), rep
+
+
+def test_bad_arguments_are_refused_on_the_host():
+    import ctypes
+    from qmoe_amd import _lib
+    lib = _lib.load()
+    one, odd = ctypes.c_void_p(256), ctypes.c_void_p(257)
+    p = _lib.MoePrepared()
+    p.meta = p.codes = 256
+    p.experts, p.d_model, p.d_ff, p.total_chunks, p.meta_bytes = 4, 64, 128, 100, 1 << 30
+    ref = ctypes.byref(p)
+    scratch = lib.sub1_moe_batch_scratch_bytes(ref, 100)
+    ws = lib.sub1_moe_workspace_bytes(100, 128)
+    assert scratch > 0
+
+    def call(te=one, x=one, tokens=100, ws=ws, scratch=scratch, at=one):
+        return lib.sub1_moe_batch_prepared(ref, te, x, one, tokens, one, ws, at, scratch, None)
+
+    assert lib.sub1_moe_batch_prepared(None, one, one, one, 1, one, ws, one, scratch, None) == -1
+    assert call(te=None) == -1 and call(at=None) == -1
+    assert call(tokens=-1) == -2 and call(tokens=(1 << 20) + 1) == -2
+    assert call(scratch=scratch - 1) == -2 and call(ws=ws - 1) == -2
+    assert call(at=odd) < 0 and call(x=odd) < 0
+    assert call(tokens=0, te=None) == 0
+    # no growth past a piece; no form where a row's codes do not fit LDS, or of too many experts
+    assert lib.sub1_moe_batch_scratch_bytes(ref, 1 << 20) <= lib.sub1_moe_batch_scratch_bytes(ref, 8192)
+    p.d_ff = 12288
+    assert lib.sub1_moe_batch_scratch_bytes(ref, 100) == 0 and call() == -2
+    p.d_ff, p.experts = 128, 4097
+    assert lib.sub1_moe_batch_scratch_bytes(ref, 100) == 0
+    assert lib.sub1_moe_batch_scratch_bytes(None, 100) == 0 and lib.sub1_moe_batch_pays(None, 100) == 0
