@@ -228,11 +228,13 @@ __device__ __forceinline__ unaligned_u32x4 eight_codes(global_u16 *codes) {
 
 // A row's non-zeros as entries.  An entry is the step from the row's position (0 at
 // the start) to the next, 0..127; a longer gap goes over zero columns, as far as each
-// step reaches.  Calls emit(step, position after it) and returns the columns that
-// the codes cover; `at` is the position reached.
-template <class E>
+// step reaches.  An entry goes to sink.add(step, position after it), sink.end_code()
+// follows every codeword (after add has had at most three entries since the last), and
+// entries of a longer gap go to sink.add_now.  Returns the columns that the codes
+// cover; `at` is the position reached.
+template <class Sink>
 __device__ __forceinline__ int walk_row(const HeldTable &table, const uint16_t *row, int n, int width,
-                                        int &at, E &&emit) {
+                                        int &at, Sink &sink) {
   global_u16 *codes = (global_u16 *)row;
   int col = 0;
   at = 0;
@@ -250,13 +252,14 @@ __device__ __forceinline__ int walk_row(const HeldTable &table, const uint16_t *
             const int zero = (at + kMaxStep) / (2 * kZeroPeriod) * (2 * kZeroPeriod);
             const int step = zero - at;
             at = zero;
-            emit(step, at);
+            sink.add_now(step, at);
           }
         const int step = target - at;
         at = target;
-        emit(step, at);
+        sink.add(step, at);
       }
     }
+    sink.end_code();
     col += 2 * static_cast<int>(w & 15u);
   };
   if (n < 8) {
@@ -303,6 +306,13 @@ struct WalkArgs {
   uint16_t *ckpt;
 };
 
+struct EntryCount {
+  int entries = 0;
+  __device__ __forceinline__ void add(int, int) { entries++; }
+  __device__ __forceinline__ void add_now(int, int) { entries++; }
+  __device__ __forceinline__ void end_code() {}
+};
+
 // How many entries the non-zeros of every row take (the step onto a zero column
 // that a padded row makes after them is not counted: it fits the padding).
 __device__ __forceinline__ void count_rows(const HeldTable &table, const WalkKind &k, int count,
@@ -314,12 +324,13 @@ __device__ __forceinline__ void count_rows(const HeldTable &table, const WalkKin
   const uint32_t past = static_cast<uint32_t>(g - static_cast<int64_t>(first_e) * k.height);
   const int e = first_e + static_cast<int>(past / static_cast<uint32_t>(k.height));
   const int r = static_cast<int>(past % static_cast<uint32_t>(k.height));
-  int n, at, entries = 0;
+  int n, at;
+  EntryCount sink;
   const uint16_t *codes = row_codes(k.source, e, r, k.height, k.width, n);
-  const int covered = walk_row(table, codes, n, k.width, at, [&](int, int) { entries++; });
+  const int covered = walk_row(table, codes, n, k.width, at, sink);
   // a row's codes cover its width rounded up to a whole pair, exactly
   if (covered != ((k.width + 1) & ~1)) atomicAdd(&status[0], 1);
-  k.row_len[g] = static_cast<uint16_t>(min(entries, kMaxRowEntries));
+  k.row_len[g] = static_cast<uint16_t>(min(sink.entries, kMaxRowEntries));
 }
 
 // Position checkpoints.  For every slice and every group of kGroupChunks chunks,
@@ -330,6 +341,52 @@ __device__ __forceinline__ void count_rows(const HeldTable &table, const WalkKin
 __device__ __forceinline__ int64_t checkpoint_entry(uint32_t slice_base, int64_t slice) {
   return static_cast<int64_t>(slice_base / kGroupChunks) + slice;
 }
+
+// A row's entries, nine to a chunk.  The lanes of a wavefront fill their chunks at
+// different times, so that nearly every place that may store one is taken by a few of
+// them: a codeword's entries, at most three, fill one at most, and it is stored in one
+// place behind them.
+struct ChunkSink {
+  uint2 *d;
+  uint16_t *ck;
+  int nch;
+  int c = 0, q = 0;
+  uint32_t lo = 0, hi = 0;              // the chunk so far, its newest entry in bits 56..62
+  uint32_t full_lo = 0, full_hi = 0;    // one that is to be stored, and the position behind it
+  int full_at = -1;
+  __device__ __forceinline__ void shift_in(int step) {
+    lo = __builtin_amdgcn_alignbit(hi, lo, kFieldBits);
+    hi = (hi >> kFieldBits) | static_cast<uint32_t>(step) << 24;
+    q++;
+  }
+  __device__ __forceinline__ void store(uint32_t l, uint32_t h, int after) {
+    if (c < nch) d[c * 64] = make_uint2(l, h);   // the slice is as long as its longest row
+    c++;
+    if (c % kGroupChunks == 0 && c < nch) ck[(c / kGroupChunks) * 64] = static_cast<uint16_t>(after);
+  }
+  __device__ __forceinline__ void add(int step, int after) {
+    shift_in(step);
+    if (q == kFields) {
+      q = 0;
+      full_lo = lo;
+      full_hi = hi;
+      full_at = after;
+    }
+  }
+  __device__ __forceinline__ void end_code() {
+    if (full_at >= 0) {
+      store(full_lo, full_hi, full_at);
+      full_at = -1;
+    }
+  }
+  __device__ __forceinline__ void add_now(int step, int after) {
+    shift_in(step);
+    if (q == kFields) {
+      q = 0;
+      store(lo, hi, after);
+    }
+  }
+};
 
 // A slice's rows, a lane each, into the interleaved stream, nine entries to a chunk;
 // a row shorter than its slice then steps onto the next zero column and stays there
@@ -345,41 +402,31 @@ __device__ __forceinline__ void emit_rows(const HeldTable &table, const WalkKind
   const int nch = chunks_of(len);
   uint2 *d = stream + static_cast<int64_t>(base) * 64 + lane;
   uint16_t *ck = ckpt + checkpoint_entry(base, k.first_slice + slice) * 64 + lane;
-  int c = 0, q = 0;
-  uint32_t lo = 0, hi = 0;   // the chunk so far, its newest entry in bits 56..62
+  ChunkSink sink{d, ck, nch};
   ck[0] = 0;
-  auto emit = [&](int step, int after) {
-    lo = __builtin_amdgcn_alignbit(hi, lo, kFieldBits);
-    hi = (hi >> kFieldBits) | static_cast<uint32_t>(step) << 24;
-    if (++q == kFields) {
-      q = 0;
-      if (c < nch) d[c * 64] = make_uint2(lo, hi);   // the slice is as long as its longest row
-      c++;
-      if (c % kGroupChunks == 0 && c < nch) ck[(c / kGroupChunks) * 64] = static_cast<uint16_t>(after);
-    }
-  };
   int at = 0;
   if (ridx != 0xffff) {
     int n;
     const uint16_t *codes = row_codes(k.source, e, ridx, k.height, k.width, n);
-    walk_row(table, codes, n, k.width, at, emit);
-    if (c * kFields + q < len && (at >> 1) % kZeroPeriod != 0) {   // padding follows: it must read zeros
+    walk_row(table, codes, n, k.width, at, sink);
+    if (sink.c * kFields + sink.q < len && (at >> 1) % kZeroPeriod != 0) {   // padding follows: it must read zeros
       const int zero = (at + 2 * kZeroPeriod - 1) / (2 * kZeroPeriod) * (2 * kZeroPeriod);
       const int step = zero - at;
       at = zero;
-      emit(step, at);
+      sink.add_now(step, at);
     }
   }
 #pragma unroll 1
-  while (c < nch) emit(0, at);
+  while (sink.c < nch) sink.add_now(0, at);
 }
 
 // Task t goes to workgroup t mod grid first: a matrix of a few slices is spread over
 // as many compute units.  128 base experts (26 million codes): counting takes 59 us
-// (194 with the two-word table in global memory and a code at a time), emitting 132
-// (313); both are bound by their instructions, about 60 and 110 a code, emitting also by the
-// stores of lanes that fill their chunks at different times.  One code a turn
-// instead of eight (a tenth of the code) measured 93 and 169.
+// (194 with the two-word table in global memory and a code at a time), emitting 112
+// (313; 132 with a store behind every entry instead of every code); both are bound by
+// their instructions, about 60 and 90 a code, emitting also by the stores of lanes that
+// fill their chunks at different times.  One code a turn instead of eight (a tenth of
+// the code) measured 93, and 169 before the stores were put together.
 template <bool kEmit>
 __global__ __launch_bounds__(kWalkThreads) void walk_rows_kernel(WalkArgs a) {
   extern __shared__ __align__(16) uint32_t held[];
