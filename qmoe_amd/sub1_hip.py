@@ -11,6 +11,7 @@ sub1_cuda_kernel.cu:78-87), `sub1matvec_tokens`, `sub1decode`, and the grouped
 expert launch `ExpertStack.forward`.
 """
 import ctypes
+from operator import attrgetter
 
 import torch
 
@@ -33,6 +34,9 @@ def clear_faults():
 def _stream():
     """torch's current stream on the current device, as the C ABI takes it."""
     return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
+
+
+_dtype_of = attrgetter('dtype')
 
 
 class _on_device:
@@ -74,16 +78,19 @@ def _need(t, dtype, name, device=None, numel=None, dim=None):
 
 def _pointers(tensors, dtype, name, device, numel=None):
     """Their addresses, each looked over as _need does.  (A layer of 128 experts
-    has 768 tensors: looking at only what can be wrong first takes a third of the
-    time of as many calls.)"""
-    index = device.index
-    out = []
-    for t in tensors:
-        if not (isinstance(t, torch.Tensor) and t.dtype is dtype and t.get_device() == index
-                and t.is_contiguous() and (numel is None or t.numel() == numel)):
+    has 768 tensors: looking at all of them for one thing at a time, without a
+    call of _need each, takes a quarter of the time.)"""
+    try:
+        fine = (set(map(torch.Tensor.get_device, tensors)) == {device.index}
+                and set(map(_dtype_of, tensors)) == {dtype}
+                and all(map(torch.Tensor.is_contiguous, tensors))
+                and (numel is None or set(map(torch.Tensor.numel, tensors)) == {numel}))
+    except (TypeError, AttributeError):      # something that is no tensor
+        fine = False
+    if not fine:
+        for t in tensors:
             _need(t, dtype, name, device, numel=numel)
-        out.append(t.data_ptr())
-    return out
+    return list(map(torch.Tensor.data_ptr, tensors))
 
 
 def route_from_mask(router_mask):
