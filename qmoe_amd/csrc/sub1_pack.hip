@@ -113,10 +113,22 @@ int fill_tables(const PackTables &t) {
   // every string below the border has to be an entry (they are distinct)
   if (short_strings != kStrings - kBorderStrings)
     return fail(SUB1_ERR_INTERNAL, "the dictionary lacks strings below the border");
-  HIP_TRY(hipMemcpy(const_cast<uint16_t *>(t.code), code.data(), code.size() * 2, hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(const_cast<uint32_t *>(t.border), border.data(), border.size() * 4, hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(const_cast<int32_t *>(t.trie), trie.data(), trie.size() * 4, hipMemcpyHostToDevice));
-  return SUB1_OK;
+  // The caller's stream may be in a capture, which a copy on the default stream fails in
+  // and spoils: a stream of its own, and this thread's calls checked against no capture
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+  hipStream_t own = nullptr;
+  hipError_t e = hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
+  const auto copy = [&](const void *to, const void *from, size_t bytes) {
+    if (e == hipSuccess) e = hipMemcpyAsync(const_cast<void *>(to), from, bytes, hipMemcpyHostToDevice, own);
+  };
+  copy(t.code, code.data(), code.size() * 2);
+  copy(t.border, border.data(), border.size() * 4);
+  copy(t.trie, trie.data(), trie.size() * 4);
+  if (e == hipSuccess) e = hipStreamSynchronize(own);
+  if (own) (void)hipStreamDestroy(own);
+  (void)hipThreadExchangeStreamCaptureMode(&mode);   // as it was
+  return e == hipSuccess ? SUB1_OK : fail(SUB1_ERR_HIP, "filling the encoder's tables: %s", hipGetErrorString(e));
 }
 
 // The three arrays on the current device (2.7 MB a GPU, filled on the first call

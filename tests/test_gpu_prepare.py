@@ -194,3 +194,47 @@ def test_expanding_codes_that_do_not_fit_the_width(gpu):
     assert torch.equal(tern[2], whole[2])
     kept = int((tern[0] != whole[0]).nonzero()[0])           # the first symbol lost
     assert 0 < kept < 4000 and torch.equal(tern[0, :kept], whole[0, :kept]) and not tern[0, kept:].any()
+
+
+FIRST_PACK_IN_A_CAPTURE = r'''
+import ctypes, sys
+sys.path.insert(0, sys.argv[1])
+import torch
+from qmoe_amd import _lib, sub1, sub1_hip
+
+lib = _lib.load()
+_lib.check_faults()
+g = torch.Generator().manual_seed(1)
+symbols = ((torch.rand((70, 200), generator=g) < 0.2) * torch.randint(1, 3, (70, 200), generator=g)).to(torch.int32).cuda()
+t = torch.empty_like(symbols)
+off = torch.zeros(71, dtype=torch.int32, device='cuda')
+stream = torch.cuda.Stream()
+c_stream = ctypes.c_void_p(stream.cuda_stream)
+torch.cuda.synchronize()
+graph = torch.cuda.CUDAGraph()
+with torch.cuda.graph(graph, stream=stream):
+    t.copy_(symbols)
+    _lib.check(lib.sub1_pack_count(sub1.TRIE.data_ptr(), t.data_ptr(), off.data_ptr(), 70, 200, c_stream))
+counted = []
+for _ in range(3):
+    off.fill_(-5)
+    graph.replay()
+    torch.cuda.synchronize()
+    counted.append(off.tolist())
+want = torch.zeros_like(off)
+sub1_hip.sub1pack(sub1.TRIE, symbols.clone(), want)
+assert counted == [want.tolist()] * 3, counted
+print('first call in a capture: fine')
+'''
+
+
+def test_the_first_pack_of_a_process_may_be_captured():
+    """The first call fills the tables that the encoder keeps on a GPU, also where its
+    stream is being captured.  (A process of its own: in this one they are there.)"""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    res = subprocess.run([sys.executable, '-c', FIRST_PACK_IN_A_CAPTURE, root], stdout=subprocess.PIPE,
+                         stderr=subprocess.STDOUT, text=True, timeout=110)
+    assert res.returncode == 0 and 'first call in a capture: fine' in res.stdout, res.stdout
