@@ -350,6 +350,13 @@ int sub1_moe_batch_prepared(const sub1_moe_prepared *prepared, const int32_t *to
                             int64_t workspace_bytes, void *scratch, int64_t scratch_bytes,
                             void *stream);
 
+/*
+ * For tests (no counterpart in the reference): how sub1_moe_batch_prepared gives the
+ * slices of a projection (0 = wi, 1 = wo) to workgroups.  plan receives three words: slices of
+ * a workgroup, wavefronts that share a slice, bytes of LDS.  Host only.
+ */
+int sub1_test_batch_plan(const sub1_moe_prepared *prepared, int projection, int32_t *plan);
+
 int sub1_moe_prepared_decode(const sub1_moe_prepared *prepared, int expert, int projection,
                              void *tern_out, void *stream);
 

@@ -98,6 +98,7 @@ PROTOTYPES = {
     'sub1_moe_batch_pays': (_int, [ctypes.POINTER(MoePrepared), _int]),
     'sub1_moe_batch_prepared': (_int, [ctypes.POINTER(MoePrepared), _vp, _vp, _vp, _int, _vp, _i64,
                                        _vp, _i64, _vp]),
+    'sub1_test_batch_plan': (_int, [ctypes.POINTER(MoePrepared), _int, ctypes.POINTER(ctypes.c_int32)]),
     'sub1_moe_prepared_decode': (_int, [ctypes.POINTER(MoePrepared), _int, _int, _vp, _vp]),
     'sub1_matrix_prepared_meta_bytes': (_i64, [_int, _int, _int]),
     'sub1_matrix_prepare_layout': (_int, [ctypes.POINTER(MatrixSet), _vp, _i64,

@@ -3287,14 +3287,19 @@ struct BatchPlan {
   size_t lds;
 };
 
-// LDS holds the codes of `fit` slices: with room for three and more, workgroups of four
-// wavefronts, one to a SIMD; for two, of eight; for one, of twelve.  (128 base experts on 4096
-// tokens: 131 us; with wi's workgroups of 8 wavefronts 134, with wo's of 6, 8 and 12
+// LDS holds the codes of `fit` slices: with room for three and more, workgroups of up to four
+// wavefronts, one to a SIMD; for two, of up to eight; for one, of twelve.  (128 base experts on
+// 4096 tokens: 131 us; with wi's workgroups of 8 wavefronts 134, with wo's of 6, 8 and 12
 // 142, 132 and 153.  40 c-2048 experts on 700 tokens, wo, whose codes take 98 KB, with
 // 4, 8, 12 and 16 wavefronts: 205, 166, 162 and 165.)  Wavefronts share a slice as long as
 // each gets a group of chunks, the least that one can expand, and take slices of their
 // own beyond that (c-2048 wi by 1, 2 and 4 to a slice: 208, 181, 166 us; base wi, of
-// hardly two groups, 134, 131, 144).
+// hardly two groups, 134, 131, 144) - but not where a compute unit would then hold fewer than
+// twelve wavefronts, as it does of rows with few entries, whose slices are short but whose codes
+// take LDS as any: more of them share a slice then, the ones without a group of chunks for its
+// multiplying alone.  (With 95 % zeros, sharing by chunks alone: 128 base experts on 4096 tokens,
+// wo's workgroups of 4 wavefronts and 99 KB, 166 us against 128; 40 c-2048 experts on 640, of 4 and
+// 98 KB, 201 against 154.)
 bool plan_batch(const Prepared &p, int kind, size_t lds_limit, BatchPlan *out) {
   const int slices[2] = {(p.height[0] + 63) / 64, (p.height[1] + 63) / 64};
   const double weight = static_cast<double>(slices[0]) * p.width[0] + static_cast<double>(slices[1]) * p.width[1];
@@ -3304,17 +3309,19 @@ bool plan_batch(const Prepared &p, int kind, size_t lds_limit, BatchPlan *out) {
   const int waves = fit >= 3 ? 4 : fit == 2 ? 8 : 12;
   int parts = 1;
   while (parts < waves && parts * kGroupChunks < 0.75 * chunks) parts *= 2;
-  parts = std::min(parts, waves);
-  int per_group = std::min(waves / parts, slices[kind]);
-  for (;; per_group--) {
+  for (;; parts *= 2) {
+    parts = std::min(parts, waves);
+    int per_group = std::min(waves / parts, slices[kind]);
+    for (; per_group > 0; per_group--) {
+      const size_t sums = parts > 1 ? static_cast<size_t>(2 * per_group * parts) * 4096 : 0;
+      out->lds = std::max(per_group * code_bytes, sums);
+      if (out->lds <= lds_limit) break;
+    }
     if (per_group == 0) return false;
-    const size_t sums = parts > 1 ? static_cast<size_t>(2 * per_group * parts) * 4096 : 0;
-    out->lds = std::max(per_group * code_bytes, sums);
-    if (out->lds <= lds_limit) break;
+    out->per_group = per_group;
+    out->parts = parts;
+    if (parts == waves || static_cast<int>(lds_limit / out->lds) * per_group * parts >= 12) return true;
   }
-  out->per_group = per_group;
-  out->parts = parts;
-  return true;
 }
 
 constexpr size_t kBatchLds = 160 * 1024 - 64;
@@ -3729,6 +3736,19 @@ extern "C" int sub1_moe_batch_pays(const sub1_moe_prepared *p, int tokens) {
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1)
     return 0;
   return batch_pays(from_moe(p), tokens, cus);
+}
+
+extern "C" int sub1_test_batch_plan(const sub1_moe_prepared *p, int projection, int32_t *plan) {
+  const char *who = "sub1_test_batch_plan";
+  if (!p || !plan) return fail(SUB1_ERR_NULL, "%s: NULL argument", who);
+  if (projection < 0 || projection > 1 || sub1_moe_batch_scratch_bytes(p, 1) <= 0)
+    return fail(SUB1_ERR_SHAPE, "%s: no such form", who);
+  BatchPlan b;
+  if (!plan_batch(from_moe(p), projection, kBatchLds, &b)) return fail(SUB1_ERR_INTERNAL, "%s: no plan", who);
+  plan[0] = b.per_group;
+  plan[1] = b.parts;
+  plan[2] = static_cast<int32_t>(b.lds);
+  return SUB1_OK;
 }
 
 extern "C" int sub1_moe_batch_prepared(const sub1_moe_prepared *p, const int32_t *token_expert, const void *x,

@@ -154,6 +154,28 @@ def test_replays_from_a_graph():
         assert torch.equal(y, want), rep
 
 
+def batch_plan(prep, projection):
+    import ctypes
+    from qmoe_amd import _lib
+    plan = (ctypes.c_int32 * 3)()
+    _lib.check(_lib.load().sub1_test_batch_plan(ctypes.byref(prep), projection, plan))
+    return tuple(plan)
+
+
+@pytest.mark.parametrize('d_model,d_ff', [(768, 3072), (1024, 4096), (2080, 6144), (1100, 3500), (512, 2000)])
+@pytest.mark.parametrize('entries', [0.06, 0.11, 0.21])      # of a weight, at 95, 90 and 80 % zeros
+def test_a_compute_unit_holds_twelve_wavefronts_of_a_product(d_model, d_ff, entries):
+    """Whatever the share of zeros: a slice of few entries takes as much LDS as any."""
+    from qmoe_amd import _lib
+    p = _lib.MoePrepared()
+    p.meta = p.codes = 256
+    p.experts, p.d_model, p.d_ff, p.meta_bytes = 64, d_model, d_ff, 1 << 40
+    p.total_chunks = int(64 * 2 * d_model * d_ff * entries / 576)
+    for projection in (0, 1):
+        slices, shared_by, lds = batch_plan(p, projection)
+        assert (160 * 1024 - 64) // lds * slices * shared_by >= 12, (projection, slices, shared_by, lds)
+
+
 def test_bad_arguments_are_refused_on_the_host():
     import ctypes
     from qmoe_amd import _lib
