@@ -338,8 +338,10 @@ int sub1_moe_grouped_prepared(const sub1_moe_prepared *prepared, const int32_t *
  * tokens: larger batches run in equal pieces.
  *
  * sub1_moe_batch_pays: 1 where this is estimated to be faster than
- * sub1_moe_grouped_prepared for `tokens` tokens spread over the experts (from about 16
- * tokens an expert on, never below 8), 0 otherwise.
+ * sub1_moe_grouped_prepared for `tokens` tokens spread over the experts, 0 otherwise.  Every
+ * piece expands the experts that it hits anew, so that what counts is a piece's tokens an
+ * expert: from about 16 on it pays, with few experts from a few hundred tokens on, below 8
+ * never - and so never with more than 1024 experts.
  */
 int64_t sub1_moe_batch_scratch_bytes(const sub1_moe_prepared *prepared, int tokens);
 

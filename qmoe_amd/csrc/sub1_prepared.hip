@@ -38,6 +38,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -3333,24 +3334,44 @@ bool batch_takes(const Prepared &p) {
          plan_batch(p, 1, kBatchLds, &plan);
 }
 
-// Whether the matrix cores are the faster way for `tokens` tokens, by estimates fitted to
-// both at 1 to 64 tokens an expert through 8 to 128 experts of the three Switch shapes and of
-// two odd ones (80 and 95 % zeros), in microseconds.  Here: 36 and, per million weights of the experts hit, 0.03 for every
-// 64 of an expert's tokens and 0.09 for every 32 (base 128: 103 measured at 16 tokens an expert
-// and 132 at 32, 105 and 133 estimated; c-2048 40: 167 at 16, 159).  Walking: as launch_prepared has
-// it, a token on a compute unit 8 + entries / 23400, less where four tokens walk together
-// (base 128: 108, 177 and 270 at 8, 16 and 32).  The estimates are some 10 % off either way,
-// so the matrix cores must promise that much: below 8 tokens an expert they never do.
+// Blocks of `per` that an expert's tokens fill, on average, where their number is spread
+// about `each` as independent tokens spread it (the k-th block is begun by more than k * per).
+double blocks_on_average(double each, int per) {
+  double blocks = 0.0;
+  for (int k = 0;; k++) {
+    const double begun = 0.5 * std::erfc((per * k + 0.5 - each) / std::sqrt(2.0 * each));
+    blocks += begun;
+    if (per * k > each && begun < 1e-3) return blocks;
+  }
+}
+
+// Whether the matrix cores are the faster way for `tokens` tokens, by estimates in microseconds
+// fitted to both at 8 to 128 tokens an expert through 1 to 2048 experts of the three Switch shapes
+// and of four odd ones, with 80 to 95 % zeros or shares that differ from row to row (464 launches).
+// Here, for every piece of a batch, which expands every expert that it hits: 42 and, per million
+// weights, 0.025 and 0.31 times the entries of a weight for every 64 of an expert's tokens, 0.073
+// for every 32 (within 9 %, root mean square).  Walking: a compute unit takes
+// token_us = 8 + entries / 23400 for a token and, where launch_prepared groups tokens by expert,
+// 7 + 1.85 (token_us - 8) for up to four, in whole rounds.  The matrix cores must promise 5 %: of those
+// launches that leaves 6 on the slower way, by 8 % at most, and 38 where they would have been
+// faster, by up to 23 %; of 196 others none and 13.  A piece with less than 8 tokens an expert never goes there.  (Pricing one
+// pass over the experts for a batch that runs in pieces, as it was done first, sent 32 768 tokens
+// through 2048 base experts this way: 5862 us, walking takes 1735.)
 bool batch_pays(const Prepared &p, int tokens, int cus) {
-  if (tokens < 8 * static_cast<int64_t>(p.count) || !batch_takes(p)) return false;
-  const double each = static_cast<double>(tokens) / p.count;
-  const double blocks = each / kBlockTokens + 0.5, chunks = blocks / kChunkBlocks;
+  const int piece = batch_piece(tokens), pieces = (tokens + piece - 1) / piece;
+  if (piece < 8 * static_cast<int64_t>(p.count) || !batch_takes(p)) return false;
+  const double each = static_cast<double>(piece) / p.count;
   const double weights = 2e-6 * p.count * p.height[0] * p.width[0];
-  const double batch_us = 36.0 + weights * (0.03 * std::max(1.0, chunks) + 0.09 * std::max(1.0, blocks));
-  const double token_us = 8.0 + static_cast<double>(p.total_chunks) * (64.0 * kFields) / p.count / 23400.0;
-  const bool together = tokens >= 4 * cus;
-  const double gain = together ? std::min(1.7, std::max(1.0, 0.85 + 0.027 * each)) : 1.0;
-  return 1.1 * batch_us < tokens * token_us / cus / gain;
+  const double entries = 1e-6 * p.total_chunks * (64.0 * kFields);
+  const double by_chunks = blocks_on_average(each, kChunkBlocks * kBlockTokens) * (0.025 * weights + 0.31 * entries);
+  const double by_blocks = blocks_on_average(each, kBlockTokens) * 0.073 * weights;
+  const double batch_us = pieces * (42.0 + 256.0 / cus * (by_chunks + by_blocks));
+  const double walk_us = 1e6 * entries / p.count / 23400.0;   // of a token, besides its 8 us
+  const bool grouped = tokens >= 4 * static_cast<int64_t>(p.count) && tokens >= 4 * cus;
+  const double rounds = (0.25 * tokens + 0.375 * p.count) / cus;
+  const double other_us = grouped ? 14.0 + std::ceil(rounds) * (7.0 + 1.85 * walk_us)
+                                  : static_cast<double>(tokens) / cus * (8.0 + walk_us);
+  return 1.05 * batch_us < other_us;
 }
 
 int launch_batch(const Prepared &p, const int32_t *token_expert, const uint16_t *x, uint16_t *y, int tokens,

@@ -456,7 +456,8 @@ class PreparedStack:
 
     def batch_pays(self, tokens):
         """Whether forward_batch is estimated to be the faster one (it never is
-        below 8 tokens an expert)."""
+        below 8 tokens an expert, nor with more than 1024 experts: a batch runs in
+        pieces of up to 8192 tokens, each of which expands its experts anew)."""
         if tokens < 128 or tokens < 8 * self.experts:
             return False
         with _on_device(self.device):

@@ -130,6 +130,50 @@ def test_large_batches_through_the_layer():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('d_model,d_ff,experts,each,pays', [
+    # us measured, walking and on the matrix cores, with 90 % zeros
+    (768, 3072, 128, 32, True),        # 270, 131
+    (2080, 6144, 40, 16, True),        # 313, 169
+    (1024, 4096, 64, 64, True),        # 419, 157
+    (768, 3072, 512, 16, True),        # 460, 365
+    (768, 3072, 1, 2048, True),        # 172, 77
+    (768, 3072, 32, 8, False),         # 35, 57
+    (768, 3072, 512, 8, False),        # 280, 363
+    # batches of several pieces: a piece has 8 tokens an expert, or fewer
+    (768, 3072, 1024, 8, False),       # 513, 742
+    (768, 3072, 1024, 16, False),      # 883, 1473
+    (768, 3072, 1024, 64, False),      # 3134, 5854
+    (768, 3072, 2048, 16, False),      # 1735, 5862
+    (512, 2000, 1024, 32, False),      # 833, 1443
+    (2080, 6144, 2048, 16, False)])    # four pieces with 4 tokens an expert
+def test_the_matrix_cores_are_taken_where_they_are_faster(d_model, d_ff, experts, each, pays):
+    import ctypes
+    from qmoe_amd import _lib
+    p = _lib.MoePrepared()
+    p.meta = p.codes = 256
+    p.experts, p.d_model, p.d_ff, p.meta_bytes = experts, d_model, d_ff, 1 << 40
+    p.total_chunks = int(experts * 2 * d_model * d_ff * 0.1045 / 576)
+    lib = _lib.load()
+    assert bool(lib.sub1_moe_batch_pays(ctypes.byref(p), experts * each)) == pays
+    for tokens in (100, 5000, 8192, 8193, 16385, 100000, 1 << 20):
+        piece = tokens / -(-tokens // 8192)
+        if lib.sub1_moe_batch_pays(ctypes.byref(p), tokens):
+            assert piece >= 8 * experts, tokens
+
+
+@pytest.mark.gpu
+def test_pieces_of_a_batch_through_many_experts():
+    from qmoe_amd import synthetic
+    prep = synthetic.build_stack(700, 96, 130, 0.9, seed=11).prepare()
+    x = synthetic.activations(17000, 96, seed=12)
+    route = synthetic.softmax_router(17000, 700, seed=13)
+    route[::50] = -1
+    y, walked = prep.forward_batch(x, route), prep.forward(x, route)
+    assert torch.equal(y[::50], x[::50])
+    assert (y.float() - walked.float()).norm() <= 2e-4 * walked.float().norm()
+
+
+@pytest.mark.gpu
 def test_replays_from_a_graph():
     from qmoe_amd import synthetic
     stack = synthetic.build_stack(4, 200, 300, 0.9, seed=7)
