@@ -329,8 +329,8 @@ int sub1_moe_grouped_prepared(const sub1_moe_prepared *prepared, const int32_t *
  * same workspace (control words); a row's result is the same fp32 sum of products
  * that are exact, taken in the matrix cores' order, so it agrees with
  * sub1_moe_grouped_prepared to rounding, not to the bit; it does not depend on the
- * other tokens.  Tokens whose x or h hold an infinity or NaN go through the walking
- * kernel, with its results.  y may be x.
+ * other tokens.  Tokens whose x or h hold an infinity or NaN, and those of an expert
+ * whose (min, max) do, go through the walking kernel, with its results.  y may be x.
  *
  * scratch: sub1_moe_batch_scratch_bytes(p, tokens) bytes of device memory, 256-byte
  * aligned, contents arbitrary before and after (0: no such form for these shapes - a

@@ -26,8 +26,9 @@
 // 64), then the start and end of workgroups that LDS holds to 12 to 16 wavefronts a compute unit.
 //
 // A token whose activations or h hold an infinity or NaN is left to the walking
-// kernel (0 x inf is NaN here, and a weight of zero adds nothing there): the passes
-// mark it, and unpack_tokens_kernel lists it for the launch that follows.
+// kernel (0 x inf is NaN here, and a weight of zero adds nothing there), and so are the
+// tokens of an expert with such a (min, max) (walking, every weight of its row meets it): the
+// passes and the products mark them, and unpack_tokens_kernel lists them for the launch that follows.
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -64,6 +65,7 @@ struct BatchArgs {
   const u32x4 *in;        // [block][step][64 lanes]: 16-byte operands
   uint16_t *out;          // [block][height][32]
   const int4 *chunks;     // (expert, first block, blocks, 0)
+  int32_t *spoiled;       // [slot]: left to the walking kernel
   const int32_t *totals;
   int steps, parts;       // parts: wavefronts that share a slice
   int per_group;          // slices of a workgroup
@@ -176,6 +178,10 @@ __device__ __forceinline__ void slices_times_tokens(const BatchArgs &a, uint32_t
   const int all_words = a.per_group * slice_words;   // a multiple of 64
   for (int i = 4 * threadIdx.x; i < all_words; i += 4 * blockDim.x)
     *reinterpret_cast<uint4 *>(lds + i) = make_uint4(0u, 0u, 0u, 0u);
+  // (an exponent of all ones in either half: the sum carries into its sign)
+  const uint32_t high = ((minmax[0] & 0x7f807f80u) + 0x00800080u) | ((minmax[1] & 0x7f807f80u) + 0x00800080u);
+  if ((high & 0x80008000u) && mine && sub == 0)
+    for (int t = 0; t < kBlocks * kBlockTokens; t++) a.spoiled[first_block * kBlockTokens + t] = 1;
   __syncthreads();
 #pragma unroll 1
   for (int c = g_lo * kGroupChunks; c < c_end; c += kGroupChunks) {

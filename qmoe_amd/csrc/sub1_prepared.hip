@@ -3423,6 +3423,7 @@ int launch_batch(const Prepared &p, const int32_t *token_expert, const uint16_t 
     b_args.out = i ? y_rows : h_rows;
     b_args.chunks = chunks;
     b_args.totals = totals;
+    b_args.spoiled = spoiled;
     b_args.steps = steps_of(k.width);
     b_args.parts = plan.parts;
     b_args.per_group = plan.per_group;

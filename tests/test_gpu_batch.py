@@ -92,6 +92,29 @@ def test_a_token_without_finite_activations_spoils_no_other(oracle):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('projection', [0, 1])
+@pytest.mark.parametrize('value', [np.inf, -np.inf, np.nan])
+def test_a_weight_that_is_not_finite_gives_what_walking_gives(oracle, projection, value):
+    """An infinite or NaN min or max, also one that no weight of its row has; the other
+    experts' tokens are as without it."""
+    layer = [[layers(oracle, 200, 96, 0.9, 1 + e) for e in range(3)], [layers(oracle, 96, 200, 0.9, 11 + e) for e in range(3)]]
+    x = torch.randn((200, 96), generator=torch.Generator().manual_seed(5)).bfloat16().cuda()
+    te = (torch.arange(200, dtype=torch.int32) % 3).cuda()
+    plain = prepared(*layer).forward_batch(x, te)
+    height, width = (200, 96) if projection == 0 else (96, 200)
+    t = np.zeros((height, width), dtype=np.int32)
+    t[:, ::7] = 1
+    t[5, ::7], t[70, 3], t[90] = 2, 2, 0          # row 5: no min; row 70: one max; row 90: nothing
+    minmax = np.tile(np.float32([-1.0, 1.0]), (height, 1))
+    minmax[5, 0] = minmax[70, 1] = minmax[90, 0] = value
+    layer[projection][1] = oracle.encode(t) + (so.f32_to_bf16_bits(minmax.ravel()),)
+    prep = prepared(*layer)
+    y, walked = prep.forward_batch(x, te), prep.forward(x, te)
+    assert torch.equal(y[1::3].view(torch.int16), walked[1::3].view(torch.int16))
+    assert torch.equal(y[::3], plain[::3]) and torch.equal(y[2::3], plain[2::3])
+
+
+@pytest.mark.gpu
 def test_large_batches_through_the_layer():
     """What Sub1Experts sends where: equal to rounding either way, a token's bits the
     same in any batch that goes through the matrix cores, batches of several pieces,
