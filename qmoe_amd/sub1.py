@@ -207,14 +207,8 @@ class Sub1Experts(nn.Module):
     matrix_cores = True
 
     def forward(self, x, expert_index):
-        return _run_experts(self._launcher(), x.contiguous(),
-                            expert_index.to(torch.int32).contiguous(), self.matrix_cores)
-
-
-def _run_experts(launcher, x, route, matrix_cores):
-    if matrix_cores and isinstance(launcher, sub1_hip.PreparedStack) and launcher.batch_pays(x.shape[0]):
-        return launcher.forward_batch(x, route)
-    return launcher.forward(x, route)
+        return self._launcher().forward(x.contiguous(), expert_index.to(torch.int32).contiguous(),
+                                        None, self.matrix_cores)
 
 
 def _router_outputs(outputs, experts):
@@ -361,7 +355,7 @@ class FasterMLP(nn.Module):
         # has an all-zero mask row: expert -1 for the launch
         route, expert_index = sub1_hip.route_from_mask(router_mask)
         x = hidden_states.reshape(-1, hidden_states.shape[-1]).to(torch.bfloat16).contiguous()
-        next_states = _run_experts(self._launcher(), x, route, self.matrix_cores)
+        next_states = self._launcher().forward(x, route, None, self.matrix_cores)
         hidden_states = router_probs * next_states.view(hidden_states.shape).to(hidden_states.dtype)
         if self.router_outputs:
             return hidden_states, (router_logits, expert_index)

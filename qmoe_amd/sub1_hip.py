@@ -316,10 +316,11 @@ class ExpertStack:
 
     workspace = _workspace
 
-    def forward(self, x, token_expert, y=None):
+    def forward(self, x, token_expert, y=None, matrix_cores=False):
         """y[t] = wo_e(relu(wi_e(x[t]))), e = token_expert[t]; tokens with a
         negative expert keep their input.  x bf16 [T, d_model], token_expert
-        int32 [T]."""
+        int32 [T].  (matrix_cores: see PreparedStack.forward; this layout has
+        one form.)"""
         dev = self.device
         _lib.check_faults()       # what earlier launches reported (host memory, no sync)
         p_x = _need(x, torch.bfloat16, 'x', dev, dim=2)
@@ -416,6 +417,7 @@ class PreparedStack:
         lib = _lib.load()
         self.device = dev
         self.experts, self.d_model, self.d_ff = experts, d_model, d_ff
+        self.batch_tokens = max(128, 8 * experts)     # batch_pays for none below
         meta_bytes = lib.sub1_moe_prepared_meta_bytes(experts, d_model, d_ff)
         if meta_bytes <= 0:
             raise ValueError('bad stack dimensions')
@@ -434,13 +436,18 @@ class PreparedStack:
 
     workspace = _workspace
 
-    def forward(self, x, token_expert, y=None):
+    def forward(self, x, token_expert, y=None, matrix_cores=False):
+        """As ExpertStack.forward.  matrix_cores: a batch for which batch_pays
+        goes through forward_batch (asked for here, where it costs a small batch
+        a comparison)."""
         dev = self.device
         _lib.check_faults()       # what earlier launches reported (host memory, no sync)
         p_x = _need(x, torch.bfloat16, 'x', dev, dim=2)
-        tokens = x.shape[0]
-        if x.shape[1] != self.d_model:
+        tokens, width = x.shape
+        if width != self.d_model:
             raise ValueError('x must be [T, %d]' % self.d_model)
+        if matrix_cores and tokens >= self.batch_tokens and self.batch_pays(tokens):
+            return self.forward_batch(x, token_expert, y)
         p_te = _need(token_expert, torch.int32, 'token_expert', dev, numel=tokens)
         if y is None:
             y = torch.empty_like(x)
@@ -458,7 +465,7 @@ class PreparedStack:
         """Whether forward_batch is estimated to be the faster one (it never is
         below 8 tokens an expert, nor with more than 1024 experts: a batch runs in
         pieces of up to 8192 tokens, each of which expands its experts anew)."""
-        if tokens < 128 or tokens < 8 * self.experts:
+        if tokens < self.batch_tokens:
             return False
         with _on_device(self.device):
             return bool(_lib.load().sub1_moe_batch_pays(ctypes.byref(self._c), tokens))

@@ -153,6 +153,24 @@ def test_large_batches_through_the_layer():
 
 
 @pytest.mark.gpu
+def test_a_small_batch_is_not_priced(monkeypatch):
+    """The calls that last as long as the host takes to make them: no estimate is asked for."""
+    from qmoe_amd import sub1, sub1_hip, synthetic
+    stack = synthetic.build_stack(4, 64, 96, 0.9, seed=14)
+    layers_of = [[sub1.Sub1Linear(1, 1) for _ in range(4)] for _ in range(2)]
+    for e in range(4):
+        for linear, buffers in zip((layers_of[0][e], layers_of[1][e]), synthetic.expert_layers(stack, e)):
+            linear.w_comp, linear.row_off, linear.ter_minmax = buffers
+    layer = sub1.Sub1Experts(*layers_of)
+    x, route = synthetic.activations(200, 64, seed=15), synthetic.softmax_router(200, 4, seed=16)
+    asked = []
+    monkeypatch.setattr(sub1_hip.PreparedStack, 'batch_pays', lambda self, tokens: bool(asked.append(tokens)))
+    for tokens in (1, 13, 127, 128, 200):
+        layer(x[:tokens], route[:tokens])
+    assert asked == [128, 200]
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize('d_model,d_ff,experts,each,pays', [
     # us measured, walking and on the matrix cores, with 90 % zeros
     (768, 3072, 128, 32, True),        # 270, 131
