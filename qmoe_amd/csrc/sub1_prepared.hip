@@ -3399,7 +3399,11 @@ int launch_batch(const Prepared &p, const int32_t *token_expert, const uint16_t 
   const auto shares = [](int work, int per) { return static_cast<unsigned>(std::max(1, std::min(16, (work + per - 1) / per))); };
   pack_tokens_kernel<<<dim3(b.max_blocks, shares(steps_of(d_model), 16)), 256, 0, s>>>(
       x, y, d_model, d_model, d_model, aligned, slots, spoiled, totals, xs);
-  const void *fn = reinterpret_cast<const void *>(batch_product_kernel);
+  // the most they may have, not what this launch has: another thread's launch, of other shapes,
+  // may lie between this call and ours
+  for (const void *fn : {reinterpret_cast<const void *>(batch_product_kernel),
+                         reinterpret_cast<const void *>(walk_listed_kernel)})
+    HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kBatchLds)));
   PreparedArgs a = {};
   a.stream = static_cast<const uint2 *>(p.codes);
   a.ckpt = reinterpret_cast<const uint16_t *>(a.stream + p.total_chunks * 64);
@@ -3432,7 +3436,6 @@ int launch_batch(const Prepared &p, const int32_t *token_expert, const uint16_t 
     b_args.per_group = plan.per_group;
     b_args.slice_groups = (k.slices + plan.per_group - 1) / plan.per_group;
     b_args.relu = i == 0;
-    HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(plan.lds)));
     batch_product_kernel<<<static_cast<unsigned>((b.max_chunks + 7) / 8 * 8 * b_args.slice_groups),
                            64 * plan.per_group * plan.parts, plan.lds, s>>>(b_args);
     if (i == 0)
@@ -3451,8 +3454,6 @@ int launch_batch(const Prepared &p, const int32_t *token_expert, const uint16_t 
   a.xdwords = activation_dwords(d_model);
   a.hdwords = activation_dwords(d_ff);
   const size_t lds = static_cast<size_t>(a.xdwords + a.hdwords) * 4;
-  HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(walk_listed_kernel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
   walk_listed_kernel<<<std::min(tokens, 256), kMaxThreads, lds, s>>>(a);
   HIP_TRY(hipGetLastError());
   sub1::note_kernel("batch_product_kernel");

@@ -215,6 +215,33 @@ def test_pieces_of_a_batch_through_many_experts():
 
 
 @pytest.mark.gpu
+def test_two_threads_with_stacks_of_other_shapes():
+    """Each on a stream of its own: their launches take different amounts of LDS."""
+    import threading
+    from qmoe_amd import synthetic
+    work = []
+    for d_model, d_ff in ((96, 5000), (700, 130)):
+        prep = synthetic.build_stack(3, d_model, d_ff, 0.9, seed=17).prepare()
+        x, route = synthetic.activations(160, d_model, seed=18), synthetic.softmax_router(160, 3, seed=19)
+        x[7, 0] = float('inf')
+        work.append((prep, x, route, prep.forward_batch(x, route), []))
+    torch.cuda.synchronize()
+
+    def run(prep, x, route, want, differ):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(40):
+                y = prep.forward_batch(x, route)
+                differ.append(not torch.equal(y.view(torch.int16), want.view(torch.int16)))
+
+    threads = [threading.Thread(target=run, args=w) for w in work]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert [w[4] for w in work] == [[False] * 40] * 2
+
+
+@pytest.mark.gpu
 def test_replays_from_a_graph():
     from qmoe_amd import synthetic
     stack = synthetic.build_stack(4, 200, 300, 0.9, seed=7)
