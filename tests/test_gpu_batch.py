@@ -40,13 +40,16 @@ def prepared(wi, wo):
     (33, 130, [0.0, 1.0, 0.5], [40, 40]),                 # whole rows and empty ones
     (768, 400, 0.9, [33, 5]), (400, 768, 0.9, [5, 64]),
     (1100, 470, [0.9] * 63 + [0.02], [70, 3]),            # a row of many groups in every slice
-    (130, 3500, 0.98, [34]),                              # eight wavefronts to a slice
-    (66, 6200, 0.985, [65])])                             # twelve, and codes that fill LDS
+    (130, 3500, 0.98, [34]), (130, 3500, 0.8, [65]),      # eight wavefronts to a slice of wo,
+    (66, 6200, 0.985, [65]), (66, 6200, 0.85, [34])])     # twelve and codes that fill LDS: most of
+                                                          # them without a group of chunks, and none
 def test_exact_sums_equal_the_oracle(oracle, d_model, d_ff, p0, counts):
     experts = len(counts)
     wi = [layers(oracle, d_ff, d_model, p0, 10 + e) for e in range(experts)]
     wo = [layers(oracle, d_model, d_ff, p0, 20 + e) for e in range(experts)]
     prep = prepared(wi, wo)
+    if d_ff > 3000:
+        assert batch_plan(prep._c, 1)[1] == (8 if d_ff == 3500 else 12)
     rng = np.random.default_rng(1)
     route = np.concatenate([np.full(n, e) for e, n in enumerate(counts)] + [[-1, experts, -7]]).astype(np.int32)
     rng.shuffle(route)
