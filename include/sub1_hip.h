@@ -92,7 +92,9 @@ int sub1_matvec_tokens(const int32_t *dec, const int16_t *w_comp,
  * OVERWRITTEN with the row's codes (row r's codes at w_tern[r*W ...]) and
  * row_off [H+1] receives the cumulative counts.  The caller then reads
  * row_off[H] (a device-to-host copy, as the reference does at
- * sub1_cuda_kernel.cu:115) to size w_comp.
+ * sub1_cuda_kernel.cu:115) to size w_comp.  The first encoder call on a GPU fills
+ * 2.7 MB of tables that the library keeps there (a copy from the host; also where
+ * `stream` is being captured).
  */
 int sub1_pack_count(const int32_t *trie, int32_t *w_tern, int32_t *row_off,
                     int height, int width, void *stream);
@@ -225,8 +227,8 @@ int sub1_route_from_mask(const void *mask, int element_bytes, int tokens, int ex
  *
  * With 10% non-zero weights this takes 0.72 bit per weight (the dictionary
  * codes: 0.69), and a weight costs the kernel one LDS read and one
- * multiply-add.  Only for the fixed dictionary (dec is compared with it, once)
- * and 1 <= d_model, d_ff <= SUB1_PREPARED_MAX_WIDTH.
+ * multiply-add.  Only for the fixed dictionary (both prepare calls compare all of dec
+ * with it on the GPU) and 1 <= d_model, d_ff <= SUB1_PREPARED_MAX_WIDTH.
  *
  *   meta_bytes = sub1_moe_prepared_meta_bytes(experts, d_model, d_ff);
  *   sub1_moe_prepared p;
@@ -334,8 +336,11 @@ int sub1_moe_grouped_prepared(const sub1_moe_prepared *prepared, const int32_t *
  *
  * scratch: sub1_moe_batch_scratch_bytes(p, tokens) bytes of device memory, 256-byte
  * aligned, contents arbitrary before and after (0: no such form for these shapes - a
- * row's codes must fit LDS - and the call is refused).  It stops growing at 8192
- * tokens: larger batches run in equal pieces.
+ * row's codes must fit LDS - and the call is refused).  An expert's tokens take
+ * whole blocks of 32 slots: at most tokens + 31 (min(tokens, experts) + 1) slots, of
+ * 4 d_ff + 2 d_model bytes (widths rounded up to 16) and 17 more each - 69 MB for 1024 tokens
+ * of 128 experts with d_model 768 and d_ff 3072, 112 MB for 4096.  It stops growing at
+ * 8192 tokens: larger batches run in equal pieces.
  *
  * sub1_moe_batch_pays: 1 where this is estimated to be faster than
  * sub1_moe_grouped_prepared for `tokens` tokens spread over the experts, 0 otherwise.  Every
@@ -587,10 +592,9 @@ int sub1_test_overstate_wait(int extra);
 
 /*
  * sub1_moe_grouped keeps the compact table it derives from `dec` by the
- * ADDRESS of dec (per device), and the prepare calls remember that they have
- * compared a dec at that address with the fixed dictionary.  Call this before freeing a dec
- * buffer whose address may be handed out again for other contents; NULL drops
- * every cached table.  Synchronises the device.  (A launch that finds other
+ * ADDRESS of dec (per device).  Call this before freeing a dec buffer whose
+ * address may be handed out again for other contents; NULL drops every cached
+ * table.  (The prepare calls compare all of dec every time.)  Synchronises the device.  (A launch that finds other
  * contents at a cached address sets the flag above and the next call derives
  * the tables afresh.)
  */

@@ -4,8 +4,9 @@
 // needs no preparation.  Written for 64-wide wavefronts.  The single product
 // (matvec_wave_kernel) gives a wavefront to a row: lane j takes codeword j of
 // each run of 64, a prefix sum across the lanes places it, a butterfly adds the
-// lanes' sums.  The expert launch (moe_kernel) gives a lane to a row, so a
-// wavefront advances 64 independent code streams without cross-lane traffic.
+// lanes' sums.  The expert launch (moe_kernel) gives a lane to a group of 32
+// codes of a row, whose start a prefix sum finds, or to a whole row where the
+// rows of a wavefront are alike.
 // Either way the work per codeword is proportional to the non-zero weights in
 // it (at most three for the fixed dictionary).
 //
@@ -436,10 +437,11 @@ __global__ __launch_bounds__(64 * kWaves) void decode_kernel(
 // once, and from the words' lengths a prefix sum over the lanes gives the column at
 // which each group starts.
 //
-// What bounds it: LDS gathers of activations (three a codeword, 8 ns a wavefront and
-// compute unit), the words outside the held head of the table (54 ns times the share
-// of lanes that miss), 27 vector instructions a codeword (11 ns).  A wavefront's 64
-// codewords take 16-20 ns.  Switch shapes with shares of zeros between 75 and 98 %,
+// What bounds it: 48 vector instructions a codeword (20 ns a wavefront and compute
+// unit: in the sweep of 2048 c-2048 experts the VALUs are 73 % busy), beside LDS gathers of
+// activations (three a codeword, 8 ns) and the words outside the held head of the
+// table (54 ns times the share of lanes that miss).  A wavefront's 64 codewords take 28 ns
+// there.  Switch shapes with shares of zeros between 75 and 98 %,
 // 64 tokens, us: base 381 -> 74, large 526 -> 105, c-2048 956 -> 230, where the lane per
 // row waited for the longest of 64; with 90 % everywhere 99 -> 51, 109 -> 61, 255 -> 133.
 struct MoeArgs {

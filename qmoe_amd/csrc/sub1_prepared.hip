@@ -425,7 +425,8 @@ __device__ __forceinline__ void emit_rows(const HeldTable &table, const WalkKind
 // as many compute units.  128 base experts (26 million codes): counting takes 59 us
 // (194 with the two-word table in global memory and a code at a time), emitting 112
 // (313; 132 with a store behind every entry instead of every code); both are bound by
-// their instructions, about 60 and 90 a code, emitting also by the stores of lanes that
+// their instructions, about 60 and 100 a code (the VALUs 56 and 58 % busy, the wavefronts
+// waiting a quarter of their time), emitting also by the stores of lanes that
 // fill their chunks at different times.  One code a turn instead of eight (a tenth of
 // the code) measured 93, and 169 before the stores were put together.
 template <bool kEmit>

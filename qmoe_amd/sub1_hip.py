@@ -473,9 +473,10 @@ class PreparedStack:
     def forward_batch(self, x, token_expert, y=None):
         """forward() on the matrix cores, for many tokens per expert: results
         agree with it to rounding, not to the bit, and a token's do not depend
-        on the other tokens.  Scratch memory (about 5 d_ff + 2 d_model bytes a
-        token, up to 8192 tokens' worth) comes from torch's allocator for the
-        call."""
+        on the other tokens.  Scratch memory comes from torch's allocator for
+        the call: an expert's tokens take whole blocks of 32 slots, at most
+        T + 31 (min(T, experts) + 1) of them for T tokens (up to 8192, larger
+        batches run in pieces), of 4 d_ff + 2 d_model bytes each and a few more."""
         dev = self.device
         _lib.check_faults()       # what earlier launches reported (host memory, no sync)
         lib = _lib.load()
