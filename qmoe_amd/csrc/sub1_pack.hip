@@ -81,7 +81,7 @@ struct PackTables {
 std::mutex g_tables_mutex;
 std::vector<int> g_tables_devices;   // where the three arrays are filled
 
-int fill_tables(const PackTables &t) {
+int fill_tables(const PackTables &t, hipStream_t stream) {
   std::vector<int32_t> dec(SUB1_DEC_WORDS), trie(SUB1_TRIE_WORDS);
   int rc = sub1_build_tables(dec.data(), trie.data());
   if (rc) return fail(rc, "sub1_build_tables failed");
@@ -113,27 +113,34 @@ int fill_tables(const PackTables &t) {
   // every string below the border has to be an entry (they are distinct)
   if (short_strings != kStrings - kBorderStrings)
     return fail(SUB1_ERR_INTERNAL, "the dictionary lacks strings below the border");
-  // The caller's stream may be in a capture, which a copy on the default stream fails in
-  // and spoils: a stream of its own, and this thread's calls checked against no capture
+  // A copy on a stream in a capture, or on the default one beside it, fails and spoils the
+  // capture: the copies then take a stream of their own, this thread's calls checked against no
+  // capture.  Only then, because that stream's hardware queue stays with the process, in which
+  // the calls that wait for a word from the GPU take 1 to 3 % longer from then on.
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
-  hipStream_t own = nullptr;
-  hipError_t e = hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  const bool unknown = hipStreamIsCapturing(stream, &capture) != hipSuccess;   // the default stream beside a capture
+  if (unknown) (void)hipGetLastError();
+  const bool aside = unknown || capture != hipStreamCaptureStatusNone;
+  hipStream_t s = stream;
+  hipError_t e = aside ? hipStreamCreateWithFlags(&s, hipStreamNonBlocking) : hipSuccess;
+  const bool own = aside && e == hipSuccess;
   const auto copy = [&](const void *to, const void *from, size_t bytes) {
-    if (e == hipSuccess) e = hipMemcpyAsync(const_cast<void *>(to), from, bytes, hipMemcpyHostToDevice, own);
+    if (e == hipSuccess) e = hipMemcpyAsync(const_cast<void *>(to), from, bytes, hipMemcpyHostToDevice, s);
   };
   copy(t.code, code.data(), code.size() * 2);
   copy(t.border, border.data(), border.size() * 4);
   copy(t.trie, trie.data(), trie.size() * 4);
-  if (e == hipSuccess) e = hipStreamSynchronize(own);
-  if (own) (void)hipStreamDestroy(own);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  if (own) (void)hipStreamDestroy(s);
   (void)hipThreadExchangeStreamCaptureMode(&mode);   // as it was
   return e == hipSuccess ? SUB1_OK : fail(SUB1_ERR_HIP, "filling the encoder's tables: %s", hipGetErrorString(e));
 }
 
 // The three arrays on the current device (2.7 MB a GPU, filled on the first call
 // there and held until the process ends).
-int tables_of_current_device(PackTables *t) {
+int tables_of_current_device(PackTables *t, hipStream_t stream) {
   int device = 0;
   void *code = nullptr, *border = nullptr, *trie = nullptr;
   HIP_TRY(hipGetDevice(&device));
@@ -144,7 +151,7 @@ int tables_of_current_device(PackTables *t) {
         static_cast<const int32_t *>(trie)};
   std::lock_guard<std::mutex> lock(g_tables_mutex);
   if (std::find(g_tables_devices.begin(), g_tables_devices.end(), device) == g_tables_devices.end()) {
-    const int rc = fill_tables(*t);
+    const int rc = fill_tables(*t, stream);
     if (rc) return rc;
     g_tables_devices.push_back(device);
   }
@@ -528,7 +535,7 @@ extern "C" int sub1_pack_count(const int32_t *trie, int32_t *w_tern, int32_t *ro
     return fail(SUB1_ERR_ALIGN, "sub1_pack_count: misaligned pointer");
   hipStream_t s = static_cast<hipStream_t>(stream);
   PackArgs a{};
-  rc = tables_of_current_device(&a.tables);
+  rc = tables_of_current_device(&a.tables, s);
   if (rc) return rc;
   // row_off[0] is zero in the end; until then it says whose trie this is
   zero_word_kernel<<<1, 1, 0, s>>>(row_off);
@@ -570,7 +577,7 @@ extern "C" int sub1_pack_weights_count(const void *w, uint16_t *codes, void *ter
     return fail(SUB1_ERR_ALIGN, "%s: misaligned pointer", who);
   hipStream_t s = static_cast<hipStream_t>(stream);
   PackArgs a{};
-  rc = tables_of_current_device(&a.tables);
+  rc = tables_of_current_device(&a.tables, s);
   if (rc) return rc;
   a.weights = static_cast<const uint16_t *>(w);
   a.codes = codes;
