@@ -188,18 +188,26 @@ __device__ __forceinline__ const uint16_t *row_codes(const KindSource &ks, int e
   return codes + ro[r];
 }
 
-// Both prepare passes walk all rows' codes, a lane to a row, through the fixed
-// dictionary in a form of one word per entry: the pair count in bits 0-3, then up
-// to three non-zeros of seven bits each, the place (0..27) below two bits that are 0
-// for none, 1 for a row min, 2 for a row max.  What bounds them is fetching that
-// word: a wavefront's gather from the 256 KB table costs a compute unit 54 ns, one
-// from LDS 3 ns.  So a compute unit takes one workgroup, persistent, that keeps the
-// table's first 40 000 words in LDS (the low codes are the frequent ones: three
-// quarters of the codes of weights with 90% zeros and more), and a lane asks for
-// eight codes and their eight words at once.
+// Both prepare passes walk all rows' codes, a lane to a row.  What bounds them is the
+// instructions for a code and, before those, fetching its dictionary entry: a wavefront's
+// gather from a table in global memory costs a compute unit 54 ns, one from LDS 3 ns.
+// So a compute unit takes one workgroup, persistent, that keeps a table in LDS, and a
+// lane asks for eight codes and their eight entries at once.
+//
+// Counting needs little of an entry, 16 bits, so that all 65 536 are held, and beside
+// them two more bits of each for the rare gap that takes several steps:
+//   bits 0-3 pairs, 4-5 non-zeros, 6-10 column of the first, 11-15 columns from the
+//   last to the entry's end (0 where there is none); symbols - 1 of the first and the
+//   last non-zero.
+// Emitting needs all of it, a word: pairs in bits 0-3, non-zeros in 4-5, then a byte for
+// each of three: 2 column + symbol - 1, the last one's again where there are fewer.  The
+// first 40 000 words are held (the low codes are the frequent ones: three quarters of
+// the codes of weights with 90% zeros and more).
 constexpr int kWalkThreads = 1024;
 constexpr int kHeldWords = 40000;
+constexpr int kCountWords = SUB1_DICT_ENTRIES / 2 + SUB1_DICT_ENTRIES / 16;   // 16-bit entries, then symbols
 constexpr size_t kWalkLds = kHeldWords * sizeof(uint32_t);
+constexpr size_t kCountLds = kCountWords * sizeof(uint32_t);
 
 struct HeldTable {
   const uint32_t *all;    // global memory
@@ -212,11 +220,21 @@ struct HeldTable {
   }
 };
 
-__device__ __forceinline__ HeldTable hold_table(const uint32_t *table, uint32_t *lds) {
-  for (int i = 4 * threadIdx.x; i < kHeldWords; i += 4 * kWalkThreads)
+struct CountTable {
+  const uint32_t *words;   // global memory: the emitting pass's words
+  const uint32_t *lds;
+  __device__ __forceinline__ uint32_t operator[](uint32_t code) const {
+    return reinterpret_cast<const uint16_t *>(lds)[code];
+  }
+  __device__ __forceinline__ uint32_t symbols(uint32_t code) const {   // bit 0 of the first, bit 1 of the last
+    return lds[SUB1_DICT_ENTRIES / 2 + (code >> 4)] >> (2 * (code & 15u));
+  }
+};
+
+__device__ __forceinline__ void hold_table(const uint32_t *table, uint32_t *lds, int words) {
+  for (int i = 4 * threadIdx.x; i < words; i += 4 * kWalkThreads)
     *reinterpret_cast<uint4 *>(lds + i) = *reinterpret_cast<const uint4 *>(table + i);
   __syncthreads();
-  return HeldTable{table, lds};
 }
 
 // The rows' codes are followed through pointers read from memory; as a global
@@ -227,64 +245,56 @@ __device__ __forceinline__ unaligned_u32x4 eight_codes(global_u16 *codes) {
   return *(const __attribute__((address_space(1))) unaligned_u32x4 *)codes;
 }
 
-// A row's non-zeros as entries.  An entry is the step from the row's position (0 at
-// the start) to the next, 0..127; a longer gap goes over zero columns, as far as each
-// step reaches.  An entry goes to sink.add(step, position after it), sink.end_code()
-// follows every codeword (after add has had at most three entries since the last), and
-// entries of a longer gap go to sink.add_now.  Returns the columns that the codes
-// cover; `at` is the position reached.
-template <class Sink>
-__device__ __forceinline__ int walk_row(const HeldTable &table, const uint16_t *row, int n, int width,
-                                        int &at, Sink &sink) {
+// A row's codes in turn to each(entry, code), eight entries fetched at a time, and the
+// last one to eight of them to last_ones(entry, code), where entries of no pairs and no
+// non-zeros stand in for what is missing to eight.
+template <class Table, class Each, class Last>
+__device__ __forceinline__ void walk_codes(const Table &table, const uint16_t *row, int n, Each &&each,
+                                           Last &&last_ones) {
   global_u16 *codes = (global_u16 *)row;
-  int col = 0;
-  at = 0;
-  auto word = [&](uint32_t w) {
-#pragma unroll
-    for (int s = 0; s < 3; s++) {
-      const uint32_t slot = w >> (4 + 7 * s);
-      const int c = col + static_cast<int>(slot & 31u);
-      if ((slot & 0x60u) && c < width) {   // digits past the width are dropped
-        const int target = position_of(c, 1) + static_cast<int>((slot >> 6) & 1u);
-        // two non-zeros of one entry are 27 columns apart at most: within a step
-        if (s == 0)
-#pragma unroll 1
-          while (target - at > kMaxStep) {
-            const int zero = (at + kMaxStep) / (2 * kZeroPeriod) * (2 * kZeroPeriod);
-            const int step = zero - at;
-            at = zero;
-            sink.add_now(step, at);
-          }
-        const int step = target - at;
-        at = target;
-        sink.add(step, at);
-      }
-    }
-    sink.end_code();
-    col += 2 * static_cast<int>(w & 15u);
-  };
   if (n < 8) {
 #pragma unroll 1
-    for (int i = 0; i < n; i++) word(table[codes[i]]);
-    return col;
+    for (int i = 0; i < n; i++) last_ones(table[codes[i]], static_cast<uint32_t>(codes[i]));
+    return;
   }
   unaligned_u32x4 next = eight_codes(codes);
-#pragma unroll 1
-  for (int i = 0; i < n; i += 8) {
-    const unaligned_u32x4 four = next;
-    // the row's last, partial eight is read from eight codes before its end
-    if (i + 8 < n) next = eight_codes(codes + min(i + 8, n - 8));
-    const int skip = max(i + 8 - n, 0);
-    uint32_t w[8];
+  uint32_t code[8], w[8];
+  auto look_up = [&]() {
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-      w[j] = table[(j & 1) ? four[j / 2] >> 16 : four[j / 2] & 0xffffu];
-      if (j < skip) w[j] = 0u;
+      code[j] = (j & 1) ? next[j / 2] >> 16 : next[j / 2] & 0xffffu;
+      w[j] = table[code[j]];
     }
+  };
+  int i = 0;
+#pragma unroll 1
+  for (; i + 8 < n; i += 8) {
+    look_up();
+    next = eight_codes(codes + min(i + 8, n - 8));   // the last, partial eight: from eight before the end
 #pragma unroll
-    for (int j = 0; j < 8; j++) word(w[j]);
+    for (int j = 0; j < 8; j++) each(w[j], code[j]);
   }
-  return col;
+  look_up();
+#pragma unroll
+  for (int j = 0; j < 8; j++) last_ones(j < i + 8 - n ? 0u : w[j], code[j]);
+}
+
+// A row's non-zeros as entries.  An entry is the step from the row's position (0 at
+// the start) to the next, 0..127; a longer gap goes over zero columns, as far as each
+// step reaches: the place that such a step ends at.
+__device__ __forceinline__ int farthest_zero(int at) {
+  return (at + kMaxStep) / (2 * kZeroPeriod) * (2 * kZeroPeriod);
+}
+// The position of 2 column + symbol - 1.  (Written out: the compiler takes one more.)
+__device__ __forceinline__ int position_at(int a) {
+  int p;
+  asm("v_lshl_add_u32 %0, %1, 1, %2" : "=v"(p) : "v"(a >> 5), "v"(a + 2));
+  return p;
+}
+// n ? a : b, without a branch around what may differ from lane to lane.
+__device__ __forceinline__ int pick(int n, int a, int b) {
+  asm volatile("" : "+v"(a), "+v"(b));
+  return n ? a : b;
 }
 
 // A prepare pass over all rows of one kind of matrices, 64 at a time; kinds with
@@ -301,22 +311,22 @@ struct WalkKind {
 struct WalkArgs {
   WalkKind k[2];
   int kinds, count;
-  const uint32_t *table;
+  const uint32_t *table;         // the emitting pass's words, all of them
+  const uint32_t *count_table;   // what the counting pass holds in LDS
   int32_t *status;
   uint2 *stream;
   uint16_t *ckpt;
 };
 
-struct EntryCount {
-  int entries = 0;
-  __device__ __forceinline__ void add(int, int) { entries++; }
-  __device__ __forceinline__ void add_now(int, int) { entries++; }
-  __device__ __forceinline__ void end_code() {}
-};
+// Columns from a row's last non-zero to the next from which on one step may not do:
+// 60 columns are 63 or 64 physical ones, 126 to 129 positions.
+constexpr int kLongGap = 60;
 
 // How many entries the non-zeros of every row take (the step onto a zero column
-// that a padded row makes after them is not counted: it fits the padding).
-__device__ __forceinline__ void count_rows(const HeldTable &table, const WalkKind &k, int count,
+// that a padded row makes after them is not counted: it fits the padding).  An entry's
+// non-zeros are 27 columns apart at most, so only the gap before the first of them can
+// take more than one.
+__device__ __forceinline__ void count_rows(const CountTable &table, const WalkKind &k, int count,
                                            int64_t task, int32_t *status) {
   // rows of a task: from row `first` of a matrix on, and of the next ones
   const int64_t g = task * 64 + (threadIdx.x & 63);
@@ -325,13 +335,46 @@ __device__ __forceinline__ void count_rows(const HeldTable &table, const WalkKin
   const uint32_t past = static_cast<uint32_t>(g - static_cast<int64_t>(first_e) * k.height);
   const int e = first_e + static_cast<int>(past / static_cast<uint32_t>(k.height));
   const int r = static_cast<int>(past % static_cast<uint32_t>(k.height));
-  int n, at;
-  EntryCount sink;
+  int n;
   const uint16_t *codes = row_codes(k.source, e, r, k.height, k.width, n);
-  const int covered = walk_row(table, codes, n, k.width, at, sink);
+  int col = 0, entries = 0;
+  int since = 0;       // columns from the last non-zero's to col (from column 0 where there is none)
+  int holder = -1;     // the code that holds the last non-zero
+  auto step = [&](uint32_t w, uint32_t code, bool over) {
+    const int nonzeros = (w >> 4) & 3u, first = (w >> 6) & 31u, tail = w >> 11;
+    const int pairs = w & 15u;
+    if (__builtin_expect(since + first >= kLongGap || over, 0)) {
+      // digits past the width are dropped: which those are, the whole entry says
+      int inside = nonzeros;
+      if (over) {
+        const uint32_t all = table.words[code];
+        inside = 0;
+        for (int j = 0; j < nonzeros; j++)
+          if (2 * col + static_cast<int>((all >> (8 + 8 * j)) & 255u) < 2 * k.width) inside++;
+      }
+      if (inside) {
+        int at = holder < 0 ? 0 : position_at(2 * (col - since)) + static_cast<int>((table.symbols(holder) >> 1) & 1u);
+        const int target = position_at(2 * (col + first)) + static_cast<int>(table.symbols(code) & 1u);
+        while (target - at > kMaxStep) {
+          at = farthest_zero(at);
+          entries++;
+        }
+      }
+      entries -= nonzeros - inside;   // what is added below; nothing follows a dropped digit
+    }
+    entries += nonzeros;
+    col += 2 * pairs;
+    since = pick(nonzeros, tail, since + 2 * pairs);
+    holder = pick(nonzeros, static_cast<int>(code), holder);
+  };
+  // (only a row's last code can reach past its width, if its codes cover it exactly)
+  walk_codes(table, codes, n, [&](uint32_t w, uint32_t code) { step(w, code, false); },
+             [&](uint32_t w, uint32_t code) {
+               step(w, code, (w & 0x30u) && col + 2 * static_cast<int>(w & 15u) > k.width);
+             });
   // a row's codes cover its width rounded up to a whole pair, exactly
-  if (covered != ((k.width + 1) & ~1)) atomicAdd(&status[0], 1);
-  k.row_len[g] = static_cast<uint16_t>(min(sink.entries, kMaxRowEntries));
+  if (col != ((k.width + 1) & ~1)) atomicAdd(&status[0], 1);
+  k.row_len[g] = static_cast<uint16_t>(min(entries, kMaxRowEntries));
 }
 
 // Position checkpoints.  For every slice and every group of kGroupChunks chunks,
@@ -343,51 +386,38 @@ __device__ __forceinline__ int64_t checkpoint_entry(uint32_t slice_base, int64_t
   return static_cast<int64_t>(slice_base / kGroupChunks) + slice;
 }
 
-// A row's entries, nine to a chunk.  The lanes of a wavefront fill their chunks at
-// different times, so that nearly every place that may store one is taken by a few of
-// them: a codeword's entries, at most three, fill one at most, and it is stored in one
-// place behind them.
+// A row's entries, nine to a chunk, a codeword's (up to three) at a time.  The lanes of a
+// wavefront fill their chunks at different times, so that nearly every place that may
+// store one is taken by a few of them: there is one such place to a codeword.
 struct ChunkSink {
-  uint2 *d;
-  uint16_t *ck;
-  int nch;
-  int c = 0, q = 0;
-  uint32_t lo = 0, hi = 0;              // the chunk so far, its newest entry in bits 56..62
-  uint32_t full_lo = 0, full_hi = 0;    // one that is to be stored, and the position behind it
-  int full_at = -1;
-  __device__ __forceinline__ void shift_in(int step) {
-    lo = __builtin_amdgcn_alignbit(hi, lo, kFieldBits);
-    hi = (hi >> kFieldBits) | static_cast<uint32_t>(step) << 24;
-    q++;
+  char *chunks, *ckpt;          // the slice's; the same in all lanes
+  uint32_t end;                 // bytes of its chunks
+  uint32_t at;                  // of this lane's next one: 512 c + 8 lane
+  int bits = 0;                 // that it holds, seven an entry
+  uint32_t lo = 0, hi = 0;
+  // The chunk is stored and the next one begins with the entries in `rest` (two at most);
+  // `position`: what the row has reached with them.
+  __device__ __forceinline__ void store(uint32_t rest, int position) {
+    if (at < end) *reinterpret_cast<uint2 *>(chunks + at) = make_uint2(lo, hi & 0x7fffffffu);
+    at += 512;
+    if ((at & (kGroupChunks - 1) << 9) == 0 && at < end)
+      *reinterpret_cast<uint16_t *>(ckpt + ((at >> 12) * 128 + (at & 511u) / 4)) =
+          static_cast<uint16_t>(position - static_cast<int>((rest & 127u) + (rest >> kFieldBits)));
+    lo = rest;
+    hi = 0;
+    bits -= kFields * kFieldBits;
   }
-  __device__ __forceinline__ void store(uint32_t l, uint32_t h, int after) {
-    if (c < nch) d[c * 64] = make_uint2(l, h);   // the slice is as long as its longest row
-    c++;
-    if (c % kGroupChunks == 0 && c < nch) ck[(c / kGroupChunks) * 64] = static_cast<uint16_t>(after);
-  }
-  __device__ __forceinline__ void add(int step, int after) {
-    shift_in(step);
-    if (q == kFields) {
-      q = 0;
-      full_lo = lo;
-      full_hi = hi;
-      full_at = after;
-    }
-  }
-  __device__ __forceinline__ void end_code() {
-    if (full_at >= 0) {
-      store(full_lo, full_hi, full_at);
-      full_at = -1;
-    }
-  }
-  __device__ __forceinline__ void add_now(int step, int after) {
-    shift_in(step);
-    if (q == kFields) {
-      q = 0;
-      store(lo, hi, after);
-    }
+  // `n` entries (0 to 3), the first in the lowest bits of `packed`.
+  __device__ __forceinline__ void add(uint32_t packed, int n, int position) {
+    const unsigned long long shifted = static_cast<unsigned long long>(packed) << bits;
+    lo |= static_cast<uint32_t>(shifted);
+    hi |= static_cast<uint32_t>(shifted >> 32);
+    const int room = kFields * kFieldBits - bits;
+    bits += kFieldBits * n;
+    if (bits >= kFields * kFieldBits) store(packed >> room, position);
   }
 };
+static_assert(kGroupChunks == 8, "a group's chunks are 4096 bytes");
 
 // A slice's rows, a lane each, into the interleaved stream, nine entries to a chunk;
 // a row shorter than its slice then steps onto the next zero column and stays there
@@ -398,51 +428,88 @@ __device__ __forceinline__ void emit_rows(const HeldTable &table, const WalkKind
   const int lane = threadIdx.x & 63;
   const int e = static_cast<int>(slice / k.slices);
   const int ridx = k.row_idx[slice * 64 + lane];
-  const uint32_t base = k.slice_base[slice];
-  const int len = k.slice_len[slice];
-  const int nch = chunks_of(len);
-  uint2 *d = stream + static_cast<int64_t>(base) * 64 + lane;
-  uint16_t *ck = ckpt + checkpoint_entry(base, k.first_slice + slice) * 64 + lane;
-  ChunkSink sink{d, ck, nch};
-  ck[0] = 0;
+  const uint32_t base = __builtin_amdgcn_readfirstlane(k.slice_base[slice]);
+  const int len = __builtin_amdgcn_readfirstlane(k.slice_len[slice]);
+  ChunkSink sink{reinterpret_cast<char *>(stream + static_cast<int64_t>(base) * 64),
+                 reinterpret_cast<char *>(ckpt + checkpoint_entry(base, k.first_slice + slice) * 64),
+                 512u * chunks_of(len), 8u * lane};
+  *reinterpret_cast<uint16_t *>(sink.ckpt + 2 * lane) = 0;
   int at = 0;
   if (ridx != 0xffff) {
     int n;
     const uint16_t *codes = row_codes(k.source, e, ridx, k.height, k.width, n);
-    walk_row(table, codes, n, k.width, at, sink);
-    if (sink.c * kFields + sink.q < len && (at >> 1) % kZeroPeriod != 0) {   // padding follows: it must read zeros
+    int from = 0;   // twice the column at which the codeword starts
+    auto step = [&](uint32_t w, uint32_t) {
+      int nonzeros = (w >> 4) & 3u;
+      const int a1 = from + static_cast<int>((w >> 16) & 255u), a2 = from + static_cast<int>(w >> 24);
+      const int p0 = position_at(from + static_cast<int>((w >> 8) & 255u));
+      int p1 = position_at(a1), p2 = position_at(a2);
+      const int end = from + 4 * static_cast<int>(w & 15u);
+      if (__builtin_expect(p0 - at > kMaxStep || end > 2 * k.width, 0)) {
+        if (end > 2 * k.width) {   // digits past the width are dropped
+          if (a2 >= 2 * k.width) {
+            nonzeros = min(nonzeros, 2);
+            p2 = p1;
+          }
+          if (a1 >= 2 * k.width) {
+            nonzeros = min(nonzeros, 1);
+            p1 = p2 = p0;
+          }
+          if (from + static_cast<int>((w >> 8) & 255u) >= 2 * k.width) nonzeros = 0;
+        }
+        if (nonzeros)
+#pragma unroll 1
+          while (p0 - at > kMaxStep) {
+            const int zero = farthest_zero(at);
+            sink.add(zero - at, 1, zero);
+            at = zero;
+          }
+      }
+      const int packed = (p0 - at) | (p1 - p0) << kFieldBits | (p2 - p1) << (2 * kFieldBits);
+      at = pick(nonzeros, p2, at);
+      sink.add(static_cast<uint32_t>(pick(nonzeros, packed, 0)), nonzeros, at);
+      from = end;
+    };
+    walk_codes(table, codes, n, step, step);
+    if (static_cast<int>(sink.at >> 9) * (kFields * kFieldBits) + sink.bits < len * kFieldBits && (at >> 1) % kZeroPeriod != 0) {
+      // padding follows: it must read zeros
       const int zero = (at + 2 * kZeroPeriod - 1) / (2 * kZeroPeriod) * (2 * kZeroPeriod);
-      const int step = zero - at;
+      sink.add(zero - at, 1, zero);
       at = zero;
-      sink.add_now(step, at);
     }
   }
 #pragma unroll 1
-  while (sink.c < nch) sink.add_now(0, at);
+  while (sink.at < sink.end) sink.store(0u, at);
 }
 
-// Task t goes to workgroup t mod grid first: a matrix of a few slices is spread over
-// as many compute units.  128 base experts (26 million codes): counting takes 59 us
-// (194 with the two-word table in global memory and a code at a time), emitting 112
-// (313; 132 with a store behind every entry instead of every code); both are bound by
-// their instructions, about 60 and 100 a code (the VALUs 56 and 58 % busy, the wavefronts
-// waiting a quarter of their time), emitting also by the stores of lanes that
-// fill their chunks at different times.  One code a turn instead of eight (a tenth of
-// the code) measured 93, and 169 before the stores were put together.
+// Task t goes to workgroup t mod grid: a matrix of a few slices is spread over as many
+// compute units.  Within it the wavefronts take the next one when they are done: a row of
+// wo has four times the codes of one of wi, and dealt out beforehand the busiest wavefront
+// has 1.7 times the average (counting 40 us, emitting 96).
+// 128 base experts (26 million codes): counting takes 32 us, 22 vector instructions a code
+// (64 with entry by entry of a whole word, 60 instructions); emitting 84 and about 65 (113
+// with a place that may store behind every entry, 99 instructions).  Both are bound by
+// issuing those, beside 6 us of filling LDS.  (32 codes asked for together instead of 8,
+// a cache line's worth: 37 and 81 us.)
 template <bool kEmit>
 __global__ __launch_bounds__(kWalkThreads) void walk_rows_kernel(WalkArgs a) {
   extern __shared__ __align__(16) uint32_t held[];
-  const HeldTable table = hold_table(a.table, held);
-  const int64_t step = static_cast<int64_t>(gridDim.x) * (kWalkThreads / 64);
-  int64_t task = blockIdx.x + static_cast<int64_t>(gridDim.x) * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (int i = 0; i < a.kinds; i++) {
-    for (; task < a.k[i].tasks; task += step) {
-      if (kEmit)
-        emit_rows(table, a.k[i], task, a.stream, a.ckpt);
-      else
-        count_rows(table, a.k[i], a.count, task, a.status);
-    }
-    task -= a.k[i].tasks;
+  __shared__ int s_turn;
+  if (threadIdx.x == 0) s_turn = 0;
+  hold_table(kEmit ? a.table : a.count_table, held, kEmit ? kHeldWords : kCountWords);
+  const int64_t all = a.k[0].tasks + (a.kinds == 2 ? a.k[1].tasks : 0);
+  for (;;) {
+    int turn = 0;
+    if ((threadIdx.x & 63) == 0) turn = atomicAdd(&s_turn, 1);
+    int64_t task = blockIdx.x + static_cast<int64_t>(gridDim.x) * __builtin_amdgcn_readfirstlane(turn);
+    if (task >= all) break;
+    const bool second = task >= a.k[0].tasks;
+    if (second) task -= a.k[0].tasks;
+    const WalkKind &k = a.k[second ? 1 : 0];
+    if (kEmit)
+      emit_rows(HeldTable{a.table, held}, k, task, a.stream, a.ckpt);
+    else
+      count_rows(CountTable{a.table, held}, k, a.count, task, a.status);
   }
 }
 
@@ -2377,42 +2444,55 @@ __global__ __launch_bounds__(kMaxThreads) void matvec_group_kernel(PreparedArgs 
 // dec to compare it there, as it was done first, took 9 ms a call, two calls to
 // a layer; the kernel and reading its answer back take about 20 us.
 static __device__ __align__(16) int32_t fixed_dec[SUB1_DEC_WORDS];
-static __device__ __align__(16) uint32_t fixed_slots[SUB1_DICT_ENTRIES];   // the walks' one-word form
+// ... and as the walks read it: whole words, and what counting holds in LDS.
+static __device__ __align__(16) uint32_t fixed_words[SUB1_DICT_ENTRIES];
+static __device__ __align__(16) uint32_t fixed_counts[kCountWords];
 std::mutex g_fixed_mutex;
 std::vector<int> g_fixed_devices;   // where fixed_dec is filled
 
-int fixed_tables_of_current_device(const int32_t **dec, const uint32_t **slots) {
+struct FixedTables {
+  const int32_t *dec;
+  const uint32_t *words, *counts;
+};
+int fixed_tables_of_current_device(FixedTables *out) {
   int device = 0;
-  void *at_dec = nullptr, *at_slots = nullptr;
+  void *at_dec = nullptr, *at_words = nullptr, *at_counts = nullptr;
   HIP_TRY(hipGetDevice(&device));
   HIP_TRY(hipGetSymbolAddress(&at_dec, HIP_SYMBOL(fixed_dec)));
-  HIP_TRY(hipGetSymbolAddress(&at_slots, HIP_SYMBOL(fixed_slots)));
+  HIP_TRY(hipGetSymbolAddress(&at_words, HIP_SYMBOL(fixed_words)));
+  HIP_TRY(hipGetSymbolAddress(&at_counts, HIP_SYMBOL(fixed_counts)));
   std::lock_guard<std::mutex> lock(g_fixed_mutex);
   if (std::find(g_fixed_devices.begin(), g_fixed_devices.end(), device) == g_fixed_devices.end()) {
     std::vector<int32_t> table(SUB1_DEC_WORDS);
     const int rc = sub1_build_tables(table.data(), nullptr);
     if (rc) return fail(rc, "sub1_build_tables failed");
-    std::vector<uint32_t> words(SUB1_DICT_ENTRIES);
+    std::vector<uint32_t> words(SUB1_DICT_ENTRIES), counts(kCountWords);
     for (int e = 0; e < SUB1_DICT_ENTRIES; e++) {
       // digit d of entry e is (dec[2e + d/14] >> (4 + 2 (d % 14))) & 3, the low nibble of
       // dec[2e] its pair count (reference sub1.py:60-72, sub1_cuda_kernel.cu:186-192)
-      uint32_t w = static_cast<uint32_t>(table[2 * e]) & 15u;
+      const uint32_t pairs = static_cast<uint32_t>(table[2 * e]) & 15u;
+      uint32_t place[3] = {0, 0, 0};   // 2 digit + symbol - 1
       int n = 0;
       for (int d = 0; d < 28; d++) {
         const uint32_t t = (static_cast<uint32_t>(table[2 * e + d / 14]) >> (4 + 2 * (d % 14))) & 3u;
         if (t == 0) continue;
-        if (t == 3 || n == 3)
+        if (t == 3 || n == 3 || d >= 2 * static_cast<int>(pairs))
           return fail(SUB1_ERR_INTERNAL, "dictionary entry %d is outside the form of the walks", e);
-        w |= (static_cast<uint32_t>(d) | t << 5) << (4 + 7 * n++);
+        for (int j = n; j < 3; j++) place[j] = 2u * d + t - 1;
+        n++;
       }
-      words[e] = w;
+      words[e] = pairs | static_cast<uint32_t>(n) << 4 | place[0] << 8 | place[1] << 16 | place[2] << 24;
+      const uint32_t tail = n ? 2 * pairs - place[2] / 2 : 0u;
+      counts[e / 2] |= (pairs | static_cast<uint32_t>(n) << 4 | place[0] / 2 << 6 | tail << 11) << (16 * (e & 1));
+      counts[SUB1_DICT_ENTRIES / 2 + e / 16] |= ((place[0] & 1u) | (place[2] & 1u) << 1) << (2 * (e & 15));
     }
     HIP_TRY(hipMemcpy(at_dec, table.data(), table.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(at_slots, words.data(), words.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(at_words, words.data(), words.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(at_counts, counts.data(), counts.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
     g_fixed_devices.push_back(device);
   }
-  *dec = static_cast<const int32_t *>(at_dec);
-  *slots = static_cast<const uint32_t *>(at_slots);
+  *out = {static_cast<const int32_t *>(at_dec), static_cast<const uint32_t *>(at_words),
+          static_cast<const uint32_t *>(at_counts)};
   return SUB1_OK;
 }
 
@@ -2440,13 +2520,15 @@ int name_bad_pointer(const void *const *table, int count, size_t align, const ch
 }
 
 // dec and the pointer tables, looked at on the GPU; `word` is a device word to
-// leave the answer in, *slots receives the dictionary as the walks read it.
+// leave the answer in; the walk's tables receive the dictionary as it reads it.
 // Synchronises the stream.
-int check_on_device(const Source &src, int32_t *word, const uint32_t **slots, hipStream_t s,
+int check_on_device(const Source &src, int32_t *word, WalkArgs &w, hipStream_t s,
                     const char *who) {
-  const int32_t *fixed = nullptr;
-  int rc = fixed_tables_of_current_device(&fixed, slots);
+  FixedTables fixed;
+  int rc = fixed_tables_of_current_device(&fixed);
   if (rc) return rc;
+  w.table = fixed.words;
+  w.count_table = fixed.counts;
   const char *const names[3] = {"w_comp", "row_off", "ter_minmax"};
   PointerTables pt{};
   pt.count = src.count;
@@ -2462,7 +2544,7 @@ int check_on_device(const Source &src, int32_t *word, const uint32_t **slots, hi
     }
   }
   zero_words_kernel<<<1, 64, 0, s>>>(word, 1);
-  check_source_kernel<<<kCheckBlocks, 256, 0, s>>>(src.dec, fixed, pt, word);
+  check_source_kernel<<<kCheckBlocks, 256, 0, s>>>(src.dec, fixed.dec, pt, word);
   HIP_TRY(hipGetLastError());
   int32_t found = 0;
   HIP_TRY(hipMemcpyAsync(&found, word, sizeof found, hipMemcpyDeviceToHost, s));
@@ -2603,9 +2685,10 @@ int launch_walk(const Source &src, const MetaLayout &m, WalkArgs &w, hipStream_t
   int device = 0, cus = 0;
   HIP_TRY(hipGetDevice(&device));
   HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+  constexpr size_t lds = kEmit ? kWalkLds : kCountLds;
   HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(walk_rows_kernel<kEmit>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kWalkLds)));
-  walk_rows_kernel<kEmit><<<static_cast<unsigned>(std::min<int64_t>(tasks, cus)), kWalkThreads, kWalkLds, s>>>(w);
+                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+  walk_rows_kernel<kEmit><<<static_cast<unsigned>(std::min<int64_t>(tasks, cus)), kWalkThreads, lds, s>>>(w);
   HIP_TRY(hipGetLastError());
   return SUB1_OK;
 }
@@ -2620,7 +2703,7 @@ int prepare_layout(const Source &src, void *meta, int64_t meta_bytes, LayoutResu
   char *base = static_cast<char *>(meta);
   int32_t *status = reinterpret_cast<int32_t *>(base + m.status);
   WalkArgs w{};
-  int rc = check_on_device(src, status + 3, &w.table, s, who);
+  int rc = check_on_device(src, status + 3, w, s, who);
   if (rc) return rc;
   int32_t *counts = reinterpret_cast<int32_t *>(base + m.counts);
   zero_words_kernel<<<1, 64, 0, s>>>(status, 3);
@@ -2686,7 +2769,7 @@ int prepare_codes(const Source &src, const Prepared &p, hipStream_t s, const cha
       p.code_bytes < p.total_chunks * 512 + (p.total_chunks / kGroupChunks + nslices + 1) * 128)
     return fail(SUB1_ERR_SHAPE, "%s: buffers smaller than the layout needs", who);
   WalkArgs w{};
-  const int rc = check_on_device(src, reinterpret_cast<int32_t *>(base + m.status) + 3, &w.table, s, who);
+  const int rc = check_on_device(src, reinterpret_cast<int32_t *>(base + m.status) + 3, w, s, who);
   if (rc) return rc;
   uint2 *stream = static_cast<uint2 *>(const_cast<void *>(p.codes));
   uint16_t *ckpt = reinterpret_cast<uint16_t *>(stream + p.total_chunks * 64);

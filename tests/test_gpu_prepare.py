@@ -54,6 +54,38 @@ def test_prepared_rows_come_back_whole(gpu, height, width, shares):
     assert torch.equal(y[0], values.gather(1, symbols[:, column:column + 1].long())[:, 0])
 
 
+@pytest.mark.parametrize('d_model,d_ff', [(303, 250), (64, 1400), (1024, 65), (229, 3001)])
+def test_long_gaps_and_dropped_digits_are_counted_as_they_are_written(gpu, oracle, d_model, d_ff):
+    """Gaps about the longest step (59 to 64 columns, at every column of sixteen and with
+    either symbol at both ends), gaps of many steps, rows of one code, of eight and of nine,
+    and digits past an odd width: as many entries as the oracle has, and the symbols back."""
+    sub1, op = gpu
+    triples, want, entries = [], [], 0
+    for kind, (height, width) in enumerate(((d_ff, d_model), (d_model, d_ff))):
+        even = (width + 1) // 2 * 2
+        g = torch.Generator().manual_seed(height * width)
+        symbols = torch.zeros((height, even), dtype=torch.uint8)
+        for r in range(height):
+            at = int(torch.randint(0, 70, (1,), generator=g))
+            while at < even:
+                symbols[r, at] = 1 + int(torch.randint(0, 2, (1,), generator=g))
+                near = int(torch.randint(58, 66, (1,), generator=g))
+                at += [near, near, 1, 2, 14, near + 60, 28 * 7, 400][int(torch.randint(0, 8, (1,), generator=g))]
+        symbols[:, even - 1] = torch.randint(0, 3, (height,), generator=g)   # past the width, where that is odd
+        symbols[0], symbols[1] = 0, 1
+        w_comp, row_off = packed(gpu, symbols.cuda())
+        codes, offsets = w_comp.cpu().numpy().view('uint16'), row_off.tolist()
+        for r in range(height):
+            # (the oracle's last entry goes from the last non-zero onto a zero column: not counted)
+            entries += max(len(oracle.gap_entries(codes[offsets[r]:offsets[r + 1]], width)) - 1, 0)
+        triples.append([(w_comp, row_off, torch.ones(2 * height, dtype=torch.bfloat16, device='cuda'))])
+        want.append(symbols[:, :width].cuda())
+    prepared = op.PreparedStack.from_layers(sub1.DEC[0], *triples)
+    assert prepared.entry_counts()[1] == entries
+    for kind in (0, 1):
+        assert torch.equal(prepared.decode(0, kind), want[kind])
+
+
 def test_preparing_names_a_bad_pointer(gpu):
     """The pointer tables are looked over on the GPU before any of them is
     followed; the message names the matrix."""
