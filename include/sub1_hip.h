@@ -123,6 +123,13 @@ int sub1_pack_weights_emit(const uint16_t *codes, const int32_t *row_off, int16_
                            int height, int width, void *stream);
 
 /*
+ * The first of the two, and *total (int32 in host memory) receives row_off[H]: the call
+ * returns once it is known.  Not for a stream that is being captured.
+ */
+int sub1_pack_weights_total(const void *w, uint16_t *codes, void *ter_minmax, int32_t *row_off,
+                            int32_t *total, int height, int width, void *stream);
+
+/*
  * Decoder without the product, for checking: out_tern (uint8 [H, W], symbols)
  * and/or out_w (bf16 [H, W], dequantised weights) may each be NULL.  What the
  * Python `decompress` of reference test.py:103-115 computes.
@@ -132,6 +139,15 @@ int sub1_pack_weights_emit(const uint16_t *codes, const int32_t *row_off, int16_
 int sub1_decode(const int32_t *dec, const int16_t *w_comp, const int32_t *row_off,
                 const void *ter_minmax, uint8_t *out_tern, void *out_w,
                 int32_t *bad_rows, int height, int width, void *stream);
+
+/*
+ * The same, and *bad_rows (int32 in host memory) receives the number of such rows: the
+ * call returns once it is known, which is when the launch's last workgroup is done.  Not
+ * for a stream that is being captured.
+ */
+int sub1_decode_counted(const int32_t *dec, const int16_t *w_comp, const int32_t *row_off,
+                        const void *ter_minmax, uint8_t *out_tern, void *out_w,
+                        int32_t *bad_rows, int height, int width, void *stream);
 
 /*
  * One MoE layer's expert FFNs in ONE persistent launch: for every token t

@@ -75,7 +75,9 @@ PROTOTYPES = {
     'sub1_pack_emit': (_int, [_vp, _vp, _vp, _int, _int, _vp]),
     'sub1_pack_weights_count': (_int, [_vp] * 4 + [_int, _int, _vp]),
     'sub1_pack_weights_emit': (_int, [_vp] * 3 + [_int, _int, _vp]),
+    'sub1_pack_weights_total': (_int, [_vp] * 4 + [ctypes.POINTER(ctypes.c_int32), _int, _int, _vp]),
     'sub1_decode': (_int, [_vp] * 7 + [_int, _int, _vp]),
+    'sub1_decode_counted': (_int, [_vp] * 6 + [ctypes.POINTER(ctypes.c_int32), _int, _int, _vp]),
     'sub1_moe_workspace_bytes': (_i64, [_int, _int]),
     'sub1_moe_grouped': (_int, [ctypes.POINTER(MoeStack), _vp, _vp, _vp, _int, _vp,
                                 _i64, _vp]),

@@ -74,6 +74,41 @@ __device__ __forceinline__ void raise_fault(int32_t *sticky, int word) {
   __hip_atomic_store(&sticky[word], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// What a kernel tells a host that waits for it (a total, a count): words in pinned host
+// memory, each with the call's ticket over its value, so that they need no clearing, no
+// order among them and no copy, and the kernels after it run on while the host goes on
+// (a copy to the host and the synchronisation with it: 25 to 45 us with the GPU idle; a word
+// seen by a host that looks for it: 3).  A slot belongs to one call at a time, whatever its
+// thread, stream or device.
+constexpr int kAnswerWords = 8;
+struct Answer {
+  unsigned long long *words;     // pinned host memory as the GPU addresses it
+  unsigned long long *counter;   // a word of device memory, zero, and left at zero
+  uint32_t ticket;
+};
+__device__ __forceinline__ void tell(const Answer &a, int word, int32_t value) {
+  __hip_atomic_store(&a.words[word], static_cast<unsigned long long>(a.ticket) << 32 | static_cast<uint32_t>(value),
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+class AnswerSlot {
+ public:
+  AnswerSlot() = default;
+  AnswerSlot(const AnswerSlot &) = delete;
+  AnswerSlot &operator=(const AnswerSlot &) = delete;
+  ~AnswerSlot();
+  // Before the launch.  Refuses a stream that is being captured: nothing runs there that
+  // could answer.
+  int take(hipStream_t stream, const char *who);
+  Answer answer() const { return answer_; }
+  // After it: the first `n` words.
+  int wait(hipStream_t stream, int n, int32_t *values, const char *who);
+
+ private:
+  int slot_ = -1;
+  Answer answer_{};
+};
+
 // Control words at the head of an expert launch's workspace.  The caller zeroes
 // the workspace once; every launch leaves the words it counts with at zero
 // again (the last workgroup out clears the ticket, the last workgroup that

@@ -18,8 +18,11 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
+#include <condition_variable>
 #include <cstdarg>
 #include <cstdio>
+#include <cstring>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -90,6 +93,78 @@ int64_t wait_limit_ticks() {
 }
 
 int expect_extra() { return g_expect_extra.load(); }
+
+namespace {
+constexpr int kAnswerSlots = 64;   // calls that may wait at once; further ones wait for a slot
+std::mutex g_answer_mutex;
+std::condition_variable g_answer_free;
+std::vector<int> g_answer_slots;   // the free ones
+unsigned long long *g_answer_host = nullptr, *g_answer_device = nullptr;   // 4 KB, held until the process ends
+std::atomic<uint32_t> g_answer_ticket{0};
+static __device__ unsigned long long answer_counters[kAnswerSlots];
+}  // namespace
+
+int AnswerSlot::take(hipStream_t stream, const char *who) {
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();   // (the launch will say)
+  if (capture != hipStreamCaptureStatusNone)
+    return fail(SUB1_ERR_HIP, "%s: waits for the GPU, which a stream that is being captured cannot", who);
+  void *counters = nullptr;
+  HIP_TRY(hipGetSymbolAddress(&counters, HIP_SYMBOL(answer_counters)));
+  std::unique_lock<std::mutex> lock(g_answer_mutex);
+  if (!g_answer_host) {
+    void *host = nullptr, *device = nullptr;
+    const size_t bytes = kAnswerSlots * kAnswerWords * sizeof(unsigned long long);
+    HIP_TRY(hipHostMalloc(&host, bytes, hipHostMallocPortable | hipHostMallocMapped));
+    memset(host, 0, bytes);
+    HIP_TRY(hipHostGetDevicePointer(&device, host, 0));
+    g_answer_host = static_cast<unsigned long long *>(host);
+    g_answer_device = static_cast<unsigned long long *>(device);
+    for (int i = 0; i < kAnswerSlots; i++) g_answer_slots.push_back(i);
+  }
+  g_answer_free.wait(lock, [] { return !g_answer_slots.empty(); });
+  slot_ = g_answer_slots.back();
+  g_answer_slots.pop_back();
+  answer_.words = g_answer_device + slot_ * kAnswerWords;
+  answer_.counter = static_cast<unsigned long long *>(counters) + slot_;
+  do answer_.ticket = ++g_answer_ticket;
+  while (answer_.ticket == 0);   // what the words hold at first
+  return SUB1_OK;
+}
+
+AnswerSlot::~AnswerSlot() {
+  if (slot_ < 0) return;
+  {
+    std::lock_guard<std::mutex> lock(g_answer_mutex);
+    g_answer_slots.push_back(slot_);
+  }
+  g_answer_free.notify_one();
+}
+
+int AnswerSlot::wait(hipStream_t stream, int n, int32_t *values, const char *who) {
+  const unsigned long long *words = g_answer_host + slot_ * kAnswerWords;
+  auto arrived = [&]() {
+    for (int i = 0; i < n; i++) {
+      const unsigned long long v = __atomic_load_n(&words[i], __ATOMIC_RELAXED);
+      if (static_cast<uint32_t>(v >> 32) != answer_.ticket) return false;
+      values[i] = static_cast<int32_t>(static_cast<uint32_t>(v));
+    }
+    return true;
+  };
+  // looked for over the time that a layer's passes may take, then waited for
+  const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(5);
+  do {
+    for (int i = 0; i < 64; i++) {
+      if (arrived()) return SUB1_OK;
+      __builtin_ia32_pause();
+    }
+  } while (std::chrono::steady_clock::now() < until);
+  const hipError_t e = hipStreamSynchronize(stream);
+  if (e == hipSuccess && arrived()) return SUB1_OK;
+  slot_ = -1;   // something may still be written there
+  if (e != hipSuccess) return fail(SUB1_ERR_HIP, "%s: %s", who, hipGetErrorString(e));
+  return fail(SUB1_ERR_INTERNAL, "%s: the launch has ended without its answer", who);
+}
 
 }  // namespace sub1
 
@@ -359,17 +434,13 @@ __device__ __forceinline__ void write_four(uint32_t w, uint32_t minmax, int64_t 
     }
 }
 
-template <int kWaves>
-__global__ __launch_bounds__(64 * kWaves) void decode_kernel(
+// (whether the row's codes cover exactly its width: the same in all lanes)
+__device__ __forceinline__ bool decode_row(
     const int32_t *__restrict__ dec, const uint16_t *__restrict__ w_comp,
     const int32_t *__restrict__ row_off, const uint32_t *__restrict__ minmax,
-    uint8_t *__restrict__ out_tern, uint16_t *__restrict__ out_w, int32_t *__restrict__ bad_rows,
-    int height, int width, int phase) {
-  __shared__ uint32_t run_lds[kWaves][kDecodeRun / 4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = blockIdx.x * kWaves + wave;
-  if (row >= height) return;
-  uint32_t *words = run_lds[wave];
+    uint8_t *__restrict__ out_tern, uint16_t *__restrict__ out_w, int width, int phase, int row,
+    uint32_t *words) {
+  const int lane = threadIdx.x & 63;
   uint8_t *bytes = reinterpret_cast<uint8_t *>(words);
   const int off = __builtin_amdgcn_readfirstlane(row_off[row]);
   const int len = __builtin_amdgcn_readfirstlane(row_off[row + 1]) - off;
@@ -415,7 +486,38 @@ __global__ __launch_bounds__(64 * kWaves) void decode_kernel(
   const int shift = static_cast<int>(at & 3);
   for (int64_t first = at - shift + 4 * lane; first < row_last; first += 256)
     write_four(0u, mm, first, at, row_last, out_tern, out_w);
-  if (bad_rows && lane == 0 && at - row_first != ((width + 1) & ~1)) atomicAdd(bad_rows, 1);
+  return at - row_first == ((width + 1) & ~1);
+}
+
+// With an answer asked for, every workgroup adds itself and its bad rows to the answer's
+// counter at once, and the last of them tells the host.
+template <int kWaves>
+__global__ __launch_bounds__(64 * kWaves) void decode_kernel(
+    const int32_t *__restrict__ dec, const uint16_t *__restrict__ w_comp,
+    const int32_t *__restrict__ row_off, const uint32_t *__restrict__ minmax,
+    uint8_t *__restrict__ out_tern, uint16_t *__restrict__ out_w, int32_t *__restrict__ bad_rows,
+    int height, int width, int phase, sub1::Answer answer) {
+  __shared__ uint32_t run_lds[kWaves][kDecodeRun / 4];
+  __shared__ int wave_bad[kWaves];
+  const int wave = threadIdx.x >> 6;
+  const int row = blockIdx.x * kWaves + wave;
+  const bool fine = row >= height || decode_row(dec, w_comp, row_off, minmax, out_tern, out_w, width, phase, row,
+                                                run_lds[wave]);
+  if (bad_rows && !fine && (threadIdx.x & 63) == 0) atomicAdd(bad_rows, 1);
+  if (!answer.words) return;
+  if ((threadIdx.x & 63) == 0) wave_bad[wave] = fine ? 0 : 1;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long bad = 0;
+    for (int w = 0; w < kWaves; w++) bad += wave_bad[w];
+    const unsigned long long sum =
+        __hip_atomic_fetch_add(answer.counter, bad << 32 | 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) +
+        (bad << 32 | 1u);
+    if (static_cast<uint32_t>(sum) == gridDim.x) {
+      __hip_atomic_store(answer.counter, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      sub1::tell(answer, 0, static_cast<int32_t>(sum >> 32));
+    }
+  }
 }
 
 // ------------------------------------------------------ grouped experts ----
@@ -869,37 +971,59 @@ extern "C" int sub1_matvec(const int32_t *dec, const int16_t *w_comp,
                             width, height, stream);
 }
 
-extern "C" int sub1_decode(const int32_t *dec, const int16_t *w_comp,
-                           const int32_t *row_off, const void *ter_minmax,
-                           uint8_t *out_tern, void *out_w, int32_t *bad_rows, int height,
-                           int width, void *stream) {
-  if (!dec || !w_comp || !row_off) return fail(SUB1_ERR_NULL, "sub1_decode: NULL argument");
-  if (out_w && !ter_minmax) return fail(SUB1_ERR_NULL, "sub1_decode: out_w needs ter_minmax");
+namespace {
+
+int launch_decode(const int32_t *dec, const int16_t *w_comp, const int32_t *row_off, const void *ter_minmax,
+                  uint8_t *out_tern, void *out_w, int32_t *bad_rows, int32_t *counted, int height, int width,
+                  hipStream_t s, const char *who) {
+  if (!dec || !w_comp || !row_off) return fail(SUB1_ERR_NULL, "%s: NULL argument", who);
+  if (out_w && !ter_minmax) return fail(SUB1_ERR_NULL, "%s: out_w needs ter_minmax", who);
   if (height < 1 || width < 1)
-    return fail(SUB1_ERR_SHAPE, "sub1_decode: height %d width %d", height, width);
+    return fail(SUB1_ERR_SHAPE, "%s: height %d width %d", who, height, width);
   if (misaligned(dec, 4) || misaligned(row_off, 4) || misaligned(w_comp, 2) ||
       misaligned(ter_minmax, 4) || misaligned(out_w, 2) || misaligned(bad_rows, 4))
-    return fail(SUB1_ERR_ALIGN, "sub1_decode: misaligned pointer");
-  hipStream_t s = static_cast<hipStream_t>(stream);
+    return fail(SUB1_ERR_ALIGN, "%s: misaligned pointer", who);
+  sub1::AnswerSlot slot;
+  if (counted) {
+    const int rc = slot.take(s, who);
+    if (rc) return rc;
+  }
   // Whole words go out where both outputs begin theirs at the same elements; else
   // (an output that begins within a word) the symbols and the weights each in a launch
   constexpr int kWaves = 4;
-  auto launch = [&](uint8_t *tern, uint16_t *w, int32_t *bad, int phase) {
+  auto launch = [&](uint8_t *tern, uint16_t *w, int32_t *bad, int phase, const sub1::Answer &answer) {
     decode_kernel<kWaves><<<(height + kWaves - 1) / kWaves, 64 * kWaves, 0, s>>>(
         dec, reinterpret_cast<const uint16_t *>(w_comp), row_off,
-        static_cast<const uint32_t *>(ter_minmax), tern, w, bad, height, width, phase);
+        static_cast<const uint32_t *>(ter_minmax), tern, w, bad, height, width, phase, answer);
   };
   uint16_t *w = static_cast<uint16_t *>(out_w);
   const int tern_phase = static_cast<int>(reinterpret_cast<uintptr_t>(out_tern) & 3);
   const int w_phase = static_cast<int>((reinterpret_cast<uintptr_t>(out_w) & 7) / 2);
   if (out_tern && w && tern_phase != w_phase) {
-    launch(out_tern, nullptr, bad_rows, tern_phase);
-    launch(nullptr, w, nullptr, w_phase);
+    launch(out_tern, nullptr, bad_rows, tern_phase, slot.answer());
+    launch(nullptr, w, nullptr, w_phase, sub1::Answer{});
   } else {
-    launch(out_tern, w, bad_rows, out_tern ? tern_phase : w_phase);
+    launch(out_tern, w, bad_rows, out_tern ? tern_phase : w_phase, slot.answer());
   }
   HIP_TRY(hipGetLastError());
-  return SUB1_OK;
+  return counted ? slot.wait(s, 1, counted, who) : SUB1_OK;
+}
+
+}  // namespace
+
+extern "C" int sub1_decode(const int32_t *dec, const int16_t *w_comp, const int32_t *row_off,
+                           const void *ter_minmax, uint8_t *out_tern, void *out_w, int32_t *bad_rows,
+                           int height, int width, void *stream) {
+  return launch_decode(dec, w_comp, row_off, ter_minmax, out_tern, out_w, bad_rows, nullptr, height, width,
+                       static_cast<hipStream_t>(stream), "sub1_decode");
+}
+
+extern "C" int sub1_decode_counted(const int32_t *dec, const int16_t *w_comp, const int32_t *row_off,
+                                   const void *ter_minmax, uint8_t *out_tern, void *out_w, int32_t *bad_rows,
+                                   int height, int width, void *stream) {
+  if (!bad_rows) return fail(SUB1_ERR_NULL, "sub1_decode_counted: NULL argument");
+  return launch_decode(dec, w_comp, row_off, ter_minmax, out_tern, out_w, nullptr, bad_rows, height, width,
+                       static_cast<hipStream_t>(stream), "sub1_decode_counted");
 }
 
 extern "C" int64_t sub1_moe_workspace_bytes(int tokens, int d_ff) {

@@ -488,8 +488,12 @@ __global__ void zero_word_kernel(int32_t *p) { *p = 0; }
 
 // ------------------------------------------------ offsets and compaction ----
 
-__global__ __launch_bounds__(sub1::kScanThreads) void row_offset_scan_kernel(int32_t *cnt, int height) {
+__global__ __launch_bounds__(sub1::kScanThreads) void row_offset_scan_kernel(int32_t *cnt, int height,
+                                                                            sub1::Answer answer) {
   sub1::scan_in_place(cnt, height);
+  if (!answer.words) return;
+  __syncthreads();
+  if (threadIdx.x == 0) sub1::tell(answer, 0, cnt[height]);
 }
 
 // A wavefront per row, lanes stride over the row's codes.
@@ -548,7 +552,7 @@ extern "C" int sub1_pack_count(const int32_t *trie, int32_t *w_tern, int32_t *ro
   rc = launch_pack_rows<false>(a, s);
   if (rc) return rc;
   pack_count_kernel<<<(height + 63) / 64, 64, 0, s>>>(trie, w_tern, row_off, height, width);
-  row_offset_scan_kernel<<<1, sub1::kScanThreads, 0, s>>>(row_off, height);
+  row_offset_scan_kernel<<<1, sub1::kScanThreads, 0, s>>>(row_off, height, sub1::Answer{});
   HIP_TRY(hipGetLastError());
   return SUB1_OK;
 }
@@ -567,15 +571,20 @@ extern "C" int sub1_pack_emit(const int32_t *w_tern, const int32_t *row_off,
   return SUB1_OK;
 }
 
-extern "C" int sub1_pack_weights_count(const void *w, uint16_t *codes, void *ter_minmax,
-                                       int32_t *row_off, int height, int width, void *stream) {
-  const char *who = "sub1_pack_weights_count";
+namespace {
+
+int pack_weights(const void *w, uint16_t *codes, void *ter_minmax, int32_t *row_off, int32_t *total, int height,
+                 int width, hipStream_t s, const char *who) {
   if (!w || !codes || !ter_minmax || !row_off) return fail(SUB1_ERR_NULL, "%s: NULL argument", who);
   int rc = check_pack_shape(who, height, width);
   if (rc) return rc;
   if (misaligned(w, 2) || misaligned(codes, 2) || misaligned(ter_minmax, 4) || misaligned(row_off, 4))
     return fail(SUB1_ERR_ALIGN, "%s: misaligned pointer", who);
-  hipStream_t s = static_cast<hipStream_t>(stream);
+  sub1::AnswerSlot slot;
+  if (total) {
+    rc = slot.take(s, who);
+    if (rc) return rc;
+  }
   PackArgs a{};
   rc = tables_of_current_device(&a.tables, s);
   if (rc) return rc;
@@ -587,9 +596,24 @@ extern "C" int sub1_pack_weights_count(const void *w, uint16_t *codes, void *ter
   a.width = width;
   rc = launch_pack_rows<true>(a, s);
   if (rc) return rc;
-  row_offset_scan_kernel<<<1, sub1::kScanThreads, 0, s>>>(row_off, height);
+  row_offset_scan_kernel<<<1, sub1::kScanThreads, 0, s>>>(row_off, height, slot.answer());
   HIP_TRY(hipGetLastError());
-  return SUB1_OK;
+  return total ? slot.wait(s, 1, total, who) : SUB1_OK;
+}
+
+}  // namespace
+
+extern "C" int sub1_pack_weights_count(const void *w, uint16_t *codes, void *ter_minmax,
+                                       int32_t *row_off, int height, int width, void *stream) {
+  return pack_weights(w, codes, ter_minmax, row_off, nullptr, height, width, static_cast<hipStream_t>(stream),
+                      "sub1_pack_weights_count");
+}
+
+extern "C" int sub1_pack_weights_total(const void *w, uint16_t *codes, void *ter_minmax, int32_t *row_off,
+                                       int32_t *total, int height, int width, void *stream) {
+  const char *who = "sub1_pack_weights_total";
+  if (!total) return fail(SUB1_ERR_NULL, "%s: NULL argument", who);
+  return pack_weights(w, codes, ter_minmax, row_off, total, height, width, static_cast<hipStream_t>(stream), who);
 }
 
 extern "C" int sub1_pack_weights_emit(const uint16_t *codes, const int32_t *row_off, int16_t *w_comp,

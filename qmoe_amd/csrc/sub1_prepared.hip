@@ -88,7 +88,7 @@ struct MetaLayout {
   int64_t counts;       // i32 [all slices + 1] chunk counts, scanned in place
   int64_t status;       // i32 [4]: [0] rows whose codes do not cover the width, [1], [2]
                         // longest slice of kind 0 / 1 in chunks, [3] what check_on_device
-                        // found, then all slices' chunks
+                        // found
   int64_t bytes;
 };
 
@@ -313,6 +313,8 @@ struct WalkArgs {
   int kinds, count;
   const uint32_t *table;         // the emitting pass's words, all of them
   const uint32_t *count_table;   // what the counting pass holds in LDS
+  const int32_t *found;          // what check_source_kernel has found: nothing is followed unless zero
+  sub1::Answer answer;           // emitting: the first word says what that is
   int32_t *status;
   uint2 *stream;
   uint16_t *ckpt;
@@ -495,6 +497,9 @@ template <bool kEmit>
 __global__ __launch_bounds__(kWalkThreads) void walk_rows_kernel(WalkArgs a) {
   extern __shared__ __align__(16) uint32_t held[];
   __shared__ int s_turn;
+  const int found = *a.found;
+  if (kEmit && blockIdx.x == 0 && threadIdx.x == 0) sub1::tell(a.answer, 0, found);
+  if (found) return;
   if (threadIdx.x == 0) s_turn = 0;
   hold_table(kEmit ? a.table : a.count_table, held, kEmit ? kHeldWords : kCountWords);
   const int64_t all = a.k[0].tasks + (a.kinds == 2 ? a.k[1].tasks : 0);
@@ -545,10 +550,12 @@ struct OrderKind {
 };
 struct OrderArgs {
   OrderKind k[2];
+  const int32_t *found;
   int32_t *status;
 };
 
 __global__ __launch_bounds__(kOrderThreads) void order_rows_kernel(OrderArgs a) {
+  if (*a.found) return;
   const int kind = blockIdx.y;
   const OrderKind &k = a.k[kind];
   const KindSource &ks = k.source;
@@ -688,11 +695,14 @@ __global__ __launch_bounds__(256) void check_source_kernel(const int32_t *__rest
   if (bad) atomicOr(found, bad);
 }
 
-// ... and the total once more beside the status words, where one copy fetches all.
-__global__ __launch_bounds__(sub1::kScanThreads) void scan_counts_kernel(int32_t *v, int n, int32_t *total) {
-  sub1::scan_in_place(v, n);
+// ... and what the host waits for: the total, then the four status words.
+__global__ __launch_bounds__(sub1::kScanThreads) void scan_counts_kernel(int32_t *v, int n, const int32_t *status,
+                                                                        sub1::Answer answer) {
+  const bool found = status[3] != 0;
+  if (!found) sub1::scan_in_place(v, n);
   __syncthreads();
-  if (threadIdx.x == 0) *total = v[n];
+  if (threadIdx.x == 0) sub1::tell(answer, 0, found ? 0 : v[n]);
+  if (threadIdx.x < 4) sub1::tell(answer, 1 + threadIdx.x, status[threadIdx.x]);
 }
 
 // The symbols of one prepared matrix back out of the stream: out[row, column]
@@ -2519,17 +2529,16 @@ int name_bad_pointer(const void *const *table, int count, size_t align, const ch
   return SUB1_OK;
 }
 
-// dec and the pointer tables, looked at on the GPU; `word` is a device word to
-// leave the answer in; the walk's tables receive the dictionary as it reads it.
-// Synchronises the stream.
-int check_on_device(const Source &src, int32_t *word, WalkArgs &w, hipStream_t s,
-                    const char *who) {
+// dec and the pointer tables, looked at on the GPU, which leaves what it finds in `found`
+// (a device word, zero before): the launches that follow go by it.  The walk's tables
+// receive the dictionary as it reads it.
+int check_on_device(const Source &src, int32_t *found, WalkArgs &w, hipStream_t s) {
   FixedTables fixed;
   int rc = fixed_tables_of_current_device(&fixed);
   if (rc) return rc;
   w.table = fixed.words;
   w.count_table = fixed.counts;
-  const char *const names[3] = {"w_comp", "row_off", "ter_minmax"};
+  w.found = found;
   PointerTables pt{};
   pt.count = src.count;
   for (int i = 0; i < src.kinds; i++) {
@@ -2543,21 +2552,28 @@ int check_on_device(const Source &src, int32_t *word, WalkArgs &w, hipStream_t s
       pt.align[pt.n++] = j == 0 ? 2 : 4;
     }
   }
-  zero_words_kernel<<<1, 64, 0, s>>>(word, 1);
-  check_source_kernel<<<kCheckBlocks, 256, 0, s>>>(src.dec, fixed.dec, pt, word);
+  check_source_kernel<<<kCheckBlocks, 256, 0, s>>>(src.dec, fixed.dec, pt, found);
   HIP_TRY(hipGetLastError());
-  int32_t found = 0;
-  HIP_TRY(hipMemcpyAsync(&found, word, sizeof found, hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
-  if (found & 2)
-    for (int t = 0; t < pt.n; t++) {
-      rc = name_bad_pointer(pt.table[t], pt.count, pt.align[t], names[t % 3], who, s);
-      if (rc) return rc;
-    }
-  if (found & 1)
-    return fail(SUB1_ERR_SHAPE,
-                "sub1_moe_prepare: dec is not the fixed dictionary; use sub1_moe_grouped");
   return SUB1_OK;
+}
+
+// The error for what it has found.
+int refuse_source(const Source &src, int found, hipStream_t s, const char *who) {
+  const char *const names[3] = {"w_comp", "row_off", "ter_minmax"};
+  if (found & 2)
+    for (int i = 0; i < src.kinds; i++) {
+      const KindSource &k = src.k[i];
+      if (!k.w_comp_of) continue;
+      const void *const *of[3] = {reinterpret_cast<const void *const *>(k.w_comp_of),
+                                  reinterpret_cast<const void *const *>(k.row_off_of),
+                                  reinterpret_cast<const void *const *>(k.minmax_of)};
+      for (int j = 0; j < 3; j++) {
+        const int rc = name_bad_pointer(of[j], src.count, j == 0 ? 2 : 4, names[j], who, s);
+        if (rc) return rc;
+      }
+    }
+  return fail(SUB1_ERR_SHAPE,
+              "sub1_moe_prepare: dec is not the fixed dictionary; use sub1_moe_grouped");
 }
 
 int check_source(const Source &src, const char *who) {
@@ -2702,11 +2718,14 @@ int prepare_layout(const Source &src, void *meta, int64_t meta_bytes, LayoutResu
     return fail(SUB1_ERR_SHAPE, "%s: meta needs %lld bytes", who, static_cast<long long>(m.bytes));
   char *base = static_cast<char *>(meta);
   int32_t *status = reinterpret_cast<int32_t *>(base + m.status);
+  sub1::AnswerSlot slot;
+  int rc = slot.take(s, who);
+  if (rc) return rc;
+  zero_words_kernel<<<1, 64, 0, s>>>(status, 4);
   WalkArgs w{};
-  int rc = check_on_device(src, status + 3, w, s, who);
+  rc = check_on_device(src, status + 3, w, s);
   if (rc) return rc;
   int32_t *counts = reinterpret_cast<int32_t *>(base + m.counts);
-  zero_words_kernel<<<1, 64, 0, s>>>(status, 3);
   w.status = status;
   for (int i = 0; i < src.kinds; i++) {
     const KindMeta &k = m.k[i];
@@ -2722,6 +2741,7 @@ int prepare_layout(const Source &src, void *meta, int64_t meta_bytes, LayoutResu
   int64_t slice0 = 0;
   OrderArgs o{};
   o.status = status;
+  o.found = status + 3;
   size_t lds = 0;
   for (int i = 0; i < src.kinds; i++) {
     const KindMeta &k = m.k[i];
@@ -2738,22 +2758,23 @@ int prepare_layout(const Source &src, void *meta, int64_t meta_bytes, LayoutResu
   }
   order_rows_kernel<<<dim3(static_cast<unsigned>(src.count), static_cast<unsigned>(src.kinds)), kOrderThreads,
                       lds, s>>>(o);
-  scan_counts_kernel<<<1, sub1::kScanThreads, 0, s>>>(counts, static_cast<int>(slice0), status + 3);
+  scan_counts_kernel<<<1, sub1::kScanThreads, 0, s>>>(counts, static_cast<int>(slice0), status, slot.answer());
   HIP_TRY(hipGetLastError());
-  int32_t host[4] = {0, 0, 0, 0};
-  HIP_TRY(hipMemcpyAsync(host, status, sizeof host, hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
-  const int32_t total = host[3];
-  if (host[0])
-    return fail(SUB1_ERR_SHAPE, "%s: the codes of %d rows do not cover the width", who, host[0]);
+  int32_t host[5] = {0, 0, 0, 0, 0};   // the total, bad rows, the longest slices, what was found
+  rc = slot.wait(s, 5, host, who);
+  if (rc) return rc;
+  if (host[4]) return refuse_source(src, host[4], s, who);
+  const int32_t total = host[0];
+  if (host[1])
+    return fail(SUB1_ERR_SHAPE, "%s: the codes of %d rows do not cover the width", who, host[1]);
   if (total < 0) return fail(SUB1_ERR_SHAPE, "%s: stream too large", who);
   out->meta_bytes = m.bytes;
   out->total_chunks = total;
   // the entry stream, then one 128-byte checkpoint entry per group of chunks
   out->code_bytes = static_cast<int64_t>(total) * 512 +
                     (static_cast<int64_t>(total) / kGroupChunks + slice0 + 1) * 128;
-  out->max_chunks[0] = host[1];
-  out->max_chunks[1] = host[2];
+  out->max_chunks[0] = host[2];
+  out->max_chunks[1] = host[3];
   return SUB1_OK;
 }
 
@@ -2768,8 +2789,13 @@ int prepare_codes(const Source &src, const Prepared &p, hipStream_t s, const cha
   if (p.total_chunks < 0 || p.meta_bytes < m.bytes ||
       p.code_bytes < p.total_chunks * 512 + (p.total_chunks / kGroupChunks + nslices + 1) * 128)
     return fail(SUB1_ERR_SHAPE, "%s: buffers smaller than the layout needs", who);
+  sub1::AnswerSlot slot;
+  int rc = slot.take(s, who);
+  if (rc) return rc;
+  int32_t *found = reinterpret_cast<int32_t *>(base + m.status) + 3;
+  zero_words_kernel<<<1, 64, 0, s>>>(found, 1);
   WalkArgs w{};
-  const int rc = check_on_device(src, reinterpret_cast<int32_t *>(base + m.status) + 3, w, s, who);
+  rc = check_on_device(src, found, w, s);
   if (rc) return rc;
   uint2 *stream = static_cast<uint2 *>(const_cast<void *>(p.codes));
   uint16_t *ckpt = reinterpret_cast<uint16_t *>(stream + p.total_chunks * 64);
@@ -2786,7 +2812,13 @@ int prepare_codes(const Source &src, const Prepared &p, hipStream_t s, const cha
     wk.tasks = static_cast<int64_t>(src.count) * k.slices;
     first_slice += wk.tasks;
   }
-  return launch_walk<true>(src, m, w, s);
+  w.answer = slot.answer();
+  rc = launch_walk<true>(src, m, w, s);
+  if (rc) return rc;
+  // the walk says what was found as it begins, and does its work behind the host's back
+  int32_t bad = 0;
+  rc = slot.wait(s, 1, &bad, who);
+  return rc ? rc : bad ? refuse_source(src, bad, s, who) : SUB1_OK;
 }
 
 // Cut of the matrices for a batch that cannot occupy the GPU with a wavefront

@@ -195,10 +195,10 @@ def sub1pack_weights(w):
     minmax = torch.empty(2 * height, dtype=torch.bfloat16, device=dev)
     codes = torch.empty((height, (width + 1) // 2), dtype=torch.int16, device=dev)
     with _on_device(dev):
-        _lib.check(lib.sub1_pack_weights_count(p_w, codes.data_ptr(), minmax.data_ptr(),
-                                               row_off.data_ptr(), height, width, _stream()))
-        total = int(row_off[height].item())      # the one host sync, as in the reference
-        w_comp = torch.empty(total, dtype=torch.int16, device=dev)
+        total = ctypes.c_int32()      # the one wait for the GPU, as in the reference
+        _lib.check(lib.sub1_pack_weights_total(p_w, codes.data_ptr(), minmax.data_ptr(), row_off.data_ptr(),
+                                               ctypes.byref(total), height, width, _stream()))
+        w_comp = torch.empty(total.value, dtype=torch.int16, device=dev)
         _lib.check(lib.sub1_pack_weights_emit(codes.data_ptr(), row_off.data_ptr(), w_comp.data_ptr(),
                                               height, width, _stream()))
     return w_comp, row_off, minmax
@@ -216,12 +216,12 @@ def sub1decode(dec, w_comp, row_off, ter_minmax, width, want_tern=True, want_w=T
         if ter_minmax is not None else None
     tern = torch.empty((height, width), dtype=torch.uint8, device=dev) if want_tern else None
     w = torch.empty((height, width), dtype=torch.bfloat16, device=dev) if want_w else None
-    bad = torch.zeros(1, dtype=torch.int32, device=dev)
+    bad = ctypes.c_int32()
     with _on_device(dev):
-        _lib.check(_lib.load().sub1_decode(
+        _lib.check(_lib.load().sub1_decode_counted(
             p_dec, p_wc, p_ro, p_mm, tern.data_ptr() if want_tern else None,
-            w.data_ptr() if want_w else None, bad.data_ptr(), height, width, _stream()))
-    return tern, w, int(bad.item())
+            w.data_ptr() if want_w else None, ctypes.byref(bad), height, width, _stream()))
+    return tern, w, bad.value
 
 
 def _workspace(stack, tokens):

@@ -228,6 +228,48 @@ def test_expanding_codes_that_do_not_fit_the_width(gpu):
     assert 0 < kept < 4000 and torch.equal(tern[0, :kept], whole[0, :kept]) and not tern[0, kept:].any()
 
 
+def test_calls_that_wait_for_the_gpu_come_from_any_thread_and_stream(gpu):
+    """More calls at once than the library has places to answer in, each with a count of its
+    own; and a stream that is being captured is refused without spoiling the capture."""
+    import threading
+    sub1, op = gpu
+    symbols = symbols_of(40, 300, [0.3], seed=2)
+    w_comp, row_off = packed(gpu, symbols)
+    minmax = torch.tensor([-1.0, 1.0] * 40, device='cuda').bfloat16()
+    weights = torch.tensor([0.0, -1.0, 1.0], device='cuda')[symbols.long()].bfloat16()
+    weights[:, 0], weights[:, 1] = -1.0, 1.0
+    whole = op.sub1pack_weights(weights)
+    torch.cuda.synchronize()
+    wrong = []
+
+    def calls(n):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for i in range(6):
+                rows = 1 + (n + 5 * i) % 39
+                moved = row_off[:rows + 1].clone()
+                moved[rows] -= n % 2                    # the last row lacks a code, or not
+                bad = op.sub1decode(sub1.DEC[0], w_comp, moved, minmax[:2 * rows], 300)[2]
+                packs = op.sub1pack_weights(weights[:rows].contiguous())
+                if bad != n % 2 or not torch.equal(packs[0], whole[0][:int(whole[1][rows])]):
+                    wrong.append((n, i, bad))
+
+    threads = [threading.Thread(target=calls, args=(n,)) for n in range(80)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+    graph, y = torch.cuda.CUDAGraph(), torch.zeros(8, device='cuda')
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        with pytest.raises(op._lib.Sub1Error, match='captured'):
+            op.sub1decode(sub1.DEC[0], w_comp, row_off, minmax, 300)
+        y += 1
+    graph.replay()
+    graph.replay()
+    assert y.tolist() == [2.0] * 8
+
+
 FIRST_PACK_IN_A_CAPTURE = r'''
 import ctypes, sys
 sys.path.insert(0, sys.argv[1])
