@@ -101,7 +101,7 @@ std::condition_variable g_answer_free;
 std::vector<int> g_answer_slots;   // the free ones
 unsigned long long *g_answer_host = nullptr, *g_answer_device = nullptr;   // 4 KB, held until the process ends
 std::atomic<uint32_t> g_answer_ticket{0};
-static __device__ unsigned long long answer_counters[kAnswerSlots];
+static __device__ unsigned long long answer_counters[kAnswerSlots * kAnswerCounterWords];
 }  // namespace
 
 int AnswerSlot::take(hipStream_t stream, const char *who) {
@@ -126,7 +126,7 @@ int AnswerSlot::take(hipStream_t stream, const char *who) {
   slot_ = g_answer_slots.back();
   g_answer_slots.pop_back();
   answer_.words = g_answer_device + slot_ * kAnswerWords;
-  answer_.counter = static_cast<unsigned long long *>(counters) + slot_;
+  answer_.counters = static_cast<unsigned long long *>(counters) + slot_ * kAnswerCounterWords;
   do answer_.ticket = ++g_answer_ticket;
   while (answer_.ticket == 0);   // what the words hold at first
   return SUB1_OK;
@@ -489,8 +489,7 @@ __device__ __forceinline__ bool decode_row(
   return at - row_first == ((width + 1) & ~1);
 }
 
-// With an answer asked for, every workgroup adds itself and its bad rows to the answer's
-// counter at once, and the last of them tells the host.
+// With an answer asked for, the host is told the number of bad rows by the last workgroup.
 template <int kWaves>
 __global__ __launch_bounds__(64 * kWaves) void decode_kernel(
     const int32_t *__restrict__ dec, const uint16_t *__restrict__ w_comp,
@@ -508,15 +507,9 @@ __global__ __launch_bounds__(64 * kWaves) void decode_kernel(
   if ((threadIdx.x & 63) == 0) wave_bad[wave] = fine ? 0 : 1;
   __syncthreads();
   if (threadIdx.x == 0) {
-    unsigned long long bad = 0;
+    int bad = 0;
     for (int w = 0; w < kWaves; w++) bad += wave_bad[w];
-    const unsigned long long sum =
-        __hip_atomic_fetch_add(answer.counter, bad << 32 | 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) +
-        (bad << 32 | 1u);
-    if (static_cast<uint32_t>(sum) == gridDim.x) {
-      __hip_atomic_store(answer.counter, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      sub1::tell(answer, 0, static_cast<int32_t>(sum >> 32));
-    }
+    sub1::tell_sum(answer, 0, bad);
   }
 }
 
