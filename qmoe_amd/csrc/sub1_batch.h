@@ -8,29 +8,34 @@
 // whole row fits whatever its length, and no form of the weights beside the stream
 // is kept in memory.  Word g of row r lies at (64 g + r) * 4: a lane expands one
 // row, so its writes never meet another lane's in a bank, wherever they go.  An
-// entry costs nine plain instructions and an LDS `or` (walking: 3.5 and a random
-// gather), then nothing per token.
+// entry costs nine plain instructions and an LDS `or` (walking: 3.5 and a random gather), then
+// nothing per token.
+//
+// wo takes its columns in the order in which wi's slices have their rows (seven
+// instructions an entry and a look into a table that says where a column's code goes): wi's
+// product, which has the weights as its first operand, then holds h just as wo's product
+// wants it, eight columns of a token to a lane, and stores it so.  (With wo's columns in
+// their own order h went out as rows of 32 tokens and through a pass that transposed
+// it, 13 us of 133 below; y through another, 6, where its two-byte stores now go straight to
+// the tokens' rows.)
 //
 // One launch: group_blocks_kernel gives every token a slot in a block of 32 of its
 // expert's tokens; pack_tokens_kernel lays a block's activations out as MFMA
-// operands; batch_product_kernel multiplies (wi, ReLU); pack_hidden_kernel lays h
-// out; batch_product_kernel (wo); unpack_tokens_kernel writes y.  The products leave
-// their rows as 64-byte runs of 32 tokens (rows come in the slices' order, so anything
-// finer would be scattered), which the passes around them transpose.
+// operands; batch_product_kernel<true> multiplies (wi, ReLU), batch_product_kernel<false>
+// (wo); walk_spoiled_kernel walks what they leave.
 //
-// 128 base experts on 4096 tokens: 274 -> 132 us (group 7, pack 7, wi 45, h 13, wo 52, y 6,
-// the listed tokens' launch 4), 40 c-2048 experts on 700 tokens 366 -> 167.  With the
-// multiplying taken out the same launch takes 82, with the expanding 120: what bounds
-// the products is the 24 instructions that make a step's two operands of weights, beside
-// two MFMAs for every block of tokens (15 plain instructions an MFMA with up to 32 tokens, 8 with
-// 64), then the start and end of workgroups that LDS holds to 12 to 16 wavefronts a compute unit.
-// No unit is full (counters: VALUs 47 % busy, matrix cores 21, LDS 10): on average a launch has
-// 1.9 wavefronts on a SIMD, each a chain of expanding, making operands and multiplying.
+// 128 base experts on 4096 tokens: walking 274 us, here 115 (133 with a pass for h and one for y);
+// 40 c-2048 experts on 640 tokens 311 and 159 (167).  Under a profiler, one after the other:
+// group 8, x 6, wi 48, wo 61, marks 4.5.  Of the products' times multiplying is 27 each (with it taken
+// out they take that less): the 24 instructions that make a step's two operands of weights, beside
+// two MFMAs for every block of tokens, issued at 80 % of what the SIMDs can; expanding 8 and 12;
+// starting, clearing LDS and adding up what the wavefronts of a slice have, in workgroups
+// that leave no LDS for another one meanwhile, the rest.
 //
 // A token whose activations or h hold an infinity or NaN is left to the walking
 // kernel (0 x inf is NaN here, and a weight of zero adds nothing there), and so are the
 // tokens of an expert with such a (min, max) (walking, every weight of its row meets it): the
-// passes and the products mark them, and unpack_tokens_kernel lists them for the launch that follows.
+// pass over x and wi's product mark them, and walk_spoiled_kernel finds the marks.
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -38,59 +43,115 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kBlockTokens = 32;     // tokens of an MFMA operand
 constexpr int kChunkBlocks = 2;      // blocks that share an expansion
-constexpr int kTurn = 2;             // steps whose operands are asked for together
+constexpr int kTurn = 4;             // steps whose operands are asked for together, and ahead
 constexpr int kStepColumns = 16;     // columns of an MFMA, and of a word of codes
 constexpr int kBatchPiece = 8192;    // tokens of a launch sequence: bounds the scratch memory
 constexpr int kBatchMaxExperts = 4096;   // group_blocks_kernel's tables in LDS
 
 __host__ __device__ constexpr int steps_of(int width) { return (width + kStepColumns - 1) / kStepColumns; }
-// A slice's codes in LDS; one row of words more, which stays zero: steps onto the last
-// zero column name it, and a turn of steps may end with it.
-__host__ __device__ constexpr int slice_code_bytes(int width) { return (steps_of(width) + 1) * 256; }
+// Steps of a product over the rows of 64-row slices.
+__host__ __device__ constexpr int steps_of_slices(int slices) { return slices * (64 / kStepColumns); }
+// A slice's codes in LDS: whole turns of steps (zeros where the last is half a one), and a
+// row of words that entries go to which stay on a zero column.
+__host__ __device__ constexpr int idle_step(int steps) { return (steps + kTurn - 1) / kTurn * kTurn; }
+__host__ __device__ constexpr int slice_code_bytes(int steps) { return (idle_step(steps) + 1) * 256; }
+__host__ __device__ constexpr int table_bytes(int width) { return (physical_columns(width) * 2 + 15) / 16 * 16; }
 
 // Totals a launch's kernels read.
 enum BatchTotals { kTotalChunks = 0, kTotalLive = 1, kTotalBlocks = 2, kTotalWords = 4 };
 
-// Column of a step that slot k of an operand holds for a lane of half h.  Position p of
-// the stream falls on bit p % 34 of word p / 34 (mod 32, bits 32 and 33 being column 15,
-// 0 and 1 the zero column, which is not written): field j of a word, bits 2j and 2j + 1,
-// is column j - 1 mod 16.  Byte b of a word holds fields 4b .. 4b + 3, and a lane of
-// half h takes fields 2h (slots 0-3, byte by byte) and 2h + 1 (slots 4-7).
-__host__ __device__ constexpr int slot_column(int h, int k) {
-  return (4 * (k & 3) + 2 * h + (k >> 2) + 15) & 15;
+// A word of codes holds a step's 16 columns: field j, bits 2j and 2j + 1, is 1 for a row
+// min, 2 for a max, 0 for neither.  Byte b holds fields 4b .. 4b + 3, and a lane of half h
+// takes fields 2h (places 0-3 of its operand, byte by byte) and 2h + 1 (places 4-7).  An entry of
+// the table: the step in bits 5 and up, twice the field in bits 0-4.
+__host__ __device__ constexpr uint32_t table_entry(int step, int half, int place) {
+  return static_cast<uint32_t>(step << 5 | 2 * (4 * (place & 3) + 2 * half + (place >> 2)));
+}
+// x's columns keep their own order and need no table: position p of the stream falls on bit
+// p % 34 of word p / 34 (mod 32, bits 32 and 33 being column 15, 0 and 1 the zero column, which
+// is not written), so that field j is column j - 1 mod 16.
+__host__ __device__ constexpr int column_of_place(int half, int place) {
+  return (4 * (place & 3) + 2 * half + (place >> 2) + 15) & 15;
+}
+// Row r of a matrix's slices as the product of them leaves it in its lanes: of 32 rows a
+// lane of half h has rows 8 g + 4 h + 0..3 for g = 0..3, which are two operands of eight.
+__host__ __device__ constexpr uint32_t entry_of_row(int r) {
+  return table_entry(r >> 4, (r >> 2) & 1, ((r >> 3) & 1) << 2 | (r & 3));
 }
 
 struct BatchArgs {
   const uint2 *stream;
   const uint16_t *ckpt;
   KindArgs k;
-  const u32x4 *in;        // [block][step][64 lanes]: 16-byte operands
-  uint16_t *out;          // [block][height][32]
-  const int4 *chunks;     // (expert, first block, blocks, 0)
-  int32_t *spoiled;       // [slot]: left to the walking kernel
+  const u32x4 *in;           // [block][step][64 lanes]: 16-byte operands
+  const uint16_t *order;     // wo: wi's rows in the order of its slices, [expert][order_rows]
+  int order_rows;
+  const uint16_t *tables;    // [expert][columns]: where LDS has no room for a table beside a slice
+  u32x4 *h;                  // wi: wo's operands, of h_steps steps
+  int h_steps;
+  const uint32_t *wo_minmax; // wi: [expert][wo_rows], looked over for tokens to be walked
+  int wo_rows;
+  uint16_t *y;               // wo
+  int64_t ldy;
+  const int32_t *slots;      // the token in every slot, or -1
+  const int4 *chunks;        // (expert, first block, blocks, 0)
+  int32_t *spoiled;          // [slot]: left to the walking kernel
   const int32_t *totals;
-  int steps, parts;       // parts: wavefronts that share a slice
-  int per_group;          // slices of a workgroup
-  int slice_groups;       // workgroups of a chunk
-  int relu;
+  int steps, parts;          // parts: wavefronts that share a slice
+  int per_group;             // slices of a workgroup
+  int slice_groups;          // workgroups of a chunk
 };
+
+// An expert's table, shared among `threads` threads.  A thread holds eight rows of wi's
+// order, asked for beforehand (a row at a time, c-2048 wo took 5 us a workgroup for its
+// table); longer orders are gone through in turns.
+__device__ __forceinline__ u32x4 order_piece(const BatchArgs &a, int e, int piece) {
+  const uint16_t *order = a.order + static_cast<int64_t>(e) * a.order_rows;   // whole slices: aligned
+  return 8 * piece < a.order_rows ? *reinterpret_cast<const u32x4 *>(order + 8 * piece)
+                                  : u32x4{~0u, ~0u, ~0u, ~0u};
+}
+__device__ __forceinline__ void fill_table(const BatchArgs &a, int e, uint16_t *table, u32x4 first, int thread,
+                                           int threads) {
+  const uint16_t idle = static_cast<uint16_t>(idle_step(a.steps) << 5);
+  for (int q = thread * kZeroPeriod; q < physical_columns(a.k.width); q += threads * kZeroPeriod) table[q] = idle;
+  const int last = physical_column(a.k.width - 1);
+  for (int q = last + 1 + thread; q < physical_columns(a.k.width); q += threads) table[q] = idle;
+  for (int piece = thread; 8 * piece < a.order_rows; piece += threads) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const int c = (first[i / 2] >> (16 * (i & 1))) & 0xffffu;
+      if (c != 0xffff) table[physical_column(c)] = static_cast<uint16_t>(entry_of_row(8 * piece + i));
+    }
+    if (8 * (piece + threads) < a.order_rows) first = order_piece(a, e, piece + threads);
+  }
+}
 
 // The nine entries of a chunk onto the row's codes.  `at` is the position reached,
 // `lane_codes` the row's word 0.  The stream's entries never leave the row (what pads
 // a row stays on a zero column or repeats its last entry, which or's the same bit).
-__device__ __forceinline__ void expand_chunk(uint2 cw, uint32_t &at, uint32_t *lane_codes) {
+template <bool kByTable>
+__device__ __forceinline__ void expand_chunk(uint2 cw, uint32_t &at, uint32_t *lane_codes, const uint16_t *table) {
   const uint32_t mid = __builtin_amdgcn_alignbit(cw.y, cw.x, 28);
+  uint32_t word[kFields], bit[kFields];
 #pragma unroll
   for (int q = 0; q < kFields; q++) {
     const uint32_t step = q < 4 ? (cw.x >> (kFieldBits * q)) & 127u
                         : q < 8 ? (mid >> (kFieldBits * (q - 4))) & 127u
                                 : (cw.y >> 24) & 127u;
     at += step;
-    const uint32_t g = __umul24(at, 30841u) >> 20;   // at / 34, exact up to 50 000
-    const uint32_t r = at - 34u * g;
-    const uint32_t bit = r < 2u ? 0u : 1u << (r & 31u);
-    __hip_atomic_fetch_or(lane_codes + g * 64u, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (kByTable) {
+      const uint32_t place = table[at >> 1];
+      word[q] = place >> 5;
+      bit[q] = 1u << ((place | (at & 1u)) & 31u);
+    } else {
+      word[q] = __umul24(at, 30841u) >> 20;   // at / 34, exact up to 50 000
+      const uint32_t r = at - 34u * word[q];
+      bit[q] = r < 2u ? 0u : 1u << (r & 31u);
+    }
   }
+#pragma unroll
+  for (int q = 0; q < kFields; q++)
+    __hip_atomic_fetch_or(lane_codes + word[q] * 64u, bit[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // Two rows' weights (a lane's B operands of a step) from their words of codes.
@@ -119,22 +180,36 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *base, in
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, bytes, 0x00020000);
 }
 
+// An exponent of all ones in either half: the sum carries into its sign.
+__device__ __forceinline__ uint32_t high_exponents(uint32_t pair) {
+  return ((pair & 0x7f807f80u) + 0x00800080u) & 0x80008000u;
+}
+__device__ __forceinline__ uint32_t bf16_pair(float lower, float upper) {
+  const bf16x2 pair = {static_cast<__bf16>(lower), static_cast<__bf16>(upper)};
+  return __builtin_bit_cast(uint32_t, pair);
+}
+__device__ __forceinline__ float relu_bits(float v) { return __uint_as_float(max(__float_as_int(v), 0)); }
+
 // What a workgroup does: its slices' codes into LDS, then every wavefront's share of a
 // slice's steps, then the sums of the wavefronts that share a slice, added in order and
 // written.  Everything that is read from memory is asked for before the codes are expanded.
-template <int kBlocks>
+template <bool kHidden, bool kTableInLds, int kBlocks>
 __device__ __forceinline__ void slices_times_tokens(const BatchArgs &a, uint32_t *lds, int e, int group,
                                                     int64_t first_block) {
   const int lane = threadIdx.x & 63, half = lane >> 5;
   const int waves = blockDim.x >> 6;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int local = wave / a.parts, sub = wave % a.parts;
+  const int local = wave / a.parts;
+  // (wavefronts with the same share of a slice on different SIMDs: the last has most to expand)
+  const int sub = (wave + local) % a.parts;
   const int s = group * a.per_group + local;
   const bool mine = s < a.k.slices;
   const int64_t sl = static_cast<int64_t>(e) * a.k.slices + (mine ? s : 0);
-  const int slice_words = (a.steps + 1) * 64;
+  const int slice_words = slice_code_bytes(a.steps) / 4;
   uint32_t *codes = lds + local * slice_words;
+  uint16_t *table_lds = reinterpret_cast<uint16_t *>(lds + a.per_group * slice_words);
 
+  const u32x4 order = !kHidden && kTableInLds ? order_piece(a, e, threadIdx.x) : u32x4{};
   const int len = a.k.slice_len[sl];
   const uint32_t base_word = a.k.slice_base[sl];
   uint32_t minmax[2];
@@ -142,8 +217,12 @@ __device__ __forceinline__ void slices_times_tokens(const BatchArgs &a, uint32_t
 #pragma unroll
   for (int j = 0; j < 2; j++) {
     minmax[j] = a.k.minmax[sl * 64 + 32 * j + (lane & 31)];
-    row[j] = a.k.row_idx[sl * 64 + 32 * j + (lane & 31)];
+    if (!kHidden) row[j] = mine ? a.k.row_idx[sl * 64 + 32 * j + (lane & 31)] : 0xffff;
   }
+  bool taken[kBlocks];   // the lane's slot: h of one without a token is not written, nor used
+#pragma unroll
+  for (int i = 0; i < kBlocks; i++)
+    taken[i] = kHidden && mine && a.slots[(first_block + i) * kBlockTokens + (lane & 31)] >= 0;
   const int nch = chunks_of(__builtin_amdgcn_readfirstlane(len));
   const uint32_t base = __builtin_amdgcn_readfirstlane(base_word);
   const int groups = (nch + kGroupChunks - 1) / kGroupChunks;
@@ -180,11 +259,22 @@ __device__ __forceinline__ void slices_times_tokens(const BatchArgs &a, uint32_t
   const int all_words = a.per_group * slice_words;   // a multiple of 64
   for (int i = 4 * threadIdx.x; i < all_words; i += 4 * blockDim.x)
     *reinterpret_cast<uint4 *>(lds + i) = make_uint4(0u, 0u, 0u, 0u);
-  // (an exponent of all ones in either half: the sum carries into its sign)
-  const uint32_t high = ((minmax[0] & 0x7f807f80u) + 0x00800080u) | ((minmax[1] & 0x7f807f80u) + 0x00800080u);
-  if ((high & 0x80008000u) && mine && sub == 0)
-    for (int t = 0; t < kBlocks * kBlockTokens; t++) a.spoiled[first_block * kBlockTokens + t] = 1;
+  if (!kHidden && kTableInLds) fill_table(a, e, table_lds, order, threadIdx.x, blockDim.x);
+  if (kHidden) {
+    // the tokens that such weights leave to the walking kernel, of wo too (its product
+    // goes by the marks as soon as it has a result)
+    uint32_t high = 0;
+    if (mine && sub == 0) high = high_exponents(minmax[0]) | high_exponents(minmax[1]);
+    if (group == 0)
+      for (int r = threadIdx.x; r < a.wo_rows; r += blockDim.x)
+        high |= high_exponents(a.wo_minmax[static_cast<int64_t>(e) * a.wo_rows + r]);
+    if (high)
+      for (int t = 0; t < kBlocks * kBlockTokens; t++) a.spoiled[first_block * kBlockTokens + t] = 1;
+  }
   __syncthreads();
+  const uint16_t *table = kHidden ? nullptr
+                          : kTableInLds ? table_lds
+                                        : a.tables + static_cast<int64_t>(e) * physical_columns(a.k.width);
 #pragma unroll 1
   for (int c = g_lo * kGroupChunks; c < c_end; c += kGroupChunks) {
     uint2 now[kGroupChunks];
@@ -195,7 +285,7 @@ __device__ __forceinline__ void slices_times_tokens(const BatchArgs &a, uint32_t
       for (int i = 0; i < kGroupChunks; i++) ask_chunk(c + kGroupChunks, i);
 #pragma unroll
     for (int i = 0; i < kGroupChunks; i++)
-      if (c + i < c_end) expand_chunk(now[i], at, codes + lane);
+      if (c + i < c_end) expand_chunk<!kHidden>(now[i], at, codes + lane, table);
   }
   __syncthreads();
 
@@ -228,70 +318,114 @@ __device__ __forceinline__ void slices_times_tokens(const BatchArgs &a, uint32_t
 #pragma unroll
       for (int i = 0; i < kBlocks; i++) {
         const bf16x8 xv = __builtin_bit_cast(bf16x8, x[u][i]);
-        acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xv, w0, acc[i][0], 0, 0, 0);
-        acc[i][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xv, w1, acc[i][1], 0, 0, 0);
+        // the first operand's 32 lie in a lane's values, the second's in the lanes
+        acc[i][0] = kHidden ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(w0, xv, acc[i][0], 0, 0, 0)
+                            : __builtin_amdgcn_mfma_f32_32x32x16_bf16(xv, w0, acc[i][0], 0, 0, 0);
+        acc[i][1] = kHidden ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(w1, xv, acc[i][1], 0, 0, 0)
+                            : __builtin_amdgcn_mfma_f32_32x32x16_bf16(xv, w1, acc[i][1], 0, 0, 0);
       }
     }
   }
 
-  // a lane has row 32 j + lane % 32 and tokens 8 g + 4 half + 0..3, values 4 g + 0..3
-  auto write = [&](const float (&v)[4], int i, int j, int g) {
-    if (!mine || row[j] == 0xffff) return;
-    uint32_t w[2];
+  // Values 4 g + 0..3 of block i and rows 32 j + 0..31.  h: a lane has token lane % 32 and rows
+  // 8 g + 4 half + 0..3; y: row lane % 32 and tokens 8 g + 4 half + 0..3.
+  uint32_t high[kBlocks];
 #pragma unroll
-    for (int m = 0; m < 2; m++) {
-      float lower = v[2 * m], upper = v[2 * m + 1];
-      if (a.relu) {
-        lower = __uint_as_float(max(__float_as_int(lower), 0));
-        upper = __uint_as_float(max(__float_as_int(upper), 0));
-      }
-      const bf16x2 pair = {static_cast<__bf16>(lower), static_cast<__bf16>(upper)};
-      w[m] = __builtin_bit_cast(uint32_t, pair);
+  for (int i = 0; i < kBlocks; i++) high[i] = 0;
+  auto tokens_of = [&](int i, int g) {   // -1: none, or one that is walked
+    if (kHidden) return make_int4(0, 0, 0, 0);
+    const int64_t slot = (first_block + i) * kBlockTokens + 8 * g + 4 * half;
+    int4 t = *reinterpret_cast<const int4 *>(a.slots + slot);
+    const int4 left = *reinterpret_cast<const int4 *>(a.spoiled + slot);
+    if (left.x) t.x = -1;
+    if (left.y) t.y = -1;
+    if (left.z) t.z = -1;
+    if (left.w) t.w = -1;
+    return t;
+  };
+  auto write = [&](const float (&v)[4], const int4 &tokens, int i, int j, int g) {
+    if (kHidden) {
+      const uint2 w = make_uint2(bf16_pair(relu_bits(v[0]), relu_bits(v[1])), bf16_pair(relu_bits(v[2]), relu_bits(v[3])));
+      high[i] |= high_exponents(w.x) | high_exponents(w.y);
+      u32x4 *to = a.h + ((first_block + i) * a.h_steps + s * 4 + 2 * j + (g >> 1)) * 64 + lane;
+      if (taken[i]) reinterpret_cast<uint2 *>(to)[g & 1] = w;
+      return;
     }
-    *reinterpret_cast<uint2 *>(a.out + ((first_block + i) * a.k.height + row[j]) * kBlockTokens + 8 * g + 4 * half) =
-        make_uint2(w[0], w[1]);
+    if (row[j] == 0xffff) return;
+    const int t[4] = {tokens.x, tokens.y, tokens.z, tokens.w};
+#pragma unroll
+    for (int m = 0; m < 4; m++)
+      if (t[m] >= 0) a.y[t[m] * a.ldy + row[j]] = __builtin_bit_cast(uint16_t, static_cast<__bf16>(v[m]));
   };
   if (a.parts == 1) {
+    int4 tokens[kBlocks][4];
+#pragma unroll
+    for (int i = 0; i < kBlocks; i++)
+#pragma unroll
+      for (int g = 0; g < 4; g++) tokens[i][g] = tokens_of(i, g);
 #pragma unroll
     for (int i = 0; i < kBlocks; i++)
 #pragma unroll
       for (int j = 0; j < 2; j++)
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-          const float v[4] = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-          write(v, i, j, g);
+        for (int g = 0; g < 4; g += kHidden ? 2 : 1) {
+          if (kHidden) {   // an operand whole
+            u32x4 w;
+#pragma unroll
+            for (int m = 0; m < 4; m++) {
+              w[m] = bf16_pair(relu_bits(acc[i][j][4 * g + 2 * m]), relu_bits(acc[i][j][4 * g + 2 * m + 1]));
+              high[i] |= high_exponents(w[m]);
+            }
+            if (taken[i]) a.h[((first_block + i) * a.h_steps + s * 4 + 2 * j + (g >> 1)) * 64 + lane] = w;
+          } else {
+            const float v[4] = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+            write(v, tokens[i][g], i, j, g);
+          }
         }
-    return;
-  }
-  float4 *sums = reinterpret_cast<float4 *>(lds);
-  __syncthreads();   // every wavefront is through with the codes, whose place the sums take
+  } else {
+    int4 tokens[kBlocks][2];   // for the one or two groups of four values that are this wavefront's
 #pragma unroll
-  for (int i = 0; i < kBlocks; i++)
+    for (int i = 0; i < kBlocks; i++)
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-      // a tile at a time, in one of two places; the parts share its groups of four values
-      float4 *place = sums + ((2 * i + j) & 1) * waves * 256;
+      for (int n = 0; n < 2; n++) tokens[i][n] = tokens_of(i, min(sub + n * a.parts, 3));
+    float4 *sums = reinterpret_cast<float4 *>(lds);
+    __syncthreads();   // every wavefront is through with the codes, whose place the sums take
 #pragma unroll
-      for (int g = 0; g < 4; g++)
-        place[wave * 256 + g * 64 + lane] =
-            make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
-      __syncthreads();
-      for (int g = sub; g < 4; g += a.parts) {
-        const float4 *from = place + (wave - sub) * 256 + g * 64 + lane;
-        float4 sum = from[0];
-        for (int p = 1; p < a.parts; p++) {
-          const float4 v = from[p * 256];
-          sum.x += v.x;
-          sum.y += v.y;
-          sum.z += v.z;
-          sum.w += v.w;
+    for (int i = 0; i < kBlocks; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        // a tile at a time, in one of two places; the parts share its groups of four values
+        float4 *place = sums + ((2 * i + j) & 1) * waves * 256;
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+          place[(local * a.parts + sub) * 256 + g * 64 + lane] =
+              make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
+        __syncthreads();
+#pragma unroll
+        for (int n = 0; n < 2; n++) {
+          const int g = sub + n * a.parts;
+          if (g >= 4) break;
+          const float4 *from = place + local * a.parts * 256 + g * 64 + lane;
+          float4 sum = from[0];
+          for (int p = 1; p < a.parts; p++) {
+            const float4 v = from[p * 256];
+            sum.x += v.x;
+            sum.y += v.y;
+            sum.z += v.z;
+            sum.w += v.w;
+          }
+          const float v[4] = {sum.x, sum.y, sum.z, sum.w};
+          write(v, tokens[i][n], i, j, g);
         }
-        const float v[4] = {sum.x, sum.y, sum.z, sum.w};
-        write(v, i, j, g);
       }
-    }
+  }
+  if (kHidden)
+#pragma unroll
+    for (int i = 0; i < kBlocks; i++)
+      if (high[i]) a.spoiled[(first_block + i) * kBlockTokens + (lane & 31)] = 1;
 }
 
+template <bool kHidden, bool kTableInLds>
 __global__ __launch_bounds__(kMaxThreads) void batch_product_kernel(BatchArgs a) {
   extern __shared__ __align__(16) uint32_t lds[];
   // the workgroups of a chunk, which read the same activations, run on one die
@@ -304,9 +438,15 @@ __global__ __launch_bounds__(kMaxThreads) void batch_product_kernel(BatchArgs a)
   const int e = __builtin_amdgcn_readfirstlane(what.x);
   const int first_block = __builtin_amdgcn_readfirstlane(what.y);
   if (__builtin_amdgcn_readfirstlane(what.z) > 1)
-    slices_times_tokens<2>(a, lds, e, group, first_block);
+    slices_times_tokens<kHidden, kTableInLds, 2>(a, lds, e, group, first_block);
   else
-    slices_times_tokens<1>(a, lds, e, group, first_block);
+    slices_times_tokens<kHidden, kTableInLds, 1>(a, lds, e, group, first_block);
+}
+
+// The tables of all experts, a workgroup each, for products that keep none in LDS.
+__global__ __launch_bounds__(kMaxThreads) void fill_tables_kernel(BatchArgs a, uint16_t *tables) {
+  fill_table(a, blockIdx.x, tables + static_cast<int64_t>(blockIdx.x) * physical_columns(a.k.width),
+             order_piece(a, blockIdx.x, threadIdx.x), threadIdx.x, blockDim.x);
 }
 
 // One workgroup.  Every token gets a slot: its expert's tokens fill blocks of 32, an
@@ -323,7 +463,7 @@ __global__ __launch_bounds__(1024) void group_blocks_kernel(
   for (int b = tid; b < buckets; b += 1024) count[b] = 0;
   __syncthreads();
   int faults = 0;
-  int bucket[kBatchPiece / 1024];
+  int bucket[kBatchPiece / 1024], rank[kBatchPiece / 1024];   // which expert's, and which of its tokens
 #pragma unroll
   for (int i = 0; i < kBatchPiece / 1024; i++) {
     const int t = i * 1024 + tid;
@@ -333,7 +473,7 @@ __global__ __launch_bounds__(1024) void group_blocks_kernel(
   }
 #pragma unroll
   for (int i = 0; i < kBatchPiece / 1024; i++)
-    if (i * 1024 + tid < tokens) atomicAdd(&count[bucket[i]], 1);
+    if (i * 1024 + tid < tokens) rank[i] = atomicAdd(&count[bucket[i]], 1);
   if (faults) atomicAdd(&ctrl[kCtrlBadIds], faults);
   __syncthreads();
   const int seg = (buckets + 1023) / 1024;
@@ -373,7 +513,6 @@ __global__ __launch_bounds__(1024) void group_blocks_kernel(
       totals[kTotalChunks] = chunk;
       totals[kTotalLive] = block;
       totals[kTotalBlocks] = block + nb;
-      ctrl[kCtrlTiles] = 0;
     } else {
       for (int i = 0; i < nb; i += kChunkBlocks)
         chunks[chunk++] = make_int4(b, block + i, min(kChunkBlocks, nb - i), 0);
@@ -385,7 +524,7 @@ __global__ __launch_bounds__(1024) void group_blocks_kernel(
   for (int i = 0; i < kBatchPiece / 1024; i++) {
     const int t = i * 1024 + tid;
     if (t < tokens) {
-      const int place = atomicAdd(&next[bucket[i]], 1);
+      const int place = next[bucket[i]] + rank[i];
       slots[place] = t;
       spoiled[place] = 0;
     }
@@ -401,7 +540,7 @@ __device__ __forceinline__ void write_operands(u32x4 *out, int64_t step, int t, 
     u32x4 w;
 #pragma unroll
     for (int k = 0; k < 4; k++)
-      w[k] = v[slot_column(h, 2 * k)] | static_cast<uint32_t>(v[slot_column(h, 2 * k + 1)]) << 16;
+      w[k] = v[column_of_place(h, 2 * k)] | static_cast<uint32_t>(v[column_of_place(h, 2 * k + 1)]) << 16;
     out[step * 64 + h * 32 + t] = w;
   }
 }
@@ -417,15 +556,13 @@ __global__ __launch_bounds__(256) void pack_tokens_kernel(
   const int t = threadIdx.x & 31;
   const int token = slots[block * kBlockTokens + t];
   const bool live = block < totals[kTotalLive];
-  const uint16_t *from = x + (token < 0 ? 0 : token) * ldx;
+  const uint16_t *from = x + token * ldx;
+  if (token < 0) return;   // what the operands hold of it goes nowhere
   bool bad = false;
   for (int st = blockIdx.y * 8 + (threadIdx.x >> 5); st < steps; st += gridDim.y * 8) {
     const int c = st * kStepColumns;
     uint16_t v[16];
-    if (token < 0) {
-#pragma unroll
-      for (int i = 0; i < 16; i++) v[i] = 0;
-    } else if (aligned && c + 16 <= width) {
+    if (aligned && c + 16 <= width) {
       const uint4 a = *reinterpret_cast<const uint4 *>(from + c);
       const uint4 b = *reinterpret_cast<const uint4 *>(from + c + 8);
       __builtin_memcpy(v, &a, 16);
@@ -438,7 +575,7 @@ __global__ __launch_bounds__(256) void pack_tokens_kernel(
 #pragma unroll
       for (int i = 0; i < 16; i++) bad |= not_finite(v[i]);
       write_operands(out + static_cast<int64_t>(block) * steps * 64, st, t, v);
-    } else if (token >= 0) {
+    } else {
       for (int i = 0; i < 16; i++)
         if (c + i < width) y[token * ldy + c + i] = v[i];
     }
@@ -446,103 +583,50 @@ __global__ __launch_bounds__(256) void pack_tokens_kernel(
   if (bad) spoiled[block * kBlockTokens + t] = 1;
 }
 
-// h, rows of 32 tokens, into operands.
-__global__ __launch_bounds__(256) void pack_hidden_kernel(
-    const uint16_t *__restrict__ rows, int width, int32_t *__restrict__ spoiled,
-    const int32_t *__restrict__ totals, u32x4 *__restrict__ out) {
-  const int block = blockIdx.x;
-  if (block >= totals[kTotalLive]) return;
-  const int steps = steps_of(width);
-  const int pair = threadIdx.x & 15;   // tokens 2 pair and 2 pair + 1
-  const uint32_t *from = reinterpret_cast<const uint32_t *>(rows + static_cast<int64_t>(block) * width * kBlockTokens) + pair;
-  uint32_t bad = 0;
-  for (int st = blockIdx.y * 16 + (threadIdx.x >> 4); st < steps; st += gridDim.y * 16) {
-    uint16_t v[2][16];
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-      const int c = st * kStepColumns + i;
-      const uint32_t w = c < width ? from[c * (kBlockTokens / 2)] : 0u;
-      v[0][i] = static_cast<uint16_t>(w);
-      v[1][i] = static_cast<uint16_t>(w >> 16);
-      if (not_finite(w)) bad |= 1;
-      if (not_finite(w >> 16)) bad |= 2;
-    }
-#pragma unroll
-    for (int m = 0; m < 2; m++)
-      write_operands(out + static_cast<int64_t>(block) * steps * 64, st, 2 * pair + m, v[m]);
-  }
-#pragma unroll
-  for (int m = 0; m < 2; m++)
-    if (bad >> m & 1) spoiled[block * kBlockTokens + 2 * pair + m] = 1;
-}
-
-// y from rows of 32 tokens; spoiled tokens are listed, one to a tile.
-__global__ __launch_bounds__(256) void unpack_tokens_kernel(
-    const uint16_t *__restrict__ rows, uint16_t *__restrict__ y, int64_t ldy, int height, bool aligned,
-    const int32_t *__restrict__ slots, const int32_t *__restrict__ spoiled,
-    const int32_t *__restrict__ block_expert, const int32_t *__restrict__ totals,
-    int2 *__restrict__ tiles, int32_t *__restrict__ ctrl) {
-  const int block = blockIdx.x;
-  if (block >= totals[kTotalLive]) return;
-  const int t = threadIdx.x & 31;
-  const int slot = block * kBlockTokens + t;
-  const int token = slots[slot];
-  if (token < 0) return;
-  if (spoiled[slot]) {
-    if (blockIdx.y == 0 && threadIdx.x < 32)
-      tiles[atomicAdd(&ctrl[kCtrlTiles], 1)] = make_int2(block_expert[block], slot);
-    return;
-  }
-  const uint16_t *from = rows + static_cast<int64_t>(block) * height * kBlockTokens + t;
-  uint16_t *to = y + token * ldy;
-  for (int c = (blockIdx.y * 8 + (threadIdx.x >> 5)) * 8; c < height; c += gridDim.y * 64) {
-    uint16_t v[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = c + i < height ? from[(c + i) * kBlockTokens] : 0;
-    if (aligned && c + 8 <= height) {
-      uint4 w;
-      __builtin_memcpy(&w, v, 16);
-      *reinterpret_cast<uint4 *>(to + c) = w;
-    } else {
-      for (int i = 0; i < 8; i++)
-        if (c + i < height) to[c + i] = v[i];
-    }
-  }
-}
-
-// The listed tokens (ctrl[kCtrlTiles] of them), a workgroup each, as
-// moe_prepared_fused_kernel walks them: the same sums.  LDS: x | h.
-__global__ __launch_bounds__(kMaxThreads) void walk_listed_kernel(PreparedArgs a) {
+// The tokens in the slots that are marked, a workgroup each, as moe_prepared_fused_kernel
+// walks them: the same sums.  LDS: x | h.  Workgroup b looks at slots b, b + grid, ...: an
+// expert's tokens, which may all be marked, lie side by side.
+__global__ __launch_bounds__(kMaxThreads) void walk_spoiled_kernel(PreparedArgs a, const int32_t *__restrict__ slots,
+                                                                   const int32_t *__restrict__ spoiled,
+                                                                   const int32_t *__restrict__ block_expert,
+                                                                   const int32_t *__restrict__ totals) {
   extern __shared__ __align__(16) uint32_t lds[];
-  const int listed = __builtin_amdgcn_readfirstlane(a.ctrl[kCtrlTiles]);
-  if (static_cast<int>(blockIdx.x) >= listed) return;
   uint32_t *xa = lds, *ha = lds + a.xdwords;
   const int waves = blockDim.x >> 6;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (int i = threadIdx.x; i < a.hdwords; i += blockDim.x) ha[i] = 0u;
-  for (int tile = blockIdx.x; tile < listed; tile += gridDim.x) {
-    const int2 what = a.groups[tile];
-    const int e = __builtin_amdgcn_readfirstlane(what.x);
-    const int t = __builtin_amdgcn_readfirstlane(a.order[what.y]);
-    __syncthreads();   // the previous token is through
-    stage_activations(xa, a.x + static_cast<int64_t>(t) * a.ldx, a.k[0].width);
-    __syncthreads();
-    for (int s = wave; s < a.k[0].slices; s += waves) {
-      SliceWalk w = load_slice(a, a.k[0], static_cast<int64_t>(e) * a.k[0].slices + s);
-      const float res = run_slice(w, a.stream, xa);
-      if (w.ridx != 0xffff) {
-        uint32_t out = f32_to_bf16(res);
-        if (out & 0x8000u) out = 0;
-        uint32_t *p = ha + 2 * physical_column(w.ridx);
-        p[0] = out;
-        p[1] = out << 16;
+  const int live = totals[kTotalLive] * kBlockTokens, grid = gridDim.x;
+  bool fresh = true;
+  for (int first = 0; first < live; first += 64 * grid) {
+    // (every wavefront looks at the same 64 slots)
+    const int mine = first + static_cast<int>(threadIdx.x & 63) * grid + static_cast<int>(blockIdx.x);
+    unsigned long long found = __ballot(mine < live && slots[mine] >= 0 && spoiled[mine]);
+    for (; found; found &= found - 1) {
+      const int slot = first + (__ffsll(found) - 1) * grid + static_cast<int>(blockIdx.x);
+      const int e = __builtin_amdgcn_readfirstlane(block_expert[slot / kBlockTokens]);
+      const int t = __builtin_amdgcn_readfirstlane(slots[slot]);
+      if (fresh)
+        for (int i = threadIdx.x; i < a.hdwords; i += blockDim.x) ha[i] = 0u;
+      fresh = false;
+      __syncthreads();   // the previous token is through
+      stage_activations(xa, a.x + static_cast<int64_t>(t) * a.ldx, a.k[0].width);
+      __syncthreads();
+      for (int s = wave; s < a.k[0].slices; s += waves) {
+        SliceWalk w = load_slice(a, a.k[0], static_cast<int64_t>(e) * a.k[0].slices + s);
+        const float res = run_slice(w, a.stream, xa);
+        if (w.ridx != 0xffff) {
+          uint32_t out = f32_to_bf16(res);
+          if (out & 0x8000u) out = 0;
+          uint32_t *p = ha + 2 * physical_column(w.ridx);
+          p[0] = out;
+          p[1] = out << 16;
+        }
       }
-    }
-    __syncthreads();
-    for (int s = wave; s < a.k[1].slices; s += waves) {
-      SliceWalk w = load_slice(a, a.k[1], static_cast<int64_t>(e) * a.k[1].slices + s);
-      const float res = run_slice(w, a.stream, ha);
-      write_row(a.y + static_cast<int64_t>(t) * a.ldy, w.ridx, res, kStore);
+      __syncthreads();
+      for (int s = wave; s < a.k[1].slices; s += waves) {
+        SliceWalk w = load_slice(a, a.k[1], static_cast<int64_t>(e) * a.k[1].slices + s);
+        const float res = run_slice(w, a.stream, ha);
+        write_row(a.y + static_cast<int64_t>(t) * a.ldy, w.ridx, res, kStore);
+      }
     }
   }
 }

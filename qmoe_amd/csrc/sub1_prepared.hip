@@ -3361,10 +3361,84 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
 
 // ---- batches on the matrix cores (sub1_batch.h) ----
 
+int batch_piece(int tokens) {
+  const int pieces = (tokens + kBatchPiece - 1) / kBatchPiece;
+  return (tokens + pieces - 1) / pieces;
+}
+
+// Steps of a product: x has its columns in their own order, h in the order of wi's slices.
+int product_steps(const Prepared &p, int kind) {
+  return kind ? steps_of_slices((p.height[0] + 63) / 64) : steps_of(p.width[0]);
+}
+
+// How a product's slices are given to workgroups.
+struct BatchPlan {
+  int per_group, parts;
+  bool table_in_lds;
+  size_t lds;
+};
+
+constexpr size_t kBatchLds = 160 * 1024 - 64;
+
+// LDS holds the codes of `fit` slices beside a table: with room for three and more, workgroups
+// of up to four wavefronts, one to a SIMD; for two, of up to eight; for one, of twelve.  (128 base
+// experts on 4096 tokens: wi 52 us with four wavefronts of a slice each, 60 with two to each
+// of two slices, 62 with eight slices; 40 c-2048 experts on 700, wo, whose codes take 98 KB, with 4, 8, 12 and 16
+// wavefronts: 205, 166, 162 and 165 for the call.)  Wavefronts share a slice as long as
+// each gets a group of chunks, the least that one can expand, and take slices of their
+// own beyond that (c-2048 wi by 1, 2 and 4 to a slice: 208, 181, 166 us) - but not where a
+// compute unit would then hold fewer than twelve wavefronts, as it does of rows with few entries,
+// whose slices are short but whose codes take LDS as any: more of them share a slice then, the
+// ones without a group of chunks for its multiplying alone (95 % zeros, sharing by chunks alone:
+// 128 base experts on 4096 tokens 166 us against 128) - nor where small workgroups with a table each
+// leave room for too few: then one holds all the slices that fit (base wo by one slice of four
+// wavefronts, two of those to a unit, 82 us, by one of eight 67, by three of four 65).  A table that
+// does not fit beside a single slice, of rows of more than 9000 columns, stays in global memory.
+bool plan_batch(const Prepared &p, int kind, size_t lds_limit, BatchPlan *out) {
+  const int slices[2] = {(p.height[0] + 63) / 64, (p.height[1] + 63) / 64};
+  const double weight = static_cast<double>(slices[0]) * p.width[0] + static_cast<double>(slices[1]) * p.width[1];
+  const double chunks = static_cast<double>(p.total_chunks) / p.count * p.width[kind] / weight;
+  const size_t code_bytes = slice_code_bytes(product_steps(p, kind));
+  // (wi needs no table)
+  const size_t wanted = kind ? table_bytes(p.width[kind]) : 0;
+  out->table_in_lds = code_bytes + wanted <= lds_limit;
+  const size_t table = out->table_in_lds ? wanted : 0;
+  if (code_bytes + table > lds_limit) return false;
+  const int fit = static_cast<int>((lds_limit - table) / code_bytes);
+  int waves = fit >= 3 ? 4 : fit == 2 ? 8 : 12;
+  for (int parts = 1;; parts *= 2) {
+    if (parts > waves) parts = waves;
+    if (parts < waves && parts * kGroupChunks < 0.75 * chunks) continue;
+    int per_group = std::min(waves / parts, slices[kind]);
+    for (; per_group > 0; per_group--) {
+      const size_t sums = parts > 1 ? static_cast<size_t>(2 * per_group * parts) * 4096 : 0;
+      out->lds = std::max(per_group * code_bytes + table, sums);
+      if (out->lds <= lds_limit) break;
+    }
+    if (per_group == 0) return false;
+    out->per_group = per_group;
+    out->parts = parts;
+    if (static_cast<int>(lds_limit / out->lds) * per_group * parts >= 12) return true;
+    if (parts == waves) {
+      if (waves == 12) return true;
+      waves = 12;   // and look on from as many parts
+      parts /= 2;
+    }
+  }
+}
+
+bool batch_takes(const Prepared &p) {
+  BatchPlan plan;
+  const size_t lds_fused = (static_cast<size_t>(activation_dwords(p.width[0])) + activation_dwords(p.width[1])) * 4;
+  return p.count <= kBatchMaxExperts && lds_fused <= kBatchLds && plan_batch(p, 0, kBatchLds, &plan) &&
+         plan_batch(p, 1, kBatchLds, &plan);
+}
+
 // The scratch memory of a piece, arrays back to back, 256-byte aligned.
 struct BatchLayout {
-  int64_t totals, slots, spoiled, block_expert, chunks, tiles;
-  int64_t x, h_rows, h;   // y's rows take x's place, which is done with by then
+  int64_t totals, slots, spoiled, block_expert, chunks;
+  int64_t x, h;        // operands
+  int64_t tables;      // where LDS has no room for them
   int64_t bytes;
   int max_blocks, max_chunks;
 };
@@ -3388,69 +3462,14 @@ BatchLayout batch_layout(const Prepared &p, int tokens) {
   b.spoiled = take(slots * 4);
   b.block_expert = take(blocks * 4);
   b.chunks = take((static_cast<int64_t>(b.max_chunks) + 7) / 8 * 8 * 16);
-  b.tiles = take(slots * 8);
-  b.x = take(blocks * std::max(steps_of(p.width[0]) * 1024, p.height[1] * kBlockTokens * 2));
-  b.h_rows = take(blocks * p.height[0] * kBlockTokens * 2);
-  b.h = take(blocks * steps_of(p.width[1]) * 1024);
+  b.x = take(blocks * product_steps(p, 0) * 1024);
+  b.h = take(blocks * product_steps(p, 1) * 1024);
+  BatchPlan plan;
+  b.tables = off;
+  if (plan_batch(p, 1, kBatchLds, &plan) && !plan.table_in_lds)
+    take(static_cast<int64_t>(p.count) * physical_columns(p.width[1]) * 2);
   b.bytes = off;
   return b;
-}
-
-int batch_piece(int tokens) {
-  const int pieces = (tokens + kBatchPiece - 1) / kBatchPiece;
-  return (tokens + pieces - 1) / pieces;
-}
-
-// How a product's slices are given to workgroups.
-struct BatchPlan {
-  int per_group, parts;
-  size_t lds;
-};
-
-// LDS holds the codes of `fit` slices: with room for three and more, workgroups of up to four
-// wavefronts, one to a SIMD; for two, of up to eight; for one, of twelve.  (128 base experts on
-// 4096 tokens: 131 us; with wi's workgroups of 8 wavefronts 134, with wo's of 6, 8 and 12
-// 142, 132 and 153.  40 c-2048 experts on 700 tokens, wo, whose codes take 98 KB, with
-// 4, 8, 12 and 16 wavefronts: 205, 166, 162 and 165.)  Wavefronts share a slice as long as
-// each gets a group of chunks, the least that one can expand, and take slices of their
-// own beyond that (c-2048 wi by 1, 2 and 4 to a slice: 208, 181, 166 us; base wi, of
-// hardly two groups, 134, 131, 144) - but not where a compute unit would then hold fewer than
-// twelve wavefronts, as it does of rows with few entries, whose slices are short but whose codes
-// take LDS as any: more of them share a slice then, the ones without a group of chunks for its
-// multiplying alone.  (With 95 % zeros, sharing by chunks alone: 128 base experts on 4096 tokens,
-// wo's workgroups of 4 wavefronts and 99 KB, 166 us against 128; 40 c-2048 experts on 640, of 4 and
-// 98 KB, 201 against 154.)
-bool plan_batch(const Prepared &p, int kind, size_t lds_limit, BatchPlan *out) {
-  const int slices[2] = {(p.height[0] + 63) / 64, (p.height[1] + 63) / 64};
-  const double weight = static_cast<double>(slices[0]) * p.width[0] + static_cast<double>(slices[1]) * p.width[1];
-  const double chunks = static_cast<double>(p.total_chunks) / p.count * p.width[kind] / weight;
-  const size_t code_bytes = slice_code_bytes(p.width[kind]);
-  const int fit = static_cast<int>(lds_limit / code_bytes);
-  const int waves = fit >= 3 ? 4 : fit == 2 ? 8 : 12;
-  int parts = 1;
-  while (parts < waves && parts * kGroupChunks < 0.75 * chunks) parts *= 2;
-  for (;; parts *= 2) {
-    parts = std::min(parts, waves);
-    int per_group = std::min(waves / parts, slices[kind]);
-    for (; per_group > 0; per_group--) {
-      const size_t sums = parts > 1 ? static_cast<size_t>(2 * per_group * parts) * 4096 : 0;
-      out->lds = std::max(per_group * code_bytes, sums);
-      if (out->lds <= lds_limit) break;
-    }
-    if (per_group == 0) return false;
-    out->per_group = per_group;
-    out->parts = parts;
-    if (parts == waves || static_cast<int>(lds_limit / out->lds) * per_group * parts >= 12) return true;
-  }
-}
-
-constexpr size_t kBatchLds = 160 * 1024 - 64;
-
-bool batch_takes(const Prepared &p) {
-  BatchPlan plan;
-  const size_t lds_fused = (static_cast<size_t>(activation_dwords(p.width[0])) + activation_dwords(p.width[1])) * 4;
-  return p.count <= kBatchMaxExperts && lds_fused <= kBatchLds && plan_batch(p, 0, kBatchLds, &plan) &&
-         plan_batch(p, 1, kBatchLds, &plan);
 }
 
 // Blocks of `per` that an expert's tokens fill, on average, where their number is spread
@@ -3465,26 +3484,26 @@ double blocks_on_average(double each, int per) {
 }
 
 // Whether the matrix cores are the faster way for `tokens` tokens, by estimates in microseconds
-// fitted to both at 8 to 128 tokens an expert through 1 to 2048 experts of the three Switch shapes
-// and of four odd ones, with 80 to 95 % zeros or shares that differ from row to row (464 launches).
-// Here, for every piece of a batch, which expands every expert that it hits: 42 and, per million
-// weights, 0.025 and 0.31 times the entries of a weight for every 64 of an expert's tokens, 0.073
-// for every 32 (within 9 %, root mean square).  Walking: a compute unit takes
+// fitted to both at 8 to 128 tokens an expert through 8 to 128 experts of the three Switch shapes
+// and of three odd ones, with 80 to 95 % zeros (168 launches).  Here, for every piece of a batch,
+// which expands every expert that it hits: 35 and, per million weights, 0.29 times the entries
+// of a weight for every 64 of an expert's tokens, 0.08 for every 32 (within 11 %, root mean
+// square).  Walking: a compute unit takes
 // token_us = 8 + entries / 23400 for a token and, where launch_prepared groups tokens by expert,
 // 7 + 1.85 (token_us - 8) for up to four, in whole rounds.  The matrix cores must promise 5 %: of those
-// launches that leaves 6 on the slower way, by 8 % at most, and 38 where they would have been
-// faster, by up to 23 %; of 196 others none and 13.  A piece with less than 8 tokens an expert never goes there.  (Pricing one
-// pass over the experts for a batch that runs in pieces, as it was done first, sent 32 768 tokens
-// through 2048 base experts this way: 5862 us, walking takes 1735.)
+// launches that leaves none on the slower way, and 18 where they would have been faster, by up to 44 %,
+// most of them where walking is estimated low.  A piece with less than 8 tokens an expert never goes
+// there.  (Pricing one pass over the experts for a batch that runs in pieces, as it was done first, sent
+// 32 768 tokens through 2048 base experts this way: 5862 us, walking takes 1735.)
 bool batch_pays(const Prepared &p, int tokens, int cus) {
   const int piece = batch_piece(tokens), pieces = (tokens + piece - 1) / piece;
   if (piece < 8 * static_cast<int64_t>(p.count) || !batch_takes(p)) return false;
   const double each = static_cast<double>(piece) / p.count;
   const double weights = 2e-6 * p.count * p.height[0] * p.width[0];
   const double entries = 1e-6 * p.total_chunks * (64.0 * kFields);
-  const double by_chunks = blocks_on_average(each, kChunkBlocks * kBlockTokens) * (0.025 * weights + 0.31 * entries);
-  const double by_blocks = blocks_on_average(each, kBlockTokens) * 0.073 * weights;
-  const double batch_us = pieces * (42.0 + 256.0 / cus * (by_chunks + by_blocks));
+  const double by_chunks = blocks_on_average(each, kChunkBlocks * kBlockTokens) * 0.29 * entries;
+  const double by_blocks = blocks_on_average(each, kBlockTokens) * 0.08 * weights;
+  const double batch_us = pieces * (35.0 + 256.0 / cus * (by_chunks + by_blocks));
   const double walk_us = 1e6 * entries / p.count / 23400.0;   // of a token, besides its 8 us
   const bool grouped = tokens >= 4 * static_cast<int64_t>(p.count) && tokens >= 4 * cus;
   const double rounds = (0.25 * tokens + 0.375 * p.count) / cus;
@@ -3503,30 +3522,20 @@ int launch_batch(const Prepared &p, const int32_t *token_expert, const uint16_t 
   int32_t *spoiled = reinterpret_cast<int32_t *>(scratch + b.spoiled);
   int32_t *block_expert = reinterpret_cast<int32_t *>(scratch + b.block_expert);
   int4 *chunks = reinterpret_cast<int4 *>(scratch + b.chunks);
-  int2 *tiles = reinterpret_cast<int2 *>(scratch + b.tiles);
   u32x4 *xs = reinterpret_cast<u32x4 *>(scratch + b.x), *hs = reinterpret_cast<u32x4 *>(scratch + b.h);
-  uint16_t *h_rows = reinterpret_cast<uint16_t *>(scratch + b.h_rows);
-  uint16_t *y_rows = reinterpret_cast<uint16_t *>(scratch + b.x);
   const int d_model = p.width[0], d_ff = p.height[0];
-  const bool aligned = d_model % 8 == 0 && !misaligned(x, 16) && !misaligned(y, 16);
+  const bool aligned = d_model % 8 == 0 && !misaligned(x, 16);
 
   group_blocks_kernel<<<1, 1024, static_cast<size_t>(p.count + 1) * 8, s>>>(
       token_expert, tokens, p.count, slots, spoiled, block_expert, chunks, totals, ctrl);
   const auto shares = [](int work, int per) { return static_cast<unsigned>(std::max(1, std::min(16, (work + per - 1) / per))); };
   pack_tokens_kernel<<<dim3(b.max_blocks, shares(steps_of(d_model), 16)), 256, 0, s>>>(
       x, y, d_model, d_model, d_model, aligned, slots, spoiled, totals, xs);
-  // the most they may have, not what this launch has: another thread's launch, of other shapes,
-  // may lie between this call and ours
-  for (const void *fn : {reinterpret_cast<const void *>(batch_product_kernel),
-                         reinterpret_cast<const void *>(walk_listed_kernel)})
-    HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kBatchLds)));
   PreparedArgs a = {};
   a.stream = static_cast<const uint2 *>(p.codes);
   a.ckpt = reinterpret_cast<const uint16_t *>(a.stream + p.total_chunks * 64);
   int64_t first_slice = 0;
   for (int i = 0; i < 2; i++) {
-    BatchPlan plan;
-    if (!plan_batch(p, i, kBatchLds, &plan)) return fail(SUB1_ERR_SHAPE, "%s: widths too large", who);
     const KindMeta &k = m.k[i];
     KindArgs &ka = a.k[i];
     ka.slice_base = reinterpret_cast<const uint32_t *>(meta + k.slice_base);
@@ -3538,39 +3547,59 @@ int launch_batch(const Prepared &p, const int32_t *token_expert, const uint16_t 
     ka.width = k.width;
     ka.first_slice = first_slice;
     first_slice += static_cast<int64_t>(p.count) * k.slices;
-    BatchArgs b_args;
+  }
+  for (int i = 0; i < 2; i++) {
+    BatchPlan plan;
+    if (!plan_batch(p, i, kBatchLds, &plan)) return fail(SUB1_ERR_SHAPE, "%s: widths too large", who);
+    BatchArgs b_args = {};
     b_args.stream = a.stream;
     b_args.ckpt = a.ckpt;
-    b_args.k = ka;
+    b_args.k = a.k[i];
     b_args.in = i ? hs : xs;
-    b_args.out = i ? y_rows : h_rows;
+    if (i == 0) {
+      b_args.h = hs;
+      b_args.h_steps = product_steps(p, 1);
+      b_args.wo_minmax = a.k[1].minmax;
+      b_args.wo_rows = a.k[1].slices * 64;
+    } else {
+      b_args.order = a.k[0].row_idx;
+      b_args.order_rows = a.k[0].slices * 64;
+      b_args.y = y;
+      b_args.ldy = d_model;
+    }
+    b_args.slots = slots;
     b_args.chunks = chunks;
     b_args.totals = totals;
     b_args.spoiled = spoiled;
-    b_args.steps = steps_of(k.width);
+    b_args.steps = product_steps(p, i);
     b_args.parts = plan.parts;
     b_args.per_group = plan.per_group;
-    b_args.slice_groups = (k.slices + plan.per_group - 1) / plan.per_group;
-    b_args.relu = i == 0;
-    batch_product_kernel<<<static_cast<unsigned>((b.max_chunks + 7) / 8 * 8 * b_args.slice_groups),
-                           64 * plan.per_group * plan.parts, plan.lds, s>>>(b_args);
-    if (i == 0)
-      pack_hidden_kernel<<<dim3(b.max_blocks, shares(steps_of(d_ff), 32)), 256, 0, s>>>(h_rows, d_ff, spoiled,
-                                                                                       totals, hs);
+    b_args.slice_groups = (a.k[i].slices + plan.per_group - 1) / plan.per_group;
+    if (i == 1 && !plan.table_in_lds) {
+      uint16_t *tables = reinterpret_cast<uint16_t *>(scratch + b.tables);
+      b_args.tables = tables;
+      fill_tables_kernel<<<p.count, kMaxThreads, 0, s>>>(b_args, tables);
+    }
+    void (*const product)(BatchArgs) = i == 0               ? batch_product_kernel<true, false>
+                                       : plan.table_in_lds ? batch_product_kernel<false, true>
+                                                           : batch_product_kernel<false, false>;
+    // the most it may have, not what this launch has: another thread's launch, of other shapes,
+    // may lie between this call and ours
+    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(product), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                static_cast<int>(kBatchLds)));
+    product<<<static_cast<unsigned>((b.max_chunks + 7) / 8 * 8 * b_args.slice_groups),
+              64 * plan.per_group * plan.parts, plan.lds, s>>>(b_args);
   }
-  unpack_tokens_kernel<<<dim3(b.max_blocks, shares(d_model, 128)), 256, 0, s>>>(
-      y_rows, y, d_model, d_model, aligned, slots, spoiled, block_expert, totals, tiles, ctrl);
-  // what the tokens listed there need of the walking kernels
-  a.order = slots;
-  a.groups = tiles;
+  // what they leave to the walking kernels
   a.x = x;
   a.y = y;
   a.ldx = a.ldy = d_model;
-  a.ctrl = ctrl;
   a.xdwords = activation_dwords(d_model);
   a.hdwords = activation_dwords(d_ff);
+  HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(walk_spoiled_kernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kBatchLds)));
   const size_t lds = static_cast<size_t>(a.xdwords + a.hdwords) * 4;
-  walk_listed_kernel<<<std::min(tokens, 256), kMaxThreads, lds, s>>>(a);
+  walk_spoiled_kernel<<<std::min(tokens, 256), kMaxThreads, lds, s>>>(a, slots, spoiled, block_expert, totals);
   HIP_TRY(hipGetLastError());
   sub1::note_kernel("batch_product_kernel");
   return SUB1_OK;

@@ -476,7 +476,7 @@ class PreparedStack:
         on the other tokens.  Scratch memory comes from torch's allocator for
         the call: an expert's tokens take whole blocks of 32 slots, at most
         T + 31 (min(T, experts) + 1) of them for T tokens (up to 8192, larger
-        batches run in pieces), of 4 d_ff + 2 d_model bytes each and a few more."""
+        batches run in pieces), of 2 d_ff + 2 d_model bytes each and a few more."""
         dev = self.device
         _lib.check_faults()       # what earlier launches reported (host memory, no sync)
         lib = _lib.load()

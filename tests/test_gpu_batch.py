@@ -71,6 +71,28 @@ def test_exact_sums_equal_the_oracle(oracle, d_model, d_ff, p0, counts):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('d_model,d_ff', [(20, 9700), (9700, 70), (51, 128), (52, 64 * 3 + 1)])
+def test_wherever_the_table_of_columns_lies(oracle, d_model, d_ff):
+    """Rows of 9700 columns: their codes fill LDS, the table of where they go is kept in
+    global memory (either projection); and steps that are no whole turns.  Exact sums, as above."""
+    wi = [layers(oracle, d_ff, d_model, 0.97, 30 + e) for e in range(2)]
+    wo = [layers(oracle, d_model, d_ff, 0.97, 40 + e) for e in range(2)]
+    prep = prepared(wi, wo)
+    route = np.repeat(np.int32([1, 0, -1]), [37, 33, 2])
+    xs = so.f32_to_bf16_bits(np.random.default_rng(5).integers(-2, 3, (route.size, d_model)).astype(np.float32))
+    x, te = bf16_dev(xs), torch.from_numpy(route).cuda()
+    y = prep.forward_batch(x, te)
+    assert torch.equal(prep.forward(x, te), y)
+    got = bits_host(y)
+    for i in (0, 36, 37, 69):
+        assert np.array_equal(got[i], oracle.expert_ffn(wi[route[i]], wo[route[i]], xs[i], order=2)[0]), i
+    x[3, d_model - 1] = float('nan')       # walked, in its own place
+    want = prep.forward(x, te)
+    assert prep.forward_batch(x, te, y=x) is x
+    assert torch.equal(x.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.gpu
 def test_a_token_without_finite_activations_spoils_no_other(oracle):
     """x with an infinity or a NaN, and x whose h overflows: what the walking kernel
     gives for the token alone; the tokens of its block are as without it."""
