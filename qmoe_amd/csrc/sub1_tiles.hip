@@ -28,27 +28,26 @@
 // serves 64 tokens that is eight instructions per MFMA instead of six, and six
 // are what an MFMA hides.)
 //
-// Kernel: a workgroup owns 64 rows x 64 tokens; its wavefronts split the
-// windows of 128 columns among themselves (wavefront v takes v, v + n, ...).  Per
-// window a wavefront brings the tokens' activations, 64 x 128, into its own
-// 16 KB of LDS (16-byte pieces, four tokens an instruction; the pieces of a
-// token are XOR-swizzled with the token's number so that neither the arrivals
-// nor the operand reads meet in a bank), and per step of 16 columns reads its
-// A operands from there, builds its B operands from the codes and adds into a
-// 64 x 64 fp32 accumulator (2 x 2 MFMA blocks).  Where x rows are 16-byte
-// aligned the loads go straight into LDS, into a second buffer, a whole window
-// ahead of the arithmetic (matvec_tiles_kernel); otherwise through registers,
-// element by element (matvec_tiles_ragged_kernel).  All of them are buffer
-// loads: what lies past the last token, past the width or past a wavefront's
-// last window is given an offset outside the buffer (or an empty buffer) and
-// reads nothing, without a branch or a mask.  At the end the partial tiles are
-// added through LDS in wavefront order, rounded to bf16 and added onto y in
-// bf16 (reference sub1_cuda_kernel.cu:199-200).  The number of wavefronts
+// Kernels: a workgroup owns 64 rows x 64 tokens, or up to 128 of either.  It
+// walks windows of 128 columns; the tokens' activations of a window lie in LDS
+// as tiles of 64 x 128 (16 KB; 16-byte pieces, four tokens an instruction; the
+// pieces of a token are XOR-swizzled with the token's number so that neither
+// the arrivals nor the operand reads meet in a bank), and per step of 16
+// columns a wavefront reads its A operands from there, builds its B operands
+// from the codes and adds into 64 x 64 fp32 accumulators (2 x 2 MFMA blocks).
+// Short launches give each wavefront windows and tiles of its own
+// (matvec_tiles_kernel: wavefront v takes windows v, v + n, ...); elsewhere the
+// wavefronts share the tiles (matvec_tiles_shared_kernel).  Where x rows are
+// 16-byte aligned the loads go straight into LDS, into a second buffer, a whole
+// window ahead of the arithmetic; otherwise the shared kernel takes them
+// through registers, in the widest loads that every row's address allows.
+// Either way what lies past the last token, past the width or past the last
+// window is given an offset outside the buffer (or an empty buffer) and reads
+// nothing, without a branch or a mask.  The columns are cut into parts, each
+// summed in order, and the parts are added in order, rounded to bf16 and added
+// onto y in bf16 (reference sub1_cuda_kernel.cu:199-200).  The number of parts
 // depends on the matrix alone, so a token's result does not depend on the
 // launch it is part of.
-//
-// Long sequences go through workgroups of four wavefronts that share each
-// window of activations in LDS instead (matvec_tiles_shared_kernel, below).
 //
 // Bound: a wavefront alone on its SIMD issues an MFMA of this shape every
 // 18 ns (the matrix core needs 13.4); with the four plain instructions per
@@ -87,8 +86,8 @@ constexpr int kTokens = 64;               // tokens per workgroup
 constexpr int kSteps = kCols / 16;        // MFMA steps per window
 constexpr int kMaxWaves = 4;              // wavefronts per workgroup, at most
 constexpr uint32_t kAllZero = 0xaaaaaaaau; // a word of codes of zero weights
-constexpr int kPartialBytes = kTokens * kRows * 4;   // one wavefront's scaled tile
 
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -373,103 +372,108 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tokens_of(const TileArgs &a, c
           : 0u);
 }
 
-// One window: eight steps of four MFMAs on the activations in `tile` (this
-// wavefront's 16 KB) and the weights in `codes`.  Each MFMA keeps the matrix
-// core busy for as long as eight plain instructions take to issue, so the next
-// step's B operands are built a quarter at a time behind the MFMAs of this one
-// and its A operands are requested at its start.
-__device__ __forceinline__ void window_steps(const unsigned char *tile, const TileLane &l,
-                                             const u32x4 (&codes)[2], f32x16 (&acc)[2][2]) {
-  const unsigned char *get = tile + l.get_at;
-  bf16x8 xa[2];
-  u32x4 wv[2];
-#pragma unroll
-  for (int i = 0; i < 2; i++) xa[i] = *reinterpret_cast<const bf16x8 *>(get + i * (32 * 256));
-  WeightsInTheMaking m;
-  decode_share<0, 1, 0>(m, codes[0][0], codes[1][0], l.rows, wv);
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int s = 0; s < kSteps; s++) {
-    bf16x8 xa_next[2];
-    u32x4 wv_next[2];
-    const int sn = s + 1 < kSteps ? s + 1 : s;   // after the last step nothing new
-    const uint32_t word0 = codes[0][sn >> 1], word1 = codes[1][sn >> 1];
-    if (s + 1 < kSteps) {
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-        xa_next[i] = *reinterpret_cast<const bf16x8 *>(
-            tile + (l.get_at ^ static_cast<uint32_t>(32 * sn)) + i * (32 * 256));
-    }
-    const bf16x8 wb0 = __builtin_bit_cast(bf16x8, wv[0]), wb1 = __builtin_bit_cast(bf16x8, wv[1]);
-    auto next_weights = [&](auto slot) {
-      constexpr int kSlot = decltype(slot)::value;
-      if (s + 1 < kSteps) {
-        if (sn & 1) decode_share<kSlot, 4, 1>(m, word0, word1, l.rows, wv_next);
-        else decode_share<kSlot, 4, 0>(m, word0, word1, l.rows, wv_next);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    };
-    acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[0], wb0, acc[0][0], 0, 0, 0);
-    next_weights(std::integral_constant<int, 0>{});
-    acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[0], wb1, acc[0][1], 0, 0, 0);
-    next_weights(std::integral_constant<int, 1>{});
-    acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[1], wb0, acc[1][0], 0, 0, 0);
-    next_weights(std::integral_constant<int, 2>{});
-    acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[1], wb1, acc[1][1], 0, 0, 0);
-    next_weights(std::integral_constant<int, 3>{});
-    if (s + 1 < kSteps) {
-      xa[0] = xa_next[0];
-      xa[1] = xa_next[1];
-      wv[0] = wv_next[0];
-      wv[1] = wv_next[1];
-    }
-  }
+// What the neighbour (lane ^ 1) has.
+__device__ __forceinline__ float neighbour(float v) {
+  constexpr int kDppQuadXor1 = 0xb1;   // quad_perm [1, 0, 3, 2]
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kDppQuadXor1, 0xf, 0xf, true));
 }
 
-// The end of a workgroup: its wavefronts' tiles added in wavefront order,
-// rounded to bf16 and added onto y in bf16 (reference sub1_cuda_kernel.cu:199-
-// 200).  The wavefronts share the tokens, a lane has row `lane` of the block;
-// the y of a lane's tokens are all requested before anything else (tokens past
-// the last: loads that return zero, stores that are dropped; a fresh y: an empty
-// buffer, and the sum is added onto zero as it would be after a fill).  `partial` is
-// LDS that no wavefront reads any more.  kPer = 64 / waves.
-template <int kPer>
-__device__ __forceinline__ void finish_tile(const TileArgs &a, const TileLane &l, int wave,
-                                            int waves, float *partial, const f32x16 (&acc)[2][2]) {
-  const int row = l.block * kRows + l.lane;
+// The end of a workgroup of kKP parts times kRG groups of rows.  The parts of a group each
+// finish a share of its tiles of 32 tokens x 32 rows: what the others have of them goes through
+// `lds`, which no wavefront reads any more, whole registers at a time, and is added in the parts' order;
+// the sum is rounded to bf16 and added onto y in bf16 (reference sub1_cuda_kernel.cu:199-200), tokens
+// past the last and rows past the height dropped.  kPairs: y takes two rows in a 4-byte store.
+// (Through LDS a token's rows at a time, with y read back where it counts as zeros, as it was done
+// first, the end took 10 of 40 us of c-2048 wi on 1136 tokens, against 2 to 3 now.)
+template <bool kPairs, int kRG, int kKP, int kNB>
+__device__ __forceinline__ void finish_tiles(const TileArgs &a, const TileLane &l, int g, int k, bool rows, int live,
+                                             unsigned char *lds, const f32x16 (&acc)[kNB][2]) {
+  constexpr int kTiles = 2 * kNB, kFinish = kTiles / kKP;
+  static_assert(kFinish * kKP == kTiles, "equal shares");
+  float4 *sums = reinterpret_cast<float4 *>(lds);
+  // of tile `n` of what part `of` finishes, from part `from`
+  auto place = [&](int of, int from, int n) {
+    return sums + ((((g * kKP + of) * (kKP - 1) + (from < of ? from : from - 1)) * kFinish + n) * 4) * 64 + l.lane;
+  };
+  if constexpr (kKP > 1) {
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < kTiles; n++)
+      if (n / kFinish != k && n / 2 < live)
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+          place(n / kFinish, k, n % kFinish)[v * 64] =
+              make_float4(acc[n >> 1][n & 1][4 * v], acc[n >> 1][n & 1][4 * v + 1], acc[n >> 1][n & 1][4 * v + 2],
+                          acc[n >> 1][n & 1][4 * v + 3]);
+    __syncthreads();
+  }
   const uint32_t y_bytes =
       static_cast<uint32_t>((static_cast<int64_t>(l.rows_here - 1) * a.ldy + a.height) * 2);
-  uint16_t *y = a.y + static_cast<int64_t>(l.t0) * a.ldy;
-  const __amdgpu_buffer_rsrc_t yb = buffer_over(y, y_bytes), was = buffer_over(y, a.fresh ? 0u : y_bytes);
-  // rows past the height: outside the buffer
-  const uint32_t y_at = row < a.height ? static_cast<uint32_t>(row * 2) : kOutside;
+  const __amdgpu_buffer_rsrc_t yb = buffer_over(a.y + static_cast<int64_t>(l.t0) * a.ldy, y_bytes);
   const uint32_t y_step = static_cast<uint32_t>(a.ldy * 2);
-  uint16_t before[kPer];
+  const bool odd = l.lane & 1;
 #pragma unroll
-  for (int k = 0; k < kPer; k++)
-    before[k] = __builtin_amdgcn_raw_buffer_load_b16(was, y_at + (wave + k * waves) * y_step, 0, 0);
-  // Element (token i, row j) of an accumulator block sits in lane
-  // j + 32 * ((i / 4) % 2), register 4 * (i / 8) + i % 4.
-  float *mine = partial + wave * (kTokens * kRows);
+  for (int n = 0; n < kTiles; n++) {
+    if (n / kFinish != k || n / 2 >= live || !rows) continue;
+    // Value v of a lane is row lane % 32 and token 8 (v / 4) + 4 half + v % 4: added in the parts'
+    // order, then exchanged with the neighbour, so that a lane has two rows of a token
+    float t[16];
 #pragma unroll
-  for (int i = 0; i < 2; i++)
+    for (int v = 0; v < 16; v++) t[v] = acc[n >> 1][n & 1][v];
+    if constexpr (kKP > 1) {
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+      for (int v = 0; v < 4; v++) {
+        float s[4] = {t[4 * v], t[4 * v + 1], t[4 * v + 2], t[4 * v + 3]};
 #pragma unroll
-      for (int v = 0; v < 16; v++) {
-        const int token = i * 32 + 8 * (v >> 2) + 4 * l.half + (v & 3);
-        mine[token * kRows + j * 32 + (l.lane & 31)] = acc[i][j][v];
+        for (int part = 0; part < kKP; part++) {
+          if (part == k) {
+#pragma unroll
+            for (int m = 0; m < 4; m++) s[m] = part ? s[m] + t[4 * v + m] : t[4 * v + m];
+          } else {
+            const float4 q = place(k, part, n % kFinish)[v * 64];
+            s[0] = part ? s[0] + q.x : q.x;
+            s[1] = part ? s[1] + q.y : q.y;
+            s[2] = part ? s[2] + q.z : q.z;
+            s[3] = part ? s[3] + q.w : q.w;
+          }
+        }
+#pragma unroll
+        for (int m = 0; m < 4; m++) t[4 * v + m] = s[m];
       }
-  __syncthreads();
+    }
+    const int row = l.block * kRows + 32 * (n & 1) + (l.lane & 30);
+    const int token = 32 * (n >> 1) + 4 * l.half + (l.lane & 1);
+    const uint32_t y_at = row < a.height ? static_cast<uint32_t>(row * 2) + token * y_step : kOutside;
+    const uint32_t y_at1 = row + 1 < a.height ? y_at + 2 : kOutside;   // !kPairs
+    uint32_t before[8];
 #pragma unroll
-  for (int k = 0; k < kPer; k++) {
-    const int t = wave + k * waves;
-    const int at = t * kRows + l.lane;
-    float sum = partial[at];
-    for (int v = 1; v < waves; v++) sum += partial[v * (kTokens * kRows) + at];
-    __builtin_amdgcn_raw_buffer_store_b16(
-        f32_to_bf16(bf16_to_f32(before[k]) + bf16_to_f32(f32_to_bf16(sum))), yb, y_at + t * y_step, 0,
-        0);
+    for (int m = 0; m < 8; m++) before[m] = 0u;   // a y that holds nothing yet
+    if (!a.fresh)
+#pragma unroll
+      for (int m = 0; m < 8; m++) {
+        const uint32_t at = (8 * (m >> 1) + 2 * (m & 1)) * y_step;
+        before[m] = kPairs ? __builtin_amdgcn_raw_buffer_load_b32(yb, y_at + at, 0, 0)
+                            : static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b16(yb, y_at + at, 0, 0)) |
+                                  static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b16(yb, y_at1 + at, 0, 0)) << 16;
+      }
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+      const float mine = odd ? t[2 * m + 1] : t[2 * m], other = odd ? t[2 * m] : t[2 * m + 1];
+      const float theirs = neighbour(other);
+      const bf16x2 sum = {static_cast<__bf16>(odd ? theirs : mine), static_cast<__bf16>(odd ? mine : theirs)};
+      const uint32_t bits = __builtin_bit_cast(uint32_t, sum);
+      // y += bf16(sum) in bf16
+      const bf16x2 out = {static_cast<__bf16>(__uint_as_float(before[m] << 16) + __uint_as_float(bits << 16)),
+                          static_cast<__bf16>(__uint_as_float(before[m] & 0xffff0000u) + __uint_as_float(bits & 0xffff0000u))};
+      const uint32_t now = __builtin_bit_cast(uint32_t, out);
+      const uint32_t at = (8 * (m >> 1) + 2 * (m & 1)) * y_step;
+      if (kPairs) {
+        __builtin_amdgcn_raw_buffer_store_b32(now, yb, y_at + at, 0, 0);
+      } else {
+        __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(now), yb, y_at + at, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(now >> 16), yb, y_at1 + at, 0, 0);
+      }
+    }
   }
 }
 
@@ -522,6 +526,11 @@ __device__ __forceinline__ Fetch fetch_of(const TileArgs &a, int lane) {
 }
 
 typedef __attribute__((address_space(3))) unsigned char *lds_bytes;
+
+// 16 bytes a lane straight into LDS.  (No template: on the host's side the size would not pass in one.)
+__device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t from, lds_bytes to, uint32_t at, uint32_t more) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(from, to, 16, at, more, 0, 0);
+}
 
 // Window w on its way: the activations into the tile at `tile`, the codes into
 // the block at `block`.  Pieces from the width on are not fetched (`edge`: this
@@ -667,23 +676,23 @@ void matvec_tiles_kernel(TileArgs a) {
       cur = next;
     }
   }
-  // nothing is on its way into LDS any more; then the partial tiles take the
-  // place of the activations
+  // nothing is on its way into LDS any more
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  finish_tile<kTokens / kWaves>(a, l, wave, kWaves, reinterpret_cast<float *>(tiles), acc);
+  finish_tiles<true, 1, kWaves, 2>(a, l, 0, wave, true, (l.rows_here + 31) / 32, tiles, acc);
 }
 
-// ---- the same alignment, y rows 4-byte aligned, an even height ---------------
+// ---- wavefronts that share what they fetch ------------------------------------
 //
-// Workgroups of four wavefronts that share what they fetch.  The wavefronts
-// form kKP parts of the windows (part k takes windows k, k + kKP, ...: the sums
-// and their order are those of matvec_tiles_kernel<kKP>) times kRG groups of 64
-// rows; a workgroup owns 64 kRG rows and 32 kNB tokens.  The kRG wavefronts of
-// a part bring each window of activations into LDS together, once, and every
-// one of them multiplies its own rows with it: a window's activations cross the
-// L1 once per 64 kRG rows instead of once per 64, and with kNB = 4 a B operand
-// serves 128 tokens.  The codes go straight into registers.
+// The four or eight wavefronts of a workgroup form kKP parts of the windows
+// (part k takes windows k, k + kKP, ...: the sums and their order are those of
+// matvec_tiles_kernel<kKP>) times kRG groups of 64 rows; a workgroup owns
+// 64 kRG rows and 32 kNB tokens.  The kRG wavefronts of a part bring each
+// window of activations into LDS together, once, and every one of them
+// multiplies its own rows with it: a window's activations cross the L1 once per
+// 64 kRG rows instead of once per 64, and with kNB = 4 a B operand serves 128
+// tokens.  The codes go straight into registers.  Eight wavefronts put two on
+// a SIMD at the LDS of four: c-2048 wo on 64 tokens 22.5 us instead of 26,
+// large wi on 568 11.1 instead of 13.6, both with the end below.
 //
 // The steps of 16 columns form one pipeline across the windows: while the
 // MFMAs of a step run, the B operands of the next step are built and its A
@@ -767,13 +776,62 @@ __device__ __forceinline__ void tile_step(StepOperands<kLive> &now, uint32_t nex
   now = next;
 }
 
-template <int kRG, int kKP, int kNB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kNB == 2 || kRG == 4 ? 2 : 1, 4)))
+// A wavefront's share of a window of activations on its way through registers: kLoads pieces
+// of eight columns a lane.  `left`: columns of the rows from the window on.  A piece that would reach
+// past them (in the last window) is taken from eight columns before the end, and shifted; rows of
+// fewer than eight columns, whose matrix is in one part (kNarrow), are read one by one.
+template <int kLoads>
+struct Pieces {
+  u32x4 v[kLoads];
+  static __device__ __forceinline__ int past(int col, int left) { return max(col - (left - 8), 0); }
+  template <bool kNarrow>
+  __device__ __forceinline__ void load(const uint16_t *x, const uint32_t (&at)[kLoads], const int (&col)[4], int left,
+                                       bool wide) {
+    if (kNarrow && !wide) {
+#pragma unroll
+      for (int u = 0; u < kLoads; u++) {
+        uint32_t e[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) e[q] = col[u & 3] + q < left ? x[at[u] + q] : 0u;
+        v[u] = u32x4{e[0] | e[1] << 16, e[2] | e[3] << 16, e[4] | e[5] << 16, e[6] | e[7] << 16};
+      }
+    } else if (left < kCols) {
+#pragma unroll
+      for (int u = 0; u < kLoads; u++)
+        __builtin_memcpy(&v[u], x + static_cast<int>(at[u]) - past(col[u & 3], left), 16);
+    } else {
+#pragma unroll
+      for (int u = 0; u < kLoads; u++) __builtin_memcpy(&v[u], x + at[u], 16);
+    }
+  }
+  __device__ __forceinline__ void store(unsigned char *to, const int (&col)[4], int left, bool wide) {
+#pragma unroll
+    for (int u = 0; u < kLoads; u++) {
+      u32x4 w = v[u];
+      if (left < kCols && wide) {
+        const int d = past(col[u & 3], left);
+        if (d & 4) w = u32x4{w[2], w[3], 0u, 0u};
+        if (d & 2) w = u32x4{w[1], w[2], w[3], 0u};
+        if (d & 1) w = u32x4{w[0] >> 16 | w[1] << 16, w[1] >> 16 | w[2] << 16, w[2] >> 16 | w[3] << 16, w[3] >> 16};
+        if (d >= 8) w = u32x4{0u, 0u, 0u, 0u};
+      }
+      *reinterpret_cast<u32x4 *>(to + u * 1024) = w;
+    }
+  }
+};
+
+// kDirect (x rows 16-byte aligned, the width a multiple of 8, y in pairs of rows): the activations
+// go straight into LDS.  Others come through registers, 16 bytes of any alignment a lane: the loads of
+// the window after the next are issued as a window begins, and written to LDS behind the barrier
+// that frees its tile.
+template <bool kDirect, int kRG, int kKP, int kNB>
+__global__ __launch_bounds__(64 * kRG * kKP)
+__attribute__((amdgpu_waves_per_eu(kRG * kKP == 8 || kNB == 2 || kRG == 4 ? 2 : 1, 4)))
 void matvec_tiles_shared_kernel(TileArgs a) {
-  static_assert(kRG * kKP == 4 && (kNB == 2 || kNB == 4), "four wavefronts");
+  static_assert((kRG * kKP == 4 || kRG * kKP == 8) && (kNB == 2 || kNB == 4), "four or eight wavefronts");
   constexpr int kTile = kNB * 32 * 256;        // a window of activations
   constexpr int kLoads = 8 * kNB / kRG;        // of them this wavefront's loads
-  static_assert(kLoads % 4 == 0, "whole groups of sixteen tokens per wavefront");
+  static_assert(kLoads >= 2, "a load is four tokens");
   extern __shared__ __align__(16384) unsigned char shared_tiles[];   // [part][2][kTile]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = wave % kRG, k = wave / kRG;
@@ -794,13 +852,22 @@ void matvec_tiles_shared_kernel(TileArgs a) {
     l.unit_at[j] = static_cast<uint32_t>(j * a.windows * 1024 + l.lane * 16);
   }
   l.get_at = static_cast<uint32_t>((l.lane & 31) * 256 + ((l.half ^ (l.lane & 15)) << 4));
-  Fetch f = fetch_of(a, l.lane);
+  // Load u of this wavefront brings tokens 4 (g kLoads + u) + lane / 16 of the block, the lane the
+  // eight columns from piece_col[u % 4] on: those that belong at its place in LDS.
+  int piece_col[4];
+  uint32_t piece_at[kLoads];   // kDirect: in bytes; else in elements, of the last token at most
 #pragma unroll
-  for (int u = 0; u < 4; u++) f.at[u] += static_cast<uint32_t>(g * (kLoads / 4)) * f.step;
+  for (int u = 0; u < 4; u++) piece_col[u] = 8 * ((l.lane & 15) ^ ((4 * (g * kLoads + u) + (l.lane >> 4)) & 15));
+#pragma unroll
+  for (int u = 0; u < kLoads; u++) {
+    const int token = 4 * (g * kLoads + u) + (l.lane >> 4);
+    piece_at[u] = kDirect ? static_cast<uint32_t>((token * a.ldx + piece_col[u & 3]) * 2)
+                          : static_cast<uint32_t>(min(token, l.rows_here - 1) * a.ldx + piece_col[u & 3]);
+  }
   const lds_bytes part_tiles = (lds_bytes)shared_tiles + k * (2 * kTile);
   const int last = a.windows - 1;
   const bool ragged_edge = (a.width & (kCols - 1)) != 0;
-  if (ragged_edge) {
+  if (kDirect && ragged_edge) {
     // places that no fetch writes must not hold what LDS happened to hold
     const u32x4 zero = {0u, 0u, 0u, 0u};
 #pragma unroll
@@ -822,10 +889,21 @@ void matvec_tiles_shared_kernel(TileArgs a) {
   // activations, into tile `buffer` of its part; and its own codes of window w.
   auto issue_x = [&](const __amdgpu_buffer_rsrc_t &xb, int w, int buffer, int u) {
     const bool edge = ragged_edge && w == last;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        xb, part_tiles + buffer * kTile + g * (kLoads * 1024) + u * 1024, 16,
-        edge && f.col[u & 3] >= a.width - w * kCols ? kOutside : f.at[u & 3] + (u >> 2) * f.step,
-        w * (kCols * 2), 0, 0);
+    load_to_lds(xb, part_tiles + buffer * kTile + g * (kLoads * 1024) + u * 1024,
+                edge && piece_col[u & 3] >= a.width - w * kCols ? kOutside : piece_at[u], w * (kCols * 2));
+  };
+  Pieces<kDirect ? 1 : kLoads> pieces;
+  auto load_pieces = [&](int w, auto may_be_narrow) {   // (narrow rows are one window)
+    if constexpr (!kDirect)
+      if (w < a.windows)
+        pieces.template load<decltype(may_be_narrow)::value>(a.x + static_cast<int64_t>(l.t0) * a.ldx + w * kCols, piece_at, piece_col,
+                                       a.width - w * kCols, a.width >= 8);
+  };
+  auto store_pieces = [&](int w, int buffer) {
+    if constexpr (!kDirect)
+      if (w < a.windows)
+        pieces.store(shared_tiles + k * (2 * kTile) + buffer * kTile + g * (kLoads * 1024) + l.lane * 16, piece_col,
+                     a.width - w * kCols, a.width >= 8);
   };
   auto issue_codes = [&](int w, u32x4 (&codes)[2]) {
     const __amdgpu_buffer_rsrc_t ub =
@@ -844,12 +922,20 @@ void matvec_tiles_shared_kernel(TileArgs a) {
   {
     const __amdgpu_buffer_rsrc_t x0 = tokens_of(a, l, k < a.windows);
     const __amdgpu_buffer_rsrc_t x1 = tokens_of(a, l, k + kKP < a.windows);
+    if constexpr (kDirect) {
 #pragma unroll
-    for (int u = 0; u < kLoads; u++) issue_x(x0, k, 0, u);
+      for (int u = 0; u < kLoads; u++) issue_x(x0, k, 0, u);
+    }
+    load_pieces(k, std::bool_constant<kKP == 1>{});
     issue_codes(k, codes_a);
+    store_pieces(k, 0);
+    if constexpr (kDirect) {
 #pragma unroll
-    for (int u = 0; u < kLoads; u++) issue_x(x1, k + kKP, 1, u);
+      for (int u = 0; u < kLoads; u++) issue_x(x1, k + kKP, 1, u);
+    }
+    load_pieces(k + kKP, std::false_type{});
     issue_codes(k + kKP, codes_b);
+    store_pieces(k + kKP, 1);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -872,6 +958,7 @@ void matvec_tiles_shared_kernel(TileArgs a) {
       const int w = __builtin_amdgcn_readfirstlane(k + turn * kKP);
       const int w2 = w + 2 * kKP;
       const __amdgpu_buffer_rsrc_t x2 = tokens_of(a, l, w2 < a.windows);
+      load_pieces(w2, std::false_type{});
       if (has_rows && w < a.windows) {
         const uint32_t get = tile_at[cur];
         tile_step<kLive, kNB, 1>(now, get ^ 32u, codes_cur[0][0], codes_cur[1][0], l.rows, acc, nothing);
@@ -887,15 +974,21 @@ void matvec_tiles_shared_kernel(TileArgs a) {
         __syncthreads();
         const uint32_t word0 = codes_nxt[0][0], word1 = codes_nxt[1][0];
         tile_step<kLive, kNB, 0>(now, tile_at[cur ^ 1], word0, word1, l.rows, acc, [&](int m) {
+          if constexpr (kDirect) {
 #pragma unroll
-          for (int u = m * kPerSlot; u < (m + 1) * kPerSlot && u < kLoads; u++) issue_x(x2, w2, cur, u);
+            for (int u = m * kPerSlot; u < (m + 1) * kPerSlot && u < kLoads; u++) issue_x(x2, w2, cur, u);
+          }
           if (m == kSlots - 1) issue_codes(w2, codes_cur);
         });
+        store_pieces(w2, cur);
       } else {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
+        if constexpr (kDirect) {
 #pragma unroll
-        for (int u = 0; u < kLoads; u++) issue_x(x2, w2, cur, u);
+          for (int u = 0; u < kLoads; u++) issue_x(x2, w2, cur, u);
+        }
+        store_pieces(w2, cur);
         issue_codes(w2, codes_cur);
       }
     };
@@ -908,146 +1001,35 @@ void matvec_tiles_shared_kernel(TileArgs a) {
     run(std::integral_constant<int, kNB>{});
   else
     run(std::integral_constant<int, kNB / 2>{});
-  // nothing is on its way into LDS any more and everyone has read its last
-  // window; then the sums take the place of the activations, 32 tokens at a time
+  // nothing is on its way into LDS any more
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  float *sums = reinterpret_cast<float *>(shared_tiles);   // [wavefront][32 tokens][64 rows]
-  const int pair = l.lane & 31;                            // rows 2 pair, 2 pair + 1 of the group
-  const int row = l.block * kRows + 2 * pair;
-  const uint32_t y_bytes =
-      static_cast<uint32_t>((static_cast<int64_t>(l.rows_here - 1) * a.ldy + a.height) * 2);
-  uint16_t *y = a.y + static_cast<int64_t>(l.t0) * a.ldy;
-  const __amdgpu_buffer_rsrc_t yb = buffer_over(y, y_bytes), was = buffer_over(y, a.fresh ? 0u : y_bytes);
-  const uint32_t y_at = has_rows && row < a.height ? static_cast<uint32_t>(row * 2) : kOutside;
-  const uint32_t y_step = static_cast<uint32_t>(a.ldy * 2);
-  constexpr int kMine = 16 / kKP;   // pairs of tokens of a block that this wavefront finishes
-#pragma unroll
-  for (int i = 0; i < kNB; i++) {
-    if (i >= live) break;
-    uint32_t before[kMine];
-#pragma unroll
-    for (int n = 0; n < kMine; n++)
-      before[n] = __builtin_amdgcn_raw_buffer_load_b32(
-          was, y_at + (32 * i + k * (32 / kKP) + 2 * n + l.half) * y_step, 0, 0);
-    // Element (token t, row r) of an accumulator block sits in lane
-    // r + 32 * ((t / 4) % 2), register 4 * (t / 8) + t % 4.
-    float *mine = sums + wave * (32 * kRows);
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int v = 0; v < 16; v++)
-        mine[(8 * (v >> 2) + 4 * l.half + (v & 3)) * kRows + j * 32 + (l.lane & 31)] = acc[i][j][v];
-    if (kKP > 1) __syncthreads();
-#pragma unroll
-    for (int n = 0; n < kMine; n++) {
-      const int t = k * (32 / kKP) + 2 * n + l.half;
-      const float *at = sums + g * (32 * kRows) + t * kRows + 2 * pair;
-      float lo = at[0], hi = at[1];
-#pragma unroll
-      for (int part = 1; part < kKP; part++) {
-        lo += at[part * kRG * (32 * kRows)];
-        hi += at[part * kRG * (32 * kRows) + 1];
-      }
-      const uint32_t now =
-          static_cast<uint32_t>(f32_to_bf16(bf16_to_f32(static_cast<uint16_t>(before[n] & 0xffffu)) +
-                                            bf16_to_f32(f32_to_bf16(lo)))) |
-          static_cast<uint32_t>(f32_to_bf16(bf16_to_f32(static_cast<uint16_t>(before[n] >> 16)) +
-                                            bf16_to_f32(f32_to_bf16(hi)))) << 16;
-      __builtin_amdgcn_raw_buffer_store_b32(now, yb, y_at + (32 * i + t) * y_step, 0, 0);
-    }
-    if (kKP > 1) __syncthreads();
-  }
+  finish_tiles<kDirect, kRG, kKP, kNB>(a, l, g, k, has_rows, live, shared_tiles, acc);
 }
 
-// ---- any x ------------------------------------------------------------------
-//
-// The same, the activations read element by element into registers and stored
-// into LDS from there (one tile per wavefront, the next window's loads issued
-// as soon as the registers are free): for x rows that are not 16-byte aligned
-// or a width that is not a multiple of 8.  The same sums in the same order.
-
-// Eight activations of one token from byte offset `at` of the buffer on, of
-// which the first `inside` lie inside the width (0 or less: none).
-__device__ __forceinline__ u32x4 load_piece(__amdgpu_buffer_rsrc_t x, uint32_t at, int inside) {
-  uint32_t e[8];
-#pragma unroll
-  for (int q = 0; q < 8; q++)
-    e[q] = __builtin_amdgcn_raw_buffer_load_b16(x, (q < inside ? at : kOutside) + 2 * q, 0, 0);
-  u32x4 v = {e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
-  return v;
-}
-
-template <int kWaves>
-__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void matvec_tiles_ragged_kernel(TileArgs a) {
-  __shared__ u32x4 tile[kWaves * 1024];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const TileLane l = tile_lane(a);
-  const __amdgpu_buffer_rsrc_t xb = tokens_of(a, l), ub = units_of(a, l.block);
-  const Fetch f = fetch_of(a, l.lane);
-  u32x4 *mine = tile + wave * 1024;
-
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; i++)
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
-
-  for (int w = wave; w < a.windows; w += kWaves) {
-    u32x4 codes[2];
-#pragma unroll
-    for (int j = 0; j < 2; j++) codes[j] = __builtin_amdgcn_raw_buffer_load_b128(ub, l.unit_at[j], w * 1024, 0);
-#pragma unroll
-    for (int u = 0; u < 16; u++)
-      mine[u * 64 + l.lane] = load_piece(xb, f.at[u & 3] + (u >> 2) * f.step + w * (kCols * 2),
-                                         a.width - w * kCols - f.col[u & 3]);
-    window_steps(reinterpret_cast<const unsigned char *>(mine), l, codes, acc);
-  }
-  __syncthreads();
-  finish_tile<kTokens / kWaves>(a, l, wave, kWaves, reinterpret_cast<float *>(tile), acc);
-}
-
-// Estimated microseconds of a launch on `tiles` blocks of 64 tokens, for a
-// matrix of `blocks` blocks of 64 rows and `windows` windows cut into n parts
-// (fitted to measurements on the six Switch shapes at 64 to 2272 tokens).
-// matvec_tiles_kernel<n>: rounds of workgroups over the chip, four wavefronts a
-// compute unit (36 KB of LDS each), each round 4 us plus 1.25 us per window that
-// a wavefront walks.
-double cost_own_tiles(int blocks, int windows, int n, int64_t tiles) {
-  const int64_t slots = 256 * (kMaxWaves / n);
-  const int64_t rounds = (blocks * tiles + slots - 1) / slots;
-  return rounds * (4.0 + 1.25 * ((windows + n - 1) / n));
-}
-// matvec_tiles_shared_kernel<4 / n, n, 2>: 1.35 us per window of a part; a
-// compute unit holds three such workgroups with one part and two with two, and
-// each one beyond the first slows the others by 0.6 of its time; more
-// workgroups than that follow as the first ones end.
-double cost_shared_tiles(int blocks, int windows, int n, int64_t tiles) {
-  const int groups = kMaxWaves / n, cap = n == 1 ? 3 : 2;
-  const int64_t workgroups = (blocks + groups - 1) / groups * tiles;
-  const int64_t per_unit = std::min<int64_t>(cap, (workgroups + 255) / 256);
-  const double fill = static_cast<double>(workgroups) / (256.0 * cap);
-  const double rounds = fill <= 1.0 ? 1.0 : 0.5 * (std::ceil(fill) + fill);
-  return rounds * (4.0 + 1.35 * ((windows + n - 1) / n) * (1.0 + 0.6 * (per_unit - 1)));
-}
-
-// Parts that the windows of a matrix are cut into: 1, 2 or 4, whichever is
-// estimated fastest at nine blocks of tokens (568, the longest sequence of the
-// Switch encoders) by the better of the two kernels.  The choice depends on
+// Parts that the windows of a matrix are cut into: 1, 2 or 4.  The choice depends on
 // the matrix alone, never on the tokens of a launch, and the parts are added in
-// the same order by both kernels: a token's result is the same whatever launch
-// it is part of.
-std::atomic<int> g_forced_kernel{0};   // sub1_test_tiles_kernel
-
-int pick_waves(int blocks, int windows) {
+// the same order by all kernels: a token's result is the same whatever launch
+// it is part of.  By estimates at nine blocks of 64 tokens (568, the longest sequence of the
+// Switch encoders) for matvec_tiles_kernel<n>, in rounds of workgroups, and for workgroups
+// of four wavefronts that share their activations.  (They price the kernels as those were first built.
+// The estimates below would cut a seventh of all matrices finer: faster on short sequences, slower
+// on long ones.  c-2048 wo in four parts: 14.5 us instead of 22.6 on 64 tokens, 43.4 and 41.7
+// on 1136, 55.7 and 47.3 on 1900.)
+int parts_of(int blocks, int windows) {
   int best = 1;
   double best_cost = 0;
   for (int n = 1; n <= kMaxWaves; n *= 2) {
-    double cost = cost_own_tiles(blocks, windows, n, 9);
-    if (n <= 2) cost = std::min(cost, cost_shared_tiles(blocks, windows, n, 9));
+    const int turns = (windows + n - 1) / n;
+    const int64_t slots = 256 * (kMaxWaves / n), tiles = 9;
+    double cost = static_cast<double>((blocks * tiles + slots - 1) / slots) * (4.0 + 1.25 * turns);
+    if (n <= 2) {
+      const int groups = kMaxWaves / n, cap = n == 1 ? 3 : 2;
+      const int64_t workgroups = (blocks + groups - 1) / groups * tiles;
+      const int64_t per_unit = std::min<int64_t>(cap, (workgroups + 255) / 256);
+      const double fill = static_cast<double>(workgroups) / (256.0 * cap);
+      const double rounds = fill <= 1.0 ? 1.0 : 0.5 * (std::ceil(fill) + fill);
+      cost = std::min(cost, rounds * (4.0 + 1.35 * turns * (1.0 + 0.6 * (per_unit - 1))));
+    }
     if (n == 1 || cost < best_cost - 1e-9) {
       best = n;
       best_cost = cost;
@@ -1056,33 +1038,90 @@ int pick_waves(int blocks, int windows) {
   return best;
 }
 
-template <int kRG, int kKP, int kNB>
+// The forms a launch of a matrix in `parts` parts may take: workgroups of `groups` groups of
+// 64 rows (0: one wavefront's own tiles, matvec_tiles_kernel) and 32 `blocks` tokens, `held` of
+// which a compute unit holds at once.  One of them takes start + turn us a window of its part; each
+// further one on the unit makes `beside` of the windows' time more.  Fitted to 14 shapes, the
+// six of Switch among them, on 64 to 2272 tokens (rms 4 to 15 %, the larger ones where 10 us of host
+// calls hide the kernel); the form estimated fastest is within 2 % of the fastest on average.
+struct TileForm {
+  int parts, groups, blocks, held;
+  double start, turn, beside;
+};
+constexpr TileForm kTileForms[] = {
+    {1, 0, 2, 4, 4.4, 0.77, 0.09}, {1, 4, 2, 3, 4.2, 0.92, 0.80}, {1, 4, 4, 2, 5.9, 1.37, 1.00},
+    {2, 0, 2, 2, 3.2, 0.86, 0.25}, {2, 2, 2, 2, 3.2, 1.16, 0.57}, {2, 4, 2, 2, 5.3, 1.40, 1.60},
+    {2, 4, 4, 1, 7.3, 2.20, 0.0},  {4, 0, 2, 1, 2.8, 1.17, 0.0},  {4, 2, 2, 1, 3.7, 1.92, 0.0}};
+double cost_of(const TileForm &f, int row_blocks, int windows, int tokens) {
+  const int groups = std::max(f.groups, 1), turns = (windows + f.parts - 1) / f.parts;
+  const int64_t workgroups = static_cast<int64_t>((row_blocks + groups - 1) / groups) *
+                             ((tokens + 32 * f.blocks - 1) / (32 * f.blocks));
+  auto with = [&](int64_t on_a_unit) { return f.start + f.turn * turns * (1.0 + f.beside * (on_a_unit - 1)); };
+  const int64_t rounds = workgroups / (256 * f.held), rest = workgroups % (256 * f.held);
+  return rounds * with(f.held) + (rest ? with((rest + 255) / 256) : 0.0);
+}
+// `direct`: x and y as the forms on the activations' straight way into LDS need them.  Blocks of
+// 128 tokens have to promise a fifth where there are two parts, and are taken where there is
+// one if blocks of 64 would make more workgroups than the chip holds at once: the fit is coarse
+// there (c-2048 wi on 1136 tokens 33.0 us, in blocks of 64 38.0; large wi 16.8 and 17.8).
+const TileForm &pick_form(int parts, int row_blocks, int windows, int tokens, bool direct) {
+  const TileForm *best = nullptr;
+  double best_cost = 0;
+  const bool wide_of_one = (row_blocks + 3) / 4 * static_cast<int64_t>((tokens + 63) / 64) > 3 * 256;
+  for (const TileForm &f : kTileForms) {
+    if (f.parts != parts || (!direct && (f.groups == 0 || f.blocks == 4))) continue;
+    if (direct && parts == 1 && f.groups && (f.blocks == 4) != wide_of_one) continue;
+    const double cost = cost_of(f, row_blocks, windows, tokens) / (parts == 2 && f.blocks == 4 ? 0.8 : 1.0);
+    if (!best || cost < best_cost) {
+      best = &f;
+      best_cost = cost;
+    }
+  }
+  return *best;
+}
+
+std::atomic<int> g_forced_kernel{0};   // sub1_test_tiles_kernel
+
+template <bool kDirect, int kRG, int kKP, int kNB>
 int launch_shared_as(const TileArgs &a, int blocks, hipStream_t stream) {
+  constexpr int waves = kRG * kKP;
   constexpr int lds = kKP * 2 * kNB * 32 * 256;
-  static_assert(lds >= 4 * 32 * kRows * 4 && lds <= 160 * 1024, "tiles, then the sums of four wavefronts");
-  HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(matvec_tiles_shared_kernel<kRG, kKP, kNB>),
+  static_assert(lds >= waves * (kKP - 1) * (2 * kNB / kKP) * 4096 && lds <= 160 * 1024, "tiles, then sums");
+  HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(matvec_tiles_shared_kernel<kDirect, kRG, kKP, kNB>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, lds));
   const dim3 grid((blocks + kRG - 1) / kRG, (a.tokens + 32 * kNB - 1) / (32 * kNB));
-  matvec_tiles_shared_kernel<kRG, kKP, kNB><<<grid, 256, lds, stream>>>(a);
+  matvec_tiles_shared_kernel<kDirect, kRG, kKP, kNB><<<grid, 64 * waves, lds, stream>>>(a);
   HIP_TRY(hipGetLastError());
   return SUB1_OK;
 }
 
-int launch_shared(const TileArgs &a, int parts, int token_blocks, int blocks, hipStream_t stream) {
-  sub1::note_kernel(token_blocks == 4 ? "matvec_tiles_shared_kernel<128>" : "matvec_tiles_shared_kernel<64>");
-  if (parts == 1) return token_blocks == 4 ? launch_shared_as<4, 1, 4>(a, blocks, stream)
-                                           : launch_shared_as<4, 1, 2>(a, blocks, stream);
-  if (parts == 2) return token_blocks == 4 ? launch_shared_as<2, 2, 4>(a, blocks, stream)
-                                           : launch_shared_as<2, 2, 2>(a, blocks, stream);
-  return launch_shared_as<1, 4, 2>(a, blocks, stream);
+template <int kWaves>
+int launch_own(const TileArgs &a, int blocks, hipStream_t stream) {
+  matvec_tiles_kernel<kWaves><<<dim3(blocks, (a.tokens + kTokens - 1) / kTokens), 64 * kWaves, 0, stream>>>(a);
+  HIP_TRY(hipGetLastError());
+  return SUB1_OK;
 }
 
-template <int kWaves>
-void launch_tiles(const TileArgs &a, bool wide, dim3 grid, hipStream_t stream) {
-  if (wide)
-    matvec_tiles_kernel<kWaves><<<grid, 64 * kWaves, 0, stream>>>(a);
-  else
-    matvec_tiles_ragged_kernel<kWaves><<<grid, 64 * kWaves, 0, stream>>>(a);
+int launch_form(const TileArgs &a, const TileForm &f, bool direct, int blocks, hipStream_t s) {
+  sub1::note_kernel(f.groups == 0   ? "matvec_tiles_kernel"
+                    : f.blocks == 4 ? "matvec_tiles_shared_kernel<128>"
+                                    : "matvec_tiles_shared_kernel<64>");
+  if (f.groups == 0) {
+    if (f.parts == 1) return launch_own<1>(a, blocks, s);
+    if (f.parts == 2) return launch_own<2>(a, blocks, s);
+    return launch_own<4>(a, blocks, s);
+  }
+  if (f.parts == 1) {
+    if (!direct) return launch_shared_as<false, 4, 1, 2>(a, blocks, s);
+    return f.blocks == 4 ? launch_shared_as<true, 4, 1, 4>(a, blocks, s) : launch_shared_as<true, 4, 1, 2>(a, blocks, s);
+  }
+  if (f.parts == 2 && f.groups == 2)
+    return direct ? launch_shared_as<true, 2, 2, 2>(a, blocks, s) : launch_shared_as<false, 2, 2, 2>(a, blocks, s);
+  if (f.parts == 2) {
+    if (!direct) return launch_shared_as<false, 4, 2, 2>(a, blocks, s);
+    return f.blocks == 4 ? launch_shared_as<true, 4, 2, 4>(a, blocks, s) : launch_shared_as<true, 4, 2, 2>(a, blocks, s);
+  }
+  return direct ? launch_shared_as<true, 2, 4, 2>(a, blocks, s) : launch_shared_as<false, 2, 4, 2>(a, blocks, s);
 }
 
 int check_set(const sub1_matrix_set *ms, const char *who) {
@@ -1222,33 +1261,23 @@ int launch_product(const sub1_tiles *t, int matrix, const void *x, int64_t ldx, 
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (ldx >= (1 << 24) || ldy >= (1 << 24))
     return fail(SUB1_ERR_SHAPE, "%s: token strides of 2^24 elements or more", who);
-  const int waves = pick_waves(l.units_down / 2, l.windows);
-  const bool shared_ok = wide && !misaligned(y, 4) && ldy % 2 == 0 && t->height % 2 == 0 &&
-                         ldx < (1 << 22) && ldy < (1 << 22);
-  // Which kernel: the one estimated faster for this many tokens (the sums and
-  // their order are the same).  Workgroups that share their activations take
-  // over where those of one wavefront's own tiles no longer fit the chip at
-  // once (20 to 35% less time on the Switch shapes from there on); with four
-  // parts they are no faster and are not used.  Blocks of 128 tokens where
-  // blocks of 64 would make more such workgroups than the chip holds at once.
-  const int blocks = l.units_down / 2;
-  const int64_t tiles_of_64 = (tokens + kTokens - 1) / kTokens;
+  // Rows of x that are 16-byte aligned and y in pairs of rows: straight into LDS, or through
+  // registers (5003 x 1501 on 64, 568 and 2272 tokens 13.5, 17.7 and 50 us; element by element,
+  // a wavefront with tiles of its own, 31, 72 and 263).
+  const bool direct = wide && !misaligned(y, 4) && ldy % 2 == 0 && t->height % 2 == 0;
+  const int blocks = l.units_down / 2, parts = parts_of(blocks, l.windows);
+  const TileForm *form = &pick_form(parts, blocks, l.windows, tokens, direct);
   const int forced = g_forced_kernel.load(std::memory_order_relaxed);
-  if (shared_ok && forced >= 2) return launch_shared(a, waves, forced == 3 && waves < 4 ? 4 : 2, blocks, s);
-  if (shared_ok && !forced && waves <= 2 &&
-      cost_shared_tiles(blocks, l.windows, waves, tiles_of_64) <
-          cost_own_tiles(blocks, l.windows, waves, tiles_of_64)) {
-    const int groups = kMaxWaves / waves;
-    const bool wide_blocks = waves == 1 && (blocks + groups - 1) / groups * tiles_of_64 > 3 * 256;
-    return launch_shared(a, waves, wide_blocks ? 4 : 2, blocks, s);
-  }
-  const dim3 grid(l.units_down / 2, (tokens + kTokens - 1) / kTokens);
-  sub1::note_kernel(wide ? "matvec_tiles_kernel" : "matvec_tiles_ragged_kernel");
-  if (waves == 1) launch_tiles<1>(a, wide, grid, s);
-  else if (waves == 2) launch_tiles<2>(a, wide, grid, s);
-  else launch_tiles<4>(a, wide, grid, s);
-  HIP_TRY(hipGetLastError());
-  return SUB1_OK;
+  // (a block's rows of x and y are addressed in 32 bits: 128 of them up to these strides)
+  const bool far = ldx >= (1 << 22) || ldy >= (1 << 22);
+  if ((forced && direct) || (far && form->blocks == 4))
+    for (const TileForm &f : kTileForms)
+      if (f.parts == parts && (forced == 1) == (f.groups == 0) &&
+          (f.blocks == 4) == (forced == 3 && parts < 4 && !far)) {
+        form = &f;
+        break;
+      }
+  return launch_form(a, *form, direct, blocks, s);
 }
 
 }  // namespace

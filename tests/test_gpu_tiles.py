@@ -180,6 +180,47 @@ def test_both_tile_kernels_give_the_same_bits_on_any_shape(gpu, oracle):
     assert lib.sub1_test_tiles_kernel(4) != 0
 
 
+@pytest.mark.parametrize('height,width,tokens', [
+    (65, 1, 64), (3, 7, 130), (64, 8, 65), (129, 9, 70), (31, 127, 64), (130, 128, 97),        # a window and less
+    (77, 129, 66), (200, 130, 129), (96, 135, 64), (515, 263, 191),                             # and a little more
+    (1001, 1501, 100), (331, 5003, 75), (640, 5600, 90), (2311, 777, 68)])                      # one, two and four parts
+def test_rows_of_any_alignment(gpu, oracle, height, width, tokens):
+    """Activations that come through registers: every token against the double-precision
+    product, the same bits for x and y that begin anywhere, with rows further apart than they
+    are long, and (where the width allows it) as the launch that loads straight into LDS; the
+    memory around them is neither used (it holds infinities) nor written.  Results below the
+    smallest normal number keep their bits too."""
+    import ctypes
+    sub1, op = gpu
+    from qmoe_amd import _lib
+    lib, stream = _lib.load(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    c = dev_case(oracle, height, width, 0.85, seed=31 * height + width)
+    tm = op.TiledMatrix(sub1.DEC[0], c['w_comp'], c['row_off_d'], c['mm_d'], width)
+    rng = np.random.default_rng(width)
+    x = rng.standard_normal((tokens, width)).astype(np.float32)
+    x[tokens - 1] *= 1e-38
+    xs = so.f32_to_bf16_bits(x)
+    pre = so.f32_to_bf16_bits(rng.standard_normal((tokens, height)).astype(np.float32))
+    pre[tokens - 1] = 0
+    outs = []
+    for ldx, ldy, at_x, at_y in ((width, height, 0, 0), (width + 3, height + 5, 1, 1), (width + 8, height + 1, 5, 2),
+                                 ((width + 7) // 8 * 8, (height + 1) // 2 * 2, 0, 0)):
+        xd = torch.full((at_x + tokens * ldx + 64,), float('inf'), dtype=torch.bfloat16, device='cuda')
+        rows = xd[at_x:at_x + tokens * ldx].view(tokens, ldx)
+        rows[:, :width] = bf16_dev(xs)
+        y = torch.full((at_y + tokens * ldy + 64,), 7.0, dtype=torch.bfloat16, device='cuda')
+        y_rows = y[at_y:at_y + tokens * ldy].view(tokens, ldy)
+        y_rows[:, :height] = bf16_dev(pre)
+        _lib.check(lib.sub1_matvec_tiles(ctypes.byref(tm._c), 0, rows.data_ptr(), ldx, y_rows.data_ptr(), ldy, tokens,
+                                         stream))
+        assert bool((y[:at_y] == 7).all()) and bool((y[at_y + tokens * ldy:] == 7).all())
+        assert bool((y_rows[:, height:] == 7).all())
+        outs.append(y_rows[:, :height].clone())
+    check_all_tokens(oracle, c, xs[:-1], pre[:-1], bits_host(outs[0][:-1].contiguous()))
+    for other in outs[1:]:
+        assert torch.equal(outs[0].view(torch.int16), other.view(torch.int16))
+
+
 def test_tiles_closed_forms(gpu, oracle):
     """Unit vectors pick a column exactly; zero activations leave y as it was;
     doubling the activations doubles the product exactly (y zero before)."""
