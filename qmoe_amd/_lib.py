@@ -134,6 +134,21 @@ PROTOTYPES = {
 }
 
 _lib = None
+_tensor_args = None
+
+
+def tensor_args():
+    """The extension that looks tensors over (csrc/tensor_args.cpp).  There is no fallback either."""
+    global _tensor_args
+    if _tensor_args is None:
+        import torch  # noqa: F401  (its libraries first)
+        try:
+            from . import _tensor_args as module
+        except ImportError as e:
+            raise ImportError('qmoe_amd/_tensor_args.so is missing or of another torch: build it with '
+                              '`python -m qmoe_amd.build` (%s)' % e) from e
+        _tensor_args = module
+    return _tensor_args
 
 
 class Sub1Error(RuntimeError):

@@ -1,11 +1,14 @@
-"""Compiles libsub1_hip.so for gfx950 with hipcc (cross-compiles without a GPU)."""
+"""Compiles libsub1_hip.so for gfx950 with hipcc (cross-compiles without a GPU), and
+the Python extension that takes tensors apart for it with g++."""
 import os
 import re
 import subprocess
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB_PATH = os.path.join(HERE, 'libsub1_hip.so')
+TENSOR_ARGS_PATH = os.path.join(HERE, '_tensor_args.so')
 SOURCES = [os.path.join(HERE, 'csrc', 'sub1_kernels.hip'),
            os.path.join(HERE, 'csrc', 'sub1_pack.hip'),
            os.path.join(HERE, 'csrc', 'sub1_prepared.hip'),
@@ -41,14 +44,31 @@ def kernels_with_scratch(compiler_output):
 SPILLS_ACCEPTED = {'_ZN12_GLOBAL__N_125moe_prepared_fused_kernelILb1ELb0EEEvNS_12PreparedArgsE': 36}
 
 
+def build_tensor_args():
+    """Builds the extension module against the installed torch's headers."""
+    import torch
+    from torch.utils import cpp_extension
+    cmd = [os.environ.get('CXX', 'g++'), '-O2', '-fPIC', '-shared', '-std=c++17', '-fvisibility=hidden',
+           '-D_GLIBCXX_USE_CXX11_ABI=%d' % torch._C._GLIBCXX_USE_CXX11_ABI,
+           os.path.join(HERE, 'csrc', 'tensor_args.cpp')]
+    cmd += ['-isystem' + path for path in cpp_extension.include_paths() + [sysconfig.get_paths()['include']]]
+    cmd += ['-L' + path for path in cpp_extension.library_paths()]
+    cmd += ['-ltorch_python', '-ltorch_cpu', '-lc10', '-o', TENSOR_ARGS_PATH]
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if res.returncode != 0:
+        raise RuntimeError('g++ failed:\n' + res.stdout)
+    return TENSOR_ARGS_PATH
+
+
 def build_library(verbose=False):
-    """Builds the library; refuses a build in which a kernel spills registers
+    """Builds the library and the extension; refuses a build in which a kernel spills registers
     to scratch memory beyond what SPILLS_ACCEPTED lists.  The kernels are
     written to fit their registers (72 to 96 of the 128 that 16 wavefronts per
     compute unit leave a lane), and a spill in a walk costs more than any of
     the tunings measured; one build of the one-token launch that spilled 12
     registers also gave results that differed from run to run (cause not
     established; the code was restructured to fit)."""
+    build_tensor_args()
     hipcc = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
     cmd = [hipcc] + HIPCC_FLAGS + SOURCES + ['-o', LIB_PATH]
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)

@@ -52,9 +52,13 @@ class Sub1Linear(nn.Module):
 
     def __init__(self, height, comp_size):
         super().__init__()
-        self.register_buffer('w_comp', torch.zeros(comp_size, dtype=torch.int16))
-        self.register_buffer('row_off', torch.zeros(height + 1, dtype=torch.int32))
-        self.register_buffer('ter_minmax', torch.zeros(2 * height, dtype=torch.bfloat16))
+        self._hold(torch.zeros(comp_size, dtype=torch.int16), torch.zeros(height + 1, dtype=torch.int32),
+                   torch.zeros(2 * height, dtype=torch.bfloat16))
+
+    def _hold(self, w_comp, row_off, ter_minmax):
+        self.register_buffer('w_comp', w_comp)
+        self.register_buffer('row_off', row_off)
+        self.register_buffer('ter_minmax', ter_minmax)
         self.register_buffer('weight', torch.zeros(0, dtype=torch.bfloat16))
 
     # forward() goes through copies of the weights made from the codes on first
@@ -78,8 +82,8 @@ class Sub1Linear(nn.Module):
     tile_tokens = 64
 
     def _copy(self, kind, width):
-        live = (self.w_comp, self.row_off, self.ter_minmax)
-        key = tuple((t.data_ptr(), t._version, t.numel()) for t in live) + (width,)
+        live = _buffers_of(self)
+        key = tuple([(t.data_ptr(), t._version, t.numel()) for t in live]) + (width,)
         cache = self.__dict__.setdefault('_copies', {})
         cached = cache.get(kind)
         if cached is None or cached[0] != key:
@@ -117,9 +121,11 @@ class Sub1Linear(nn.Module):
         {row min, 0, row max} (reference sub1.py:145-166; ties go to max)."""
         if w.device.type != 'cuda' or not GPUS:
             raise RuntimeError('the compressed-expert kernels need a GPU; got %s' % w.device)
-        linear = Sub1Linear(0, 0)
-        linear.w_comp, linear.row_off, linear.ter_minmax = sub1_hip.sub1pack_weights(
-            w.bfloat16().contiguous())
+        w_comp, row_off, ter_minmax = sub1_hip.sub1pack_weights(w.bfloat16().contiguous())
+        # the module around these buffers, without empty ones first (a fifth of a call)
+        linear = Sub1Linear.__new__(Sub1Linear)
+        nn.Module.__init__(linear)
+        linear._hold(w_comp, row_off, ter_minmax)
         return linear
 
 
@@ -286,12 +292,15 @@ class FasterMLP(nn.Module):
                 raise ValueError('FasterMLP runs ReLU experts; this one has %r' % (act,))
 
     matrix_cores = True     # as Sub1Experts.matrix_cores
+    _released = False       # (defaults of the class: a Module takes a microsecond to say that it has none)
+    _launcher_cache = None
 
     def _sentinels(self):
         # a few of the experts' tensors stand for all of them in the per-call
         # check (looking at every tensor of 2048 experts costs milliseconds)
-        first, last = self.experts[0], self.experts[len(self.experts) - 1]
-        return [first.wi.w_comp, first.wi.ter_minmax, last.wo.w_comp, last.wo.ter_minmax]
+        experts = self.experts._modules     # (by name: a ModuleList's index costs a microsecond)
+        first, last = _buffers_of(experts['0'].wi), _buffers_of(experts[str(len(experts) - 1)].wo)
+        return [first[0], first[2], last[0], last[2]]
 
     def refresh(self):
         """Forget the stacked copy of the experts; the next forward rebuilds it.
@@ -318,7 +327,7 @@ class FasterMLP(nn.Module):
                 layer.__dict__.pop("_copies", None)
 
     def _forget(self):
-        if getattr(self, '_released', False):
+        if self._released:
             raise RuntimeError('the packed buffers of this layer were released; '
                                'it cannot be moved, reloaded or refreshed')
         self._launcher_cache = None
@@ -332,11 +341,11 @@ class FasterMLP(nn.Module):
         return super()._load_from_state_dict(*args, **kwargs)
 
     def _launcher(self):
-        cached = getattr(self, '_launcher_cache', None)
-        if getattr(self, '_released', False):
+        cached = self._launcher_cache
+        if self._released:
             return cached[1]
         live = self._sentinels()
-        key = tuple((t.data_ptr(), t._version, t.numel()) for t in live)
+        key = [(t.data_ptr(), t._version, t.numel()) for t in live]
         if cached is None or cached[0] != key:
             layer = Sub1Experts([e.wi for e in self.experts], [e.wo for e in self.experts])
             # the aliases keep the keyed addresses from being reused while cached

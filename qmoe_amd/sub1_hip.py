@@ -11,7 +11,6 @@ sub1_cuda_kernel.cu:78-87), `sub1matvec_tokens`, `sub1decode`, and the grouped
 expert launch `ExpertStack.forward`.
 """
 import ctypes
-from operator import attrgetter
 
 import torch
 
@@ -33,10 +32,7 @@ def clear_faults():
 
 def _stream():
     """torch's current stream on the current device, as the C ABI takes it."""
-    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
-
-
-_dtype_of = attrgetter('dtype')
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 class _on_device:
@@ -58,6 +54,16 @@ class _on_device:
         return False
 
 
+def _launch(device, function, *args):
+    """function(*args, torch's current stream there) with `device` as the current one."""
+    if torch._C._cuda_getDevice() == device.index:
+        status = function(*args, torch._C._cuda_getCurrentRawStream(device.index))
+    else:
+        with torch.cuda.device(device):
+            status = function(*args, _stream())
+    _lib.check(status)
+
+
 def _need(t, dtype, name, device=None, numel=None, dim=None):
     if not isinstance(t, torch.Tensor):
         raise TypeError('%s must be a torch.Tensor' % name)
@@ -76,21 +82,22 @@ def _need(t, dtype, name, device=None, numel=None, dim=None):
     return t.data_ptr()
 
 
-def _pointers(tensors, dtype, name, device, numel=None):
-    """Their addresses, each looked over as _need does.  (A layer of 128 experts
-    has 768 tensors: looking at all of them for one thing at a time, without a
-    call of _need each, takes a quarter of the time.)"""
-    try:
-        fine = (set(map(torch.Tensor.get_device, tensors)) == {device.index}
-                and set(map(_dtype_of, tensors)) == {dtype}
-                and all(map(torch.Tensor.is_contiguous, tensors))
-                and (numel is None or set(map(torch.Tensor.numel, tensors)) == {numel}))
-    except (TypeError, AttributeError):      # something that is no tensor
-        fine = False
-    if not fine:
-        for t in tensors:
-            _need(t, dtype, name, device, numel=numel)
-    return list(map(torch.Tensor.data_ptr, tensors))
+def _addresses(spec, tensors, numels, device):
+    """Addresses of the tensors, each looked over as _need does: spec holds (dtype,
+    name, dimensions or -1), numels the elements or -1.  Plain tensors in order are
+    looked over in C++; anything else goes through _need, for its error."""
+    got = _lib.tensor_args().addresses(spec, tensors, numels, getattr(device, 'index', None))
+    if got is None:
+        got = [_need(t, dtype, name, device, None if n < 0 else n, None if dim < 0 else dim)
+               for t, (dtype, name, dim), n in zip(tensors, spec, numels)]
+    return got
+
+
+_MATRIX = ((torch.int32, 'dec', -1), (torch.int16, 'w_comp', -1), (torch.int32, 'row_off', -1),
+           (torch.bfloat16, 'ter_minmax', -1))
+_MATVEC = _MATRIX + ((torch.bfloat16, 'x', -1), (torch.bfloat16, 'y', -1))
+_MATVEC_TOKENS = _MATRIX + ((torch.bfloat16, 'x', 2), (torch.bfloat16, 'y', 2))
+_ROUTED = ((torch.bfloat16, 'x', 2), (torch.int32, 'token_expert', -1))
 
 
 def route_from_mask(router_mask):
@@ -111,9 +118,8 @@ def route_from_mask(router_mask):
     index = torch.empty(mask.shape[:-1], dtype=torch.int64, device=mask.device)
     if tokens == 0:
         return route, index
-    with _on_device(mask.device):
-        _lib.check(_lib.load().sub1_route_from_mask(mask.data_ptr(), size, tokens, experts,
-                                                    route.data_ptr(), index.data_ptr(), _stream()))
+    _launch(mask.device, _lib.load().sub1_route_from_mask, mask.data_ptr(), size, tokens, experts,
+            route.data_ptr(), index.data_ptr())
     return route, index
 
 
@@ -132,36 +138,21 @@ def sub1matvec(dec, w_comp, row_off, ter_minmax, x, y):
     dev = dec.device if isinstance(dec, torch.Tensor) else None
     _lib.check_faults()
     height, width = y.numel(), x.numel()
-    args = [
-        _need(dec, torch.int32, 'dec', numel=_lib.DEC_WORDS),
-        _need(w_comp, torch.int16, 'w_comp', dev),
-        _need(row_off, torch.int32, 'row_off', dev, numel=height + 1),
-        _need(ter_minmax, torch.bfloat16, 'ter_minmax', dev, numel=2 * height),
-        _need(x, torch.bfloat16, 'x', dev),
-        _need(y, torch.bfloat16, 'y', dev),
-    ]
-    with _on_device(dev):
-        _lib.check(_lib.load().sub1_matvec(*args, height, width, _stream()))
+    args = _addresses(_MATVEC, (dec, w_comp, row_off, ter_minmax, x, y),
+                      (_lib.DEC_WORDS, -1, height + 1, 2 * height, -1, -1), dev)
+    _launch(dev, _lib.load().sub1_matvec, *args, height, width)
 
 
 def sub1matvec_tokens(dec, w_comp, row_off, ter_minmax, x, y):
     """y[t] += W x[t] for x [T, W], y [T, H] in one launch."""
     dev = dec.device if isinstance(dec, torch.Tensor) else None
-    args = [
-        _need(dec, torch.int32, 'dec', numel=_lib.DEC_WORDS),
-        _need(w_comp, torch.int16, 'w_comp', dev),
-        _need(row_off, torch.int32, 'row_off', dev),
-        _need(ter_minmax, torch.bfloat16, 'ter_minmax', dev),
-        _need(x, torch.bfloat16, 'x', dev, dim=2),
-        _need(y, torch.bfloat16, 'y', dev, dim=2),
-    ]
+    args = _addresses(_MATVEC_TOKENS, (dec, w_comp, row_off, ter_minmax, x, y),
+                      (_lib.DEC_WORDS, -1, -1, -1, -1, -1), dev)
     tokens, width = x.shape
     height = row_off.numel() - 1
     if y.shape != (tokens, height) or ter_minmax.numel() != 2 * height:
         raise ValueError('y must be [%d, %d] and ter_minmax [%d]' % (tokens, height, 2 * height))
-    with _on_device(dev):
-        _lib.check(_lib.load().sub1_matvec_tokens(*args, height, width, tokens,
-                                                  width, height, _stream()))
+    _launch(dev, _lib.load().sub1_matvec_tokens, *args, height, width, tokens, width, height)
 
 
 def sub1pack(trie, w_tern, row_off):
@@ -235,7 +226,7 @@ def _workspace(stack, tokens):
     torch's allocator, which hands it out again only in the order of the stream
     it was allocated on."""
     need = _lib.load().sub1_moe_workspace_bytes(tokens, stack.d_ff)
-    key = _stream().value
+    key = _stream()
     epoch = _lib.fault_epoch()
     ws = stack._ws.get(key)
     if ws is None or ws.numel() < need:
@@ -251,9 +242,28 @@ def _workspace(stack, tokens):
     return ws
 
 
+def _arguments(stack, x, token_expert):
+    """(address of x, of token_expert, tokens) of a forward."""
+    p_x, p_te = _addresses(_ROUTED, (x, token_expert), (-1, -1), stack.device)
+    tokens, width = x.shape
+    if width != stack.d_model:
+        raise ValueError('x must be [T, %d]' % stack.d_model)
+    if token_expert.numel() != tokens:
+        raise ValueError('token_expert must hold %d elements, got %d' % (tokens, token_expert.numel()))
+    return p_x, p_te, tokens
+
+
+def _result(y, x, device):
+    """(y, its address): what the caller gave, looked over, or a new tensor like x."""
+    if y is None:
+        y = torch.empty_like(x)
+        return y, y.data_ptr()
+    return y, _need(y, torch.bfloat16, 'y', device, numel=x.numel()) if x.shape[0] else None
+
+
 def _fault_delta(stack, tokens):
     # words 1 and 2 of the workspace count over all launches; report what is new
-    key = _stream().value
+    key = _stream()
     ctrl = stack.workspace(tokens)[:16].view(torch.int32).tolist()
     before = stack._seen.get(key, (0, 0))
     stack._seen[key] = (ctrl[1], ctrl[2])
@@ -315,6 +325,7 @@ class ExpertStack:
                 + 2 * self.wo_minmax.numel())
 
     workspace = _workspace
+    _arguments = _arguments
 
     def forward(self, x, token_expert, y=None, matrix_cores=False):
         """y[t] = wo_e(relu(wi_e(x[t]))), e = token_expert[t]; tokens with a
@@ -323,21 +334,13 @@ class ExpertStack:
         one form.)"""
         dev = self.device
         _lib.check_faults()       # what earlier launches reported (host memory, no sync)
-        p_x = _need(x, torch.bfloat16, 'x', dev, dim=2)
-        tokens = x.shape[0]
-        if x.shape[1] != self.d_model:
-            raise ValueError('x must be [T, %d]' % self.d_model)
-        p_te = _need(token_expert, torch.int32, 'token_expert', dev, numel=tokens)
-        if y is None:
-            y = torch.empty_like(x)
+        p_x, p_te, tokens = self._arguments(x, token_expert)
+        y, p_y = _result(y, x, dev)
         if tokens == 0:
             return y
-        p_y = _need(y, torch.bfloat16, 'y', dev, numel=x.numel())
         ws = self.workspace(tokens)
-        with _on_device(dev):
-            _lib.check(_lib.load().sub1_moe_grouped(
-                ctypes.byref(self._c), p_te, p_x, p_y, tokens, ws.data_ptr(),
-                ws.numel(), _stream()))
+        _launch(dev, _lib.load().sub1_moe_grouped, ctypes.byref(self._c), p_te, p_x, p_y, tokens,
+                ws.data_ptr(), ws.numel())
         return y
 
     def can_prepare(self):
@@ -387,13 +390,16 @@ class PreparedStack:
             raise ValueError('as many wi as wo layers, at least one')
         d_ff = wi_layers[0][1].numel() - 1
         d_model = wo_layers[0][1].numel() - 1
-        columns = []
-        for layers, rows in ((wi_layers, d_ff), (wo_layers, d_model)):
-            codes, offsets, minmax = zip(*layers)
-            columns += [_pointers(codes, torch.int16, 'w_comp', dev),
-                        _pointers(offsets, torch.int32, 'row_off', dev, rows + 1),
-                        _pointers(minmax, torch.bfloat16, 'ter_minmax', dev, 2 * rows)]
-        tables = torch.tensor(columns, dtype=torch.int64).to(dev)
+        # the tables of addresses, from pinned memory: the copy waits for nothing
+        table = torch.empty((6, experts), dtype=torch.int64, pin_memory=True)
+        for row, layers, rows in ((0, wi_layers, d_ff), (3, wo_layers, d_model)):
+            numels = (-1, rows + 1, 2 * rows)
+            if not _lib.tensor_args().layer_addresses(table, row, list(layers), _MATRIX[1:], numels, dev.index):
+                codes, offsets, minmax = zip(*layers)
+                for tensors, (dtype, name, _), n in zip((codes, offsets, minmax), _MATRIX[1:], numels):
+                    table[row] = torch.tensor([_need(t, dtype, name, dev, None if n < 0 else n) for t in tensors])
+                    row += 1
+        tables = table.to(dev, non_blocking=True)
         wi_c, wi_r, wi_m, wo_c, wo_r, wo_m = (tables.data_ptr() + 8 * experts * i for i in range(6))
         c_layers = _lib.MoeLayers(_need(dec, torch.int32, 'dec', numel=_lib.DEC_WORDS), wi_c, wo_c,
                                   wi_r, wo_r, wi_m, wo_m, experts, d_model, d_ff)
@@ -435,6 +441,7 @@ class PreparedStack:
         self._seen = {}      # per workspace: the fault counts launch_faults() last returned from
 
     workspace = _workspace
+    _arguments = _arguments
 
     def forward(self, x, token_expert, y=None, matrix_cores=False):
         """As ExpertStack.forward.  matrix_cores: a batch for which batch_pays
@@ -442,23 +449,15 @@ class PreparedStack:
         a comparison)."""
         dev = self.device
         _lib.check_faults()       # what earlier launches reported (host memory, no sync)
-        p_x = _need(x, torch.bfloat16, 'x', dev, dim=2)
-        tokens, width = x.shape
-        if width != self.d_model:
-            raise ValueError('x must be [T, %d]' % self.d_model)
+        p_x, p_te, tokens = self._arguments(x, token_expert)
         if matrix_cores and tokens >= self.batch_tokens and self.batch_pays(tokens):
             return self.forward_batch(x, token_expert, y)
-        p_te = _need(token_expert, torch.int32, 'token_expert', dev, numel=tokens)
-        if y is None:
-            y = torch.empty_like(x)
+        y, p_y = _result(y, x, dev)
         if tokens == 0:
             return y
-        p_y = _need(y, torch.bfloat16, 'y', dev, numel=x.numel())
         ws = self.workspace(tokens)
-        with _on_device(dev):
-            _lib.check(_lib.load().sub1_moe_grouped_prepared(
-                ctypes.byref(self._c), p_te, p_x, p_y, tokens, ws.data_ptr(), ws.numel(),
-                _stream()))
+        _launch(dev, _lib.load().sub1_moe_grouped_prepared, ctypes.byref(self._c), p_te, p_x, p_y, tokens,
+                ws.data_ptr(), ws.numel())
         return y
 
     def batch_pays(self, tokens):
@@ -480,16 +479,10 @@ class PreparedStack:
         dev = self.device
         _lib.check_faults()       # what earlier launches reported (host memory, no sync)
         lib = _lib.load()
-        p_x = _need(x, torch.bfloat16, 'x', dev, dim=2)
-        tokens = x.shape[0]
-        if x.shape[1] != self.d_model:
-            raise ValueError('x must be [T, %d]' % self.d_model)
-        p_te = _need(token_expert, torch.int32, 'token_expert', dev, numel=tokens)
-        if y is None:
-            y = torch.empty_like(x)
+        p_x, p_te, tokens = self._arguments(x, token_expert)
+        y, p_y = _result(y, x, dev)
         if tokens == 0:
             return y
-        p_y = _need(y, torch.bfloat16, 'y', dev, numel=x.numel())
         ws = self.workspace(tokens)
         need = lib.sub1_moe_batch_scratch_bytes(ctypes.byref(self._c), tokens)
         if need <= 0:
@@ -588,10 +581,8 @@ class PreparedMatrix:
             raise ValueError('token_matrix is required with %d matrices' % self.count)
         y = torch.empty((tokens, self.height), dtype=torch.bfloat16, device=self.device)
         if tokens:
-            with _on_device(self.device):
-                _lib.check(_lib.load().sub1_product_prepared(
-                    ctypes.byref(self._c), p_x, self.width, y.data_ptr(), self.height, tokens,
-                    _stream()))
+            _launch(self.device, _lib.load().sub1_product_prepared, ctypes.byref(self._c), p_x, self.width,
+                    y.data_ptr(), self.height, tokens)
         return y
 
     def decode(self, matrix=0):
@@ -665,10 +656,8 @@ class TiledMatrix:
             raise ValueError('x must be [T, %d]' % self.width)
         y = torch.empty((tokens, self.height), dtype=torch.bfloat16, device=self.device)
         if tokens:
-            with _on_device(self.device):
-                _lib.check(_lib.load().sub1_product_tiles(
-                    ctypes.byref(self._c), matrix, p_x, self.width, y.data_ptr(), self.height, tokens,
-                    _stream()))
+            _launch(self.device, _lib.load().sub1_product_tiles, ctypes.byref(self._c), matrix, p_x, self.width,
+                    y.data_ptr(), self.height, tokens)
         return y
 
     def decode(self, matrix=0):
