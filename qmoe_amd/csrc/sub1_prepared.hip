@@ -520,14 +520,17 @@ __global__ __launch_bounds__(kWalkThreads) void walk_rows_kernel(WalkArgs a) {
 
 // One workgroup per matrix: order the rows by entry count, longest first, rows
 // of equal count by row number, and describe the 64-row slices.  A counting sort,
-// the same order on every run: a histogram over the counts between the smallest
-// and the largest, its prefix sums, then the rows 64 at a time, each after the
-// places that the ones before it have taken.  That last part is a chain, so only
-// what has to be is in it: a row's rank among the equal counts of its 64 is found
-// beforehand by all wavefronts (a ballot per bit of the count), one wavefront then
-// needs two LDS accesses per 64 rows.  128 base experts: 24 us
-// for wi (3072 rows), 10 for wo, where one thread that walked the histogram and took
-// the rows one by one needed 750 and 325.
+// the same order on every run: the rows are cut into parts, one per wavefront, each
+// with a histogram of its own over the counts between the smallest and the largest;
+// prefix sums over the bins, and within a bin over the parts, say where each
+// part's rows of a count begin; then every wavefront places its rows 64 at a time,
+// each after the places that the ones before it have taken.  A row's rank among
+// the equal counts of its 64 is found with the histogram (a ballot per bit of the
+// count).  Where the counts spread so far that a histogram for every wavefront does not
+// fit, there are fewer parts, down to one.
+// 128 base experts, wi and wo (3072 and 768 rows): 13 us.  One wavefront that placed
+// all rows, two dependent LDS accesses per 64, took 23; one thread that walked the
+// histogram and took the rows one by one 750 for wi alone.
 // Dynamic LDS: the bins, the entry count of the first row of up to 1024 slices
 // (65534 rows), a few words per wavefront, and a byte per row.
 constexpr int kOrderThreads = 1024;
@@ -595,27 +598,46 @@ __global__ __launch_bounds__(kOrderThreads) void order_rows_kernel(OrderArgs a) 
     high = max(high, wave_b[w]);
   }
   const int range = high - low + 1;   // bin b: the rows of high - b entries
-  for (int i = tid; i < range; i += kOrderThreads) bins[i] = 0;
+  int parts = kOrderWaves;            // bins[range * part + b]: part's rows in bin b, then where the next one goes
+  while (parts > 1 && parts * range > kOrderBins) parts >>= 1;
+  const int groups = (height + 63) / 64, part_groups = (groups + parts - 1) / parts;
+  const int from = 64 * part_groups * wave, to = min(from + 64 * part_groups, height);   // this wavefront's rows
+  for (int i = tid; i < parts * range; i += kOrderThreads) bins[i] = 0;
   __syncthreads();
-  for (int r0 = wave * 64; r0 < height; r0 += kOrderThreads) {
-    const int r = r0 + lane;
-    const int bin = r < height ? high - rl[r] : 0;
-    unsigned long long same = __ballot(r < height);
-    for (int bit = 1; bit < range; bit <<= 1) {
-      const unsigned long long with = __ballot((bin & bit) != 0);
-      same &= (bin & bit) ? with : ~with;
+  int *mine = bins + range * wave;
+  if (wave < parts)
+    for (int r0 = from; r0 < to; r0 += 64 * kOrderAhead) {
+      int len[kOrderAhead];
+#pragma unroll
+      for (int u = 0; u < kOrderAhead; u++) {
+        const int r = r0 + 64 * u + lane;
+        len[u] = r < to ? rl[r] : 0;
+      }
+#pragma unroll
+      for (int u = 0; u < kOrderAhead; u++) {
+        if (r0 + 64 * u >= to) break;
+        const int r = r0 + 64 * u + lane;
+        const int bin = r < to ? high - len[u] : 0;
+        unsigned long long same = __ballot(r < to);
+        for (int bit = 1; bit < range; bit <<= 1) {
+          const unsigned long long with = __ballot((bin & bit) != 0);
+          same &= (bin & bit) ? with : ~with;
+        }
+        if (r < to) {
+          const int before = __popcll(same & ((1ull << lane) - 1));
+          const bool last = lane == 63 - __clzll(same);
+          rank[r] = static_cast<uint8_t>(before | (last ? 64 : 0));
+          if (last) atomicAdd(&mine[bin], before + 1);
+        }
+      }
     }
-    if (r < height) {
-      const int before = __popcll(same & ((1ull << lane) - 1));
-      const bool last = lane == 63 - __clzll(same);
-      rank[r] = static_cast<uint8_t>(before | (last ? 64 : 0));
-      if (last) atomicAdd(&bins[bin], before + 1);
-    }
-  }
   __syncthreads();
   int carry = 0;
-  for (int b0 = 0; b0 < range; b0 += kOrderThreads) {   // every bin's first place
-    const int n = b0 + tid < range ? bins[b0 + tid] : 0;
+  for (int b0 = 0; b0 < range; b0 += kOrderThreads) {   // every bin's first place, and every part's in it
+    const int b = b0 + tid;
+    int n = 0;
+    if (b < range)
+      for (int q = 0; q < parts; q++) n += bins[range * q + b];
     int upto = n;
     for (int d = 1; d < 64; d <<= 1) {
       const int v = __shfl_up(upto, d, 64);
@@ -628,38 +650,45 @@ __global__ __launch_bounds__(kOrderThreads) void order_rows_kernel(OrderArgs a) 
       if (w < wave) before += wave_a[w];
       carry += wave_a[w];
     }
-    if (b0 + tid < range) bins[b0 + tid] = before + upto - n;
+    int place = before + upto - n;
+    if (b < range)
+      for (int q = 0; q < parts; q++) {
+        const int rows = bins[range * q + b];
+        bins[range * q + b] = place;
+        place += rows;
+      }
     __syncthreads();
   }
-  if (wave == 0) {
-    volatile int *place = bins;   // read and written by this wavefront alone, in program order
-    for (int r0 = 0; r0 < height; r0 += 64 * kOrderAhead) {
+  if (wave < parts) {
+    volatile int *place = mine;   // read and written by this wavefront alone, in program order
+    for (int r0 = from; r0 < to; r0 += 64 * kOrderAhead) {
       int len[kOrderAhead];
+      uint32_t values[kOrderAhead];
 #pragma unroll
       for (int u = 0; u < kOrderAhead; u++) {
         const int r = r0 + 64 * u + lane;
-        len[u] = r < height ? rl[r] : 0;
+        len[u] = r < to ? rl[r] : 0;
+        values[u] = r < to ? mm[r] : 0u;
       }
 #pragma unroll
       for (int u = 0; u < kOrderAhead; u++) {
         const int r = r0 + 64 * u + lane;
-        if (r < height) {
-          const int mine = rank[r];
-          const int p = place[high - len[u]] + (mine & 63);
-          if (mine & 64) place[high - len[u]] = p + 1;
+        if (r < to) {
+          const int before = rank[r];
+          const int p = place[high - len[u]] + (before & 63);
+          if (before & 64) place[high - len[u]] = p + 1;
           row_idx[lane0 + p] = static_cast<uint16_t>(r);
+          minmax_sorted[lane0 + p] = values[u];
           if ((p & 63) == 0) first_len[p >> 6] = len[u];
         }
       }
     }
-  } else {
-    for (int p = height + tid - 64; p < slices * 64; p += kOrderThreads - 64) {
-      row_idx[lane0 + p] = 0xffffu;
-      minmax_sorted[lane0 + p] = 0u;
-    }
   }
-  __syncthreads();   // covers row_idx too: one workgroup, one L1
-  for (int p = tid; p < height; p += kOrderThreads) minmax_sorted[lane0 + p] = mm[row_idx[lane0 + p]];
+  for (int p = height + tid; p < slices * 64; p += kOrderThreads) {
+    row_idx[lane0 + p] = 0xffffu;
+    minmax_sorted[lane0 + p] = 0u;
+  }
+  __syncthreads();
   for (int s = tid; s < slices; s += kOrderThreads) {
     const int len = max(first_len[s], 1);   // a slice is as long as its first row, and at least one entry
     const int64_t g = static_cast<int64_t>(e) * slices + s;

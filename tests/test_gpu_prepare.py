@@ -312,3 +312,10 @@ def test_the_first_pack_of_a_process_may_be_captured():
     res = subprocess.run([sys.executable, '-c', FIRST_PACK_IN_A_CAPTURE, root], stdout=subprocess.PIPE,
                          stderr=subprocess.STDOUT, text=True, timeout=110)
     assert res.returncode == 0 and 'first call in a capture: fine' in res.stdout, res.stdout
+
+
+@pytest.mark.parametrize('height,width,shares', [
+    (1088, 900, [0.0, 0.1, 0.9]), (1023, 1100, [0.02, 1.0]),                  # a part per wavefront, some without rows
+    (2000, 3100, [0.0, 0.5, 0.99]), (700, 6000, [0.0, 0.9]), (8200, 40, [0.1, 0.5])])   # fewer parts; a turn of a part and more
+def test_rows_that_are_ordered_in_parts_come_back_whole(gpu, height, width, shares):
+    test_prepared_rows_come_back_whole(gpu, height, width, shares)
