@@ -391,13 +391,14 @@ class PreparedStack:
         d_ff = wi_layers[0][1].numel() - 1
         d_model = wo_layers[0][1].numel() - 1
         # the tables of addresses, from pinned memory: the copy waits for nothing
-        table = torch.empty((6, experts), dtype=torch.int64, pin_memory=True)
+        table = torch.empty((6, experts), dtype=torch.int64, device='cpu', pin_memory=True)
         for row, layers, rows in ((0, wi_layers, d_ff), (3, wo_layers, d_model)):
             numels = (-1, rows + 1, 2 * rows)
             if not _lib.tensor_args().layer_addresses(table, row, list(layers), _MATRIX[1:], numels, dev.index):
                 codes, offsets, minmax = zip(*layers)
                 for tensors, (dtype, name, _), n in zip((codes, offsets, minmax), _MATRIX[1:], numels):
-                    table[row] = torch.tensor([_need(t, dtype, name, dev, None if n < 0 else n) for t in tensors])
+                    table[row] = torch.tensor([_need(t, dtype, name, dev, None if n < 0 else n) for t in tensors],
+                                              device='cpu')
                     row += 1
         tables = table.to(dev, non_blocking=True)
         wi_c, wi_r, wi_m, wo_c, wo_r, wo_m = (tables.data_ptr() + 8 * experts * i for i in range(6))

@@ -61,3 +61,16 @@ def test_a_layer_may_come_in_any_form(form):
                           ((wo[1][0], None, wo[1][2]), TypeError)):
         with pytest.raises(error):
             sub1_hip.PreparedStack.from_layers(sub1.DEC[0], wi, [wo[0], broken, wo[2]])
+
+
+@pytest.mark.gpu
+def test_a_layer_is_prepared_the_same_under_another_default_device():
+    from qmoe_amd import sub1, synthetic
+    stack = synthetic.build_stack(2, 96, 160, 0.9, seed=5)
+    wi, wo = zip(*[synthetic.expert_layers(stack, e) for e in range(2)])
+    wo = (wo[0], (wo[1][0].as_subclass(Wrapped),) + tuple(wo[1][1:]))     # one half of the table each way
+    x, route = synthetic.activations(4, 96, 6), torch.arange(4, dtype=torch.int32, device='cuda') % 2
+    want = stack.prepare().forward(x, route)
+    with torch.device('cuda'):
+        made = sub1_hip.PreparedStack.from_layers(sub1.DEC[0], wi, wo)
+    assert torch.equal(made.forward(x, route).view(torch.int16), want.view(torch.int16))
