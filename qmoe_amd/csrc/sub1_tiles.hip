@@ -261,6 +261,7 @@ struct TileArgs {
   int height, width, tokens;
   int units_down, windows, matrix;
   int fresh;   // y holds nothing yet: it counts as zeros and is not read
+  int column_blocks, larger_columns;   // shared kernel: blocks of 32 tokens a column; one more in the first ones
 };
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -720,9 +721,10 @@ __device__ __forceinline__ void lds_request_blocks(uint32_t at, u32x4 (&v)[kN]) 
 }
 template <int kN>
 __device__ __forceinline__ void lds_arrived_blocks(u32x4 (&v)[kN]) {
-  static_assert(kN == 1 || kN == 2 || kN == 4, "one, two or four blocks");
+  static_assert(kN >= 1 && kN <= 4, "one to four blocks");
   if constexpr (kN == 1) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0])::"memory");
   if constexpr (kN == 2) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]), "+v"(v[1])::"memory");
+  if constexpr (kN == 3) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2])::"memory");
   if constexpr (kN == 4)
     asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])::"memory");
 }
@@ -841,9 +843,9 @@ void matvec_tiles_shared_kernel(TileArgs a) {
   l.half = l.lane >> 5;
   l.block = blockIdx.x * kRG + g;
   const bool has_rows = l.block < blocks;
-  l.t0 = blockIdx.y * (32 * kNB);
-  l.rows_here = min(32 * kNB, a.tokens - l.t0);
-  const int live = (l.rows_here + 31) / 32;
+  const int live = a.column_blocks + (static_cast<int>(blockIdx.y) < a.larger_columns ? 1 : 0);
+  l.t0 = 32 * (blockIdx.y * a.column_blocks + min(static_cast<int>(blockIdx.y), a.larger_columns));
+  l.rows_here = min(32 * live, a.tokens - l.t0);
 #pragma unroll
   for (int j = 0; j < 2; j++) {
     const int row = l.block * kRows + j * kUnitRows + (l.lane & 31);
@@ -997,8 +999,10 @@ void matvec_tiles_shared_kernel(TileArgs a) {
       if (turn + 1 < turns) turn_of(turn + 1, 1, codes_b, codes_a);
     }
   };
-  if (live > kNB / 2)
+  if (live == kNB)
     run(std::integral_constant<int, kNB>{});
+  else if (kNB == 4 && live == 3)
+    run(std::integral_constant<int, kNB == 4 ? 3 : kNB>{});
   else
     run(std::integral_constant<int, kNB / 2>{});
   // nothing is on its way into LDS any more
@@ -1082,14 +1086,38 @@ const TileForm &pick_form(int parts, int row_blocks, int windows, int tokens, bo
 
 std::atomic<int> g_forced_kernel{0};   // sub1_test_tiles_kernel
 
+// The columns of workgroups that a launch's blocks of 32 tokens are shared among, `most` blocks to
+// a column or fewer, the larger ones first.  Columns of four blocks that make 1.1 or 1.7
+// workgroups a compute unit cost the time of two on every unit; as many columns as make
+// whole rounds, if some unit then has fewer blocks to do, even them out (c-2048 wi on 2272 tokens:
+// 21 columns of three and four blocks for 18 of four, seven blocks a unit instead of eight:
+// 59.4 -> 55.5 us; c-2048 wo 69.4 -> 58.7).
+// Launches of many rounds have little to gain.
+int columns_of(int tokens, int most, int row_groups) {
+  const int token_blocks = (tokens + 31) / 32, least = (token_blocks + most - 1) / most;
+  const int64_t rounds = (static_cast<int64_t>(least) * row_groups + 255) / 256;
+  if (most < 4 || rounds > 4) return least;
+  auto longest = [&](int64_t columns) {   // blocks of the unit that has most
+    return token_blocks / columns * rounds + (token_blocks % columns * row_groups + 255) / 256;
+  };
+  int best = least;
+  for (int64_t n = least + 1; n <= std::min<int64_t>(rounds * 256 / row_groups, token_blocks / 2); n++)
+    if (longest(n) < longest(best)) best = static_cast<int>(n);
+  return best;
+}
+
 template <bool kDirect, int kRG, int kKP, int kNB>
-int launch_shared_as(const TileArgs &a, int blocks, hipStream_t stream) {
+int launch_shared_as(TileArgs a, int blocks, hipStream_t stream) {
   constexpr int waves = kRG * kKP;
   constexpr int lds = kKP * 2 * kNB * 32 * 256;
   static_assert(lds >= waves * (kKP - 1) * (2 * kNB / kKP) * 4096 && lds <= 160 * 1024, "tiles, then sums");
   HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(matvec_tiles_shared_kernel<kDirect, kRG, kKP, kNB>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-  const dim3 grid((blocks + kRG - 1) / kRG, (a.tokens + 32 * kNB - 1) / (32 * kNB));
+  const int row_groups = (blocks + kRG - 1) / kRG, token_blocks = (a.tokens + 31) / 32;
+  const int columns = columns_of(a.tokens, kNB, row_groups);
+  a.column_blocks = token_blocks / columns;
+  a.larger_columns = token_blocks % columns;
+  const dim3 grid(row_groups, columns);
   matvec_tiles_shared_kernel<kDirect, kRG, kKP, kNB><<<grid, 64 * waves, lds, stream>>>(a);
   HIP_TRY(hipGetLastError());
   return SUB1_OK;

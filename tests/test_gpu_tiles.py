@@ -98,7 +98,9 @@ def test_tiles_product(gpu, oracle, height, width, p0, tokens):
     (3072, 768, 0.9, 700, 64),       # windows split two ways, rows in groups of 128
     (4096, 1024, 0.88, 1100, 64),    # one part, rows in groups of 256
     (3200, 2080, 0.9, 1500, 64),     # 50 blocks of rows (not a multiple of four), a ragged last window
-    (6272, 520, 0.9, 2100, 128)])    # blocks of 128 tokens, the last with 52
+    (6272, 520, 0.9, 2100, 128),     # blocks of 128 tokens and less, the last with 52
+    (6144, 640, 0.9, 2272, 128),     # columns of four blocks of 32 and of three
+    (6144, 520, 0.9, 2246, 128)])    # the same, the last with six tokens
 def test_long_sequences_share_their_activations(gpu, oracle, height, width, p0, tokens, blocks_of):
     """From the number of tokens on at which the one-wavefront workgroups no
     longer fit the chip at once, workgroups of four wavefronts share each window
