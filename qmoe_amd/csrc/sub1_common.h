@@ -128,6 +128,8 @@ class AnswerSlot {
 
  private:
   int slot_ = -1;
+  bool open_ = false;   // taken, and not answered
+  hipStream_t stream_ = nullptr;
   Answer answer_{};
 };
 

@@ -129,11 +129,18 @@ int AnswerSlot::take(hipStream_t stream, const char *who) {
   answer_.counters = static_cast<unsigned long long *>(counters) + slot_ * kAnswerCounterWords;
   do answer_.ticket = ++g_answer_ticket;
   while (answer_.ticket == 0);   // what the words hold at first
+  stream_ = stream;
+  open_ = true;
   return SUB1_OK;
 }
 
 AnswerSlot::~AnswerSlot() {
   if (slot_ < 0) return;
+  // a call that ends without its answer, by an error: what it has launched still counts and stores
+  if (open_ && hipStreamSynchronize(stream_) != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
   {
     std::lock_guard<std::mutex> lock(g_answer_mutex);
     g_answer_slots.push_back(slot_);
@@ -155,12 +162,18 @@ int AnswerSlot::wait(hipStream_t stream, int n, int32_t *values, const char *who
   const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(5);
   do {
     for (int i = 0; i < 64; i++) {
-      if (arrived()) return SUB1_OK;
+      if (arrived()) {
+        open_ = false;
+        return SUB1_OK;
+      }
       __builtin_ia32_pause();
     }
   } while (std::chrono::steady_clock::now() < until);
   const hipError_t e = hipStreamSynchronize(stream);
-  if (e == hipSuccess && arrived()) return SUB1_OK;
+  if (e == hipSuccess && arrived()) {
+    open_ = false;
+    return SUB1_OK;
+  }
   slot_ = -1;   // something may still be written there
   if (e != hipSuccess) return fail(SUB1_ERR_HIP, "%s: %s", who, hipGetErrorString(e));
   return fail(SUB1_ERR_INTERNAL, "%s: the launch has ended without its answer", who);
