@@ -95,7 +95,9 @@ __device__ __forceinline__ void tell(const Answer &a, int word, int32_t value) {
 
 // One thread of every workgroup says what its workgroup counted; the last of them tells the
 // sum.  A count goes up together with the number of workgroups in it, so nothing has to be in
-// order.  (In two steps: 750 workgroups that add to one word queue up for 8 us.)
+// order.  (In two steps: 750 workgroups that add to one word queue up for 8 us.)  A counter is
+// put back to zero by an exchange, and what that returns is what is told: the zeros are in
+// place before the host hears of the sum and gives the slot to a call on another stream.
 __device__ __forceinline__ void tell_sum(const Answer &a, int word, int32_t value) {
   const int shard = blockIdx.x % kAnswerShards;
   const int shards = min(static_cast<int>(gridDim.x), kAnswerShards);
@@ -105,8 +107,8 @@ __device__ __forceinline__ void tell_sum(const Answer &a, int word, int32_t valu
   for (int step = 0; step < 2; step++) {
     const unsigned long long sum = one + __hip_atomic_fetch_add(counter, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (static_cast<int>(static_cast<uint32_t>(sum)) != workgroups) return;
-    __hip_atomic_store(counter, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    one = (sum >> 32) << 32 | 1u;
+    const unsigned long long whole = __hip_atomic_exchange(counter, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    one = (whole >> 32) << 32 | 1u;
     counter = a.counters;
     workgroups = shards;
   }

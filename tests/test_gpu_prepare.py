@@ -270,6 +270,24 @@ def test_calls_that_wait_for_the_gpu_come_from_any_thread_and_stream(gpu):
     assert y.tolist() == [2.0] * 8
 
 
+def test_a_count_starts_from_zero_on_whichever_stream_the_next_call_is(gpu):
+    """Calls that take turns on two streams get one place to answer in after another: what
+    one has counted is gone before the next, on the other stream, adds to it."""
+    sub1, op = gpu
+    rows = 700
+    symbols = symbols_of(rows, 64, [0.3], seed=6)
+    w_comp, row_off = packed(gpu, symbols)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    short = [row_off.clone() for _ in range(4)]
+    for n in range(4):                              # n rows lack their last code, n have one too many
+        short[n][1:2 * n + 1:2] -= 1
+    torch.cuda.synchronize()
+    for i in range(200):
+        with torch.cuda.stream(streams[i % 2]):
+            n = i * 7 % 4
+            assert op.sub1decode(sub1.DEC[0], w_comp, short[n], None, 64, want_w=False)[2] == 2 * n, i
+
+
 FIRST_PACK_IN_A_CAPTURE = r'''
 import ctypes, sys
 sys.path.insert(0, sys.argv[1])
