@@ -141,9 +141,9 @@ int sub1_decode(const int32_t *dec, const int16_t *w_comp, const int32_t *row_of
                 int32_t *bad_rows, int height, int width, void *stream);
 
 /*
- * The same, and *bad_rows (int32 in host memory) receives the number of such rows: the
- * call returns once it is known, which is when the launch's last workgroup is done.  Not
- * for a stream that is being captured.
+ * The same, and *bad_rows (int32 in host memory) receives the number of such rows.  The
+ * call returns when both outputs are complete, so that any stream may read them.  Not for a
+ * stream that is being captured.
  */
 int sub1_decode_counted(const int32_t *dec, const int16_t *w_comp, const int32_t *row_off,
                         const void *ter_minmax, uint8_t *out_tern, void *out_w,

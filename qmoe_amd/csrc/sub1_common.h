@@ -83,36 +83,13 @@ __device__ __forceinline__ void raise_fault(int32_t *sticky, int word) {
 constexpr int kAnswerWords = 8;
 struct Answer {
   unsigned long long *words;     // pinned host memory as the GPU addresses it
-  unsigned long long *counters;  // device memory, zeros, and left at zeros: kAnswerShards and one, 64 bytes apart
+  int32_t *count;                // device memory for a launch to add to: zero, and left at zero
   uint32_t ticket;
 };
-constexpr int kAnswerShards = 16;
-constexpr int kAnswerCounterWords = (kAnswerShards + 1) * 8;
+constexpr int kAnswerCountStride = 16;   // words from one slot's count to the next
 __device__ __forceinline__ void tell(const Answer &a, int word, int32_t value) {
   __hip_atomic_store(&a.words[word], static_cast<unsigned long long>(a.ticket) << 32 | static_cast<uint32_t>(value),
                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-// One thread of every workgroup says what its workgroup counted; the last of them tells the
-// sum.  A count goes up together with the number of workgroups in it, so nothing has to be in
-// order.  (In two steps: 750 workgroups that add to one word queue up for 8 us.)  A counter is
-// put back to zero by an exchange, and what that returns is what is told: the zeros are in
-// place before the host hears of the sum and gives the slot to a call on another stream.
-__device__ __forceinline__ void tell_sum(const Answer &a, int word, int32_t value) {
-  const int shard = blockIdx.x % kAnswerShards;
-  const int shards = min(static_cast<int>(gridDim.x), kAnswerShards);
-  unsigned long long *counter = a.counters + (1 + shard) * 8;
-  int workgroups = (gridDim.x - shard + kAnswerShards - 1) / kAnswerShards;
-  unsigned long long one = static_cast<unsigned long long>(static_cast<uint32_t>(value)) << 32 | 1u;
-  for (int step = 0; step < 2; step++) {
-    const unsigned long long sum = one + __hip_atomic_fetch_add(counter, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (static_cast<int>(static_cast<uint32_t>(sum)) != workgroups) return;
-    const unsigned long long whole = __hip_atomic_exchange(counter, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    one = (whole >> 32) << 32 | 1u;
-    counter = a.counters;
-    workgroups = shards;
-  }
-  tell(a, word, static_cast<int32_t>(one >> 32));
 }
 
 class AnswerSlot {

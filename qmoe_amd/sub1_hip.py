@@ -197,7 +197,8 @@ def sub1pack_weights(w):
 
 def sub1decode(dec, w_comp, row_off, ter_minmax, width, want_tern=True, want_w=True):
     """Decode without multiplying: (symbols uint8 [H, W] or None, weights bf16
-    [H, W] or None, number of rows whose codes do not cover the width)."""
+    [H, W] or None, number of rows whose codes do not cover the width).  Waits
+    for the GPU: the outputs are complete when it returns, on any stream."""
     dev = dec.device if isinstance(dec, torch.Tensor) else None
     height = row_off.numel() - 1
     p_dec = _need(dec, torch.int32, 'dec', numel=_lib.DEC_WORDS)

@@ -288,6 +288,34 @@ def test_a_count_starts_from_zero_on_whichever_stream_the_next_call_is(gpu):
             assert op.sub1decode(sub1.DEC[0], w_comp, short[n], None, 64, want_w=False)[2] == 2 * n, i
 
 
+@pytest.mark.parametrize('at_t,at_w', [(0, 0), (1, 0)])      # one launch, and one for each output
+def test_what_a_counted_expansion_wrote_may_be_read_anywhere_once_it_returns(gpu, at_t, at_w):
+    import ctypes
+    sub1, op = gpu
+    height, width = 3072, 2080
+    symbols = symbols_of(height, width, [0.1], seed=3)
+    w_comp, row_off = packed(gpu, symbols)
+    minmax = torch.tensor([-1.0, 1.0] * height, device='cuda').bfloat16()
+    want = torch.tensor([0.0, -1.0, 1.0], device='cuda')[symbols.long()].bfloat16()
+    n = height * width
+    t_buf, w_buf = torch.zeros(n + 8, dtype=torch.uint8, device='cuda'), torch.zeros(n + 8, dtype=torch.bfloat16, device='cuda')
+    lib, here, there, bad = op._lib.load(), torch.cuda.Stream(), torch.cuda.Stream(), ctypes.c_int32(-1)
+    torch.cuda.synchronize()
+    for i in range(20):
+        with torch.cuda.stream(here):
+            t_buf.fill_(77)
+            w_buf.fill_(77)
+        assert lib.sub1_decode_counted(sub1.DEC[0].data_ptr(), w_comp.data_ptr(), row_off.data_ptr(), minmax.data_ptr(),
+                                       t_buf[at_t:].data_ptr(), w_buf[at_w:].data_ptr(), ctypes.byref(bad), height, width,
+                                       here.cuda_stream) == 0
+        with torch.cuda.stream(there):      # (the last first: they are the last to be written)
+            got_w, got_t = w_buf.flip(0)[8 - at_w:][:n], t_buf.flip(0)[8 - at_t:][:n]
+        there.synchronize()
+        assert bad.value == 0
+        assert torch.equal(got_w.flip(0).view(height, width), want), i
+        assert torch.equal(got_t.flip(0).view(height, width), symbols), i
+
+
 FIRST_PACK_IN_A_CAPTURE = r'''
 import ctypes, sys
 sys.path.insert(0, sys.argv[1])
