@@ -123,8 +123,9 @@ int sub1_pack_weights_emit(const uint16_t *codes, const int32_t *row_off, int16_
                            int height, int width, void *stream);
 
 /*
- * The first of the two, and *total (int32 in host memory) receives row_off[H]: the call
- * returns once it is known.  Not for a stream that is being captured.
+ * The first of the two, and *total (int32 in host memory) receives row_off[H].  The call
+ * returns when all it writes is complete, so that any stream may read it.  Not for a stream
+ * that is being captured.
  */
 int sub1_pack_weights_total(const void *w, uint16_t *codes, void *ter_minmax, int32_t *row_off,
                             int32_t *total, int height, int width, void *stream);

@@ -492,8 +492,13 @@ __global__ __launch_bounds__(sub1::kScanThreads) void row_offset_scan_kernel(int
                                                                             sub1::Answer answer) {
   sub1::scan_in_place(cnt, height);
   if (!answer.words) return;
+  // all offsets are in memory, for any stream to read, before the host hears of the last
+  sub1::drain_stores();
   __syncthreads();
-  if (threadIdx.x == 0) sub1::tell(answer, 0, cnt[height]);
+  if (threadIdx.x == 0) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    sub1::tell(answer, 0, cnt[height]);
+  }
 }
 
 // A wavefront per row, lanes stride over the row's codes.

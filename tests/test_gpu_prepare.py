@@ -316,6 +316,30 @@ def test_what_a_counted_expansion_wrote_may_be_read_anywhere_once_it_returns(gpu
         assert torch.equal(got_t.flip(0).view(height, width), symbols), i
 
 
+def test_what_a_compression_counted_may_be_read_anywhere_once_it_returns(gpu):
+    import ctypes
+    _, op = gpu
+    height, width = 6144, 96
+    weights = torch.randn((height, 3), generator=torch.Generator().manual_seed(5)).cuda().bfloat16()
+    weights[:, 0] = 0
+    weights = weights.gather(1, symbols_of(height, width, [0.1, 0.5], seed=7).long()).contiguous()
+    _, want, minmax = op.sub1pack_weights(weights)
+    codes = torch.empty((height, width // 2), dtype=torch.int16, device='cuda')
+    row_off, pairs = torch.empty_like(want), torch.empty_like(minmax)
+    lib, here, there, total = op._lib.load(), torch.cuda.Stream(), torch.cuda.Stream(), ctypes.c_int32(-1)
+    torch.cuda.synchronize()
+    for i in range(20):
+        with torch.cuda.stream(here):
+            row_off.fill_(-1)
+            pairs.zero_()
+        assert lib.sub1_pack_weights_total(weights.data_ptr(), codes.data_ptr(), pairs.data_ptr(), row_off.data_ptr(),
+                                           ctypes.byref(total), height, width, here.cuda_stream) == 0
+        with torch.cuda.stream(there):
+            got, got_pairs = row_off.flip(0), pairs.clone()
+        there.synchronize()
+        assert total.value == int(want[-1]) and torch.equal(got.flip(0), want) and torch.equal(got_pairs, minmax), i
+
+
 FIRST_PACK_IN_A_CAPTURE = r'''
 import ctypes, sys
 sys.path.insert(0, sys.argv[1])
