@@ -608,6 +608,19 @@ int sub1_set_wait_limit_us(int64_t microseconds);
 int sub1_test_overstate_wait(int extra);
 
 /*
+ * Calls that wait for the GPU (sub1_pack_weights_total, sub1_decode_counted and the prepare
+ * calls) each take one of 64 places to be answered in; further ones wait for a place.  One that
+ * cannot wait for what it has launched leaves its place unusable, and when all are
+ * these calls return SUB1_ERR_INTERNAL.  For tests:
+ *   sub1_test_fail_answers(k)  the next k of them end by SUB1_ERR_INTERNAL behind their
+ *                              first launches.
+ *   sub1_test_slot_pool(n, k)  hands round n places of a pool of its own, k of them lost on
+ *                              the way, then all.  Host only.
+ */
+int sub1_test_fail_answers(int calls);
+int sub1_test_slot_pool(int slots, int lost);
+
+/*
  * sub1_moe_grouped keeps the compact table it derives from `dec` by the
  * ADDRESS of dec (per device).  Call this before freeing a dec buffer whose
  * address may be handed out again for other contents; NULL drops every cached

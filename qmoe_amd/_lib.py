@@ -130,6 +130,8 @@ PROTOTYPES = {
     'sub1_set_wait_limit_us': (_int, [_i64]),
     'sub1_test_overstate_wait': (_int, [_int]),
     'sub1_test_tiles_kernel': (_int, [_int]),
+    'sub1_test_fail_answers': (_int, [_int]),
+    'sub1_test_slot_pool': (_int, [_int, _int]),
     'sub1_unregister_dec': (_int, [_vp]),
 }
 

@@ -4,7 +4,10 @@
 
 #include <hip/hip_runtime.h>
 
+#include <condition_variable>
 #include <cstdint>
+#include <mutex>
+#include <vector>
 
 #include "sub1_hip.h"
 
@@ -92,6 +95,22 @@ __device__ __forceinline__ void tell(const Answer &a, int word, int32_t value) {
                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Slots by number, each of one call at a time; further calls wait for one.  A slot that
+// something may still be written to is lost, and when all of them are nobody waits any more.
+class SlotPool {
+ public:
+  explicit SlotPool(int slots);
+  int take();   // -1: none will come back
+  void give_back(int slot);
+  void lose();
+
+ private:
+  std::mutex mutex_;
+  std::condition_variable changed_;
+  std::vector<int> free_;
+  int left_;    // not lost
+};
+
 class AnswerSlot {
  public:
   AnswerSlot() = default;
@@ -102,12 +121,15 @@ class AnswerSlot {
   // could answer.
   int take(hipStream_t stream, const char *who);
   Answer answer() const { return answer_; }
+  // Behind the first launch of a call: its error (or that of a test).  From then on the GPU may
+  // have the slot in use.
+  int launched(const char *who);
   // After it: the first `n` words.
   int wait(hipStream_t stream, int n, int32_t *values, const char *who);
 
  private:
   int slot_ = -1;
-  bool open_ = false;   // taken, and not answered
+  bool open_ = false;   // launched, and not answered
   hipStream_t stream_ = nullptr;
   Answer answer_{};
 };

@@ -19,12 +19,12 @@
 #include <algorithm>
 #include <atomic>
 #include <chrono>
-#include <condition_variable>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "sub1_common.h"
@@ -95,14 +95,47 @@ int64_t wait_limit_ticks() {
 int expect_extra() { return g_expect_extra.load(); }
 
 namespace {
-constexpr int kAnswerSlots = 64;   // calls that may wait at once; further ones wait for a slot
-std::mutex g_answer_mutex;
-std::condition_variable g_answer_free;
-std::vector<int> g_answer_slots;   // the free ones
+constexpr int kAnswerSlots = 64;   // calls that may wait at once
+std::mutex g_answer_mutex;         // over the two below
 unsigned long long *g_answer_host = nullptr, *g_answer_device = nullptr;   // 4 KB, held until the process ends
 std::atomic<uint32_t> g_answer_ticket{0};
+std::atomic<int> g_fail_answers{0};   // sub1_test_fail_answers
 static __device__ int32_t answer_counts[kAnswerSlots * kAnswerCountStride];
+__global__ void clear_count_kernel(int32_t *count) { *count = 0; }
+SlotPool &answer_slots() {
+  static SlotPool *pool = new SlotPool(kAnswerSlots);   // (never destroyed: threads may still wait at the process's end)
+  return *pool;
+}
 }  // namespace
+
+SlotPool::SlotPool(int slots) : left_(slots) {
+  for (int i = 0; i < slots; i++) free_.push_back(i);
+}
+
+int SlotPool::take() {
+  std::unique_lock<std::mutex> lock(mutex_);
+  changed_.wait(lock, [this] { return !free_.empty() || left_ == 0; });
+  if (left_ == 0) return -1;
+  const int slot = free_.back();
+  free_.pop_back();
+  return slot;
+}
+
+void SlotPool::give_back(int slot) {
+  {
+    std::lock_guard<std::mutex> lock(mutex_);
+    free_.push_back(slot);
+  }
+  changed_.notify_one();
+}
+
+void SlotPool::lose() {
+  {
+    std::lock_guard<std::mutex> lock(mutex_);
+    left_--;
+  }
+  changed_.notify_all();
+}
 
 int AnswerSlot::take(hipStream_t stream, const char *who) {
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
@@ -111,41 +144,52 @@ int AnswerSlot::take(hipStream_t stream, const char *who) {
     return fail(SUB1_ERR_HIP, "%s: waits for the GPU, which a stream that is being captured cannot", who);
   void *counts = nullptr;
   HIP_TRY(hipGetSymbolAddress(&counts, HIP_SYMBOL(answer_counts)));
-  std::unique_lock<std::mutex> lock(g_answer_mutex);
-  if (!g_answer_host) {
-    void *host = nullptr, *device = nullptr;
-    const size_t bytes = kAnswerSlots * kAnswerWords * sizeof(unsigned long long);
-    HIP_TRY(hipHostMalloc(&host, bytes, hipHostMallocPortable | hipHostMallocMapped));
-    memset(host, 0, bytes);
-    HIP_TRY(hipHostGetDevicePointer(&device, host, 0));
-    g_answer_host = static_cast<unsigned long long *>(host);
-    g_answer_device = static_cast<unsigned long long *>(device);
-    for (int i = 0; i < kAnswerSlots; i++) g_answer_slots.push_back(i);
+  {
+    std::lock_guard<std::mutex> lock(g_answer_mutex);
+    if (!g_answer_host) {
+      void *host = nullptr, *device = nullptr;
+      const size_t bytes = kAnswerSlots * kAnswerWords * sizeof(unsigned long long);
+      HIP_TRY(hipHostMalloc(&host, bytes, hipHostMallocPortable | hipHostMallocMapped));
+      memset(host, 0, bytes);
+      HIP_TRY(hipHostGetDevicePointer(&device, host, 0));
+      g_answer_host = static_cast<unsigned long long *>(host);
+      g_answer_device = static_cast<unsigned long long *>(device);
+    }
   }
-  g_answer_free.wait(lock, [] { return !g_answer_slots.empty(); });
-  slot_ = g_answer_slots.back();
-  g_answer_slots.pop_back();
+  slot_ = answer_slots().take();
+  if (slot_ < 0)
+    return fail(SUB1_ERR_INTERNAL, "%s: %d calls could not wait for the GPU, and none waits after them", who, kAnswerSlots);
   answer_.words = g_answer_device + slot_ * kAnswerWords;
   answer_.count = static_cast<int32_t *>(counts) + slot_ * kAnswerCountStride;
   do answer_.ticket = ++g_answer_ticket;
   while (answer_.ticket == 0);   // what the words hold at first
   stream_ = stream;
+  return SUB1_OK;
+}
+
+int AnswerSlot::launched(const char *who) {
+  HIP_TRY(hipGetLastError());
   open_ = true;
+  int left = g_fail_answers.load();
+  while (left > 0)
+    if (g_fail_answers.compare_exchange_weak(left, left - 1))
+      return fail(SUB1_ERR_INTERNAL, "%s: made to fail by sub1_test_fail_answers", who);
   return SUB1_OK;
 }
 
 AnswerSlot::~AnswerSlot() {
   if (slot_ < 0) return;
-  // a call that ends without its answer, by an error: what it has launched still counts and stores
-  if (open_ && hipStreamSynchronize(stream_) != hipSuccess) {
-    (void)hipGetLastError();
-    return;
+  if (open_) {
+    // a call that ends without its answer, by an error: what it has launched still counts and stores
+    clear_count_kernel<<<1, 1, 0, stream_>>>(answer_.count);
+    const bool cleared = hipGetLastError() == hipSuccess;
+    if (hipStreamSynchronize(stream_) != hipSuccess || !cleared) {
+      (void)hipGetLastError();
+      answer_slots().lose();
+      return;
+    }
   }
-  {
-    std::lock_guard<std::mutex> lock(g_answer_mutex);
-    g_answer_slots.push_back(slot_);
-  }
-  g_answer_free.notify_one();
+  answer_slots().give_back(slot_);
 }
 
 int AnswerSlot::wait(hipStream_t stream, int n, int32_t *values, const char *who) {
@@ -174,7 +218,6 @@ int AnswerSlot::wait(hipStream_t stream, int n, int32_t *values, const char *who
     open_ = false;
     return SUB1_OK;
   }
-  slot_ = -1;   // something may still be written there
   if (e != hipSuccess) return fail(SUB1_ERR_HIP, "%s: %s", who, hipGetErrorString(e));
   return fail(SUB1_ERR_INTERNAL, "%s: the launch has ended without its answer", who);
 }
@@ -996,13 +1039,17 @@ int launch_decode(const int32_t *dec, const int16_t *w_comp, const int32_t *row_
   uint16_t *w = static_cast<uint16_t *>(out_w);
   const int tern_phase = static_cast<int>(reinterpret_cast<uintptr_t>(out_tern) & 3);
   const int w_phase = static_cast<int>((reinterpret_cast<uintptr_t>(out_w) & 7) / 2);
-  if (out_tern && w && tern_phase != w_phase) {
-    launch(out_tern, nullptr, bad_rows, tern_phase);
-    launch(nullptr, w, nullptr, w_phase);
-  } else {
-    launch(out_tern, w, bad_rows, out_tern ? tern_phase : w_phase);
-  }
+  const bool each = out_tern && w && tern_phase != w_phase;
+  launch(out_tern, each ? nullptr : w, bad_rows, out_tern ? tern_phase : w_phase);
   HIP_TRY(hipGetLastError());
+  if (counted) {
+    const int rc = slot.launched(who);
+    if (rc) return rc;
+  }
+  if (each) {
+    launch(nullptr, w, nullptr, w_phase);
+    HIP_TRY(hipGetLastError());
+  }
   if (!counted) return SUB1_OK;
   tell_count_kernel<<<1, 1, 0, s>>>(slot.answer());
   HIP_TRY(hipGetLastError());
@@ -1275,6 +1322,35 @@ extern "C" int sub1_set_wait_limit_us(int64_t microseconds) {
 extern "C" int sub1_test_overstate_wait(int extra) {
   if (extra < 0) return fail(SUB1_ERR_SHAPE, "sub1_test_overstate_wait: negative count");
   sub1::g_expect_extra.store(extra);
+  return SUB1_OK;
+}
+
+extern "C" int sub1_test_fail_answers(int calls) {
+  if (calls < 0) return fail(SUB1_ERR_SHAPE, "sub1_test_fail_answers: negative count");
+  sub1::g_fail_answers.store(calls);
+  return SUB1_OK;
+}
+
+extern "C" int sub1_test_slot_pool(int slots, int lost) {
+  const char *who = "sub1_test_slot_pool";
+  if (lost < 0 || slots <= lost || slots > 4096) return fail(SUB1_ERR_SHAPE, "%s: %d of %d", who, lost, slots);
+  sub1::SlotPool pool(slots);
+  std::vector<int> held;
+  for (int i = 0; i < slots; i++) held.push_back(pool.take());
+  std::sort(held.begin(), held.end());
+  for (int i = 0; i < slots; i++)
+    if (held[i] != i) return fail(SUB1_ERR_INTERNAL, "%s: a slot was handed out twice", who);
+  for (int i = 0; i < lost; i++) pool.lose();
+  int got = -2;
+  std::thread waits([&]() { got = pool.take(); });
+  pool.give_back(held.back());
+  waits.join();
+  if (got != held.back()) return fail(SUB1_ERR_INTERNAL, "%s: %d taken, %d was free", who, got, held.back());
+  got = -2;
+  std::thread waits_for_none([&]() { got = pool.take(); });
+  for (int i = lost; i < slots; i++) pool.lose();
+  waits_for_none.join();
+  if (got != -1 || pool.take() != -1) return fail(SUB1_ERR_INTERNAL, "%s: a lost slot was handed out", who);
   return SUB1_OK;
 }
 

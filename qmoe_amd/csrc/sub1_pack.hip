@@ -601,6 +601,10 @@ int pack_weights(const void *w, uint16_t *codes, void *ter_minmax, int32_t *row_
   a.width = width;
   rc = launch_pack_rows<true>(a, s);
   if (rc) return rc;
+  if (total) {
+    rc = slot.launched(who);
+    if (rc) return rc;
+  }
   row_offset_scan_kernel<<<1, sub1::kScanThreads, 0, s>>>(row_off, height, slot.answer());
   HIP_TRY(hipGetLastError());
   return total ? slot.wait(s, 1, total, who) : SUB1_OK;

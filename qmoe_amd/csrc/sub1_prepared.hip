@@ -2753,6 +2753,7 @@ int prepare_layout(const Source &src, void *meta, int64_t meta_bytes, LayoutResu
   zero_words_kernel<<<1, 64, 0, s>>>(status, 4);
   WalkArgs w{};
   rc = check_on_device(src, status + 3, w, s);
+  if (!rc) rc = slot.launched(who);
   if (rc) return rc;
   int32_t *counts = reinterpret_cast<int32_t *>(base + m.counts);
   w.status = status;
@@ -2825,6 +2826,7 @@ int prepare_codes(const Source &src, const Prepared &p, hipStream_t s, const cha
   zero_words_kernel<<<1, 64, 0, s>>>(found, 1);
   WalkArgs w{};
   rc = check_on_device(src, found, w, s);
+  if (!rc) rc = slot.launched(who);
   if (rc) return rc;
   uint2 *stream = static_cast<uint2 *>(const_cast<void *>(p.codes));
   uint16_t *ckpt = reinterpret_cast<uint16_t *>(stream + p.total_chunks * 64);

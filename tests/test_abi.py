@@ -32,6 +32,23 @@ def test_every_declared_symbol_is_exported_and_bound():
     assert lib.sub1_abi_version() == 4
 
 
+@pytest.mark.parametrize('slots,lost', [(1, 0), (5, 0), (5, 4), (64, 30)])
+def test_nobody_waits_for_a_slot_that_is_lost(slots, lost):
+    import threading
+    lib, status = _lib.load(), []
+    thread = threading.Thread(target=lambda: status.append((lib.sub1_test_slot_pool(slots, lost), lib.sub1_last_error())),
+                              daemon=True)
+    thread.start()
+    thread.join(20)
+    assert status and status[0][0] == 0, status      # no status: it still waits
+
+
+def test_slot_pools_that_make_no_sense_are_refused():
+    lib = _lib.load()
+    for slots, lost in ((0, 0), (3, 3), (3, -1), (5000, 0)):
+        assert lib.sub1_test_slot_pool(slots, lost) != 0
+
+
 def test_header_constants_match_binding():
     text = open(os.path.join(ROOT, 'include', 'sub1_hip.h')).read()
     assert int(re.search(r'#define SUB1_MAX_WIDTH (\d+)', text).group(1)) == _lib.MAX_WIDTH

@@ -340,6 +340,36 @@ def test_what_a_compression_counted_may_be_read_anywhere_once_it_returns(gpu):
         assert total.value == int(want[-1]) and torch.equal(got.flip(0), want) and torch.equal(got_pairs, minmax), i
 
 
+def test_calls_that_end_by_an_error_leave_their_places_as_they_were(gpu):
+    """More of them than there are places, each behind launches that count and store."""
+    from qmoe_amd import synthetic
+    sub1, op = gpu
+    lib = op._lib.load()
+    symbols = symbols_of(40, 300, [0.3], seed=2)
+    w_comp, row_off = packed(gpu, symbols)
+    short = row_off.clone()
+    short[1:7:2] -= 1                       # six bad rows
+    weights = torch.tensor([0.0, -1.0, 1.0], device='cuda')[symbols.long()].bfloat16()
+    whole = op.sub1pack_weights(weights)
+    stack = synthetic.build_stack(2, 96, 160, 0.9, seed=5)
+    calls = (lambda: op.sub1decode(sub1.DEC[0], w_comp, short, None, 300, want_w=False)[2],
+             lambda: op.sub1pack_weights(weights), stack.prepare)
+    try:
+        for call in calls:
+            op._lib.check(lib.sub1_test_fail_answers(70))
+            for _ in range(70):
+                with pytest.raises(op._lib.Sub1Error, match='made to fail'):
+                    call()
+    finally:
+        op._lib.check(lib.sub1_test_fail_answers(0))
+    assert lib.sub1_test_fail_answers(-1) != 0
+    for _ in range(70):
+        assert calls[0]() == 6
+    assert all(torch.equal(a, b) for a, b in zip(calls[1](), whole))
+    x, route = synthetic.activations(4, 96, 6), torch.arange(4, dtype=torch.int32, device='cuda') % 2
+    assert calls[2]().forward(x, route).isfinite().all()
+
+
 FIRST_PACK_IN_A_CAPTURE = r'''
 import ctypes, sys
 sys.path.insert(0, sys.argv[1])
