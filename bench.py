@@ -453,9 +453,8 @@ def main():
     args = ap.parse_args()
     if args.gpus != 1:
         sys.exit('bench.py measures one GPU: this build has no multi-GPU path (--gpus 1 only)')
-    from qmoe_amd import _lib, build as _build
-    if not os.path.exists(_lib.LIB_PATH):      # uses what is built; builds only if nothing is
-        _build.build_library()
+    from qmoe_amd import build as _build
+    _build.build_what_is_missing()      # uses what is built
     import ctypes
     import torch
     from qmoe_amd import _lib, synthetic

@@ -143,9 +143,13 @@ def tensor_args():
     """The extension that looks tensors over (csrc/tensor_args.cpp).  There is no fallback either."""
     global _tensor_args
     if _tensor_args is None:
-        import torch  # noqa: F401  (its libraries first)
+        from . import build
+        wanted = build.torch_mark()     # (imports torch: its libraries first)
         try:
             from . import _tensor_args as module
+            found = getattr(module, 'built_against', 'no torch that it names')
+            if found != wanted:
+                raise ImportError('it is of %r, this is %r' % (found, wanted))
         except ImportError as e:
             raise ImportError('qmoe_amd/_tensor_args.so is missing or of another torch: build it with '
                               '`python -m qmoe_amd.build` (%s)' % e) from e

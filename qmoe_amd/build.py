@@ -44,12 +44,19 @@ def kernels_with_scratch(compiler_output):
 SPILLS_ACCEPTED = {'_ZN12_GLOBAL__N_125moe_prepared_fused_kernelILb1ELb0EEEvNS_12PreparedArgsE': 36}
 
 
+def torch_mark():
+    """What the extension says of the torch that it was built against, of the one installed."""
+    import torch
+    return 'qmoe_amd, built against torch ' + torch.__version__
+
+
 def build_tensor_args():
     """Builds the extension module against the installed torch's headers."""
     import torch
     from torch.utils import cpp_extension
     cmd = [os.environ.get('CXX', 'g++'), '-O2', '-fPIC', '-shared', '-std=c++17', '-fvisibility=hidden',
            '-D_GLIBCXX_USE_CXX11_ABI=%d' % torch._C._GLIBCXX_USE_CXX11_ABI,
+           '-DSUB1_TORCH_VERSION="%s"' % torch.__version__,
            os.path.join(HERE, 'csrc', 'tensor_args.cpp')]
     cmd += ['-isystem' + path for path in cpp_extension.include_paths() + [sysconfig.get_paths()['include']]]
     cmd += ['-L' + path for path in cpp_extension.library_paths()]
@@ -83,6 +90,24 @@ def build_library(verbose=False):
         print('\n'.join(l for l in res.stdout.splitlines() if 'kernel-resource-usage' not in l
                         and not l.lstrip().startswith(('|', '^')) and '__global__' not in l))
     return LIB_PATH
+
+
+def tensor_args_fit():
+    """Whether the extension is there and of the installed torch (looked up in the file: a
+    module that has been loaded cannot be loaded again once it is rebuilt)."""
+    try:
+        with open(TENSOR_ARGS_PATH, 'rb') as f:
+            return torch_mark().encode() + b'\0' in f.read()
+    except FileNotFoundError:
+        return False
+
+
+def build_what_is_missing():
+    """For programs that use what is built: builds only what is not there."""
+    if not os.path.exists(LIB_PATH):
+        build_library()
+    elif not tensor_args_fit():
+        build_tensor_args()
 
 
 if __name__ == '__main__':

@@ -140,4 +140,16 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_tensor_args", nullptr, -1, kMeth
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__tensor_args() { return PyModule_Create(&kModule); }
+#ifndef SUB1_TORCH_VERSION
+#error "the build says which torch these headers are of"
+#endif
+// The classes behind a tensor differ from one torch to the next and nothing in the library's symbols
+// says so: whoever loads the module compares this with the torch it has.
+PyMODINIT_FUNC PyInit__tensor_args() {
+  PyObject *module = PyModule_Create(&kModule);
+  if (module && PyModule_AddStringConstant(module, "built_against", "qmoe_amd, built against torch " SUB1_TORCH_VERSION) < 0) {
+    Py_DECREF(module);
+    return nullptr;
+  }
+  return module;
+}

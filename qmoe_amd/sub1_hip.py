@@ -1,7 +1,8 @@
 """Operator module with the surface of the reference's `sub1_cuda` extension
 (reference sub1_cuda.cpp:56-59): `sub1matvec` and `sub1pack`, same positional
 arguments, tensors in, launched on torch's current stream.  Underneath is the C
-ABI of libsub1_hip.so; torch only supplies device memory and the stream.
+ABI of libsub1_hip.so; torch supplies device memory, the stream and, through the
+extension _tensor_args, the tensors' addresses.
 
     import qmoe_amd.sub1_hip as sub1_cuda      # drop-in for `import sub1_cuda`
 

@@ -10,12 +10,10 @@ if ROOT not in sys.path:
 
 def pytest_configure(config):
     config.addinivalue_line('markers', 'gpu: needs a real MI355X (run with -m gpu)')
-    # The package refuses to import without its library (there is no CPU
+    # The package refuses to import without its libraries (there is no CPU
     # fallback).  The tests use what is built and build only if nothing is.
-    from qmoe_amd import _lib
-    if not os.path.exists(_lib.LIB_PATH):
-        from qmoe_amd import build
-        build.build_library()
+    from qmoe_amd import build
+    build.build_what_is_missing()
 
 
 @pytest.fixture(scope='session')
