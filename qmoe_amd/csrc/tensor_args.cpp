@@ -104,7 +104,7 @@ PyObject *layer_addresses(PyObject *, PyObject *const *args, Py_ssize_t n) {
   try {
     const at::Tensor &t = THPVariable_Unpack(args[0]);
     if (!t.defined() || !t.is_cpu() || t.scalar_type() != at::kLong || t.dim() != 2 || !t.is_contiguous() ||
-        t.size(1) != count || row < 0 || row + columns > t.size(0))
+        t.size(1) != count || row < 0 || row > t.size(0) - columns)
       Py_RETURN_FALSE;
     table = static_cast<int64_t *>(t.data_ptr()) + row * count;
   } catch (...) {

@@ -26,6 +26,43 @@ def test_nothing_but_plain_gpu_tensors_goes_by_its_address():
         assert fill(*args) is False
 
 
+def with_one_changed(args, changes):
+    for at, values in changes.items():
+        for value in values:
+            yield args[:at] + (value,) + args[at + 1:]
+
+
+@pytest.mark.gpu
+def test_each_argument_is_looked_at_where_the_tensors_are_in_order():
+    """What is refused here is refused for the one thing that is wrong with it."""
+    good = (torch.zeros(2, 4, dtype=torch.bfloat16, device='cuda'), torch.zeros(3, dtype=torch.int32, device='cuda'))
+    look, fill = _lib.tensor_args().addresses, _lib.tensor_args().layer_addresses
+    addresses = [t.data_ptr() for t in good]
+    numels = [(8,), (8, 3, 1), [8, 3], (None, 3), (1 << 70, 3), (8.0, 3), (7, 3), (8, 4), None]
+    devices = [None, 1, -1, 0.0, 1 << 70, torch.device('cuda:0')]
+    specs = [SPEC[:1], SPEC * 2, list(SPEC), (SPEC[0], SPEC[1][:2]), (SPEC[0], list(SPEC[1])), (SPEC[0], (1, 'b', -1)),
+             (SPEC[0], (torch.int64, 'b', -1)), (SPEC[0], (torch.int32, 'b', 2)), (SPEC[0], (torch.int32, 'b', None)), None]
+
+    args = (SPEC, good, (8, 3), 0)
+    assert list(look(*args)) == addresses
+    for broken in with_one_changed(args, {0: specs, 1: [good[:1], list(good), good + good, None], 2: numels, 3: devices}):
+        assert look(*broken) is None, broken
+
+    table = torch.full((5, 2), -7, dtype=torch.int64)
+    args = (table, 1, [good, good], SPEC, (8, 3), 0)
+    assert fill(*args) is True
+    assert table.tolist() == [[-7, -7], [addresses[0]] * 2, [addresses[1]] * 2, [-7, -7], [-7, -7]]
+    assert fill(table, 3, *args[2:]) is True and table[3:].tolist() == table[1:3].tolist()      # the last rows
+    table.fill_(-7)
+    wide = torch.full((5, 4), -7, dtype=torch.int64)
+    other = [table.int(), table.double(), table.view(-1), table[None], wide, wide[:, ::2], table.cuda(), table.as_subclass(Wrapped),
+             table[:2], None]
+    layers = [(good, good), [good], [good] * 3, [good, good[:1]], [good, list(good)], [good, good + good], [good, None], None]
+    for broken in with_one_changed(args, {0: other, 1: [4, 5, 1 << 40, (1 << 63) - 1, -1, None, 1.0], 2: layers, 3: specs, 4: numels, 5: devices}):
+        assert fill(*broken) is False, broken
+    assert (wide == -7).all() and (table[0] == -7).all() and (table[3:] == -7).all()
+
+
 @pytest.mark.gpu
 def test_addresses_and_refusals_are_those_of_the_slow_way():
     dev = torch.device('cuda:0')
