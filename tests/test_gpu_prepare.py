@@ -370,6 +370,26 @@ def test_calls_that_end_by_an_error_leave_their_places_as_they_were(gpu):
     assert calls[2]().forward(x, route).isfinite().all()
 
 
+@pytest.mark.parametrize('height,width', [(1, 1), (70, 200), (1025, 31), (4100, 16)])
+def test_counting_without_waiting_gives_what_counting_with_it_does(gpu, height, width):
+    import ctypes
+    _, op = gpu
+    lib, stream = op._lib.load(), torch.cuda.current_stream().cuda_stream
+    weights = torch.tensor([0.0, -1.5, 2.0], device='cuda')[symbols_of(height, width, [0.2, 0.9], seed=4).long()].bfloat16()
+    results, total = [], ctypes.c_int32(-1)
+    for function, extra in ((lib.sub1_pack_weights_count, ()), (lib.sub1_pack_weights_total, (ctypes.byref(total),))):
+        codes = torch.zeros((height, (width + 1) // 2), dtype=torch.int16, device='cuda')
+        minmax, row_off = torch.zeros(2 * height, dtype=torch.bfloat16, device='cuda'), torch.zeros(height + 1, dtype=torch.int32, device='cuda')
+        assert function(weights.data_ptr(), codes.data_ptr(), minmax.data_ptr(), row_off.data_ptr(), *extra, height, width, stream) == 0
+        w_comp = torch.zeros(int(row_off[height]), dtype=torch.int16, device='cuda')
+        assert lib.sub1_pack_weights_emit(codes.data_ptr(), row_off.data_ptr(), w_comp.data_ptr(), height, width, stream) == 0
+        results.append((row_off, minmax, w_comp))
+    assert total.value == results[0][2].numel() > 0
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+    w_comp, row_off, minmax = op.sub1pack_weights(weights)
+    assert all(torch.equal(a, b) for a, b in zip(results[0], (row_off, minmax, w_comp)))
+
+
 FIRST_PACK_IN_A_CAPTURE = r'''
 import ctypes, sys
 sys.path.insert(0, sys.argv[1])
