@@ -3423,8 +3423,19 @@ constexpr size_t kBatchLds = 160 * 1024 - 64;
 // ones without a group of chunks for its multiplying alone (95 % zeros, sharing by chunks alone:
 // 128 base experts on 4096 tokens 166 us against 128) - nor where small workgroups with a table each
 // leave room for too few: then one holds all the slices that fit (base wo by one slice of four
-// wavefronts, two of those to a unit, 82 us, by one of eight 67, by three of four 65).  A table that
-// does not fit beside a single slice, of rows of more than 9000 columns, stays in global memory.
+// wavefronts, two of those to a unit, 82 us, by one of eight 67, by three of four 65).
+//
+// Where two slices fit beside one table and two workgroups with a table each do not (wo of about
+// 4500 to 4730 columns), one workgroup of 16 wavefronts takes both (58 experts of 1000 x 4600, 92 % zeros,
+// 9 and 64 tokens an expert: by one slice of twelve 104 and 177 us, by two of eight 87 and 158) - unless
+// one slice is much longer than the others, which the other one's wavefronts then wait for, and the layer
+// has not two for every compute unit (12 experts of 1500 x 4650, shares of zeros that differ from row
+// to row, 72 and 79 us; 58 of 1000 x 4600 155 and 142).  Where two slices fit only without a table (up to
+// about 5050), the table stays in global memory for two workgroups of a slice, if the layer has two for
+// every compute unit and no slice is much longer, one long chain of looks into it (55 experts of
+// 1000 x 4800, 92 % zeros 172 and 150 us, 80 % 206 and 195, differing shares 226 and 232; 20 experts of
+// 1000 x 5030, 85 % 63 and 67).  A table that does not fit beside a single slice, of rows of more than
+// 9000 columns, stays there too.
 bool plan_batch(const Prepared &p, int kind, size_t lds_limit, BatchPlan *out) {
   const int slices[2] = {(p.height[0] + 63) / 64, (p.height[1] + 63) / 64};
   const double weight = static_cast<double>(slices[0]) * p.width[0] + static_cast<double>(slices[1]) * p.width[1];
@@ -3432,10 +3443,20 @@ bool plan_batch(const Prepared &p, int kind, size_t lds_limit, BatchPlan *out) {
   const size_t code_bytes = slice_code_bytes(product_steps(p, kind));
   // (wi needs no table)
   const size_t wanted = kind ? table_bytes(p.width[kind]) : 0;
-  out->table_in_lds = code_bytes + wanted <= lds_limit;
+  const bool even = p.max_chunks[kind] <= 2.0 * chunks;
+  const bool many = static_cast<int64_t>(p.count) * slices[kind] >= 2 * 256;
+  const bool pair = 2 * code_bytes <= lds_limit;
+  out->table_in_lds = code_bytes + wanted <= lds_limit &&
+                      !(pair && 2 * code_bytes + wanted > lds_limit && even && many);
   const size_t table = out->table_in_lds ? wanted : 0;
   if (code_bytes + table > lds_limit) return false;
   const int fit = static_cast<int>((lds_limit - table) / code_bytes);
+  if (fit == 2 && 2 * (code_bytes + table) > lds_limit && slices[kind] > 1 && (even || many)) {
+    out->per_group = 2;
+    out->parts = 8;
+    out->lds = 2 * code_bytes + table;
+    return true;
+  }
   int waves = fit >= 3 ? 4 : fit == 2 ? 8 : 12;
   for (int parts = 1;; parts *= 2) {
     if (parts > waves) parts = waves;

@@ -93,6 +93,31 @@ def test_wherever_the_table_of_columns_lies(oracle, d_model, d_ff):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('d_model,d_ff,copies,plan', [
+    (100, 4600, 1, (2, 8)), (113, 4530, 1, (2, 8)),       # both slices in one workgroup of sixteen wavefronts
+    (50, 4600, 1, (1, 12)),                               # one slice alone
+    (130, 4700, 1, (2, 8)),                               # three slices: the second workgroup has one
+    (66, 4800, 128, (1, 8)), (66, 4800, 127, (1, 12)),    # a table in global memory; slices too few for that
+    (66, 5040, 128, (1, 8)), (66, 5060, 128, (1, 12))])
+def test_two_slices_and_a_table_that_do_not_fit_twice(oracle, d_model, d_ff, copies, plan):
+    """Exact sums, as above (130 x 4700 has few enough weights for that at 90 % zeros)."""
+    wi = [layers(oracle, d_ff, d_model, 0.9, 50 + e) for e in range(2)]
+    wo = [layers(oracle, d_model, d_ff, 0.9, 60 + e) for e in range(2)]
+    prep = prepared(wi * copies, wo * copies)
+    assert batch_plan(prep._c, 1)[:2] == plan
+    last = 2 * copies - 1
+    route = np.repeat(np.int32([last, 0, -1, last // 2]), [70, 33, 2, 3])
+    xs = so.f32_to_bf16_bits(np.random.default_rng(6).integers(-2, 3, (route.size, d_model)).astype(np.float32))
+    x, te = bf16_dev(xs), torch.from_numpy(route).cuda()
+    y = prep.forward_batch(x, te)
+    assert torch.equal(prep.forward(x, te), y)
+    got = bits_host(y)
+    for i in (0, 69, 70, 102, 105, 107):
+        e = route[i] % 2
+        assert np.array_equal(got[i], oracle.expert_ffn(wi[e], wo[e], xs[i], order=2)[0]), i
+
+
+@pytest.mark.gpu
 def test_a_token_without_finite_activations_spoils_no_other(oracle):
     """x with an infinity or a NaN, and x whose h overflows: what the walking kernel
     gives for the token alone; the tokens of its block are as without it."""
