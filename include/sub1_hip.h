@@ -355,9 +355,10 @@ int sub1_moe_grouped_prepared(const sub1_moe_prepared *prepared, const int32_t *
  * aligned, contents arbitrary before and after (0: no such form for these shapes - a
  * row's codes must fit LDS - and the call is refused).  An expert's tokens take
  * whole blocks of 32 slots: at most tokens + 31 (min(tokens, experts) + 1) slots, of
- * 4 d_ff + 2 d_model bytes (widths rounded up to 16) and 17 more each - 69 MB for 1024 tokens
- * of 128 experts with d_model 768 and d_ff 3072, 112 MB for 4096.  It stops growing at
- * 8192 tokens: larger batches run in equal pieces.
+ * 2 d_ff + 2 d_model bytes (d_ff rounded up to 64, d_model to 16) and 9 more each - 39 MB for
+ * 1024 tokens of 128 experts with d_model 768 and d_ff 3072, 62 MB for 4096 - and, of layers with
+ * 4700 to 5050 and with more than 9000 columns in wo, 2.2 d_ff bytes an expert.  It stops growing
+ * at 8192 tokens: larger batches run in equal pieces.
  *
  * sub1_moe_batch_pays: 1 where this is estimated to be faster than
  * sub1_moe_grouped_prepared for `tokens` tokens spread over the experts, 0 otherwise.  Every

@@ -1047,7 +1047,11 @@ int parts_of(int blocks, int windows) {
 // which a compute unit holds at once.  One of them takes start + turn us a window of its part; each
 // further one on the unit makes `beside` of the windows' time more.  Fitted to 14 shapes, the
 // six of Switch among them, on 64 to 2272 tokens (rms 4 to 15 %, the larger ones where 10 us of host
-// calls hide the kernel); the form estimated fastest is within 2 % of the fastest on average.
+// calls hide the kernel), before columns of 128 tokens were evened out (columns_of), which made those
+// faster than the estimate knows.  Of 168 launches now (12 shapes, the six among them, 64 to 2272
+// tokens) the form picked is 3.7 % off the fastest on average; 49 are off by more than 5 %: 26 on blocks of
+// 64 tokens where 128 would do, by up to 21 % (c-2048 wi on 720 tokens 28.5 us, 23.6 in blocks of 128; large
+// wi on 1136 16.3 and 13.9), the others by up to 10 %.
 struct TileForm {
   int parts, groups, blocks, held;
   double start, turn, beside;
