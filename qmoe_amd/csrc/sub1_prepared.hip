@@ -3423,7 +3423,12 @@ constexpr size_t kBatchLds = 160 * 1024 - 64;
 // ones without a group of chunks for its multiplying alone (95 % zeros, sharing by chunks alone:
 // 128 base experts on 4096 tokens 166 us against 128) - nor where small workgroups with a table each
 // leave room for too few: then one holds all the slices that fit (base wo by one slice of four
-// wavefronts, two of those to a unit, 82 us, by one of eight 67, by three of four 65).
+// wavefronts, two of those to a unit, 82 us, by one of eight 67, by three of four 65) - if that divides
+// the slices and four wavefronts are enough for one; else two workgroups of one slice and eight wavefronts
+// share the unit (28 layers of 9 to 33 slices, rows of 3072 to 3152 columns, 9 to 64 tokens an expert: by
+// three of four 1.02 to 1.17 times the time where 3 does not divide the slices, so that the last
+// workgroup of an expert has places empty, 0.98 to 1.12 where it does; 50 experts of 2000 x 3100, 88 %
+// zeros 200 us and 182).
 //
 // Where two slices fit beside one table and two workgroups with a table each do not (wo of about
 // 4500 to 4730 columns), one workgroup of 16 wavefronts takes both (58 experts of 1000 x 4600, 92 % zeros,
@@ -3432,9 +3437,9 @@ constexpr size_t kBatchLds = 160 * 1024 - 64;
 // has not two for every compute unit (12 experts of 1500 x 4650, shares of zeros that differ from row
 // to row, 72 and 79 us; 58 of 1000 x 4600 155 and 142).  Where two slices fit only without a table (up to
 // about 5050), the table stays in global memory for two workgroups of a slice, if the layer has two for
-// every compute unit and no slice is much longer, one long chain of looks into it (55 experts of
-// 1000 x 4800, 92 % zeros 172 and 150 us, 80 % 206 and 195, differing shares 226 and 232; 20 experts of
-// 1000 x 5030, 85 % 63 and 67).  A table that does not fit beside a single slice, of rows of more than
+// every compute unit, no slice is much longer, one long chain of looks into it, and the entries are few
+// (55 experts of 1000 x 4800, 92 % zeros 172 and 150 us, 80 % 206 and 195, 70 % 210 and 227, differing
+// shares 226 and 232; 20 experts of 1000 x 5030, 85 % 63 and 67).  A table that does not fit beside a single slice, of rows of more than
 // 9000 columns, stays there too.
 bool plan_batch(const Prepared &p, int kind, size_t lds_limit, BatchPlan *out) {
   const int slices[2] = {(p.height[0] + 63) / 64, (p.height[1] + 63) / 64};
@@ -3443,11 +3448,11 @@ bool plan_batch(const Prepared &p, int kind, size_t lds_limit, BatchPlan *out) {
   const size_t code_bytes = slice_code_bytes(product_steps(p, kind));
   // (wi needs no table)
   const size_t wanted = kind ? table_bytes(p.width[kind]) : 0;
-  const bool even = p.max_chunks[kind] <= 2.0 * chunks;
+  const bool even = p.max_chunks[kind] <= 2.0 * chunks, few = chunks * kFields <= 0.25 * p.width[kind];
   const bool many = static_cast<int64_t>(p.count) * slices[kind] >= 2 * 256;
   const bool pair = 2 * code_bytes <= lds_limit;
   out->table_in_lds = code_bytes + wanted <= lds_limit &&
-                      !(pair && 2 * code_bytes + wanted > lds_limit && even && many);
+                      !(pair && 2 * code_bytes + wanted > lds_limit && even && few && many);
   const size_t table = out->table_in_lds ? wanted : 0;
   if (code_bytes + table > lds_limit) return false;
   const int fit = static_cast<int>((lds_limit - table) / code_bytes);
@@ -3473,6 +3478,12 @@ bool plan_batch(const Prepared &p, int kind, size_t lds_limit, BatchPlan *out) {
     if (static_cast<int>(lds_limit / out->lds) * per_group * parts >= 12) return true;
     if (parts == waves) {
       if (waves == 12) return true;
+      if (waves == 4 && (slices[kind] % fit || waves * kGroupChunks < 0.75 * chunks) && 2 * (code_bytes + table) <= lds_limit) {
+        out->per_group = 1;
+        out->parts = 8;
+        out->lds = std::max(code_bytes + table, static_cast<size_t>(2 * 8) * 4096);
+        return true;
+      }
       waves = 12;   // and look on from as many parts
       parts /= 2;
     }

@@ -98,11 +98,13 @@ def test_wherever_the_table_of_columns_lies(oracle, d_model, d_ff):
     (50, 4600, 1, (1, 12)),                               # one slice alone
     (130, 4700, 1, (2, 8)),                               # three slices: the second workgroup has one
     (66, 4800, 128, (1, 8)), (66, 4800, 127, (1, 12)),    # a table in global memory; slices too few for that
-    (66, 5040, 128, (1, 8)), (66, 5060, 128, (1, 12))])
+    (66, 5040, 128, (1, 8)), (66, 5060, 128, (1, 12)),
+    (150, 3072, 1, (3, 4)), (250, 3072, 1, (1, 8)),       # three slices fill a workgroup, four do not
+    (300, 3150, 1, (1, 8))])
 def test_two_slices_and_a_table_that_do_not_fit_twice(oracle, d_model, d_ff, copies, plan):
-    """Exact sums, as above (130 x 4700 has few enough weights for that at 90 % zeros)."""
-    wi = [layers(oracle, d_ff, d_model, 0.9, 50 + e) for e in range(2)]
-    wo = [layers(oracle, d_model, d_ff, 0.9, 60 + e) for e in range(2)]
+    """Exact sums, as above (at 93 % zeros the wider ones have few enough weights for that)."""
+    wi = [layers(oracle, d_ff, d_model, 0.93, 50 + e) for e in range(2)]
+    wo = [layers(oracle, d_model, d_ff, 0.93, 60 + e) for e in range(2)]
     prep = prepared(wi * copies, wo * copies)
     assert batch_plan(prep._c, 1)[:2] == plan
     last = 2 * copies - 1
