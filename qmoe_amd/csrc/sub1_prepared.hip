@@ -3551,13 +3551,13 @@ double blocks_on_average(double each, int per) {
 // and of three odd ones, with 80 to 95 % zeros (168 launches).  Here, for every piece of a batch,
 // which expands every expert that it hits: 35 and, per million weights, 0.29 times the entries
 // of a weight for every 64 of an expert's tokens, 0.08 for every 32 (within 11 %, root mean
-// square; on the 700 below 11 % low on average, within 12 %).  Walking: a compute unit takes
+// square; on the 1300 below 11 % low on average, within 13 %).  Walking: a compute unit takes
 // token_us = 8 + entries / 23400 for a token and, where launch_prepared groups tokens by expert,
 // 7 + 1.85 (token_us - 8) for up to four, in whole rounds.  The matrix cores must promise 5 %: of those
 // launches that leaves none on the slower way, and 18 where they would have been faster, by up to 44 %.
-// Of 700 others (70 layers of 4 to 300 experts, Switch shapes and odd ones, 80 to 95 % zeros or shares that
-// differ from row to row, 8 to 48 tokens an expert) 2 go the slower way, by 1 %, and 77 walk that would be
-// faster here, 48 of them by more than 10 % and one by 83 %: few experts or uneven rows, whose walking
+// Of 1300 others (130 layers of 4 to 300 experts, Switch shapes and odd ones, 80 to 95 % zeros or shares that
+// differ from row to row, 8 to 48 tokens an expert) 3 go the slower way, by 3 % at most, and 137 walk that
+// would be faster here, 90 of them by more than 10 % and one by 98 %: few experts or uneven rows, whose walking
 // is estimated low (a quarter on average; 38 us for 140 tokens through 7 uneven large experts, which take
 // 125, and 68 here).  A piece with less than 8 tokens an expert never goes there.  (Pricing one pass over
 // the experts for a batch that runs in pieces, as it was done first, sent 32 768 tokens through 2048 base
