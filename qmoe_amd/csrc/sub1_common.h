@@ -227,6 +227,46 @@ __device__ __forceinline__ void leave_launch(int32_t *ctrl, int workgroups) {
   }
 }
 
+// dpp_ctrl values of the row shifts, the shift by a lane and the row broadcasts (CDNA ISA, DPP)
+constexpr int kDppRowShr1 = 0x111, kDppRowShr2 = 0x112, kDppRowShr4 = 0x114, kDppRowShr8 = 0x118;
+constexpr int kDppWaveShr1 = 0x138, kDppBcast15 = 0x142, kDppBcast31 = 0x143;
+
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ int dpp_or_zero(int v) {
+  // lanes outside the row mask and lanes whose source lies outside the row get 0
+  return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRowMask, 0xf, false);
+}
+
+// Inclusive prefix sum over the 64 lanes.
+__device__ __forceinline__ int wave_prefix_sum(int v) {
+  v += dpp_or_zero<kDppRowShr1, 0xf>(v);
+  v += dpp_or_zero<kDppRowShr2, 0xf>(v);
+  v += dpp_or_zero<kDppRowShr4, 0xf>(v);
+  v += dpp_or_zero<kDppRowShr8, 0xf>(v);
+  v += dpp_or_zero<kDppBcast15, 0xa>(v);   // row 0 -> row 1, row 2 -> row 3
+  v += dpp_or_zero<kDppBcast31, 0xc>(v);   // rows 0-1 -> rows 2-3
+  return v;
+}
+
+// The largest value of the lanes below, of values that are not negative (lane 0: 0).
+__device__ __forceinline__ int wave_max_below(int v) {
+  v = max(v, dpp_or_zero<kDppRowShr1, 0xf>(v));
+  v = max(v, dpp_or_zero<kDppRowShr2, 0xf>(v));
+  v = max(v, dpp_or_zero<kDppRowShr4, 0xf>(v));
+  v = max(v, dpp_or_zero<kDppRowShr8, 0xf>(v));
+  v = max(v, dpp_or_zero<kDppBcast15, 0xa>(v));
+  v = max(v, dpp_or_zero<kDppBcast31, 0xc>(v));
+  return dpp_or_zero<kDppWaveShr1, 0xf>(v);
+}
+
+__device__ __forceinline__ void wave_lds_fence() {
+  // LDS accesses of a wavefront take place in program order; this keeps the
+  // compiler to it across lanes
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // In-place inclusive prefix sum over v[1..n], v[0] = 0, by one workgroup of
 // kScanThreads: 4096 values a turn, the next turn's loads in flight behind it
 // (a thread with a run of its own, as it was first, reads every line 64 times).

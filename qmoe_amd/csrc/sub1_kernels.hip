@@ -231,6 +231,7 @@ using sub1::f32_to_bf16;
 using sub1::fail;
 using sub1::misaligned;
 using sub1::row_result;
+using sub1::wave_prefix_sum;
 
 // ------------------------------------------------------------ slot table ---
 //
@@ -350,28 +351,9 @@ __device__ __forceinline__ uint32_t table_word(const uint32_t *__restrict__ tab,
 // fused multiply-add each; then six butterfly steps, lane l adding lane l ^ m
 // for m = 1, 2, 4, 8, 16, 32; bf16; y += in bf16.
 
-// dpp_ctrl values of the row shifts and row broadcasts (CDNA ISA, DPP)
-constexpr int kDppRowShr1 = 0x111, kDppRowShr2 = 0x112, kDppRowShr4 = 0x114, kDppRowShr8 = 0x118;
-constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;
+// dpp_ctrl values (CDNA ISA, DPP)
 constexpr int kDppQuadXor1 = 0xb1, kDppQuadXor2 = 0x4e;      // quad_perm [1,0,3,2], [2,3,0,1]
 constexpr int kDppHalfMirror = 0x141, kDppRowMirror = 0x140;
-
-template <int kCtrl, int kRowMask>
-__device__ __forceinline__ int dpp_or_zero(int v) {
-  // lanes outside the row mask and lanes whose source lies outside the row get 0
-  return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRowMask, 0xf, false);
-}
-
-// Inclusive prefix sum over the 64 lanes.
-__device__ __forceinline__ int wave_prefix_sum(int v) {
-  v += dpp_or_zero<kDppRowShr1, 0xf>(v);
-  v += dpp_or_zero<kDppRowShr2, 0xf>(v);
-  v += dpp_or_zero<kDppRowShr4, 0xf>(v);
-  v += dpp_or_zero<kDppRowShr8, 0xf>(v);
-  v += dpp_or_zero<kDppBcast15, 0xa>(v);   // row 0 -> row 1, row 2 -> row 3
-  v += dpp_or_zero<kDppBcast31, 0xc>(v);   // rows 0-1 -> rows 2-3
-  return v;
-}
 
 template <int kCtrl>
 __device__ __forceinline__ float dpp_float(float v) {

@@ -29,6 +29,7 @@ namespace {
 
 using sub1::fail;
 using sub1::misaligned;
+using sub1::wave_lds_fence;
 
 // ------------------------------------------------ the dictionary by string --
 
@@ -183,14 +184,6 @@ constexpr int kLookahead = 2 * kMaxPairs;   // symbols past a place that decide 
 __host__ __device__ constexpr int plane_words(int window) { return (2 * window + kLookahead + 31) / 32 + 1; }
 __host__ __device__ constexpr size_t pack_lds_per_wave(int window) {
   return static_cast<size_t>(2 * plane_words(window)) * 4 + (static_cast<size_t>(window) * 2 + 15) / 16 * 16;
-}
-
-__device__ __forceinline__ void wave_lds_fence() {
-  // LDS accesses of a wavefront take place in program order; this keeps the
-  // compiler to it across lanes
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 __device__ __forceinline__ uint32_t plane_bits(const uint32_t *plane, int at) {

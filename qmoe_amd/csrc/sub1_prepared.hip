@@ -82,13 +82,15 @@ struct KindMeta {
   int height, width;
 };
 
+constexpr int kStatusWords = 64, kStatusLong = 5, kLongBits = 32 * (kStatusWords - kStatusLong);
 struct MetaLayout {
   KindMeta k[2];
   int kinds;
   int64_t counts;       // i32 [all slices + 1] chunk counts, scanned in place
-  int64_t status;       // i32 [4]: [0] rows whose codes do not cover the width, [1], [2]
+  int64_t status;       // i32 [kStatusWords]: [0] rows whose codes do not cover the width, [1], [2]
                         // longest slice of kind 0 / 1 in chunks, [3] what check_on_device
-                        // found
+                        // found, [4] whether there are long rows (counting); from [5] on a bit for
+                        // every slice, mod kLongBits, that has some (emitting)
   int64_t bytes;
 };
 
@@ -122,7 +124,7 @@ MetaLayout meta_layout(int experts, int kinds, const int height[2], const int wi
   }
   m.counts = take((nslices + 1) * 4);
   for (int i = 0; i < kinds; i++) m.k[i].slice_base = m.counts + first[i] * 4;
-  m.status = take(16);
+  m.status = take(kStatusWords * 4);
   m.bytes = off;
   return m;
 }
@@ -177,12 +179,16 @@ struct KindSource {
   const uint32_t *const *minmax_of;
 };
 
+// A row of more than twice its matrix's average of codes (and a few) is a LONG one.
+constexpr int kLongRowsFrom = 16;
 __device__ __forceinline__ const uint16_t *row_codes(const KindSource &ks, int e, int r,
-                                                     int height, int width, int &n) {
+                                                     int height, int width, int &n, bool &is_long) {
   const int32_t *ro = ks.row_off_of ? ks.row_off_of[e]
                                     : ks.row_off + static_cast<int64_t>(e) * (height + 1);
   n = ro[r + 1] - ro[r];
-  if (n < 1 || n > (width + 1) / 2) n = 0;   // counted as a bad row by count_entries_kernel
+  if (n < 1 || n > (width + 1) / 2) n = 0;   // counted as a bad row by walk_rows_kernel
+  // (the sixteen: short rows stay with the lanes; in floating point, which a division costs less in)
+  is_long = n > kLongRowsFrom && static_cast<float>(n - kLongRowsFrom) * height > 2.f * static_cast<float>(ro[height]);
   const uint16_t *codes = ks.w_comp_of ? ks.w_comp_of[e]
                                        : ks.w_comp + (ks.code_base ? ks.code_base[e] : 0);
   return codes + ro[r];
@@ -193,6 +199,10 @@ __device__ __forceinline__ const uint16_t *row_codes(const KindSource &ks, int e
 // gather from a table in global memory costs a compute unit 54 ns, one from LDS 3 ns.
 // So a compute unit takes one workgroup, persistent, that keeps a table in LDS, and a
 // lane asks for eight codes and their eight entries at once.
+//
+// A wavefront of rows takes as long as the longest of them, and a row without zeros has
+// seven times the codes of others.  Long rows are therefore left aside: order_rows_kernel counts
+// them before it orders the rows, emit_long_rows_kernel emits them, a lane to eight of their codes.
 //
 // Counting needs little of an entry, 16 bits, so that all 65 536 are held, and beside
 // them two more bits of each for the rare gap that takes several steps:
@@ -282,8 +292,16 @@ __device__ __forceinline__ void walk_codes(const Table &table, const uint16_t *r
 // A row's non-zeros as entries.  An entry is the step from the row's position (0 at
 // the start) to the next, 0..127; a longer gap goes over zero columns, as far as each
 // step reaches: the place that such a step ends at.
-__device__ __forceinline__ int farthest_zero(int at) {
+constexpr int kZeroStep = kMaxStep / (2 * kZeroPeriod) * (2 * kZeroPeriod);   // from one zero column as far as a step goes
+__host__ __device__ constexpr int farthest_zero(int at) {
   return (at + kMaxStep) / (2 * kZeroPeriod) * (2 * kZeroPeriod);
+}
+// Entries before the last one of a gap: while the target is too far, to the farthest zero
+// column; from the second such step on they are of one length.
+__host__ __device__ constexpr int steps_between(int at, int target) {
+  if (target - at <= kMaxStep) return 0;
+  const int rest = target - farthest_zero(at) - kMaxStep;
+  return 1 + (rest > 0 ? (rest + kZeroStep - 1) / kZeroStep : 0);
 }
 // The position of 2 column + symbol - 1.  (Written out: the compiler takes one more.)
 __device__ __forceinline__ int position_at(int a) {
@@ -314,8 +332,10 @@ struct WalkArgs {
   const uint32_t *table;         // the emitting pass's words, all of them
   const uint32_t *count_table;   // what the counting pass holds in LDS
   const int32_t *found;          // what check_source_kernel has found: nothing is followed unless zero
+  uint32_t *long_bits;           // emitting: long rows are another launch's, and these slices have some (NULL: they are not)
   sub1::Answer answer;           // emitting: the first word says what that is
   int32_t *status;
+  int32_t *any_long;             // counting sets it (zero before) where it has left long rows
   uint2 *stream;
   uint16_t *ckpt;
 };
@@ -329,7 +349,7 @@ constexpr int kLongGap = 60;
 // non-zeros are 27 columns apart at most, so only the gap before the first of them can
 // take more than one.
 __device__ __forceinline__ void count_rows(const CountTable &table, const WalkKind &k, int count,
-                                           int64_t task, int32_t *status) {
+                                           int64_t task, int32_t *status, int32_t *any_long) {
   // rows of a task: from row `first` of a matrix on, and of the next ones
   const int64_t g = task * 64 + (threadIdx.x & 63);
   if (g >= static_cast<int64_t>(count) * k.height) return;
@@ -338,7 +358,12 @@ __device__ __forceinline__ void count_rows(const CountTable &table, const WalkKi
   const int e = first_e + static_cast<int>(past / static_cast<uint32_t>(k.height));
   const int r = static_cast<int>(past % static_cast<uint32_t>(k.height));
   int n;
-  const uint16_t *codes = row_codes(k.source, e, r, k.height, k.width, n);
+  bool is_long;
+  const uint16_t *codes = row_codes(k.source, e, r, k.height, k.width, n, is_long);
+  if (is_long) {
+    *any_long = 1;
+    return;
+  }
   int col = 0, entries = 0;
   int since = 0;       // columns from the last non-zero's to col (from column 0 where there is none)
   int holder = -1;     // the code that holds the last non-zero
@@ -391,16 +416,28 @@ __device__ __forceinline__ int64_t checkpoint_entry(uint32_t slice_base, int64_t
 // A row's entries, nine to a chunk, a codeword's (up to three) at a time.  The lanes of a
 // wavefront fill their chunks at different times, so that nearly every place that may
 // store one is taken by a few of them: there is one such place to a codeword.
+// kShared: a chunk may hold entries of other lanes', before these or behind, and is zero before
+// all of them.
+template <bool kShared>
 struct ChunkSink {
-  char *chunks, *ckpt;          // the slice's; the same in all lanes
+  char *chunks, *ckpt;          // the slice's; the same in all lanes (kShared: a row of the slice each)
   uint32_t end;                 // bytes of its chunks
-  uint32_t at;                  // of this lane's next one: 512 c + 8 lane
+  uint32_t at;                  // of this lane's next one: 512 c + 8 (the row's place)
   int bits = 0;                 // that it holds, seven an entry
   uint32_t lo = 0, hi = 0;
+  __device__ __forceinline__ void put() {
+    if (at >= end) return;
+    if (kShared)
+      __hip_atomic_fetch_or(reinterpret_cast<unsigned long long *>(chunks + at),
+                            static_cast<unsigned long long>(hi & 0x7fffffffu) << 32 | lo, __ATOMIC_RELAXED,
+                            __HIP_MEMORY_SCOPE_WORKGROUP);
+    else
+      *reinterpret_cast<uint2 *>(chunks + at) = make_uint2(lo, hi & 0x7fffffffu);
+  }
   // The chunk is stored and the next one begins with the entries in `rest` (two at most);
   // `position`: what the row has reached with them.
   __device__ __forceinline__ void store(uint32_t rest, int position) {
-    if (at < end) *reinterpret_cast<uint2 *>(chunks + at) = make_uint2(lo, hi & 0x7fffffffu);
+    put();
     at += 512;
     if ((at & (kGroupChunks - 1) << 9) == 0 && at < end)
       *reinterpret_cast<uint16_t *>(ckpt + ((at >> 12) * 128 + (at & 511u) / 4)) =
@@ -421,44 +458,68 @@ struct ChunkSink {
 };
 static_assert(kGroupChunks == 8, "a group's chunks are 4096 bytes");
 
+// The zero column from which on a row stays where it is.
+__device__ __forceinline__ int next_zero(int at) { return (at + 2 * kZeroPeriod - 1) / (2 * kZeroPeriod) * (2 * kZeroPeriod); }
+// Non-zeros of a codeword (places a0, a1, a2: 2 column + symbol - 1) that are within the width; the
+// others' positions become the last one's.
+__device__ __forceinline__ int inside_width(int nonzeros, int a0, int a1, int a2, int width, int p0, int &p1, int &p2) {
+  if (a2 >= 2 * width) {   // digits past the width are dropped
+    nonzeros = min(nonzeros, 2);
+    p2 = p1;
+  }
+  if (a1 >= 2 * width) {
+    nonzeros = min(nonzeros, 1);
+    p1 = p2 = p0;
+  }
+  return a0 >= 2 * width ? 0 : nonzeros;
+}
+
+// Where a slice goes.
+struct SliceOut {
+  char *chunks, *ckpt;
+  int len;
+  uint32_t end;   // bytes of its chunks
+};
+__device__ __forceinline__ SliceOut slice_out(const WalkKind &k, int64_t slice, uint2 *stream, uint16_t *ckpt) {
+  const uint32_t base = __builtin_amdgcn_readfirstlane(k.slice_base[slice]);
+  const int len = __builtin_amdgcn_readfirstlane(k.slice_len[slice]);
+  return {reinterpret_cast<char *>(stream + static_cast<int64_t>(base) * 64),
+          reinterpret_cast<char *>(ckpt + checkpoint_entry(base, k.first_slice + slice) * 64), len, 512u * chunks_of(len)};
+}
+
 // A slice's rows, a lane each, into the interleaved stream, nine entries to a chunk;
 // a row shorter than its slice then steps onto the next zero column and stays there
 // (steps of 0) to the end of the slice's last chunk; and the row's position at the
 // start of every group of chunks into the checkpoints.
 __device__ __forceinline__ void emit_rows(const HeldTable &table, const WalkKind &k, int64_t slice,
-                                          uint2 *__restrict__ stream, uint16_t *__restrict__ ckpt) {
+                                          uint2 *__restrict__ stream, uint16_t *__restrict__ ckpt,
+                                          uint32_t *long_bits) {
   const int lane = threadIdx.x & 63;
   const int e = static_cast<int>(slice / k.slices);
   const int ridx = k.row_idx[slice * 64 + lane];
-  const uint32_t base = __builtin_amdgcn_readfirstlane(k.slice_base[slice]);
-  const int len = __builtin_amdgcn_readfirstlane(k.slice_len[slice]);
-  ChunkSink sink{reinterpret_cast<char *>(stream + static_cast<int64_t>(base) * 64),
-                 reinterpret_cast<char *>(ckpt + checkpoint_entry(base, k.first_slice + slice) * 64),
-                 512u * chunks_of(len), 8u * lane};
+  const SliceOut s = slice_out(k, slice, stream, ckpt);
+  ChunkSink<false> sink{s.chunks, s.ckpt, s.end, 8u * lane};
   *reinterpret_cast<uint16_t *>(sink.ckpt + 2 * lane) = 0;
   int at = 0;
   if (ridx != 0xffff) {
     int n;
-    const uint16_t *codes = row_codes(k.source, e, ridx, k.height, k.width, n);
+    bool is_long;
+    const uint16_t *codes = row_codes(k.source, e, ridx, k.height, k.width, n, is_long);
+    if (is_long && long_bits) {
+      const uint32_t bit = static_cast<uint32_t>(k.first_slice + slice) % kLongBits;
+      atomicOr(&long_bits[bit / 32], 1u << (bit % 32));
+      return;
+    }
     int from = 0;   // twice the column at which the codeword starts
     auto step = [&](uint32_t w, uint32_t) {
       int nonzeros = (w >> 4) & 3u;
-      const int a1 = from + static_cast<int>((w >> 16) & 255u), a2 = from + static_cast<int>(w >> 24);
-      const int p0 = position_at(from + static_cast<int>((w >> 8) & 255u));
+      const int a0 = from + static_cast<int>((w >> 8) & 255u), a1 = from + static_cast<int>((w >> 16) & 255u);
+      const int a2 = from + static_cast<int>(w >> 24);
+      const int p0 = position_at(a0);
       int p1 = position_at(a1), p2 = position_at(a2);
       const int end = from + 4 * static_cast<int>(w & 15u);
       if (__builtin_expect(p0 - at > kMaxStep || end > 2 * k.width, 0)) {
-        if (end > 2 * k.width) {   // digits past the width are dropped
-          if (a2 >= 2 * k.width) {
-            nonzeros = min(nonzeros, 2);
-            p2 = p1;
-          }
-          if (a1 >= 2 * k.width) {
-            nonzeros = min(nonzeros, 1);
-            p1 = p2 = p0;
-          }
-          if (from + static_cast<int>((w >> 8) & 255u) >= 2 * k.width) nonzeros = 0;
-        }
+        if (end > 2 * k.width) nonzeros = inside_width(nonzeros, a0, a1, a2, k.width, p0, p1, p2);
         if (nonzeros)
 #pragma unroll 1
           while (p0 - at > kMaxStep) {
@@ -473,9 +534,9 @@ __device__ __forceinline__ void emit_rows(const HeldTable &table, const WalkKind
       from = end;
     };
     walk_codes(table, codes, n, step, step);
-    if (static_cast<int>(sink.at >> 9) * (kFields * kFieldBits) + sink.bits < len * kFieldBits && (at >> 1) % kZeroPeriod != 0) {
+    if (static_cast<int>(sink.at >> 9) * (kFields * kFieldBits) + sink.bits < s.len * kFieldBits && (at >> 1) % kZeroPeriod != 0) {
       // padding follows: it must read zeros
-      const int zero = (at + 2 * kZeroPeriod - 1) / (2 * kZeroPeriod) * (2 * kZeroPeriod);
+      const int zero = next_zero(at);
       sink.add(zero - at, 1, zero);
       at = zero;
     }
@@ -512,9 +573,210 @@ __global__ __launch_bounds__(kWalkThreads) void walk_rows_kernel(WalkArgs a) {
     if (second) task -= a.k[0].tasks;
     const WalkKind &k = a.k[second ? 1 : 0];
     if (kEmit)
-      emit_rows(HeldTable{a.table, held}, k, task, a.stream, a.ckpt);
+      emit_rows(HeldTable{a.table, held}, k, task, a.stream, a.ckpt, a.long_bits);
     else
-      count_rows(CountTable{a.table, held}, k, a.count, task, a.status);
+      count_rows(CountTable{a.table, held}, k, a.count, task, a.status, a.any_long);
+  }
+}
+
+// ------------------------------------------------------------- long rows --
+//
+// A wavefront takes a long row, a lane a GROUP of eight of its codes.  What a group has to know
+// of the codes before it (the column, the last non-zero, the entries so far) comes from prefix
+// sums over the lanes and, from one turn of 64 groups to the next, from the last lane: twice the
+// instructions a code, but a row of 1024 codes is two turns and not 1024 steps.  The dictionary's words
+// come from global memory: these are few codes.
+//
+// 63 base experts whose rows have 75 to 98 % zeros, one in a hundred none: counting 177 us before,
+// 50 and 16 (in order_rows_kernel), emitting 303 before, 101 and 79.  (Taken by groups within the walks
+// themselves they make those of even rows slower, by 2 of 33 and 4 of 85 us, with none there.)
+constexpr int kGroupOfCodes = 8;
+
+// Eight of a row's codes, from code `at` on, and which of them there are.  (Loads stay within
+// the row: its last, partial eight is read from eight before its end.)
+struct EightCodes {
+  unaligned_u32x4 v;
+  uint32_t present;
+  __device__ __forceinline__ EightCodes(const uint16_t *codes, int n, int at) {   // n > kLongRowsFrom
+    const int here = min(max(n - at, 0), kGroupOfCodes);
+    present = (0xffu << (kGroupOfCodes - here)) & 0xffu;
+    v = here ? eight_codes((global_u16 *)codes + min(at, n - kGroupOfCodes)) : unaligned_u32x4{0, 0, 0, 0};
+  }
+  __device__ __forceinline__ uint32_t word(const uint32_t *table, int j) const {
+    const uint32_t code = (j & 1) ? v[j / 2] >> 16 : v[j / 2] & 0xffffu;
+    return table[code] & static_cast<uint32_t>(static_cast<int32_t>(present << (31 - j)) >> 31);
+  }
+};
+
+// A codeword's entries: long steps, then a step to each non-zero.
+struct CodeSteps {
+  int more, nonzeros;
+  uint32_t packed;
+  // from (twice the column) and at (the position): where the row stands before it, and then behind it
+  __device__ __forceinline__ CodeSteps(uint32_t w, int width, int &from, int &at) {
+    nonzeros = (w >> 4) & 3u;
+    const int a0 = from + static_cast<int>((w >> 8) & 255u), a1 = from + static_cast<int>((w >> 16) & 255u);
+    const int a2 = from + static_cast<int>(w >> 24);
+    const int p0 = position_at(a0);
+    int p1 = position_at(a1), p2 = position_at(a2), here = at;
+    more = 0;
+    from += 4 * static_cast<int>(w & 15u);
+    if (__builtin_expect(p0 - at > kMaxStep || from > 2 * width, 0)) {
+      if (from > 2 * width) nonzeros = inside_width(nonzeros, a0, a1, a2, width, p0, p1, p2);
+      if (nonzeros) {
+        more = steps_between(at, p0);
+        if (more) here = farthest_zero(at) + (more - 1) * kZeroStep;
+      }
+    }
+    packed = static_cast<uint32_t>(
+        pick(nonzeros, (p0 - here) | (p1 - p0) << kFieldBits | (p2 - p1) << (2 * kFieldBits), 0));
+    at = pick(nonzeros, p2, at);
+  }
+};
+
+// A long row's turns of 64 groups to turn(words, from, at), which moves from and at (twice the
+// column and the position, before the group) on to behind it; all lanes together.
+template <class Turn>
+__device__ __forceinline__ void walk_long_row(const uint32_t *table, const uint16_t *codes, int n, Turn &&turn) {
+  const int lane = threadIdx.x & 63;
+  int carry_from = 0, carry_at = 0;
+  EightCodes next(codes, n, kGroupOfCodes * lane);
+#pragma unroll 1
+  for (int first = 0; first < n; first += 64 * kGroupOfCodes) {
+    const EightCodes now = next;
+    next = EightCodes(codes, n, first + (64 + lane) * kGroupOfCodes);
+    uint32_t w[kGroupOfCodes];
+#pragma unroll
+    for (int j = 0; j < kGroupOfCodes; j++) w[j] = now.word(table, j);
+    int span = 0, key = 0;   // twice the group's columns; one more than its last non-zero's 2 column + symbol - 1
+#pragma unroll
+    for (int j = 0; j < kGroupOfCodes; j++) {
+      key = pick(w[j] & 0x30u, span + static_cast<int>(w[j] >> 24) + 1, key);
+      span += 4 * static_cast<int>(w[j] & 15u);
+    }
+    const int before = sub1::wave_prefix_sum(span) - span;
+    const int below = sub1::wave_max_below(key ? before + key : 0);
+    int from = carry_from + before;
+    int at = below ? position_at(carry_from + below - 1) : carry_at;
+    turn(w, from, at, first + kGroupOfCodes * lane < n, first + kGroupOfCodes * (lane + 1) >= n);
+    carry_from = __builtin_amdgcn_readlane(from, 63);
+    carry_at = __builtin_amdgcn_readlane(at, 63);
+  }
+}
+
+__device__ __forceinline__ const uint16_t *codes_of_lane(const uint16_t *codes, int lane) {
+  const uint64_t address = reinterpret_cast<uint64_t>(codes);
+  const uint32_t low = __builtin_amdgcn_readlane(static_cast<int>(address), lane);
+  const uint32_t high = __builtin_amdgcn_readlane(static_cast<int>(address >> 32), lane);
+  return reinterpret_cast<const uint16_t *>(static_cast<uint64_t>(high) << 32 | low);
+}
+
+// The entries of a matrix's long rows, by a workgroup.
+__device__ __forceinline__ void count_long_rows(const KindSource &source, int e, int height, int width,
+                                                const uint32_t *table, uint16_t *row_len, int32_t *status) {
+  const int lane = threadIdx.x & 63;
+  for (int r0 = threadIdx.x & ~63; r0 < height; r0 += blockDim.x) {
+    int n = 0;
+    bool is_long = false;
+    const uint16_t *codes = nullptr;
+    if (r0 + lane < height) codes = row_codes(source, e, r0 + lane, height, width, n, is_long);
+    for (unsigned long long longs = __ballot(is_long); longs; longs &= longs - 1) {
+      const int who = __ffsll(longs) - 1;
+      int entries = 0;
+      walk_long_row(table, codes_of_lane(codes, who), __builtin_amdgcn_readlane(n, who),
+                    [&](const uint32_t (&w)[kGroupOfCodes], int &from, int &at, bool live, bool ends) {
+#pragma unroll
+                      for (int j = 0; j < kGroupOfCodes; j++) {
+                        const CodeSteps c(w[j], width, from, at);
+                        entries += c.nonzeros + c.more;
+                      }
+                      // a row's codes cover its width rounded up to a whole pair, exactly
+                      if (live && ends && from != 2 * ((width + 1) & ~1)) atomicAdd(&status[0], 1);
+                    });
+      entries = __builtin_amdgcn_readlane(sub1::wave_prefix_sum(entries), 63);
+      if (lane == 0) row_len[r0 + who] = static_cast<uint16_t>(min(entries, kMaxRowEntries));
+    }
+  }
+}
+
+// The long rows into the stream.  They are the first ones of a matrix's first slices: four small
+// workgroups share a slice's, on different dies (on one the rows' entries, which share cache
+// lines, wait for each other in its L2: 127 us instead of 79).
+constexpr int kLongThreads = 256, kLongShares = 4;
+constexpr int kLongWaves = kLongShares * kLongThreads / 64;   // of a slice
+__global__ __launch_bounds__(kLongThreads) void emit_long_rows_kernel(WalkArgs a) {
+  if (*a.found) return;
+  const int lane = threadIdx.x & 63;
+  const int64_t all = a.k[0].tasks + (a.kinds == 2 ? a.k[1].tasks : 0);
+  for (int64_t t = blockIdx.x; t < kLongShares * all; t += gridDim.x) {
+    const int64_t task = t / kLongShares;
+    const int wave = static_cast<int>(t % kLongShares) * (kLongThreads / 64) + static_cast<int>(threadIdx.x >> 6);
+    const bool second = task >= a.k[0].tasks;
+    const WalkKind &k = a.k[second ? 1 : 0];
+    const int64_t slice = second ? task - a.k[0].tasks : task;
+    const uint32_t bit = static_cast<uint32_t>(k.first_slice + slice) % kLongBits;
+    if (!((a.long_bits[bit / 32] >> (bit % 32)) & 1u)) continue;
+    const int ridx = k.row_idx[slice * 64 + lane];
+    int n = 0;
+    bool is_long = false;
+    const uint16_t *codes = nullptr;
+    if (ridx != 0xffff)
+      codes = row_codes(k.source, static_cast<int>(slice / k.slices), ridx, k.height, k.width, n, is_long);
+    const SliceOut s = slice_out(k, slice, a.stream, a.ckpt);
+    int turn_of = 0;   // the wavefronts take the long rows in turn
+    for (unsigned long long longs = __ballot(is_long); longs; longs &= longs - 1) {
+      if (turn_of++ % kLongWaves != wave) continue;
+      const int who = __ffsll(longs) - 1;
+      // its chunks are put together in memory: zeros first, which the padding is too
+      for (uint32_t c = 512u * lane; c < s.end; c += 512u * 64)
+        *reinterpret_cast<uint2 *>(s.chunks + 8 * who + c) = make_uint2(0u, 0u);
+      sub1::drain_stores();
+      int carry_entries = 0;
+      walk_long_row(a.table, codes_of_lane(codes, who), __builtin_amdgcn_readlane(n, who),
+                    [&](const uint32_t (&w)[kGroupOfCodes], int &from, int &at, bool live, bool ends) {
+        // the steps of every codeword (7 bits each), how many (2 bits), and over them how many long
+        // ones come first (up to 256)
+        uint32_t steps[kGroupOfCodes];
+        int entries = 0, reached = at;
+#pragma unroll
+        for (int j = 0; j < kGroupOfCodes; j++) {
+          const CodeSteps c(w[j], k.width, from, at);
+          steps[j] = c.packed | static_cast<uint32_t>(c.nonzeros) << (3 * kFieldBits) |
+                     static_cast<uint32_t>(c.more) << (3 * kFieldBits + 2);
+          entries += c.nonzeros + c.more;
+        }
+        const int behind = carry_entries + sub1::wave_prefix_sum(entries), first = behind - entries;
+        ChunkSink<true> sink{s.chunks, s.ckpt, s.end, 512u * (first / kFields) + 8u * who, kFieldBits * (first % kFields)};
+#pragma unroll
+        for (int j = 0; j < kGroupOfCodes; j++) {
+          int more = steps[j] >> (3 * kFieldBits + 2);
+          if (__builtin_expect(more != 0, 0)) {
+            int zero = farthest_zero(reached);
+#pragma unroll 1
+            for (; more > 0; more--) {
+              sink.add(zero - reached, 1, zero);
+              reached = zero;
+              zero += kZeroStep;
+            }
+          }
+          const uint32_t three = steps[j] & ((1u << (3 * kFieldBits)) - 1);
+          reached += static_cast<int>((three & 127u) + ((three >> kFieldBits) & 127u) + (three >> (2 * kFieldBits)));
+          sink.add(three, (steps[j] >> (3 * kFieldBits)) & 3u, reached);
+        }
+        if (live && ends && behind < s.len && (at >> 1) % kZeroPeriod != 0) {
+          const int zero = next_zero(at);
+          sink.add(zero - at, 1, zero);
+          at = zero;
+        }
+        if (sink.lo | sink.hi) sink.put();
+        if (live && ends) {   // where the groups of chunks that hold nothing but padding begin
+          const uint32_t filled = (sink.at & ~511u) + (sink.bits ? 512u : 0u);
+          for (uint32_t c = (filled + 4095u) >> 12; c << 12 < s.end; c++)
+            *reinterpret_cast<uint16_t *>(s.ckpt + c * 128 + 2 * who) = static_cast<uint16_t>(at);
+        }
+        carry_entries = __builtin_amdgcn_readlane(behind, 63);
+      });
+    }
   }
 }
 
@@ -544,16 +806,17 @@ size_t order_rows_lds(int height) {
 // experts then take as long as wi alone (24 us, 34 one kind after the other).
 struct OrderKind {
   KindSource source;
-  const uint16_t *row_len;
+  uint16_t *row_len;
   uint16_t *row_idx;
   uint32_t *minmax;
   uint16_t *slice_len;
   int32_t *counts;
-  int height, slices;
+  int height, width, slices;
 };
 struct OrderArgs {
   OrderKind k[2];
-  const int32_t *found;
+  const int32_t *found, *any_long;
+  const uint32_t *table;
   int32_t *status;
 };
 
@@ -579,6 +842,10 @@ __global__ __launch_bounds__(kOrderThreads) void order_rows_kernel(OrderArgs a) 
   const uint32_t *mm = ks.minmax_of ? ks.minmax_of[e] : ks.minmax + static_cast<int64_t>(e) * height;
   const int64_t lane0 = static_cast<int64_t>(e) * slices * 64;
 
+  if (*a.any_long) {
+    count_long_rows(ks, e, height, k.width, a.table, k.row_len + static_cast<int64_t>(e) * height, status);
+    __syncthreads();
+  }
   int low = kMaxRowEntries, high = 0;
   for (int r = tid; r < height; r += kOrderThreads) {
     low = min(low, static_cast<int>(rl[r]));
@@ -2735,6 +3002,8 @@ int launch_walk(const Source &src, const MetaLayout &m, WalkArgs &w, hipStream_t
                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
   walk_rows_kernel<kEmit><<<static_cast<unsigned>(std::min<int64_t>(tasks, cus)), kWalkThreads, lds, s>>>(w);
   HIP_TRY(hipGetLastError());
+  if (w.long_bits) emit_long_rows_kernel<<<static_cast<unsigned>(std::min<int64_t>(tasks * kLongShares, 8 * cus)), kLongThreads, 0, s>>>(w);
+  HIP_TRY(hipGetLastError());
   return SUB1_OK;
 }
 
@@ -2750,13 +3019,14 @@ int prepare_layout(const Source &src, void *meta, int64_t meta_bytes, LayoutResu
   sub1::AnswerSlot slot;
   int rc = slot.take(s, who);
   if (rc) return rc;
-  zero_words_kernel<<<1, 64, 0, s>>>(status, 4);
+  zero_words_kernel<<<1, 64, 0, s>>>(status, 5);
   WalkArgs w{};
   rc = check_on_device(src, status + 3, w, s);
   if (!rc) rc = slot.launched(who);
   if (rc) return rc;
   int32_t *counts = reinterpret_cast<int32_t *>(base + m.counts);
   w.status = status;
+  w.any_long = status + 4;
   for (int i = 0; i < src.kinds; i++) {
     const KindMeta &k = m.k[i];
     WalkKind &wk = w.k[walk_place(src, i)];
@@ -2772,16 +3042,19 @@ int prepare_layout(const Source &src, void *meta, int64_t meta_bytes, LayoutResu
   OrderArgs o{};
   o.status = status;
   o.found = status + 3;
+  o.any_long = status + 4;
+  o.table = w.table;
   size_t lds = 0;
   for (int i = 0; i < src.kinds; i++) {
     const KindMeta &k = m.k[i];
     o.k[i] = {src.k[i],
-              reinterpret_cast<const uint16_t *>(base + k.row_len),
+              reinterpret_cast<uint16_t *>(base + k.row_len),
               reinterpret_cast<uint16_t *>(base + k.row_idx),
               reinterpret_cast<uint32_t *>(base + k.minmax),
               reinterpret_cast<uint16_t *>(base + k.slice_len),
               counts + slice0,
               k.height,
+              k.width,
               k.slices};
     lds = std::max(lds, order_rows_lds(k.height));
     slice0 += static_cast<int64_t>(src.count) * k.slices;
@@ -2823,13 +3096,20 @@ int prepare_codes(const Source &src, const Prepared &p, hipStream_t s, const cha
   int rc = slot.take(s, who);
   if (rc) return rc;
   int32_t *found = reinterpret_cast<int32_t *>(base + m.status) + 3;
-  zero_words_kernel<<<1, 64, 0, s>>>(found, 1);
+  zero_words_kernel<<<1, 64, 0, s>>>(found, kStatusWords - 3);
   WalkArgs w{};
   rc = check_on_device(src, found, w, s);
   if (!rc) rc = slot.launched(who);
   if (rc) return rc;
   uint2 *stream = static_cast<uint2 *>(const_cast<void *>(p.codes));
   uint16_t *ckpt = reinterpret_cast<uint16_t *>(stream + p.total_chunks * 64);
+  // Where a kind's longest slice is twice what the stream's size says of an average one, some rows
+  // are long ones (or a few rows are, of a narrow matrix: the launch for them then finds none, 4 us).
+  double weights = 0.0;
+  for (int i = 0; i < src.kinds; i++) weights += static_cast<double>(src.count) * src.height[i] * src.width[i];
+  for (int i = 0; i < src.kinds; i++)
+    if (p.max_chunks[i] > 2.0 * static_cast<double>(p.total_chunks) * 64.0 / weights * src.width[i] + 2.0)
+      w.long_bits = reinterpret_cast<uint32_t *>(base + m.status) + kStatusLong;
   w.stream = stream;
   w.ckpt = ckpt;
   int64_t first_slice = 0;

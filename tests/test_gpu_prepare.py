@@ -86,6 +86,56 @@ def test_long_gaps_and_dropped_digits_are_counted_as_they_are_written(gpu, oracl
         assert torch.equal(prepared.decode(0, kind), want[kind])
 
 
+@pytest.mark.parametrize('width,codes', [
+    (141, [27, 64, 65, 71]), (1601, [511, 512, 513, 801]), (8193, [1024, 1025, 1537, 4097])])
+def test_rows_of_many_codes_come_back_whole(gpu, oracle, width, codes):
+    """Rows of more than twice the average of codes: about a lane's eight and a turn's 512 of
+    them, alone and side by side, with gaps of many steps between and digits past an odd
+    width; and rows of this kind that are bad."""
+    sub1, op = gpu
+    even = (width + 1) // 2 * 2
+    g = torch.Generator().manual_seed(width)
+    symbols = torch.zeros((200, even), dtype=torch.uint8)
+    symbols[::3, 0] = 1
+    for i, n in enumerate(codes * 3):
+        r = [0, 70, 71, 72, 73, 74, 150, 151, 152, 190, 191, 199][i]
+        pairs = min(n, even // 2)       # (a code to a pair without zeros)
+        first = 2 * int(torch.randint(0, even // 2 - pairs + 1, (1,), generator=g))
+        symbols[r, first:first + 2 * pairs] = torch.randint(1, 3, (2 * pairs,), generator=g).to(torch.uint8)
+        if i % 3 == 2:
+            symbols[r, -1] = 2
+            symbols[r, first + pairs // 2:first + pairs // 2 + even // 5] = 0
+    w_comp, row_off = packed(gpu, symbols.cuda())
+    sizes = row_off[1:] - row_off[:-1]
+    longs = [r for r in range(200) if (int(sizes[r]) - 16) * 200 > 2 * int(row_off[-1])]
+    assert len(longs) >= 9
+    pairs = torch.ones(400, dtype=torch.bfloat16, device='cuda')
+    other = packed(gpu, torch.zeros((width, 200), dtype=torch.uint8, device='cuda'))
+    prepared = op.PreparedStack.from_layers(
+        sub1.DEC[0], [(w_comp, row_off, pairs)],
+        [other + (torch.ones(2 * width, dtype=torch.bfloat16, device='cuda'),)])
+    assert torch.equal(prepared.decode(0, 0), symbols[:, :width].cuda())
+    want, offsets = w_comp.cpu().numpy().view('uint16'), row_off.tolist()
+    entries = sum(max(len(oracle.gap_entries(want[offsets[r]:offsets[r + 1]], width)) - 1, 0) for r in range(200))
+    assert prepared.entry_counts()[1] == entries
+    # walked from the checkpoints by many wavefronts, and from the front: the same sums
+    matrix = op.PreparedMatrix(sub1.DEC[0], w_comp, row_off, pairs, width)
+    x = torch.randn((1, width), generator=torch.Generator().manual_seed(3)).bfloat16().cuda()
+    few, many = (matrix.product_tokens(x.expand(t, width).contiguous()) for t in (1, 600))
+    assert torch.equal(few[0], many[599])
+    exact = (symbols[:, :width] > 0).double() @ x[0].double().cpu()
+    # bf16 of a sum of up to 8193 terms of 2 or so in fp32
+    assert ((few[0].double().cpu() - exact).abs() <= 2 ** -8 * exact.abs() + 8193 * 2 ** -24 * 200).all()
+    # the last code of two long rows missing: they are counted, and the rows behind them, with one too many
+    a = longs[1]
+    b = next(r for r in longs if r > a + 1)
+    short = row_off.clone()
+    short[a + 1] -= 1
+    short[b + 1] -= 1
+    with pytest.raises(op._lib.Sub1Error, match='codes of 4 rows'):
+        op.PreparedMatrix(sub1.DEC[0], w_comp, short, pairs, width)
+
+
 def test_preparing_names_a_bad_pointer(gpu):
     """The pointer tables are looked over on the GPU before any of them is
     followed; the message names the matrix."""
