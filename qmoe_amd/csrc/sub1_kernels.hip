@@ -548,7 +548,10 @@ __global__ void tell_count_kernel(sub1::Answer answer) {
 // ticket.  A wo tile of token t needs all of h[t], so it waits until the wi tiles
 // of t have signalled; those have smaller tickets, were therefore taken by
 // workgroups that are already running, and never wait themselves, so the wait
-// always ends.
+// always ends.  A few tokens have a workgroup for every tile instead, all of them running at
+// once: a wo tile's has its rows' codes and their words of the table by the time h is there.
+// (One token of base and c-2048 shapes 28.9 -> 17.3 us and 44.5 -> 22.5, nine of base shapes 43.8 -> 21.3,
+// with tickets and everything fetched behind the wait.)
 //
 // Within a tile the wavefronts take runs of rows from a counter in LDS and give a
 // LANE to a GROUP of 32 codes, not to a row: a row's sum is the sum of its groups'
@@ -583,6 +586,7 @@ struct MoeArgs {
   int32_t *ctrl;  // the control words (sub1_common.h): ticket, fault counts, a word per token
   int tokens, d_model, d_ff, experts;
   int wi_tiles, wo_tiles;  // per token
+  bool at_once;            // a workgroup for every tile, all of them running: tile b is workgroup b's
   int act_dwords;          // LDS dwords of the activations; the table's first words follow
   int held;                // words of the table kept in LDS (0: none)
   int wi_expect;           // wi tiles a wo tile waits for (wi_tiles outside tests)
@@ -685,82 +689,110 @@ __device__ __forceinline__ void row_by_lane(const uint32_t *__restrict__ tab, co
   s2 += p2;
 }
 
-// Rows row0 .. row0 + rows - 1 of one matrix (rows <= 64, a wavefront): lane r
-// receives the sums of row row0 + r.  `partial` is the wavefront's own LDS, 64 pairs.
+// Rows row0 .. row0 + rows - 1 of one matrix (rows <= 64, a wavefront), 64 groups a turn.  Where
+// the table is in memory, what a turn needs of the matrix is fetched ahead: the first one's before the
+// activations are there.  (With the table's head in LDS the wavefronts of a compute unit are four times
+// as many, and their registers do not hold it.)
 template <bool kHeld>
-__device__ __forceinline__ void rows_by_groups(const uint32_t *__restrict__ tab, const uint32_t *held_words,
-                                               uint32_t held, const uint16_t *__restrict__ codes,
-                                               const int32_t *__restrict__ row_off, int row0, int rows,
-                                               const float *X, float2 *partial, float &s1, float &s2) {
-  const int lane = threadIdx.x & 63;
-  const bool mine = lane < rows;
-  const int off = mine ? row_off[row0 + lane] : 0;
-  const int len = mine ? row_off[row0 + lane + 1] - off : 0;
-  const int groups = (max(len, 0) + kGroupCodes - 1) / kGroupCodes;
-  const int last = wave_prefix_sum(groups), first = last - groups;   // the row's groups, among the run's
-  const int total = __builtin_amdgcn_readlane(last, 63);
-  // A lane to a row instead where the rows are alike and there are enough of them: it
-  // then takes as many steps as the longest has codes, and no prefix sums.  (256
-  // tokens, us: groups always 125 base, 163 large, 428 c-2048; rows always 103, 163,
-  // 483, and 685, 960, 2176 where the shares of zeros differ from row to row; by this
-  // rule 98, 149, 416, and 165, 263, 651.)
-  int longest = len;
-  for (int m = 1; m < 64; m <<= 1) longest = max(longest, __shfl_xor(longest, m, 64));
-  if ((longest + 7) / 8 * 8 <= (total + 63) / 64 * kGroupStep) {
-    row_by_lane<kHeld>(tab, held_words, held, codes + off, len, X, s1, s2);
-    return;
+struct RowRun {
+  const uint32_t *tab, *held_words;
+  uint32_t held;
+  const uint16_t *codes;
+  int off, len;               // a lane's row
+  int first, last, total;     // its groups, among the run's; all groups
+  bool by_lane;               // the rows are walked by a lane each
+  int turn;
+  // of a lane's group in the turn
+  int r_first;                // its row's first group
+  uint32_t e[kGroupCodes];
+
+  __device__ __forceinline__ void take(const uint16_t *matrix, const int32_t *__restrict__ row_off, int row0, int rows) {
+    const int lane = threadIdx.x & 63;
+    const bool mine = lane < rows;
+    codes = matrix;
+    off = mine ? row_off[row0 + lane] : 0;
+    len = mine ? row_off[row0 + lane + 1] - off : 0;
+    const int groups = (max(len, 0) + kGroupCodes - 1) / kGroupCodes;
+    last = wave_prefix_sum(groups);
+    first = last - groups;
+    total = __builtin_amdgcn_readlane(last, 63);
+    // A lane to a row instead where the rows are alike and there are enough of them: it
+    // then takes as many steps as the longest has codes, and no prefix sums.  (256
+    // tokens, us: groups always 125 base, 163 large, 428 c-2048; rows always 103, 163,
+    // 483, and 685, 960, 2176 where the shares of zeros differ from row to row; by this
+    // rule 98, 149, 416, and 165, 263, 651.)
+    int longest = len;
+    for (int m = 1; m < 64; m <<= 1) longest = max(longest, __shfl_xor(longest, m, 64));
+    by_lane = (longest + 7) / 8 * 8 <= (total + 63) / 64 * kGroupStep;
+    turn = 0;
+    if (!kHeld && !by_lane && total) fetch();
   }
-  s1 = 0.f;
-  s2 = 0.f;
-  int carry = 0;   // the column reached in a row that goes on from the turn before
-  for (int turn = 0; turn < total; turn += 64) {
+
+  __device__ __forceinline__ void fetch() {
     // the row of this lane's group: the first whose groups end behind it
+    const int lane = threadIdx.x & 63;
     const int g = min(turn + lane, total - 1);
     int r = 0;
 #pragma unroll
     for (int step = 32; step >= 1; step >>= 1)
       if (__shfl(last, r + step - 1, 64) <= g) r += step;
-    const int r_first = __shfl(first, r, 64);
+    r_first = __shfl(first, r, 64);
     const int r_off = __shfl(off, r, 64), r_len = __shfl(len, r, 64);
     const bool active = turn + lane < total;
     const int in_row = active ? kGroupCodes * (g - r_first) : 0;
     const int count = active ? min(r_len - in_row, kGroupCodes) : 0;
-    uint32_t e[kGroupCodes];
     group_words<kHeld>(tab, held_words, held, codes + r_off + in_row, count, r_len >= 8, e);
-    int span = 0;
-#pragma unroll
-    for (int i = 0; i < kGroupCodes; i++) span += static_cast<int>(e[i] & 15u);
-    span *= 2;
-    const int before = wave_prefix_sum(span) - span;
-    const int row_before = __shfl(before, max(r_first - turn, 0), 64);
-    const int at = before - row_before + (r_first < turn ? carry : 0);
-    carry = __builtin_amdgcn_readlane(at + span, 63);
-    float2 p = {0.f, 0.f};
-    int col = at;
-#pragma unroll
-    for (int i = 0; i < kGroupCodes; i++) add_codeword(e[i], X, col, p.x, p.y);
-    partial[lane] = p;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    for (int i = max(first - turn, 0); i < min(last - turn, 64); i++) {
-      const float2 q = partial[i];
-      s1 += q.x;
-      s2 += q.y;
-    }
-    __builtin_amdgcn_wave_barrier();
   }
-}
+
+  // Lane r receives the sums of row row0 + r.  `partial` is the wavefront's own LDS, 64 pairs.
+  __device__ __forceinline__ void sums(const float *X, float2 *partial, float &s1, float &s2) {
+    if (by_lane) {
+      row_by_lane<kHeld>(tab, held_words, held, codes + off, len, X, s1, s2);
+      return;
+    }
+    const int lane = threadIdx.x & 63;
+    s1 = 0.f;
+    s2 = 0.f;
+    int carry = 0;   // the column reached in a row that goes on from the turn before
+    while (turn < total) {
+      if (kHeld) fetch();
+      int span = 0;
+#pragma unroll
+      for (int i = 0; i < kGroupCodes; i++) span += static_cast<int>(e[i] & 15u);
+      span *= 2;
+      const int before = wave_prefix_sum(span) - span;
+      const int row_before = __shfl(before, max(r_first - turn, 0), 64);
+      const int at = before - row_before + (r_first < turn ? carry : 0);
+      carry = __builtin_amdgcn_readlane(at + span, 63);
+      float2 p = {0.f, 0.f};
+      int col = at;
+#pragma unroll
+      for (int i = 0; i < kGroupCodes; i++) add_codeword(e[i], X, col, p.x, p.y);
+      partial[lane] = p;
+      sub1::wave_lds_fence();
+      for (int i = max(first - turn, 0); i < min(last - turn, 64); i++) {
+        const float2 q = partial[i];
+        s1 += q.x;
+        s2 += q.y;
+      }
+      __builtin_amdgcn_wave_barrier();
+      turn += 64;
+      if (!kHeld && turn < total) fetch();
+    }
+  }
+};
 
 // Rows that a wavefront takes at a time: a lane each where a tile has that many
 // for all its wavefronts, but at least about 64 groups of them (a row of W weights
-// with 90% zeros has W / 23 codes).
-__device__ __forceinline__ int rows_at_a_time(int rows, int width, int waves) {
+// with 90% zeros has W / 23 codes); where there are enough workgroups for all tiles at
+// once, as many as make all wavefronts work side by side.
+__device__ __forceinline__ int rows_at_a_time(int rows, int width, int waves, bool at_once) {
+  if (at_once) return min((rows + waves - 1) / waves, 64);
   return min(max(max(rows / waves, 64 * 640 / (width + 640)), 1), 64);
 }
 
 template <int kThreads>
-__global__ __launch_bounds__(kThreads, 4) void moe_kernel(MoeArgs a) {
+__global__ __launch_bounds__(kThreads, kThreads == 1024 ? 4 : 2) void moe_kernel(MoeArgs a) {
   constexpr bool kHeld = kThreads == 1024;   // the form with the table's head in LDS
   extern __shared__ __align__(16) float lds[];
   __shared__ int s_ticket, s_row;
@@ -774,14 +806,23 @@ __global__ __launch_bounds__(kThreads, 4) void moe_kernel(MoeArgs a) {
     for (int i = 4 * threadIdx.x; i < a.held; i += 4 * kThreads)
       *reinterpret_cast<uint4 *>(held_words + i) = *reinterpret_cast<const uint4 *>(a.tab + i);
   float2 *partial = s_partial + (threadIdx.x & ~63u);
+  constexpr int kWaves = kThreads / 64;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  RowRun<kHeld> run;
+  run.tab = a.tab;
+  run.held_words = held_words;
+  run.held = a.held;
   for (;;) {
-    __syncthreads();  // previous tile's readers of lds and s_ticket are done
-    if (threadIdx.x == 0)
-      s_ticket = __hip_atomic_fetch_add(&a.ctrl[0], 1, __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    const int ticket = s_ticket;
-    if (ticket >= n_all) break;
+    int ticket = blockIdx.x;
+    if (!a.at_once) {
+      __syncthreads();  // previous tile's readers of lds and s_ticket are done
+      if (threadIdx.x == 0)
+        s_ticket = __hip_atomic_fetch_add(&a.ctrl[0], 1, __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+      ticket = s_ticket;
+      if (ticket >= n_all) break;
+    }
 
     const bool is_wi = ticket < n_wi;
     const int j = is_wi ? ticket : ticket - n_wi;
@@ -803,10 +844,17 @@ __global__ __launch_bounds__(kThreads, 4) void moe_kernel(MoeArgs a) {
           const int64_t i = static_cast<int64_t>(t) * a.d_model + row;
           a.y[i] = a.x[i];
         }
+      if (a.at_once) break;
       continue;   // a dropped token's word stays untouched
     }
+    const int32_t *row_off = (is_wi ? a.wi_row_off : a.wo_row_off) + static_cast<int64_t>(e) * (height + 1);
+    const uint16_t *codes = a.w_comp + (is_wi ? a.wi_code_base : a.wo_code_base)[e];
+    const uint32_t *minmax = (is_wi ? a.wi_minmax : a.wo_minmax) + static_cast<int64_t>(e) * height;
+    const int at_a_time = rows_at_a_time(row_end - row_begin, width, kWaves, a.at_once);
+    int row0 = row_begin + at_a_time * wave;   // the first run; further ones from s_row
+    if (row0 < row_end) run.take(codes, row_off, row0, min(at_a_time, row_end - row0));
     if (threadIdx.x == 0) {
-      s_row = row_begin;
+      s_row = row_begin + at_a_time * kWaves;
       if (!is_wi)
         sub1::bounded_wait(&a.ctrl[sub1::token_word(t)], a.wi_expect, a.wait_ticks, a.sticky,
                            &a.ctrl[sub1::kCtrlGaveUp]);
@@ -814,20 +862,12 @@ __global__ __launch_bounds__(kThreads, 4) void moe_kernel(MoeArgs a) {
     __syncthreads();  // thread 0's acquire covers the whole workgroup
     stage_activations<kThreads>(lds, (is_wi ? a.x : a.h) + static_cast<int64_t>(t) * width, width);
     __syncthreads();
-    const int32_t *row_off = (is_wi ? a.wi_row_off : a.wo_row_off) + static_cast<int64_t>(e) * (height + 1);
-    const uint16_t *codes = a.w_comp + (is_wi ? a.wi_code_base : a.wo_code_base)[e];
-    const uint32_t *minmax = (is_wi ? a.wi_minmax : a.wo_minmax) + static_cast<int64_t>(e) * height;
-    const int at_a_time = rows_at_a_time(row_end - row_begin, width, kThreads / 64);
-    for (;;) {
-      int row0 = 0;
-      if ((threadIdx.x & 63) == 0) row0 = atomicAdd(&s_row, at_a_time);
-      row0 = __builtin_amdgcn_readfirstlane(row0);
-      if (row0 >= row_end) break;
+    while (row0 < row_end) {
       const int rows = min(at_a_time, row_end - row0);
-      const int row = row0 + (threadIdx.x & 63);
+      const int row = row0 + lane;
       float s1, s2;
-      rows_by_groups<kHeld>(a.tab, held_words, a.held, codes, row_off, row0, rows, lds, partial, s1, s2);
-      if ((threadIdx.x & 63) < rows) {
+      run.sums(lds, partial, s1, s2);
+      if (lane < rows) {
         uint16_t b = f32_to_bf16(row_result(minmax[row], s1, s2));
         if (is_wi) {
           if (b & 0x8000u) b = 0;  // relu
@@ -839,6 +879,10 @@ __global__ __launch_bounds__(kThreads, 4) void moe_kernel(MoeArgs a) {
           a.y[static_cast<int64_t>(t) * a.d_model + row] = b;
         }
       }
+      row0 = 0;
+      if (lane == 0) row0 = atomicAdd(&s_row, at_a_time);
+      row0 = __builtin_amdgcn_readfirstlane(row0);
+      if (row0 < row_end) run.take(codes, row_off, row0, min(at_a_time, row_end - row0));
     }
     if (is_wi) {
       // every wavefront waits for its h stores to be acknowledged, then the
@@ -853,8 +897,9 @@ __global__ __launch_bounds__(kThreads, 4) void moe_kernel(MoeArgs a) {
       // said once the tile's work is done: it takes a round trip to memory
       sub1::waited_on(&a.ctrl[sub1::token_word(t)], a.wo_tiles);
     }
+    if (a.at_once) break;
   }
-  if (threadIdx.x == 0) sub1::leave_launch(a.ctrl, gridDim.x);
+  if (!a.at_once && threadIdx.x == 0) sub1::leave_launch(a.ctrl, gridDim.x);
 }
 
 __global__ void zero_i32_kernel(int32_t *p, int n) {
@@ -932,6 +977,7 @@ int slot_table_for(const int32_t *dec, hipStream_t stream, TableSlot *out, int32
 }
 
 constexpr int kMoeThreads = 256;
+constexpr int kGroupsAtOnce = 48 * kMoeThreads / 64;   // groups that a workgroup's wavefronts take in a turn, with room
 constexpr int kMoeSweepThreads = 1024;   // one workgroup per compute unit, the table's head in its LDS
 
 template <typename K>
@@ -1120,15 +1166,12 @@ extern "C" int sub1_moe_grouped(const sub1_moe_stack *st, const int32_t *token_e
   const int wmax = st->d_model > st->d_ff ? st->d_model : st->d_ff;
   a.act_dwords = lds_dwords_for_width(wmax);
   // One workgroup of 16 wavefronts per compute unit with all the LDS that the
-  // activations leave for the table's first words, or workgroups of 4 wavefronts,
-  // several to a compute unit, and the table from memory.  Staging the table takes
-  // a workgroup about 10 us, which it has back once it has a few microseconds' worth of
-  // codes: 12 tokens through the base, large and c-2048 shapes 44, 45 and 63 us
-  // against 50, 61 and 107; 8 tokens 43, 45 and 62 against 39, 48 and 89; one token
-  // 42, 42 and 56 against 30, 31 and 45.
+  // activations leave for the table's first words, or workgroups of 4 wavefronts
+  // and the table from memory, which from some 90 million weights on takes longer:
+  // base shapes, 16, 32 and 48 tokens 42, 46 and 48 us against 23, 35 and 51; large ones, 16 and 24 tokens
+  // 44 and 48 against 37 and 51; c-2048, 4, 8 and 12 tokens 57, 58 and 61 against 36, 50 and 64.
   const size_t lds_limit = 160 * 1024 - 64 - kMoeSweepThreads * sizeof(float2);
-  const bool worth_it = tokens >= cus || (tokens >= 10 && static_cast<int64_t>(tokens) * st->d_model *
-                                                              st->d_ff >= (1 << 24));
+  const bool worth_it = tokens >= cus || (tokens >= 10 && static_cast<int64_t>(tokens) * st->d_model * st->d_ff >= 90000000);
   const bool sweep = worth_it &&
                      a.act_dwords * sizeof(float) + 16384 * sizeof(uint32_t) <= lds_limit;
   const int threads = sweep ? kMoeSweepThreads : kMoeThreads;
@@ -1150,27 +1193,42 @@ extern "C" int sub1_moe_grouped(const sub1_moe_stack *st, const int32_t *token_e
   if (rc) return rc;
   if (per_cu < 1) return fail(SUB1_ERR_INTERNAL, "sub1_moe_grouped: kernel does not fit a CU");
   int64_t grid = static_cast<int64_t>(cus) * per_cu;
-  // Parts of a projection: the number with which its tiles take the least time in
-  // rounds of the grid.  A tile costs about 8 us (ticket, activations, the wait, the
-  // wavefronts that finish early) besides its share of the projection, of which a
-  // compute unit takes some 80 000 weights a microsecond.
-  const double tile_share = 8.0 * 80000.0 / (static_cast<double>(st->d_model) * st->d_ff);
-  const int threads_rows = threads / 4;   // at least so many rows to a tile
-  auto parts_of = [&](int height) {
-    int best = 1;
-    double best_cost = 1e30;
-    for (int parts = 1; parts <= std::max(1, height / threads_rows); parts++) {
-      const int64_t rounds = (static_cast<int64_t>(tokens) * parts + grid - 1) / grid;
-      const double cost = rounds * (1.0 / parts + tile_share);
-      if (cost < best_cost - 1e-9) {
-        best_cost = cost;
-        best = parts;
-      }
-    }
-    return best;
+  // A few tokens: a workgroup for every tile.  As many tiles as give every wavefront a turn of its
+  // own (64 groups, of which a row of W weights with 90 % zeros has W / 736 and a half), more where compute
+  // units would have none, and at most one of either projection for each.  (More are slower again:
+  // each counts itself and asks for words of the table.  Base and c-2048 shapes, 48, 96 and 192 tiles a
+  // token, us: one token 17.4, 19.7, 26.6 and 29.9, 22.9, 29.4.)
+  const int most = sweep ? 0 : cus / tokens;
+  const auto tiles_of = [&](int height, int width) {
+    const int turns = static_cast<int>(height * (width / 736.0 + 0.5) / kGroupsAtOnce) + 1;
+    return std::min({std::max(turns, std::min(48, cus / (2 * tokens))), most, (height + 3) / 4});
   };
-  a.wi_tiles = parts_of(st->d_ff);
-  a.wo_tiles = parts_of(st->d_model);
+  a.wi_tiles = tiles_of(st->d_ff, st->d_model);
+  a.wo_tiles = tiles_of(st->d_model, st->d_ff);
+  a.at_once = most > 0 && static_cast<int64_t>(tokens) * (a.wi_tiles + a.wo_tiles) <= grid;
+  if (!a.at_once) {
+    // Parts of a projection: the number with which its tiles take the least time in
+    // rounds of the grid.  A tile costs about 8 us (ticket, activations, the wait, the
+    // wavefronts that finish early) besides its share of the projection, of which a
+    // compute unit takes some 80 000 weights a microsecond.
+    const double tile_share = 8.0 * 80000.0 / (static_cast<double>(st->d_model) * st->d_ff);
+    const int threads_rows = threads / 4;   // at least so many rows to a tile
+    auto parts_of = [&](int height) {
+      int best = 1;
+      double best_cost = 1e30;
+      for (int parts = 1; parts <= std::max(1, height / threads_rows); parts++) {
+        const int64_t rounds = (static_cast<int64_t>(tokens) * parts + grid - 1) / grid;
+        const double cost = rounds * (1.0 / parts + tile_share);
+        if (cost < best_cost - 1e-9) {
+          best_cost = cost;
+          best = parts;
+        }
+      }
+      return best;
+    };
+    a.wi_tiles = parts_of(st->d_ff);
+    a.wo_tiles = parts_of(st->d_model);
+  }
   a.wi_expect = a.wi_tiles + sub1::expect_extra();
   const int64_t tiles = static_cast<int64_t>(tokens) * (a.wi_tiles + a.wo_tiles);
   if (tiles > INT32_MAX - (1 << 20))

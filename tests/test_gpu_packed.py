@@ -49,3 +49,33 @@ def test_rows_of_different_lengths_on_the_packed_layout(oracle, d_model, d_ff, s
             want, _ = oracle.expert_ffn(wi[int(route[i])], wo[int(route[i])], xs[i], order=1)
             assert np.array_equal(got[i], want), (tokens, i)
     assert kernels == {'moe_kernel<256>', 'moe_kernel<1024>'}
+
+
+@pytest.mark.parametrize('d_model,d_ff,experts,tokens', [
+    (3, 5, 2, 1), (64, 3, 3, 255), (5, 300, 2, 96),        # fewer rows than wavefronts; a tile or two a token
+    (1200, 2100, 3, 9), (768, 3072, 4, 38), (768, 3072, 4, 39)])   # a turn a wavefront; the last before the other form
+def test_a_workgroup_for_every_tile(oracle, d_model, d_ff, experts, tokens):
+    from qmoe_amd import sub1, sub1_hip
+    wi = [uneven_layer(oracle, d_ff, d_model, [0.1, 0.3], 10 + e) for e in range(experts)]
+    wo = [uneven_layer(oracle, d_model, d_ff, [0.1, 0.02, 1.0], 20 + e) for e in range(experts)]
+
+    def dev(layer):
+        codes, row_off, minmax = layer
+        return torch.from_numpy(codes.view(np.int16)).cuda(), torch.from_numpy(row_off).cuda(), bf16_dev(minmax)
+
+    stack = sub1_hip.ExpertStack.from_layers(sub1.DEC[0], [dev(l) for l in wi], [dev(l) for l in wo])
+    xs = np.stack([so.synthetic_activation(d_model, 30 + i) for i in range(tokens)])
+    route = [i * 7 % experts for i in range(tokens)]
+    bad = [i for i in (3, 8) if i < tokens]
+    for i, e in zip(bad, (-1, experts)):
+        route[i] = e
+    x, te = bf16_dev(xs), torch.tensor(route, dtype=torch.int32).cuda()
+    for _ in range(3):                  # the control words are left as they were found
+        got = bits_host(stack.forward(x, te))
+        assert stack.launch_faults(tokens) == (0, len(bad) // 2)
+        for i in sorted({0, tokens // 2, tokens - 1} | set(bad)):
+            want = xs[i] if i in bad else oracle.expert_ffn(wi[route[i]], wo[route[i]], xs[i], order=1)[0]
+            assert np.array_equal(got[i], want), i
+    weights = tokens * d_model * d_ff
+    assert sub1_hip._lib.load().sub1_last_kernel().decode() == (
+        'moe_kernel<1024>' if tokens >= 10 and weights >= 90000000 else 'moe_kernel<256>')
