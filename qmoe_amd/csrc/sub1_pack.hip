@@ -173,17 +173,22 @@ struct PackArgs {
   int window;                // pairs of a row taken at a time
 };
 
-constexpr int kPackWaves = 4;           // rows per workgroup
+constexpr int kPackWaves = 4;           // of a workgroup: a row each, or one row together
+constexpr int kSharedRows = 10, kSharedWidth = 2048;   // up to so many rows a compute unit, and from this width on, wavefronts share a row
+constexpr int kJumpRounds = 4;          // sixteen entries at a time
 constexpr int kPackWindow = 4096;       // pairs of a row in LDS at most
 constexpr int kBorderLdsWords = (kBorderStrings / 32 + 3) / 4 * 4;
 constexpr int kAhead = 4;               // loads of a lane that are asked for together
 constexpr int kLookahead = 2 * kMaxPairs;   // symbols past a place that decide its entry
 
-// LDS of a wavefront: two bit planes over the window's symbols (which are not
-// zero, which are 2), and the pairs at which the parse has an entry.
+// LDS of a row: two bit planes over the window's symbols (which are not
+// zero, which are 2), the pairs at which the parse has an entry and, where wavefronts share
+// a row, what they tell each other, the longest entry at every pair and, twice, where
+// several of them in turn lead to.
 __host__ __device__ constexpr int plane_words(int window) { return (2 * window + kLookahead + 31) / 32 + 1; }
-__host__ __device__ constexpr size_t pack_lds_per_wave(int window) {
-  return static_cast<size_t>(2 * plane_words(window)) * 4 + (static_cast<size_t>(window) * 2 + 15) / 16 * 16;
+__host__ __device__ constexpr size_t pack_lds_per_row(int window, bool shared) {
+  return static_cast<size_t>(2 * plane_words(window)) * 4 + (static_cast<size_t>(window) * 2 + 15) / 16 * 16 +
+         (shared ? 2 * kPackWaves * sizeof(int) + (static_cast<size_t>(window) + 15) / 16 * 16 * 5 : 0);
 }
 
 __device__ __forceinline__ uint32_t plane_bits(const uint32_t *plane, int at) {
@@ -198,6 +203,7 @@ __device__ __forceinline__ uint32_t plane_bits(const uint32_t *plane, int at) {
 __device__ __forceinline__ int from_of(int at, int width) { return max(min(at, width - 8), 0); }
 struct EightWeights {
   uint32_t v[4];
+  EightWeights() = default;
   __device__ __forceinline__ EightWeights(const uint16_t *row, int at, int width) {
     if (width >= 8) {
       __builtin_memcpy(v, row + from_of(at, width), sizeof v);
@@ -210,6 +216,7 @@ struct EightWeights {
 };
 struct EightSymbols {
   uint32_t v[8];
+  EightSymbols() = default;
   __device__ __forceinline__ EightSymbols(const int32_t *row, int at, int width) {
     if (width >= 8) {
       __builtin_memcpy(v, row + from_of(at, width), sizeof v);
@@ -255,42 +262,72 @@ __device__ __forceinline__ auto row_source(const uint16_t *w, const int32_t *t) 
   if constexpr (kWeights) return w; else return t;
 }
 
-// What bounds it: instructions.  A 6144 x 2080 matrix takes 33 us, of which 7.5
-// find the rows' extremes (25 MB read, 5 us at the copy rate), 5.5 the planes, 10 the
-// lengths (75 vector instructions for 64 places, 7.5 million over the chip), 6 the
-// way from entry to entry (a scalar read of a lane each, hidden behind the other
-// five rows of a SIMD), 2.5 the codes; 2080 x 6144: 45, with two rows a SIMD its
-// latencies show.  The walk of the trie took 472 us after 60 for the symbols and 33
-// for the extremes in torch.  Looking border strings up only where the parse comes
+// What bounds it: instructions.  A 6144 x 2080 matrix takes 31 us, of which 7.5
+// find the rows' extremes (25 MB read, 5 us at the copy rate), 4 the planes (of the
+// same registers, as far as they hold the row), 10 the lengths (75 vector instructions for 64 places,
+// 7.5 million over the chip), 6 the way from entry to entry (a scalar read of a lane each, hidden behind
+// the other five rows of a SIMD), 2.5 the codes.  The walk of the trie took 472 us after 60 for the
+// symbols and 33 for the extremes in torch.  Looking border strings up only where the parse comes
 // by them (in scalar code) measured 41, the lengths in LDS instead of registers 37.
-template <bool kWeights>
+//
+// Few, wide rows leave a SIMD one or two wavefronts, whose latencies then show, above all that way
+// (36 ns an entry).  There a workgroup's wavefronts share a row, and go from entry to entry by
+// sixteens: where sixteen entries from a place lead to is found for all places at once, by going
+// twice as far four times.  526 x 3775 with 80 % zeros: 26.4 -> 16.1 us, 1024 x 4096 with a hundredth
+// of the rows without zeros 85 -> 29, 2080 x 6144 47 -> 40.  (Shared by four wavefronts with the way entry by entry:
+// 21.9, 79 and 47; rows of fewer than 2048 weights or more of them are faster apart: 3500 x 2080 23.5
+// against 29.1, 2500 x 1500 16.1 and 19.4.)
+template <bool kWeights, bool kShared>
 __global__ __launch_bounds__(64 * kPackWaves) void pack_rows_kernel(PackArgs a) {
   extern __shared__ uint32_t pack_lds[];
   if (a.foreign && *a.foreign) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = blockIdx.x * kPackWaves + wave;
+  constexpr int kSharing = kShared ? kPackWaves : 1;   // wavefronts of a row
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row = kShared ? blockIdx.x : blockIdx.x * kPackWaves + wave;
+  const int sub = kShared ? wave : 0;
+  const auto row_fence = [&]() {
+    if (kShared)
+      __syncthreads();
+    else
+      wave_lds_fence();
+  };
+  // (asked for first, and put into LDS behind the row's extremes)
   uint32_t *border = pack_lds;
-  for (int i = threadIdx.x; i < kBorderStrings / 32; i += 64 * kPackWaves) border[i] = a.tables.border[i];
-  __syncthreads();
-  if (row >= a.height) return;
+  constexpr int kBorderTurns = (kBorderStrings / 32 + 64 * kPackWaves - 1) / (64 * kPackWaves);
+  uint32_t border_part[kBorderTurns];
+#pragma unroll
+  for (int k = 0; k < kBorderTurns; k++)
+    border_part[k] = a.tables.border[min(static_cast<int>(threadIdx.x) + 64 * kPackWaves * k, kBorderStrings / 32 - 1)];
+  const bool mine = row < a.height;
   const int words = plane_words(a.window);
-  uint32_t *nz_plane = pack_lds + kBorderLdsWords + wave * (pack_lds_per_wave(a.window) / 4);
+  uint32_t *nz_plane = pack_lds + kBorderLdsWords + (kShared ? 0 : wave) * (pack_lds_per_row(a.window, kShared) / 4);
   uint32_t *mx_plane = nz_plane + words;
   uint16_t *entry_at = reinterpret_cast<uint16_t *>(mx_plane + words);
+  int *told = reinterpret_cast<int *>(entry_at + (a.window + 7) / 8 * 8);   // kShared
+  uint8_t *longest_at = reinterpret_cast<uint8_t *>(told + 2 * kPackWaves);
+  const int places = (a.window + 15) / 16 * 16;
+  uint16_t *jump = reinterpret_cast<uint16_t *>(longest_at + places);
   const int64_t row_first = static_cast<int64_t>(row) * a.width;
   const uint16_t *w = kWeights ? a.weights + row_first : nullptr;
   int32_t *t = kWeights ? nullptr : a.symbols + row_first;
 
   // the row's smallest and largest weight, and what finds them: bits sought, under a mask
   uint32_t low = 0, high = 0, low_mask = 0, high_mask = 0;
-  if (kWeights) {
+  using Loaded = std::conditional_t<kWeights, EightWeights, EightSymbols>;
+  Loaded kept[kAhead] = {};   // kWeights: the row's first ones
+  if (kWeights && mine) {
     i16x2 least = {0x7fff, 0x7fff}, most = {-0x8000, -0x8000};
-    for (int c0 = 8 * lane; c0 - 8 * lane < a.width; c0 += 512 * kAhead) {
-      EightWeights v[kAhead] = {{w, c0, a.width}, {w, c0 + 512, a.width}, {w, c0 + 1024, a.width},
-                                {w, c0 + 1536, a.width}};
+    constexpr int kStep = 512 * kSharing;
+    for (int c0 = 8 * lane + 512 * sub; c0 - 8 * lane < a.width; c0 += kStep * kAhead) {
+      EightWeights v[kAhead] = {{w, c0, a.width}, {w, c0 + kStep, a.width}, {w, c0 + 2 * kStep, a.width},
+                                {w, c0 + 3 * kStep, a.width}};
+      if constexpr (kWeights)
+        if (c0 < kStep)
+#pragma unroll
+          for (int u = 0; u < kAhead; u++) kept[u] = v[u];
 #pragma unroll
       for (int u = 0; u < kAhead; u++) {
-        if (c0 - 8 * lane + 512 * u >= a.width) break;
+        if (c0 - 8 * lane + kStep * u >= a.width) break;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
           const i16x2 o = ordered(__builtin_bit_cast(i16x2, v[u].v[j]));
@@ -304,17 +341,35 @@ __global__ __launch_bounds__(64 * kPackWaves) void pack_rows_kernel(PackArgs a) 
       l = min(l, __shfl_xor(l, m, 64));
       h = max(h, __shfl_xor(h, m, 64));
     }
+    if (kShared) {
+      if (lane == 0) {
+        told[2 * wave] = l;
+        told[2 * wave + 1] = h;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < kPackWaves; k++) {
+        l = min(l, told[2 * k]);
+        h = max(h, told[2 * k + 1]);
+      }
+      __syncthreads();
+    }
     low = static_cast<uint16_t>(ordered_one(static_cast<int16_t>(l)));
     high = static_cast<uint16_t>(ordered_one(static_cast<int16_t>(h)));
     const bool nan = h > 0x7f80 || l < ordered_one(static_cast<int16_t>(0xff80));
     if (nan) low = high = 0x7fc0;   // a NaN makes both NaN, and nothing equals one
-    if (lane == 0) a.minmax[row] = low | high << 16;
+    if (lane == 0 && sub == 0) a.minmax[row] = low | high << 16;
     low_mask = low & 0x7fffu ? 0xffffffffu : 0x7fff7fffu;
     high_mask = high & 0x7fffu ? 0xffffffffu : 0x7fff7fffu;
     if (nan) low_mask = high_mask = 0;   // (x & 0) ^ 0x7fc0 is never zero
     low = (low | low << 16) & (nan ? ~0u : low_mask);
     high = (high | high << 16) & (nan ? ~0u : high_mask);
   }
+#pragma unroll
+  for (int k = 0; k < kBorderTurns; k++)
+    border[min(static_cast<int>(threadIdx.x) + 64 * kPackWaves * k, kBorderStrings / 32 - 1)] = border_part[k];
+  __syncthreads();
+  if (!mine) return;
 
   const int pairs = (a.width + 1) / 2;
   int first = 0, out = 0;   // the window's first pair, the row's codes so far
@@ -323,15 +378,21 @@ __global__ __launch_bounds__(64 * kPackWaves) void pack_rows_kernel(PackArgs a) 
     const int col0 = 2 * first;
     // eight symbols a lane to a byte of either plane, zeros past the row's end
     const int bytes = min(4 * words, (a.width - col0 + 7) / 8 + 8);   // with zeros to look ahead into
-    for (int b0 = lane; b0 - lane < bytes; b0 += 64 * kAhead) {
-      using Loaded = std::conditional_t<kWeights, EightWeights, EightSymbols>;
+    constexpr int kStep = 64 * kSharing;   // bytes
+    for (int b0 = lane + 64 * sub; b0 - lane < bytes; b0 += kStep * kAhead) {
       const auto *src = row_source<kWeights>(w, t);
       const int c0 = col0 + 8 * b0;
-      Loaded v[kAhead] = {{src, c0, a.width}, {src, c0 + 512, a.width}, {src, c0 + 1024, a.width},
-                          {src, c0 + 1536, a.width}};
+      Loaded v[kAhead];
+      if (kWeights && c0 < 8 * kStep) {   // (of the first window)
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) v[u] = kept[u];
+      } else {
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) v[u] = Loaded(src, c0 + 8 * kStep * u, a.width);
+      }
 #pragma unroll
       for (int u = 0; u < kAhead; u++) {
-        if (b0 - lane + 64 * u >= bytes) break;
+        if (b0 - lane + kStep * u >= bytes) break;
         uint32_t nz, mx;
         if constexpr (kWeights) {
           uint32_t not_mx[4], neither[4];
@@ -349,7 +410,7 @@ __global__ __launch_bounds__(64 * kPackWaves) void pack_rows_kernel(PackArgs a) 
           nz = even_bits(both | both >> 1);
           mx = even_bits(both >> 1);
         }
-        const int b = b0 + 64 * u;
+        const int b = b0 + kStep * u;
         if (b < bytes) {
           const int at = col0 + 8 * b;
           reinterpret_cast<uint8_t *>(nz_plane)[b] = static_cast<uint8_t>(eight_bits(nz, at, a.width));
@@ -357,53 +418,103 @@ __global__ __launch_bounds__(64 * kPackWaves) void pack_rows_kernel(PackArgs a) 
         }
       }
     }
-    wave_lds_fence();
-    // The longest entry at every pair, a lane each, two runs of 64 at a time: up to
-    // the pair of the third non-zero, or up to that of the fourth as far as entries
-    // with three reach.  Then from entry to entry by scalar reads of the lengths.
+    row_fence();
+    // The longest entry at every pair, a lane each: up to the pair of the third
+    // non-zero, or up to that of the fourth as far as entries with three reach.
+    const auto longest_from = [&](int p) {
+      const uint32_t nz = plane_bits(nz_plane, 2 * p);
+      uint32_t rest = nz & (nz - 1);
+      rest &= rest - 1;                                                        // from the third non-zero on
+      const uint32_t end = 1u << kLookahead;
+      const int upto2 = __builtin_ctz(rest | end) >> 1;
+      const uint32_t rest3 = rest & (rest - 1);
+      const int upto3 = min(__builtin_ctz(rest3 | end) >> 1, kBorderPairs);
+      const int longest = min(max(upto2, upto3), pairs - first - p);
+      // for every lane, so that several runs' LDS reads are in flight together: a
+      // string of other than three non-zeros looks up something within the table
+      const uint32_t three = (nz & ((1u << (2 * kBorderPairs)) - 1)) | 7u << (2 * kBorderPairs);
+      const int i = min(string_places(three, plane_bits(mx_plane, 2 * p), kFreeNonzeros + 1), kBorderStrings - 1);
+      const int entry = (border[i >> 5] >> (i & 31)) & 1u;
+      const bool at_border = upto3 == kBorderPairs && upto2 < kBorderPairs && longest == kBorderPairs;
+      return at_border ? kBorderPairs - 1 + entry : longest;
+    };
     int n = 0, at = 0;   // entries found, the pair after the last of them
-    for (int p0 = 0; p0 < here; p0 += 128) {
-      int len[2];
-#pragma unroll
-      for (int u = 0; u < 2; u++) {
-        const int p = min(p0 + 64 * u + lane, here - 1);
-        const uint32_t nz = plane_bits(nz_plane, 2 * p);
-        uint32_t rest = nz & (nz - 1);
-        rest &= rest - 1;                                                        // from the third non-zero on
-        const uint32_t end = 1u << kLookahead;
-        const int upto2 = __builtin_ctz(rest | end) >> 1;
-        const uint32_t rest3 = rest & (rest - 1);
-        const int upto3 = min(__builtin_ctz(rest3 | end) >> 1, kBorderPairs);
-        const int longest = min(max(upto2, upto3), pairs - first - p);
-        // for every lane, so that the two runs' LDS reads are in flight together: a
-        // string of other than three non-zeros looks up something within the table
-        const uint32_t three = (nz & ((1u << (2 * kBorderPairs)) - 1)) | 7u << (2 * kBorderPairs);
-        const int i = min(string_places(three, plane_bits(mx_plane, 2 * p), kFreeNonzeros + 1), kBorderStrings - 1);
-        const int entry = (border[i >> 5] >> (i & 31)) & 1u;
-        const bool at_border = upto3 == kBorderPairs && upto2 < kBorderPairs && longest == kBorderPairs;
-        len[u] = at_border ? kBorderPairs - 1 + entry : longest;
-      }
-#pragma unroll
-      for (int u = 0; u < 2; u++) {
-        const int limit = min(here - p0 - 64 * u, 64);
-        unsigned long long starts = 0;
-        int q = at - p0 - 64 * u;
-        while (q < limit) {
-          starts |= 1ull << q;
-          q += __builtin_amdgcn_readlane(len[u], q);
+    if constexpr (kShared) {
+      const int thread = threadIdx.x;
+      for (int p0 = 0; p0 < here; p0 += 64 * kPackWaves) {
+        const int p = p0 + thread, len = longest_from(min(p, here - 1));
+        if (p < here) {
+          longest_at[p] = static_cast<uint8_t>(len);
+          jump[p] = static_cast<uint16_t>(p + len);
         }
-        at = p0 + 64 * u + q;
-        if ((starts >> lane) & 1)
-          entry_at[n + __popcll(starts & ((1ull << lane) - 1))] = static_cast<uint16_t>(p0 + 64 * u + lane);
-        n += __popcll(starts);
+      }
+      __syncthreads();
+      // Where two entries from a pair lead to, then four, eight, sixteen.
+#pragma unroll
+      for (int round = 0; round < kJumpRounds; round++) {
+        const uint16_t *from = jump + (round & 1 ? places : 0);
+        uint16_t *to = jump + (round & 1 ? 0 : places);
+        for (int p = thread; p < here; p += 64 * kPackWaves) {
+          const int q = from[p];
+          to[p] = q < here ? from[q] : static_cast<uint16_t>(q);
+        }
+        __syncthreads();
+      }
+      // Every sixteenth entry, one after the other; then a thread goes from each to the next.
+      uint16_t *every = jump + places;   // (the last round has left it)
+      static_assert(kJumpRounds % 2 == 0 && 64 * kPackWaves << kJumpRounds >= kPackWindow, "a thread for each of these");
+      if (sub == 0) {
+        int steps = 0;
+        for (; at < here; steps++) {
+          if (lane == 0) every[steps] = static_cast<uint16_t>(at);
+          at = __builtin_amdgcn_readfirstlane(jump[at]);
+        }
+        if (lane == 0) {
+          told[0] = steps;
+          told[1] = at;
+        }
+      }
+      __syncthreads();
+      const int steps = told[0];
+      at = __builtin_amdgcn_readfirstlane(told[1]);
+      if (thread < steps) {
+        int p = every[thread], i = thread << kJumpRounds;
+        for (const int end = i + (1 << kJumpRounds); i < end && p < here; i++) {
+          entry_at[i] = static_cast<uint16_t>(p);
+          p += longest_at[p];
+        }
+        if (thread == steps - 1) told[2] = i;
+      }
+      __syncthreads();
+      n = __builtin_amdgcn_readfirstlane(told[2]);
+    } else {
+      // Two runs of 64 at a time, from entry to entry by scalar reads of the lengths.
+      for (int p0 = 0; p0 < here; p0 += 128) {
+        int len[2];
+#pragma unroll
+        for (int u = 0; u < 2; u++) len[u] = longest_from(min(p0 + 64 * u + lane, here - 1));
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          const int limit = min(here - p0 - 64 * u, 64);
+          unsigned long long starts = 0;
+          int q = at - p0 - 64 * u;
+          while (q < limit) {
+            starts |= 1ull << q;
+            q += __builtin_amdgcn_readlane(len[u], q);
+          }
+          at = p0 + 64 * u + q;
+          if ((starts >> lane) & 1)
+            entry_at[n + __popcll(starts & ((1ull << lane) - 1))] = static_cast<uint16_t>(p0 + 64 * u + lane);
+          n += __popcll(starts);
+        }
       }
     }
-    wave_lds_fence();
-    for (int i0 = 0; i0 < n; i0 += 64 * kAhead) {
+    if (!kShared) wave_lds_fence();
+    for (int i0 = 64 * sub; i0 < n; i0 += 64 * kSharing * kAhead) {
       uint16_t code[kAhead];
 #pragma unroll
       for (int u = 0; u < kAhead; u++) {
-        const int i = i0 + 64 * u + lane;
+        const int i = i0 + 64 * kSharing * u + lane;
         if (i < n) {
           const int from = entry_at[i];
           const int len = (i + 1 < n ? entry_at[i + 1] : at) - from;
@@ -414,7 +525,7 @@ __global__ __launch_bounds__(64 * kPackWaves) void pack_rows_kernel(PackArgs a) 
       }
 #pragma unroll
       for (int u = 0; u < kAhead; u++) {
-        const int i = i0 + 64 * u + lane;
+        const int i = i0 + 64 * kSharing * u + lane;
         if (i < n) {
           if (kWeights)
             a.codes[static_cast<int64_t>(row) * pairs + out + i] = code[u];
@@ -425,9 +536,9 @@ __global__ __launch_bounds__(64 * kPackWaves) void pack_rows_kernel(PackArgs a) 
     }
     out += n;
     first += at;
-    wave_lds_fence();
+    row_fence();
   }
-  if (lane == 0) a.row_cnt[row + 1] = out;
+  if (lane == 0 && sub == 0) a.row_cnt[row + 1] = out;
 }
 
 // ---------------------------------------------------- a caller's own trie ---
@@ -520,8 +631,15 @@ int check_pack_shape(const char *who, int height, int width) {
 template <bool kWeights>
 int launch_pack_rows(PackArgs &a, hipStream_t s) {
   a.window = std::min((a.width + 1) / 2, kPackWindow);
-  pack_rows_kernel<kWeights><<<(a.height + kPackWaves - 1) / kPackWaves, 64 * kPackWaves,
-                               kBorderLdsWords * 4 + kPackWaves * pack_lds_per_wave(a.window), s>>>(a);
+  int device = 0, cus = 0;
+  HIP_TRY(hipGetDevice(&device));
+  HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+  if (a.width >= kSharedWidth && a.height <= kSharedRows * cus)
+    pack_rows_kernel<kWeights, true><<<a.height, 64 * kPackWaves,
+                                       kBorderLdsWords * 4 + pack_lds_per_row(a.window, true), s>>>(a);
+  else
+    pack_rows_kernel<kWeights, false><<<(a.height + kPackWaves - 1) / kPackWaves, 64 * kPackWaves,
+                                        kBorderLdsWords * 4 + kPackWaves * pack_lds_per_row(a.window, false), s>>>(a);
   HIP_TRY(hipGetLastError());
   return SUB1_OK;
 }

@@ -201,6 +201,27 @@ def test_weights_pack_like_their_symbols(gpu, oracle, height, width, share):
     assert torch.equal(p_comp, w_comp) and torch.equal(p_off, row_off)
 
 
+@pytest.mark.parametrize('width', [2047, 2048, 2300, 4096, 8194, 16400])   # a form for narrow rows; one window and several
+def test_rows_pack_alike_alone_and_by_a_workgroup(gpu, width):
+    """Few wide rows are packed by a workgroup each, many by a wavefront each: the same codes."""
+    sub1, op = gpu
+    rows, cus = 40, torch.cuda.get_device_properties(0).multi_processor_count
+    symbols = symbols_of(rows, width, [0.1, 0.05, 0.0, 1.0, 0.3], seed=width)
+    symbols[7, :width // 2] = 0                                   # entries of many and of few pairs, and where they meet
+    symbols[8, width // 3:] = 0
+    w = torch.tensor([0.0, -1.0, 1.0], device='cuda')[symbols.long()].bfloat16()
+    few = op.sub1pack_weights(w)
+    many = op.sub1pack_weights(w.repeat(10 * cus // rows + 1, 1))
+    codes = few[0].numel()
+    assert torch.equal(many[1][:rows + 1], few[1]) and torch.equal(many[0][:codes], few[0])
+    assert torch.equal(many[0][-codes:], few[0])
+    symbols, _ = symbols_by_torch(w)
+    s_comp, s_off = packed(gpu, symbols)
+    assert torch.equal(s_comp, few[0]) and torch.equal(s_off, few[1])
+    m_comp, _ = packed(gpu, symbols.repeat(10 * cus // rows + 1, 1))
+    assert torch.equal(m_comp, many[0])
+
+
 def test_packing_with_a_trie_of_ones_own(gpu):
     """A trie that is not the fixed dictionary's (here: cut off below three
     pairs, and with the symbols' order of a few entries changed) is walked as it
