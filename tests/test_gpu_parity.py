@@ -121,6 +121,48 @@ def test_matvec_against_oracle(gpu, oracle, height, width, p0):
     check_product(oracle, c, bits_host(y))
 
 
+def test_matvec_of_long_rows_and_of_entries_with_many_digits(gpu):
+    """Rows of a run of 64 codes, of a turn of 256 and of several, a code more and less; and a
+    dictionary with entries of four and 28 non-zeros.  Sums of small whole numbers: exact in any order."""
+    sub1, op = gpu
+    g = torch.Generator().manual_seed(3)
+    lengths = [1, 63, 64, 65, 255, 256, 257, 511, 512, 513, 1000]
+    width = 2 * max(lengths) + 28 * 11
+    dec = sub1.dec.clone()
+    digits = torch.zeros((3, 28), dtype=torch.int64)            # of three codes with entries of their own
+    digits[0, [0, 3, 4, 11]], digits[1], digits[2, [1, 27]] = torch.tensor([1, 2, 2, 1]), 2, 1
+    own = [65535, 40000, 17]
+    for code, d in zip(own, digits):
+        for half in (0, 1):
+            word = sum(int(v) << (4 + 2 * i) for i, v in enumerate(d[14 * half:14 * half + 14])) | (14 if half == 0 else 0)
+            dec[2 * code + half] = word - (1 << 32) if word >= 1 << 31 else word
+    pair = next(c for c in range(65536) if c not in own and (int(dec[2 * c]) & 15) == 1 and int(dec[2 * c]) >> 4 & 15 == 9)
+    codes, off, dense = [], [0], torch.zeros((len(lengths), width + 28), dtype=torch.int64)
+    for r, n in enumerate(lengths):                             # pairs (1, 2), with an own entry now and then
+        at = 0
+        for i in range(n):
+            if i % 97 == 5:
+                which = i % 3
+                codes.append(own[which])
+                dense[r, at:at + 28] = digits[which]
+                at += 28
+            else:
+                codes.append(pair)
+                dense[r, at], dense[r, at + 1] = 1, 2
+                at += 2
+        off.append(len(codes))
+    codes[0], dense[0, :28] = own[1], 2                         # one code of 28
+    x = torch.randint(-3, 4, (width,), generator=g)
+    want = torch.where(dense[:, :width] == 1, -1, torch.where(dense[:, :width] == 2, 2, 0)) @ x
+    dev = lambda t: t.cuda()
+    minmax = dev(torch.tensor([-1.0, 2.0] * len(lengths)).bfloat16())
+    y = torch.zeros(len(lengths), dtype=torch.bfloat16, device='cuda')
+    own_dec = dev(dec)
+    op.sub1matvec(own_dec, dev(torch.tensor(codes, dtype=torch.int32).to(torch.int16)), dev(torch.tensor(off, dtype=torch.int32)),
+                  minmax, dev(x.bfloat16()), y)
+    assert torch.equal(y.cpu(), want.float().bfloat16())
+
+
 def test_matvec_accumulates_into_y(gpu, oracle):
     sub1, op = gpu
     c = dev_case(oracle, 200, 512, 0.9, seed=5)
