@@ -41,7 +41,7 @@ def kernels_with_scratch(compiler_output):
 
 # Kernels known to spill, and how many bytes per lane: the fused kernel's form for
 # tokens grouped by expert keeps four tokens' sums per lane.
-SPILLS_ACCEPTED = {'_ZN12_GLOBAL__N_125moe_prepared_fused_kernelILb1ELb0EEEvNS_12PreparedArgsE': 36}
+SPILLS_ACCEPTED = {'_ZN12_GLOBAL__N_125moe_prepared_fused_kernelILb1ELb0ELb0EEEvNS_12PreparedArgsE': 36}
 
 
 def torch_mark():

@@ -1801,10 +1801,10 @@ __device__ __forceinline__ void publish_h(const PreparedArgs &a, int t) {
 // slice, each a run of its chunk groups, partial sums in `partials`
 // (a.tail_room groups of 64 lanes).
 template <class Before, class Out>
-__device__ __forceinline__ void walk_tile(const PreparedArgs &a, const KindArgs &k, int64_t first,
-                                          int stride, int all, const uint32_t *act,
-                                          float *partials, Before &&before, Out &&out,
-                                          bool active = true) {
+__device__ __forceinline__ void walk_alike(const PreparedArgs &a, const KindArgs &k, int64_t first,
+                                           int stride, int all, const uint32_t *act,
+                                           float *partials, Before &&before, Out &&out,
+                                           bool active = true) {
   const int waves = blockDim.x >> 6;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int split = 1;
@@ -1884,6 +1884,143 @@ __device__ __forceinline__ void walk_tile(const PreparedArgs &a, const KindArgs 
   }
 }
 
+// The slices that all of a workgroup's wavefronts share, where lengths differ: the
+// longest ones, each by as many wavefronts as make their shares alike.
+struct SharedSlices {
+  int slice;            // this wavefront's, among the shared ones; -1: none
+  int split, sub;       // the wavefronts that share it, and which of them this is
+  int groups, first_group;   // its groups; where their partial sums begin
+  int len;
+  uint32_t base;
+};
+
+// `count` slices (at most half of `waves`) from `first` on, every `stride`-th.  A row without zeros
+// has ten times the entries of the others, and a slice of 64 such rows kept one or two
+// wavefronts walking long after the rest.
+__device__ __forceinline__ SharedSlices share_slices(const PreparedArgs &a, const KindArgs &k, int64_t first, int stride,
+                                                     int count, int waves, int wave) {
+  const int lane = threadIdx.x & 63;
+  const int64_t sl = first + static_cast<int64_t>(min(lane, count - 1)) * stride;
+  const int len = k.slice_len[sl];
+  const uint32_t base = k.slice_base[sl];
+  const bool mine = lane < count;
+  const int groups = mine ? (chunks_of(len) + kGroupChunks - 1) / kGroupChunks : 0;
+  const int total = __builtin_amdgcn_readlane(sub1::wave_prefix_sum(groups), 63);
+  // the fewest groups a wavefront may have at most with which there are wavefronts enough, and room
+  // for the partial sums of the slices that several share (at the latest with as many as the longest has)
+  int split, split_upto, partials, partials_upto;
+  for (int most = max((total + waves - 1) / waves, 1);; most++) {
+    split = mine ? max((groups + most - 1) / most, 1) : 0;
+    partials = split > 1 ? groups : 0;
+    split_upto = sub1::wave_prefix_sum(split);
+    partials_upto = sub1::wave_prefix_sum(partials);
+    if (__builtin_amdgcn_readlane(split_upto, 63) <= waves && __builtin_amdgcn_readlane(partials_upto, 63) <= a.tail_room)
+      break;
+  }
+  const int which = __popcll(__ballot(mine && split_upto - split <= wave)) - 1;
+  SharedSlices s;
+  s.split = __builtin_amdgcn_readlane(split, which);
+  s.sub = wave - (__builtin_amdgcn_readlane(split_upto, which) - s.split);
+  s.slice = s.sub < s.split ? which : -1;
+  s.groups = __builtin_amdgcn_readlane(groups, which);
+  s.first_group = __builtin_amdgcn_readlane(partials_upto, which) - __builtin_amdgcn_readlane(partials, which);
+  s.len = __builtin_amdgcn_readlane(len, which);
+  s.base = __builtin_amdgcn_readlane(base, which);
+  return s;
+}
+
+// As walk_alike, where lengths differ: the last pass has the longest slices instead, as many as make the
+// passes before it full or half as many as there are wavefronts, and the wavefronts by length.
+//
+// Bound by the longest slice's chain of groups: a wavefront walked it alone, or a few did where eight
+// slices' partial sums, at the longest one's size, fit LDS (beyond rows of some 4400 columns without zeros they
+// did not, and the launch fell back on tiles of one projection).  Rows of 75 to 98 % zeros, one in a
+// hundred without, us before / so: 587 x 4467 one token 22.5 / 18.7, 60 tokens 106 / 31, 200 108 / 62;
+// c-2048 13 tokens 48.6 / 33.7, 60 104 / 66, 120 197 / 105, 512 418 / 376; large 60 47 / 33, 200 120 / 85; base 60
+// 36 / 26, 400 110 / 88.  (With sixteen slices in that pass, a wavefront each at least, large 200 took 136.)
+template <class Before, class Out>
+__device__ __forceinline__ void walk_by_length(const PreparedArgs &a, const KindArgs &k, int64_t first,
+                                               int stride, int all, const uint32_t *act,
+                                               float *partials, Before &&before, Out &&out,
+                                               bool active = true) {
+  const int waves = blockDim.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int rest = all % waves;
+  // (each has a wavefront at least, so that more than half as many slices would leave the longest too few)
+  const int longest = rest && 2 * rest <= waves ? rest : min(all, waves / 2);
+  const int count = all - longest, passes = (count + waves - 1) / waves + 1;
+  SharedSlices mine;
+  mine.slice = -1;
+  if (longest == 1) {
+    const int len_word = k.slice_len[first];
+    const uint32_t base_word = k.slice_base[first];
+    mine.len = __builtin_amdgcn_readfirstlane(len_word);
+    mine.base = __builtin_amdgcn_readfirstlane(base_word);
+    mine.groups = (chunks_of(mine.len) + kGroupChunks - 1) / kGroupChunks;
+    mine.split = waves;
+    mine.sub = wave;
+    mine.slice = 0;
+    mine.first_group = 0;
+  } else if (longest) {
+    mine = share_slices(a, k, first, stride, longest, waves, wave);
+  }
+  const int64_t slice = first + static_cast<int64_t>(max(mine.slice, 0)) * stride;
+  const bool shares = mine.slice >= 0 && active;
+  int g_lo = 0, g_hi = 0;
+  if (shares) {
+    g_lo = mine.sub * mine.groups / mine.split;
+    g_hi = (mine.sub + 1) * mine.groups / mine.split;
+  }
+  float *sums = shares && mine.split > 1 ? partials + mine.first_group * 64 : nullptr;
+  // where that pass is the whole walk its loads go out before the wait and the staging
+  Walk<kSplitRing> ahead;
+  int ridx = 0xffff;   // the rows of the slice, in the wavefront that adds them up
+  if (shares && mine.sub == 0) ridx = k.row_idx[slice * 64 + lane];
+  if (count == 0 && g_lo < g_hi) ahead = load_slice_described<kSplitRing>(a, k, slice, mine.len, mine.base, g_lo, g_hi);
+  first += static_cast<int64_t>(longest) * stride;
+  int s = slice_of_pass(0, wave, waves, count);
+  SliceWalk cur;
+  if (s < count && active) cur = load_slice(a, k, first + static_cast<int64_t>(s) * stride);
+  before();
+  for (int pass = 0; s < count; pass++) {
+    const int s_next = slice_of_pass(pass + 1, wave, waves, count);
+    SliceWalk nxt;
+    if (active) {
+      if (s_next < count) nxt = load_slice(a, k, first + static_cast<int64_t>(s_next) * stride);
+      const float res = run_slice(cur, a.stream, act, nullptr, pass, passes);
+      out(cur.ridx, res, first + static_cast<int64_t>(s) * stride);
+      if (s_next < count) cur = nxt;
+    }
+    s = s_next;
+  }
+  __builtin_amdgcn_s_setprio(0);
+  float sum = 0.f;
+  if (g_lo < g_hi) {
+    if (count == 0) {
+      sum = run_slice(ahead, a.stream, act, sums);
+    } else {
+      SliceWalk walk = load_slice_described(a, k, slice, mine.len, mine.base, g_lo, g_hi);
+      sum = run_slice(walk, a.stream, act, sums);
+    }
+  }
+  __syncthreads();
+  if (shares && mine.sub == 0) {
+    if (sums) {
+      sum = 0.f;
+#pragma unroll 8
+      for (int g = 0; g < mine.groups; g++) sum += sums[g * 64 + lane];
+    }
+    out(ridx, sum, slice);
+  }
+}
+
+// (A form of its own of each kernel: the choice within one cost even rows 0.2 us of 12.)
+template <bool kUneven, class... Args>
+__device__ __forceinline__ void walk_tile(const PreparedArgs &a, const KindArgs &k, Args &&...args) {
+  if constexpr (kUneven) walk_by_length(a, k, static_cast<Args &&>(args)...);
+  else walk_alike(a, k, static_cast<Args &&>(args)...);
+}
+
 // Persistent grid.  A tile is (token, projection, part): the slices of one
 // matrix, or of one of `parts` equal ranges of them when there are too few
 // tokens to occupy the GPU otherwise; a workgroup stages the token's
@@ -1895,6 +2032,7 @@ __device__ __forceinline__ void walk_tile(const PreparedArgs &a, const KindArgs 
 // stores and the workgroup barrier) and picked up by one acquire; an agent-scope
 // fence costs an L2 write-back on this part, which is why the lanes do not fence
 // individually.
+template <bool kUneven>
 __global__ __launch_bounds__(kMaxThreads) void moe_prepared_kernel(PreparedArgs a) {
   extern __shared__ __align__(16) uint32_t lds[];
   __shared__ int s_ticket;
@@ -1937,7 +2075,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_kernel(PreparedArgs 
     if (e >= 0) {
       int mode;
       uint16_t *dst = tile_output(a, k, kind, t, mode);
-      walk_tile(a, k, static_cast<int64_t>(e) * k.slices + s_lo, 1, s_hi - s_lo, xa,
+      walk_tile<kUneven>(a, k, static_cast<int64_t>(e) * k.slices + s_lo, 1, s_hi - s_lo, xa,
                 reinterpret_cast<float *>(xa + a.xdwords),
                 [&]() { await_activations(a, k, kind, t, xa); },
                 [&](int ridx, float res, int64_t) { write_row(dst, ridx, res, mode); });
@@ -2135,8 +2273,8 @@ __device__ __forceinline__ void fused_group_tile(const PreparedArgs &a, uint32_t
 // LDS, already in the layout wo reads its activations from.  No workspace
 // traffic for h, no waiting between workgroups; tickets only balance the load.
 // LDS: x (wi's activations) | h (wo's activations).
-// kOnce: see load_chunk.
-template <bool kGrouped, bool kOnce>
+// kOnce: see load_chunk.  kUneven: the longest slices are shared (walk_tile; LDS: x | h | partial sums).
+template <bool kGrouped, bool kOnce, bool kUneven = false>
 __global__ __launch_bounds__(kMaxThreads) void moe_prepared_fused_kernel(PreparedArgs a) {
   typedef Walk<kRing, kOnce> TokenWalk;
   extern __shared__ __align__(16) uint32_t lds[];
@@ -2192,6 +2330,29 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_fused_kernel(Prepare
     }
     // wi: x -> relu(h) into LDS
     const int64_t first_i = static_cast<int64_t>(e) * ki.slices;
+    if constexpr (kUneven) {
+      float *partials = reinterpret_cast<float *>(ha + a.hdwords);
+      walk_tile<true>(a, ki, first_i, 1, ki.slices, xa, partials,
+                      [&]() {
+                        stage_activations(xa, a.x + static_cast<int64_t>(t) * a.ldx, ki.width);
+                        __syncthreads();
+                      },
+                      [&](int ridx, float res, int64_t) {
+                        if (ridx == 0xffff) return;
+                        uint32_t out = f32_to_bf16(res);
+                        if (out & 0x8000u) out = 0;
+                        uint32_t *p = ha + 2 * physical_column(ridx);
+                        p[0] = out;
+                        p[1] = out << 16;
+                      });
+      fetch_next();
+      uint16_t *dst = a.y + static_cast<int64_t>(t) * a.ldy;
+      walk_tile<true>(a, ko, static_cast<int64_t>(e) * ko.slices, 1, ko.slices, ha, partials,
+                      [&]() { __syncthreads(); },
+                      [&](int ridx, float res, int64_t) { write_row(dst, ridx, res, kStore); });
+      __builtin_amdgcn_s_setprio(0);
+      continue;
+    }
     int s = slice_of_pass(0, wave, waves, ki.slices);
     TokenWalk cur;
     if (s < ki.slices) cur = load_slice<kRing, kOnce>(a, ki, first_i + s);
@@ -2451,6 +2612,7 @@ __device__ __forceinline__ void leave_tagged(int32_t *ctrl, int workgroups) {
 // then hold the lowest places, the places of a token are consecutive, so at
 // most one token is partly on the GPU whatever order the hardware starts
 // workgroups in; all others run to completion and make room.
+template <bool kUneven>
 __global__ __launch_bounds__(kMaxThreads) void moe_prepared_shared_kernel(PreparedArgs a) {
   extern __shared__ __align__(16) uint32_t lds[];
   __shared__ int s_place;
@@ -2484,7 +2646,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_shared_kernel(Prepar
     return;
   }
   uint16_t *h = a.h + static_cast<int64_t>(t) * ki.height;
-  walk_tile(a, ki, static_cast<int64_t>(e) * ki.slices + part, parts,
+  walk_tile<kUneven>(a, ki, static_cast<int64_t>(e) * ki.slices + part, parts,
             (ki.slices - part + parts - 1) / parts, xa, partials,
             [&]() {
               stage_finish(xa, x, ki.width, x_ahead);
@@ -2493,7 +2655,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_shared_kernel(Prepar
             [&](int ridx, float res, int64_t) { write_row(h, ridx, res, kStoreRelu); });
   publish_h(a, t);
   uint16_t *y = a.y + static_cast<int64_t>(t) * a.ldy;
-  walk_tile(a, ko, static_cast<int64_t>(e) * ko.slices + part, parts,
+  walk_tile<kUneven>(a, ko, static_cast<int64_t>(e) * ko.slices + part, parts,
             (ko.slices - part + parts - 1) / parts, xa, partials,
             [&]() { await_activations(a, ko, 1, t, xa); },
             [&](int ridx, float res, int64_t) { write_row(y, ridx, res, kStore); });
@@ -2505,6 +2667,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_shared_kernel(Prepar
 // await_tagged): no drain, no barrier, no count between the projections, and no
 // word to give back at the end.  A workgroup's place is its index: the grid is
 // at most 64 workgroups.
+template <bool kUneven>
 __global__ __launch_bounds__(kMaxThreads) void moe_prepared_tagged_kernel(PreparedArgs a) {
   extern __shared__ __align__(16) uint32_t lds[];
   uint32_t *xa = lds;
@@ -2533,7 +2696,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_tagged_kernel(Prepar
     return;
   }
   unsigned long long *ht = a.tagged + static_cast<int64_t>(t) * sub1::kTaggedWidth;
-  walk_tile(a, ki, static_cast<int64_t>(e) * ki.slices + part, parts,
+  walk_tile<kUneven>(a, ki, static_cast<int64_t>(e) * ki.slices + part, parts,
             (ki.slices - part + parts - 1) / parts, xa, partials,
             [&]() {
               stage_finish(xa, x, ki.width, x_ahead);
@@ -2544,7 +2707,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_tagged_kernel(Prepar
   uint16_t *y = a.y + static_cast<int64_t>(t) * a.ldy;
   // (a test that overstates the wait looks for a tag that nobody writes)
   const unsigned long long want = a.wi_expect == parts ? tag : tag + 1;
-  walk_tile(a, ko, static_cast<int64_t>(e) * ko.slices + part, parts,
+  walk_tile<kUneven>(a, ko, static_cast<int64_t>(e) * ko.slices + part, parts,
             (ko.slices - part + parts - 1) / parts, xa, partials,
             [&]() { await_tagged(a, ko, ht, want, xa); },
             [&](int ridx, float res, int64_t) { write_row(y, ridx, res, kStore); });
@@ -2567,6 +2730,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_tagged_kernel(Prepar
 // expert 11.5 -> 10.7, a large one 11.7 -> 11.5.
 // 62 KB of code, each instruction of it run about once: where it lies makes 0.15 us
 // (the same instructions behind kernels of another size 11.83 and 11.97), so it has a place of its own.
+template <bool kUneven>
 __global__ __launch_bounds__(kMaxThreads) __attribute__((aligned(65536)))
 void moe_prepared_tagged_split_kernel(PreparedArgs a) {
   extern __shared__ __align__(16) uint32_t lds[];
@@ -2599,7 +2763,7 @@ void moe_prepared_tagged_split_kernel(PreparedArgs a) {
   }
   unsigned long long *ht = a.tagged + static_cast<int64_t>(t) * sub1::kTaggedWidth;
   if (!for_wo) {
-    walk_tile(a, ki, static_cast<int64_t>(e) * ki.slices + place, ki.parts,
+    walk_tile<kUneven>(a, ki, static_cast<int64_t>(e) * ki.slices + place, ki.parts,
               (ki.slices - place + ki.parts - 1) / ki.parts, xa, partials,
               [&]() {
                 stage_finish(xa, x, ki.width, x_ahead);
@@ -2619,7 +2783,7 @@ void moe_prepared_tagged_split_kernel(PreparedArgs a) {
     uint16_t *y = a.y + static_cast<int64_t>(t) * a.ldy;
     // (a test that overstates the wait looks for a tag that nobody writes)
     const unsigned long long want = a.wi_expect == ki.parts ? tag : tag + 1;
-    walk_tile(a, ko, static_cast<int64_t>(e) * ko.slices + part, ko.parts,
+    walk_tile<kUneven>(a, ko, static_cast<int64_t>(e) * ko.slices + part, ko.parts,
               (ko.slices - part + ko.parts - 1) / ko.parts, xa, partials,
               [&]() {
                 await_tagged_placed(a, ko, ht,
@@ -3239,6 +3403,20 @@ double part_passes(int slices, int waves, int groups_max) {
   return passes;
 }
 
+// Chunks of an average slice of a kind, by what its width is of the stream.
+double average_chunks(const Prepared &p, int kind) {
+  double weight = 0.0;
+  for (int i = 0; i < p.kinds; i++) weight += static_cast<double>((p.height[i] + 63) / 64) * p.width[i];
+  return static_cast<double>(p.total_chunks) / p.count * p.width[kind] / weight;
+}
+
+// The longest slice of rows of one share of zeros has 1.2 to 1.4 times an average one's chunks (1.7 of 500
+// columns with 95 %, hence the two chunks), of rows of which one in a hundred has no zeros 5 to 10 times.
+// Even rows lose 0.2 us of 12 by the form for differing lengths; layers in between were not measured.
+bool is_uneven(const Prepared &p, int kind) {
+  return p.max_chunks[kind] > 2.0 * average_chunks(p, kind) + 2.0;
+}
+
 // Launch of the prepared kernels.  kinds == 2: y = wo(relu(wi x)) per token,
 // workspace required; kinds == 1: y += W x per token, no workspace.
 // `piece`: 0 for a caller's launch; 1 and 2 for the two pieces when a launch is
@@ -3333,7 +3511,7 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
   // starting from a position checkpoint.  plan_small picks the cut by estimate.
   const int want = (cus + tokens - 1) / tokens;   // tiles per token and projection
   int64_t first_slice = 0;
-  bool idle_units = false;
+  bool idle_units = false, uneven = false;
   for (int i = 0; i < p.kinds; i++) {
     KindArgs &k = a.k[i];
     k.first_slice = first_slice;
@@ -3341,6 +3519,7 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
     k.groups_max = (p.max_chunks[i] + kGroupChunks - 1) / kGroupChunks;
     k.split = 1;
     k.tail_split = 0;
+    uneven = uneven || is_uneven(p, i);
     const int max_parts = (k.slices + waves - 1) / waves;
     if (want > max_parts) idle_units = true;
     // Parts per matrix for the streaming kernel: the count that needs the fewest
@@ -3413,7 +3592,16 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
                             activation_dwords(a.k[1].width)) * 4;
   bool fused = false;
   int fused_per_cu = 1;
-  int shared_parts = 0;
+  int shared_parts = 0, shared_room = 0;
+  // Partial sums of a shared pass (walk_tile), in groups of 64 lanes: those of half the wavefronts'
+  // slices; of slices whose lengths differ what LDS has room for, the longest one's at least.
+  const auto tail_groups = [&](size_t room_bytes) {
+    const int room = static_cast<int>(room_bytes / 256);
+    int longest = 0;
+    for (int i = 0; i < p.kinds; i++) longest = std::max(longest, a.k[i].groups_max);
+    const int most = (uneven ? waves : waves / 2) * longest;
+    return most <= room ? most : uneven && longest <= room ? room : 0;
+  };
   if (p.kinds == 2 && lds_fused <= lds_limit) {
     const double token_us = 8.0 + static_cast<double>(p.total_chunks) * (64.0 * kFields) /
                                       p.count / 23400.0;
@@ -3449,12 +3637,11 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
     // the Switch shapes it is the fastest form from 2 tokens (1 for the smaller
     // shapes) to half the compute units: 1.1 to 1.5 times faster than cutting
     // by projection.
-    const size_t lds_shared = lds_base + static_cast<size_t>(waves / 2) *
-                                             std::max(a.k[0].groups_max, a.k[1].groups_max) * 256;
+    shared_room = tail_groups(lds_limit - lds_base);
     auto shared_estimate = [&](int64_t n, int *best_parts) {
       double best_us = 1e30;
       *best_parts = 0;
-      if (n > cus || lds_shared > lds_limit) return best_us;
+      if (n > cus || !shared_room) return best_us;
       for (int parts = 2; parts <= 64 && n * parts <= 2 * cus; parts++) {
         // beyond one workgroup per compute unit the rest of the grid starts as
         // the first tokens finish: two rounds, measured 7% above twice one
@@ -3513,11 +3700,12 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
       a.k[i].parts = shared_parts;
       a.k[i].split = 1;
     }
-    a.tail_room = (waves / 2) * std::max(a.k[0].groups_max, a.k[1].groups_max);
+    a.tail_room = shared_room;
     a.wi_expect = a.k[0].parts + sub1::expect_extra();
     a.by_ticket = static_cast<int64_t>(tokens) * shared_parts > cus;
     const size_t lds_shared = lds_base + static_cast<size_t>(a.tail_room) * 256;
-    const void *fn = reinterpret_cast<const void *>(moe_prepared_shared_kernel);
+    void (*const shared)(PreparedArgs) = uneven ? moe_prepared_shared_kernel<true> : moe_prepared_shared_kernel<false>;
+    const void *fn = reinterpret_cast<const void *>(shared);
     HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 static_cast<int>(lds_shared)));
     // A token or two: h goes from wi to wo by tag (every workgroup of wo reads
@@ -3541,10 +3729,11 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
                           static_cast<int64_t>(tokens) * (shared_parts + wo_parts * lane_parts) <= cus;
       if (own_wo || static_cast<int64_t>(tokens) * shared_parts <= 64) {
         a.tagged = reinterpret_cast<unsigned long long *>(a.ctrl + sub1::kCtrlTagged);
-        const void *tagged_fn =
-            own_wo ? reinterpret_cast<const void *>(moe_prepared_tagged_split_kernel)
-                   : reinterpret_cast<const void *>(moe_prepared_tagged_kernel);
-        HIP_TRY(hipFuncSetAttribute(tagged_fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+        void (*const tagged)(PreparedArgs) =
+            own_wo ? uneven ? moe_prepared_tagged_split_kernel<true> : moe_prepared_tagged_split_kernel<false>
+            : uneven ? moe_prepared_tagged_kernel<true>
+                     : moe_prepared_tagged_kernel<false>;
+        HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(tagged), hipFuncAttributeMaxDynamicSharedMemorySize,
                                     static_cast<int>(lds_shared)));
         if (own_wo) {
           a.k[1].parts = wo_parts;
@@ -3559,18 +3748,17 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
           a.k[0].parts = shared_parts;
           a.wi_expect = a.k[0].parts + sub1::expect_extra();
           sub1::note_kernel("moe_prepared_tagged_split_kernel");
-          moe_prepared_tagged_split_kernel<<<tokens * (shared_parts + wo_parts * lane_parts), 64 * waves,
-                                             lds_shared, s>>>(a);
+          tagged<<<tokens * (shared_parts + wo_parts * lane_parts), 64 * waves, lds_shared, s>>>(a);
         } else {
           sub1::note_kernel("moe_prepared_tagged_kernel");
-          moe_prepared_tagged_kernel<<<tokens * shared_parts, 64 * waves, lds_shared, s>>>(a);
+          tagged<<<tokens * shared_parts, 64 * waves, lds_shared, s>>>(a);
         }
         HIP_TRY(hipGetLastError());
         return SUB1_OK;
       }
     }
     sub1::note_kernel("moe_prepared_shared_kernel");
-    moe_prepared_shared_kernel<<<tokens * shared_parts, 64 * waves, lds_shared, s>>>(a);
+    shared<<<tokens * shared_parts, 64 * waves, lds_shared, s>>>(a);
     HIP_TRY(hipGetLastError());
     return SUB1_OK;
   }
@@ -3595,7 +3783,9 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
     // workgroups of 16 but two, each twice as long, of workgroups of 8): one's
     // barriers between the phases of a token fall into the other's work
     // (measured 3% faster than one of 16 on 2048 tokens).
-    const int per_cu = fused_per_cu;
+    // (Where lengths differ, one if two leave no room for the partial sums of a long slice.)
+    const bool by_length = uneven && !grouped && tail_groups(lds_limit - lds_fused) > 0;
+    const int per_cu = by_length && tail_groups(lds_limit / fused_per_cu - lds_fused) == 0 ? 1 : fused_per_cu;
     const int fw = waves / per_cu;   // wavefronts per workgroup
     const int rest = ko.slices % fw;
     if (rest > 0 && rest * 2 <= fw && ko.groups_max > 1) {
@@ -3608,6 +3798,18 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
     // a stream larger than the last-level cache (256 MB), swept by at least a
     // token per compute unit: the chunks are loaded as read-once data
     const bool once = !grouped && p.total_chunks * 512 > (256ll << 20);
+    // where lengths differ the longest slices are shared by length, with partial sums behind h
+    if (by_length) {
+      a.tail_room = tail_groups(lds_limit / per_cu - lds_fused);
+      const size_t lds_uneven = lds_fused + static_cast<size_t>(a.tail_room) * 256;
+      HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(moe_prepared_fused_kernel<false, false, true>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_uneven)));
+      sub1::note_kernel("moe_prepared_fused_kernel<false, false, true>");
+      moe_prepared_fused_kernel<false, false, true>
+          <<<tokens < cus * per_cu ? tokens : cus * per_cu, 64 * fw, lds_uneven, s>>>(a);
+      HIP_TRY(hipGetLastError());
+      return SUB1_OK;
+    }
     const void *fn = grouped ? reinterpret_cast<const void *>(moe_prepared_fused_kernel<true, false>)
                      : once  ? reinterpret_cast<const void *>(moe_prepared_fused_kernel<false, true>)
                              : reinterpret_cast<const void *>(moe_prepared_fused_kernel<false, false>);
@@ -3640,21 +3842,18 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
   size_t lds_tail = 0;
   a.tail_room = 0;
   if (!small) {
-    int groups_max = 0;
-    for (int i = 0; i < p.kinds; i++) groups_max = std::max(groups_max, a.k[i].groups_max);
-    lds_tail = static_cast<size_t>(waves / 2) * groups_max * 256;
-    if (lds_base + lds_tail <= lds_limit)
-      a.tail_room = (waves / 2) * groups_max;
-    else
-      lds_tail = 0;
+    a.tail_room = tail_groups(lds_limit - lds_base);
+    lds_tail = static_cast<size_t>(a.tail_room) * 256;
   }
+  uneven = uneven && a.tail_room;
   const size_t lds = lds_base + lds_partials + lds_tail;
   a.wi_expect = a.k[0].parts + sub1::expect_extra();
   // Batches too small to occupy the GPU with a wavefront per slice go to the
   // latency kernel, everything else to the persistent one; either way at most
   // a workgroup per compute unit (16 wavefronts of 72 to 80 registers each).
   const void *fn = small ? reinterpret_cast<const void *>(moe_prepared_small_kernel)
-                         : reinterpret_cast<const void *>(moe_prepared_kernel);
+                   : uneven ? reinterpret_cast<const void *>(moe_prepared_kernel<true>)
+                            : reinterpret_cast<const void *>(moe_prepared_kernel<false>);
   HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                               static_cast<int>(lds)));
   if (small) {
@@ -3664,7 +3863,10 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
   } else {
     const int64_t grid = tiles < cus ? tiles : cus;
     sub1::note_kernel("moe_prepared_kernel");
-    moe_prepared_kernel<<<static_cast<unsigned>(grid), 64 * waves, lds, s>>>(a);
+    if (uneven)
+      moe_prepared_kernel<true><<<static_cast<unsigned>(grid), 64 * waves, lds, s>>>(a);
+    else
+      moe_prepared_kernel<false><<<static_cast<unsigned>(grid), 64 * waves, lds, s>>>(a);
   }
   HIP_TRY(hipGetLastError());
   return SUB1_OK;
@@ -3723,8 +3925,7 @@ constexpr size_t kBatchLds = 160 * 1024 - 64;
 // 9000 columns, stays there too.
 bool plan_batch(const Prepared &p, int kind, size_t lds_limit, BatchPlan *out) {
   const int slices[2] = {(p.height[0] + 63) / 64, (p.height[1] + 63) / 64};
-  const double weight = static_cast<double>(slices[0]) * p.width[0] + static_cast<double>(slices[1]) * p.width[1];
-  const double chunks = static_cast<double>(p.total_chunks) / p.count * p.width[kind] / weight;
+  const double chunks = average_chunks(p, kind);
   const size_t code_bytes = slice_code_bytes(product_steps(p, kind));
   // (wi needs no table)
   const size_t wanted = kind ? table_bytes(p.width[kind]) : 0;

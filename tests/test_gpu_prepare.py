@@ -510,3 +510,39 @@ def test_the_first_pack_of_a_process_may_be_captured():
     (2000, 3100, [0.0, 0.5, 0.99]), (700, 6000, [0.0, 0.9]), (8200, 40, [0.1, 0.5])])   # fewer parts; a turn of a part and more
 def test_rows_that_are_ordered_in_parts_come_back_whole(gpu, height, width, shares):
     test_prepared_rows_come_back_whole(gpu, height, width, shares)
+
+
+@pytest.mark.parametrize('d_model,d_ff,long_rows', [
+    (300, 4467, 5),          # wo: one slice of 62 groups of entries and four of a few
+    (2080, 1100, 70),        # wi: one and a bit of 29 groups, wo of 33 slices
+    (900, 900, 1), (130, 12000, 64)])   # a single long row; partial sums for which LDS has no room
+def test_a_few_tokens_share_long_rows(oracle, d_model, d_ff, long_rows):
+    """The longest slices of a matrix are shared by wavefronts according to their lengths, to the bit."""
+    import numpy as np
+    from oracle import sub1_oracle as so
+    from qmoe_amd import sub1, sub1_hip
+    rng = np.random.default_rng(d_model)
+
+    def layer(height, width):
+        share = rng.uniform(0.0, 0.3, (height, 1))
+        share[rng.permutation(height)[:min(long_rows, height // 4)]] = 1.0
+        t = ((rng.random((height, width)) < share) * rng.integers(1, 3, (height, width))).astype(np.int32)
+        minmax = np.abs(rng.standard_normal((height, 2))) * (-1.0, 1.0)
+        return oracle.encode(t) + (so.f32_to_bf16_bits(minmax.ravel().astype(np.float32)),)
+
+    def dev(l):
+        return torch.from_numpy(l[0].view(np.int16)).cuda(), torch.from_numpy(l[1]).cuda(), \
+            torch.from_numpy(l[2].view(np.int16)).cuda().view(torch.bfloat16)
+
+    wi, wo = [layer(d_ff, d_model) for _ in range(2)], [layer(d_model, d_ff) for _ in range(2)]
+    stack = sub1_hip.PreparedStack.from_layers(sub1.DEC[0], [dev(l) for l in wi], [dev(l) for l in wo])
+    xs = np.stack([so.synthetic_activation(d_model, 30 + i) for i in range(4)])
+    want = [oracle.expert_ffn(wi[i % 2], wo[i % 2], xs[i], order=2)[0] for i in range(4)]
+    x = torch.from_numpy(xs.view(np.int16)).cuda().view(torch.bfloat16)
+    for tokens in (1, 2, 3, 9, 33, 64, 128, 255, 600):
+        ids = torch.arange(tokens) % 4
+        for _ in range(2):                  # the control words are left as they were found
+            y = stack.forward(x[ids.cuda()].contiguous(), (ids % 2).to(torch.int32).cuda(), None, False)
+            got = y.view(torch.int16).cpu().numpy().view(np.uint16)
+            assert stack.launch_faults(tokens) == (0, 0)
+            assert (got == np.stack(want)[ids]).all(), tokens
