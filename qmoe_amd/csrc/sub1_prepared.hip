@@ -2731,8 +2731,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_tagged_kernel(Prepar
 // 62 KB of code, each instruction of it run about once: where it lies makes 0.15 us
 // (the same instructions behind kernels of another size 11.83 and 11.97), so it has a place of its own.
 template <bool kUneven>
-__global__ __launch_bounds__(kMaxThreads) __attribute__((aligned(65536)))
-void moe_prepared_tagged_split_kernel(PreparedArgs a) {
+__device__ __forceinline__ void tagged_split(const PreparedArgs &a) {
   extern __shared__ __align__(16) uint32_t lds[];
   uint32_t *xa = lds;
   float *partials = reinterpret_cast<float *>(xa + a.xdwords);
@@ -2794,6 +2793,9 @@ void moe_prepared_tagged_split_kernel(PreparedArgs a) {
   }
   if (threadIdx.x == 0) leave_tagged(a.ctrl, gridDim.x);
 }
+__global__ __launch_bounds__(kMaxThreads) __attribute__((aligned(65536)))
+void moe_prepared_tagged_split_kernel(PreparedArgs a) { tagged_split<false>(a); }
+__global__ __launch_bounds__(kMaxThreads) void moe_prepared_uneven_split_kernel(PreparedArgs a) { tagged_split<true>(a); }
 
 // For the batches too small to occupy the GPU with a wavefront per slice: built
 // for latency.  `split` wavefronts share a slice (split_begin / split_run) and
@@ -3730,7 +3732,7 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
       if (own_wo || static_cast<int64_t>(tokens) * shared_parts <= 64) {
         a.tagged = reinterpret_cast<unsigned long long *>(a.ctrl + sub1::kCtrlTagged);
         void (*const tagged)(PreparedArgs) =
-            own_wo ? uneven ? moe_prepared_tagged_split_kernel<true> : moe_prepared_tagged_split_kernel<false>
+            own_wo ? uneven ? moe_prepared_uneven_split_kernel : moe_prepared_tagged_split_kernel
             : uneven ? moe_prepared_tagged_kernel<true>
                      : moe_prepared_tagged_kernel<false>;
         HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(tagged), hipFuncAttributeMaxDynamicSharedMemorySize,
