@@ -389,8 +389,8 @@ __device__ __forceinline__ float neighbour(float v) {
 template <bool kPairs, int kRG, int kKP, int kNB>
 __device__ __forceinline__ void finish_tiles(const TileArgs &a, const TileLane &l, int g, int k, bool rows, int live,
                                              unsigned char *lds, const f32x16 (&acc)[kNB][2]) {
-  constexpr int kTiles = 2 * kNB, kFinish = kTiles / kKP;
-  static_assert(kFinish * kKP == kTiles, "equal shares");
+  constexpr int kTiles = 2 * kNB, kFinish = (kTiles + kKP - 1) / kKP;
+  static_assert(kTiles % kFinish == 0, "equal shares (where there are fewer tiles than parts the last ones have none)");
   float4 *sums = reinterpret_cast<float4 *>(lds);
   // of tile `n` of what part `of` finishes, from part `from`
   auto place = [&](int of, int from, int n) {
@@ -828,9 +828,10 @@ struct Pieces {
 // that frees its tile.
 template <bool kDirect, int kRG, int kKP, int kNB>
 __global__ __launch_bounds__(64 * kRG * kKP)
-__attribute__((amdgpu_waves_per_eu(kRG * kKP == 8 || kNB == 2 || kRG == 4 ? 2 : 1, 4)))
+__attribute__((amdgpu_waves_per_eu(kRG * kKP == 8 || kNB <= 2 || kRG == 4 ? 2 : 1, 4)))
 void matvec_tiles_shared_kernel(TileArgs a) {
-  static_assert((kRG * kKP == 4 || kRG * kKP == 8) && (kNB == 2 || kNB == 4), "four or eight wavefronts");
+  static_assert(kNB == 1 ? kRG == 1 : (kRG * kKP == 4 || kRG * kKP == 8) && (kNB == 2 || kNB == 4),
+                "four or eight wavefronts; blocks of 32 tokens: a wavefront a part");
   constexpr int kTile = kNB * 32 * 256;        // a window of activations
   constexpr int kLoads = 8 * kNB / kRG;        // of them this wavefront's loads
   static_assert(kLoads >= 2, "a load is four tokens");
@@ -999,12 +1000,12 @@ void matvec_tiles_shared_kernel(TileArgs a) {
       if (turn + 1 < turns) turn_of(turn + 1, 1, codes_b, codes_a);
     }
   };
-  if (live == kNB)
+  if (kNB == 1 || live == kNB)
     run(std::integral_constant<int, kNB>{});
   else if (kNB == 4 && live == 3)
     run(std::integral_constant<int, kNB == 4 ? 3 : kNB>{});
   else
-    run(std::integral_constant<int, kNB / 2>{});
+    run(std::integral_constant<int, (kNB + 1) / 2>{});
   // nothing is on its way into LDS any more
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   finish_tiles<kDirect, kRG, kKP, kNB>(a, l, g, k, has_rows, live, shared_tiles, acc);
@@ -1068,11 +1069,23 @@ double cost_of(const TileForm &f, int row_blocks, int windows, int tokens) {
   const int64_t rounds = workgroups / (256 * f.held), rest = workgroups % (256 * f.held);
   return rounds * with(f.held) + (rest ? with((rest + 255) / 256) : 0.0);
 }
-// `direct`: x and y as the forms on the activations' straight way into LDS need them.  Blocks of
+// `direct`: x and y as the forms on the activations' straight way into LDS need them (`wide`: x).  Blocks of
 // 128 tokens have to promise a fifth where there are two parts, and are taken where there is
 // one if blocks of 64 would make more workgroups than the chip holds at once: the fit is coarse
 // there (c-2048 wi on 1136 tokens 33.0 us, in blocks of 64 38.0; large wi 16.8 and 17.8).
-const TileForm &pick_form(int parts, int row_blocks, int windows, int tokens, bool direct) {
+//
+// Activations that come through registers, in two or four parts: a workgroup of 64 rows and 32 tokens
+// with a wavefront a part, where there are at most two of them for each compute unit (one, where rows of x
+// are aligned after all: 1999 x 4000 on 250 tokens 23.5 / 20.4, on 400, 416 workgroups, 24.4 / 26.4).  The forms above
+// are then few workgroups, whose loads and decoding nothing hides (us, blocks of 64 tokens / so:
+// 1293 x 5497 on 64, 336, 568 tokens 28.4 / 19.1, 33.2 / 23.4, 31.6 / 28.4, on 900, 609 workgroups, 35.4 / 47.1;
+// 1675 x 4874 on 336 25.2 / 20.6, on 900, 783, 27.5 / 37.6; in two parts 5003 x 1501 on 128, 316
+// workgroups, 13.2 / 12.1, on 200, 553, 14.3 / 14.7, 2081 x 6143 on 400, 429, 48.2 / 41.0).  Where they go straight into LDS it gained 7 % on
+// two shapes of thirteen and lost elsewhere.
+constexpr TileForm kNarrowForms[] = {{2, 1, 1, 2, 0.0, 0.0, 0.0}, {4, 1, 1, 2, 0.0, 0.0, 0.0}};
+const TileForm &pick_form(int parts, int row_blocks, int windows, int tokens, bool direct, bool wide) {
+  if (!direct && parts > 1 && static_cast<int64_t>(row_blocks) * ((tokens + 31) / 32) <= (wide ? 1 : 2) * 256)
+    return kNarrowForms[parts == 2 ? 0 : 1];
   const TileForm *best = nullptr;
   double best_cost = 0;
   const bool wide_of_one = (row_blocks + 3) / 4 * static_cast<int64_t>((tokens + 63) / 64) > 3 * 256;
@@ -1114,7 +1127,7 @@ template <bool kDirect, int kRG, int kKP, int kNB>
 int launch_shared_as(TileArgs a, int blocks, hipStream_t stream) {
   constexpr int waves = kRG * kKP;
   constexpr int lds = kKP * 2 * kNB * 32 * 256;
-  static_assert(lds >= waves * (kKP - 1) * (2 * kNB / kKP) * 4096 && lds <= 160 * 1024, "tiles, then sums");
+  static_assert(lds >= waves * (kKP - 1) * ((2 * kNB + kKP - 1) / kKP) * 4096 && lds <= 160 * 1024, "tiles, then sums");
   HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(matvec_tiles_shared_kernel<kDirect, kRG, kKP, kNB>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, lds));
   const int row_groups = (blocks + kRG - 1) / kRG, token_blocks = (a.tokens + 31) / 32;
@@ -1137,12 +1150,14 @@ int launch_own(const TileArgs &a, int blocks, hipStream_t stream) {
 int launch_form(const TileArgs &a, const TileForm &f, bool direct, int blocks, hipStream_t s) {
   sub1::note_kernel(f.groups == 0   ? "matvec_tiles_kernel"
                     : f.blocks == 4 ? "matvec_tiles_shared_kernel<128>"
+                    : f.blocks == 1 ? "matvec_tiles_shared_kernel<32>"
                                     : "matvec_tiles_shared_kernel<64>");
   if (f.groups == 0) {
     if (f.parts == 1) return launch_own<1>(a, blocks, s);
     if (f.parts == 2) return launch_own<2>(a, blocks, s);
     return launch_own<4>(a, blocks, s);
   }
+  if (f.blocks == 1) return f.parts == 2 ? launch_shared_as<false, 1, 2, 1>(a, blocks, s) : launch_shared_as<false, 1, 4, 1>(a, blocks, s);
   if (f.parts == 1) {
     if (!direct) return launch_shared_as<false, 4, 1, 2>(a, blocks, s);
     return f.blocks == 4 ? launch_shared_as<true, 4, 1, 4>(a, blocks, s) : launch_shared_as<true, 4, 1, 2>(a, blocks, s);
@@ -1298,7 +1313,7 @@ int launch_product(const sub1_tiles *t, int matrix, const void *x, int64_t ldx, 
   // a wavefront with tiles of its own, 31, 72 and 263).
   const bool direct = wide && !misaligned(y, 4) && ldy % 2 == 0 && t->height % 2 == 0;
   const int blocks = l.units_down / 2, parts = parts_of(blocks, l.windows);
-  const TileForm *form = &pick_form(parts, blocks, l.windows, tokens, direct);
+  const TileForm *form = &pick_form(parts, blocks, l.windows, tokens, direct, wide);
   const int forced = g_forced_kernel.load(std::memory_order_relaxed);
   // (a block's rows of x and y are addressed in 32 bits: 128 of them up to these strides)
   const bool far = ldx >= (1 << 22) || ldy >= (1 << 22);

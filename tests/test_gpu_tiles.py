@@ -376,3 +376,31 @@ def test_a_product_into_a_new_tensor_is_the_sum_onto_zeros(gpu, oracle, height, 
             finally:
                 _lib.check(_lib.load().sub1_test_tiles_kernel(0))
             assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (make.__name__, which)
+
+
+@pytest.mark.parametrize('height,width,tokens,narrow', [
+    (700, 4637, 64, True), (700, 4637, 1472, True), (700, 4637, 1473, False),   # 11 blocks of rows: 46 of 32 tokens make 506
+    (1, 2305, 65, True), (65, 2305, 97, True),      # four parts of five windows, the last of one column
+    (5003, 1501, 65, True), (3001, 1023, 129, True)])   # two parts
+def test_few_tokens_through_registers(gpu, oracle, height, width, tokens, narrow):
+    """Blocks of 32 tokens where rows have any alignment and workgroups are few: against the
+    double-precision product, and to the bit what a launch of more tokens gives for the same ones."""
+    sub1, op = gpu
+    from qmoe_amd import _lib
+    c = dev_case(oracle, height, width, 0.9, seed=height + width + tokens)
+    tm = op.TiledMatrix(sub1.DEC[0], c['w_comp'], c['row_off_d'], c['mm_d'], width)
+    rng = np.random.default_rng(tokens + height)
+    longer = 4096                                     # more workgroups than that form takes
+    xs = so.f32_to_bf16_bits(rng.standard_normal((tokens, width)).astype(np.float32))
+    pre = so.f32_to_bf16_bits(rng.standard_normal((tokens, height)).astype(np.float32))
+    x, y = bf16_dev(xs), bf16_dev(pre).clone()
+    tm.matvec_tokens(x, y)
+    assert (_lib.load().sub1_last_kernel() == b'matvec_tiles_shared_kernel<32>') == narrow
+    got = bits_host(y)
+    check_tokens(oracle, c, xs, pre, got, sorted({0, 31, 32, 63, tokens - 1}))
+    if height > 100:
+        repeat = (longer + tokens - 1) // tokens * 4
+        y = bf16_dev(pre).repeat(repeat, 1)
+        tm.matvec_tokens(x.repeat(repeat, 1), y)
+        assert _lib.load().sub1_last_kernel() != b'matvec_tiles_shared_kernel<32>'
+        assert np.array_equal(bits_host(y[-tokens:].contiguous()), got)
