@@ -19,14 +19,13 @@
 // it, 13 us of 133 below; y through another, 6, where its two-byte stores now go straight to
 // the tokens' rows.)
 //
-// One launch: group_blocks_kernel gives every token a slot in a block of 32 of its
-// expert's tokens; pack_tokens_kernel lays a block's activations out as MFMA
-// operands; batch_product_kernel<true> multiplies (wi, ReLU), batch_product_kernel<false>
+// One launch: pack_blocks_kernel gives every token a slot in a block of 32 of its
+// expert's tokens and lays a block's activations out as MFMA operands; batch_product_kernel<true> multiplies (wi, ReLU), batch_product_kernel<false>
 // (wo); walk_spoiled_kernel walks what they leave.
 //
-// 128 base experts on 4096 tokens: walking 274 us, here 115 (133 with a pass for h and one for y);
+// 128 base experts on 4096 tokens: walking 274 us, here 110 (133 with a pass for h and one for y);
 // 40 c-2048 experts on 640 tokens 311 and 159 (167).  Under a profiler, one after the other:
-// group 8, x 6, wi 48, wo 61, marks 4.5.  Of the products' times multiplying is 27 each (with it taken
+// slots and x 9, wi 48, wo 60, marks 4.5.  Of the products' times multiplying is 27 each (with it taken
 // out they take that less): the 24 instructions that make a step's two operands of weights, beside
 // two MFMAs for every block of tokens, issued at 80 % of what the SIMDs can; expanding 8 and 12;
 // starting, clearing LDS and adding up what the wavefronts of a slice have, in workgroups
@@ -46,7 +45,7 @@ constexpr int kChunkBlocks = 2;      // blocks that share an expansion
 constexpr int kTurn = 4;             // steps whose operands are asked for together, and ahead
 constexpr int kStepColumns = 16;     // columns of an MFMA, and of a word of codes
 constexpr int kBatchPiece = 8192;    // tokens of a launch sequence: bounds the scratch memory
-constexpr int kBatchMaxExperts = 4096;   // group_blocks_kernel's tables in LDS
+constexpr int kBatchMaxExperts = 4096;   // pack_blocks_kernel's counts in LDS
 
 __host__ __device__ constexpr int steps_of(int width) { return (width + kStepColumns - 1) / kStepColumns; }
 // Steps of a product over the rows of 64-row slices.
@@ -449,88 +448,6 @@ __global__ __launch_bounds__(kMaxThreads) void fill_tables_kernel(BatchArgs a, u
              order_piece(a, blockIdx.x, threadIdx.x), threadIdx.x, blockDim.x);
 }
 
-// One workgroup.  Every token gets a slot: its expert's tokens fill blocks of 32, an
-// expert's blocks lie together, those of tokens without an expert come last.
-__global__ __launch_bounds__(1024) void group_blocks_kernel(
-    const int32_t *__restrict__ token_expert, int tokens, int experts, int32_t *__restrict__ slots,
-    int32_t *__restrict__ spoiled, int32_t *__restrict__ block_expert, int4 *__restrict__ chunks,
-    int32_t *__restrict__ totals, int32_t *__restrict__ ctrl) {
-  extern __shared__ __align__(16) int32_t table[];
-  __shared__ int32_t wave_blocks[16], wave_chunks[16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int buckets = experts + 1;
-  int32_t *count = table, *next = table + buckets;
-  for (int b = tid; b < buckets; b += 1024) count[b] = 0;
-  __syncthreads();
-  int faults = 0;
-  int bucket[kBatchPiece / 1024], rank[kBatchPiece / 1024];   // which expert's, and which of its tokens
-#pragma unroll
-  for (int i = 0; i < kBatchPiece / 1024; i++) {
-    const int t = i * 1024 + tid;
-    const int e = t < tokens ? token_expert[t] : -1;
-    if (e >= experts) faults++;
-    bucket[i] = e < 0 || e >= experts ? experts : e;
-  }
-#pragma unroll
-  for (int i = 0; i < kBatchPiece / 1024; i++)
-    if (i * 1024 + tid < tokens) rank[i] = atomicAdd(&count[bucket[i]], 1);
-  if (faults) atomicAdd(&ctrl[kCtrlBadIds], faults);
-  __syncthreads();
-  const int seg = (buckets + 1023) / 1024;
-  const int lo = min(tid * seg, buckets), hi = min(lo + seg, buckets);
-  auto blocks_of = [](int n) { return (n + kBlockTokens - 1) / kBlockTokens; };
-  auto chunks_in = [](int n) { return (n + kChunkBlocks - 1) / kChunkBlocks; };
-  int32_t n_blocks = 0, n_chunks = 0;
-  for (int b = lo; b < hi; b++) {
-    const int n = blocks_of(count[b]);
-    n_blocks += n;
-    if (b != experts) n_chunks += chunks_in(n);
-  }
-  int32_t up_blocks = n_blocks, up_chunks = n_chunks;
-  for (int d = 1; d < 64; d <<= 1) {
-    const int32_t u = __shfl_up(up_blocks, d, 64), v = __shfl_up(up_chunks, d, 64);
-    if (lane >= d) {
-      up_blocks += u;
-      up_chunks += v;
-    }
-  }
-  if (lane == 63) {
-    wave_blocks[wave] = up_blocks;
-    wave_chunks[wave] = up_chunks;
-  }
-  __syncthreads();
-  int32_t block = up_blocks - n_blocks, chunk = up_chunks - n_chunks;
-  for (int w = 0; w < wave; w++) {
-    block += wave_blocks[w];
-    chunk += wave_chunks[w];
-  }
-  for (int b = lo; b < hi; b++) {
-    const int n = count[b], nb = blocks_of(n);
-    next[b] = block * kBlockTokens;
-    for (int i = n; i < nb * kBlockTokens; i++) slots[block * kBlockTokens + i] = -1;
-    for (int i = 0; i < nb; i++) block_expert[block + i] = b == experts ? -1 : b;
-    if (b == experts) {
-      totals[kTotalChunks] = chunk;
-      totals[kTotalLive] = block;
-      totals[kTotalBlocks] = block + nb;
-    } else {
-      for (int i = 0; i < nb; i += kChunkBlocks)
-        chunks[chunk++] = make_int4(b, block + i, min(kChunkBlocks, nb - i), 0);
-    }
-    block += nb;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < kBatchPiece / 1024; i++) {
-    const int t = i * 1024 + tid;
-    if (t < tokens) {
-      const int place = next[bucket[i]] + rank[i];
-      slots[place] = t;
-      spoiled[place] = 0;
-    }
-  }
-}
-
 __device__ __forceinline__ bool not_finite(uint32_t bits) { return (bits & 0x7f80u) == 0x7f80u; }
 
 // A step's 16 columns of a token (bits, zeros past the width) as its two operands.
@@ -545,42 +462,153 @@ __device__ __forceinline__ void write_operands(u32x4 *out, int64_t step, int t, 
   }
 }
 
-// x by blocks of 32 slots into operands; tokens without an expert keep their input.
-__global__ __launch_bounds__(256) void pack_tokens_kernel(
-    const uint16_t *x, uint16_t *y, int64_t ldx, int64_t ldy, int width, bool aligned,
-    const int32_t *__restrict__ slots, int32_t *__restrict__ spoiled, const int32_t *__restrict__ totals,
-    u32x4 *__restrict__ out) {
-  const int block = blockIdx.x;
-  if (block >= totals[kTotalBlocks]) return;
-  const int steps = steps_of(width);
-  const int t = threadIdx.x & 31;
-  const int token = slots[block * kBlockTokens + t];
-  const bool live = block < totals[kTotalLive];
-  const uint16_t *from = x + token * ldx;
-  if (token < 0) return;   // what the operands hold of it goes nowhere
-  bool bad = false;
-  for (int st = blockIdx.y * 8 + (threadIdx.x >> 5); st < steps; st += gridDim.y * 8) {
-    const int c = st * kStepColumns;
-    uint16_t v[16];
-    if (aligned && c + 16 <= width) {
-      const uint4 a = *reinterpret_cast<const uint4 *>(from + c);
-      const uint4 b = *reinterpret_cast<const uint4 *>(from + c + 8);
-      __builtin_memcpy(v, &a, 16);
-      __builtin_memcpy(v + 8, &b, 16);
-    } else {
+// Prefix sum over a workgroup of 1024: what the threads below have, and the total.
+__device__ __forceinline__ int below_in_workgroup(int v, int32_t *wave_sums, int *total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int upto = sub1::wave_prefix_sum(v);
+  if (lane == 63) wave_sums[wave] = upto;
+  __syncthreads();
+  int below = upto - v, all = 0;
 #pragma unroll
-      for (int i = 0; i < 16; i++) v[i] = c + i < width ? from[c + i] : 0;
-    }
-    if (live) {
-#pragma unroll
-      for (int i = 0; i < 16; i++) bad |= not_finite(v[i]);
-      write_operands(out + static_cast<int64_t>(block) * steps * 64, st, t, v);
-    } else {
-      for (int i = 0; i < 16; i++)
-        if (c + i < width) y[token * ldy + c + i] = v[i];
-    }
+  for (int w = 0; w < 16; w++) {
+    if (w < wave) below += wave_sums[w];
+    all += wave_sums[w];
   }
-  if (bad) spoiled[block * kBlockTokens + t] = 1;
+  *total = all;
+  return below;
+}
+
+// Every token gets a slot: its expert's tokens, in order, fill blocks of 32, an expert's blocks lie
+// together, those of tokens without an expert come last.  A workgroup finds out for itself which tokens
+// make its block - counts per expert, whose blocks these are, and which of that expert's tokens come
+// before - and lays their activations out as operands; tokens without an expert keep their input.
+// Bound by the chain of those stations.  (In a launch of one workgroup that grouped and one that laid
+// out: 8.1 and 5.7 us for 4096 tokens of 128 base experts, here 8.6; the call 114 and 110.
+// 30 experts of 901 x 2503 on 700 tokens 46.7 and 45.8, 51.1 with a block to a single workgroup.)
+__global__ __launch_bounds__(kMaxThreads) void pack_blocks_kernel(
+    const int32_t *__restrict__ token_expert, const uint16_t *x, uint16_t *y, int64_t ldx, int64_t ldy, int width,
+    bool aligned, int tokens, int experts, int32_t *__restrict__ slots, int32_t *__restrict__ spoiled,
+    int32_t *__restrict__ block_expert, int4 *__restrict__ chunks, int32_t *__restrict__ totals,
+    int32_t *__restrict__ ctrl, u32x4 *__restrict__ out) {
+  extern __shared__ __align__(16) int32_t count[];   // tokens of every expert, then of none
+  __shared__ int32_t sums[3][16];
+  __shared__ int s_bucket, s_nth, s_blocks, s_chunk;
+  __shared__ int32_t s_token[kBlockTokens], s_bad[kBlockTokens];
+  const int tid = threadIdx.x, block = blockIdx.x;
+  const int buckets = experts + 1;
+  // a thread's tokens are neighbours
+  constexpr int kMine = kBatchPiece / kMaxThreads;
+  const int each = (tokens + kMaxThreads - 1) / kMaxThreads;
+  int bucket[kMine], faults = 0;
+#pragma unroll
+  for (int i = 0; i < kMine; i++) {
+    const int t = tid * each + i;
+    const bool mine = i < each && t < tokens;
+    const int e = mine ? token_expert[t] : -1;
+    if (e >= experts) faults++;
+    bucket[i] = !mine ? -1 : e < 0 || e >= experts ? experts : e;
+  }
+  for (int b = tid; b < buckets; b += kMaxThreads) count[b] = 0;
+  if (tid < kBlockTokens) {
+    s_token[tid] = -1;
+    s_bad[tid] = 0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kMine; i++)
+    if (bucket[i] >= 0) atomicAdd(&count[bucket[i]], 1);
+  if (block == 0 && blockIdx.y == 0 && faults) atomicAdd(&ctrl[kCtrlBadIds], faults);
+  __syncthreads();
+  // whose block this is
+  const int seg = (buckets + kMaxThreads - 1) / kMaxThreads;
+  const int lo = min(tid * seg, buckets), hi = min(lo + seg, buckets);
+  auto blocks_of = [](int n) { return (n + kBlockTokens - 1) / kBlockTokens; };
+  auto chunks_in = [](int n) { return (n + kChunkBlocks - 1) / kChunkBlocks; };
+  int n_blocks = 0, n_chunks = 0;
+  for (int b = lo; b < hi; b++) {
+    const int n = blocks_of(count[b]);
+    n_blocks += n;
+    if (b != experts) n_chunks += chunks_in(n);
+  }
+  int all_blocks, all_chunks;
+  int at = below_in_workgroup(n_blocks, sums[0], &all_blocks);
+  int chunk = below_in_workgroup(n_chunks, sums[1], &all_chunks);
+  const int live_blocks = all_blocks - blocks_of(count[experts]);
+  if (block == 0 && blockIdx.y == 0 && tid == 0) {
+    totals[kTotalChunks] = all_chunks;
+    totals[kTotalLive] = live_blocks;
+    totals[kTotalBlocks] = all_blocks;
+  }
+  if (block >= all_blocks) return;
+  for (int b = lo; b < hi; b++) {
+    const int n = blocks_of(count[b]);
+    if (block >= at && block < at + n) {
+      s_bucket = b;
+      s_nth = block - at;
+      s_blocks = n;
+      s_chunk = chunk;
+    }
+    at += n;
+    chunk += chunks_in(n);
+  }
+  __syncthreads();
+  const int mine = s_bucket, nth = s_nth;
+  const bool live = mine != experts;
+  // which of its tokens: 32 of them from number 32 nth on
+  int found = 0;
+#pragma unroll
+  for (int i = 0; i < kMine; i++) found += bucket[i] == mine;
+  int all_found;
+  int number = below_in_workgroup(found, sums[2], &all_found) - kBlockTokens * nth;
+#pragma unroll
+  for (int i = 0; i < kMine; i++)
+    if (bucket[i] == mine) {
+      if (number >= 0 && number < kBlockTokens) s_token[number] = tid * each + i;
+      number++;
+    }
+  __syncthreads();
+  if (blockIdx.y == 0 && tid == 0) {
+    block_expert[block] = live ? mine : -1;
+    if (live && nth % kChunkBlocks == 0)
+      chunks[s_chunk + nth / kChunkBlocks] = make_int4(mine, block, min(kChunkBlocks, s_blocks - nth), 0);
+  }
+  const int steps = steps_of(width);
+  // the tokens of a block are shared by the workgroups of a column
+  const int tokens_here = kBlockTokens / gridDim.y, first_here = blockIdx.y * tokens_here;
+  const int t = first_here + tid % tokens_here;
+  const int token = s_token[t];
+  if (token >= 0) {   // (what the operands hold of an empty slot goes nowhere)
+    const uint16_t *from = x + token * ldx;
+    bool bad = false;
+    for (int st = tid / tokens_here; st < steps; st += kMaxThreads / tokens_here) {
+      const int c = st * kStepColumns;
+      uint16_t v[16];
+      if (aligned && c + 16 <= width) {
+        const uint4 a = *reinterpret_cast<const uint4 *>(from + c);
+        const uint4 b = *reinterpret_cast<const uint4 *>(from + c + 8);
+        __builtin_memcpy(v, &a, 16);
+        __builtin_memcpy(v + 8, &b, 16);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; i++) v[i] = c + i < width ? from[c + i] : 0;
+      }
+      if (live) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) bad |= not_finite(v[i]);
+        write_operands(out + static_cast<int64_t>(block) * steps * 64, st, t, v);
+      } else {
+        for (int i = 0; i < 16; i++)
+          if (c + i < width) y[token * ldy + c + i] = v[i];
+      }
+    }
+    if (bad) s_bad[t] = 1;
+  }
+  __syncthreads();
+  if (tid < tokens_here) {
+    const int slot = block * kBlockTokens + first_here + tid;
+    slots[slot] = s_token[first_here + tid];
+    spoiled[slot] = s_bad[first_here + tid];
+  }
 }
 
 // The tokens in the slots that are marked, a workgroup each, as moe_prepared_fused_kernel

@@ -4076,11 +4076,12 @@ int launch_batch(const Prepared &p, const int32_t *token_expert, const uint16_t 
   const int d_model = p.width[0], d_ff = p.height[0];
   const bool aligned = d_model % 8 == 0 && !misaligned(x, 16);
 
-  group_blocks_kernel<<<1, 1024, static_cast<size_t>(p.count + 1) * 8, s>>>(
-      token_expert, tokens, p.count, slots, spoiled, block_expert, chunks, totals, ctrl);
-  const auto shares = [](int work, int per) { return static_cast<unsigned>(std::max(1, std::min(16, (work + per - 1) / per))); };
-  pack_tokens_kernel<<<dim3(b.max_blocks, shares(steps_of(d_model), 16)), 256, 0, s>>>(
-      x, y, d_model, d_model, d_model, aligned, slots, spoiled, totals, xs);
+  // workgroups that share a block's tokens: as many as leave each thread a step, within two to a unit
+  unsigned shares = 1;
+  while (shares < 4 && steps_of(d_model) > 32 * static_cast<int>(shares) && 2 * shares * b.max_blocks <= 2 * 256) shares *= 2;
+  pack_blocks_kernel<<<dim3(b.max_blocks, shares), kMaxThreads, static_cast<size_t>(p.count + 1) * 4, s>>>(
+      token_expert, x, y, d_model, d_model, d_model, aligned, tokens, p.count, slots, spoiled, block_expert, chunks,
+      totals, ctrl, xs);
   PreparedArgs a = {};
   a.stream = static_cast<const uint2 *>(p.codes);
   a.ckpt = reinterpret_cast<const uint16_t *>(a.stream + p.total_chunks * 64);

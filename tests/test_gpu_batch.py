@@ -369,3 +369,25 @@ def test_bad_arguments_are_refused_on_the_host():
     p.d_ff, p.experts = 128, 4097
     assert lib.sub1_moe_batch_scratch_bytes(ref, 100) == 0
     assert lib.sub1_moe_batch_scratch_bytes(None, 100) == 0 and lib.sub1_moe_batch_pays(None, 100) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('experts,tokens,kept', [
+    (3, 1, 1), (3, 1023, 3), (3, 1024, 1), (3, 1025, 2),     # a token a thread and more; all of one expert
+    (1030, 2049, 1030), (40, 8192, 40), (40, 8193, 1),      # more experts than threads; a piece, and pieces of one expert
+    (2, 100, 0)])                                           # no token with an expert
+def test_every_token_has_a_slot(oracle, experts, tokens, kept):
+    """Tokens in blocks of their expert's, whatever their number: exact sums, so that the walking kernels'
+    bits are the answer; dropped ones keep their input."""
+    made = [(layers(oracle, 20, 24, 0.5, 10 + e), layers(oracle, 24, 20, 0.5, 20 + e)) for e in range(3)]
+    prep = prepared([made[e % 3][0] for e in range(experts)], [made[e % 3][1] for e in range(experts)])
+    rng = np.random.default_rng(tokens)
+    route = rng.integers(0, kept, tokens) if kept else np.full(tokens, -1)
+    drop = rng.random(tokens) < 0.1
+    route[drop] = rng.choice([-1, experts], int(drop.sum()))
+    xs = rng.integers(-2, 3, (tokens, 24)).astype(np.float32)
+    x, te = bf16_dev(so.f32_to_bf16_bits(xs)), torch.from_numpy(route.astype(np.int32)).cuda()
+    for _ in range(2):
+        got = bits_host(prep.forward_batch(x, te))
+        assert prep.launch_faults(tokens) == (0, int((route == experts).sum()))
+    assert np.array_equal(got, bits_host(prep.forward(x, te)))
