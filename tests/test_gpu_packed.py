@@ -26,6 +26,7 @@ def uneven_layer(oracle, height, width, shares, seed):
     (100, 200, [0.0]), (64, 66, [1.0]),      # all alike: one code after another, none without a weight
     (700, 130, [0.1] * 63 + [0.95]),         # one long row among 64
     (900, 2100, [0.05, 0.25, 0.5, 0.9, 0.0]),   # cut into parts, a wavefront's rows into turns
+    (311, 1037, [0.1]),                      # runs of rows that do not divide a tile's
     (12288, 40, [0.02, 0.9, 0.0, 0.3])])     # rows of up to 150 groups
 def test_rows_of_different_lengths_on_the_packed_layout(oracle, d_model, d_ff, shares):
     from qmoe_amd import sub1, sub1_hip
