@@ -546,3 +546,38 @@ def test_a_few_tokens_share_long_rows(oracle, d_model, d_ff, long_rows):
             got = y.view(torch.int16).cpu().numpy().view(np.uint16)
             assert stack.launch_faults(tokens) == (0, 0)
             assert (got == np.stack(want)[ids]).all(), tokens
+
+
+@pytest.mark.parametrize('height,width,long_rows', [(3000, 1100, 40), (1100, 4467, 70), (64 * 33, 700, 3)])
+def test_matrices_of_long_rows(oracle, height, width, long_rows):
+    """Single matrices, a token through its own of them: tiles whose longest slices are shared by length, to the bit."""
+    import numpy as np
+    from oracle import sub1_oracle as so
+    from qmoe_amd import _lib, sub1, sub1_hip
+    rng = np.random.default_rng(height)
+
+    def one():
+        share = rng.uniform(0.0, 0.3, (height, 1))
+        share[rng.permutation(height)[:long_rows]] = 1.0
+        t = ((rng.random((height, width)) < share) * rng.integers(1, 3, (height, width))).astype(np.int32)
+        minmax = np.abs(rng.standard_normal((height, 2))) * (-1.0, 1.0)
+        return oracle.encode(t) + (so.f32_to_bf16_bits(minmax.ravel().astype(np.float32)),)
+
+    def dev(bits):
+        return torch.from_numpy(bits.view(np.int16)).cuda().view(torch.bfloat16)
+
+    made = [one() for _ in range(2)]
+    pm = sub1_hip.PreparedMatrix(sub1.DEC[0], [torch.from_numpy(m[0].view(np.int16)).cuda() for m in made],
+                                 [torch.from_numpy(m[1]).cuda() for m in made], [dev(m[2]) for m in made], width)
+    xs = np.stack([so.synthetic_activation(width, 30 + i) for i in range(4)])
+    zero = np.zeros(height, np.uint16)
+    want = np.stack([oracle.matvec_gap(*made[i % 2], xs[i], y=zero) for i in range(4)])
+    kernels = set()
+    for tokens in (1, 7, 100, 300):
+        ids = np.arange(tokens) % 4
+        y = torch.zeros((tokens, height), dtype=torch.bfloat16, device='cuda')
+        pm.matvec_tokens(dev(xs)[torch.from_numpy(ids).cuda()].contiguous(), y,
+                         torch.from_numpy((ids % 2).astype(np.int32)).cuda())
+        kernels.add(_lib.load().sub1_last_kernel())
+        assert (y.view(torch.int16).cpu().numpy().view(np.uint16) == want[ids]).all(), tokens
+    assert b'moe_prepared_kernel' in kernels
