@@ -202,18 +202,17 @@ def sub1decode(dec, w_comp, row_off, ter_minmax, width, want_tern=True, want_w=T
     for the GPU: the outputs are complete when it returns, on any stream."""
     dev = dec.device if isinstance(dec, torch.Tensor) else None
     height = row_off.numel() - 1
-    p_dec = _need(dec, torch.int32, 'dec', numel=_lib.DEC_WORDS)
-    p_wc = _need(w_comp, torch.int16, 'w_comp', dev)
-    p_ro = _need(row_off, torch.int32, 'row_off', dev)
-    p_mm = _need(ter_minmax, torch.bfloat16, 'ter_minmax', dev, numel=2 * height) \
-        if ter_minmax is not None else None
+    if ter_minmax is None:
+        p_dec, p_wc, p_ro = _addresses(_MATRIX[:3], (dec, w_comp, row_off), (_lib.DEC_WORDS, -1, -1), dev)
+        p_mm = None
+    else:
+        p_dec, p_wc, p_ro, p_mm = _addresses(_MATRIX, (dec, w_comp, row_off, ter_minmax),
+                                             (_lib.DEC_WORDS, -1, -1, 2 * height), dev)
     tern = torch.empty((height, width), dtype=torch.uint8, device=dev) if want_tern else None
     w = torch.empty((height, width), dtype=torch.bfloat16, device=dev) if want_w else None
     bad = ctypes.c_int32()
-    with _on_device(dev):
-        _lib.check(_lib.load().sub1_decode_counted(
-            p_dec, p_wc, p_ro, p_mm, tern.data_ptr() if want_tern else None,
-            w.data_ptr() if want_w else None, ctypes.byref(bad), height, width, _stream()))
+    _launch(dev, _lib.load().sub1_decode_counted, p_dec, p_wc, p_ro, p_mm, tern.data_ptr() if want_tern else None,
+            w.data_ptr() if want_w else None, ctypes.byref(bad), height, width)
     return tern, w, bad.value
 
 
