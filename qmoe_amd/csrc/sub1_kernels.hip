@@ -638,7 +638,6 @@ struct MoeArgs {
   int32_t *ctrl;  // the control words (sub1_common.h): ticket, fault counts, a word per token
   int tokens, d_model, d_ff, experts;
   int wi_tiles, wo_tiles;  // per token
-  bool at_once;            // a workgroup for every tile, all of them running: tile b is workgroup b's
   int act_dwords;          // LDS dwords of the activations; the table's first words follow
   int held;                // words of the table kept in LDS (0: none)
   int wi_expect;           // wi tiles a wo tile waits for (wi_tiles outside tests)
@@ -840,14 +839,15 @@ struct RowRun {
 // once, as many as make all wavefronts work side by side.  (Rounded up: a run more than there are wavefronts
 // is a turn of its own for one of them.  99 tokens, 569 x 3563, 61.2 -> 58.7 us; 130, 900 x 2500, 95.6 -> 90.8;
 // 61, 1501 x 3001, 65.2 -> 63.6; sizes that divide as before.)
-__device__ __forceinline__ int rows_at_a_time(int rows, int width, int waves, bool at_once) {
-  if (at_once) return min((rows + waves - 1) / waves, 64);
+template <bool kHeld>
+__device__ __forceinline__ int rows_at_a_time(int rows, int width, int waves) {
+  if (!kHeld) return min((rows + waves - 1) / waves, 64);
   return min(max((rows + waves - 1) / waves, max(64 * 640 / (width + 640), 1)), 64);
 }
 
 template <int kThreads>
 __global__ __launch_bounds__(kThreads, kThreads == 1024 ? 4 : 2) void moe_kernel(MoeArgs a) {
-  constexpr bool kHeld = kThreads == 1024;   // the form with the table's head in LDS
+  constexpr bool kHeld = kThreads == 1024;   // the form with the table's head in LDS, and with tickets
   extern __shared__ __align__(16) float lds[];
   __shared__ int s_ticket, s_row;
   __shared__ float2 s_partial[kThreads];
@@ -868,7 +868,7 @@ __global__ __launch_bounds__(kThreads, kThreads == 1024 ? 4 : 2) void moe_kernel
   run.held = a.held;
   for (;;) {
     int ticket = blockIdx.x;
-    if (!a.at_once) {
+    if (kHeld) {
       __syncthreads();  // previous tile's readers of lds and s_ticket are done
       if (threadIdx.x == 0)
         s_ticket = __hip_atomic_fetch_add(&a.ctrl[0], 1, __ATOMIC_RELAXED,
@@ -898,13 +898,13 @@ __global__ __launch_bounds__(kThreads, kThreads == 1024 ? 4 : 2) void moe_kernel
           const int64_t i = static_cast<int64_t>(t) * a.d_model + row;
           a.y[i] = a.x[i];
         }
-      if (a.at_once) break;
+      if (!kHeld) break;
       continue;   // a dropped token's word stays untouched
     }
     const int32_t *row_off = (is_wi ? a.wi_row_off : a.wo_row_off) + static_cast<int64_t>(e) * (height + 1);
     const uint16_t *codes = a.w_comp + (is_wi ? a.wi_code_base : a.wo_code_base)[e];
     const uint32_t *minmax = (is_wi ? a.wi_minmax : a.wo_minmax) + static_cast<int64_t>(e) * height;
-    const int at_a_time = rows_at_a_time(row_end - row_begin, width, kWaves, a.at_once);
+    const int at_a_time = rows_at_a_time<kHeld>(row_end - row_begin, width, kWaves);
     int row0 = row_begin + at_a_time * wave;   // the first run; further ones from s_row
     if (row0 < row_end) run.take(codes, row_off, row0, min(at_a_time, row_end - row0));
     if (threadIdx.x == 0) {
@@ -951,9 +951,9 @@ __global__ __launch_bounds__(kThreads, kThreads == 1024 ? 4 : 2) void moe_kernel
       // said once the tile's work is done: it takes a round trip to memory
       sub1::waited_on(&a.ctrl[sub1::token_word(t)], a.wo_tiles);
     }
-    if (a.at_once) break;
+    if (!kHeld) break;
   }
-  if (!a.at_once && threadIdx.x == 0) sub1::leave_launch(a.ctrl, gridDim.x);
+  if (kHeld && threadIdx.x == 0) sub1::leave_launch(a.ctrl, gridDim.x);
 }
 
 __global__ void zero_i32_kernel(int32_t *p, int n) {
@@ -1214,7 +1214,7 @@ extern "C" int sub1_moe_grouped(const sub1_moe_stack *st, const int32_t *token_e
   a.d_ff = st->d_ff;
   a.experts = st->experts;
   a.wait_ticks = sub1::wait_limit_ticks();
-  int device = 0, cus = 0, per_cu = 0;
+  int device = 0, cus = 0;
   HIP_TRY(hipGetDevice(&device));
   HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
   const int wmax = st->d_model > st->d_ff ? st->d_model : st->d_ff;
@@ -1224,53 +1224,25 @@ extern "C" int sub1_moe_grouped(const sub1_moe_stack *st, const int32_t *token_e
   // and the table from memory, which from some 90 million weights on takes longer:
   // base shapes, 16, 32 and 48 tokens 42, 46 and 48 us against 23, 35 and 51; large ones, 16 and 24 tokens
   // 44 and 48 against 37 and 51; c-2048, 4, 8 and 12 tokens 57, 58 and 61 against 36, 50 and 64.
-  const size_t lds_limit = 160 * 1024 - 64 - kMoeSweepThreads * sizeof(float2);
-  const bool worth_it = tokens >= cus || (tokens >= 10 && static_cast<int64_t>(tokens) * st->d_model * st->d_ff >= 90000000);
-  const bool sweep = worth_it &&
-                     a.act_dwords * sizeof(float) + 16384 * sizeof(uint32_t) <= lds_limit;
-  const int threads = sweep ? kMoeSweepThreads : kMoeThreads;
+  constexpr size_t lds_limit = 160 * 1024 - 64 - kMoeSweepThreads * sizeof(float2);
+  static_assert(lds_dwords_for_width(SUB1_MAX_WIDTH) * sizeof(float) + 16384 * sizeof(uint32_t) <= lds_limit,
+                "room for a head of the table beside any activations");
+  const bool sweep = tokens >= cus || (tokens >= 10 && static_cast<int64_t>(tokens) * st->d_model * st->d_ff >= 90000000);
   a.held = 0;
+  int64_t grid = cus;
   if (sweep) {
     const size_t room = (lds_limit - a.act_dwords * sizeof(float)) / sizeof(uint32_t) / 4 * 4;
     a.held = static_cast<int>(room < SUB1_DICT_ENTRIES ? room : SUB1_DICT_ENTRIES);
-  }
-  const size_t lds = (static_cast<size_t>(a.act_dwords) + a.held) * sizeof(float);
-  if (sweep) {
-    rc = allow_lds(moe_kernel<kMoeSweepThreads>, lds);
-    per_cu = 1;
-  } else {
-    rc = allow_lds(moe_kernel<kMoeThreads>, lds);
-    if (!rc)
-      HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, moe_kernel<kMoeThreads>,
-                                                           kMoeThreads, lds));
-  }
-  if (rc) return rc;
-  if (per_cu < 1) return fail(SUB1_ERR_INTERNAL, "sub1_moe_grouped: kernel does not fit a CU");
-  int64_t grid = static_cast<int64_t>(cus) * per_cu;
-  // A few tokens: a workgroup for every tile.  As many tiles as give every wavefront a turn of its
-  // own (64 groups, of which a row of W weights with 90 % zeros has W / 736 and a half), more where compute
-  // units would have none, and at most one of either projection for each.  (More are slower again:
-  // each counts itself and asks for words of the table.  Base and c-2048 shapes, 48, 96 and 192 tiles a
-  // token, us: one token 17.4, 19.7, 26.6 and 29.9, 22.9, 29.4.)
-  const int most = sweep ? 0 : cus / tokens;
-  const auto tiles_of = [&](int height, int width) {
-    const int turns = static_cast<int>(height * (width / 736.0 + 0.5) / kGroupsAtOnce) + 1;
-    return std::min({std::max(turns, std::min(48, cus / (2 * tokens))), most, (height + 3) / 4});
-  };
-  a.wi_tiles = tiles_of(st->d_ff, st->d_model);
-  a.wo_tiles = tiles_of(st->d_model, st->d_ff);
-  a.at_once = most > 0 && static_cast<int64_t>(tokens) * (a.wi_tiles + a.wo_tiles) <= grid;
-  if (!a.at_once) {
     // Parts of a projection: the number with which its tiles take the least time in
     // rounds of the grid.  A tile costs about 8 us (ticket, activations, the wait, the
     // wavefronts that finish early) besides its share of the projection, of which a
     // compute unit takes some 80 000 weights a microsecond.
     const double tile_share = 8.0 * 80000.0 / (static_cast<double>(st->d_model) * st->d_ff);
-    const int threads_rows = threads / 4;   // at least so many rows to a tile
+    constexpr int least_rows = kMoeSweepThreads / 4;   // of a tile
     auto parts_of = [&](int height) {
       int best = 1;
       double best_cost = 1e30;
-      for (int parts = 1; parts <= std::max(1, height / threads_rows); parts++) {
+      for (int parts = 1; parts <= std::max(1, height / least_rows); parts++) {
         const int64_t rounds = (static_cast<int64_t>(tokens) * parts + grid - 1) / grid;
         const double cost = rounds * (1.0 / parts + tile_share);
         if (cost < best_cost - 1e-9) {
@@ -1282,19 +1254,33 @@ extern "C" int sub1_moe_grouped(const sub1_moe_stack *st, const int32_t *token_e
     };
     a.wi_tiles = parts_of(st->d_ff);
     a.wo_tiles = parts_of(st->d_model);
+  } else {
+    // A workgroup for every tile.  As many tiles as give every wavefront a turn of its
+    // own (64 groups, of which a row of W weights with 90 % zeros has W / 736 and a half), more where compute
+    // units would have none, and at most one of either projection for each.  (More are slower again:
+    // each counts itself and asks for words of the table.  Base and c-2048 shapes, 48, 96 and 192 tiles a
+    // token, us: one token 17.4, 19.7, 26.6 and 29.9, 22.9, 29.4.)
+    const auto tiles_of = [&](int height, int width) {
+      const int turns = static_cast<int>(height * (width / 736.0 + 0.5) / kGroupsAtOnce) + 1;
+      return std::min({std::max(turns, std::min(48, cus / (2 * tokens))), cus / tokens, (height + 3) / 4});
+    };
+    a.wi_tiles = tiles_of(st->d_ff, st->d_model);
+    a.wo_tiles = tiles_of(st->d_model, st->d_ff);
   }
+  const size_t lds = (static_cast<size_t>(a.act_dwords) + a.held) * sizeof(float);
+  rc = sweep ? allow_lds(moe_kernel<kMoeSweepThreads>, lds) : allow_lds(moe_kernel<kMoeThreads>, lds);
+  if (rc) return rc;
   a.wi_expect = a.wi_tiles + sub1::expect_extra();
   const int64_t tiles = static_cast<int64_t>(tokens) * (a.wi_tiles + a.wo_tiles);
   if (tiles > INT32_MAX - (1 << 20))
     return fail(SUB1_ERR_SHAPE, "sub1_moe_grouped: too many tiles");
-  if (grid > tiles) grid = tiles;
 
   if (sweep) {
     sub1::note_kernel("moe_kernel<1024>");
-    moe_kernel<kMoeSweepThreads><<<static_cast<unsigned>(grid), threads, lds, s>>>(a);
+    moe_kernel<kMoeSweepThreads><<<static_cast<unsigned>(std::min(grid, tiles)), kMoeSweepThreads, lds, s>>>(a);
   } else {
     sub1::note_kernel("moe_kernel<256>");
-    moe_kernel<kMoeThreads><<<static_cast<unsigned>(grid), threads, lds, s>>>(a);
+    moe_kernel<kMoeThreads><<<static_cast<unsigned>(tiles), kMoeThreads, lds, s>>>(a);
   }
   HIP_TRY(hipGetLastError());
   return SUB1_OK;
