@@ -599,6 +599,10 @@ int sub1_timing_end(void *stream, double *elapsed_us);
  *   sub1_test_overstate_wait(k)  for tests of the above: later launches expect k
  *                             more workgroups in every wait than will ever
  *                             report, so each wait runs into the bound.
+ *   sub1_test_late_tiles(n)   for tests: in later packed expert launches with a
+ *                             workgroup for every tile, every other workgroup
+ *                             of wi stands still for n us, 0 .. 10 000, before it
+ *                             starts, as if it had found no room on the GPU.
  */
 int sub1_init(void);
 int sub1_fault_flags(int32_t *flags);
@@ -607,6 +611,7 @@ int sub1_clear_faults(void);
 int64_t sub1_fault_epoch(void);
 int sub1_set_wait_limit_us(int64_t microseconds);
 int sub1_test_overstate_wait(int extra);
+int sub1_test_late_tiles(int microseconds);
 
 /*
  * Calls that wait for the GPU (sub1_pack_weights_total, sub1_decode_counted and the prepare

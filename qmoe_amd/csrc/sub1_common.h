@@ -70,6 +70,7 @@ bool fault_flag_host(int word);
 // Longest wait between workgroups, in ticks of the device's constant-rate
 // clock (wall_clock64), and how much the tests overstate the count a wait
 // expects (0 outside tests).
+int64_t ticks_of(int64_t microseconds);   // of wall_clock64
 int64_t wait_limit_ticks();
 int expect_extra();
 

@@ -52,6 +52,7 @@ int32_t *g_fault_host = nullptr;     // pinned, mapped: kFaultWords words
 int32_t *g_fault_device = nullptr;   // the same words as the GPUs address them
 std::atomic<int64_t> g_wait_limit_us{250000};
 std::atomic<int> g_expect_extra{0};
+std::atomic<int> g_late_us{0};
 std::atomic<int> g_clock_khz{0};     // rate of wall_clock64 on the device first asked
 }  // namespace
 
@@ -77,7 +78,7 @@ bool fault_flag_host(int word) {
   return g_fault_host && *const_cast<volatile int32_t *>(&g_fault_host[word]) != 0;
 }
 
-int64_t wait_limit_ticks() {
+int64_t ticks_of(int64_t microseconds) {
   int khz = g_clock_khz.load();
   if (khz <= 0) {
     int device = 0, rate = 0;
@@ -89,8 +90,10 @@ int64_t wait_limit_ticks() {
       khz = 100000;   // 100 MHz
     g_clock_khz.store(khz);
   }
-  return g_wait_limit_us.load() * khz / 1000;
+  return microseconds * khz / 1000;
 }
+
+int64_t wait_limit_ticks() { return ticks_of(g_wait_limit_us.load()); }
 
 int expect_extra() { return g_expect_extra.load(); }
 
@@ -600,10 +603,18 @@ __global__ void tell_count_kernel(sub1::Answer answer) {
 // ticket.  A wo tile of token t needs all of h[t], so it waits until the wi tiles
 // of t have signalled; those have smaller tickets, were therefore taken by
 // workgroups that are already running, and never wait themselves, so the wait
-// always ends.  A few tokens have a workgroup for every tile instead, all of them running at
-// once: a wo tile's has its rows' codes and their words of the table by the time h is there.
+// always ends.
+//
+// A few tokens have a workgroup for every tile instead, by number, so that wi's tiles lie one to a compute
+// unit, and a wo tile's has its rows' codes and their words of the table by the time h is there.
 // (One token of base and c-2048 shapes 28.9 -> 17.3 us and 44.5 -> 22.5, nine of base shapes 43.8 -> 21.3,
-// with tickets and everything fetched behind the wait.)
+// with tickets and everything fetched behind the wait; with a ticket that only says which tile, of the launch
+// or of the token, 14 tokens of base shapes 22.6 -> 28.8 and 24.5, nine of c-2048 50.5 -> 62 and 68, as wi's tiles
+// then share units.)  They run all at once on a GPU that does nothing else; where other launches hold
+// units, workgroups that wait may keep those that they wait for from starting.  Every wi tile is therefore
+// CLAIMED by the workgroup that does it, and one that has waited for some time claims what nobody has, does
+// it and waits on: nobody waits for a tile that no running workgroup has, so this wait always ends too.
+// (Claims take 0.5 us of the 17 to 25 of a few tokens of base and large shapes.)
 //
 // Within a tile the wavefronts take runs of rows from a counter in LDS and give a
 // LANE to a GROUP of 32 codes, not to a row: a row's sum is the sum of its groups'
@@ -641,6 +652,8 @@ struct MoeArgs {
   int act_dwords;          // LDS dwords of the activations; the table's first words follow
   int held;                // words of the table kept in LDS (0: none)
   int wi_expect;           // wi tiles a wo tile waits for (wi_tiles outside tests)
+  int64_t patience;        // a workgroup for every tile: ticks after which a wo tile's claims tiles of wi
+  int64_t late;            // tests: ticks that every other wi tile's workgroup starts late
   int64_t wait_ticks;      // longest wait, in ticks of wall_clock64
   int32_t *sticky;         // fault flags in pinned host memory
   const int32_t *dec;      // the caller's table and the words kept of it
@@ -845,11 +858,73 @@ __device__ __forceinline__ int rows_at_a_time(int rows, int width, int waves) {
   return min(max((rows + waves - 1) / waves, max(64 * 640 / (width + 640), 1)), 64);
 }
 
+// Claims of a token's wi tiles, and its word where there are some: 64 bits, with a third count beside the
+// two of the others' (sub1_common.h), tiles that were done by workgroups of wo.  All of it is zero between launches.
+constexpr int kClaimWord = 2;          // from the token's word on: a bit for every tile
+constexpr int kMostClaims = 256;
+static_assert(kClaimWord + kMostClaims / 32 <= sub1::kCtrlTokenStride && sub1::kCtrlHeader % 2 == 0, "within the token's words");
+constexpr unsigned long long kTokenHelped = 1ull << 32;
+
+// Whether the tile was free.
+__device__ __forceinline__ bool claim_tile(int32_t *token, int tile) {
+  const int32_t bit = static_cast<int32_t>(1u << (tile & 31));
+  return !(__hip_atomic_fetch_or(&token[kClaimWord + tile / 32], bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit);
+}
+
+// Thread 0 of a wo tile's workgroup: bounded_wait, which after `patience` ticks claims a wi tile that
+// nobody has started and returns it; -1 once h is there (or the time is up).
+__device__ __forceinline__ int wait_or_claim(const MoeArgs &a, int32_t *token, int64_t patience) {
+  int looks = 0;
+  int64_t t0 = 0;
+  while ((__hip_atomic_load(token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xffff) < a.wi_expect) {
+    if ((++looks & 15) == 1) {
+      const int64_t now = static_cast<int64_t>(wall_clock64());
+      if (looks == 1) t0 = now;
+      if (now - t0 >= patience)
+        for (int first = 0; first < a.wi_tiles; first += 32) {
+          const uint32_t all = a.wi_tiles - first < 32 ? (1u << (a.wi_tiles - first)) - 1 : ~0u;
+          const uint32_t free = all & ~static_cast<uint32_t>(__hip_atomic_load(&token[kClaimWord + first / 32], __ATOMIC_RELAXED,
+                                                                               __HIP_MEMORY_SCOPE_AGENT));
+          if (!free) continue;
+          const int tile = first + __ffs(free) - 1;
+          // (counted first: whose tile it was leaves once it finds the claim)
+          unsigned long long *word = reinterpret_cast<unsigned long long *>(token);
+          __hip_atomic_fetch_add(word, kTokenHelped, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          sub1::drain_stores();
+          if (claim_tile(token, tile)) return tile;
+          __hip_atomic_fetch_add(word, ~0ull << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          break;   // somebody was faster: look again
+        }
+      if (now - t0 > a.wait_ticks) {
+        sub1::raise_fault(a.sticky, sub1::kFaultWait);
+        __hip_atomic_fetch_add(&a.ctrl[sub1::kCtrlGaveUp], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        break;
+      }
+    }
+    __builtin_amdgcn_s_sleep(2);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  return -1;
+}
+
+// Thread 0 of a workgroup of wo that is done, or of one of wi whose tile another has done.  With the last of
+// them nobody looks at the token's words any more, and they go back to zero.
+__device__ __forceinline__ void leave_token(const MoeArgs &a, int32_t *token) {
+  unsigned long long *word = reinterpret_cast<unsigned long long *>(token);
+  const unsigned long long before = __hip_atomic_fetch_add(word, static_cast<unsigned long long>(sub1::kTokenWaited),
+                                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int left = static_cast<int>(before >> 16 & 0xffff) + 1;
+  if (left != a.wo_tiles + static_cast<int>(before >> 32)) return;
+  for (int i = 0; i < (a.wi_tiles + 31) / 32; i++)
+    __hip_atomic_store(&token[kClaimWord + i], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 template <int kThreads>
 __global__ __launch_bounds__(kThreads, kThreads == 1024 ? 4 : 2) void moe_kernel(MoeArgs a) {
   constexpr bool kHeld = kThreads == 1024;   // the form with the table's head in LDS, and with tickets
   extern __shared__ __align__(16) float lds[];
-  __shared__ int s_ticket, s_row;
+  __shared__ int s_ticket, s_row, s_claimed;
   __shared__ float2 s_partial[kThreads];
   const int n_wi = a.tokens * a.wi_tiles;
   const int n_all = n_wi + a.tokens * a.wo_tiles;
@@ -866,8 +941,10 @@ __global__ __launch_bounds__(kThreads, kThreads == 1024 ? 4 : 2) void moe_kernel
   run.tab = a.tab;
   run.held_words = held_words;
   run.held = a.held;
+  int help = -1;   // a workgroup for every tile, of wo: one of wi that it does first
+  bool waited = false;
   for (;;) {
-    int ticket = blockIdx.x;
+    int ticket = !kHeld && help >= 0 ? help : static_cast<int>(blockIdx.x);
     if (kHeld) {
       __syncthreads();  // previous tile's readers of lds and s_ticket are done
       if (threadIdx.x == 0)
@@ -904,18 +981,39 @@ __global__ __launch_bounds__(kThreads, kThreads == 1024 ? 4 : 2) void moe_kernel
     const int32_t *row_off = (is_wi ? a.wi_row_off : a.wo_row_off) + static_cast<int64_t>(e) * (height + 1);
     const uint16_t *codes = a.w_comp + (is_wi ? a.wi_code_base : a.wo_code_base)[e];
     const uint32_t *minmax = (is_wi ? a.wi_minmax : a.wo_minmax) + static_cast<int64_t>(e) * height;
+    int32_t *token = &a.ctrl[sub1::token_word(t)];
+    bool taken = false;   // thread 0: somebody else does this tile of wi
+    if (!kHeld && is_wi && help < 0) {
+      if (a.late && part % 2 == 0) {
+        const int64_t t0 = static_cast<int64_t>(wall_clock64());
+        while (static_cast<int64_t>(wall_clock64()) - t0 < a.late) __builtin_amdgcn_s_sleep(64);
+      }
+      if (threadIdx.x == 0) taken = !claim_tile(token, part);
+    }
     const int at_a_time = rows_at_a_time<kHeld>(row_end - row_begin, width, kWaves);
     int row0 = row_begin + at_a_time * wave;   // the first run; further ones from s_row
     if (row0 < row_end) run.take(codes, row_off, row0, min(at_a_time, row_end - row0));
     if (threadIdx.x == 0) {
       s_row = row_begin + at_a_time * kWaves;
-      if (!is_wi)
-        sub1::bounded_wait(&a.ctrl[sub1::token_word(t)], a.wi_expect, a.wait_ticks, a.sticky,
-                           &a.ctrl[sub1::kCtrlGaveUp]);
+      if (kHeld && !is_wi) sub1::bounded_wait(token, a.wi_expect, a.wait_ticks, a.sticky, &a.ctrl[sub1::kCtrlGaveUp]);
+      if (!kHeld && !is_wi) s_claimed = wait_or_claim(a, token, waited ? 0 : a.patience);
     }
     __syncthreads();  // thread 0's acquire covers the whole workgroup
+    if (!kHeld && !is_wi) {
+      waited = true;
+      if (s_claimed >= 0) {
+        help = t * a.wi_tiles + s_claimed;
+        continue;
+      }
+    }
     stage_activations<kThreads>(lds, (is_wi ? a.x : a.h) + static_cast<int64_t>(t) * width, width);
+    // (asked for above: by now its answer is here)
+    if (!kHeld && is_wi && threadIdx.x == 0) s_claimed = taken;
     __syncthreads();
+    if (!kHeld && is_wi && s_claimed) {
+      if (threadIdx.x == 0) leave_token(a, token);
+      break;
+    }
     while (row0 < row_end) {
       const int rows = min(at_a_time, row_end - row0);
       const int row = row0 + lane;
@@ -945,13 +1043,16 @@ __global__ __launch_bounds__(kThreads, kThreads == 1024 ? 4 : 2) void moe_kernel
       sub1::drain_stores();
       __syncthreads();
       if (threadIdx.x == 0)
-        __hip_atomic_fetch_add(&a.ctrl[sub1::token_word(t)], 1, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_fetch_add(token, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     } else if (threadIdx.x == 0) {
       // said once the tile's work is done: it takes a round trip to memory
-      sub1::waited_on(&a.ctrl[sub1::token_word(t)], a.wo_tiles);
+      if (kHeld)
+        sub1::waited_on(token, a.wo_tiles);
+      else
+        leave_token(a, token);
     }
-    if (!kHeld) break;
+    if (!kHeld && help < 0) break;
+    help = -1;   // (its own tile next)
   }
   if (kHeld && threadIdx.x == 0) sub1::leave_launch(a.ctrl, gridDim.x);
 }
@@ -1032,6 +1133,7 @@ int slot_table_for(const int32_t *dec, hipStream_t stream, TableSlot *out, int32
 
 constexpr int kMoeThreads = 256;
 constexpr int kGroupsAtOnce = 48 * kMoeThreads / 64;   // groups that a workgroup's wavefronts take in a turn, with room
+constexpr int kPatienceUs = 20;          // all workgroups of a launch have started by then on a GPU that does nothing else
 constexpr int kMoeSweepThreads = 1024;   // one workgroup per compute unit, the table's head in its LDS
 
 template <typename K>
@@ -1214,6 +1316,8 @@ extern "C" int sub1_moe_grouped(const sub1_moe_stack *st, const int32_t *token_e
   a.d_ff = st->d_ff;
   a.experts = st->experts;
   a.wait_ticks = sub1::wait_limit_ticks();
+  a.patience = sub1::ticks_of(kPatienceUs);
+  a.late = sub1::ticks_of(sub1::g_late_us.load());
   int device = 0, cus = 0;
   HIP_TRY(hipGetDevice(&device));
   HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
@@ -1262,7 +1366,7 @@ extern "C" int sub1_moe_grouped(const sub1_moe_stack *st, const int32_t *token_e
     // token, us: one token 17.4, 19.7, 26.6 and 29.9, 22.9, 29.4.)
     const auto tiles_of = [&](int height, int width) {
       const int turns = static_cast<int>(height * (width / 736.0 + 0.5) / kGroupsAtOnce) + 1;
-      return std::min({std::max(turns, std::min(48, cus / (2 * tokens))), cus / tokens, (height + 3) / 4});
+      return std::min({std::max(turns, std::min(48, cus / (2 * tokens))), cus / tokens, (height + 3) / 4, kMostClaims});
     };
     a.wi_tiles = tiles_of(st->d_ff, st->d_model);
     a.wo_tiles = tiles_of(st->d_model, st->d_ff);
@@ -1408,6 +1512,13 @@ extern "C" int sub1_test_overstate_wait(int extra) {
 extern "C" int sub1_test_fail_answers(int calls) {
   if (calls < 0) return fail(SUB1_ERR_SHAPE, "sub1_test_fail_answers: negative count");
   sub1::g_fail_answers.store(calls);
+  return SUB1_OK;
+}
+
+extern "C" int sub1_test_late_tiles(int microseconds) {
+  if (microseconds < 0 || microseconds > 10000)
+    return fail(SUB1_ERR_SHAPE, "sub1_test_late_tiles: %d us outside 0..10000", microseconds);
+  sub1::g_late_us.store(microseconds);
   return SUB1_OK;
 }
 

@@ -80,3 +80,47 @@ def test_a_workgroup_for_every_tile(oracle, d_model, d_ff, experts, tokens):
     weights = tokens * d_model * d_ff
     assert sub1_hip._lib.load().sub1_last_kernel().decode() == (
         'moe_kernel<1024>' if tokens >= 10 and weights >= 90000000 else 'moe_kernel<256>')
+
+
+TOKEN_WORDS = 4 * (64 + 2 * 2 * 12288)     # where in a workspace the words begin that launches count with, 64 bytes a token
+
+
+@pytest.mark.parametrize('late', [0, 200])
+@pytest.mark.parametrize('d_model,d_ff', [(768, 3072), (64, 3), (2080, 1100)])
+def test_tiles_whose_workgroups_start_late_are_done_by_others(oracle, d_model, d_ff, late):
+    """A workgroup of wo that waits for a tile of wi that nobody has begun does it itself, and the one that
+    comes for it later finds that; on several streams, that all overlap, too."""
+    from qmoe_amd import sub1, sub1_hip
+    lib = sub1_hip._lib.load()
+    wi = [uneven_layer(oracle, d_ff, d_model, [0.1, 0.3], 10 + e) for e in range(2)]
+    wo = [uneven_layer(oracle, d_model, d_ff, [0.1, 0.02, 1.0], 20 + e) for e in range(2)]
+
+    def dev(layer):
+        codes, row_off, minmax = layer
+        return torch.from_numpy(codes.view(np.int16)).cuda(), torch.from_numpy(row_off).cuda(), bf16_dev(minmax)
+
+    stack = sub1_hip.ExpertStack.from_layers(sub1.DEC[0], [dev(l) for l in wi], [dev(l) for l in wo])
+    xs = np.stack([so.synthetic_activation(d_model, 30 + i) for i in range(4)])
+    want = np.stack([oracle.expert_ffn(wi[i % 2], wo[i % 2], xs[i], order=1)[0] for i in range(4)])
+    calls = [np.arange(t) % 4 for t in (38, 1, 14, 9)]
+    inputs = [(bf16_dev(xs[i]), torch.from_numpy((i % 2).astype(np.int32)).cuda()) for i in calls]
+    streams = [torch.cuda.Stream() for _ in calls]
+    assert lib.sub1_test_late_tiles(-1) != 0 and lib.sub1_test_late_tiles(10001) != 0
+    torch.cuda.synchronize()
+    try:
+        sub1_hip._lib.check(lib.sub1_test_late_tiles(late))
+        outs = []
+        for _ in range(5):
+            for k, stream in enumerate(streams):
+                with torch.cuda.stream(stream):
+                    outs.append((k, stack.forward(*inputs[k])))
+                assert lib.sub1_last_kernel() == b'moe_kernel<256>'
+        torch.cuda.synchronize()
+    finally:
+        sub1_hip._lib.check(lib.sub1_test_late_tiles(0))
+    assert all(np.array_equal(bits_host(y), want[calls[k]]) for k, y in outs)
+    for k, stream in enumerate(streams):
+        with torch.cuda.stream(stream):
+            tokens = len(calls[k])
+            assert stack.launch_faults(tokens) == (0, 0)
+            assert not bool(stack.workspace(tokens)[TOKEN_WORDS:TOKEN_WORDS + 64 * tokens].any())
