@@ -82,15 +82,15 @@ struct KindMeta {
   int height, width;
 };
 
-constexpr int kStatusWords = 64, kStatusLong = 5, kLongBits = 32 * (kStatusWords - kStatusLong);
+constexpr int kStatusWords = 64, kStatusLong = 4, kLongBits = 32 * (kStatusWords - kStatusLong);
 struct MetaLayout {
   KindMeta k[2];
   int kinds;
   int64_t counts;       // i32 [all slices + 1] chunk counts, scanned in place
   int64_t status;       // i32 [kStatusWords]: [0] rows whose codes do not cover the width, [1], [2]
                         // longest slice of kind 0 / 1 in chunks, [3] what check_on_device
-                        // found, [4] whether there are long rows (counting); from [5] on a bit for
-                        // every slice, mod kLongBits, that has some (emitting)
+                        // found; from [4] on a bit for every slice, mod kLongBits, that has long
+                        // rows (emitting)
   int64_t bytes;
 };
 
@@ -179,16 +179,23 @@ struct KindSource {
   const uint32_t *const *minmax_of;
 };
 
-// A row of more than twice its matrix's average of codes (and a few) is a LONG one.
+// A row of more than `average` times its matrix's average of codes (and a few) is a LONG one.  Twice
+// where there is at most one group of 64 rows or two to a compute unit: a group waits for its longest row, and
+// hardly anything else is there to do.  More of them hide that, and the words of the dictionary that long rows take
+// from memory count: as many times as a unit has groups, up to 4.2.  (Preparing, rows with 90 % zeros, us, a lane to every
+// row / to eight codes of the rows without zeros, of which there are a tenth, a fifth, two fifths.  One 6144 x 2080
+// 325 / 171, 331 / 181, 323 / 195; eight, 3 groups a unit, 372 / 253, 361 / 331, 346 / 500; 64 base
+// experts, 15 a unit, 523 / 509, 509 / 740, 501 / 1300; 30 of c-2048 936 / 1000, 959 / 1630, 1055 / 2770.)
+constexpr float kLongFromFew = 2.f, kLongFromMany = 4.2f;
 constexpr int kLongRowsFrom = 16;
-__device__ __forceinline__ const uint16_t *row_codes(const KindSource &ks, int e, int r,
-                                                     int height, int width, int &n, bool &is_long) {
+__device__ __forceinline__ const uint16_t *row_codes(const KindSource &ks, int e, int r, int height, int width,
+                                                     float average, int &n, bool &is_long) {
   const int32_t *ro = ks.row_off_of ? ks.row_off_of[e]
                                     : ks.row_off + static_cast<int64_t>(e) * (height + 1);
   n = ro[r + 1] - ro[r];
   if (n < 1 || n > (width + 1) / 2) n = 0;   // counted as a bad row by walk_rows_kernel
   // (the sixteen: short rows stay with the lanes; in floating point, which a division costs less in)
-  is_long = n > kLongRowsFrom && static_cast<float>(n - kLongRowsFrom) * height > 2.f * static_cast<float>(ro[height]);
+  is_long = n > kLongRowsFrom && static_cast<float>(n - kLongRowsFrom) * height > average * static_cast<float>(ro[height]);
   const uint16_t *codes = ks.w_comp_of ? ks.w_comp_of[e]
                                        : ks.w_comp + (ks.code_base ? ks.code_base[e] : 0);
   return codes + ro[r];
@@ -201,8 +208,8 @@ __device__ __forceinline__ const uint16_t *row_codes(const KindSource &ks, int e
 // lane asks for eight codes and their eight entries at once.
 //
 // A wavefront of rows takes as long as the longest of them, and a row without zeros has
-// seven times the codes of others.  Long rows are therefore left aside: order_rows_kernel counts
-// them before it orders the rows, emit_long_rows_kernel emits them, a lane to eight of their codes.
+// seven times the codes of others.  Long rows are therefore left aside, for a lane to take eight of
+// their codes: counting notes them in LDS and does them last, emit_long_rows_kernel emits them.
 //
 // Counting needs little of an entry, 16 bits, so that all 65 536 are held, and beside
 // them two more bits of each for the rare gap that takes several steps:
@@ -217,7 +224,8 @@ constexpr int kWalkThreads = 1024;
 constexpr int kHeldWords = 40000;
 constexpr int kCountWords = SUB1_DICT_ENTRIES / 2 + SUB1_DICT_ENTRIES / 16;   // 16-bit entries, then symbols
 constexpr size_t kWalkLds = kHeldWords * sizeof(uint32_t);
-constexpr size_t kCountLds = kCountWords * sizeof(uint32_t);
+constexpr int kLongList = 2048;   // long rows of a workgroup that counting leaves aside (a lane walks what there are more)
+constexpr size_t kCountLds = (kCountWords + kLongList) * sizeof(uint32_t);
 
 struct HeldTable {
   const uint32_t *all;    // global memory
@@ -320,6 +328,7 @@ __device__ __forceinline__ int pick(int n, int a, int b) {
 struct WalkKind {
   KindSource source;
   int height, width, slices;
+  float long_from;              // from how many times a matrix's average of codes on a row is a long one
   int64_t tasks;                // of 64 rows (counting: in the matrices' own order; emitting: slices)
   int64_t first_slice;          // emitting: among all kinds' slices
   uint16_t *row_len;            // counting
@@ -335,7 +344,6 @@ struct WalkArgs {
   uint32_t *long_bits;           // emitting: long rows are another launch's, and these slices have some (NULL: they are not)
   sub1::Answer answer;           // emitting: the first word says what that is
   int32_t *status;
-  int32_t *any_long;             // counting sets it (zero before) where it has left long rows
   uint2 *stream;
   uint16_t *ckpt;
 };
@@ -348,21 +356,28 @@ constexpr int kLongGap = 60;
 // that a padded row makes after them is not counted: it fits the padding).  An entry's
 // non-zeros are 27 columns apart at most, so only the gap before the first of them can
 // take more than one.
-__device__ __forceinline__ void count_rows(const CountTable &table, const WalkKind &k, int count,
-                                           int64_t task, int32_t *status, int32_t *any_long) {
+__device__ __forceinline__ const uint16_t *task_row(const WalkKind &k, int64_t task, int lane, int &n, bool &is_long) {
   // rows of a task: from row `first` of a matrix on, and of the next ones
-  const int64_t g = task * 64 + (threadIdx.x & 63);
-  if (g >= static_cast<int64_t>(count) * k.height) return;
   const int first_e = static_cast<int>(task * 64 / k.height);
-  const uint32_t past = static_cast<uint32_t>(g - static_cast<int64_t>(first_e) * k.height);
+  const uint32_t past = static_cast<uint32_t>(task * 64 + lane - static_cast<int64_t>(first_e) * k.height);
   const int e = first_e + static_cast<int>(past / static_cast<uint32_t>(k.height));
   const int r = static_cast<int>(past % static_cast<uint32_t>(k.height));
+  return row_codes(k.source, e, r, k.height, k.width, k.long_from, n, is_long);
+}
+__device__ __forceinline__ void count_rows(const CountTable &table, const WalkKind &k, int count,
+                                           int64_t task, int turn, int32_t *status, uint32_t *longs, int *n_longs) {
+  const int lane = threadIdx.x & 63;
+  const int64_t g = task * 64 + lane;
+  if (g >= static_cast<int64_t>(count) * k.height) return;
   int n;
   bool is_long;
-  const uint16_t *codes = row_codes(k.source, e, r, k.height, k.width, n, is_long);
+  const uint16_t *codes = task_row(k, task, lane, n, is_long);
   if (is_long) {
-    *any_long = 1;
-    return;
+    const int i = atomicAdd(n_longs, 1);
+    if (i < kLongList) {
+      longs[i] = static_cast<uint32_t>(turn) << 6 | static_cast<uint32_t>(lane);
+      return;
+    }
   }
   int col = 0, entries = 0;
   int since = 0;       // columns from the last non-zero's to col (from column 0 where there is none)
@@ -504,7 +519,7 @@ __device__ __forceinline__ void emit_rows(const HeldTable &table, const WalkKind
   if (ridx != 0xffff) {
     int n;
     bool is_long;
-    const uint16_t *codes = row_codes(k.source, e, ridx, k.height, k.width, n, is_long);
+    const uint16_t *codes = row_codes(k.source, e, ridx, k.height, k.width, k.long_from, n, is_long);
     if (is_long && long_bits) {
       const uint32_t bit = static_cast<uint32_t>(k.first_slice + slice) % kLongBits;
       atomicOr(&long_bits[bit / 32], 1u << (bit % 32));
@@ -545,40 +560,6 @@ __device__ __forceinline__ void emit_rows(const HeldTable &table, const WalkKind
   while (sink.at < sink.end) sink.store(0u, at);
 }
 
-// Task t goes to workgroup t mod grid: a matrix of a few slices is spread over as many
-// compute units.  Within it the wavefronts take the next one when they are done: a row of
-// wo has four times the codes of one of wi, and dealt out beforehand the busiest wavefront
-// has 1.7 times the average (counting 40 us, emitting 96).
-// 128 base experts (26 million codes): counting takes 32 us, 22 vector instructions a code
-// (64 with entry by entry of a whole word, 60 instructions); emitting 84 and about 65 (113
-// with a place that may store behind every entry, 99 instructions).  Both are bound by
-// issuing those, beside 6 us of filling LDS.  (32 codes asked for together instead of 8,
-// a cache line's worth: 37 and 81 us.)
-template <bool kEmit>
-__global__ __launch_bounds__(kWalkThreads) void walk_rows_kernel(WalkArgs a) {
-  extern __shared__ __align__(16) uint32_t held[];
-  __shared__ int s_turn;
-  const int found = *a.found;
-  if (kEmit && blockIdx.x == 0 && threadIdx.x == 0) sub1::tell(a.answer, 0, found);
-  if (found) return;
-  if (threadIdx.x == 0) s_turn = 0;
-  hold_table(kEmit ? a.table : a.count_table, held, kEmit ? kHeldWords : kCountWords);
-  const int64_t all = a.k[0].tasks + (a.kinds == 2 ? a.k[1].tasks : 0);
-  for (;;) {
-    int turn = 0;
-    if ((threadIdx.x & 63) == 0) turn = atomicAdd(&s_turn, 1);
-    int64_t task = blockIdx.x + static_cast<int64_t>(gridDim.x) * __builtin_amdgcn_readfirstlane(turn);
-    if (task >= all) break;
-    const bool second = task >= a.k[0].tasks;
-    if (second) task -= a.k[0].tasks;
-    const WalkKind &k = a.k[second ? 1 : 0];
-    if (kEmit)
-      emit_rows(HeldTable{a.table, held}, k, task, a.stream, a.ckpt, a.long_bits);
-    else
-      count_rows(CountTable{a.table, held}, k, a.count, task, a.status, a.any_long);
-  }
-}
-
 // ------------------------------------------------------------- long rows --
 //
 // A wavefront takes a long row, a lane a GROUP of eight of its codes.  What a group has to know
@@ -588,8 +569,10 @@ __global__ __launch_bounds__(kWalkThreads) void walk_rows_kernel(WalkArgs a) {
 // come from global memory: these are few codes.
 //
 // 63 base experts whose rows have 75 to 98 % zeros, one in a hundred none: counting 177 us before,
-// 50 and 16 (in order_rows_kernel), emitting 303 before, 101 and 79.  (Taken by groups within the walks
-// themselves they make those of even rows slower, by 2 of 33 and 4 of 85 us, with none there.)
+// 54 with that (ordering them 15), emitting 303, 104 and 75 in a launch of its own.  (Taken by groups where they are met
+// they make the walks of even rows slower, by 2 of 33 and 4 of 85 us, with none there; counted by the
+// workgroup that orders their matrix, one 6144 x 2080 with two fifths of them takes 1400 us to prepare, 320 with a
+// lane to each, 195 now.)
 constexpr int kGroupOfCodes = 8;
 
 // Eight of a row's codes, from code `at` on, and which of them there are.  (Loads stay within
@@ -671,19 +654,33 @@ __device__ __forceinline__ const uint16_t *codes_of_lane(const uint16_t *codes, 
   return reinterpret_cast<const uint16_t *>(static_cast<uint64_t>(high) << 32 | low);
 }
 
-// The entries of a matrix's long rows, by a workgroup.
-__device__ __forceinline__ void count_long_rows(const KindSource &source, int e, int height, int width,
-                                                const uint32_t *table, uint16_t *row_len, int32_t *status) {
-  const int lane = threadIdx.x & 63;
-  for (int r0 = threadIdx.x & ~63; r0 < height; r0 += blockDim.x) {
+// The entries of the long rows that a workgroup has left aside (as `turn` << 6 | lane), its
+// wavefronts in turn.
+__device__ __forceinline__ void count_long_rows(const WalkArgs &a, const uint32_t *longs, int n_longs) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int kWaves = kWalkThreads / 64;
+  for (int first = wave; first < n_longs; first += 64 * kWaves) {
+    // a lane asks for where one of them is
+    const int i = first + kWaves * lane;
+    const int here = min((n_longs - first + kWaves - 1) / kWaves, 64);
     int n = 0;
-    bool is_long = false;
+    int64_t g = 0;
+    bool second = false;
     const uint16_t *codes = nullptr;
-    if (r0 + lane < height) codes = row_codes(source, e, r0 + lane, height, width, n, is_long);
-    for (unsigned long long longs = __ballot(is_long); longs; longs &= longs - 1) {
-      const int who = __ffsll(longs) - 1;
+    if (lane < here) {
+      const uint32_t what = longs[i];
+      int64_t task = blockIdx.x + static_cast<int64_t>(gridDim.x) * (what >> 6);
+      second = task >= a.k[0].tasks;
+      if (second) task -= a.k[0].tasks;
+      bool is_long;
+      codes = task_row(a.k[second ? 1 : 0], task, what & 63u, n, is_long);
+      g = task * 64 + (what & 63u);
+    }
+    uint16_t entries_of = 0;
+    for (int who = 0; who < here; who++) {
+      const int width = a.k[__builtin_amdgcn_readlane(second, who)].width;
       int entries = 0;
-      walk_long_row(table, codes_of_lane(codes, who), __builtin_amdgcn_readlane(n, who),
+      walk_long_row(a.table, codes_of_lane(codes, who), __builtin_amdgcn_readlane(n, who),
                     [&](const uint32_t (&w)[kGroupOfCodes], int &from, int &at, bool live, bool ends) {
 #pragma unroll
                       for (int j = 0; j < kGroupOfCodes; j++) {
@@ -691,11 +688,54 @@ __device__ __forceinline__ void count_long_rows(const KindSource &source, int e,
                         entries += c.nonzeros + c.more;
                       }
                       // a row's codes cover its width rounded up to a whole pair, exactly
-                      if (live && ends && from != 2 * ((width + 1) & ~1)) atomicAdd(&status[0], 1);
+                      if (live && ends && from != 2 * ((width + 1) & ~1)) atomicAdd(&a.status[0], 1);
                     });
       entries = __builtin_amdgcn_readlane(sub1::wave_prefix_sum(entries), 63);
-      if (lane == 0) row_len[r0 + who] = static_cast<uint16_t>(min(entries, kMaxRowEntries));
+      if (lane == who) entries_of = static_cast<uint16_t>(min(entries, kMaxRowEntries));
     }
+    if (lane < here) a.k[second ? 1 : 0].row_len[g] = entries_of;
+  }
+}
+
+// Task t goes to workgroup t mod grid: a matrix of a few slices is spread over as many
+// compute units.  Within it the wavefronts take the next one when they are done: a row of
+// wo has four times the codes of one of wi, and dealt out beforehand the busiest wavefront
+// has 1.7 times the average (counting 40 us, emitting 96).
+// 128 base experts (26 million codes): counting takes 32 us, 22 vector instructions a code
+// (64 with entry by entry of a whole word, 60 instructions); emitting 84 and about 65 (113
+// with a place that may store behind every entry, 99 instructions).  Both are bound by
+// issuing those, beside 6 us of filling LDS.  (32 codes asked for together instead of 8,
+// a cache line's worth: 37 and 81 us.)
+template <bool kEmit>
+__global__ __launch_bounds__(kWalkThreads) void walk_rows_kernel(WalkArgs a) {
+  extern __shared__ __align__(16) uint32_t held[];
+  __shared__ int s_turn, s_longs;
+  const int found = *a.found;
+  if (kEmit && blockIdx.x == 0 && threadIdx.x == 0) sub1::tell(a.answer, 0, found);
+  if (found) return;
+  if (threadIdx.x == 0) {
+    s_turn = 0;
+    s_longs = 0;
+  }
+  hold_table(kEmit ? a.table : a.count_table, held, kEmit ? kHeldWords : kCountWords);
+  const int64_t all = a.k[0].tasks + (a.kinds == 2 ? a.k[1].tasks : 0);
+  for (;;) {
+    int turn = 0;
+    if ((threadIdx.x & 63) == 0) turn = atomicAdd(&s_turn, 1);
+    turn = __builtin_amdgcn_readfirstlane(turn);
+    int64_t task = blockIdx.x + static_cast<int64_t>(gridDim.x) * turn;
+    if (task >= all) break;
+    const bool second = task >= a.k[0].tasks;
+    if (second) task -= a.k[0].tasks;
+    const WalkKind &k = a.k[second ? 1 : 0];
+    if (kEmit)
+      emit_rows(HeldTable{a.table, held}, k, task, a.stream, a.ckpt, a.long_bits);
+    else
+      count_rows(CountTable{a.table, held}, k, a.count, task, turn, a.status, held + kCountWords, &s_longs);
+  }
+  if (!kEmit) {
+    __syncthreads();
+    count_long_rows(a, held + kCountWords, min(s_longs, kLongList));
   }
 }
 
@@ -721,7 +761,7 @@ __global__ __launch_bounds__(kLongThreads) void emit_long_rows_kernel(WalkArgs a
     bool is_long = false;
     const uint16_t *codes = nullptr;
     if (ridx != 0xffff)
-      codes = row_codes(k.source, static_cast<int>(slice / k.slices), ridx, k.height, k.width, n, is_long);
+      codes = row_codes(k.source, static_cast<int>(slice / k.slices), ridx, k.height, k.width, k.long_from, n, is_long);
     const SliceOut s = slice_out(k, slice, a.stream, a.ckpt);
     int turn_of = 0;   // the wavefronts take the long rows in turn
     for (unsigned long long longs = __ballot(is_long); longs; longs &= longs - 1) {
@@ -806,17 +846,16 @@ size_t order_rows_lds(int height) {
 // experts then take as long as wi alone (24 us, 34 one kind after the other).
 struct OrderKind {
   KindSource source;
-  uint16_t *row_len;
+  const uint16_t *row_len;
   uint16_t *row_idx;
   uint32_t *minmax;
   uint16_t *slice_len;
   int32_t *counts;
-  int height, width, slices;
+  int height, slices;
 };
 struct OrderArgs {
   OrderKind k[2];
-  const int32_t *found, *any_long;
-  const uint32_t *table;
+  const int32_t *found;
   int32_t *status;
 };
 
@@ -842,10 +881,6 @@ __global__ __launch_bounds__(kOrderThreads) void order_rows_kernel(OrderArgs a) 
   const uint32_t *mm = ks.minmax_of ? ks.minmax_of[e] : ks.minmax + static_cast<int64_t>(e) * height;
   const int64_t lane0 = static_cast<int64_t>(e) * slices * 64;
 
-  if (*a.any_long) {
-    count_long_rows(ks, e, height, k.width, a.table, k.row_len + static_cast<int64_t>(e) * height, status);
-    __syncthreads();
-  }
   int low = kMaxRowEntries, high = 0;
   for (int r = tid; r < height; r += kOrderThreads) {
     low = min(low, static_cast<int>(rl[r]));
@@ -3151,18 +3186,20 @@ template <bool kEmit>
 int launch_walk(const Source &src, const MetaLayout &m, WalkArgs &w, hipStream_t s) {
   w.kinds = src.kinds;
   w.count = src.count;
-  int64_t tasks = 0;
+  int device = 0, cus = 0;
+  HIP_TRY(hipGetDevice(&device));
+  HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+  int64_t tasks = 0, groups = 0;
+  for (int i = 0; i < src.kinds; i++) groups += static_cast<int64_t>(src.count) * m.k[i].slices;
   for (int i = 0; i < src.kinds; i++) {
     WalkKind &k = w.k[walk_place(src, i)];
+    k.long_from = std::min(std::max(static_cast<float>(groups) / cus, kLongFromFew), kLongFromMany);
     k.source = src.k[i];
     k.height = m.k[i].height;
     k.width = m.k[i].width;
     k.slices = m.k[i].slices;
     tasks += k.tasks;
   }
-  int device = 0, cus = 0;
-  HIP_TRY(hipGetDevice(&device));
-  HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
   constexpr size_t lds = kEmit ? kWalkLds : kCountLds;
   HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(walk_rows_kernel<kEmit>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
@@ -3185,14 +3222,13 @@ int prepare_layout(const Source &src, void *meta, int64_t meta_bytes, LayoutResu
   sub1::AnswerSlot slot;
   int rc = slot.take(s, who);
   if (rc) return rc;
-  zero_words_kernel<<<1, 64, 0, s>>>(status, 5);
+  zero_words_kernel<<<1, 64, 0, s>>>(status, 4);
   WalkArgs w{};
   rc = check_on_device(src, status + 3, w, s);
   if (!rc) rc = slot.launched(who);
   if (rc) return rc;
   int32_t *counts = reinterpret_cast<int32_t *>(base + m.counts);
   w.status = status;
-  w.any_long = status + 4;
   for (int i = 0; i < src.kinds; i++) {
     const KindMeta &k = m.k[i];
     WalkKind &wk = w.k[walk_place(src, i)];
@@ -3208,19 +3244,16 @@ int prepare_layout(const Source &src, void *meta, int64_t meta_bytes, LayoutResu
   OrderArgs o{};
   o.status = status;
   o.found = status + 3;
-  o.any_long = status + 4;
-  o.table = w.table;
   size_t lds = 0;
   for (int i = 0; i < src.kinds; i++) {
     const KindMeta &k = m.k[i];
     o.k[i] = {src.k[i],
-              reinterpret_cast<uint16_t *>(base + k.row_len),
+              reinterpret_cast<const uint16_t *>(base + k.row_len),
               reinterpret_cast<uint16_t *>(base + k.row_idx),
               reinterpret_cast<uint32_t *>(base + k.minmax),
               reinterpret_cast<uint16_t *>(base + k.slice_len),
               counts + slice0,
               k.height,
-              k.width,
               k.slices};
     lds = std::max(lds, order_rows_lds(k.height));
     slice0 += static_cast<int64_t>(src.count) * k.slices;

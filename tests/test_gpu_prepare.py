@@ -54,6 +54,20 @@ def test_prepared_rows_come_back_whole(gpu, height, width, shares):
     assert torch.equal(y[0], values.gather(1, symbols[:, column:column + 1].long())[:, 0])
 
 
+@pytest.mark.parametrize('height,width,count,shares', [
+    (700, 2000, 3, [1.0, 0.1, 0.1]),                 # a few of them to a workgroup
+    (65534, 300, 34, [1.0, 0.0, 0.0, 0.0])])         # more than it keeps a list of
+def test_many_long_rows_come_back_whole(gpu, height, width, count, shares):
+    sub1, op = gpu
+    symbols = symbols_of(height, width, shares, seed=height + width)
+    w_comp, row_off = packed(gpu, symbols)
+    minmax = torch.randn(2 * height, generator=torch.Generator().manual_seed(1)).bfloat16().cuda()
+    prepared = op.PreparedMatrix(sub1.DEC[0], w_comp, row_off.repeat(count), minmax.repeat(count), width,
+                                 torch.zeros(count, dtype=torch.int64, device='cuda'))
+    for matrix in (0, count // 2, count - 1):
+        assert torch.equal(prepared.decode(matrix), symbols), matrix
+
+
 @pytest.mark.parametrize('d_model,d_ff', [(303, 250), (64, 1400), (1024, 65), (229, 3001)])
 def test_long_gaps_and_dropped_digits_are_counted_as_they_are_written(gpu, oracle, d_model, d_ff):
     """Gaps about the longest step (59 to 64 columns, at every column of sixteen and with
