@@ -48,6 +48,16 @@ __device__ __forceinline__ void drain_stores() {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// The dynamic LDS that launches of a kernel may have: the most that any of them asks for, and never
+// this launch's own, as another thread's, of other shapes, may lie between this call and the launch.
+constexpr size_t kMostLds = 160 * 1024 - 64;   // beside some words of a kernel's own
+template <size_t kBytes, class Kernel>
+inline hipError_t allow_lds(Kernel *kernel) {
+  static_assert(kBytes <= 160 * 1024, "what a compute unit has");
+  return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                             static_cast<int>(kBytes));
+}
+
 inline bool misaligned(const void *p, size_t a) {
   return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0;
 }

@@ -1136,15 +1136,6 @@ constexpr int kGroupsAtOnce = 48 * kMoeThreads / 64;   // groups that a workgrou
 constexpr int kPatienceUs = 20;          // all workgroups of a launch have started by then on a GPU that does nothing else
 constexpr int kMoeSweepThreads = 1024;   // one workgroup per compute unit, the table's head in its LDS
 
-template <typename K>
-int allow_lds(K kernel, size_t bytes) {
-  if (bytes > 48 * 1024)
-    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                static_cast<int>(bytes)));
-  return SUB1_OK;
-}
-
 hipEvent_t g_ev_begin = nullptr, g_ev_end = nullptr;
 
 }  // namespace
@@ -1328,8 +1319,9 @@ extern "C" int sub1_moe_grouped(const sub1_moe_stack *st, const int32_t *token_e
   // and the table from memory, which from some 90 million weights on takes longer:
   // base shapes, 16, 32 and 48 tokens 42, 46 and 48 us against 23, 35 and 51; large ones, 16 and 24 tokens
   // 44 and 48 against 37 and 51; c-2048, 4, 8 and 12 tokens 57, 58 and 61 against 36, 50 and 64.
-  constexpr size_t lds_limit = 160 * 1024 - 64 - kMoeSweepThreads * sizeof(float2);
-  static_assert(lds_dwords_for_width(SUB1_MAX_WIDTH) * sizeof(float) + 16384 * sizeof(uint32_t) <= lds_limit,
+  constexpr size_t lds_limit = sub1::kMostLds - kMoeSweepThreads * sizeof(float2);
+  constexpr size_t most_activations = lds_dwords_for_width(SUB1_MAX_WIDTH) * sizeof(float);
+  static_assert(most_activations + 16384 * sizeof(uint32_t) <= lds_limit,
                 "room for a head of the table beside any activations");
   const bool sweep = tokens >= cus || (tokens >= 10 && static_cast<int64_t>(tokens) * st->d_model * st->d_ff >= 90000000);
   a.held = 0;
@@ -1372,8 +1364,10 @@ extern "C" int sub1_moe_grouped(const sub1_moe_stack *st, const int32_t *token_e
     a.wo_tiles = tiles_of(st->d_model, st->d_ff);
   }
   const size_t lds = (static_cast<size_t>(a.act_dwords) + a.held) * sizeof(float);
-  rc = sweep ? allow_lds(moe_kernel<kMoeSweepThreads>, lds) : allow_lds(moe_kernel<kMoeThreads>, lds);
-  if (rc) return rc;
+  if (sweep)
+    HIP_TRY(sub1::allow_lds<lds_limit>(moe_kernel<kMoeSweepThreads>));
+  else
+    HIP_TRY(sub1::allow_lds<most_activations>(moe_kernel<kMoeThreads>));
   a.wi_expect = a.wi_tiles + sub1::expect_extra();
   const int64_t tiles = static_cast<int64_t>(tokens) * (a.wi_tiles + a.wo_tiles);
   if (tiles > INT32_MAX - (1 << 20))

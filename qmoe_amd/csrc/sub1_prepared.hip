@@ -839,7 +839,7 @@ constexpr int kOrderThreads = 1024;
 constexpr int kOrderWaves = kOrderThreads / 64;
 constexpr int kOrderBins = kMaxRowEntries + 1;
 constexpr int kOrderAhead = 8;   // runs of 64 rows whose counts are asked for together
-size_t order_rows_lds(int height) {
+constexpr size_t order_rows_lds(int height) {
   return (kOrderBins + 1024 + 2 * kOrderWaves) * sizeof(int) + static_cast<size_t>(height + 63) / 64 * 64;
 }
 // Both kinds of a layer in one launch, a matrix of either to a workgroup: 128 base
@@ -3201,8 +3201,7 @@ int launch_walk(const Source &src, const MetaLayout &m, WalkArgs &w, hipStream_t
     tasks += k.tasks;
   }
   constexpr size_t lds = kEmit ? kWalkLds : kCountLds;
-  HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(walk_rows_kernel<kEmit>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+  HIP_TRY(sub1::allow_lds<lds>(walk_rows_kernel<kEmit>));
   walk_rows_kernel<kEmit><<<static_cast<unsigned>(std::min<int64_t>(tasks, cus)), kWalkThreads, lds, s>>>(w);
   HIP_TRY(hipGetLastError());
   if (w.long_bits) emit_long_rows_kernel<<<static_cast<unsigned>(std::min<int64_t>(tasks * kLongShares, 8 * cus)), kLongThreads, 0, s>>>(w);
@@ -3237,9 +3236,7 @@ int prepare_layout(const Source &src, void *meta, int64_t meta_bytes, LayoutResu
   }
   rc = launch_walk<false>(src, m, w, s);
   if (rc) return rc;
-  HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(order_rows_kernel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                              static_cast<int>(order_rows_lds(65534))));
+  HIP_TRY(sub1::allow_lds<order_rows_lds(65534)>(order_rows_kernel));
   int64_t slice0 = 0;
   OrderArgs o{};
   o.status = status;
@@ -3535,7 +3532,7 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
     const int rc = sub1::fault_words(&a.sticky, may_allocate);
     if (rc) return rc;
   }
-  const size_t lds_limit = 160 * 1024 - 64;
+  constexpr size_t lds_limit = sub1::kMostLds;
   const size_t lds_base = static_cast<size_t>(a.xdwords) * 4;
   if (lds_base > lds_limit) return fail(SUB1_ERR_SHAPE, "%s: width %d does not fit LDS", who, wmax);
   // Tiles.  Whole matrices when the tokens alone keep every compute unit busy;
@@ -3596,9 +3593,7 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
       }
     }
     const int64_t tiles = static_cast<int64_t>(groups) * k.parts;
-    const void *fn = reinterpret_cast<const void *>(matvec_group_kernel);
-    HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                static_cast<int>(lds_base)));
+    HIP_TRY(sub1::allow_lds<lds_limit>(matvec_group_kernel));
     sub1::note_kernel("matvec_group_kernel");
     matvec_group_kernel<<<static_cast<unsigned>(tiles < cus ? tiles : cus), 64 * waves, lds_base,
                           s>>>(a);
@@ -3740,9 +3735,7 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
     a.by_ticket = static_cast<int64_t>(tokens) * shared_parts > cus;
     const size_t lds_shared = lds_base + static_cast<size_t>(a.tail_room) * 256;
     void (*const shared)(PreparedArgs) = uneven ? moe_prepared_shared_kernel<true> : moe_prepared_shared_kernel<false>;
-    const void *fn = reinterpret_cast<const void *>(shared);
-    HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                static_cast<int>(lds_shared)));
+    HIP_TRY(sub1::allow_lds<lds_limit>(shared));
     // A token or two: h goes from wi to wo by tag (every workgroup of wo reads
     // all of it, eight bytes an entry: for small grids only).  One token, and
     // two where wo's rows are long (eight groups of chunks and more: the c-2048
@@ -3768,8 +3761,7 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
             own_wo ? uneven ? moe_prepared_uneven_split_kernel : moe_prepared_tagged_split_kernel
             : uneven ? moe_prepared_tagged_kernel<true>
                      : moe_prepared_tagged_kernel<false>;
-        HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(tagged), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    static_cast<int>(lds_shared)));
+        HIP_TRY(sub1::allow_lds<lds_limit>(tagged));
         if (own_wo) {
           a.k[1].parts = wo_parts;
           // wi's workgroups wait for nobody, so the more of them the shorter their
@@ -3837,19 +3829,16 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
     if (by_length) {
       a.tail_room = tail_groups(lds_limit / per_cu - lds_fused);
       const size_t lds_uneven = lds_fused + static_cast<size_t>(a.tail_room) * 256;
-      HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(moe_prepared_fused_kernel<false, false, true>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_uneven)));
+      HIP_TRY(sub1::allow_lds<lds_limit>(moe_prepared_fused_kernel<false, false, true>));
       sub1::note_kernel("moe_prepared_fused_kernel<false, false, true>");
       moe_prepared_fused_kernel<false, false, true>
           <<<tokens < cus * per_cu ? tokens : cus * per_cu, 64 * fw, lds_uneven, s>>>(a);
       HIP_TRY(hipGetLastError());
       return SUB1_OK;
     }
-    const void *fn = grouped ? reinterpret_cast<const void *>(moe_prepared_fused_kernel<true, false>)
-                     : once  ? reinterpret_cast<const void *>(moe_prepared_fused_kernel<false, true>)
-                             : reinterpret_cast<const void *>(moe_prepared_fused_kernel<false, false>);
-    HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                static_cast<int>(lds_fused)));
+    HIP_TRY(sub1::allow_lds<lds_limit>(grouped ? moe_prepared_fused_kernel<true, false>
+                                       : once  ? moe_prepared_fused_kernel<false, true>
+                                               : moe_prepared_fused_kernel<false, false>));
     if (grouped) {
       int32_t *tab = reinterpret_cast<int32_t *>(a.h);
       int32_t *order = tab + table_ints;
@@ -3886,11 +3875,9 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
   // Batches too small to occupy the GPU with a wavefront per slice go to the
   // latency kernel, everything else to the persistent one; either way at most
   // a workgroup per compute unit (16 wavefronts of 72 to 80 registers each).
-  const void *fn = small ? reinterpret_cast<const void *>(moe_prepared_small_kernel)
-                   : uneven ? reinterpret_cast<const void *>(moe_prepared_kernel<true>)
-                            : reinterpret_cast<const void *>(moe_prepared_kernel<false>);
-  HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              static_cast<int>(lds)));
+  HIP_TRY(sub1::allow_lds<lds_limit>(small ? moe_prepared_small_kernel
+                                     : uneven ? moe_prepared_kernel<true>
+                                              : moe_prepared_kernel<false>));
   if (small) {
     const int64_t grid = tiles < cus ? tiles : cus;
     sub1::note_kernel("moe_prepared_small_kernel");
@@ -3926,7 +3913,7 @@ struct BatchPlan {
   size_t lds;
 };
 
-constexpr size_t kBatchLds = 160 * 1024 - 64;
+constexpr size_t kBatchLds = sub1::kMostLds;
 
 // LDS holds the codes of `fit` slices beside a table: with room for three and more, workgroups
 // of up to four wavefronts, one to a SIMD; for two, of up to eight; for one, of twelve.  (128 base
@@ -4167,10 +4154,7 @@ int launch_batch(const Prepared &p, const int32_t *token_expert, const uint16_t 
     void (*const product)(BatchArgs) = i == 0               ? batch_product_kernel<true, false>
                                        : plan.table_in_lds ? batch_product_kernel<false, true>
                                                            : batch_product_kernel<false, false>;
-    // the most it may have, not what this launch has: another thread's launch, of other shapes,
-    // may lie between this call and ours
-    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(product), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                static_cast<int>(kBatchLds)));
+    HIP_TRY(sub1::allow_lds<kBatchLds>(product));
     product<<<static_cast<unsigned>((b.max_chunks + 7) / 8 * 8 * b_args.slice_groups),
               64 * plan.per_group * plan.parts, plan.lds, s>>>(b_args);
   }
@@ -4180,8 +4164,7 @@ int launch_batch(const Prepared &p, const int32_t *token_expert, const uint16_t 
   a.ldx = a.ldy = d_model;
   a.xdwords = activation_dwords(d_model);
   a.hdwords = activation_dwords(d_ff);
-  HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(walk_spoiled_kernel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kBatchLds)));
+  HIP_TRY(sub1::allow_lds<kBatchLds>(walk_spoiled_kernel));
   const size_t lds = static_cast<size_t>(a.xdwords + a.hdwords) * 4;
   walk_spoiled_kernel<<<std::min(tokens, 256), kMaxThreads, lds, s>>>(a, slots, spoiled, block_expert, totals);
   HIP_TRY(hipGetLastError());

@@ -1128,8 +1128,7 @@ int launch_shared_as(TileArgs a, int blocks, hipStream_t stream) {
   constexpr int waves = kRG * kKP;
   constexpr int lds = kKP * 2 * kNB * 32 * 256;
   static_assert(lds >= waves * (kKP - 1) * ((2 * kNB + kKP - 1) / kKP) * 4096 && lds <= 160 * 1024, "tiles, then sums");
-  HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(matvec_tiles_shared_kernel<kDirect, kRG, kKP, kNB>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+  HIP_TRY(sub1::allow_lds<lds>(matvec_tiles_shared_kernel<kDirect, kRG, kKP, kNB>));
   const int row_groups = (blocks + kRG - 1) / kRG, token_blocks = (a.tokens + 31) / 32;
   const int columns = columns_of(a.tokens, kNB, row_groups);
   a.column_blocks = token_blocks / columns;

@@ -39,3 +39,17 @@ def test_an_extension_of_another_torch_is_built_again_and_not_loaded(monkeypatch
         monkeypatch.setattr(qmoe_amd, '_tensor_args', other, raising=False)
         with pytest.raises(ImportError, match='of another torch'):
             _lib.tensor_args()
+
+
+def test_a_kernels_limit_of_lds_is_the_same_for_all_its_launches():
+    """Set to what a launch has, it can be another thread's by the time of that launch: it goes
+    through a function that takes a constant."""
+    import glob
+    import os
+    uses = {}
+    for path in glob.glob(os.path.join(build.HERE, 'csrc', '*')):
+        with open(path) as f:
+            text = f.read()
+        uses[os.path.basename(path)] = text.count('hipFuncSetAttribute'), text.count('allow_lds<')
+    assert {name: n for name, (n, _) in uses.items() if n} == {'sub1_common.h': 1}
+    assert uses['sub1_prepared.hip'][1] and uses['sub1_kernels.hip'][1]

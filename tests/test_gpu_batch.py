@@ -294,6 +294,33 @@ def test_two_threads_with_stacks_of_other_shapes():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('tokens', [1, 40, 300])
+def test_two_threads_with_uneven_stacks_of_other_shapes(tokens):
+    """As above, the forms that share long slices, and the packed launch."""
+    import threading
+    from qmoe_amd import synthetic
+    work = []
+    for d_model, d_ff in ((587, 4467), (700, 330)):
+        stack = synthetic.build_stack(3, d_model, d_ff, synthetic.ROWS, seed=21)
+        x, route = synthetic.activations(tokens, d_model, seed=18), synthetic.softmax_router(tokens, 3, seed=19)
+        work += [(s, x, route, s.forward(x, route), []) for s in (stack.prepare(), stack)]
+    torch.cuda.synchronize()
+
+    def run(stack, x, route, want, differ):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(40):
+                y = stack.forward(x, route)
+                differ.append(not torch.equal(y.view(torch.int16), want.view(torch.int16)))
+
+    threads = [threading.Thread(target=run, args=w) for w in work]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert [w[4] for w in work] == [[False] * 40] * 4
+
+
+@pytest.mark.gpu
 def test_replays_from_a_graph():
     from qmoe_amd import synthetic
     stack = synthetic.build_stack(4, 200, 300, 0.9, seed=7)
