@@ -1328,6 +1328,7 @@ typedef Walk<kRing> SliceWalk;
 
 // g_lo, g_hi: the run of chunk groups to walk, for a wavefront that shares the
 // slice with others (it then starts from the position checkpoint of group g_lo).
+constexpr int kAllGroups = 1 << 20;
 // (len, base: the slice's description, where the caller has read it already.)
 template <int R = kRing, bool kOnce = false>
 __device__ __forceinline__ Walk<R, kOnce> load_slice_described(const PreparedArgs &a,
@@ -1355,7 +1356,7 @@ __device__ __forceinline__ Walk<R, kOnce> load_slice_described(const PreparedArg
 template <int R = kRing, bool kOnce = false>
 __device__ __forceinline__ Walk<R, kOnce> load_slice(const PreparedArgs &a, const KindArgs &k,
                                                      int64_t sl, int g_lo = 0,
-                                                     int g_hi = 1 << 20) {
+                                                     int g_hi = kAllGroups) {
   const int len_word = k.slice_len[sl];
   const uint32_t base_word = k.slice_base[sl];
   return load_slice_described<R, kOnce>(a, k, sl, __builtin_amdgcn_readfirstlane(len_word),
@@ -1367,12 +1368,29 @@ __device__ __forceinline__ Walk<R, kOnce> load_slice(const PreparedArgs &a, cons
 // by the chunk R further on.
 // kChecked: the walk's last chunks, fewer than R whole ones and then chunk
 // nch - 1 with its `last` entries; nothing is requested any more.
-template <bool kChecked, int R, bool kOnce>
+// kEarly: the next R chunks are asked for before these are begun.  (Left to the compiler the last of them may be
+// asked for just before the loop waits for them all, which shows where a wavefront walks alone at the end.)
+constexpr int kAllButLoads = 0x38f;   // what may be moved over a sched_barrier: ALU and LDS instructions
+template <bool kChecked, bool kEarly = false, int R, bool kOnce>
 __device__ __forceinline__ void run_chunks(Walk<R, kOnce> &w, const uint2 *p, int c, uint32_t &at,
                                            float &part, bf16x2 minmax) {
   const int nch = w.nch;
   // the deep ring is the one of the walks built for latency
   constexpr bool kAhead = R == kSplitRing;
+  if (kEarly && !kChecked) {
+    uint2 cw[R];
+#pragma unroll
+    for (int i = 0; i < R; i++) cw[i] = w.ring[i];
+#pragma unroll
+    for (int i = 0; i < R; i++) w.ring[i] = load_chunk<kOnce>(p + min(c + i + R, nch - 1) * 64);
+    __builtin_amdgcn_sched_barrier(kAllButLoads);
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+      if (kAhead) add_chunk_ahead(cw[i], at, part, minmax);
+      else add_chunk(cw[i], at, part, minmax);
+    }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < R; i++) {
     if (!kChecked) {
@@ -1418,7 +1436,7 @@ __device__ __forceinline__ void progress_priority(int done, int total) {
 // sum at part[group * 64 + lane] for the wavefront that adds them up.
 // pass / passes (passes != 0): this slice is the wavefront's pass-th of `passes`
 // about equal ones in the current phase; sets the priority by progress.
-template <int R, bool kOnce>
+template <bool kEarly = false, int R, bool kOnce>
 __device__ __forceinline__ float run_slice(Walk<R, kOnce> &w, const uint2 *stream,
                                            const uint32_t *xa, float *part = nullptr,
                                            int pass = 0, int passes = 0) {
@@ -1445,7 +1463,7 @@ __device__ __forceinline__ float run_slice(Walk<R, kOnce> &w, const uint2 *strea
     partial = 0.f;
   };
   for (; c + R <= w.nch - 1; c += R) {
-    run_chunks<false>(w, p, c, at, partial, minmax);
+    run_chunks<false, kEarly>(w, p, c, at, partial, minmax);
     if ((c + R) % kGroupChunks == 0) group_done();
   }
   // fewer than R whole chunks are left, and the last chunk
@@ -1929,28 +1947,76 @@ struct SharedSlices {
   uint32_t base;
 };
 
-// `count` slices (at most half of `waves`) from `first` on, every `stride`-th.  A row without zeros
-// has ten times the entries of the others, and a slice of 64 such rows kept one or two
-// wavefronts walking long after the rest.
-__device__ __forceinline__ SharedSlices share_slices(const PreparedArgs &a, const KindArgs &k, int64_t first, int stride,
-                                                     int count, int waves, int wave) {
+// What is known of a tile's first 64 slices (from `first` on, every `stride`-th, longest first) before
+// they are walked: those of slice `lane`.
+struct SliceLengths {
+  int len;
+  uint32_t base;
+  int chunks, groups;   // zero: there is no such slice
+};
+__device__ __forceinline__ SliceLengths slice_lengths(const KindArgs &k, int64_t first, int stride, int all) {
   const int lane = threadIdx.x & 63;
-  const int64_t sl = first + static_cast<int64_t>(min(lane, count - 1)) * stride;
-  const int len = k.slice_len[sl];
-  const uint32_t base = k.slice_base[sl];
+  SliceLengths s = {};
+  if (all == 0) return s;
+  const int64_t sl = first + static_cast<int64_t>(min(lane, all - 1)) * stride;
+  s.len = k.slice_len[sl];
+  s.base = k.slice_base[sl];
+  s.chunks = lane < all ? chunks_of(s.len) : 0;
+  s.groups = (s.chunks + kGroupChunks - 1) / kGroupChunks;
+  return s;
+}
+
+// How many of the longest slices the wavefronts share: at most half as many as there are of those, and
+// as many as have room for their partial sums.  All of a few slices; of more those that leave whole passes, or half
+// as many as wavefronts, if what is left is short.  Else as many as give the least for what a wavefront has of them
+// and the first wavefront of the others, or none where long ones would be left all the same (a wavefront that
+// walks one has its share of the others' behind it).
+__host__ __device__ constexpr bool all_shared(int all, int waves, int groups_max, int room) {
+  return all <= waves / 2 && all * groups_max <= room;
+}
+__device__ __forceinline__ int slices_to_share(const SliceLengths &s, int all, int waves, int groups_max, int room) {
+  if (all_shared(all, waves, groups_max, room)) return all;   // (known before the lengths are here)
+  const int lane = threadIdx.x & 63;
+  const int groups_upto = sub1::wave_prefix_sum(s.groups);
+  const int rest = all % waves, usual = rest && 2 * rest <= waves ? rest : min(all, waves / 2);
+  const int longest = __builtin_amdgcn_readfirstlane(s.chunks);
+  // (nothing is left of a few slices: chunks of none are zero)
+  if (__builtin_expect(__builtin_amdgcn_readlane(groups_upto, max(usual, 1) - 1) <= room &&
+                           2 * __builtin_amdgcn_readlane(s.chunks, usual) <= longest, 1))
+    return usual;
+  // lane c: with c of them (0.4 us).  Slices beyond the 64 weigh about the same whatever c.
+  int others = 0;
+#pragma unroll 1
+  for (int at = 0; at < 64 && at < all; at += waves) others += __shfl(s.chunks, at + lane, 64);
+  // (the barrier and adding up: another group's time)
+  const int cost = sub1::wave_prefix_sum(s.chunks) - s.chunks + waves * (others + (lane ? kGroupChunks : 0));
+  const bool may = lane <= min(all, waves / 2) && groups_upto - s.groups <= room && (lane == 0 || 2 * s.chunks <= longest);
+  constexpr int kMost = (1 << 26) - 1;
+  const int gain = may ? max(kMost - cost, 1) : 0;
+  // the largest of lanes 0 to 15
+  int best = gain;
+  best = max(best, sub1::dpp_or_zero<sub1::kDppRowShr1, 0xf>(best));
+  best = max(best, sub1::dpp_or_zero<sub1::kDppRowShr2, 0xf>(best));
+  best = max(best, sub1::dpp_or_zero<sub1::kDppRowShr4, 0xf>(best));
+  best = max(best, sub1::dpp_or_zero<sub1::kDppRowShr8, 0xf>(best));
+  return __ffsll(__ballot(gain == __builtin_amdgcn_readlane(best, 15))) - 1;
+}
+
+// The `count` longest slices (at most half of `waves`).  A row without zeros has ten times the
+// entries of the others, and a slice of 64 such rows kept one or two wavefronts walking long after the rest.
+__device__ __forceinline__ SharedSlices share_slices(const SliceLengths &lengths, int count, int waves, int wave) {
+  const int lane = threadIdx.x & 63;
   const bool mine = lane < count;
-  const int groups = mine ? (chunks_of(len) + kGroupChunks - 1) / kGroupChunks : 0;
-  const int total = __builtin_amdgcn_readlane(sub1::wave_prefix_sum(groups), 63);
-  // the fewest groups a wavefront may have at most with which there are wavefronts enough, and room
-  // for the partial sums of the slices that several share (at the latest with as many as the longest has)
-  int split, split_upto, partials, partials_upto;
+  const int groups = mine ? lengths.groups : 0;
+  const int groups_upto = sub1::wave_prefix_sum(groups);
+  const int total = __builtin_amdgcn_readlane(groups_upto, 63);
+  // the fewest groups a wavefront may have at most with which there are wavefronts enough
+  // (at the latest with twice as many as they have on average)
+  int split, split_upto;
   for (int most = max((total + waves - 1) / waves, 1);; most++) {
     split = mine ? max((groups + most - 1) / most, 1) : 0;
-    partials = split > 1 ? groups : 0;
     split_upto = sub1::wave_prefix_sum(split);
-    partials_upto = sub1::wave_prefix_sum(partials);
-    if (__builtin_amdgcn_readlane(split_upto, 63) <= waves && __builtin_amdgcn_readlane(partials_upto, 63) <= a.tail_room)
-      break;
+    if (__builtin_amdgcn_readlane(split_upto, 63) <= waves) break;
   }
   const int which = __popcll(__ballot(mine && split_upto - split <= wave)) - 1;
   SharedSlices s;
@@ -1958,46 +2024,62 @@ __device__ __forceinline__ SharedSlices share_slices(const PreparedArgs &a, cons
   s.sub = wave - (__builtin_amdgcn_readlane(split_upto, which) - s.split);
   s.slice = s.sub < s.split ? which : -1;
   s.groups = __builtin_amdgcn_readlane(groups, which);
-  s.first_group = __builtin_amdgcn_readlane(partials_upto, which) - __builtin_amdgcn_readlane(partials, which);
-  s.len = __builtin_amdgcn_readlane(len, which);
-  s.base = __builtin_amdgcn_readlane(base, which);
+  s.first_group = __builtin_amdgcn_readlane(groups_upto, which) - s.groups;
+  s.len = __builtin_amdgcn_readlane(lengths.len, which);
+  s.base = __builtin_amdgcn_readlane(lengths.base, which);
   return s;
 }
 
-// As walk_alike, where lengths differ: the last pass has the longest slices instead, as many as make the
-// passes before it full or half as many as there are wavefronts, and the wavefronts by length.
+// Slices of a tile: of about one length; of differing lengths, so few that the wavefronts share all
+// of them (all_shared); of differing lengths, of which they share those that slices_to_share says.
+enum Lengths { kAlike, kFew, kDiffer };
+
+// As walk_alike, where lengths differ: the last pass has the longest slices instead, and the
+// wavefronts by length.
 //
 // Bound by the longest slice's chain of groups: a wavefront walked it alone, or a few did where eight
 // slices' partial sums, at the longest one's size, fit LDS (beyond rows of some 4400 columns without zeros they
 // did not, and the launch fell back on tiles of one projection).  Rows of 75 to 98 % zeros, one in a
-// hundred without, us before / so: 587 x 4467 one token 22.5 / 18.7, 60 tokens 106 / 31, 200 108 / 62;
-// c-2048 13 tokens 48.6 / 33.7, 60 104 / 66, 120 197 / 105, 512 418 / 376; large 60 47 / 33, 200 120 / 85; base 60
-// 36 / 26, 400 110 / 88.  (With sixteen slices in that pass, a wavefront each at least, large 200 took 136.)
-template <class Before, class Out>
+// hundred without, us, alike / so: 587 x 4467 one token 22.5 / 17.9, 60 tokens 106 / 30, 200 108 / 54;
+// c-2048 13 tokens 48.6 / 33.0, 60 104 / 64, 120 197 / 101, 512 418 / 361; large 60 47 / 32, 200 120 / 72; base 60
+// 36 / 25, 400 110 / 79.  (With sixteen slices in that pass, a wavefront each at least, large 200 took 136.)
+// More long rows than that pass takes, as slices_to_share counts / with half as many slices as
+// wavefronts or those that leave whole passes: c-2048, a tenth of the rows, 128 tokens 109 / 173, 200 196 / 330, 600
+// 490 / 757; 1100 x 9000, a fifth, 200 273 / 391; 2048 x 12000, a tenth, 200 459 / 631 (alike 185, 234, 672, 265, 448).
+//
+// kAhead: where that pass is the whole walk its loads go out before the wait and the staging.  (Whole tokens have
+// others to walk, and the code for both costs their loop: base 400 tokens 87 / 81, with kEarly 79.)
+template <Lengths kLengths, bool kAhead, class Before, class Out>
 __device__ __forceinline__ void walk_by_length(const PreparedArgs &a, const KindArgs &k, int64_t first,
                                                int stride, int all, const uint32_t *act,
                                                float *partials, Before &&before, Out &&out,
                                                bool active = true) {
   const int waves = blockDim.x >> 6, lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int rest = all % waves;
-  // (each has a wavefront at least, so that more than half as many slices would leave the longest too few)
-  const int longest = rest && 2 * rest <= waves ? rest : min(all, waves / 2);
+  const SliceLengths lengths = slice_lengths(k, first, stride, all);
+  const int longest = kLengths == kFew ? all : slices_to_share(lengths, all, waves, k.groups_max, a.tail_room);
   const int count = all - longest, passes = (count + waves - 1) / waves + 1;
+  const int64_t other = first + static_cast<int64_t>(longest) * stride;   // the first of the others
+  int s = slice_of_pass(0, wave, waves, count);
+  SliceWalk cur;
+  if (s < count && active) {
+    // (its description is here already)
+    const int at = longest + s;
+    cur = load_slice_described(a, k, other + static_cast<int64_t>(s) * stride, __builtin_amdgcn_readlane(lengths.len, at),
+                               __builtin_amdgcn_readlane(lengths.base, at), 0, kAllGroups);
+  }
   SharedSlices mine;
   mine.slice = -1;
   if (longest == 1) {
-    const int len_word = k.slice_len[first];
-    const uint32_t base_word = k.slice_base[first];
-    mine.len = __builtin_amdgcn_readfirstlane(len_word);
-    mine.base = __builtin_amdgcn_readfirstlane(base_word);
-    mine.groups = (chunks_of(mine.len) + kGroupChunks - 1) / kGroupChunks;
+    mine.len = __builtin_amdgcn_readfirstlane(lengths.len);
+    mine.base = __builtin_amdgcn_readfirstlane(lengths.base);
+    mine.groups = __builtin_amdgcn_readfirstlane(lengths.groups);
     mine.split = waves;
     mine.sub = wave;
     mine.slice = 0;
     mine.first_group = 0;
   } else if (longest) {
-    mine = share_slices(a, k, first, stride, longest, waves, wave);
+    mine = share_slices(lengths, longest, waves, wave);
   }
   const int64_t slice = first + static_cast<int64_t>(max(mine.slice, 0)) * stride;
   const bool shares = mine.slice >= 0 && active;
@@ -2007,23 +2089,18 @@ __device__ __forceinline__ void walk_by_length(const PreparedArgs &a, const Kind
     g_hi = (mine.sub + 1) * mine.groups / mine.split;
   }
   float *sums = shares && mine.split > 1 ? partials + mine.first_group * 64 : nullptr;
-  // where that pass is the whole walk its loads go out before the wait and the staging
   Walk<kSplitRing> ahead;
   int ridx = 0xffff;   // the rows of the slice, in the wavefront that adds them up
   if (shares && mine.sub == 0) ridx = k.row_idx[slice * 64 + lane];
-  if (count == 0 && g_lo < g_hi) ahead = load_slice_described<kSplitRing>(a, k, slice, mine.len, mine.base, g_lo, g_hi);
-  first += static_cast<int64_t>(longest) * stride;
-  int s = slice_of_pass(0, wave, waves, count);
-  SliceWalk cur;
-  if (s < count && active) cur = load_slice(a, k, first + static_cast<int64_t>(s) * stride);
+  if (kAhead && count == 0 && g_lo < g_hi) ahead = load_slice_described<kSplitRing>(a, k, slice, mine.len, mine.base, g_lo, g_hi);
   before();
   for (int pass = 0; s < count; pass++) {
     const int s_next = slice_of_pass(pass + 1, wave, waves, count);
     SliceWalk nxt;
     if (active) {
-      if (s_next < count) nxt = load_slice(a, k, first + static_cast<int64_t>(s_next) * stride);
-      const float res = run_slice(cur, a.stream, act, nullptr, pass, passes);
-      out(cur.ridx, res, first + static_cast<int64_t>(s) * stride);
+      if (s_next < count) nxt = load_slice(a, k, other + static_cast<int64_t>(s_next) * stride);
+      const float res = run_slice<!kAhead>(cur, a.stream, act, nullptr, pass, passes);
+      out(cur.ridx, res, other + static_cast<int64_t>(s) * stride);
       if (s_next < count) cur = nxt;
     }
     s = s_next;
@@ -2031,11 +2108,11 @@ __device__ __forceinline__ void walk_by_length(const PreparedArgs &a, const Kind
   __builtin_amdgcn_s_setprio(0);
   float sum = 0.f;
   if (g_lo < g_hi) {
-    if (count == 0) {
+    if (kAhead && count == 0) {
       sum = run_slice(ahead, a.stream, act, sums);
     } else {
       SliceWalk walk = load_slice_described(a, k, slice, mine.len, mine.base, g_lo, g_hi);
-      sum = run_slice(walk, a.stream, act, sums);
+      sum = run_slice<!kAhead>(walk, a.stream, act, sums);
     }
   }
   __syncthreads();
@@ -2050,9 +2127,9 @@ __device__ __forceinline__ void walk_by_length(const PreparedArgs &a, const Kind
 }
 
 // (A form of its own of each kernel: the choice within one cost even rows 0.2 us of 12.)
-template <bool kUneven, class... Args>
+template <Lengths kLengths, class... Args>
 __device__ __forceinline__ void walk_tile(const PreparedArgs &a, const KindArgs &k, Args &&...args) {
-  if constexpr (kUneven) walk_by_length(a, k, static_cast<Args &&>(args)...);
+  if constexpr (kLengths != kAlike) walk_by_length<kLengths, true>(a, k, static_cast<Args &&>(args)...);
   else walk_alike(a, k, static_cast<Args &&>(args)...);
 }
 
@@ -2067,7 +2144,7 @@ __device__ __forceinline__ void walk_tile(const PreparedArgs &a, const KindArgs 
 // stores and the workgroup barrier) and picked up by one acquire; an agent-scope
 // fence costs an L2 write-back on this part, which is why the lanes do not fence
 // individually.
-template <bool kUneven>
+template <Lengths kLengths>
 __global__ __launch_bounds__(kMaxThreads) void moe_prepared_kernel(PreparedArgs a) {
   extern __shared__ __align__(16) uint32_t lds[];
   __shared__ int s_ticket;
@@ -2110,7 +2187,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_kernel(PreparedArgs 
     if (e >= 0) {
       int mode;
       uint16_t *dst = tile_output(a, k, kind, t, mode);
-      walk_tile<kUneven>(a, k, static_cast<int64_t>(e) * k.slices + s_lo, 1, s_hi - s_lo, xa,
+      walk_tile<kLengths>(a, k, static_cast<int64_t>(e) * k.slices + s_lo, 1, s_hi - s_lo, xa,
                 reinterpret_cast<float *>(xa + a.xdwords),
                 [&]() { await_activations(a, k, kind, t, xa); },
                 [&](int ridx, float res, int64_t) { write_row(dst, ridx, res, mode); });
@@ -2367,7 +2444,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_fused_kernel(Prepare
     const int64_t first_i = static_cast<int64_t>(e) * ki.slices;
     if constexpr (kUneven) {
       float *partials = reinterpret_cast<float *>(ha + a.hdwords);
-      walk_tile<true>(a, ki, first_i, 1, ki.slices, xa, partials,
+      walk_by_length<kDiffer, false>(a, ki, first_i, 1, ki.slices, xa, partials,
                       [&]() {
                         stage_activations(xa, a.x + static_cast<int64_t>(t) * a.ldx, ki.width);
                         __syncthreads();
@@ -2382,7 +2459,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_fused_kernel(Prepare
                       });
       fetch_next();
       uint16_t *dst = a.y + static_cast<int64_t>(t) * a.ldy;
-      walk_tile<true>(a, ko, static_cast<int64_t>(e) * ko.slices, 1, ko.slices, ha, partials,
+      walk_by_length<kDiffer, false>(a, ko, static_cast<int64_t>(e) * ko.slices, 1, ko.slices, ha, partials,
                       [&]() { __syncthreads(); },
                       [&](int ridx, float res, int64_t) { write_row(dst, ridx, res, kStore); });
       __builtin_amdgcn_s_setprio(0);
@@ -2647,7 +2724,7 @@ __device__ __forceinline__ void leave_tagged(int32_t *ctrl, int workgroups) {
 // then hold the lowest places, the places of a token are consecutive, so at
 // most one token is partly on the GPU whatever order the hardware starts
 // workgroups in; all others run to completion and make room.
-template <bool kUneven>
+template <Lengths kOfWi, Lengths kOfWo>
 __global__ __launch_bounds__(kMaxThreads) void moe_prepared_shared_kernel(PreparedArgs a) {
   extern __shared__ __align__(16) uint32_t lds[];
   __shared__ int s_place;
@@ -2681,7 +2758,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_shared_kernel(Prepar
     return;
   }
   uint16_t *h = a.h + static_cast<int64_t>(t) * ki.height;
-  walk_tile<kUneven>(a, ki, static_cast<int64_t>(e) * ki.slices + part, parts,
+  walk_tile<kOfWi>(a, ki, static_cast<int64_t>(e) * ki.slices + part, parts,
             (ki.slices - part + parts - 1) / parts, xa, partials,
             [&]() {
               stage_finish(xa, x, ki.width, x_ahead);
@@ -2690,7 +2767,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_shared_kernel(Prepar
             [&](int ridx, float res, int64_t) { write_row(h, ridx, res, kStoreRelu); });
   publish_h(a, t);
   uint16_t *y = a.y + static_cast<int64_t>(t) * a.ldy;
-  walk_tile<kUneven>(a, ko, static_cast<int64_t>(e) * ko.slices + part, parts,
+  walk_tile<kOfWo>(a, ko, static_cast<int64_t>(e) * ko.slices + part, parts,
             (ko.slices - part + parts - 1) / parts, xa, partials,
             [&]() { await_activations(a, ko, 1, t, xa); },
             [&](int ridx, float res, int64_t) { write_row(y, ridx, res, kStore); });
@@ -2702,7 +2779,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_shared_kernel(Prepar
 // await_tagged): no drain, no barrier, no count between the projections, and no
 // word to give back at the end.  A workgroup's place is its index: the grid is
 // at most 64 workgroups.
-template <bool kUneven>
+template <Lengths kLengths>
 __global__ __launch_bounds__(kMaxThreads) void moe_prepared_tagged_kernel(PreparedArgs a) {
   extern __shared__ __align__(16) uint32_t lds[];
   uint32_t *xa = lds;
@@ -2731,7 +2808,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_tagged_kernel(Prepar
     return;
   }
   unsigned long long *ht = a.tagged + static_cast<int64_t>(t) * sub1::kTaggedWidth;
-  walk_tile<kUneven>(a, ki, static_cast<int64_t>(e) * ki.slices + part, parts,
+  walk_tile<kLengths>(a, ki, static_cast<int64_t>(e) * ki.slices + part, parts,
             (ki.slices - part + parts - 1) / parts, xa, partials,
             [&]() {
               stage_finish(xa, x, ki.width, x_ahead);
@@ -2742,7 +2819,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_tagged_kernel(Prepar
   uint16_t *y = a.y + static_cast<int64_t>(t) * a.ldy;
   // (a test that overstates the wait looks for a tag that nobody writes)
   const unsigned long long want = a.wi_expect == parts ? tag : tag + 1;
-  walk_tile<kUneven>(a, ko, static_cast<int64_t>(e) * ko.slices + part, parts,
+  walk_tile<kLengths>(a, ko, static_cast<int64_t>(e) * ko.slices + part, parts,
             (ko.slices - part + parts - 1) / parts, xa, partials,
             [&]() { await_tagged(a, ko, ht, want, xa); },
             [&](int ridx, float res, int64_t) { write_row(y, ridx, res, kStore); });
@@ -2765,7 +2842,7 @@ __global__ __launch_bounds__(kMaxThreads) void moe_prepared_tagged_kernel(Prepar
 // expert 11.5 -> 10.7, a large one 11.7 -> 11.5.
 // 62 KB of code, each instruction of it run about once: where it lies makes 0.15 us
 // (the same instructions behind kernels of another size 11.83 and 11.97), so it has a place of its own.
-template <bool kUneven>
+template <Lengths kLengths>
 __device__ __forceinline__ void tagged_split(const PreparedArgs &a) {
   extern __shared__ __align__(16) uint32_t lds[];
   uint32_t *xa = lds;
@@ -2797,7 +2874,7 @@ __device__ __forceinline__ void tagged_split(const PreparedArgs &a) {
   }
   unsigned long long *ht = a.tagged + static_cast<int64_t>(t) * sub1::kTaggedWidth;
   if (!for_wo) {
-    walk_tile<kUneven>(a, ki, static_cast<int64_t>(e) * ki.slices + place, ki.parts,
+    walk_tile<kLengths>(a, ki, static_cast<int64_t>(e) * ki.slices + place, ki.parts,
               (ki.slices - place + ki.parts - 1) / ki.parts, xa, partials,
               [&]() {
                 stage_finish(xa, x, ki.width, x_ahead);
@@ -2817,7 +2894,7 @@ __device__ __forceinline__ void tagged_split(const PreparedArgs &a) {
     uint16_t *y = a.y + static_cast<int64_t>(t) * a.ldy;
     // (a test that overstates the wait looks for a tag that nobody writes)
     const unsigned long long want = a.wi_expect == ki.parts ? tag : tag + 1;
-    walk_tile<kUneven>(a, ko, static_cast<int64_t>(e) * ko.slices + part, ko.parts,
+    walk_tile<kLengths>(a, ko, static_cast<int64_t>(e) * ko.slices + part, ko.parts,
               (ko.slices - part + ko.parts - 1) / ko.parts, xa, partials,
               [&]() {
                 await_tagged_placed(a, ko, ht,
@@ -2829,8 +2906,9 @@ __device__ __forceinline__ void tagged_split(const PreparedArgs &a) {
   if (threadIdx.x == 0) leave_tagged(a.ctrl, gridDim.x);
 }
 __global__ __launch_bounds__(kMaxThreads) __attribute__((aligned(65536)))
-void moe_prepared_tagged_split_kernel(PreparedArgs a) { tagged_split<false>(a); }
-__global__ __launch_bounds__(kMaxThreads) void moe_prepared_uneven_split_kernel(PreparedArgs a) { tagged_split<true>(a); }
+void moe_prepared_tagged_split_kernel(PreparedArgs a) { tagged_split<kAlike>(a); }
+template <Lengths kLengths>
+__global__ __launch_bounds__(kMaxThreads) void moe_prepared_uneven_split_kernel(PreparedArgs a) { tagged_split<kLengths>(a); }
 
 // For the batches too small to occupy the GPU with a wavefront per slice: built
 // for latency.  `split` wavefronts share a slice (split_begin / split_run) and
@@ -3680,7 +3758,12 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
         for (int i = 0; i < 2; i++) {
           const KindArgs &k = a.k[i];
           const double pass_us = (token_us - 8.0) * waves * p.max_chunks[i] / weight;
-          task += part_passes((k.slices + parts - 1) / parts, waves, k.groups_max) * pass_us + 0.5;
+          double passes = part_passes((k.slices + parts - 1) / parts, waves, k.groups_max);
+          // the slices of the longest one's length, if the others have a seventh: a wavefront walks each of a
+          // workgroup's if there is no room for the partial sums of all of them
+          const double longest = std::max((k.slices * average_chunks(p, i) / p.max_chunks[i] - k.slices / 7.0) * 7 / 6, 1.0);
+          if (uneven && std::ceil(longest / parts) * k.groups_max > shared_room) passes = std::max(passes, 1.0);
+          task += passes * pass_us + 0.5;
         }
         const double us = 8.0 + (rounds == 2 ? 2.24 : 1.0) * task + 0.008 * n * parts;
         if (us < best_us) {
@@ -3734,8 +3817,12 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
     a.wi_expect = a.k[0].parts + sub1::expect_extra();
     a.by_ticket = static_cast<int64_t>(tokens) * shared_parts > cus;
     const size_t lds_shared = lds_base + static_cast<size_t>(a.tail_room) * 256;
-    void (*const shared)(PreparedArgs) = uneven ? moe_prepared_shared_kernel<true> : moe_prepared_shared_kernel<false>;
-    HIP_TRY(sub1::allow_lds<lds_limit>(shared));
+    // (sharing all of a few slices needs no choice, which is 0.4 us, nor code for others)
+    const auto lengths = [&](int i) {
+      const int most = (a.k[i].slices + a.k[i].parts - 1) / a.k[i].parts;
+      return !uneven ? kAlike : all_shared(most, waves, a.k[i].groups_max, a.tail_room) ? kFew : kDiffer;
+    };
+    const auto lengths_of_both = [&]() { return std::max(lengths(0), lengths(1)); };
     // A token or two: h goes from wi to wo by tag (every workgroup of wo reads
     // all of it, eight bytes an entry: for small grids only).  One token, and
     // two where wo's rows are long (eight groups of chunks and more: the c-2048
@@ -3757,11 +3844,6 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
                           static_cast<int64_t>(tokens) * (shared_parts + wo_parts * lane_parts) <= cus;
       if (own_wo || static_cast<int64_t>(tokens) * shared_parts <= 64) {
         a.tagged = reinterpret_cast<unsigned long long *>(a.ctrl + sub1::kCtrlTagged);
-        void (*const tagged)(PreparedArgs) =
-            own_wo ? uneven ? moe_prepared_uneven_split_kernel : moe_prepared_tagged_split_kernel
-            : uneven ? moe_prepared_tagged_kernel<true>
-                     : moe_prepared_tagged_kernel<false>;
-        HIP_TRY(sub1::allow_lds<lds_limit>(tagged));
         if (own_wo) {
           a.k[1].parts = wo_parts;
           // wi's workgroups wait for nobody, so the more of them the shorter their
@@ -3774,9 +3856,19 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
                                   std::min(a.k[0].slices, (cus / tokens - wo_parts * lane_parts) * 2 / 3));
           a.k[0].parts = shared_parts;
           a.wi_expect = a.k[0].parts + sub1::expect_extra();
+          const Lengths both = lengths_of_both();
+          void (*const split)(PreparedArgs) = both == kAlike ? moe_prepared_tagged_split_kernel
+                                              : both == kFew ? moe_prepared_uneven_split_kernel<kFew>
+                                                             : moe_prepared_uneven_split_kernel<kDiffer>;
+          HIP_TRY(sub1::allow_lds<lds_limit>(split));
           sub1::note_kernel("moe_prepared_tagged_split_kernel");
-          tagged<<<tokens * (shared_parts + wo_parts * lane_parts), 64 * waves, lds_shared, s>>>(a);
+          split<<<tokens * (shared_parts + wo_parts * lane_parts), 64 * waves, lds_shared, s>>>(a);
         } else {
+          const Lengths both = lengths_of_both();
+          void (*const tagged)(PreparedArgs) = both == kAlike ? moe_prepared_tagged_kernel<kAlike>
+                                               : both == kFew ? moe_prepared_tagged_kernel<kFew>
+                                                              : moe_prepared_tagged_kernel<kDiffer>;
+          HIP_TRY(sub1::allow_lds<lds_limit>(tagged));
           sub1::note_kernel("moe_prepared_tagged_kernel");
           tagged<<<tokens * shared_parts, 64 * waves, lds_shared, s>>>(a);
         }
@@ -3784,6 +3876,11 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
         return SUB1_OK;
       }
     }
+    void (*const shared)(PreparedArgs) = !uneven                    ? moe_prepared_shared_kernel<kAlike, kAlike>
+                                         : lengths_of_both() == kFew ? moe_prepared_shared_kernel<kFew, kFew>
+                                         : lengths(1) == kFew        ? moe_prepared_shared_kernel<kDiffer, kFew>
+                                                                     : moe_prepared_shared_kernel<kDiffer, kDiffer>;
+    HIP_TRY(sub1::allow_lds<lds_limit>(shared));
     sub1::note_kernel("moe_prepared_shared_kernel");
     shared<<<tokens * shared_parts, 64 * waves, lds_shared, s>>>(a);
     HIP_TRY(hipGetLastError());
@@ -3876,8 +3973,8 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
   // latency kernel, everything else to the persistent one; either way at most
   // a workgroup per compute unit (16 wavefronts of 72 to 80 registers each).
   HIP_TRY(sub1::allow_lds<lds_limit>(small ? moe_prepared_small_kernel
-                                     : uneven ? moe_prepared_kernel<true>
-                                              : moe_prepared_kernel<false>));
+                                     : uneven ? moe_prepared_kernel<kDiffer>
+                                              : moe_prepared_kernel<kAlike>));
   if (small) {
     const int64_t grid = tiles < cus ? tiles : cus;
     sub1::note_kernel("moe_prepared_small_kernel");
@@ -3886,9 +3983,9 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
     const int64_t grid = tiles < cus ? tiles : cus;
     sub1::note_kernel("moe_prepared_kernel");
     if (uneven)
-      moe_prepared_kernel<true><<<static_cast<unsigned>(grid), 64 * waves, lds, s>>>(a);
+      moe_prepared_kernel<kDiffer><<<static_cast<unsigned>(grid), 64 * waves, lds, s>>>(a);
     else
-      moe_prepared_kernel<false><<<static_cast<unsigned>(grid), 64 * waves, lds, s>>>(a);
+      moe_prepared_kernel<kAlike><<<static_cast<unsigned>(grid), 64 * waves, lds, s>>>(a);
   }
   HIP_TRY(hipGetLastError());
   return SUB1_OK;

@@ -529,7 +529,8 @@ def test_rows_that_are_ordered_in_parts_come_back_whole(gpu, height, width, shar
 @pytest.mark.parametrize('d_model,d_ff,long_rows', [
     (300, 4467, 5),          # wo: one slice of 62 groups of entries and four of a few
     (2080, 1100, 70),        # wi: one and a bit of 29 groups, wo of 33 slices
-    (900, 900, 1), (130, 12000, 64)])   # a single long row; partial sums for which LDS has no room
+    (900, 900, 1), (130, 12000, 64),    # a single long row; partial sums for which LDS has no room
+    (650, 3000, 750), (600, 9000, 150)])   # more long slices than are shared; three, with room for two
 def test_a_few_tokens_share_long_rows(oracle, d_model, d_ff, long_rows):
     """The longest slices of a matrix are shared by wavefronts according to their lengths, to the bit."""
     import numpy as np
