@@ -3861,7 +3861,9 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
                                               : both == kFew ? moe_prepared_uneven_split_kernel<kFew>
                                                              : moe_prepared_uneven_split_kernel<kDiffer>;
           HIP_TRY(sub1::allow_lds<lds_limit>(split));
-          sub1::note_kernel("moe_prepared_tagged_split_kernel");
+          sub1::note_kernel(both == kAlike ? "moe_prepared_tagged_split_kernel"
+                            : both == kFew ? "moe_prepared_uneven_split_kernel<kFew>"
+                                           : "moe_prepared_uneven_split_kernel<kDiffer>");
           split<<<tokens * (shared_parts + wo_parts * lane_parts), 64 * waves, lds_shared, s>>>(a);
         } else {
           const Lengths both = lengths_of_both();
@@ -3869,7 +3871,9 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
                                                : both == kFew ? moe_prepared_tagged_kernel<kFew>
                                                               : moe_prepared_tagged_kernel<kDiffer>;
           HIP_TRY(sub1::allow_lds<lds_limit>(tagged));
-          sub1::note_kernel("moe_prepared_tagged_kernel");
+          sub1::note_kernel(both == kAlike ? "moe_prepared_tagged_kernel"
+                            : both == kFew ? "moe_prepared_tagged_kernel<kFew>"
+                                           : "moe_prepared_tagged_kernel<kDiffer>");
           tagged<<<tokens * shared_parts, 64 * waves, lds_shared, s>>>(a);
         }
         HIP_TRY(hipGetLastError());
@@ -3881,7 +3885,10 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
                                          : lengths(1) == kFew        ? moe_prepared_shared_kernel<kDiffer, kFew>
                                                                      : moe_prepared_shared_kernel<kDiffer, kDiffer>;
     HIP_TRY(sub1::allow_lds<lds_limit>(shared));
-    sub1::note_kernel("moe_prepared_shared_kernel");
+    sub1::note_kernel(!uneven                     ? "moe_prepared_shared_kernel"
+                      : lengths_of_both() == kFew ? "moe_prepared_shared_kernel<kFew, kFew>"
+                      : lengths(1) == kFew        ? "moe_prepared_shared_kernel<kDiffer, kFew>"
+                                                  : "moe_prepared_shared_kernel<kDiffer, kDiffer>");
     shared<<<tokens * shared_parts, 64 * waves, lds_shared, s>>>(a);
     HIP_TRY(hipGetLastError());
     return SUB1_OK;
@@ -3981,7 +3988,7 @@ int launch_prepared(const Prepared &p, const int32_t *token_matrix, const void *
     moe_prepared_small_kernel<<<static_cast<unsigned>(grid), 64 * waves, lds, s>>>(a);
   } else {
     const int64_t grid = tiles < cus ? tiles : cus;
-    sub1::note_kernel("moe_prepared_kernel");
+    sub1::note_kernel(uneven ? "moe_prepared_kernel<kDiffer>" : "moe_prepared_kernel");
     if (uneven)
       moe_prepared_kernel<kDiffer><<<static_cast<unsigned>(grid), 64 * waves, lds, s>>>(a);
     else

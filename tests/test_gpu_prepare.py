@@ -526,13 +526,20 @@ def test_rows_that_are_ordered_in_parts_come_back_whole(gpu, height, width, shar
     test_prepared_rows_come_back_whole(gpu, height, width, shares)
 
 
-@pytest.mark.parametrize('d_model,d_ff,long_rows', [
-    (300, 4467, 5),          # wo: one slice of 62 groups of entries and four of a few
-    (2080, 1100, 70),        # wi: one and a bit of 29 groups, wo of 33 slices
-    (900, 900, 1), (130, 12000, 64),    # a single long row; partial sums for which LDS has no room
-    (650, 3000, 750), (600, 9000, 150)])   # more long slices than are shared; three, with room for two
-def test_a_few_tokens_share_long_rows(oracle, d_model, d_ff, long_rows):
-    """The longest slices of a matrix are shared by wavefronts according to their lengths, to the bit."""
+UNEVEN_SPLIT, UNEVEN_SHARED = 'moe_prepared_uneven_split_kernel<%s>', 'moe_prepared_shared_kernel<%s, %s>'
+UNEVEN_FUSED = 'moe_prepared_fused_kernel<false, false, true>'
+
+
+@pytest.mark.parametrize('d_model,d_ff,long_rows,shared', [
+    (300, 4467, 5, ['Few Few', 'Differ Few']),          # wo: one slice of 62 groups of entries and four of a few
+    (2080, 1100, 70, ['Few Few', 'Differ Differ']),     # wi: one and a bit of 29 groups, wo of 33 slices
+    (900, 900, 1, ['Few Few']),                         # a single long row
+    (130, 12000, 64, ['Differ Few', 'Differ Differ']),  # partial sums for which LDS has no room
+    (650, 3000, 750, ['Few Few', 'Differ Few']),        # more long slices than are shared
+    (600, 9000, 150, ['Few Few', 'Differ Few', 'Differ Differ'])])   # three, with room for two
+def test_a_few_tokens_share_long_rows(oracle, d_model, d_ff, long_rows, shared):
+    """The longest slices of a matrix are shared by wavefronts according to their lengths, to the bit:
+    all the slices that a workgroup has, if they are few, or those that their lengths say."""
     import numpy as np
     from oracle import sub1_oracle as so
     from qmoe_amd import sub1, sub1_hip
@@ -554,6 +561,7 @@ def test_a_few_tokens_share_long_rows(oracle, d_model, d_ff, long_rows):
     xs = np.stack([so.synthetic_activation(d_model, 30 + i) for i in range(4)])
     want = [oracle.expert_ffn(wi[i % 2], wo[i % 2], xs[i], order=2)[0] for i in range(4)]
     x = torch.from_numpy(xs.view(np.int16)).cuda().view(torch.bfloat16)
+    kernels = set()
     for tokens in (1, 2, 3, 9, 33, 64, 128, 255, 600):
         ids = torch.arange(tokens) % 4
         for _ in range(2):                  # the control words are left as they were found
@@ -561,6 +569,30 @@ def test_a_few_tokens_share_long_rows(oracle, d_model, d_ff, long_rows):
             got = y.view(torch.int16).cpu().numpy().view(np.uint16)
             assert stack.launch_faults(tokens) == (0, 0)
             assert (got == np.stack(want)[ids]).all(), tokens
+            kernels.add(sub1_hip._lib.load().sub1_last_kernel().decode())
+    assert kernels == {UNEVEN_SPLIT % 'kFew', UNEVEN_FUSED} | {
+        UNEVEN_SHARED % tuple('k' + kind for kind in kinds.split()) for kinds in shared}
+
+
+@pytest.mark.parametrize('d_model,d_ff,tokens,kernel', [
+    (6144, 12000, 1, UNEVEN_SPLIT % 'kDiffer'),        # several slices of wi to a workgroup, and little room
+    (7000, 700, 1, 'moe_prepared_tagged_kernel<kFew>'), (7000, 12000, 1, 'moe_prepared_tagged_kernel<kDiffer>')])
+def test_a_token_or_two_through_large_uneven_rows(oracle, d_model, d_ff, tokens, kernel):
+    import numpy as np
+    from qmoe_amd import _lib, synthetic
+    stack = synthetic.build_stack(1, d_model, d_ff, synthetic.ROWS, seed=d_model)
+    prepared = stack.prepare()
+    x = synthetic.activations(tokens, d_model, seed=3)
+    y = prepared.forward(x, torch.zeros(tokens, dtype=torch.int32, device='cuda'))
+    assert _lib.load().sub1_last_kernel().decode() == kernel
+
+    def bits(t):
+        return t.view(torch.int16).cpu().numpy().view(np.uint16) if t.dtype != torch.int32 else t.cpu().numpy()
+
+    wi, wo = [tuple(bits(t) for t in layer) for layer in synthetic.expert_layers(stack, 0)]
+    for got, token in zip(bits(y), bits(x)):
+        assert (got == oracle.expert_ffn(wi, wo, token, order=2)[0]).all()
+    assert prepared.launch_faults(tokens) == (0, 0)
 
 
 @pytest.mark.parametrize('height,width,long_rows', [(3000, 1100, 40), (1100, 4467, 70), (64 * 33, 700, 3)])
@@ -595,4 +627,4 @@ def test_matrices_of_long_rows(oracle, height, width, long_rows):
                          torch.from_numpy((ids % 2).astype(np.int32)).cuda())
         kernels.add(_lib.load().sub1_last_kernel())
         assert (y.view(torch.int16).cpu().numpy().view(np.uint16) == want[ids]).all(), tokens
-    assert b'moe_prepared_kernel' in kernels
+    assert b'moe_prepared_kernel<kDiffer>' in kernels
