@@ -3250,6 +3250,23 @@ struct Prepared {
   int max_chunks[2];
 };
 
+// Chunks of an average slice of a kind, by what its width is of the stream.
+double average_chunks(const Prepared &p, int kind) {
+  double weight = 0.0;
+  for (int i = 0; i < p.kinds; i++) weight += static_cast<double>((p.height[i] + 63) / 64) * p.width[i];
+  return static_cast<double>(p.total_chunks) / p.count * p.width[kind] / weight;
+}
+
+// The longest slice of rows of one share of zeros has 1.2 to 1.4 times an average one's chunks (1.7 of 500
+// columns with 95 %, hence the two chunks), of rows of which one in a hundred has no zeros 5 to 10 times.
+// In between, rows of 90 % zeros and one in a hundred of fewer, the forms for differing lengths begin to pay at
+// 2 (few tokens) to 2.8 times (whole tokens).  us, alike / differing, the longest slice 1.9 times an average one: base, 4, 60 and
+// 200 tokens 12.6 / 12.4, 17.6 / 19.2, 35.6 / 38.1, c-2048 17.9 / 17.7, 51.6 / 53.3, 128 / 137; 2.4 times: 12.9 / 12.7, 19.6 / 19.9,
+// 37.8 / 38.4, 18.9 / 18.7, 55.8 / 51.3, 129 / 135; 2.9 times: 13.8 / 13.2, 20.3 / 20.5, 41.5 / 39.0, 19.6 / 19.3, 63.9 / 53.0, 135 / 135.
+bool is_uneven(const Prepared &p, int kind) {
+  return p.max_chunks[kind] > 2.0 * average_chunks(p, kind) + 2.0;
+}
+
 struct LayoutResult {
   int64_t meta_bytes, code_bytes, total_chunks;
   int max_chunks[2];
@@ -3377,12 +3394,9 @@ int prepare_codes(const Source &src, const Prepared &p, hipStream_t s, const cha
   if (rc) return rc;
   uint2 *stream = static_cast<uint2 *>(const_cast<void *>(p.codes));
   uint16_t *ckpt = reinterpret_cast<uint16_t *>(stream + p.total_chunks * 64);
-  // Where a kind's longest slice is twice what the stream's size says of an average one, some rows
-  // are long ones (or a few rows are, of a narrow matrix: the launch for them then finds none, 4 us).
-  double weights = 0.0;
-  for (int i = 0; i < src.kinds; i++) weights += static_cast<double>(src.count) * src.height[i] * src.width[i];
+  // Some rows are long ones, if any are (or a few are, of a narrow matrix: the launch for them then finds none, 4 us).
   for (int i = 0; i < src.kinds; i++)
-    if (p.max_chunks[i] > 2.0 * static_cast<double>(p.total_chunks) * 64.0 / weights * src.width[i] + 2.0)
+    if (is_uneven(p, i))
       w.long_bits = reinterpret_cast<uint32_t *>(base + m.status) + kStatusLong;
   w.stream = stream;
   w.ckpt = ckpt;
@@ -3511,20 +3525,6 @@ double part_passes(int slices, int waves, int groups_max) {
     passes += std::max(static_cast<double>(rest * split) / waves, 0.3) / split;
   }
   return passes;
-}
-
-// Chunks of an average slice of a kind, by what its width is of the stream.
-double average_chunks(const Prepared &p, int kind) {
-  double weight = 0.0;
-  for (int i = 0; i < p.kinds; i++) weight += static_cast<double>((p.height[i] + 63) / 64) * p.width[i];
-  return static_cast<double>(p.total_chunks) / p.count * p.width[kind] / weight;
-}
-
-// The longest slice of rows of one share of zeros has 1.2 to 1.4 times an average one's chunks (1.7 of 500
-// columns with 95 %, hence the two chunks), of rows of which one in a hundred has no zeros 5 to 10 times.
-// Even rows lose 0.2 us of 12 by the form for differing lengths; layers in between were not measured.
-bool is_uneven(const Prepared &p, int kind) {
-  return p.max_chunks[kind] > 2.0 * average_chunks(p, kind) + 2.0;
 }
 
 // Launch of the prepared kernels.  kinds == 2: y = wo(relu(wi x)) per token,
