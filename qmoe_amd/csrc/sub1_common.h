@@ -172,6 +172,7 @@ constexpr int kCtrlHeader = kCtrlTagged + kTaggedTokens * kTaggedWidth * 2;   //
 // The words lie 64 bytes apart: every workgroup of a token adds to its word and
 // polls it, and words that share a 64-byte sector queue behind each other in
 // the L2 (16 tokens' words in one sector cost a 16-token launch 1.5-2.5 us).
+// (A packed launch with a workgroup for every tile uses the words behind a token's own too.)
 constexpr int kTokenWaited = 1 << 16;
 constexpr int kCtrlTokenStride = 16;   // int32 words from one token's word to the next
 

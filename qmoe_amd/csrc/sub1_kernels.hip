@@ -607,14 +607,15 @@ __global__ void tell_count_kernel(sub1::Answer answer) {
 //
 // A few tokens have a workgroup for every tile instead, by number, so that wi's tiles lie one to a compute
 // unit, and a wo tile's has its rows' codes and their words of the table by the time h is there.
-// (One token of base and c-2048 shapes 28.9 -> 17.3 us and 44.5 -> 22.5, nine of base shapes 43.8 -> 21.3,
-// with tickets and everything fetched behind the wait; with a ticket that only says which tile, of the launch
+// (One token of base and c-2048 shapes 17.7 us and 23.4, nine of base shapes 21.9; 28.9, 44.5 and 43.8 with
+// tickets and everything fetched behind the wait; with a ticket that only says which tile, of the launch
 // or of the token, 14 tokens of base shapes 22.6 -> 28.8 and 24.5, nine of c-2048 50.5 -> 62 and 68, as wi's tiles
 // then share units.)  They run all at once on a GPU that does nothing else; where other launches hold
 // units, workgroups that wait may keep those that they wait for from starting.  Every wi tile is therefore
 // CLAIMED by the workgroup that does it, and one that has waited for some time claims what nobody has, does
 // it and waits on: nobody waits for a tile that no running workgroup has, so this wait always ends too.
-// (Claims take 0.5 us of the 17 to 25 of a few tokens of base and large shapes.)
+// (Claims take 0.5 us of the 17 to 25 of a few tokens of base and large shapes.  Asked for behind the loads, which
+// wait for the answer, they come so late that others are claimed for nothing: c-2048, two tokens, 30 -> 45.)
 //
 // Within a tile the wavefronts take runs of rows from a counter in LDS and give a
 // LANE to a GROUP of 32 codes, not to a row: a row's sum is the sum of its groups'
